@@ -4,12 +4,14 @@ There is no CPU or PyTorch fallback: if the library is missing, or a tensor is
 not on a HIP device, the call raises.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("LLMK_LIB", os.path.join(_HERE, "libllmk_gfx950.so"))
+HOST_PATH = os.path.join(_HERE, "llmk_host.so")
 
 F32, F16, BF16 = 0, 1, 2
 ROUND_HALF_AWAY, ROUND_HALF_UP = 0, 1
@@ -96,6 +98,29 @@ def load():
         fn.restype = _RESTYPE.get(name, _i)
     _lib = lib
     return lib
+
+
+class _Host:
+    """The operators' native host side (csrc/host.cpp: checks, outputs, scratch and the call through the C ABI), loaded
+    when the first of its functions is called."""
+
+    def __getattr__(self, name):
+        if name.startswith("__"):
+            raise AttributeError(name)
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise LlmkError("llmk_host.so is not built (%s). Run `python -m llm_kernels_amd.build`" % HOST_PATH)
+        spec = importlib.util.spec_from_file_location("llmk_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind(LIB_PATH, LlmkError, _ws)
+        for k, v in vars(mod).items():
+            if not k.startswith("__"):
+                setattr(self, k, v)
+        return getattr(mod, name)
+
+
+host = _Host()
 
 
 def dt(dtype: torch.dtype) -> int:

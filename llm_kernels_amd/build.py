@@ -1,8 +1,9 @@
-"""Build libllmk_gfx950.so from csrc/*.hip with hipcc (cross-compiles without a GPU).
+"""Build libllmk_gfx950.so from csrc/*.hip with hipcc (cross-compiles without a GPU), and llmk_host.so, the operators'
+CPython side, from csrc/host.cpp.
 
     python -m llm_kernels_amd.build [-j N]
 
-The library lands next to this file so that it travels with the source tree.
+Both land next to this file so that they travel with the source tree.
 """
 import concurrent.futures as cf
 import os
@@ -14,6 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libllmk_gfx950.so")
+HOST = os.path.join(HERE, "llmk_host.so")
 
 # -packed-fp32-ops off: hipcc must not form v_pk_{add,mul,fma}_f32 from scalar float code
 FLAGS = [
@@ -37,6 +39,25 @@ def _compile(src):
     if r.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, r.stdout, r.stderr))
     return obj
+
+
+def _host_module():
+    """The CPython side of the operators (host code only: no kernels, so the host compiler builds it)."""
+    import sysconfig
+    import torch
+    t = os.path.dirname(torch.__file__)
+    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"]]
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+    for d in inc:
+        cmd += ["-isystem", d]
+    cmd += [os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + os.path.join(t, "lib"), "-lc10", "-ltorch_cpu", "-ltorch", "-lc10_hip",
+            "-ltorch_hip", "-ltorch_python", "-ldl"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for host.cpp:\n%s\n%s" % (r.stdout, r.stderr))
+    return HOST
 
 
 def _assembly(src):
@@ -72,9 +93,11 @@ def build(jobs=None, verbose=True):
     # source is checked (a source without such loads has nothing to flag); a source whose text, or a header it
     # includes, contains hand-issued loads must show at least one in its assembly, otherwise the check has gone blind.
     with cf.ThreadPoolExecutor(jobs) as ex:
+        host_job = ex.submit(_host_module)
         asm_jobs = [(s, ex.submit(_assembly, s)) for s in srcs]
         objs = list(ex.map(_compile, srcs))
         checked = 0
+        host_job.result()
         for src, j in asm_jobs:
             n, problems = check_asm.check_file(j.result())
             checked += n

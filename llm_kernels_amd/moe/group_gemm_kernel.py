@@ -31,16 +31,11 @@ def run_moe_ep_preproess(topk_ids: torch.Tensor, num_experts: int):
     """Stable sort of the flattened expert ids -> (sorted ids, src2dst int32 [T*topk], seg_indptr int64 [E+1])."""
     _lib.require_gpu(topk_ids)
     n = topk_ids.numel()
-    st = _lib.stream(topk_ids)
     if (n <= PREPROCESS_MAX_IDS and num_experts <= PREPROCESS_MAX_EXPERTS and topk_ids.is_contiguous()
             and topk_ids.dtype in (torch.int32, torch.int64)):
         # the id counts of one forward pass: one launch instead of the eight of sort + pointers + map
-        reorder_topk_ids = torch.empty(n, device=topk_ids.device, dtype=topk_ids.dtype)
-        seg_indptr = torch.empty(num_experts + 1, device=topk_ids.device, dtype=torch.int64)
-        src2dst = torch.empty(n, device=topk_ids.device, dtype=torch.int32)
-        _lib.call("llmk_moe_ep_preprocess", _lib.ptr(topk_ids), _ids_bytes(topk_ids), n, int(num_experts),
-                  _lib.ptr(reorder_topk_ids), _lib.ptr(src2dst), _lib.ptr(seg_indptr), st)
-        return reorder_topk_ids, src2dst, seg_indptr
+        return _lib.host.ep_preprocess(topk_ids, int(num_experts))
+    st = _lib.stream(topk_ids)
     reorder_topk_ids, reorder_ids = torch.sort(topk_ids.view(-1), stable=True)
     seg_indptr = torch.zeros(num_experts + 1, device=topk_ids.device, dtype=torch.int64)
     src2dst = torch.empty(n, device=topk_ids.device, dtype=torch.int32)
@@ -101,26 +96,18 @@ def gelu_and_mul(gateup_output, down_input, hidden_size, reorder_topk_ids, scale
 def post_reorder(down_output, output, src2dst, topk_ids, topk_weights, start_expert_id, end_expert_id, topk,
                  hidden_size):
     """output[t] = sum_j down_output[src2dst[t, j]] * dtype(topk_weights[t, j]), summed in the tensor dtype."""
-    _lib.require_gpu(down_output, output, src2dst, topk_ids, topk_weights)
-    assert down_output.is_contiguous() and output.is_contiguous() and topk_weights.is_contiguous()
-    assert down_output.dtype == output.dtype
-    T = output.numel() // hidden_size
-    _lib.call("llmk_moe_post_reorder", _lib.ptr(down_output), _lib.ptr(output), _lib.dt(output.dtype),
-              _lib.ptr(src2dst), _lib.ptr(topk_ids), _ids_bytes(topk_ids), _lib.ptr(topk_weights),
-              _lib.dt(topk_weights.dtype), int(start_expert_id), int(end_expert_id), int(topk), T,
-              int(hidden_size), _lib.stream(output))
-    return output
+    return _lib.host.post_reorder(down_output, output, src2dst, topk_ids, topk_weights, int(start_expert_id),
+                                  int(end_expert_id), int(topk), int(hidden_size))
 
 
-def _quant_buffers(rows, cols, quant_dtype, device):
-    """(q, s, kind, round_mode) for the 1 x 128 activation format that goes with a weight dtype."""
-    assert cols % 128 == 0, 'row length must be a multiple of 128'
-    if quant_dtype == torch.float8_e4m3fn:
-        return (torch.empty(rows, cols, device=device, dtype=torch.float8_e4m3fn),
-                torch.empty(rows, cols // 128, device=device, dtype=torch.float32), _lib.KIND_FP8, 0)
-    assert quant_dtype == torch.int8, 'quant_dtype must be torch.int8 or torch.float8_e4m3fn'
-    return (torch.empty(rows, cols, device=device, dtype=torch.int8),
-            torch.empty(rows, cols // 128, device=device, dtype=torch.float16), _lib.KIND_I8, 0)
+def _is_fp8(quant_dtype):
+    """Which 1 x 128 activation format goes with a weight dtype: e4m3 with fp32 scales, or int8 with fp16 scales."""
+    fp8 = quant_dtype == torch.float8_e4m3fn
+    assert fp8 or quant_dtype == torch.int8, 'quant_dtype must be torch.int8 or torch.float8_e4m3fn'
+    return fp8
+
+
+_ACTS = {"silu": 0, "gelu": 1}
 
 
 def pre_reorder_quant(input, src2dst, topk_ids, a1_scales, start_expert_id, end_expert_id, topk, hidden_size,
@@ -128,16 +115,8 @@ def pre_reorder_quant(input, src2dst, topk_ids, a1_scales, start_expert_id, end_
     """pre_reorder followed by the 1 x 128 activation quantizer, in one pass (the reference's TODO at
     sglang_moe_all_gather_all_reduce.py:295-296).  Returns (q [T*topk, hidden], s [T*topk, hidden/128]); equal
     bit for bit to act_quant(pre_reorder(...)).  Rows of non-local experts are left unwritten."""
-    _lib.require_gpu(input, src2dst, topk_ids)
-    assert input.is_contiguous() and src2dst.is_contiguous() and topk_ids.is_contiguous()
-    assert input.dtype in (torch.float16, torch.bfloat16)
-    T = input.numel() // hidden_size
-    q, s, kind, mode = _quant_buffers(T * topk, hidden_size, quant_dtype, input.device)
-    sc = _f32_or_none(a1_scales)
-    _lib.call("llmk_moe_pre_reorder_quant", _lib.ptr(input), _lib.dt(input.dtype), _lib.ptr(q), _lib.ptr(s), kind, mode,
-              _lib.ptr(src2dst), _lib.ptr(topk_ids), _ids_bytes(topk_ids), _lib.ptr(sc), int(start_expert_id),
-              int(end_expert_id), int(topk), T, int(hidden_size), _lib.stream(input))
-    return q, s
+    return _lib.host.pre_reorder_quant(input, src2dst, topk_ids, a1_scales, int(start_expert_id), int(end_expert_id),
+                                       int(topk), int(hidden_size), _is_fp8(quant_dtype))
 
 
 def act_and_mul_quant(gateup_output, hidden_size, reorder_topk_ids, scales, start_expert_id, end_expert_id, quant_dtype,
@@ -145,26 +124,14 @@ def act_and_mul_quant(gateup_output, hidden_size, reorder_topk_ids, scales, star
     """silu_and_mul / gelu_and_mul followed by the 1 x 128 activation quantizer, in one pass (the reference's TODO
     at sglang_moe_all_gather_all_reduce.py:365,407-408).  `hidden_size` is the gate+up width 2I as in
     silu_and_mul.  Returns (q [M, I], s [M, I/128]); equal bit for bit to act_quant(silu_and_mul(...))."""
-    _lib.require_gpu(gateup_output, reorder_topk_ids)
-    assert gateup_output.is_contiguous() and reorder_topk_ids.is_contiguous()
-    assert gateup_output.dtype in (torch.float16, torch.bfloat16)
-    M = gateup_output.numel() // hidden_size
-    q, s, kind, mode = _quant_buffers(M, hidden_size // 2, quant_dtype, gateup_output.device)
-    sc = _f32_or_none(scales)
-    _lib.call("llmk_moe_act_and_mul_quant", _lib.ptr(gateup_output), _lib.dt(gateup_output.dtype), _lib.ptr(q),
-              _lib.ptr(s), kind, mode, _lib.ptr(reorder_topk_ids), _ids_bytes(reorder_topk_ids), _lib.ptr(sc),
-              int(start_expert_id), int(end_expert_id), M, int(hidden_size), {"silu": 0, "gelu": 1}[activation],
-              _lib.stream(gateup_output))
-    return q, s
+    return _lib.host.act_and_mul_quant(gateup_output, int(hidden_size), reorder_topk_ids, scales, int(start_expert_id),
+                                       int(end_expert_id), _is_fp8(quant_dtype), _ACTS[activation])
 
 
 def grouped_gemm_swiglu_quant_fused(a, b, batch_size):
     """True when `grouped_gemm_swiglu_quant` runs this gate / up projection in one kernel (shapes that the 256-column
     tile kernel takes); otherwise run grouped_gemm_triton and act_and_mul_quant."""
-    kind = {torch.int8: _lib.KIND_I8, torch.float8_e4m3fn: _lib.KIND_FP8}.get(b.dtype)
-    if kind is None or a.dtype != b.dtype or b.dim() != 3:
-        return False
-    return bool(_lib.load().llmk_grouped_gemm_swiglu_quant_fused(kind, int(batch_size), a.shape[0], b.shape[1], b.shape[2]))
+    return _lib.host.swiglu_fused(a, b, int(batch_size))
 
 
 def grouped_gemm_swiglu_quant(a, scale_a, b, scale_b, batch_size, seg_indptr, weight_indices, mid_dtype, activation="silu"):
@@ -174,26 +141,9 @@ def grouped_gemm_swiglu_quant(a, scale_a, b, scale_b, batch_size, seg_indptr, we
     the three kernels one after the other, sglang_moe_all_gather_all_reduce.py:330-408).  a [M, K] and b [E, 2I, K]
     int8 or float8_e4m3fn with 1 x 128 / 128 x 128 block scales.  Returns (q [M, I], s [M, I/128]); rows outside every
     segment are left unwritten.  Only for shapes for which grouped_gemm_swiglu_quant_fused() is true."""
-    _lib.require_gpu(a, b, scale_a, scale_b, seg_indptr)
-    assert a.is_contiguous() and b.is_contiguous() and a.dtype == b.dtype and b.dim() == 3 and a.shape[-1] == b.shape[-1]
     assert mid_dtype in (torch.float16, torch.bfloat16)
-    M, two_i, K = a.shape[0], b.shape[1], b.shape[2]
-    q, s, kind, mode = _quant_buffers(M, two_i // 2, b.dtype, a.device)
-    scale_a, scale_b = scale_a.contiguous(), scale_b.contiguous()
-    if scale_b.dtype != scale_a.dtype:
-        scale_b = scale_b.to(scale_a.dtype)
-    seg = (seg_indptr if seg_indptr.dtype == torch.int64 else seg_indptr.to(torch.int64)).contiguous()
-    wi = None
-    if weight_indices is not None:
-        wi = (weight_indices if weight_indices.dtype == torch.int64 else weight_indices.to(torch.int64)).contiguous()
-    ws, ws_bytes = None, 0
-    if scale_a.dtype != torch.float32:
-        ws_bytes = M * (K // 128) * 4
-        ws = _lib.ptr(_lib.workspace(a.device, ws_bytes))
-    _lib.call("llmk_grouped_gemm_swiglu_quant", _lib.ptr(a), _lib.ptr(b), _lib.ptr(q), _lib.ptr(s), kind, _lib.dt(mid_dtype),
-              mode, int(batch_size), M, two_i, K, _lib.ptr(seg), _lib.ptr(wi), _lib.ptr(scale_a), _lib.ptr(scale_b),
-              _lib.dt(scale_a.dtype), {"silu": 0, "gelu": 1}[activation], ws, ws_bytes, _lib.stream(a), exc=AssertionError)
-    return q, s
+    return _lib.host.swiglu_quant(a, scale_a, b, scale_b, int(batch_size), seg_indptr, weight_indices, _lib.dt(mid_dtype),
+                                  _ACTS[activation])
 
 
 class _GridCall:
@@ -277,27 +227,4 @@ def grouped_gemm_triton(
                   a.shape[0], b.shape[1], b.shape[2], _lib.ptr(scale_a), _lib.ptr(scale_b), _lib.dt(sdt), _lib.stream(a))
     elif quantised_w:
         raise AssertionError('quantised weights need block_shape=[128, 128] and scale_b, or use_fp8_w8a8 with per-expert scales')
-    assert a.is_contiguous() and b.is_contiguous() and c.is_contiguous(), 'Input tensors must be contiguous'
-    assert b.dim() == 3 and a.shape[-1] == b.shape[-1] and c.shape[-1] == b.shape[1] and c.shape[0] == a.shape[0]
-    assert a.dtype == b.dtype, 'a and b must share a dtype after activation quantisation'
-    kind = {torch.int8: _lib.KIND_I8, torch.float8_e4m3fn: _lib.KIND_FP8,
-            torch.float16: _lib.KIND_F16, torch.bfloat16: _lib.KIND_BF16}.get(b.dtype)
-    assert kind is not None, 'unsupported operand dtype %s' % b.dtype
-    s_dt = 0
-    if kind in (_lib.KIND_I8, _lib.KIND_FP8):
-        scale_b = scale_b.contiguous()
-        if scale_b.dtype != scale_a.dtype:
-            scale_b = scale_b.to(scale_a.dtype)
-        s_dt = _lib.dt(scale_a.dtype)
-    else:
-        scale_a = scale_b = None
-    seg = seg_indptr if seg_indptr.dtype == torch.int64 else seg_indptr.to(torch.int64)
-    seg = seg.contiguous()
-    wi = None
-    if weight_indices is not None:
-        wi = (weight_indices if weight_indices.dtype == torch.int64 else weight_indices.to(torch.int64)).contiguous()
-    _lib.call("llmk_grouped_gemm", _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), kind, _lib.dt(c.dtype), int(batch_size),
-              a.shape[0], b.shape[1], b.shape[2], _lib.ptr(seg), _lib.ptr(wi), _lib.ptr(scale_a), _lib.ptr(scale_b),
-              s_dt, *_lib.gemm_workspace(a.device, a.shape[0], b.shape[1], b.shape[2]), _lib.stream(a),
-              exc=AssertionError)
-    return c
+    return _lib.host.grouped_gemm(a, b, c, int(batch_size), seg_indptr, weight_indices, scale_a, scale_b)

@@ -18,14 +18,7 @@ except ImportError:  # this directory itself is on sys.path (the reference's top
 
 def int8_quant(x: torch.Tensor, block_size: int = 32) -> Tuple[torch.Tensor, torch.Tensor]:
     """1 x block_size groups: s = max|x| / 127 (fp32), y = floor(x / s + 0.5) as int8, s stored as float16."""
-    assert x.is_contiguous(), 'Input tensor must be contiguous'
-    assert x.size(-1) % block_size == 0, f'Last dimension size must be divisible by block_size (block_size={block_size})'
-    _lib.require_gpu(x)
-    y = torch.empty_like(x, dtype=torch.int8)
-    s = x.new_empty(*x.size()[:-1], x.size(-1) // block_size, dtype=torch.float16)
-    _lib.call("llmk_act_quant_i8", _lib.ptr(x), _lib.dt(x.dtype), _lib.ptr(y), _lib.ptr(s),
-              x.numel() // block_size, block_size, 1, _lib.stream(x), exc=AssertionError)
-    return y, s
+    return _lib.host.act_quant(x, block_size, 3)
 
 
 def _dequant(y, s, output_dtype, kind):
@@ -47,14 +40,7 @@ def int8_dequant(y: torch.Tensor, s: torch.Tensor, output_dtype: torch.dtype) ->
 
 def fp8_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, torch.Tensor]:
     """1 x block_size groups: s = max|x| / 448 (fp32), y = (x / s) as float8_e4m3fn, s stored as float16."""
-    assert x.is_contiguous(), 'Input tensor must be contiguous'
-    assert x.size(-1) % block_size == 0, f'Last dimension size must be divisible by block_size (block_size={block_size})'
-    _lib.require_gpu(x)
-    y = torch.empty_like(x, dtype=torch.float8_e4m3fn)
-    s = x.new_empty(*x.size()[:-1], x.size(-1) // block_size, dtype=torch.float16)
-    _lib.call("llmk_comm_quant_fp8", _lib.ptr(x), _lib.dt(x.dtype), _lib.ptr(y), _lib.ptr(s), _lib.dt(s.dtype),
-              x.numel() // block_size, block_size, _lib.stream(x), exc=AssertionError)
-    return y, s
+    return _lib.host.act_quant(x, block_size, 4)
 
 
 def fp8_dequant(y: torch.Tensor, s: torch.Tensor, output_dtype: torch.dtype) -> torch.Tensor:

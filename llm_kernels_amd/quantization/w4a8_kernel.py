@@ -21,14 +21,7 @@ W_BITS = 4
 
 def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, torch.Tensor]:
     """1 x block_size groups: s = max|x| / 127 (fp32), y = floor(x / s + 0.5) int8, s stored fp16."""
-    assert x.is_contiguous(), 'Input tensor must be contiguous'
-    assert x.size(-1) % block_size == 0, f'Last dimension size must be divisible by block_size (block_size={block_size})'
-    _lib.require_gpu(x)
-    y = torch.empty_like(x, dtype=torch.int8)
-    s = x.new_empty(*x.size()[:-1], x.size(-1) // block_size, dtype=torch.float16)
-    _lib.call("llmk_act_quant_i8", _lib.ptr(x), _lib.dt(x.dtype), _lib.ptr(y), _lib.ptr(s),
-              x.numel() // block_size, block_size, _lib.ROUND_HALF_UP, _lib.stream(x))
-    return y, s
+    return _lib.host.act_quant(x, block_size, 2)
 
 
 def weight_quant(x: torch.Tensor, block_size: int = 128, group_size_int4: int = 128,
@@ -80,22 +73,6 @@ def w4a8_gemm(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor,
               GROUP_SIZE_INT4: int = 128, elements_per_sample: int = 8,
               pack_direction: str = "row") -> torch.Tensor:
     """c = a(int8) x dequant_int8(b)^T with per-128-K a_s * b_s scaling; default dtype out."""
-    assert a.is_contiguous() and b.is_contiguous(), 'Input tensors must be contiguous'
-    assert a_s.is_contiguous() and b_s.is_contiguous(), 'Scaling factor tensors must be contiguous'
-    assert b_s4.is_contiguous() and b_z4.is_contiguous(), 'Scaling factor and zero point tensors must be contiguous'
     assert pack_direction == "row", "Only row packing is supported for dequantization"
     assert elements_per_sample == PACKING_BITS // W_BITS, 'weights must be packed 8 nibbles per int32'
-    _lib.require_gpu(a, a_s, b, b_s, b_s4, b_z4)
-    K = a.size(-1)
-    M = a.numel() // K
-    N = b.size(0) * elements_per_sample
-    assert a_s.dtype == b_s.dtype, 'activation and weight scales must share a dtype'
-    c = a.new_empty(*a.size()[:-1], N, dtype=torch.get_default_dtype())
-    # what this shape's kernels use: nothing for the fused decode kernel with K <= 4096, fp32 partial sums for its
-    # K ranges or the K slices of the fused tile kernels, the expanded int8 weights + the int8 GEMM's scratch otherwise
-    need = _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, GROUP_SIZE_INT4)
-    ws = _lib.workspace(a.device, need) if need > 0 else None
-    _lib.call("llmk_gemm_w4a8", _lib.ptr(a), _lib.ptr(a_s), _lib.ptr(b), _lib.ptr(b_s), _lib.dt(a_s.dtype),
-              _lib.ptr(b_s4), _lib.ptr(b_z4), _lib.ptr(c), _lib.dt(c.dtype), M, N, K, GROUP_SIZE_INT4,
-              _lib.ptr(ws), need if ws is not None else 0, _lib.stream(a), exc=AssertionError)
-    return c
+    return _lib.host.w4a8_gemm(a, a_s, b, b_s, b_s4, b_z4, GROUP_SIZE_INT4)
