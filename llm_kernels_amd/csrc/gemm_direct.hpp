@@ -16,8 +16,13 @@ namespace llmk {
 enum : int { K_FP8_BLOCK = 0, K_I8_BLOCK = 1, K_I8_ROWCOL = 2, K_F16 = 3, K_BF16 = 4,
              K_W4NK = 5,      // fp16 activations x 4-bit weights packed [N, K/8] (tile kernels only)
              K_W4MARLIN = 6,  // the same with weights and scales in the Marlin layout
+             K_W4NKB = 8,     // K_W4NK with bf16 activations (bf16 weights (q - 8) * scale)
              K_W4A8 = 7 };    // int8 activations x uint4 weights packed eight rows per word [N/8, K] with int8 zero
                               // point and scale per (row, 128-K group) and 128 x 128 block scales (tile kernels only)
+
+constexpr bool is_w4nk(int kind) { return kind == K_W4NK || kind == K_W4NKB; }
+// kinds whose activations (and expanded weights) are 16-bit
+constexpr bool is_half(int kind) { return kind == K_F16 || kind == K_BF16 || is_w4nk(kind) || kind == K_W4MARLIN; }
 
 __device__ __forceinline__ float ld_scale(const void* p, int64_t i, int dt) {
     if (dt == LLMK_F32) return ((const float*)p)[i];

@@ -98,6 +98,23 @@ __device__ __forceinline__ v4i w4_word_to_f16x8(unsigned w, v2h sc) {
     o[3] = (int)__builtin_amdgcn_perm(p37, p26, 0x07060302u);
     return o;
 }
+// The same for bf16, which has no packed arithmetic here: byte -> fp32 converts, one fma per weight ((q - 8) * scale is
+// exact in fp32: 15 significant bits) and one rounding to bf16, the value nk_dequant_bf16_kernel stores.
+__device__ __forceinline__ v4i w4_word_to_bf16x8(unsigned w, float sc) {
+    const unsigned even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+    const float c = -8.0f * sc;
+    v4i o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        o[i] = (int)pack_bf16x2(fmaf((float)((even >> (8 * i)) & 0xffu), sc, c), fmaf((float)((odd >> (8 * i)) & 0xffu), sc, c));
+    return o;
+}
+// one packed word and its group scale (fp16 bits) -> eight weights in the activation type of the kind
+template <int KIND>
+__device__ __forceinline__ v4i w4_word_x8(unsigned w, unsigned s16) {
+    if constexpr (KIND == K_W4NKB) return w4_word_to_bf16x8(w, f16_to_f32((unsigned short)s16));
+    else return w4_word_to_f16x8(w, w4_as_h2(s16 | (s16 << 16)));
+}
 // ---- uint4 weights packed eight rows per word, dequantised to int8 (K_W4A8) ----
 // A word holds the nibbles of eight weight rows at one k.  b8 = int8(int8(q - z) * s) with two's-complement wrap is
 // the low byte of (q - z) * s in any wider arithmetic, i.e. of q * s + c with c = -(z * s): one packed 16-bit
@@ -226,7 +243,7 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
     // SCALED: 8-bit operands with per-128-K block scales.  Otherwise no scales inside the K loop (fp16 / bf16
     // operands, or int8 with per-token and per-channel scales applied in the epilogue): a K step is still
     // one 128-byte row segment (two MFMAs per tile) and the MFMAs accumulate directly.
-    // K_W4NK: fp16 activations by direct-to-LDS loads as for K_F16; the weight rows of a stage are expanded
+    // K_W4NK(B): fp16 (bf16) activations by direct-to-LDS loads as for K_F16 (K_BF16); the weight rows of a stage are expanded
     // from the packed words by the threads themselves (one 8-byte load, 16 weights, two 16-byte LDS writes per
     // thread and K step), one K step behind the loads and one ahead of the multiplication.
     constexpr bool SCALED = (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_W4A8);
@@ -236,9 +253,9 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
     // from words that pack eight rows each: a thread loads four consecutive words of one packed row (16 bytes)
     // and writes four int8 weights of each of the eight rows; the zero points and second-level scales of the
     // tile's 128 rows for every K step sit in an LDS table filled before the pipeline starts.
-    constexpr bool W4NK = (KIND == K_W4NK), W4M = (KIND == K_W4MARLIN), W4A8 = (KIND == K_W4A8);
+    constexpr bool W4NK = is_w4nk(KIND), W4M = (KIND == K_W4MARLIN), W4A8 = (KIND == K_W4A8);
     constexpr bool W4H = W4NK || W4M, W4 = W4H || W4A8;
-    constexpr int ESZ = (KIND == K_F16 || KIND == K_BF16 || W4H) ? 2 : 1;
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
     const int N = p.N;
     const int K = p.K * ESZ;                 // row length in bytes
     const int KT_all = K >> 7;
@@ -414,11 +431,9 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
             }
         }
         if constexpr (W4NK) {
-            const unsigned s16 = w4_scale16;
-            const v2h sc = w4_as_h2(s16 | (s16 << 16));
             uint8_t* dst = lds + (kt % D_NSTAGE) * D_STAGE + D_A + w4_lds;
-            *(v4i*)dst = w4_word_to_f16x8((unsigned)w4_words, sc);
-            *(v4i*)(dst + ((w4_lds & 16u) ? -16 : 16)) = w4_word_to_f16x8((unsigned)(w4_words >> 32), sc);
+            *(v4i*)dst = w4_word_x8<KIND>((unsigned)w4_words, w4_scale16);
+            *(v4i*)(dst + ((w4_lds & 16u) ? -16 : 16)) = w4_word_x8<KIND>((unsigned)(w4_words >> 32), w4_scale16);
         }
         if constexpr (W4M) {
             const v2h k1032 = {(_Float16)1032.f, (_Float16)1032.f};

@@ -331,15 +331,15 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
     static_assert(WIDE ? (MT == 8 || MT == 4) : (MT == 4 || MT == 2), "tile rows");
     constexpr int BN = mdp_bn(WIDE), NSUB = mdp_nsub(WIDE), RED_ROW = BN + 4;
     static_assert(BN * NSUB * 128 == MD_B && RED_ROW == (WIDE ? 132 : MD_RED_ROW), "weight stage of 32 KB");
-    static_assert(KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL || KIND == K_F16 || KIND == K_BF16 || KIND == K_W4NK,
+    static_assert(KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL || KIND == K_F16 || KIND == K_BF16 || is_w4nk(KIND),
                   "8- and 16-bit operands, or fp16 activations with row-packed 4-bit weights");
     constexpr int BM = 16 * MT;
     // K_W4NK: the producers load packed words [N, K/8] and their group scales (fp16, groups of 64 * 2^j elements) and write
     // fp16 weight rows (q - 8) * scale into the weight stage; the rest is the fp16 kind
-    constexpr bool W4NK = (KIND == K_W4NK);
+    constexpr bool W4NK = is_w4nk(KIND);
     constexpr bool SCALED = (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK);
     constexpr bool ROWCOL = (KIND == K_I8_ROWCOL);
-    constexpr int ESZ = (KIND == K_F16 || KIND == K_BF16 || W4NK) ? 2 : 1;
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
     constexpr int MD_A = mdp_a(MT, WIDE), STAGE = mdp_stage(MT, WIDE);
     constexpr int RB = MDP_RB;
     constexpr int NPA = 2 * MT * NSUB / 4;                  // activation pieces per producer wave and step
@@ -455,9 +455,8 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
             if constexpr (W4NK) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const v2h sc = w4_as_h2(rsc[i] | (rsc[i] << 16));
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) *(v4i*)(st + blds[i] + (w4_chunk[i] ^ (uint32_t)(c * 16))) = w4_word_to_f16x8((unsigned)rs[i][c], sc);
+                    for (int c = 0; c < 4; ++c) *(v4i*)(st + blds[i] + (w4_chunk[i] ^ (uint32_t)(c * 16))) = w4_word_x8<KIND>((unsigned)rs[i][c], rsc[i]);
                 }
             } else {
 #pragma unroll
@@ -674,9 +673,9 @@ inline MidPlan midw_plan(int64_t M, int64_t N, int64_t kbytes) {
 // K_W4A8 kind room for its table behind the stages.
 template <int KIND>
 inline bool mid_eligible(const DirectArgs& p, int mt, int ksplit) {
-    constexpr int ESZ = (KIND == K_F16 || KIND == K_BF16 || KIND == K_W4NK) ? 2 : 1;
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
     if (!dma_eligible(p, ESZ)) return false;
-    if (KIND == K_W4NK && (p.group < 64 || (p.group & (p.group - 1)))) return false;      // groups of 64 * 2^j elements
+    if (is_w4nk(KIND) && (p.group < 64 || (p.group & (p.group - 1)))) return false;      // groups of 64 * 2^j elements
     const int KT_all = (p.K * ESZ) >> 7;
     const int per = ksplit > 1 ? ((((KT_all + ksplit - 1) / ksplit) + 3) & ~3) : KT_all;
     return md_lds(mt, KIND == K_W4A8 ? per : 0) <= D_LDS_MAX;
@@ -694,7 +693,7 @@ int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
         if constexpr (W4) return gemm_mid_kernel<KIND, MT, AS16>;
         else return gemm_mid_pc_kernel<KIND, MT, AS16, WIDE>;
     }();
-    constexpr int ESZ = (KIND == K_F16 || KIND == K_BF16 || KIND == K_W4NK) ? 2 : 1;
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
     const int KT_all = (p.K * ESZ) >> 7;
     const bool split = p.ksplit > 1 && p.partial;
     const int per = split ? ((((KT_all + p.ksplit - 1) / p.ksplit) + 3) & ~3) : KT_all;

@@ -848,17 +848,64 @@ int launch_nk_stream(const _Float16* A, const int32_t* B, const _Float16* S, _Fl
 // weight matrix is large, where the tile kernel with split-K beats the weight-streaming kernels (which read
 // the activations once per 16 columns), provided the scratch for its partial sums is there.
 // `wide`: the layout also has the expansion inside the 256-column tile kernel (row-packed layout only).  Up to 512
-// rows the fused tile kernels win everywhere (1.3-2.8x); beyond that the fused 256 x 256 kernel wins over the
-// dequantisation pass + fp16 GEMM only when the problem takes two or more rounds of 256 tiles (4096 x 28672 x 4096:
-// 741 vs 758 us, 2048 x 14336 x 4096: 198 vs 201 us), and loses on one round (4096^3: 109 vs 105 us).
-bool w4_tiles_expand(int64_t M, int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes, bool wide = false) {
-    if (M > 512) return wide && ((M + 255) / 256) * ((N + 255) / 256) >= 512;
+// rows the fused tile kernels win everywhere (1.3-2.8x).  Up to 1024 rows, where the separate pass is a good part of the
+// call, by the estimates of the tile shapes (1.65 x for 16-bit operands) against that pass, N * 1.86e-3 us at K = 4096 (2.5
+// bytes per weight at 5.5 TB/s), and the plain 16-bit GEMM: bf16 600 x 28672 x 4096 242 us in two passes, 192 fused, 1024 x
+// 14336 x 4096 122 and 105.  Beyond, every row tile expands the weights again and the fused form needs two rounds of
+// 256 x 256 tiles to win (fp16 4096 x 28672 x 4096: 741 vs 758 us, 2048 x 14336 x 4096: 198 vs 201; on one round 1300 x 6144
+// x 4096: 119 vs 86), the dearer bf16 expansion at most 2048 rows as well (1500 x 28672 x 4096: 319 vs 344, 4096 rows: 775 vs 762).
+bool w4_tiles_expand(int64_t M, int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes, bool wide = false, bool bf = false) {
+    if (M > 512) {
+        if (!wide) return false;
+        if (M > 1024) return ((M + 255) / 256) * ((N + 255) / 256) >= 512 && (!bf || M <= 2048);
+        llmk::DirectArgs p{};
+        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
+        const double fused = bf ? llmk::dma_tile_estimate<llmk::K_W4NKB, false>(p).cost : llmk::dma_tile_estimate<llmk::K_W4NK, false>(p).cost;
+        return 1.65 * fused < 1.65 * llmk::dma_tile_estimate<llmk::K_F16, false>(p).cost + (double)N * 1.86e-3;
+    }
     if (M > 64) return true;
     if (M <= 32 || K % 64) return false;
     const int64_t nk = N * K;
     if (!(K > 4096 ? nk >= ((int64_t)32 << 20) : nk >= ((int64_t)96 << 20))) return false;
     const int z = llmk::splitk_factor_half(M, N, K);
     return z <= 1 || (workspace && workspace_bytes >= (int64_t)z * M * N * 4 && !((uintptr_t)workspace & 15));
+}
+
+// Mid-size M (and large M on many tiles): the tile kernels expand the row-packed words themselves, so every weight byte is
+// read once; the separate expansion pass would write and re-read four times as much (bf16, 300 x 14336 x 4096: 26 us of
+// pass and 51 us of GEMM, 58 us in one kernel).  false: not a shape for them.
+template <int KIND>
+bool launch_nk_tiles(const void* a, const int32_t* b_packed, void* c, const void* s, int dtype, int64_t M, int64_t N, int64_t K,
+                     int groupsize, void* workspace, int64_t workspace_bytes, hipStream_t st, int& rc) {
+    llmk::DirectArgs p{};
+    p.a = (const uint8_t*)a; p.b = (const uint8_t*)b_packed; p.b_s = s; p.c = c; p.c_dtype = dtype;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = groupsize;
+    auto slices = [&](llmk::MidPlan& pl) {
+        if (pl.z > 1 && !(workspace && workspace_bytes >= (int64_t)pl.z * M * N * 4 && !((uintptr_t)workspace & 15))) pl.z = 1;
+    };
+    auto take = [&](const llmk::MidPlan& pl) { if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; } };
+    // few column tiles and short rows: the 64-column kernel with 512-byte K steps (128 x 4096 x 4096: 18.3 -> 14 us)
+    if (2 * K <= 8192 && llmk::mid_wanted(M, N, 2 * K)) {       // (rows beyond 8 KB: measured only for the 8-bit kinds)
+        llmk::MidPlan pl = llmk::mid_plan(M, N, 2 * K);
+        slices(pl);
+        if (llmk::mid_eligible<KIND>(p, pl.mt, pl.z)) {
+            take(pl);
+            rc = pl.mt == 4 ? llmk::launch_mid<KIND, 4>(p, st, "gemm_w4a16_nk(mid)") : llmk::launch_mid<KIND, 2>(p, st, "gemm_w4a16_nk(mid)");
+            return true;
+        }
+    }
+    if (!llmk::dma_eligible(p, 2)) return false;
+    // wider weights on one round of 128-column tiles: the 128-column form of that kernel
+    if (2 * K <= 8192 && llmk::midw_wanted(M, N, 2 * K) && (groupsize & (groupsize - 1)) == 0) {       // (longer rows: measured for fp8 only)
+        llmk::MidPlan pl = llmk::midw_plan(M, N, 2 * K);
+        slices(pl);
+        take(pl);
+        rc = pl.mt == 4 ? llmk::launch_mid<KIND, 4, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)")
+                        : llmk::launch_mid<KIND, 8, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)");
+        return true;
+    }
+    rc = llmk::launch_big_half<KIND, false>(p, st, "gemm_w4a16_nk(fused tiles)", workspace, workspace_bytes);
+    return true;
 }
 
 // launch shape of the Marlin-layout kernel for a given problem
@@ -999,32 +1046,11 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
                          (nz_bf == 1 || ((M * N) % 4 == 0 && workspace && workspace_bytes >= (int64_t)nz_bf * M * N * 4 &&
                                          !((uintptr_t)workspace & 15)));
     if (bf_ring) return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, nz_bf, (float*)workspace, true, st);
-    if (!bf && w4_tiles_expand(M, N, K, workspace, workspace_bytes, true) && K % 64 == 0 && groupsize % 64 == 0) {
-        // mid-size M: the 128-column tile kernels expand the packed words themselves (every weight byte is
-        // read once; the separate expansion pass would write and re-read four times as much).
-        llmk::DirectArgs p{};
-        p.a = (const uint8_t*)a; p.b = (const uint8_t*)b_packed; p.b_s = s; p.c = c; p.c_dtype = LLMK_F16;
-        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = groupsize;
-        // few column tiles and short rows: the 64-column kernel with 512-byte K steps (128 x 4096 x 4096: 18.3 -> 14 us)
-        if (2 * K <= 8192 && llmk::mid_wanted(M, N, 2 * K)) {       // (rows beyond 8 KB: measured only for the 8-bit kinds)
-            llmk::MidPlan pl = llmk::mid_plan(M, N, 2 * K);
-            if (pl.z > 1 && !(workspace && workspace_bytes >= (int64_t)pl.z * M * N * 4 && !((uintptr_t)workspace & 15))) pl.z = 1;
-            if (llmk::mid_eligible<llmk::K_W4NK>(p, pl.mt, pl.z)) {
-                if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; }
-                return pl.mt == 4 ? llmk::launch_mid<llmk::K_W4NK, 4>(p, st, "gemm_w4a16_nk(mid)")
-                                  : llmk::launch_mid<llmk::K_W4NK, 2>(p, st, "gemm_w4a16_nk(mid)");
-            }
-        }
-        // wider weights on one round of 128-column tiles: the 128-column form of that kernel
-        if (2 * K <= 8192 && llmk::midw_wanted(M, N, 2 * K) && llmk::dma_eligible(p, 2) && (groupsize & (groupsize - 1)) == 0) {       // (longer rows: measured for fp8 only)
-            llmk::MidPlan pl = llmk::midw_plan(M, N, 2 * K);
-            if (pl.z > 1 && !(workspace && workspace_bytes >= (int64_t)pl.z * M * N * 4 && !((uintptr_t)workspace & 15))) pl.z = 1;
-            if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; }
-            return pl.mt == 4 ? llmk::launch_mid<llmk::K_W4NK, 4, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)")
-                              : llmk::launch_mid<llmk::K_W4NK, 8, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)");
-        }
-        if (llmk::dma_eligible(p, 2))
-            return llmk::launch_big_half<llmk::K_W4NK, false>(p, st, "gemm_w4a16_nk(fused tiles)", workspace, workspace_bytes);
+    if (w4_tiles_expand(M, N, K, workspace, workspace_bytes, true, bf) && K % 64 == 0 && groupsize % 64 == 0) {
+        int rc = LLMK_OK;
+        const bool taken = bf ? launch_nk_tiles<llmk::K_W4NKB>(a, b_packed, c, s, ac_dtype, M, N, K, groupsize, workspace, workspace_bytes, st, rc)
+                              : launch_nk_tiles<llmk::K_W4NK>(a, b_packed, c, s, ac_dtype, M, N, K, groupsize, workspace, workspace_bytes, st, rc);
+        if (taken) return rc;
     }
     if ((M > 64 || bf) && K % 64 == 0 && workspace && workspace_bytes >= N * K * 2 && !((uintptr_t)workspace & 15)) {
         // compute-bound: expand W once to fp16 / bf16 [N, K], then run the tiled MFMA GEMM on it

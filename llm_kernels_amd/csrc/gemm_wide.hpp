@@ -188,9 +188,9 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     constexpr bool SCALED = (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK);
     // 4-bit weights (fp16 activations): the weight rows of a stage are not loaded into LDS but expanded there by
     // the threads themselves from packed words that travel HBM -> registers, see w4_request / w4_expand
-    constexpr bool W4NK = (KIND == K_W4NK), W4 = W4NK;
-    static_assert(KIND != K_W4MARLIN && KIND != K_W4A8 && !(W4 && GROUPED), "4-bit weights: row-packed fp16 layout, dense launches only");
-    constexpr int ESZ = (KIND == K_F16 || KIND == K_BF16 || W4) ? 2 : 1;
+    constexpr bool W4NK = is_w4nk(KIND), W4 = W4NK;
+    static_assert(KIND != K_W4MARLIN && KIND != K_W4A8 && !(W4 && GROUPED), "4-bit weights: row-packed layout, dense launches only");
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
     const int N = p.N;
     const int K = p.K * ESZ;                 // row length in bytes
     const int KT_all = K >> 7;
@@ -307,11 +307,9 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
         uint8_t* bst = lds + (kt & 1) * W_STAGE + W_A;
         const int h = piece >> 1, jj = piece & 1;
         if constexpr (W4NK) {
-            const unsigned s16 = w4_scale16[h];
-            const v2h sc = w4_as_h2(s16 | (s16 << 16));
             uint8_t* dst = bst + w4_lds[h];
-            if (jj == 0) *(v4i*)dst = w4_word_to_f16x8((unsigned)w4_words[h], sc);
-            else *(v4i*)(dst + ((w4_lds[h] & 16u) ? -16 : 16)) = w4_word_to_f16x8((unsigned)(w4_words[h] >> 32), sc);
+            if (jj == 0) *(v4i*)dst = w4_word_x8<KIND>((unsigned)w4_words[h], w4_scale16[h]);
+            else *(v4i*)(dst + ((w4_lds[h] & 16u) ? -16 : 16)) = w4_word_x8<KIND>((unsigned)(w4_words[h] >> 32), w4_scale16[h]);
         }
     };
     auto w4_expand = [&](int kt) {
@@ -698,7 +696,7 @@ int launch_wide(const DirectArgs& p0, hipStream_t stream, const char* name, void
     static std::atomic<uint64_t> configured{0};
     auto kern = gemm_wide_kernel<KIND, GROUPED, R>;
     constexpr int W_BM = w_bm(R), W_LDS = w_lds(R);
-    constexpr int ESZ = (KIND == K_F16 || KIND == K_BF16 || KIND == K_W4NK) ? 2 : 1;
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
     if (int rc = llmk_reserve_lds((const void*)kern, W_LDS, configured, name)) return rc;
     DirectArgs p = p0;
     const int tiles_m = GROUPED ? grouped_row_tiles(p.M, p.E, W_BM) : (p.M + W_BM - 1) / W_BM;
@@ -791,40 +789,47 @@ inline bool mid_m_prefers_tiles(int64_t M, int64_t N, int64_t K) {
 // Tile shape by estimated time: rounds of 256 workgroups times the measured cost of one round of each tile
 // shape (60 / 36 / 43 / 26 / 16 microseconds for 256 x 256, 128 x 256, 256 x 128, 128 x 128 and 64 x 128 at K = 4096
 // for fp8; the ratios hold for the other kinds and K).  Ties go to the larger tile (less operand re-reading).  Segments of a grouped GEMM are judged by their average length.
-// which tile shape the estimate picks: 8 / 9 = the 256 x 256 / 128 x 256 tile of gemm_wide_kernel, 4 / 2 / 1 = MI of gemm_dma_kernel
+// A workgroup that expands 4-bit weights expands its columns whatever its rows, which a lower tile hides less:
+// 65 / 42 / 43 for fp16, 65 / 46 / 43 for bf16 (one more instruction per weight) on the first three.
+// choice: 8 / 9 = the 256 x 256 / 128 x 256 tile of gemm_wide_kernel, 4 / 2 / 1 = MI of gemm_dma_kernel; cost: the estimate
+struct TileChoice {
+    int choice;
+    double cost;
+};
 template <int KIND, bool GROUPED>
-int dma_tile_choice(const DirectArgs& p) {
+TileChoice dma_tile_estimate(const DirectArgs& p) {
     // 4-bit weights: the row-packed layout, dense launches (the Marlin scatter of 2-byte pieces measured 4-9 % slower
     // inside the 256-column kernel than the dequantisation pass at every M > 512)
-    constexpr bool HAS_WIDE = KIND != K_W4MARLIN && KIND != K_W4A8 && !(GROUPED && KIND == K_W4NK);
+    constexpr bool HAS_WIDE = KIND != K_W4MARLIN && KIND != K_W4A8 && !(GROUPED && is_w4nk(KIND));
+    constexpr double WIDE = is_w4nk(KIND) ? 65.0 : 60.0, HALF = KIND == K_W4NK ? 42.0 : (KIND == K_W4NKB ? 46.0 : 36.0);
     const int64_t rows = GROUPED ? p.M / (p.E > 0 ? p.E : 1) : p.M;
     const int64_t groups = GROUPED ? p.E : 1;
     // a segment of a grouped GEMM rarely ends on a tile boundary: count one ragged tile per segment on top of
     // the full ones (with the plain ceiling, segments of 128 +- a few rows looked like one 128-row tile each and
     // went to a tile shape that needed two; -8 % on the Mixtral forward at 256 and 512 tokens)
     auto rounds = [&](int bm, int bn) { return (((p.N + bn - 1) / bn) * groups * (GROUPED ? rows / bm + 1 : (rows + bm - 1) / bm) + LLMK_CUS - 1) / LLMK_CUS; };
-    const double t_wide = 60.0 * rounds(256, 256), t4 = 43.0 * rounds(256, 128), t2 = 26.0 * rounds(128, 128),
+    const double t_wide = WIDE * rounds(256, 256), t_half = HALF * rounds(128, 256), t4 = 43.0 * rounds(256, 128), t2 = 26.0 * rounds(128, 128),
                  t1 = 16.0 * rounds(64, 128);
     if constexpr (HAS_WIDE) {
         if (t_wide <= t4 && t_wide <= t2 && t_wide <= t1) {
             // problems whose 256 x 256 tiles do not fill a round: the 128 x 256 tile of the same kernel
             // (a tie goes to the 128-row tile for block-scaled int8, whose per-step conversions leave the tall
             // tile less of its advantage: grouped Mixtral down projection -3 %; +1 % for fp8)
-            const double t_half = 36.0 * rounds(128, 256);
-            if (t_half < t_wide || (KIND == K_I8_BLOCK && GROUPED && t_half == t_wide)) return 9;
-            return 8;
+            if (t_half < t_wide || (KIND == K_I8_BLOCK && GROUPED && t_half == t_wide)) return {9, t_half};
+            return {8, t_wide};
         }
-        const double t_half = 36.0 * rounds(128, 256);
-        if (t_half < t4 && t_half <= t2 && t_half <= t1) return 9;
+        if (t_half < t4 && t_half <= t2 && t_half <= t1) return {9, t_half};
     }
     int max_mi = 4;
     if constexpr (KIND == K_W4A8) max_mi = w4a8_max_mi(p);       // the table of zero points and scales must fit behind the stages
     if constexpr (KIND != K_W4A8) {
-        if (t4 <= t2 && t4 <= t1 && max_mi >= 4) return 4;
+        if (t4 <= t2 && t4 <= t1 && max_mi >= 4) return {4, t4};
     }
-    if (t2 <= t1 && max_mi >= 2) return 2;
-    return 1;
+    if (t2 <= t1 && max_mi >= 2) return {2, t2};
+    return {1, t1};
 }
+template <int KIND, bool GROUPED>
+int dma_tile_choice(const DirectArgs& p) { return dma_tile_estimate<KIND, GROUPED>(p).choice; }
 
 // AS16 (16-bit activation scales staged as they are): the 64- and 128-row tiles of gemm_dma_kernel only, see launch_big
 template <int KIND, bool GROUPED, bool AS16 = false>
@@ -832,7 +837,7 @@ int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* 
     if (!GROUPED && p.ksplit > 1) return launch_dma_mi<KIND, GROUPED, 1, AS16>(p, stream, name);
     const int choice = dma_tile_choice<KIND, GROUPED>(p);
     if constexpr (!AS16) {
-        if constexpr (KIND != K_W4MARLIN && KIND != K_W4A8 && !(GROUPED && KIND == K_W4NK)) {
+        if constexpr (KIND != K_W4MARLIN && KIND != K_W4A8 && !(GROUPED && is_w4nk(KIND))) {
             if (choice == 9) return launch_wide<KIND, GROUPED, 4>(p, stream, name, ws, ws_bytes);
             if (choice == 8) return launch_wide<KIND, GROUPED, 8>(p, stream, name, ws, ws_bytes);
         }

@@ -307,3 +307,26 @@ def test_w4a16_nk_bf16_decode_is_exact_for_small_integers(dev):
     y = w4a16.w4a16_gemm(x.bfloat16().to(dev), torch.from_numpy(packed).to(dev), s.to(dev), 128)
     ref = x.double() @ (qn.double() - 8).T
     assert torch.equal(y.cpu().double(), ref.bfloat16().double())
+
+
+@pytest.mark.parametrize("M,N,K,gs", [(65, 72, 128, 64), (130, 4096, 1024, 128), (512, 264, 4096, 128), (300, 14344, 512, 128),
+                                      (200, 20000, 640, 128), (500, 8192, 384, 192), (600, 10000, 1024, 128), (1024, 28672, 256, 128)])
+def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
+    """bf16 on the tile kernels that expand the words: both column widths, K slices, groups that are no power of two, the
+    256-column tiles, ragged rows and columns; single weights exactly (one activation per row, no sum to round)."""
+    announce("w4a16 nk bf16 tiles", M, N, K, gs)
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K).bfloat16()
+    qn, s = q.w4a16_quant_nk(torch.randn(N, K) * 0.02, gs)
+    packed, s = torch.from_numpy(bp.pack_cols(qn.numpy(), 4, 32)[0]).to(dev), s.to(dev)
+    y = w4a16.w4a16_gemm(x.to(dev), packed, s, gs)
+    deq = (qn.double() - 8) * s.cpu().double().repeat_interleave(gs, 1)
+    # the weights this path multiplies are (q - 8) * s rounded to bf16: against those only the output's rounding (2^-9 of
+    # it) and fp32 sums are left.  Against unrounded weights every product is off by up to 2^-9 too, and of 29 M sums of
+    # 256 such errors (0.0011 of the output scale each) three lie nine deviations out, at the 1e-2 bound.
+    assert_close_scaled(y, x.double() @ deq.bfloat16().double().T, rtol=2 ** -8, atol=1e-4, what="w4a16 nk bf16 tiles")
+    one = torch.zeros(M, K)
+    k = torch.randint(0, K, (M,))
+    one[torch.arange(M), k] = 1.0
+    y = w4a16.w4a16_gemm(one.bfloat16().to(dev), packed, s, gs)
+    assert torch.equal(y.cpu(), deq.bfloat16().T[k])
