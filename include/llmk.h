@@ -221,6 +221,14 @@ int llmk_moe_src2dst(const int64_t* reorder_ids, int32_t* src2dst, int64_t num_t
 #define LLMK_MOE_PREPROCESS_MAX_IDS 32768
 int llmk_moe_ep_preprocess(const void* topk_ids, int ids_bytes, int64_t num_toks, int num_experts,
                            void* sorted_ids, int32_t* src2dst, int64_t* seg_indptr, void* stream);
+/* Router of a softmax top-k expert layer: p = softmax(logits[t, :E]) in fp32, the topk largest in descending order (equal
+ * values: lower index first, NaN largest as torch.topk ranks it), ids int64 and weights fp32 [T, topk], the weights divided
+ * by their sum when renormalize is set.  E and topk up to LLMK_ROUTER_MAX_EXPERTS / LLMK_ROUTER_MAX_TOPK.
+ * ref: the routing in front of moe/sglang_moe_all_gather_all_reduce.py:267-312 (there a gate module of torch calls). */
+#define LLMK_ROUTER_MAX_EXPERTS 512
+#define LLMK_ROUTER_MAX_TOPK 64
+int llmk_moe_softmax_topk(const void* logits, int dtype, int64_t* ids, float* weights, int64_t T, int E, int topk,
+                          int renormalize, void* stream);
 /* ids_bytes: 4 or 8 (topk_ids int32 / int64).  a1_scales may be NULL (fp32 per expert). */
 int llmk_moe_pre_reorder(const void* x, int x_dtype, void* out, int out_dtype, const int32_t* src2dst,
                          const void* topk_ids, int ids_bytes, const float* a1_scales,

@@ -25,7 +25,7 @@ namespace {
     X(llmk_gemm_w4a8_workspace_bytes) X(llmk_gemm_w4a16_marlin) X(llmk_gemm_w4a16_marlin_workspace_bytes)             \
     X(llmk_gemm_w4a16_nk) X(llmk_moe_ep_preprocess) X(llmk_moe_pre_reorder_quant) X(llmk_moe_act_and_mul_quant)       \
     X(llmk_moe_post_reorder) X(llmk_grouped_gemm) X(llmk_grouped_gemm_swiglu_quant)                                   \
-    X(llmk_grouped_gemm_swiglu_quant_fused)
+    X(llmk_grouped_gemm_swiglu_quant_fused) X(llmk_moe_softmax_topk)
 
 // one per imported module object: the package and the top-level module layout may both be imported
 struct State {
@@ -325,6 +325,16 @@ PyObject* marlin_mul(const Args& g) {
 }
 
 // ------------------------------------------------------------------ mixture of experts
+// softmax_topk(logits [.., E], topk, renormalize) -> (ids int64, weights fp32)
+PyObject* softmax_topk(const Args& g) {
+    const at::Tensor x = g.tensor(0).contiguous();
+    const int64_t topk = g.integer(1), E = last_size(x), T = rows_of(x, E);
+    at::Tensor ids = empty(with_last(x, topk), at::kLong, x), w = empty(with_last(x, topk), at::kFloat, x);
+    g.check(g.st->llmk_moe_softmax_topk(x.data_ptr(), float_code(x.scalar_type()), (int64_t*)ids.data_ptr(), (float*)w.data_ptr(), T, (int)E, (int)topk, g.integer(2) != 0, stream_of(x)),
+            "llmk_moe_softmax_topk");
+    return wrap_all(std::move(ids), std::move(w));
+}
+
 // ep_preprocess(topk_ids, num_experts) -> (sorted ids, src2dst, seg_indptr); contiguous int32 / int64 ids within the limits
 PyObject* ep_preprocess(const Args& g) {
     const at::Tensor& ids = g.tensor(0);
@@ -491,7 +501,7 @@ PyObject* call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
-    FN(act_quant, 3), FN(rowwise_quant, 1), FN(fp8_gemm, 4), FN(int8_gemm, 4), FN(int8_gemm_per_token, 5), FN(w4a8_gemm, 7),
+    FN(act_quant, 3), FN(rowwise_quant, 1), FN(softmax_topk, 3), FN(fp8_gemm, 4), FN(int8_gemm, 4), FN(int8_gemm_per_token, 5), FN(w4a8_gemm, 7),
     FN(w4a16_gemm, 4), FN(marlin_mul, 4), FN(ep_preprocess, 2), FN(pre_reorder_quant, 9), FN(act_and_mul_quant, 8),
     FN(post_reorder, 9), FN(grouped_gemm, 8), FN(swiglu_fused, 3), FN(swiglu_quant, 9),
     {nullptr, nullptr, 0, nullptr}};

@@ -34,60 +34,66 @@ __device__ __forceinline__ int64_t ld_id(const void* p, int64_t i, int bytes) {
 // map as by-products: what torch.sort(stable) + seg_indptr_kernel + src2dst_kernel produce in eight launches.
 // Bucket 0 takes negative ids, bucket e + 1 expert e, bucket E + 1 ids >= E (both out-of-range buckets keep
 // their arrival order; a well-formed input leaves them empty).
-// Workgroup g places the ids [1024 g, 1024 g + 1024).  It counts, per bucket, all ids (-> bucket starts) and
+// Workgroup g places the ids [g THREADS, (g + 1) THREADS).  It counts, per bucket, all ids (-> bucket starts) and
 // the ids in front of its chunk, by reading the whole id list (at most PP_MAX_IDS ids, from L2); a lane's
 // position is then bucket start + ids of the bucket in earlier chunks + those in the lower waves of the
 // chunk + its rank among the equal ids of its own wave.  No workgroup waits for another.
-constexpr int PP_THREADS = 1024, PP_WAVES = PP_THREADS / 64, PP_MAX_EXPERTS = 512, PP_BUCKETS = PP_MAX_EXPERTS + 2;
+// Bound by latency: a chain of one load, three barriers and a scan.  Few buckets are counted in 64 columns per bucket, one
+// per lane, so that the ids of a wave never meet on one LDS address (ballots per bucket, the form before, took
+// 12.2 us for 8192 ids of 8 experts, this one 8.9); 65 to 256 ids get a workgroup of 256.
+constexpr int PP_THREADS = 1024, PP_MAX_EXPERTS = 512, PP_BUCKETS = PP_MAX_EXPERTS + 2, PP_FEW = 66;
 
-__global__ __launch_bounds__(PP_THREADS) void ep_preprocess_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
-                                                                   void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
-                                                                   int64_t* __restrict__ seg_indptr) {
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
+                                                                void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
+                                                                int64_t* __restrict__ seg_indptr) {
+    constexpr int WAVES = THREADS / 64;
     __shared__ int tot[PP_BUCKETS];      // ids per bucket, then the bucket's first position
     __shared__ int pre[PP_BUCKETS];      // ids per bucket in front of this workgroup's chunk
-    __shared__ int wcount[PP_WAVES][PP_BUCKETS];
+    // either the columns of a few buckets (two counts per cell: ids in front of the chunk in the low half, the others in
+    // the high half; at most PP_MAX_IDS / 64 ids a column) or nothing; afterwards the counts per wave
+    constexpr int CELLS = PP_FEW * 64, WCELLS = WAVES * PP_BUCKETS;
+    __shared__ int cells[CELLS > WCELLS ? CELLS : WCELLS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = E + 2;
-    const int c0 = blockIdx.x * PP_THREADS;
+    const int c0 = blockIdx.x * THREADS;
     auto bucket_at = [&](int i) {
         if (i >= n) return -1;
         const int64_t id = ld_id(ids, i, ids_bytes);
         return id < 0 ? 0 : (id >= E ? E + 1 : (int)id + 1);
     };
-    for (int b = tid; b < nb; b += PP_THREADS) { tot[b] = 0; pre[b] = 0; }
-    for (int i = tid; i < PP_WAVES * nb; i += PP_THREADS) wcount[i / nb][i % nb] = 0;
+    const int b = bucket_at(c0 + tid);   // the id this thread places: requested before anything else
+    const bool few = nb <= PP_FEW;
+    for (int k = tid; k < nb; k += THREADS) { tot[k] = 0; pre[k] = 0; }
+    if (few) for (int i = tid; i < nb * 64; i += THREADS) cells[i] = 0;
     __syncthreads();
     constexpr int U = 4;                 // rounds whose loads are in flight together
-    if (nb <= 64) {
-        // few buckets: lane k of every wave counts bucket k from ballots (one LDS atomic per id would
-        // serialise on the few addresses)
-        int acc_t = 0, acc_p = 0;
-        for (int r0 = 0; r0 < n; r0 += U * PP_THREADS) {
-            int b[U];
+    for (int r0 = 0; r0 < n; r0 += U * THREADS) {
+        int v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) b[u] = bucket_at(r0 + u * PP_THREADS + tid);
+        for (int u = 0; u < U; ++u) v[u] = bucket_at(r0 + u * THREADS + tid);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool before = r0 + u * PP_THREADS < c0;        // whole rounds lie in front of the chunk or not
-                for (int k = 0; k < nb; ++k) {
-                    const int c = __popcll(__ballot(b[u] == k));
-                    if (lane == k) { acc_t += c; if (before) acc_p += c; }
-                }
-            }
-        }
-        if (lane < nb) { atomicAdd(&tot[lane], acc_t); atomicAdd(&pre[lane], acc_p); }
-    } else {
-        for (int r0 = 0; r0 < n; r0 += U * PP_THREADS) {
-            int b[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) b[u] = bucket_at(r0 + u * PP_THREADS + tid);
-#pragma unroll
-            for (int u = 0; u < U; ++u) if (b[u] >= 0) {
-                atomicAdd(&tot[b[u]], 1);
-                if (r0 + u * PP_THREADS < c0) atomicAdd(&pre[b[u]], 1);
+        for (int u = 0; u < U; ++u) if (v[u] >= 0) {
+            const bool before = r0 + u * THREADS < c0;           // whole rounds lie in front of the chunk or not
+            if (few) {
+                atomicAdd(&cells[v[u] * 64 + lane], before ? 1 : 1 << 16);
+            } else {
+                atomicAdd(&tot[v[u]], 1);
+                if (before) atomicAdd(&pre[v[u]], 1);
             }
         }
     }
     __syncthreads();
+    if (few) {
+        for (int k = wave; k < nb; k += WAVES) {
+            const int c = cells[k * 64 + lane];
+            int lo = c & 0xffff, all = lo + (c >> 16);
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) { lo += __shfl_xor(lo, o, 64); all += __shfl_xor(all, o, 64); }
+            if (lane == 0) { pre[k] = lo; tot[k] = all; }
+        }
+        __syncthreads();
+    }
+    for (int i = tid; i < WAVES * nb; i += THREADS) cells[i] = 0;
     if (wave == 0) {
         // exclusive scan of the bucket counts: a run of buckets per lane, then a scan over the lanes
         const int per = (nb + 63) / 64, b0 = lane * per;
@@ -109,11 +115,9 @@ __global__ __launch_bounds__(PP_THREADS) void ep_preprocess_kernel(const void* _
     __syncthreads();
     // seg_indptr[e + 1] = number of ids <= e = start of bucket e + 2; seg_indptr[0] = 0
     if (blockIdx.x == 0)
-        for (int e = tid; e <= E; e += PP_THREADS) seg_indptr[e] = e == 0 ? 0 : (int64_t)tot[e + 1];
+        for (int e = tid; e <= E; e += THREADS) seg_indptr[e] = e == 0 ? 0 : (int64_t)tot[e + 1];
 
     // rank of a lane among the lanes of its wave with the same bucket, one leader per bucket publishes the count
-    const int i = c0 + tid;
-    const int b = bucket_at(i);
     int rank = 0;
     uint64_t todo = __ballot(b >= 0);
     while (todo) {                                       // one pass per distinct bucket of the wave
@@ -122,17 +126,111 @@ __global__ __launch_bounds__(PP_THREADS) void ep_preprocess_kernel(const void* _
         const uint64_t m = __ballot(b == v);
         if (b == v) {
             rank = __popcll(m & ((1ull << lane) - 1ull));
-            if (lane == l) wcount[wave][b] = __popcll(m);
+            if (lane == l) cells[wave * nb + b] = __popcll(m);
         }
         todo &= ~m;
     }
-    __syncthreads();
+    if constexpr (WAVES > 1) __syncthreads();
     if (b >= 0) {
         int pos = tot[b] + pre[b] + rank;
-        for (int w = 0; w < wave; ++w) pos += wcount[w][b];
+        for (int w = 0; w < wave; ++w) pos += cells[w * nb + b];
+        const int i = c0 + tid;
         const int64_t id = (b >= 1 && b <= E) ? (int64_t)(b - 1) : ld_id(ids, i, ids_bytes);
         if (ids_bytes == 8) ((int64_t*)sorted_out)[pos] = id; else ((int32_t*)sorted_out)[pos] = (int32_t)id;
         src2dst[i] = pos;
+    }
+}
+
+// The same for at most 64 ids: one wave, a lane per id, no LDS.  Every lane counts the ids of lower buckets and the equal
+// ids of lower lanes, one pass per distinct bucket.  What such a launch costs behind a kernel that streamed the experts'
+// weights is fetching its code from memory again, so the code is short (32 ids, 8 experts: 5.4 us in the general form,
+// 2.0 here).
+__global__ __launch_bounds__(64) void ep_preprocess_wave_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
+                                                                void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
+                                                                int64_t* __restrict__ seg_indptr) {
+    const int lane = threadIdx.x;
+    const bool live = lane < n;
+    const int64_t id = live ? ld_id(ids, lane, ids_bytes) : 0;
+    const int b = !live ? E + 2 : (id < 0 ? 0 : (id >= E ? E + 1 : (int)id + 1));
+    int pos = 0;
+    for (int e0 = 0; e0 <= E; e0 += 64) {
+        int below = 0;                                   // ids of the buckets up to e0 + lane
+        uint64_t todo = __ballot(live);
+        while (todo) {
+            const int v = __builtin_amdgcn_readlane(b, __ffsll((unsigned long long)todo) - 1);
+            const uint64_t m = __ballot(b == v);
+            const int c = __popcll(m);
+            if (v <= e0 + lane) below += c;
+            if (e0 == 0) pos += v < b ? c : (v == b ? __popcll(m & ((1ull << lane) - 1ull)) : 0);
+            todo &= ~m;
+        }
+        const int e = e0 + lane;
+        if (e <= E) seg_indptr[e] = e == 0 ? 0 : below;
+    }
+    if (live) {
+        if (ids_bytes == 8) ((int64_t*)sorted_out)[pos] = id; else ((int32_t*)sorted_out)[pos] = (int32_t)id;
+        src2dst[lane] = pos;
+    }
+}
+
+// ---------------------------------------------------------------- softmax top-k router
+// L lanes own one token, V experts each (expert v * L + lane), topk <= L; a wave owns 64 / L tokens.  Bound by latency: a token is a few
+// dozen bytes, and what the launch costs is one dependent chain (load, max, sum, topk rounds of an arg-max over the lanes),
+// so everything stays in registers and lanes.  As five torch kernels the same routing took 31 us of GPU time for 16 tokens
+// and 43 us for 4096; one launch here takes 2.1 and 3.4 us.
+// A probability is ranked by its bit pattern (monotone for the non-negative values, a NaN above all of them), joined with
+// the complement of the index, so equal values go to the lower index and one 64-bit maximum decides a round.
+template <int DT, int L, int V>
+__global__ __launch_bounds__(256) void softmax_topk_kernel(const void* __restrict__ logits, int64_t* __restrict__ ids,
+                                                           float* __restrict__ wts, int64_t T, int E, int topk, bool renorm) {
+    const int64_t t = ((int64_t)blockIdx.x * 256 + threadIdx.x) / L;
+    const int lane = threadIdx.x & (L - 1);
+    const bool live = t < T;
+    float x[V];
+    float m = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int e = v * L + lane;
+        x[v] = (live && e < E) ? FloatIO<DT>::ld(logits, t * E + e) : -INFINITY;
+        m = fmaxf(m, x[v]);
+    }
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));      // (signed: group_max is for magnitudes)
+    float sum = 0.f;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int e = v * L + lane;
+        x[v] = e < E ? expf(x[v] - m) : 0.f;
+        sum += x[v];
+    }
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    uint64_t key[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int e = v * L + lane;
+        key[v] = e < E ? ((uint64_t)__float_as_uint(x[v] / sum) << 32) | (uint64_t)(0xffffffffu - (unsigned)e) : 0;
+    }
+    float total = 0.f, mine = 0.f;                       // lane k keeps the k-th weight (topk <= L)
+    unsigned mine_e = 0;
+    for (int k = 0; k < topk; ++k) {
+        uint64_t best = key[0];
+#pragma unroll
+        for (int v = 1; v < V; ++v) best = key[v] > best ? key[v] : best;
+#pragma unroll
+        for (int o = L / 2; o > 0; o >>= 1) {
+            const uint64_t other = __shfl_xor((unsigned long long)best, o, 64);
+            best = other > best ? other : best;
+        }
+        const float w = __uint_as_float((unsigned)(best >> 32));
+        total += w;
+        if (lane == k) { mine = w; mine_e = 0xffffffffu - (unsigned)best; }
+#pragma unroll
+        for (int v = 0; v < V; ++v) if (key[v] == best) key[v] = 0;
+    }
+    if (live && lane < topk) {
+        ids[t * topk + lane] = (int64_t)mine_e;
+        wts[t * topk + lane] = renorm ? mine / total : mine;
     }
 }
 
@@ -254,47 +352,47 @@ __global__ void act_mul_quant_kernel(const void* __restrict__ gateup, void* __re
 
 // Token permutation and 1 x 128 activation quantisation in one pass: a token's row is read once, quantised
 // (after the optional per-expert scale, rounded to the tensor dtype as the separate kernels do) and written
-// to the destination row of each of its local experts.
-constexpr int PRQ_UNROLL = 1;      // groups per thread of the fused permutation + quantisation kernel (2 and 4: no faster)
-
-template <int IDT, bool FP8>
+// to the destination row of each of its local experts.  Without per-expert scales the values are the same for
+// every expert and are quantised once (bound by HBM then: 4096 tokens x 2 experts x 4096 bf16 19.6 us; quantising per
+// expert took 25.8 us).
+template <int IDT, bool FP8, bool SCALED>
 __global__ void pre_reorder_quant_kernel(const void* __restrict__ x, void* __restrict__ q_out, void* __restrict__ s_out,
                                          const int32_t* __restrict__ src2dst, const void* __restrict__ topk_ids,
                                          int ids_bytes, const float* __restrict__ a1_scales, int start_e, int end_e,
                                          int topk, int64_t T, int64_t hidden, int mode) {
     const int64_t gpr = hidden / 128;
     const int sub = threadIdx.x & 15;
-    int64_t t[PRQ_UNROLL], gi[PRQ_UNROLL];
-    bool live[PRQ_UNROLL];
-    float v[PRQ_UNROLL][EPL];
+    const int64_t grp = (int64_t)blockIdx.x * (blockDim.x >> 4) + (threadIdx.x >> 4);
+    const bool live = grp < T * gpr;
+    const int64_t gs = live ? grp : 0;
+    const int64_t t = gs / gpr, gi = gs - t * gpr, col = gi * 128 + sub * EPL;
+    float v[EPL];
+    load8<IDT>(x, t * hidden + col, v);
+    float sc = 0.f;
+    uint2 w = make_uint2(0, 0);
+    if constexpr (!SCALED) {
+        float m = 0.f;
 #pragma unroll
-    for (int u = 0; u < PRQ_UNROLL; ++u) {
-        const int64_t grp = ((int64_t)blockIdx.x * PRQ_UNROLL + u) * (blockDim.x >> 4) + (threadIdx.x >> 4);
-        live[u] = grp < T * gpr;
-        const int64_t gs = live[u] ? grp : 0;
-        t[u] = gs / gpr;
-        gi[u] = gs - t[u] * gpr;
-        load8<IDT>(x, t[u] * hidden + gi[u] * 128 + sub * EPL, v[u]);
+        for (int k = 0; k < EPL; ++k) m = fmaxf(m, fabsf(v[k]));
+        w = quant8<FP8>(v, group_max<16>(m), mode, sc);
     }
-#pragma unroll
-    for (int u = 0; u < PRQ_UNROLL; ++u) {
-        const int64_t col = gi[u] * 128 + sub * EPL;
-        for (int j = 0; j < topk; ++j) {
-            const int64_t e = ld_id(topk_ids, t[u] * topk + j, ids_bytes);
-            const bool local = e >= start_e && e <= end_e;
-            const float scale = (a1_scales && local) ? 1.0f / a1_scales[e - start_e] : 1.0f;
-            float w[EPL];
+    for (int j = 0; j < topk; ++j) {
+        const int64_t e = ld_id(topk_ids, t * topk + j, ids_bytes);
+        const bool local = e >= start_e && e <= end_e;
+        if constexpr (SCALED) {
+            const float scale = local ? 1.0f / a1_scales[e - start_e] : 1.0f;
+            float u[EPL];
             float m = 0.f;
 #pragma unroll
             for (int k = 0; k < EPL; ++k) {
-                w[k] = rnd<IDT>(v[u][k] * scale);
-                m = fmaxf(m, fabsf(w[k]));
+                u[k] = rnd<IDT>(v[k] * scale);
+                m = fmaxf(m, fabsf(u[k]));
             }
-            m = group_max<16>(m);
-            if (!live[u] || !local) continue;
-            const int64_t dst = src2dst[t[u] * topk + j];
-            quant_store8<FP8>(w, m, q_out, dst * hidden + col, s_out, dst * gpr + gi[u], sub == 0, mode);
+            w = quant8<FP8>(u, group_max<16>(m), mode, sc);
         }
+        if (!live || !local) continue;
+        const int64_t dst = src2dst[t * topk + j];
+        store_quant8<FP8>(w, sc, q_out, dst * hidden + col, s_out, dst * gpr + gi, sub == 0);
     }
 }
 
@@ -410,9 +508,39 @@ extern "C" int llmk_moe_ep_preprocess(const void* topk_ids, int ids_bytes, int64
     if (!seg_indptr || (num_toks && (!topk_ids || !sorted_ids || !src2dst))) LLMK_FAIL(LLMK_ERR_ARG, "moe_ep_preprocess: null pointer");
     static_assert(LLMK_MOE_PREPROCESS_MAX_EXPERTS == PP_MAX_EXPERTS, "header limit and kernel table size differ");
     const unsigned grid = (unsigned)(num_toks > 0 ? cdiv64(num_toks, PP_THREADS) : 1);
-    ep_preprocess_kernel<<<grid, PP_THREADS, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
+    // one workgroup of the smallest size that holds the ids, chunks of PP_THREADS beyond
+    if (num_toks <= 64) ep_preprocess_wave_kernel<<<1, 64, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
+    else if (num_toks <= 256) ep_preprocess_kernel<256><<<1, 256, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
+    else ep_preprocess_kernel<PP_THREADS><<<grid, PP_THREADS, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
     LLMK_CHECK_LAUNCH("moe_ep_preprocess");
     return LLMK_OK;
+}
+
+template <int DT>
+static int launch_router(const void* logits, int64_t* ids, float* w, int64_t T, int E, int topk, bool renorm, hipStream_t st) {
+    // the narrowest group of lanes that holds a token's experts one each, then more experts per lane
+#define CALL(L, V) softmax_topk_kernel<DT, L, V><<<(unsigned)cdiv64(T * L, 256), 256, 0, st>>>(logits, ids, w, T, E, topk, renorm)
+    if (E <= 8) CALL(8, 1);
+    else if (E <= 16) CALL(16, 1);
+    else if (E <= 32) CALL(32, 1);
+    else if (E <= 64) CALL(64, 1);
+    else if (E <= 128) CALL(64, 2);
+    else if (E <= 256) CALL(64, 4);
+    else CALL(64, 8);
+#undef CALL
+    LLMK_CHECK_LAUNCH("moe_softmax_topk");
+    return LLMK_OK;
+}
+
+extern "C" int llmk_moe_softmax_topk(const void* logits, int dtype, int64_t* ids, float* weights, int64_t T, int E, int topk,
+                                     int renormalize, void* stream) {
+    if (T < 0 || E < 1 || topk < 1 || topk > E || E > LLMK_ROUTER_MAX_EXPERTS || topk > LLMK_ROUTER_MAX_TOPK || T > (1ll << 24))
+        LLMK_FAIL(LLMK_ERR_SHAPE, "moe_softmax_topk: T=%lld E=%d topk=%d", (long long)T, E, topk);
+    if (T == 0) return LLMK_OK;
+    if (!logits || !ids || !weights) LLMK_FAIL(LLMK_ERR_ARG, "moe_softmax_topk: null pointer");
+    int rc = LLMK_OK;
+    LLMK_DISPATCH_FLOAT(dtype, DT, rc = launch_router<DT>(logits, ids, weights, T, E, topk, renormalize != 0, (hipStream_t)stream));
+    return rc;
 }
 
 extern "C" int llmk_moe_pre_reorder(const void* x, int x_dtype, void* out, int out_dtype, const int32_t* src2dst,
@@ -485,11 +613,13 @@ extern "C" int llmk_moe_pre_reorder_quant(const void* x, int x_dtype, void* q_ou
     if (!x || !q_out || !s_out || !src2dst || !topk_ids) LLMK_FAIL(LLMK_ERR_ARG, "moe_pre_reorder_quant: null pointer");
     if (((uintptr_t)x | (uintptr_t)q_out) & 15) LLMK_FAIL(LLMK_ERR_ARG, "moe_pre_reorder_quant: buffers must be 16-byte aligned");
     const int64_t threads = T * (hidden / 128) * 16;
-    const unsigned grid = (unsigned)cdiv64(threads, 256 * PRQ_UNROLL);
+    const unsigned grid = (unsigned)cdiv64(threads, 256);
+#define CALL(FP8, SCALED) pre_reorder_quant_kernel<IDT, FP8, SCALED><<<grid, 256, 0, (hipStream_t)stream>>>(x, q_out, s_out, src2dst, topk_ids, ids_bytes, a1_scales, start_expert, end_expert, topk, T, hidden, round_mode)
     LLMK_DISPATCH_FLOAT(x_dtype, IDT, {
-        if (kind == LLMK_KIND_FP8) pre_reorder_quant_kernel<IDT, true><<<grid, 256, 0, (hipStream_t)stream>>>(x, q_out, s_out, src2dst, topk_ids, ids_bytes, a1_scales, start_expert, end_expert, topk, T, hidden, round_mode);
-        else pre_reorder_quant_kernel<IDT, false><<<grid, 256, 0, (hipStream_t)stream>>>(x, q_out, s_out, src2dst, topk_ids, ids_bytes, a1_scales, start_expert, end_expert, topk, T, hidden, round_mode);
+        if (kind == LLMK_KIND_FP8) { if (a1_scales) CALL(true, true); else CALL(true, false); }
+        else { if (a1_scales) CALL(false, true); else CALL(false, false); }
     });
+#undef CALL
     LLMK_CHECK_LAUNCH("moe_pre_reorder_quant");
     return LLMK_OK;
 }

@@ -218,8 +218,8 @@ __global__ void w4a8_level2_kernel(int8_t* __restrict__ y, int8_t* __restrict__ 
     float mx = v[0], mn = v[0];
 #pragma unroll
     for (int j = 1; j < EPL; ++j) { mx = fmaxf(mx, v[j]); mn = fminf(mn, v[j]); }
-    mx = group_max<LPG>(mx);
-    mn = group_min<LPG>(mn);
+    mx = (float)group_imax<LPG>((int)mx);
+    mn = (float)group_imin<LPG>((int)mn);
     if (!live) return;
     const float fs4 = floorf((mx - mn) / 15.0f + 0.5f);
     const float fz4 = floorf(-mn / fs4 + 0.5f);

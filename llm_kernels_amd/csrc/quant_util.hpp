@@ -55,19 +55,33 @@ __device__ __forceinline__ unsigned pack_fp8x4(float a, float b, float c, float 
     return (unsigned)w;
 }
 
-// group max over the LPG lanes that share a group (LPG power of two <= 64)
-template <int LPG>
-__device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-    for (int o = LPG / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+// the value of the lane that reduction step O of a group of lanes exchanges with: groups of up to 16 lanes are a DPP row,
+// where the exchange is an operand modifier of the reducing instruction; a shuffle through LDS costs an address, a trip of
+// about 60 cycles and a wait.  (Steps 4 and 8 mirror half a row and a row: the lanes of a group of 4, or 8, hold the same
+// value by then.)
+template <int O>
+__device__ __forceinline__ int lane_step(int v) {
+    if constexpr (O <= 8) {
+        constexpr int CTRL = O == 1 ? 0xB1 : (O == 2 ? 0x4E : (O == 4 ? 0x141 : 0x140));
+        return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+    } else {
+        return __shfl_xor(v, O, 64);
+    }
 }
-template <int LPG>
-__device__ __forceinline__ float group_min(float v) {
-#pragma unroll
-    for (int o = LPG / 2; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-    return v;
+template <int LPG, int O = 1>
+__device__ __forceinline__ int group_imax(int v) {
+    if constexpr (O < LPG) return group_imax<LPG, 2 * O>(max(v, lane_step<O>(v)));
+    else return v;
 }
+template <int LPG, int O = 1>
+__device__ __forceinline__ int group_imin(int v) {
+    if constexpr (O < LPG) return group_imin<LPG, 2 * O>(min(v, lane_step<O>(v)));
+    else return v;
+}
+// maximum of non-negative values (and no NaN: what fmaxf made of absolute values) over the LPG lanes that share a group
+// (LPG power of two <= 64).  Their bits order as integers, whose maximum needs no quieting of its operands.
+template <int LPG>
+__device__ __forceinline__ float group_max(float v) { return __int_as_float(group_imax<LPG>(__float_as_int(v))); }
 
 
 // a / b from r = RN(1 / b): one product and the residual correction q - (q b - a) r, both in fma.  The
@@ -88,43 +102,50 @@ __device__ __forceinline__ float div_by(float a, float b, float r) {
 // zero in the 8-bit result anyway
 __device__ __forceinline__ bool div_by_ok(float b) { return b > 1e-30f && b < 1e30f; }
 
-// quantise the 8 values of a lane whose group absmax is m and store them (and, from the group's first
-// lane, the scale): exactly the arithmetic of the 1 x 128 activation quantizers
+// the 8 values of a lane whose group absmax is m as 8 bytes, and the group's scale: exactly the arithmetic of the
+// 1 x 128 activation quantizers
 template <bool FP8>
-__device__ __forceinline__ void quant_store8(const float (&v)[EPL], float m, void* y, int64_t off, void* s, int64_t grp,
-                                             bool first_lane, int mode, bool fp8_scale_f16 = false) {
+__device__ __forceinline__ uint2 quant8(const float (&v)[EPL], float m, int mode, float& sc) {
+    sc = m / (FP8 ? 448.f : 127.f);
+    const bool fast = div_by_ok(sc);
+    const float r = fast ? 1.0f / sc : 0.f;
     if constexpr (FP8) {
-        const float sc = m / 448.f;
         float q[EPL];
-        if (div_by_ok(sc)) {
-            const float r = 1.0f / sc;
+        if (fast) {
 #pragma unroll
             for (int j = 0; j < EPL; ++j) q[j] = div_by(v[j], sc, r);
         } else {
 #pragma unroll
             for (int j = 0; j < EPL; ++j) q[j] = v[j] / sc;
         }
-        uint2 o;
-        o.x = pack_fp8x4(q[0], q[1], q[2], q[3]);
-        o.y = pack_fp8x4(q[4], q[5], q[6], q[7]);
-        *(uint2*)((uint8_t*)y + off) = o;
-        if (first_lane) {
-            if (fp8_scale_f16) ((unsigned short*)s)[grp] = f32_to_f16(sc);
-            else ((float*)s)[grp] = sc;
-        }
+        return make_uint2(pack_fp8x4(q[0], q[1], q[2], q[3]), pack_fp8x4(q[4], q[5], q[6], q[7]));
     } else {
-        const float sc = m / 127.f;
         unsigned w[2] = {0, 0};
-        const bool fast = div_by_ok(sc);
-        const float r = fast ? 1.0f / sc : 0.f;
 #pragma unroll
         for (int j = 0; j < EPL; ++j) {
             int qi = (int)round_mode(fast ? div_by(v[j], sc, r) : v[j] / sc, mode);
             w[j >> 2] |= ((unsigned)(qi & 0xff)) << (8 * (j & 3));
         }
-        *(uint2*)((int8_t*)y + off) = make_uint2(w[0], w[1]);
-        if (first_lane) ((unsigned short*)s)[grp] = f32_to_f16(sc);
+        return make_uint2(w[0], w[1]);
     }
+}
+
+// stores what quant8 returned (the scale from the group's first lane; e4m3: fp32, or fp16 in the payload format)
+template <bool FP8>
+__device__ __forceinline__ void store_quant8(uint2 w, float sc, void* y, int64_t off, void* s, int64_t grp, bool first_lane,
+                                             bool fp8_scale_f16 = false) {
+    *(uint2*)((uint8_t*)y + off) = w;
+    if (!first_lane) return;
+    if (FP8 && !fp8_scale_f16) ((float*)s)[grp] = sc;
+    else ((unsigned short*)s)[grp] = f32_to_f16(sc);
+}
+
+template <bool FP8>
+__device__ __forceinline__ void quant_store8(const float (&v)[EPL], float m, void* y, int64_t off, void* s, int64_t grp,
+                                             bool first_lane, int mode, bool fp8_scale_f16 = false) {
+    float sc;
+    const uint2 w = quant8<FP8>(v, m, mode, sc);
+    store_quant8<FP8>(w, sc, y, off, s, grp, first_lane, fp8_scale_f16);
 }
 
 // round-trip through the storage type: the reference multiplies in the tensor dtype

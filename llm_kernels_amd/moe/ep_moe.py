@@ -12,12 +12,27 @@ from typing import List, Optional
 import torch
 from torch import nn
 
+try:
+    from .. import _lib
+except ImportError:  # this directory's parent itself is on sys.path (the reference's top-level module layout)
+    import _lib
 from .group_gemm_kernel import (grouped_gemm_triton, post_reorder, pre_reorder, run_moe_ep_preproess,
                                 silu_and_mul, gelu_and_mul, pre_reorder_quant, act_and_mul_quant,
                                 grouped_gemm_swiglu_quant, grouped_gemm_swiglu_quant_fused)
 
 
+# limits of the one-launch router (LLMK_ROUTER_MAX_* of the C header)
+ROUTER_MAX_EXPERTS = 512
+ROUTER_MAX_TOPK = 64
+
+
 def softmax_topk_router(router_logits: torch.Tensor, top_k: int = 2, renormalize: bool = True):
+    """softmax over the experts in fp32 and its top_k: (ids int64, weights fp32) [.., top_k], largest first."""
+    if (router_logits.is_cuda and router_logits.dtype in (torch.float32, torch.float16, torch.bfloat16)
+            and 0 < top_k <= ROUTER_MAX_TOPK and top_k <= router_logits.shape[-1] <= ROUTER_MAX_EXPERTS
+            and not (router_logits.requires_grad and torch.is_grad_enabled())):
+        return _lib.host.softmax_topk(router_logits, top_k, renormalize)
+    # host tensors, training and larger routers
     p = torch.softmax(router_logits.float(), dim=-1)
     w, ids = torch.topk(p, top_k, dim=-1)
     if renormalize:

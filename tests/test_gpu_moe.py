@@ -21,6 +21,44 @@ def test_preprocess_worked_example(dev):
     assert seg.tolist() == [0, 3, 6, 9, 12] and seg.dtype == torch.int64 and src2dst.dtype == torch.int32
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,E,topk", [(1, 1, 1), (33, 8, 2), (4096, 8, 8), (5, 9, 3), (64, 33, 4), (7, 64, 64), (100, 65, 8),
+                                      (31, 160, 6), (9, 257, 8), (3, 512, 64)])
+def test_router_in_one_launch(dev, dtype, T, E, topk):
+    """Every lanes-per-token form, up to its last expert, against the float64 softmax of the same logits."""
+    announce("softmax top-k router", dtype, T, E, topk)
+    torch.manual_seed(T + E)
+    logits = torch.stack([torch.randperm(E) for _ in range(T)]).float() / E * 6 - 3      # distinct in every dtype
+    logits = logits.to(dtype)
+    p = torch.softmax(logits.double(), -1)
+    for renorm in (True, False):
+        ids, w = softmax_topk_router(logits.to(dev), topk, renorm)
+        ref, rid = torch.topk(p, topk, dim=-1)
+        ref = ref / ref.sum(-1, keepdim=True) if renorm else ref
+        assert ids.dtype == torch.int64 and w.dtype == torch.float32
+        assert torch.equal(torch.gather(logits, 1, ids.cpu()), torch.gather(logits, 1, rid))
+        # in units of 2^-24: x - max for |x - max| < 8 4, exp 2, up to 8 + 6 additions, division 1, the same again for
+        # the renormalised weights' sum and quotient
+        assert torch.allclose(w.cpu().double(), ref, rtol=48 * 2 ** -24, atol=0)
+
+
+def test_router_breaks_ties_by_index(dev):
+    announce("router ties")
+    ids, w = softmax_topk_router(torch.zeros(5, 12, device=dev), 3)
+    assert ids.tolist() == [[0, 1, 2]] * 5 and torch.allclose(w, torch.full_like(w, 1 / 3))
+
+
+@pytest.mark.parametrize("n,E", [(1, 3), (64, 512), (65, 64), (256, 63), (257, 65), (1024, 8), (1025, 64), (32768, 64)])
+def test_preprocess_workgroup_sizes(dev, n, E):
+    """Edges of the workgroup sizes and of the two ways of counting (64 experts and below, above)."""
+    announce("moe preprocess edges", n, E)
+    torch.manual_seed(n + E)
+    ids = torch.randint(0, E, (n, 1))
+    rids, s2d, seg = gk.run_moe_ep_preproess(ids.to(dev), E)
+    orids, os2d, oseg = m.run_moe_ep_preprocess(ids, E)
+    assert torch.equal(rids.cpu(), orids) and torch.equal(s2d.cpu(), os2d) and torch.equal(seg.cpu(), oseg)
+
+
 @pytest.mark.parametrize("T,E,topk", [(4096, 8, 2), (37, 16, 4), (1, 4, 2), (64, 8, 1)])
 def test_preprocess_random_incl_empty_experts(dev, T, E, topk):
     announce("moe preprocess", T, E, topk)
