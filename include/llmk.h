@@ -94,6 +94,13 @@ int llmk_weight_quant_fp8_block(const void* x, int x_dtype, void* y_e4m3, float*
 int llmk_weight_quant_w4a8_level2(int8_t* y, int8_t* s4, int8_t* z4, int64_t M, int64_t N,
                                   int group, void* stream);
 
+/* Both levels for 128 x 128 blocks and the packing of eight rows per word, in one pass over W [N, K] (N a multiple of 8,
+ * K of 128, group a power of two in 8..128, W and packed 16-byte aligned): packed [N/8, K], s fp16 [ceil(N/128), K/128],
+ * s4 / z4 [N, K/group], equal to llmk_weight_quant_i8_block (qmax 119, half-up, clamp), llmk_weight_quant_w4a8_level2 and
+ * llmk_pack_rows one after the other.   ref: quantization/w4a8_kernel.py:265-314 */
+int llmk_weight_quant_w4a8(const void* x, int x_dtype, int32_t* packed, void* s_f16, int8_t* s4, int8_t* z4,
+                           int64_t N, int64_t K, int group, void* stream);
+
 /* dequantizers: y = fp32(x) * s[block]  ref: fp8_kernel.py:55-105, int8_kernel.py:116-166 */
 int llmk_weight_dequant_fp8_block(const void* x_e4m3, const float* s, void* y, int y_dtype,
                                   int64_t M, int64_t N, int block, void* stream);

@@ -38,6 +38,7 @@ SIGNATURES = {
     "llmk_weight_quant_fp8_block": [_p, _i, _p, _p, _l, _l, _i, _p],
     "llmk_quant_w4_nk": [_p, _i, _p, _p, _p, _l, _l, _i, _p],
     "llmk_weight_quant_w4a8_level2": [_p, _p, _p, _l, _l, _i, _p],
+    "llmk_weight_quant_w4a8": [_p, _i, _p, _p, _p, _p, _l, _l, _i, _p],
     "llmk_weight_dequant_fp8_block": [_p, _p, _p, _i, _l, _l, _i, _p],
     "llmk_weight_dequant_i8_block": [_p, _p, _i, _p, _i, _l, _l, _i, _p],
     "llmk_weight_dequant_w4a8": [_p, _p, _p, _p, _p, _l, _l, _i, _i, _p],

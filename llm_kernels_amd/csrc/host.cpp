@@ -25,7 +25,9 @@ namespace {
     X(llmk_gemm_w4a8_workspace_bytes) X(llmk_gemm_w4a16_marlin) X(llmk_gemm_w4a16_marlin_workspace_bytes)             \
     X(llmk_gemm_w4a16_nk) X(llmk_moe_ep_preprocess) X(llmk_moe_pre_reorder_quant) X(llmk_moe_act_and_mul_quant)       \
     X(llmk_moe_post_reorder) X(llmk_grouped_gemm) X(llmk_grouped_gemm_swiglu_quant)                                   \
-    X(llmk_grouped_gemm_swiglu_quant_fused) X(llmk_moe_softmax_topk)
+    X(llmk_grouped_gemm_swiglu_quant_fused) X(llmk_moe_softmax_topk) X(llmk_weight_quant_w4a8)                        \
+    X(llmk_weight_quant_i8_block) X(llmk_weight_quant_fp8_block) X(llmk_weight_dequant_fp8_block)                     \
+    X(llmk_weight_dequant_i8_block) X(llmk_weight_dequant_w4a8) X(llmk_quant_w4_nk)
 
 // one per imported module object: the package and the top-level module layout may both be imported
 struct State {
@@ -186,6 +188,84 @@ PyObject* rowwise_quant(const Args& a) {
     a.check(a.st->llmk_quant_i8_rowwise(x.data_ptr(), float_code(x.scalar_type()), (int8_t*)y.data_ptr(), (float*)s.data_ptr(), rows, cols, stream_of(x)),
             "llmk_quant_i8_rowwise");
     return wrap_all(std::move(y), std::move(s));
+}
+
+// weight_quant(x, block, fp8): block x block tiles, e4m3 with fp32 scales or int8 (half-away) with fp16 scales
+PyObject* weight_quant(const Args& g) {
+    const at::Tensor& x = g.tensor(0);
+    const int64_t block = g.integer(1);
+    const bool fp8 = g.integer(2) != 0;
+    require(x.is_contiguous(), "Input tensor must be contiguous");
+    require(x.dim() == 2, "Input tensors must have 2 dimensions");
+    g.on_gpu(x);
+    if (block == 0) raise(PyExc_ZeroDivisionError, "integer division or modulo by zero");
+    const int dt = float_code(x.scalar_type());
+    const int64_t N = x.size(0), K = x.size(1), nb = std::max<int64_t>(0, (N + block - 1) / block), kb = std::max<int64_t>(0, (K + block - 1) / block);
+    at::Tensor y = empty(x.sizes(), fp8 ? at::kFloat8_e4m3fn : at::kChar, x), s = empty({nb, kb}, fp8 ? at::kFloat : at::kHalf, x);
+    if (fp8) g.check(g.st->llmk_weight_quant_fp8_block(x.data_ptr(), dt, y.data_ptr(), (float*)s.data_ptr(), N, K, (int)block, stream_of(x)), "llmk_weight_quant_fp8_block");
+    else g.check(g.st->llmk_weight_quant_i8_block(x.data_ptr(), dt, (int8_t*)y.data_ptr(), s.data_ptr(), N, K, (int)block, 127.f, LLMK_ROUND_HALF_AWAY, 0, stream_of(x)),
+                 "llmk_weight_quant_i8_block");
+    return wrap_all(std::move(y), std::move(s));
+}
+
+// weight_dequant(y, s, block, fp8) in the default dtype
+PyObject* weight_dequant(const Args& g) {
+    const at::Tensor &x = g.tensor(0), &s = g.tensor(1);
+    const int64_t block = g.integer(2);
+    const bool fp8 = g.integer(3) != 0;
+    require(x.is_contiguous() && s.is_contiguous(), "Input tensors must be contiguous");
+    require(x.dim() == 2 && s.dim() == 2, "Input tensors must have 2 dimensions");
+    g.on_gpu(x, s);
+    const at::ScalarType out = default_dtype();
+    at::Tensor y = empty(x.sizes(), out, x);
+    if (fp8) {
+        const at::Tensor s32 = as_type(s, at::kFloat);
+        g.check(g.st->llmk_weight_dequant_fp8_block(x.data_ptr(), (const float*)s32.data_ptr(), y.data_ptr(), float_code(out), x.size(0), x.size(1), (int)block, stream_of(x)),
+                "llmk_weight_dequant_fp8_block");
+    } else {
+        g.check(g.st->llmk_weight_dequant_i8_block((const int8_t*)x.data_ptr(), s.data_ptr(), float_code(s.scalar_type()), y.data_ptr(), float_code(out), x.size(0), x.size(1), (int)block,
+                                                   stream_of(x)), "llmk_weight_dequant_i8_block");
+    }
+    return wrap(std::move(y));
+}
+
+// w4a8_weight_quant(x, group): 128 x 128 blocks, both levels and the packing
+PyObject* w4a8_weight_quant(const Args& g) {
+    const at::Tensor& x = g.tensor(0);
+    const int64_t group = g.integer(1), N = x.size(0), K = x.size(1);
+    at::Tensor packed = empty({N / 8, K}, at::kInt, x), s = empty({(N + 127) / 128, K / 128}, at::kHalf, x);
+    at::Tensor s4 = empty({N, K / group}, at::kChar, x), z4 = empty({N, K / group}, at::kChar, x);
+    g.check(g.st->llmk_weight_quant_w4a8(x.data_ptr(), float_code(x.scalar_type()), (int32_t*)packed.data_ptr(), s.data_ptr(), (int8_t*)s4.data_ptr(), (int8_t*)z4.data_ptr(), N, K, (int)group,
+                                         stream_of(x)), "llmk_weight_quant_w4a8");
+    return wrap_all(std::move(packed), std::move(s), std::move(s4), std::move(z4));
+}
+
+// w4a8_weight_dequant(packed, s, s4, z4, block, group) -> fp16
+PyObject* w4a8_weight_dequant(const Args& g) {
+    const at::Tensor& y = g.tensor(0);
+    g.on_gpu(y, g.tensor(1), g.tensor(2), g.tensor(3));
+    const at::Tensor s = g.tensor(1).contiguous(), s4 = g.tensor(2).contiguous(), z4 = g.tensor(3).contiguous();
+    const int64_t K = y.size(1), N = y.size(0) * 8;
+    at::Tensor out = empty({N, K}, at::kHalf, y);
+    g.check(g.st->llmk_weight_dequant_w4a8((const int32_t*)y.data_ptr(), s.data_ptr(), (const int8_t*)s4.data_ptr(), (const int8_t*)z4.data_ptr(), out.data_ptr(), N, K, (int)g.integer(4),
+                                           (int)g.integer(5), stream_of(y)), "llmk_weight_dequant_w4a8");
+    return wrap(std::move(out));
+}
+
+// w4_quantize_nk(w, group) -> (packed, scales, codes)
+PyObject* w4_quantize_nk(const Args& g) {
+    const int64_t group = g.integer(1);
+    if (group == 0) raise(PyExc_ZeroDivisionError, "integer division or modulo by zero");
+    require(g.tensor(0).dim() == 2 && g.tensor(0).size(1) % group == 0, "");
+    const at::ScalarType t = g.tensor(0).scalar_type();
+    require(t == at::kFloat || t == at::kHalf || t == at::kBFloat16, "weights must be fp32, fp16 or bf16");
+    g.on_gpu(g.tensor(0));
+    const at::Tensor w = g.tensor(0).contiguous();
+    const int64_t N = w.size(0), K = w.size(1);
+    at::Tensor packed = empty({N, K / 8}, at::kInt, w), s = empty({N, K / group}, at::kHalf, w), q = empty({N, K}, at::kByte, w);
+    g.check(g.st->llmk_quant_w4_nk(w.data_ptr(), float_code(t), (int32_t*)packed.data_ptr(), s.data_ptr(), (uint8_t*)q.data_ptr(), N, K, (int)group, stream_of(w)), "llmk_quant_w4_nk",
+            PyExc_AssertionError);
+    return wrap_all(std::move(packed), std::move(s), std::move(q));
 }
 
 // ------------------------------------------------------------------ dense GEMMs
@@ -501,7 +581,8 @@ PyObject* call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
-    FN(act_quant, 3), FN(rowwise_quant, 1), FN(softmax_topk, 3), FN(fp8_gemm, 4), FN(int8_gemm, 4), FN(int8_gemm_per_token, 5), FN(w4a8_gemm, 7),
+    FN(act_quant, 3), FN(rowwise_quant, 1), FN(weight_quant, 3), FN(weight_dequant, 4), FN(w4a8_weight_quant, 2),
+    FN(w4a8_weight_dequant, 6), FN(w4_quantize_nk, 2), FN(softmax_topk, 3), FN(fp8_gemm, 4), FN(int8_gemm, 4), FN(int8_gemm_per_token, 5), FN(w4a8_gemm, 7),
     FN(w4a16_gemm, 4), FN(marlin_mul, 4), FN(ep_preprocess, 2), FN(pre_reorder_quant, 9), FN(act_and_mul_quant, 8),
     FN(post_reorder, 9), FN(grouped_gemm, 8), FN(swiglu_fused, 3), FN(swiglu_quant, 9),
     {nullptr, nullptr, 0, nullptr}};

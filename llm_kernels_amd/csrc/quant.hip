@@ -234,6 +234,105 @@ __global__ void w4a8_level2_kernel(int8_t* __restrict__ y, int8_t* __restrict__ 
     if (tid % LPG == 0) { s4[grp] = (int8_t)(int)fs4; z4[grp] = (int8_t)(int)fz4; }
 }
 
+// ---------------------------------------------------------------- both w4a8 levels and the packing in one pass
+// One workgroup per 128 x 128 block of W [N, K].  A thread owns 8 consecutive rows x 8 consecutive columns, which are 8
+// whole words of the [N/8, K] packed layout, so nothing is exchanged but the block maximum and the group extrema (LPG
+// lanes per 8 * LPG-column group): W is read once and the words written once, where the three separate kernels wrote and
+// re-read the int8 matrix twice (14336 x 4096 fp16: 108 us).  What bounds it is the vector ALU beside that stream: the
+// arithmetic as the separate kernels write it (about 26 instructions per weight) took 48 us, the forms below 33.
+// The loaded 16-bit values stay packed between the two passes over them (32 registers instead of 64).
+// First level as weight_quant_block_kernel (qmax 119, half-up, clamped), second as w4a8_level2_kernel: same results.
+template <int DT, int LPG>
+__global__ __launch_bounds__(256) void weight_quant_w4a8_kernel(const void* __restrict__ x, int32_t* __restrict__ packed,
+                                                                unsigned short* __restrict__ s, int8_t* __restrict__ s4,
+                                                                int8_t* __restrict__ z4, int64_t N, int64_t K) {
+    constexpr float QMAX = 119.f;
+    __shared__ float red[4];
+    const int t = threadIdx.x;
+    const int64_t r0 = (int64_t)blockIdx.y * 128 + (t >> 4) * 8, c0 = (int64_t)blockIdx.x * 128 + (t & 15) * EPL;
+    const bool live = r0 < N;                            // N is a multiple of 8: a thread's rows exist together
+    constexpr int CHUNKS = DT == LLMK_F32 ? 2 : 1;
+    uint4 raw[8][CHUNKS];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int h = 0; h < CHUNKS; ++h)
+            raw[j][h] = live ? ((const uint4*)((const uint8_t*)x + ((r0 + j) * K + c0) * (DT == LLMK_F32 ? 4 : 2)))[h] : make_uint4(0, 0, 0, 0);
+    float m = 0.f;
+    if constexpr (DT == LLMK_F16) {                      // two magnitudes per instruction
+        v2h mm = {(_Float16)0, (_Float16)0};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const unsigned w[4] = {raw[j][0].x, raw[j][0].y, raw[j][0].z, raw[j][0].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) asm("v_pk_max_f16 %0, %0, %1" : "+v"(mm) : "v"(w[e] & 0x7fff7fffu));
+        }
+        m = fmaxf((float)mm[0], (float)mm[1]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float v[EPL];
+            load8<DT>(&raw[j][0], 0, v);
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) m = fmaxf(m, fabsf(v[e]));
+        }
+    }
+    m = group_max<64>(m);
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float sc = m / QMAX;
+    const bool fast = div_by_ok(sc);
+    const float rcp = fast ? 1.0f / sc : 0.f;
+    const int64_t ng = K / (8 * LPG);
+    int8_t* const ps4 = s4 + r0 * ng + c0 / (8 * LPG);
+    int8_t* const pz4 = z4 + r0 * ng + c0 / (8 * LPG);
+    const bool first = live && (t & (LPG - 1)) == 0;
+    unsigned word[EPL] = {0, 0, 0, 0, 0, 0, 0, 0};
+    auto row = [&](int j, auto level1) __attribute__((always_inline)) {
+        float v[EPL];
+        load8<DT>(&raw[j][0], 0, v);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) v[e] = level1(v[e]);
+        float mx = v[0], mn = v[0];
+#pragma unroll
+        for (int e = 1; e < EPL; ++e) { mx = fmaxf(mx, v[e]); mn = fminf(mn, v[e]); }
+        mx = (float)group_imax<LPG>((int)mx);
+        mn = (float)group_imin<LPG>((int)mn);
+        // The second level's quotients are of integers: |mx - mn| <= 238 by 15 (never half-way, at least 1 / 30 away from
+        // it), and |v| <= 119 by 1 <= fs4 <= 16, whose v / fs4 + 0.5 is an integer or at least 1 / 32 away from one.  So a
+        // product with the reciprocal does, once 2^-10 lifts the integers over its rounding errors (below 2^-15).
+        const float fs4 = floorf(fmaf(mx - mn, 1.0f / 15.0f, 0.5f));
+        const bool spread = fs4 > 0.f;
+        const float r4 = spread ? __builtin_amdgcn_rcpf(fs4) : 0.f;
+        const float fz4 = floorf(fmaf(-mn, r4, 0.5f + 0x1p-10f));
+        // clamp(floor(v / fs4 + 0.5) + fz4, 0, 15): truncated after the clamp.  Equal values (fs4 = 0) have quotients
+        // inf - inf there, which that clamp turns into code 0, and a zero point of inf or NaN as int8: -1 below zero, else 0.
+        const float c4 = spread ? fz4 + (0.5f + 0x1p-10f) : 0.f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e)
+            word[e] |= (unsigned)__builtin_amdgcn_fmed3f(fmaf(v[e], r4, c4), 0.f, 15.f) << (4 * j);
+        if (first) {
+            ps4[j * ng] = (int8_t)(int)fs4;
+            pz4[j * ng] = (int8_t)(spread ? (int)fz4 : (mn < 0.f ? -1 : 0));
+        }
+    };
+    if (fast) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            row(j, [&](float x) { return __builtin_amdgcn_fmed3f(floorf(div_by(x, sc, rcp) + 0.5f), -QMAX, QMAX); });
+    } else {                                             // a block of zeros among others: the order that drops a NaN
+        for (int j = 0; j < 8; ++j)
+            row(j, [&](float x) { return fminf(fmaxf(floorf(x / sc + 0.5f), -QMAX), QMAX); });
+    }
+    if (live) {
+        uint4* o = (uint4*)(packed + (r0 >> 3) * K + c0);
+        o[0] = make_uint4(word[0], word[1], word[2], word[3]);
+        o[1] = make_uint4(word[4], word[5], word[6], word[7]);
+    }
+    if (t == 0) s[(int64_t)blockIdx.y * (K >> 7) + blockIdx.x] = f32_to_f16(sc);
+}
+
 // ---------------------------------------------------------------- dequantizers
 template <int ODT, int SDT, bool FP8>
 __global__ void weight_dequant_block_kernel(const uint8_t* __restrict__ x, const void* __restrict__ s,
@@ -542,6 +641,28 @@ extern "C" int llmk_weight_quant_w4a8_level2(int8_t* y, int8_t* s4, int8_t* z4, 
     LPG_SWITCH(group, CALL)
 #undef CALL
     LLMK_CHECK_LAUNCH("w4a8_level2");
+    return LLMK_OK;
+}
+
+extern "C" int llmk_weight_quant_w4a8(const void* x, int x_dtype, int32_t* packed, void* s, int8_t* s4, int8_t* z4,
+                                      int64_t N, int64_t K, int group, void* stream) {
+    if (!lpg_ok(group) || group > 128 || N < 0 || K < 0 || N % 8 || K % 128)
+        LLMK_FAIL(LLMK_ERR_SHAPE, "weight_quant_w4a8: N=%lld K=%lld group=%d (need N %% 8, K %% 128, group a power of two in 8..128)", (long long)N, (long long)K, group);
+    if (N == 0 || K == 0) return LLMK_OK;
+    if (!x || !packed || !s || !s4 || !z4) LLMK_FAIL(LLMK_ERR_ARG, "weight_quant_w4a8: null pointer");
+    if ((((uintptr_t)x) | ((uintptr_t)packed)) & 15) LLMK_FAIL(LLMK_ERR_ARG, "weight_quant_w4a8: W and the packed words must be 16-byte aligned");
+    if (N > 128ll * 65535) LLMK_FAIL(LLMK_ERR_SHAPE, "weight_quant_w4a8: N=%lld exceeds the grid", (long long)N);
+    dim3 grid((unsigned)(K / 128), (unsigned)cdiv64(N, 128));
+#define CALL(L) LLMK_DISPATCH_FLOAT(x_dtype, DT, (weight_quant_w4a8_kernel<DT, L><<<grid, 256, 0, (hipStream_t)stream>>>(x, packed, (unsigned short*)s, s4, z4, N, K)))
+    switch (group / EPL) {
+        case 1: CALL(1); break;
+        case 2: CALL(2); break;
+        case 4: CALL(4); break;
+        case 8: CALL(8); break;
+        default: CALL(16); break;
+    }
+#undef CALL
+    LLMK_CHECK_LAUNCH("weight_quant_w4a8");
     return LLMK_OK;
 }
 

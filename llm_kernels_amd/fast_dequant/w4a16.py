@@ -18,17 +18,7 @@ def quantize_nk(w: torch.Tensor, group_size: int = 128):
     One pass over W on the GPU: s = absmax / 7 rounded to fp16, q = clamp(rne(w / s), -8, 7) + 8 with the
     quotient by the rounded scale in fp32, nibble i of a packed word is k = 8 * word + i (the layout of
     quantization.bitpack.pack_weights_over_cols(q, 4, 32, transpose=False))."""
-    assert w.dim() == 2 and w.shape[1] % group_size == 0
-    assert w.dtype in (torch.float32, torch.float16, torch.bfloat16), 'weights must be fp32, fp16 or bf16'
-    _lib.require_gpu(w)
-    w = w.contiguous()
-    N, K = w.shape
-    packed = torch.empty(N, K // 8, dtype=torch.int32, device=w.device)
-    s = torch.empty(N, K // group_size, dtype=torch.float16, device=w.device)
-    q = torch.empty(N, K, dtype=torch.uint8, device=w.device)
-    _lib.call("llmk_quant_w4_nk", _lib.ptr(w), _lib.dt(w.dtype), _lib.ptr(packed), _lib.ptr(s), _lib.ptr(q),
-              N, K, group_size, _lib.stream(w), exc=AssertionError)
-    return packed, s, q
+    return _lib.host.w4_quantize_nk(w, group_size)
 
 
 def w4a16_gemm(x: torch.Tensor, w_packed: torch.Tensor, scales: torch.Tensor, group_size: int = 128):

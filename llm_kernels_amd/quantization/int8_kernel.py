@@ -21,26 +21,12 @@ def act_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, tor
 
 def weight_quant(x: torch.Tensor, block_size: int = 128) -> Tuple[torch.Tensor, torch.Tensor]:
     """block x block tiles of W [N, K]: s = blockmax / 127, half-away rounding, fp16 scales."""
-    assert x.is_contiguous(), 'Input tensor must be contiguous'
-    assert x.dim() == 2, 'Input tensors must have 2 dimensions'
-    _lib.require_gpu(x)
-    M, N = x.size()
-    y = torch.empty_like(x, dtype=torch.int8)
-    s = x.new_empty(((M + block_size - 1) // block_size, (N + block_size - 1) // block_size), dtype=torch.float16)
-    _lib.call("llmk_weight_quant_i8_block", _lib.ptr(x), _lib.dt(x.dtype), _lib.ptr(y), _lib.ptr(s),
-              M, N, block_size, 127.0, _lib.ROUND_HALF_AWAY, 0, _lib.stream(x))
-    return y, s
+    return _lib.host.weight_quant(x, block_size, False)
 
 
 def weight_dequant(x: torch.Tensor, s: torch.Tensor, block_size: int = 128) -> torch.Tensor:
-    assert x.is_contiguous() and s.is_contiguous(), 'Input tensors must be contiguous'
-    assert x.dim() == 2 and s.dim() == 2, 'Input tensors must have 2 dimensions'
-    _lib.require_gpu(x, s)
-    M, N = x.size()
-    y = torch.empty_like(x, dtype=torch.get_default_dtype())
-    _lib.call("llmk_weight_dequant_i8_block", _lib.ptr(x), _lib.ptr(s), _lib.dt(s.dtype), _lib.ptr(y),
-              _lib.dt(y.dtype), M, N, block_size, _lib.stream(x))
-    return y
+    """y = fp32(x) * s[block] in torch's default dtype."""
+    return _lib.host.weight_dequant(x, s, block_size, False)
 
 
 def int8_gemm(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.Tensor):

@@ -154,3 +154,27 @@ def test_fp8_quantisers_keep_the_sign_of_zero(dev, dtype):
     y, s = fp8_kernel.weight_quant(x.to(dev))
     oy, os_ = q.weight_quant_fp8(x)
     assert torch.equal(s.cpu(), os_) and torch.equal(y.cpu().view(torch.uint8), oy.view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,K,group", [(8, 128, 128), (136, 256, 64), (128, 384, 32), (264, 128, 16), (392, 256, 8)])
+def test_w4a8_weight_quant_in_one_pass(dev, dtype, N, K, group):
+    """Partial row blocks, every group width, a block of zeros (scale 0) and groups of equal values (second scale 0)."""
+    announce("w4a8 weight_quant one pass", dtype, N, K, group)
+    torch.manual_seed(N + K + group)
+    w = (torch.randn(N, K) * 0.02).to(dtype)
+    w[:, 128:256] = 0
+    w[3, :128] = 0.05
+    w[5, :128] = -0.05
+    wd = w.to(dev)
+    packed, s, s4, z4 = w4a8_kernel.weight_quant(wd, 128, group)
+    y = torch.empty(N, K, dtype=torch.int8, device=dev)
+    s_ref = torch.empty_like(s)
+    s4_ref, z4_ref = torch.empty_like(s4), torch.empty_like(z4)
+    _lib.call("llmk_weight_quant_i8_block", _lib.ptr(wd), _lib.dt(dtype), _lib.ptr(y), _lib.ptr(s_ref), N, K, 128, 119.0,
+              _lib.ROUND_HALF_UP, 1, None)
+    _lib.call("llmk_weight_quant_w4a8_level2", _lib.ptr(y), _lib.ptr(s4_ref), _lib.ptr(z4_ref), N, K, group, None)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(bp.pack_rows(y.cpu().numpy().astype("uint8"), 4, 32)[0])
+    assert torch.equal(packed.cpu(), want)
+    assert torch.equal(s, s_ref) and torch.equal(s4, s4_ref) and torch.equal(z4, z4_ref)
