@@ -90,6 +90,28 @@ __device__ __forceinline__ v4f step_dot(const v8i& a, const v8i& b) {
     }
 }
 
+// The same in the form the MFMA leaves it (int32 bits for the integer kinds) and its conversion: a loop that scales a
+// product while later ones multiply converts it then too, a conversion right behind the MFMA waits for it.
+template <int KIND>
+__device__ __forceinline__ v4f step_raw(const v8i& a, const v8i& b) {
+    if constexpr (KIND == K_I8_BLOCK || KIND == K_W4A8) {
+        v4i t = mfma_i8_16x16x64((v4i){a[0], a[1], a[2], a[3]}, (v4i){b[0], b[1], b[2], b[3]}, (v4i){0, 0, 0, 0});
+        t = mfma_i8_16x16x64((v4i){a[4], a[5], a[6], a[7]}, (v4i){b[4], b[5], b[6], b[7]}, t);
+        return __builtin_bit_cast(v4f, t);
+    } else {
+        return step_dot<KIND>(a, b);
+    }
+}
+template <int KIND>
+__device__ __forceinline__ v4f raw_f32(const v4f& t) {
+    if constexpr (KIND == K_I8_BLOCK || KIND == K_W4A8) {
+        const v4i i = __builtin_bit_cast(v4i, t);
+        return (v4f){(float)i[0], (float)i[1], (float)i[2], (float)i[3]};
+    } else {
+        return t;
+    }
+}
+
 struct DirectArgs {
     const uint8_t* a;      // [M, K] elements of ESZ bytes
     const uint8_t* b;      // [N, K] or [E, N, K]

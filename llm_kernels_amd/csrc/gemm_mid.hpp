@@ -208,8 +208,8 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_kernel(DirectArgs p) {
             if (i + 1 < MT) af[(i + 1) & 1] = ldfrag(As + (i + 1) * 2048);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                if (i < MT) t[i & 1][j] = step_dot<KIND>(bf[j], af[i & 1]);
-                if (i > 0) acc[i - 1][j] += t[(i - 1) & 1][j] * sa[i - 1];
+                if (i < MT) t[i & 1][j] = step_raw<KIND>(bf[j], af[i & 1]);
+                if (i > 0) acc[i - 1][j] += raw_f32<KIND>(t[(i - 1) & 1][j]) * sa[i - 1];
             }
             // nothing moves across a tile row: the lag of one row between product and accumulation stays, and
             // the fragments of at most two rows are live
@@ -553,8 +553,8 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
                     if (i + 1 < MT) af[(i + 1) & 1] = ldfrag(As + (i + 1) * 2048);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        if (i < MT) t[i & 1][j] = step_dot<KIND>(bf[j], af[i & 1]);
-                        if (i > 0) acc[i - 1][j] += t[(i - 1) & 1][j] * sa[i - 1];
+                        if (i < MT) t[i & 1][j] = step_raw<KIND>(bf[j], af[i & 1]);
+                        if (i > 0) acc[i - 1][j] += raw_f32<KIND>(t[(i - 1) & 1][j]) * sa[i - 1];
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }

@@ -488,10 +488,12 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
+                // (int8: t waits as int32 and is converted where it is retired, a tile row later, and not behind its MFMA:
+                // 4096x14336x4096 295 -> 279 us, 2048x4096x4096 51.4 -> 48.9, experts 4096 tokens 2043 -> 1930)
                 if constexpr (SCALED) {
-                    if (i < NR) t[i & 1][j] = step_dot<KIND>(bf[j], af[i & 1]);
-                    if (i > 0 && i <= NR) acc[i - 1][j] += t[(i - 1) & 1][j] * sa[i - 1];
-                    else if (i == 0 && NR == R) acc[R - 1][j] += t[1][j] * sprev;
+                    if (i < NR) t[i & 1][j] = step_raw<KIND>(bf[j], af[i & 1]);
+                    if (i > 0 && i <= NR) acc[i - 1][j] += raw_f32<KIND>(t[(i - 1) & 1][j]) * sa[i - 1];
+                    else if (i == 0 && NR == R) acc[R - 1][j] += raw_f32<KIND>(t[1][j]) * sprev;
                 } else {
                     if (i < NR) acc[i][j] = mma_plain<KIND>(bf[j], af[i & 1], acc[i][j]);
                 }
@@ -537,7 +539,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
         if (kt < KT) step(kt, no, no, nr_c);
         if constexpr (SCALED && decltype(nr_c)::value == R) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[R - 1][j] += t[1][j] * sprev;
+            for (int j = 0; j < 4; ++j) acc[R - 1][j] += raw_f32<KIND>(t[1][j]) * sprev;
         }
     };
     if constexpr (GROUPED) {
