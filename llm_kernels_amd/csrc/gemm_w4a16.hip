@@ -558,10 +558,15 @@ __global__ __launch_bounds__(512) void w4a16_nk_stream_kernel(
 }
 
 // Ring variant of the weight-streaming kernel for 128-wide groups, at most 16 rows per workgroup and a K range
-// of at most 32 steps (steps % 4 == 0): wave w owns the four consecutive 128-K steps 4w .. 4w + 3 of every
+// of 4 to 32 steps: wave w owns the four consecutive 128-K steps 4w .. 4w + 3 of every
 // 16-column tile, its activation fragments stay in registers, and the packed words and group scales of the
 // next DEPTH - 1 tiles are in flight in a ring of registers filled by hand-issued loads (see stream_ring.hpp:
 // one s_waitcnt per tile that leaves exactly the younger tiles outstanding).
+// Every wave loads four steps, so that one wait count serves all: where fewer are left in the range the share is moved
+// back to its last four steps (the repeated ones hit L2) and the steps that another wave owns count as zero activations
+// and zero scales.  (Ranges that are no multiple of
+// 512 went through a bf16 copy of W, or the stream kernel for fp16; us per call, cold weights: bf16 3 x 4672 x 9088
+// 70.6 -> 14.8, 16 x 14336 x 2176 32.7 -> 11.7, 60 x 24000 x 3968 90.0 -> 36.7; fp16 15.1 -> 15.3, 13.2 -> 12.4, 50.2 -> 41.1.)
 // BF: bf16 activations and outputs.  A nibble becomes the bf16 number 128 + q by OR-ing it into 0x4300 (exact:
 // seven mantissa bits, q < 16), and the missing "- 136" of every product is the accumulator the MFMA chain of a
 // step starts from: -136 * sum_k a[m][k] over the step, computed once per wave with the same MFMA and a weight
@@ -580,8 +585,8 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     const int steps = K >> 7, ngroups = Kfull >> 7, kwords = Kfull >> 3;
     const int m0 = blockIdx.y * 16;
     const int ntiles = (N + 15) >> 4;
-    const bool wvalid = 4 * wave < steps;                // waves past the K range multiply by zero scales
-    const int s0 = wvalid ? 4 * wave : 0;                // first step of this wave
+    const int s0 = min(4 * wave, steps - 4);             // first step this wave loads
+    const int u0 = min(4 * wave - s0, 4);                // steps s0 .. s0 + u0 - 1 belong to other waves
 
     // ---- activations, requested first: row i of the wave's K slice (512 elements = 1 KiB) is one fully
     // coalesced load.  (Fetching the MFMA fragments straight from global memory costs 2 us per launch: every
@@ -643,6 +648,11 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
                 a[4 * u + j] = y;
             }
         }
+        if (u0 > 0) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (i < 4 * u0) a[i] = (v4i){0, 0, 0, 0};
+        }
     }
 
     // bf16: the bias of step u, -136 * sum_k a[row][k] in every column of the MFMA result
@@ -669,7 +679,7 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const unsigned sraw = ((unsigned)(u < 2 ? ts[0] : ts[1]) >> (16 * (u & 1))) & 0xffffu;
-            const float sc = wvalid ? f16_to_f32((unsigned short)sraw) : 0.f;
+            const float sc = u < u0 ? 0.f : f16_to_f32((unsigned short)sraw);
             v4f t = bias[u];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -748,12 +758,12 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     ring_drain<0>();
 }
 
-// The ring kernel takes 128-wide groups, K ranges of at most 32 steps in whole four-step shares, 8-byte aligned
-// scale rows and operands below 4 GiB (32-bit lane offsets); nz = number of K ranges.
-bool nk_ring_ok(int64_t M, int64_t N, int64_t K, int groupsize, int nz, const void* S) {
-    const int64_t steps_all = K >> 7, steps = (steps_all + nz - 1) / nz;
-    return groupsize == 128 && steps <= 32 && steps_all % 4 == 0 && steps % 4 == 0 && !(((uintptr_t)S) & 7) &&
-           N * (K / 2) < (1ll << 32) && M * K * 2 < (1ll << 32);
+// The ring kernel takes 128-wide groups, K ranges of 4 to 32 steps (the last one takes what is left) and operands below
+// 4 GiB (32-bit lane offsets); nz = number of K ranges.  The four group scales of a share are one 8-byte load at a
+// multiple of two bytes: scale rows of any length (K / 128 not a multiple of four) are read as they lie.
+bool nk_ring_ok(int64_t M, int64_t N, int64_t K, int groupsize, int nz) {
+    const int64_t steps_all = K >> 7, steps = (steps_all + nz - 1) / nz, last = steps_all - (nz - 1) * steps;
+    return groupsize == 128 && steps <= 32 && last >= 4 && N * (K / 2) < (1ll << 32) && M * K * 2 < (1ll << 32);
 }
 
 // fp16 or bf16 (bf) activations / outputs; partial: fp32 planes for nz > 1 (a summing pass follows)
@@ -796,7 +806,7 @@ template <int MT, int NT>
 int launch_nk_stream(const _Float16* A, const int32_t* B, const _Float16* S, _Float16* C, int M, int N, int K, int groupsize,
                      int nz, float* partial, hipStream_t st) {
     if constexpr (MT == 1 && NT == 1) {
-        if (nk_ring_ok(M, N, K, groupsize, nz, S)) return launch_nk_ring(A, B, S, C, M, N, K, nz, partial, false, st);
+        if (nk_ring_ok(M, N, K, groupsize, nz)) return launch_nk_ring(A, B, S, C, M, N, K, nz, partial, false, st);
     }
     constexpr int U = MT == 1 ? 4 : (MT == 2 ? 2 : 1);
     // nz K ranges, equally long up to one step
@@ -1042,7 +1052,7 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
     _Float16* C = (_Float16*)c;
     // bf16: the weight-streaming ring kernel for decode sizes, everything else through the bf16 copy of W
     const int nz_bf = (int)((K / 128 + 31) / 32);
-    const bool bf_ring = bf && M <= 64 && nk_ring_ok(M, N, K, groupsize, nz_bf, s) && !((uintptr_t)c & 7) &&
+    const bool bf_ring = bf && M <= 64 && nk_ring_ok(M, N, K, groupsize, nz_bf) && !((uintptr_t)c & 7) &&
                          (nz_bf == 1 || ((M * N) % 4 == 0 && workspace && workspace_bytes >= (int64_t)nz_bf * M * N * 4 &&
                                          !((uintptr_t)workspace & 15)));
     if (bf_ring) return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, nz_bf, (float*)workspace, true, st);

@@ -356,11 +356,11 @@ PyObject* w4a16_gemm(const Args& g) {
     const bool bf = x.scalar_type() == at::kBFloat16;
     at::Tensor y = empty(with_last(x, N), x.scalar_type(), x);
     // bf16 at decode size runs on the weight-streaming ring kernel under exactly the conditions the library
-    // checks (128-wide groups, K ranges of at most 32 steps in whole four-step shares, 8-byte aligned scale rows
-    // and outputs, 32-bit lane offsets, and with more than one K range M * N % 4 == 0 for the summing pass);
+    // checks (128-wide groups, K ranges of 4 to 32 steps, 8-byte aligned outputs, 32-bit lane offsets, and with more than
+    // one K range M * N % 4 == 0 for the summing pass);
     // every other bf16 call goes through the bf16 copy of W and needs room for it
     const int64_t steps = K / 128, nz = std::max<int64_t>(1, (steps + 31) / 32), per = (steps + nz - 1) / nz;
-    const bool ring_ok = group == 128 && per <= 32 && steps % 4 == 0 && per % 4 == 0 && ((uintptr_t)s.data_ptr() & 7) == 0 &&
+    const bool ring_ok = group == 128 && per <= 32 && steps - (nz - 1) * per >= 4 &&
                          N * (K / 2) < (1ll << 32) && M * K * 2 < (1ll << 32);
     const bool bf_decode = bf && M <= 64 && ring_ok && ((uintptr_t)y.data_ptr() & 7) == 0 && (nz == 1 || (M * N) % 4 == 0);
     int64_t need = 0;

@@ -309,6 +309,30 @@ def test_w4a16_nk_bf16_decode_is_exact_for_small_integers(dev):
     assert torch.equal(y.cpu().double(), ref.bfloat16().double())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 512), (3, 40, 640), (16, 1000, 768), (17, 136, 896), (64, 264, 1408), (5, 5000, 3968),
+                                   (4, 72, 4224), (64, 136, 8320), (3, 4672, 9088)])
+def test_w4a16_nk_decode_any_number_of_steps(dev, dtype, M, N, K):
+    """K ranges of the ring kernel that are no multiple of its waves' four-step shares, one range and several of unequal
+    length, scale rows at every two-byte offset.  Small integers and power-of-two scales: every sum is exact in fp32, so the
+    result is the rounded product (bf16 via -136 biases included).  fp16: an infinite activation reaches its own row only."""
+    announce("w4a16 nk decode steps", dtype, M, N, K)
+    torch.manual_seed(M + N + K)
+    x = torch.randint(-2, 3, (M, K)).to(dtype)
+    qn = torch.randint(0, 16, (N, K), dtype=torch.uint8)
+    s = torch.exp2(torch.randint(-4, 1, (N, K // 128)).float()).half()
+    packed = torch.from_numpy(bp.pack_cols(qn.numpy(), 4, 32)[0]).to(dev)
+    w = (qn.double() - 8) * s.double().repeat_interleave(128, 1)
+    y = w4a16.w4a16_gemm(x.to(dev), packed, s.to(dev), 128)
+    assert torch.equal(y.cpu(), (x.double() @ w.T).to(dtype))
+    if dtype == torch.float16:
+        x[0, K - 1] = float("inf")
+        y = w4a16.w4a16_gemm(x.to(dev), packed, s.to(dev), 128).cpu()
+        ref = (x.double() @ w.T).to(dtype)
+        assert torch.equal(y[1:], ref[1:]) and torch.equal(y[0].isnan(), ref[0].isnan())
+        assert torch.equal(y[0].nan_to_num(0.0), ref[0].nan_to_num(0.0))
+
+
 @pytest.mark.parametrize("M,N,K,gs", [(65, 72, 128, 64), (130, 4096, 1024, 128), (512, 264, 4096, 128), (300, 14344, 512, 128),
                                       (200, 20000, 640, 128), (500, 8192, 384, 192), (600, 10000, 1024, 128), (1024, 28672, 256, 128)])
 def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
