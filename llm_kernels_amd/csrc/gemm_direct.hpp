@@ -137,6 +137,53 @@ struct DirectArgs {
     int round_mode;        // int8 rounding of the quantiser
 };
 
+// Grouped launches: a tile list in which segment e owns ceil(rows of e / bm) * mult consecutive entries.
+// segment_of finds the owner of entry `want`; rest = the entry's index inside the segment; not found: s0 = length of the list.
+// Every lane takes one segment and a wave scan adds up the entries: with 64 experts the walk over the segments one after the
+// other (a dependent scalar load each) was a fixed cost of every tile.  (Grouped launches of 8, 16 and 64 experts, us per expert layer:
+// 64 experts 2 tokens 102 -> 52, 40 tokens 161 -> 132, 400 tokens 223 -> 164; 16 experts 3 tokens 104 -> 75; 8 large experts,
+// 4096 tokens, 1589 -> 1543.)
+// All 64 lanes of the wave must be active; segment ends are ascending.
+struct SegmentTile {
+    bool found;
+    int e, s0, s1, rest;
+};
+__device__ __forceinline__ int wave_scan_add(int v) {        // inclusive prefix sum over the 64 lanes
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);      // row_bcast:31 into rows 2 and 3
+    return v;
+}
+__device__ __forceinline__ SegmentTile segment_of(const int64_t* __restrict__ ptr, int E, int bm, int mult, int want) {
+    SegmentTile t{false, 0, 0, 0, 0};
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int a = (int)ptr[min(e0 + lane, E)], b = (int)ptr[min(e0 + lane + 1, E)];
+        const int own = ((b - a + bm - 1) / bm) * mult, end = base + wave_scan_add(own);
+        const uint64_t hit = __ballot(want < end);
+        if (hit) {
+            const int l = __builtin_ctzll(hit);
+            t.found = true;
+            t.e = e0 + l;
+            t.s0 = __builtin_amdgcn_readlane(a, l);
+            t.s1 = __builtin_amdgcn_readlane(b, l);
+            t.rest = want - __builtin_amdgcn_readlane(end - own, l);
+            return t;
+        }
+        base = __builtin_amdgcn_readlane(end, 63);
+    }
+    t.s0 = base;
+    return t;
+}
+// length of the list
+__device__ __forceinline__ int segment_entries(const int64_t* __restrict__ ptr, int E, int bm, int mult) {
+    return segment_of(ptr, E, bm, mult, 0x7fffffff).s0;
+}
+
 // Upper bound of the row tiles of a grouped GEMM (segment ends are only known on the device): every segment
 // adds at most one ragged tile, and no segment has more tiles than rows.
 inline int grouped_row_tiles(int M, int E, int tile_rows) {
@@ -171,19 +218,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
     const uint8_t* bbase = p.b;
     int64_t bs_off = 0;
     if constexpr (GROUPED) {
-        // locate the segment that owns m-tile blockIdx.y
-        int tile = blockIdx.y, e = 0, cum = 0;
-        int64_t s0 = p.seg_indptr[0];
-        bool found = false;
-        for (; e < p.E; ++e) {
-            int64_t s1 = p.seg_indptr[e + 1];
-            int t = (int)((s1 - s0 + 16 * MT - 1) / (16 * MT));
-            if (tile < cum + t) { found = true; m_start = (int)s0 + (tile - cum) * 16 * MT; m_end = min((int)s1, m_start + 16 * MT); break; }
-            cum += t;
-            s0 = s1;
-        }
-        if (!found) return;
-        const int64_t widx = p.weight_indices ? p.weight_indices[e] : e;
+        const SegmentTile sg = segment_of(p.seg_indptr, p.E, 16 * MT, 1, (int)blockIdx.y);
+        if (!sg.found) return;
+        m_start = sg.s0 + sg.rest * 16 * MT;
+        m_end = min(sg.s1, m_start + 16 * MT);
+        const int64_t widx = p.weight_indices ? p.weight_indices[sg.e] : sg.e;
         bbase += widx * (int64_t)N * K * ESZ;
         bs_off = widx * (int64_t)((N + 127) / 128) * steps;
     } else {

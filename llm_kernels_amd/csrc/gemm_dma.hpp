@@ -272,18 +272,11 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
     const uint8_t* bbase = p.b;
     int64_t bs_off = 0;
     if constexpr (GROUPED) {
-        int tile = blockIdx.y, e = 0, cum = 0;
-        int64_t s0 = p.seg_indptr[0];
-        bool found = false;
-        for (; e < p.E; ++e) {
-            const int64_t s1 = p.seg_indptr[e + 1];
-            const int t = (int)((s1 - s0 + BM - 1) / BM);
-            if (tile < cum + t) { found = true; m_start = (int)s0 + (tile - cum) * BM; m_end = min((int)s1, m_start + BM); break; }
-            cum += t;
-            s0 = s1;
-        }
-        if (!found) return;
-        const int64_t widx = p.weight_indices ? p.weight_indices[e] : e;
+        const SegmentTile sg = segment_of(p.seg_indptr, p.E, BM, 1, (int)blockIdx.y);
+        if (!sg.found) return;
+        m_start = sg.s0 + sg.rest * BM;
+        m_end = min(sg.s1, m_start + BM);
+        const int64_t widx = p.weight_indices ? p.weight_indices[sg.e] : sg.e;
         bbase += widx * (int64_t)N * K;
         bs_off = widx * (int64_t)((N + 127) / 128) * KT_all;
     } else {

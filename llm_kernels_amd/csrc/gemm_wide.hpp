@@ -37,6 +37,14 @@ struct WideTile {
     bool found;
 };
 
+// number of tiles of the launch (the valid linear ids are 0 .. total - 1)
+template <bool GROUPED, int R>
+__device__ __forceinline__ int wide_total_tiles(const DirectArgs& p, int gx) {
+    constexpr int W_BM = w_bm(R);
+    if constexpr (!GROUPED) return gx * ((p.M + W_BM - 1) / W_BM);
+    return segment_entries(p.seg_indptr, p.E, W_BM, gx);
+}
+
 template <bool GROUPED, int R>
 __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, int gx) {
     constexpr int W_BM = w_bm(R);
@@ -66,70 +74,48 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
         t.m_end = min(p.M, t.m_start + W_BM);
         t.found = true;
     } else {
-        int e = 0;
-        int64_t s0 = p.seg_indptr[0];
-        if (gx % 8 == 0) {
-            // XCD x (workgroup id mod 8) owns the column tiles x, x + 8, ...; it walks them segment by
-            // segment, and for every column tile the row tiles of the segment back to back, so the workgroups
-            // that share a weight tile run at the same time on the L2 that holds it.  Long segments go in strips of
-            // four row tiles (the last strip takes what is left, one to five), each strip across all column tiles
-            // of the XCD: its 32 concurrent workgroups then share 8 weight tiles and 4 activation tiles, where one
-            // column tile x 32 row tiles would pull 33 operand tiles per K step through the L2 instead of 12.
-            const int x = lin & 7, cx = gx >> 3;
-            int s = lin >> 3;
-            for (; e < p.E; ++e) {
-                const int64_t s1 = p.seg_indptr[e + 1];
-                const int tl = (int)((s1 - s0 + W_BM - 1) / W_BM);
-                if (s < tl * cx) {
-                    const int full = max(1, (tl + 2) >> 2) - 1;          // strips of four in front of the last one
-                    int bl, rt;
-                    if (s < 4 * cx * full) {
-                        const int st = s / (4 * cx), r4 = s - st * 4 * cx;
-                        bl = r4 >> 2;
-                        rt = 4 * st + (r4 & 3);
-                    } else {
-                        const int r4 = s - 4 * cx * full, h = tl - 4 * full;
-                        bl = r4 / h;
-                        rt = 4 * full + (r4 - bl * h);
-                    }
-                    t.found = true;
-                    t.bx = bl * 8 + x;
-                    t.m_start = (int)s0 + rt * W_BM;
-                    t.m_end = min((int)s1, t.m_start + W_BM);
-                    break;
-                }
-                s -= tl * cx;
-                s0 = s1;
-            }
-        } else {
-            int tile = lin / gx, cum = 0;
-            t.bx = lin % gx;
-            for (; e < p.E; ++e) {
-                const int64_t s1 = p.seg_indptr[e + 1];
-                const int tl = (int)((s1 - s0 + W_BM - 1) / W_BM);
-                if (tile < cum + tl) { t.found = true; t.m_start = (int)s0 + (tile - cum) * W_BM; t.m_end = min((int)s1, t.m_start + W_BM); break; }
-                cum += tl;
-                s0 = s1;
-            }
+        // Two walks over the tiles, both segment by segment, long segments in strips of four row tiles (the last strip takes
+        // what is left, one to five), in every strip column tile by column tile with the row tiles of a column back to back:
+        // the workgroups that share a weight tile run at the same time on the L2 that holds it, and the 32 concurrent ones
+        // of an XCD share 8 weight tiles and 4 activation tiles.
+        // By columns: XCD x (workgroup id mod 8) owns the column tiles x, x + 8, ... of every segment.
+        // By segments: XCD x walks an eighth of the whole list, so an expert's weights and rows are read by one XCD (two
+        // where an eighth ends inside it).  
+        // Column counts that are multiples of eight go by columns: the XCDs then have the same mix of full and ragged tiles
+        // (4096 tokens, us per layer, by segments against by columns: 8 experts of 14336 1617, 1543; 16 experts 541, 529; 64
+        // experts of 1408, whose down projection has 8 column tiles, 367, 369).  Other counts go by segments, where the plain
+        // row-major walk reads every weight tile on several XCDs (64 experts of 1408, 11 column tiles of gate and up, 2727
+        // tokens: 420 row-major, 387 by segments; 4096 tokens 560, 516).
+        const int x = lin & 7;
+        const bool by_columns = gx % 8 == 0;
+        const int cx = by_columns ? gx >> 3 : gx;
+        int want = lin >> 3;
+        if (!by_columns) {
+            const int total = wide_total_tiles<GROUPED, R>(p, gx);
+            if (lin >= total) return t;
+            want += x * (total >> 3) + min(x, total & 7);
         }
-        t.e = e;
+        const SegmentTile sg = segment_of(p.seg_indptr, p.E, W_BM, cx, want);
+        if (!sg.found) return t;
+        const int tl = (sg.s1 - sg.s0 + W_BM - 1) / W_BM;
+        const int full = max(1, (tl + 2) >> 2) - 1;          // strips of four in front of the last one
+        int bl, rt;
+        if (sg.rest < 4 * cx * full) {
+            const int st = sg.rest / (4 * cx), r4 = sg.rest - st * 4 * cx;
+            bl = r4 >> 2;
+            rt = 4 * st + (r4 & 3);
+        } else {
+            const int r4 = sg.rest - 4 * cx * full, h = tl - 4 * full;
+            bl = r4 / h;
+            rt = 4 * full + (r4 - bl * h);
+        }
+        t.found = true;
+        t.bx = by_columns ? bl * 8 + x : bl;
+        t.m_start = sg.s0 + rt * W_BM;
+        t.m_end = min(sg.s1, t.m_start + W_BM);
+        t.e = sg.e;
     }
     return t;
-}
-
-// number of tiles of the launch (the valid linear ids are 0 .. total - 1 under both orders above)
-template <bool GROUPED, int R>
-__device__ __forceinline__ int wide_total_tiles(const DirectArgs& p, int gx) {
-    constexpr int W_BM = w_bm(R);
-    if constexpr (!GROUPED) return gx * ((p.M + W_BM - 1) / W_BM);
-    int rows = 0;
-    int64_t s0 = p.seg_indptr[0];
-    for (int e = 0; e < p.E; ++e) {
-        const int64_t s1 = p.seg_indptr[e + 1];
-        rows += (int)((s1 - s0 + W_BM - 1) / W_BM);
-        s0 = s1;
-    }
-    return rows * gx;
 }
 
 // A launch of `total` tiles runs in rounds of 256 (one workgroup per CU).  When the last round holds at most 128

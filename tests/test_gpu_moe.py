@@ -306,6 +306,34 @@ def test_grouped_gemm_split_last_round_exact(dev, M, N, K, E):
     assert torch.all(out[used:] == 5.0)
 
 
+@pytest.mark.parametrize("E", [1, 63, 64, 65, 128, 131])
+@pytest.mark.parametrize("rows,N,K", [(2, 48, 256), (40, 272, 256), (130, 768, 128), (300, 2304, 128), (300, 2048, 128)])
+def test_grouped_gemm_many_segments_exact(dev, E, rows, N, K):
+    """The lookup of a tile's segment over the edges of a wave's 64 segments, in every grouped kernel (16-row tiles, 64-
+    and 128-row tiles, the large tiles in both tile walks): empty segments first, last and in the middle, rows behind the
+    last segment keep their fill value.  Exact integers as above."""
+    announce("grouped many segments", E, rows, N, K)
+    torch.manual_seed(E + rows + N)
+    lens = torch.randint(0, 2 * rows, (E,))
+    lens[::7] = 0
+    lens[E // 2] = rows + 1
+    if E > 2:
+        lens[-1] = 0
+    seg = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    used = int(seg[-1])
+    M = used + 3
+    widx = torch.randperm(E)
+    a = torch.randint(-7, 8, (M, K), dtype=torch.int8)
+    b = torch.randint(-7, 8, (E, N, K), dtype=torch.int8)
+    c = torch.full((M, N), 5.0, dtype=torch.float32, device=dev)
+    _lib_call_grouped_i8(dev, a, torch.ones(M, K // 128), b, torch.ones(E, (N + 127) // 128, K // 128), c, seg, widx)
+    out = c.cpu()
+    for e in range(E):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        assert torch.equal(out[lo:hi], a[lo:hi].float() @ b[widx[e]].float().T), "segment %d" % e
+    assert torch.all(out[used:] == 5.0)
+
+
 def _lib_call_grouped_i8(dev, a, a_s, b, b_s, c, seg, widx):
     """grouped_gemm_triton on activations that are already int8 with their 1 x 128 scales."""
     d = [t.to(dev).contiguous() for t in (a, a_s, b, b_s, seg.long(), widx.long())]
