@@ -53,7 +53,7 @@ static int64_t workspace_core_bytes(int64_t M, int64_t N, int64_t K) {
     // large-M kernels stream fp32 activation scales; 16-bit scales are widened into the workspace first;
     // mid-size M with few tiles adds the fp32 split-K partials behind them
     if (K <= 0) return 0;
-    if (M <= 64 && !mid_m_prefers_tiles(M, N, K)) {
+    if (M <= 64 && !mid_m_prefers_tiles(M, N, K) && !mid_wanted(M, N, K)) {
         const int nz = stream_k_ranges(M, N, K);
         return nz > 1 ? (int64_t)nz * M * N * 4 : 0;
     }
@@ -79,7 +79,7 @@ extern "C" int llmk_gemm_fp8_block(const void* a, const float* a_s, const void* 
     DirectArgs p{};
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = LLMK_F32; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
-    if (M > 64 || (mid_m_prefers_tiles(M, N, K) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K)))
+    if (M > 64 || ((mid_m_prefers_tiles(M, N, K) || mid_wanted(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K)))
         return launch_big<K_FP8_BLOCK, false>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_fp8_block(tiled)");
     return launch_stream<K_FP8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_fp8_block");
 }
@@ -110,7 +110,7 @@ extern "C" int llmk_gemm_i8_block(const int8_t* a, const void* a_s, const int8_t
     DirectArgs p{};
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = s_dtype; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
-    if (M > 64 || (mid_m_prefers_tiles(M, N, K) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K)))
+    if (M > 64 || ((mid_m_prefers_tiles(M, N, K) || mid_wanted(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K)))
         return launch_big<K_I8_BLOCK, false>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_i8_block(tiled)");
     return launch_stream<K_I8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_i8_block");
 }
@@ -127,7 +127,10 @@ extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.c_i32 = c_i32; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = LLMK_F32; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
     // large M: the tile kernels accumulate int32 over the whole K range inside the MFMA and scale in the epilogue
-    if (M > 64 && dma_eligible(p)) {
+    // (from the rows that the mid-size kernel takes, and from 17 rows on large weights as for the block-scaled kinds: 64 x 4096
+    // x 14336 44.4 us on the weight-streaming kernel, 30.0 in K slices, 64 x 28672 x 4096 76.4 and 35.3)
+    if ((M > 64 || ((mid_wanted(M, N, K) || mid_m_prefers_tiles(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K))) &&
+        dma_eligible(p)) {
         // few tiles and a long K: K slices over the CUs, int32 partial sums in the workspace, one pass that adds
         // them as integers and scales (same bits as the unsplit kernel)
         if (mid_wanted(M, N, K)) {

@@ -643,7 +643,7 @@ inline int mid_splitk(int64_t tiles, int64_t kbytes) {
 }
 
 // Shape of a mid-size launch: tile height (16 mt rows) and K slices.  The 32-row tile when the 64-row tile would leave
-// more than half of the CUs without a workgroup.
+// more than half of the CUs without a workgroup, or would be half empty itself.
 struct MidPlan {
     int mt, z;
     int64_t tiles;
@@ -652,7 +652,7 @@ inline MidPlan mid_plan(int64_t M, int64_t N, int64_t kbytes) {
     MidPlan pl;
     const int64_t gx = (N + MD_BN - 1) / MD_BN;
     const int64_t t4 = ((M + 63) / 64) * gx, t2 = ((M + 31) / 32) * gx;
-    pl.mt = (t4 <= LLMK_CUS / 2 && t2 > t4) ? 2 : 4;
+    pl.mt = M <= 32 || (t4 <= LLMK_CUS / 2 && t2 > t4) ? 2 : 4;
     pl.tiles = pl.mt == 4 ? t4 : t2;
     pl.z = mid_splitk(pl.tiles, kbytes);
     return pl;

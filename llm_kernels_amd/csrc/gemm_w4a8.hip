@@ -472,9 +472,10 @@ W4A8Plan w4a8_plan(int64_t M, int64_t N, int64_t K, int group_int4) {
     const bool long_k_ok = pl.nz == 1 || row_blocks <= 2;
     // (the hand-issued loads of the fused kernel take 32-bit lane offsets into the activations and the tables)
     const bool small_offsets = M * K < (1ll << 32) && N * (K / 128) < (1ll << 32);
-    // 65 to 256 rows on at most one 64-column workgroup per CU: the tile kernel with 512-byte K steps
-    const bool mid = M > 64 && M <= 256 && mid_plan(M, N, K).tiles <= LLMK_CUS && K <= 16384;
-    pl.stream = fused_wins && long_k_ok && small_offsets && group_int4 == 128 && !mid;
+    // up to 256 rows on at most one 64-column workgroup per CU: the tile kernel with 512-byte K steps
+    const bool mid = mid_rows(M, N, K) && M <= 256 && mid_plan(M, N, K).tiles <= LLMK_CUS && K <= 16384;
+    // (up to 64 rows the fused kernel stays behind it for operands that the tile kernel does not take)
+    pl.stream = fused_wins && long_k_ok && small_offsets && group_int4 == 128 && !(mid && M > 64);
     // Mid-size M: the tile kernels unpack and dequantise inside their K loop (one pass over the packed words; the
     // separate expansion writes and re-reads N * K bytes).  Measured (us per launch, fused | expansion + int8 GEMM):
     // the 64-column kernel with 512-byte K steps on at most one workgroup per CU: 256 x 4096 x 4096 19.4 | 29.8,
@@ -482,10 +483,12 @@ W4A8Plan w4a8_plan(int64_t M, int64_t N, int64_t K, int group_int4) {
     // 128 x 4096 x 14336 41.2 | 46.5; from there on the two passes win (512 x 4096 x 4096 34 | 30, 512 x 14336 x 4096 80 | 60).
     DirectArgs q{};
     q.M = (int)M; q.N = (int)N; q.K = (int)K;
-    pl.tiles = !pl.stream && M > 64 && (mid || M <= 128) && group_int4 == 128 && N <= 0x7fffffff &&
+    pl.tiles = (mid || (!pl.stream && M > 64 && M <= 128)) && group_int4 == 128 && N <= 0x7fffffff &&
                K <= 0x7fffffff && dma_eligible(q);
-    if (pl.stream) pl.bytes = pl.nz > 1 ? pl.nz * M * N * 4 : 0;
-    else if (pl.tiles) pl.bytes = llmk_gemm_workspace_bytes(M, N, K);      // fp32 activation scales + split-K partial sums
+    const int64_t ranges = pl.stream && pl.nz > 1 ? pl.nz * M * N * 4 : 0;
+    const int64_t z = mid && M <= 64 ? mid_plan(M, N, K).z : 1, slices = z > 1 ? z * M * N * 4 : 0;
+    if (pl.tiles) pl.bytes = std::max({llmk_gemm_workspace_bytes(M, N, K), slices, ranges});      // fp32 activation scales + split-K partial sums
+    else if (pl.stream) pl.bytes = ranges;
     else pl.bytes = w4a8_two_pass_scales_off(N, K) + w4a8_widened_bytes(M, N, K) + llmk_gemm_workspace_bytes(M, N, K);
     return pl;
 }
@@ -531,7 +534,8 @@ extern "C" int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b
     if (!a || !a_s || !b_packed || !b_s || !b_s4 || !b_z4 || !c) LLMK_FAIL(LLMK_ERR_ARG, "gemm_w4a8: null pointer");
     const W4A8Plan pl = w4a8_plan(M, N, K, group_int4);
     const bool ranges_ok = pl.nz == 1 || (workspace && workspace_bytes >= pl.nz * M * N * 4 && !(((uintptr_t)workspace) & 15));
-    if (pl.stream && ranges_ok && !(((uintptr_t)a | (uintptr_t)b_packed) & 15)) {
+    const bool tiles_ok = pl.tiles && !(((uintptr_t)a | (uintptr_t)b_packed | (uintptr_t)workspace) & 15);
+    if (pl.stream && !tiles_ok && ranges_ok && !(((uintptr_t)a | (uintptr_t)b_packed) & 15)) {
         W4A8Args p{a, a_s, b_packed, b_s, b_s4, b_z4, c, c_dtype, (int)M, (int)N, (int)K, 0, nullptr};
         if (c_dtype != LLMK_F32 && c_dtype != LLMK_F16 && c_dtype != LLMK_BF16) LLMK_FAIL(LLMK_ERR_DTYPE, "gemm_w4a8: c_dtype %d", c_dtype);
         hipStream_t st = (hipStream_t)stream;
@@ -547,7 +551,7 @@ extern "C" int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b
 #undef LLMK_W4A8_MT
         LLMK_FAIL(LLMK_ERR_DTYPE, "gemm_w4a8: s_dtype %d", s_dtype);
     }
-    if (pl.tiles && !(((uintptr_t)a | (uintptr_t)b_packed | (uintptr_t)workspace) & 15)) {
+    if (tiles_ok) {
         if (!workspace) workspace_bytes = 0;                // no scratch: no K split, everything else as with it
         if (s_dtype != LLMK_F32 && s_dtype != LLMK_F16 && s_dtype != LLMK_BF16) LLMK_FAIL(LLMK_ERR_DTYPE, "gemm_w4a8: s_dtype %d", s_dtype);
         if (c_dtype != LLMK_F32 && c_dtype != LLMK_F16 && c_dtype != LLMK_BF16) LLMK_FAIL(LLMK_ERR_DTYPE, "gemm_w4a8: c_dtype %d", c_dtype);

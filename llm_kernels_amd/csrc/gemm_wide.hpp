@@ -742,14 +742,27 @@ inline int splitk_factor(int64_t M, int64_t N, int64_t K) {
     return (int)(z > 8 ? 8 : (z < 1 ? 1 : z));
 }
 
-// Shapes for the mid-size kernel (gemm_mid.hpp): more than 64 rows, at most one workgroup per CU and a K range of at
+// 16 < M <= 64: the weight-streaming kernel re-reads the activations for every 16 columns, which costs more
+// than the 64-row tile kernel (with split-K when its tiles are few) once the weight matrix is large (measured
+// crossover between 17 M and 25 M elements).
+inline bool mid_m_prefers_tiles(int64_t M, int64_t N, int64_t K) {
+    return M > 16 && M <= 64 && N * K >= (int64_t)20 << 20;
+}
+
+// Rows from which the mid-size kernels beat the weight-streaming ones: 33, and 17 on large weights (us per layer, quantiser
+// and GEMM, streaming or 64-row tiles | mid-size: fp8 64 x 14336 x 4096 28.4 | 23.0, 48 x 4096 x 4096 16.1 | 13.4, 20 x 14336
+// x 4096 23.0 | 20.2, but 20 x 4096 x 4096 11.2 | 12.7; per-token int8 64 x 15368 x 3072 48.7 | 21.9, 32 x 4096 x 4096 12.9 |
+// 15.0; w4a8 48 x 15368 x 3072 34.1 | 20.9, 32 x 4096 x 14336 27.9 | 23.0, 32 x 4096 x 4096 13.6 | 16.1).
+inline bool mid_rows(int64_t M, int64_t N, int64_t K) { return M > 32 || mid_m_prefers_tiles(M, N, K); }
+
+// Shapes for the mid-size kernel (gemm_mid.hpp): rows as above, at most one workgroup per CU and a K range of at
 // most 8 KB per row, 16 KB on the 64-row tile.  Measured against the 128-column tile kernels (fp8, us per launch, cold
 // weights): 128 x 4096 x 4096 16.7 -> 12.7, 256 x 4096 x 4096 23.1 -> 15.3, 256 x 4096 x 8192 28.7 -> 24.2,
 // 256 x 4096 x 14336 44.2 -> 39.0 (K slices of the 64 x 128 tile before); with more than one round of workgroups, or on
 // the 32-row tile with rows beyond 8 KB, it loses (512 x 4096 x 4096 15.5 -> 23.4, 256 x 6144 x 4096 23.5 -> 27.9,
 // 128 x 4096 x 14336 28.4 -> 29.2, per-token int8 26.2 -> 30.4).
 inline bool mid_wanted(int64_t M, int64_t N, int64_t kbytes) {
-    if (M <= 64 || M > 512) return false;
+    if (!mid_rows(M, N, kbytes) || M > 512) return false;
     const MidPlan pl = mid_plan(M, N, kbytes);
     return pl.tiles <= LLMK_CUS && kbytes <= (pl.mt == 4 ? 16384 : 8192);
 }
@@ -765,13 +778,6 @@ inline bool mid_wanted(int64_t M, int64_t N, int64_t kbytes) {
 inline bool midw_wanted(int64_t M, int64_t N, int64_t kbytes) {
     if (M <= 64 || M > 512 || kbytes > 16384) return false;
     return midw_plan(M, N, kbytes).tiles <= LLMK_CUS;
-}
-
-// 16 < M <= 64: the weight-streaming kernel re-reads the activations for every 16 columns, which costs more
-// than the 64-row tile kernel (with split-K when its tiles are few) once the weight matrix is large (measured
-// crossover between 17 M and 25 M elements).
-inline bool mid_m_prefers_tiles(int64_t M, int64_t N, int64_t K) {
-    return M > 16 && M <= 64 && N * K >= (int64_t)20 << 20;
 }
 
 // Tile shape by estimated time: rounds of 256 workgroups times the measured cost of one round of each tile

@@ -200,6 +200,8 @@ def test_w4a8_decode_exact_mixed_wrap(dev, M, N, K, sdt):
                                        (256, 1032, 2176, torch.bfloat16), (161, 8, 128, torch.float16),
                                        (250, 2048, 8192, torch.float16), (256, 264, 14336, torch.float32),
                                        (130, 4104, 4096, torch.bfloat16),
+                                       (17, 14336, 1536, torch.float16), (33, 8, 128, torch.float32), (64, 2048, 7168, torch.float16),
+                                       (32, 1600, 16384, torch.bfloat16), (48, 15368, 1408, torch.float32),
                                        # more than 256 tiles of 64 columns, up to 128 rows: the 128-column tile kernel
                                        (97, 9000, 4096, torch.float16), (128, 8200, 4224, torch.float32)])
 def test_w4a8_mid_m_fused_tiles_exact_mixed_wrap(dev, M, N, K, sdt):
@@ -271,7 +273,11 @@ def _random_mid_shapes(n, seed):
     return shapes
 
 
-@pytest.mark.parametrize("M,N,K", _random_mid_shapes(28, 7))
+@pytest.mark.parametrize("M,N,K", _random_mid_shapes(28, 7) + [
+    # 17 to 64 rows: the first rows and both tile heights of the mid-size kernels, K slices, ragged columns, and the shapes
+    # on either side of the row and weight-size rules that stay on the weight-streaming kernel or the 64-row tiles
+    (17, 14336, 1536), (32, 16384, 1280), (17, 14344, 1408), (32, 4096, 4096), (33, 8, 128), (33, 4104, 4096), (48, 520, 8192),
+    (64, 2048, 7168), (64, 15368, 3072), (64, 16392, 1280), (20, 3000, 14336), (64, 1030, 8320), (40, 72, 16384)])
 def test_mid_and_small_tile_kernels_exact_integers(dev, M, N, K):
     """Random mid-size shapes (ragged row and column tiles, K tails, split K, one or more rounds of tiles) with small
     integer operands, unit block scales of a random dtype and fp32 output: the block-scaled int8 and fp8 GEMMs and the
