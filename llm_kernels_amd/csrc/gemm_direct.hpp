@@ -196,7 +196,10 @@ inline int grouped_row_tiles(int M, int E, int tile_rows) {
 // VEC: the weight scales of a batch are one vector load (needs four steps per batch and steps % 4 == 0).
 // KR: blockIdx.z selects a K range of p.kc_steps steps (short enough for RESIDENT); the workgroup writes its
 // fp32 sums to p.partial[blockIdx.z] and a second kernel adds the ranges.
-template <int KIND, int MT, int NW, bool GROUPED, bool RESIDENT, int SDT, bool VEC = false, bool KR = false>
+// SU: K steps per wave and batch where K is short (1 to 3), 0: the number that goes with MT.  (16 rows, us per layer, four
+// steps against as many as needed: fp8 28672 x 1024 22.9 -> 12.2, 25728 x 1408 23.3 -> 16.1, 28672 x 2048 24.2 -> 18.1, 24000
+// x 2304 22.2 -> 19.4, 4096 x 1024 9.2 -> 6.3; per-token int8 28672 x 1024 23.7 -> 12.7.)
+template <int KIND, int MT, int NW, bool GROUPED, bool RESIDENT, int SDT, bool VEC = false, bool KR = false, int SU = 0>
 __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
     static_assert(!KR || (RESIDENT && !GROUPED && !VEC), "K ranges: dense, resident activations");
     typedef typename ScaleIO<SDT>::Raw SRaw;
@@ -243,7 +246,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
     // one batch (RESIDENT), the activation fragments are loaded once and reused for every column tile the
     // workgroup processes, and the weight batch of the next tile is requested before the current tile is
     // reduced; otherwise batches are double-buffered along K.
-    constexpr int U = MT == 1 ? 4 : (MT == 2 ? 2 : 1);
+    constexpr int U = SU ? SU : (MT == 1 ? 4 : (MT == 2 ? 2 : 1));
     struct BBatch {
         v8i b[U];
         SRaw bs[U];           // raw weight scales, converted when the batch is multiplied
@@ -540,20 +543,26 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
     // long K: consecutive steps per wave, one load for the four weight scales of a batch (measured faster at
     // K = 14336, slower at K = 4096 where the interleaved order spreads the first requests over more channels)
     const bool vec = CAN_VEC && !resident && steps % 4 == 0;
-    static std::atomic<int> slots_cache[2];   // resident workgroups on the whole device, per kernel variant
-    int slots[2] = {slots_cache[0].load(std::memory_order_relaxed), slots_cache[1].load(std::memory_order_relaxed)};
-    if (slots[resident] == 0) {
+    // short K: a batch of four steps per wave would mostly repeat the last step (K = 1408: 32 requests for 11 steps)
+    constexpr int SU1 = MT == 1 ? 1 : 0, SU2 = MT == 1 ? 2 : 0, SU3 = MT == 1 ? 3 : 0;
+    const int variant = MT == 1 && steps <= 3 * NW ? 2 + (steps + NW - 1) / NW : (resident ? 1 : 0);
+    static std::atomic<int> slots_cache[6];   // resident workgroups on the whole device, per kernel variant
+    int slots = slots_cache[variant].load(std::memory_order_relaxed);
+    if (slots == 0) {
         int dev = 0, cus = 0, per_cu = 0;
         hipError_t e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess)
-            e = resident ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT>, NW * 64, 64 * 1024)
-                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT>, NW * 64, 64 * 1024);
+            e = variant == 2 || variant == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1>, NW * 64, 64 * 1024)
+                : variant == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2>, NW * 64, 64 * 1024)
+                : variant == 5 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3>, NW * 64, 64 * 1024)
+                : resident ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT>, NW * 64, 64 * 1024)
+                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT>, NW * 64, 64 * 1024);
         if (e != hipSuccess) LLMK_FAIL(LLMK_ERR_LAUNCH, "%s: occupancy query failed: %s", name, hipGetErrorString(e));
-        slots[resident] = max(1, cus * max(1, per_cu));
-        slots_cache[resident].store(slots[resident], std::memory_order_relaxed);
+        slots = max(1, cus * max(1, per_cu));
+        slots_cache[variant].store(slots, std::memory_order_relaxed);
     }
-    int gx = min(ntiles, max(1, slots[resident] / min(mtiles, slots[resident])));
+    int gx = min(ntiles, max(1, slots / min(mtiles, slots)));
     // every workgroup the same number of column tiles (the slowest one sets the time): fewer workgroups
     // rather than a last round that only some of them take part in
     { const int per_wg = (ntiles + gx - 1) / gx; gx = (ntiles + per_wg - 1) / per_wg; }
@@ -565,7 +574,10 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
             return LLMK_OK;
         }
     }
-    if (resident) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT><<<grid, block, smem, stream>>>(p);
+    if (variant == 2 || variant == 3) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1><<<grid, block, smem, stream>>>(p);
+    else if (variant == 4) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2><<<grid, block, smem, stream>>>(p);
+    else if (variant == 5) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3><<<grid, block, smem, stream>>>(p);
+    else if (resident) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT><<<grid, block, smem, stream>>>(p);
     else gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT><<<grid, block, smem, stream>>>(p);
     LLMK_CHECK_LAUNCH(name);
     return LLMK_OK;

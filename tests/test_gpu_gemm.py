@@ -277,7 +277,9 @@ def _random_mid_shapes(n, seed):
     # 17 to 64 rows: the first rows and both tile heights of the mid-size kernels, K slices, ragged columns, and the shapes
     # on either side of the row and weight-size rules that stay on the weight-streaming kernel or the 64-row tiles
     (17, 14336, 1536), (32, 16384, 1280), (17, 14344, 1408), (32, 4096, 4096), (33, 8, 128), (33, 4104, 4096), (48, 520, 8192),
-    (64, 2048, 7168), (64, 15368, 3072), (64, 16392, 1280), (20, 3000, 14336), (64, 1030, 8320), (40, 72, 16384)])
+    (64, 2048, 7168), (64, 15368, 3072), (64, 16392, 1280), (20, 3000, 14336), (64, 1030, 8320), (40, 72, 16384),
+    # decode sizes on short K: one to four K steps per wave, whole and partial
+    (2, 8, 128), (1, 1000, 1024), (16, 4104, 1152), (5, 520, 2048), (16, 72, 2176), (1, 1000, 3072), (20, 264, 3200), (16, 28680, 1408)])
 def test_mid_and_small_tile_kernels_exact_integers(dev, M, N, K):
     """Random mid-size shapes (ragged row and column tiles, K tails, split K, one or more rounds of tiles) with small
     integer operands, unit block scales of a random dtype and fp32 output: the block-scaled int8 and fp8 GEMMs and the

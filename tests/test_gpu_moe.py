@@ -307,7 +307,7 @@ def test_grouped_gemm_split_last_round_exact(dev, M, N, K, E):
 
 
 @pytest.mark.parametrize("E", [1, 63, 64, 65, 128, 131])
-@pytest.mark.parametrize("rows,N,K", [(2, 48, 256), (40, 272, 256), (130, 768, 128), (300, 2304, 128), (300, 2048, 128)])
+@pytest.mark.parametrize("rows,N,K", [(2, 48, 256), (1, 48, 1280), (1, 48, 2176), (40, 272, 256), (130, 768, 128), (300, 2304, 128), (300, 2048, 128)])
 def test_grouped_gemm_many_segments_exact(dev, E, rows, N, K):
     """The lookup of a tile's segment over the edges of a wave's 64 segments, in every grouped kernel (16-row tiles, 64-
     and 128-row tiles, the large tiles in both tile walks): empty segments first, last and in the middle, rows behind the
