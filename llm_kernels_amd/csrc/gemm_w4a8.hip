@@ -71,9 +71,13 @@ struct W4A8Args {
     float* partial;     // more than one range: fp32 partial sums [gridDim.z][M][N], summed by a second kernel
 };
 
-template <int MT, int SDT, int ROUNDS>
+// U = K steps of a wave, 1 to 4, for K ranges of up to 1024 U: a tile costs its vector-ALU work per step of a wave (unpacking,
+// scaling), also for steps past the end of the range.  (16 rows, us per
+// layer, four steps against as many as needed: 28672 x 1024 22.2 -> 12.4, 25600 x 1408 22.8 -> 16.0, 4096 x 1024 10.0 -> 6.6,
+// 24000 x 2304 21.0 -> 18.5, 16000 x 3072 18.1 -> 15.6.)  A second workgroup per CU gains nothing (25600 x 1408, 30 rows: 20.0 -> 25.1).
+template <int MT, int SDT, int U>
 __global__ __launch_bounds__(512) void w4a8_stream_kernel(W4A8Args p) {
-    constexpr int NW = 8, U = 4, D = 3;
+    constexpr int NW = 8, D = 3, ROUNDS = U <= 2 ? 1 : 2;
     constexpr bool TAB_REGS = MT == 1;                    // per-row sums and scales in registers, else in LDS
     constexpr int ROWSTRIDE = ROUNDS * 8192 + 64;         // +64: the two packed rows of a tile start in different banks
     constexpr int TB = 2 * ROWSTRIDE;
@@ -181,16 +185,13 @@ __global__ __launch_bounds__(512) void w4a8_stream_kernel(W4A8Args p) {
     float ascale[U][MT];
     {
         constexpr int NY = (D - 1) * LPT;
-        static_assert(U == 4 && (MT == 1 || MT == 2), "the waits below are spelled out for these sizes");
-        if constexpr (MT == 1) {
-            ring_wait<NY>(alo[0][0], alo[1][0], alo[2][0], alo[3][0], ahi[0][0], ahi[1][0], ahi[2][0], ahi[3][0]);
-            ring_wait<NY>(araw[0][0], araw[1][0], araw[2][0], araw[3][0]);
-        } else {
-            ring_wait<NY>(alo[0][0], alo[1][0], alo[2][0], alo[3][0], ahi[0][0], ahi[1][0], ahi[2][0], ahi[3][0]);
-            ring_wait<NY>(alo[0][MT - 1], alo[1][MT - 1], alo[2][MT - 1], alo[3][MT - 1], ahi[0][MT - 1], ahi[1][MT - 1], ahi[2][MT - 1], ahi[3][MT - 1]);
-            ring_wait<NY>(araw[0][0], araw[1][0], araw[2][0], araw[3][0]);
-            ring_wait<NY>(araw[0][MT - 1], araw[1][MT - 1], araw[2][MT - 1], araw[3][MT - 1]);
-        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                ring_wait<NY>(alo[u][mt], ahi[u][mt]);
+                ring_wait<NY>(araw[u][mt]);
+            }
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -414,22 +415,21 @@ int launch_w4a8_stream(W4A8Args p, void* workspace, int64_t workspace_bytes, hip
             LLMK_FAIL(LLMK_ERR_ARG, "gemm_w4a8: K > 4096 needs %lld bytes of 16-byte aligned workspace", (long long)nz * p.M * p.N * 4);
         p.partial = (float*)workspace;
     }
-    const int steps = p.Kc >> 7, rounds = p.Kc * 4 > 8192 ? 2 : 1;
+    const int steps = p.Kc >> 7, per_wave = (steps + 7) / 8, rounds = per_wave <= 2 ? 1 : 2;
     const int ntiles = (p.N + 15) >> 4, mtiles = (p.M + 16 * MT - 1) / (16 * MT);
     const size_t smem = (size_t)2 * 8 * MT * 256 * 4 + (size_t)MT * 16 * steps * 8 + (size_t)2 * 2 * (rounds * 8192 + 64);
-    auto k1 = w4a8_stream_kernel<MT, SDT, 1>;
-    auto k2 = w4a8_stream_kernel<MT, SDT, 2>;
-    static std::atomic<uint64_t> cfg1{0}, cfg2{0};
-    if (int rc = llmk_reserve_lds((const void*)k1, 160 * 1024, cfg1, "gemm_w4a8")) return rc;
-    if (int rc = llmk_reserve_lds((const void*)k2, 160 * 1024, cfg2, "gemm_w4a8")) return rc;
+    void (*const kernels[4])(W4A8Args) = {w4a8_stream_kernel<MT, SDT, 1>, w4a8_stream_kernel<MT, SDT, 2>, w4a8_stream_kernel<MT, SDT, 3>,
+                                          w4a8_stream_kernel<MT, SDT, 4>};
+    const auto kern = kernels[per_wave - 1];
+    static std::atomic<uint64_t> configured[4];
+    if (int rc = llmk_reserve_lds((const void*)kern, 160 * 1024, configured[per_wave - 1], "gemm_w4a8")) return rc;
     const int cus = llmk_device_cus();
     if (cus <= 0) LLMK_FAIL(LLMK_ERR_LAUNCH, "gemm_w4a8: cannot query the device");
     const int rows = mtiles * nz;                                      // workgroup rows that share the column tiles
-    int gx = min(ntiles, max(1, cus / min(rows, cus)));                // one workgroup per CU (LDS bound)
+    int gx = min(ntiles, max(1, cus / min(rows, cus)));                // one workgroup per CU (see the kernel)
     { const int per_wg = (ntiles + gx - 1) / gx; gx = (ntiles + per_wg - 1) / per_wg; }   // equal tile counts
     dim3 grid((unsigned)gx, (unsigned)mtiles, (unsigned)nz);
-    if (rounds == 1) k1<<<grid, 512, smem, st>>>(p);
-    else k2<<<grid, 512, smem, st>>>(p);
+    kern<<<grid, 512, smem, st>>>(p);
     LLMK_CHECK_LAUNCH("gemm_w4a8(stream)");
     if (nz > 1) {
         const int64_t mn = (int64_t)p.M * p.N;

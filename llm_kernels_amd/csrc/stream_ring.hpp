@@ -79,6 +79,10 @@ __device__ __forceinline__ void ring_wait(v4i& a, v4i& b) {
     asm volatile("s_waitcnt vmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N) : "memory");
 }
 template <int N>
+__device__ __forceinline__ void ring_wait(int& a) {
+    asm volatile("s_waitcnt vmcnt(%1)" : "+v"(a) : "n"(N) : "memory");
+}
+template <int N>
 __device__ __forceinline__ void ring_wait(int& a, int& b, int& c) {
     asm volatile("s_waitcnt vmcnt(%3)" : "+v"(a), "+v"(b), "+v"(c) : "n"(N) : "memory");
 }

@@ -172,7 +172,9 @@ def test_w4a8_exact_and_wrap(dev):
     assert torch.equal(c.cpu().long(), a.long() @ b8.long().T)
 
 
-@pytest.mark.parametrize("M,N,K,sdt", [(16, 5000, 1024, torch.float16), (40, 8192, 4096, torch.float32),
+@pytest.mark.parametrize("M,N,K,sdt", [(16, 5000, 1024, torch.float16), (16, 4104, 128, torch.float32),
+                                       (3, 264, 1408, torch.bfloat16), (30, 1040, 1920, torch.float16),
+                                       (16, 72, 3072, torch.float32), (1, 8, 2176, torch.float16), (40, 8192, 4096, torch.float32),
                                        (3, 312, 384, torch.bfloat16), (16, 1032, 8320, torch.float16),
                                        (50, 264, 14336, torch.float32)])
 def test_w4a8_decode_exact_mixed_wrap(dev, M, N, K, sdt):
