@@ -558,12 +558,12 @@ __global__ __launch_bounds__(512) void w4a16_nk_stream_kernel(
 }
 
 // Ring variant of the weight-streaming kernel for 128-wide groups, at most 16 rows per workgroup and a K range
-// of 4 to 32 steps: wave w owns the four consecutive 128-K steps 4w .. 4w + 3 of every
+// of 4 to 32 steps: wave w owns U = ceil(steps / 8) consecutive 128-K steps from U w of every
 // 16-column tile, its activation fragments stay in registers, and the packed words and group scales of the
 // next DEPTH - 1 tiles are in flight in a ring of registers filled by hand-issued loads (see stream_ring.hpp:
 // one s_waitcnt per tile that leaves exactly the younger tiles outstanding).
-// Every wave loads four steps, so that one wait count serves all: where fewer are left in the range the share is moved
-// back to its last four steps (the repeated ones hit L2) and the steps that another wave owns count as zero activations
+// Every wave loads U steps, so that one wait count serves all: where fewer are left in the range the share is moved
+// back to its last U steps (the repeated ones hit L2) and the steps that another wave owns count as zero activations
 // and zero scales.  (Ranges that are no multiple of
 // 512 went through a bf16 copy of W, or the stream kernel for fp16; us per call, cold weights: bf16 3 x 4672 x 9088
 // 70.6 -> 14.8, 16 x 14336 x 2176 32.7 -> 11.7, 60 x 24000 x 3968 90.0 -> 36.7; fp16 15.1 -> 15.3, 13.2 -> 12.4, 50.2 -> 41.1.)
@@ -571,12 +571,14 @@ __global__ __launch_bounds__(512) void w4a16_nk_stream_kernel(
 // seven mantissa bits, q < 16), and the missing "- 136" of every product is the accumulator the MFMA chain of a
 // step starts from: -136 * sum_k a[m][k] over the step, computed once per wave with the same MFMA and a weight
 // fragment of constant 136 (the same for every tile).
-template <int DEPTH, bool BF = false>
+// (U = 4 for every K before; us per call: 16 x 28672 x 1024 13.6 -> 6.9, fp16 60 x 28672 x 1024 43.2 -> 15.6, 16 x 25600 x 1408
+// 13.9 -> 9.4, 16 x 4096 x 1024 5.2 -> 3.3, 60 x 15368 x 3072 25.0 -> 20.4, 3 x 4672 x 9088 in three ranges 14.9 -> 12.8.)
+template <int DEPTH, int U, bool BF = false>
 __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     const unsigned short* __restrict__ A, const int32_t* __restrict__ B, const _Float16* __restrict__ S,
     unsigned short* __restrict__ C, int M, int N, int Kfull, int Kc, float* __restrict__ partial) {
     using namespace llmk;
-    constexpr int NW = 8, LPT = 5;                       // loads per tile and lane: four word vectors + the scales
+    constexpr int NW = 8, LPT = U + 1;                   // loads per tile and lane: U word vectors + the scales
     extern __shared__ float red[];                       // [2][NW][64][4]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -585,39 +587,40 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     const int steps = K >> 7, ngroups = Kfull >> 7, kwords = Kfull >> 3;
     const int m0 = blockIdx.y * 16;
     const int ntiles = (N + 15) >> 4;
-    const int s0 = min(4 * wave, steps - 4);             // first step this wave loads
-    const int u0 = min(4 * wave - s0, 4);                // steps s0 .. s0 + u0 - 1 belong to other waves
+    const int s0 = min(U * wave, steps - U);             // first step this wave loads
+    const int u0 = min(U * wave - s0, U);                // steps s0 .. s0 + u0 - 1 belong to other waves
 
     // ---- activations, requested first: row i of the wave's K slice (512 elements = 1 KiB) is one fully
     // coalesced load.  (Fetching the MFMA fragments straight from global memory costs 2 us per launch: every
     // 16-lane group of such a load touches 16 different cache lines, 16 bytes of each.)  They pass through a
     // wave-private LDS area once and stay in registers as fragments for every tile.
-    v4i a[16];
+    v4i a[4 * U];
     {
         // load 4 u + q: rows 4 q .. 4 q + 3 of the 256-byte slab of step u (a 16-lane group reads 256 contiguous bytes)
         const RingBase ab = ring_base((const char*)A + ((int64_t)k0 + s0 * 128) * 2);
         const uint32_t rowb = (uint32_t)(Kfull * 2), lrow = (uint32_t)(lane >> 4), lcol = 16u * (uint32_t)(lane & 15);
 #define LLMK_LDA(u, q) a[4 * u + q] = ring_load_b128<u * 256>((uint32_t)min(m0 + 4 * q + (int)lrow, M - 1) * rowb + lcol, ab)
         LLMK_LDA(0, 0); LLMK_LDA(0, 1); LLMK_LDA(0, 2); LLMK_LDA(0, 3);
-        LLMK_LDA(1, 0); LLMK_LDA(1, 1); LLMK_LDA(1, 2); LLMK_LDA(1, 3);
-        LLMK_LDA(2, 0); LLMK_LDA(2, 1); LLMK_LDA(2, 2); LLMK_LDA(2, 3);
-        LLMK_LDA(3, 0); LLMK_LDA(3, 1); LLMK_LDA(3, 2); LLMK_LDA(3, 3);
+        if constexpr (U > 1) { LLMK_LDA(1, 0); LLMK_LDA(1, 1); LLMK_LDA(1, 2); LLMK_LDA(1, 3); }
+        if constexpr (U > 2) { LLMK_LDA(2, 0); LLMK_LDA(2, 1); LLMK_LDA(2, 2); LLMK_LDA(2, 3); }
+        if constexpr (U > 3) { LLMK_LDA(3, 0); LLMK_LDA(3, 1); LLMK_LDA(3, 2); LLMK_LDA(3, 3); }
 #undef LLMK_LDA
     }
     // ---- ring of weight tiles
-    v4i w[DEPTH][4];
+    v4i w[DEPTH][U];
     v2i sv[DEPTH];
     const char* bb = (const char*)B + ((int64_t)(k0 >> 3) + s0 * 16) * 4;
-    const char* sb = (const char*)S + ((int64_t)(k0 >> 7) + s0) * 2;
-    auto issue = [&](v4i (&tw)[4], v2i& ts, int tile) __attribute__((always_inline)) {
+    const int sq = U == 4 ? s0 : min(s0, steps - 4);                   // the scales of four steps are loaded, this wave's among them
+    const char* sb = (const char*)S + ((int64_t)(k0 >> 7) + sq) * 2;
+    auto issue = [&](v4i (&tw)[U], v2i& ts, int tile) __attribute__((always_inline)) {
         const int rowbase = tile * 16;
         const uint32_t row = (uint32_t)min(r, N - 1 - rowbase);             // rows past N repeat the last row
         const uint32_t vo = row * (uint32_t)(kwords * 4) + 16u * (uint32_t)g;
         const RingBase tb = ring_base(bb + (int64_t)rowbase * kwords * 4);
         tw[0] = ring_load_b128<0>(vo, tb);
-        tw[1] = ring_load_b128<64>(vo, tb);
-        tw[2] = ring_load_b128<128>(vo, tb);
-        tw[3] = ring_load_b128<192>(vo, tb);
+        if constexpr (U > 1) tw[1] = ring_load_b128<64>(vo, tb);
+        if constexpr (U > 2) tw[2] = ring_load_b128<128>(vo, tb);
+        if constexpr (U > 3) tw[3] = ring_load_b128<192>(vo, tb);
         ts = ring_load_b64<0>(row * (uint32_t)(ngroups * 2), ring_base(sb + (int64_t)rowbase * ngroups * 2));
     };
     int tile = blockIdx.x;
@@ -625,14 +628,15 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; ++d) issue(w[d], sv[d], min(tile + d * stride, last));
     // the activations were requested before (DEPTH - 1) * LPT ring loads
-    ring_wait16<(DEPTH - 1) * LPT>(a);
+#pragma unroll
+    for (int i = 0; i < 4 * U; ++i) ring_wait<(DEPTH - 1) * LPT>(a[i]);
     {
         // one slab (16 rows x 256 bytes) at a time through the wave's LDS area; rows of 256 + 16 bytes, so that
         // the 16 rows of a fragment read fall into 16 different bank groups
         constexpr int AROW = 256 + 16;
         uint8_t* stage = (uint8_t*)red + 2 * NW * 256 * sizeof(float) + wave * (16 * AROW);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) *(v4i*)(stage + (4 * q + (lane >> 4)) * AROW + 16 * (lane & 15)) = a[4 * u + q];
             // fragment (u, j) of lane (r, g): elements 128 u + 32 g + 8 j .. + 7 of row r.  The k order of a
@@ -650,21 +654,21 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
         }
         if (u0 > 0) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
+            for (int i = 0; i < 4 * U; ++i)
                 if (i < 4 * u0) a[i] = (v4i){0, 0, 0, 0};
         }
     }
 
     // bf16: the bias of step u, -136 * sum_k a[row][k] in every column of the MFMA result
-    v4f bias[4];
+    v4f bias[U];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) bias[u] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < U; ++u) bias[u] = (v4f){0.f, 0.f, 0.f, 0.f};
     if constexpr (BF) {
         const v4i c136 = {(int)0xc308c308u, (int)0xc308c308u, (int)0xc308c308u, (int)0xc308c308u};   // bf16 -136
         v8bf neg136;
         __builtin_memcpy(&neg136, &c136, 16);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 v8bf af;
@@ -674,11 +678,13 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     }
 
     int parity = 0;
-    auto tile_done = [&](const v4i (&tw)[4], const v2i& ts, int tl) __attribute__((always_inline)) {
+    auto tile_done = [&](const v4i (&tw)[U], const v2i& ts, int tl) __attribute__((always_inline)) {
         v4f acc = {0.f, 0.f, 0.f, 0.f};
+        uint64_t sc4 = 0;
+        if constexpr (U < 4) sc4 = ((uint64_t)(uint32_t)ts[1] << 32 | (uint32_t)ts[0]) >> (16 * (s0 - sq));
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const unsigned sraw = ((unsigned)(u < 2 ? ts[0] : ts[1]) >> (16 * (u & 1))) & 0xffffu;
+        for (int u = 0; u < U; ++u) {
+            const unsigned sraw = (U < 4 ? (unsigned)(sc4 >> (16 * u)) : (unsigned)(u < 2 ? ts[0] : ts[1]) >> (16 * (u & 1))) & 0xffffu;
             const float sc = u < u0 ? 0.f : f16_to_f32((unsigned short)sraw);
             v4f t = bias[u];
 #pragma unroll
@@ -731,16 +737,25 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     // my_tiles % DEPTH tiles, all requested by then, follow as straight-line code.  Requests past the last tile
     // of the workgroup are clamped to the last tile of the matrix (cache hits) and never consumed.
     const int my_tiles = (ntiles - (int)blockIdx.x + stride - 1) / stride;
+    auto landed = [&](auto nc, v4i (&tw)[U], v2i& ts) __attribute__((always_inline)) {
+        if constexpr (U == 4) {
+            ring_wait<decltype(nc)::value>(tw[0], tw[1], tw[2], tw[3], ts);
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) ring_wait<decltype(nc)::value>(tw[u]);
+            ring_wait<decltype(nc)::value>(ts);
+        }
+    };
     auto slot = [&](auto dc) __attribute__((always_inline)) {
         constexpr int d = decltype(dc)::value, NEXT = DEPTH - 1;
         issue(w[(d + NEXT) % DEPTH], sv[(d + NEXT) % DEPTH], min(tile + NEXT * stride, last));
-        ring_wait<(DEPTH - 1) * LPT>(w[d][0], w[d][1], w[d][2], w[d][3], sv[d]);
+        landed(std::integral_constant<int, (DEPTH - 1) * LPT>{}, w[d], sv[d]);
         tile_done(w[d], sv[d], tile);
         tile += stride;
     };
     auto tail = [&](auto dc) __attribute__((always_inline)) {
         constexpr int d = decltype(dc)::value;
-        ring_wait<(DEPTH - 2 - d) * LPT>(w[d][0], w[d][1], w[d][2], w[d][3], sv[d]);
+        landed(std::integral_constant<int, (DEPTH - 2 - d) * LPT>{}, w[d], sv[d]);
         tile_done(w[d], sv[d], tile);
         tile += stride;
     };
@@ -783,15 +798,17 @@ int launch_nk_ring(const void* A, const int32_t* B, const _Float16* S, void* C, 
     const unsigned short* a16 = (const unsigned short*)A;
     unsigned short* c16 = (unsigned short*)C;
     float* part = nz > 1 ? partial : nullptr;
-#define LLMK_RING(D)                                                                                             \
-    do {                                                                                                         \
-        if (bf) w4a16_nk_ring_kernel<D, true><<<rgrid, 512, rsmem, st>>>(a16, B, S, c16, M, N, K, Kc, part);      \
-        else w4a16_nk_ring_kernel<D, false><<<rgrid, 512, rsmem, st>>>(a16, B, S, c16, M, N, K, Kc, part);        \
-    } while (0)
-    if (per_wg >= 4) LLMK_RING(4);
-    else if (per_wg == 3) LLMK_RING(3);
-    else LLMK_RING(2);
-#undef LLMK_RING
+    auto ring = [&](auto uc) {
+        constexpr int U = decltype(uc)::value;
+        auto run = [&](auto kern) { kern<<<rgrid, 512, rsmem, st>>>(a16, B, S, c16, M, N, K, Kc, part); };
+        if (per_wg >= 4) bf ? run(w4a16_nk_ring_kernel<4, U, true>) : run(w4a16_nk_ring_kernel<4, U, false>);
+        else if (per_wg == 3) bf ? run(w4a16_nk_ring_kernel<3, U, true>) : run(w4a16_nk_ring_kernel<3, U, false>);
+        else bf ? run(w4a16_nk_ring_kernel<2, U, true>) : run(w4a16_nk_ring_kernel<2, U, false>);
+    };
+    if (steps <= 8) ring(std::integral_constant<int, 1>{});
+    else if (steps <= 16) ring(std::integral_constant<int, 2>{});
+    else if (steps <= 24) ring(std::integral_constant<int, 3>{});
+    else ring(std::integral_constant<int, 4>{});
     LLMK_CHECK_LAUNCH("gemm_w4a16_nk(ring)");
     if (nz > 1) {
         const int64_t mn = (int64_t)M * N;
