@@ -40,7 +40,9 @@ __device__ __forceinline__ int64_t ld_id(const void* p, int64_t i, int bytes) {
 // chunk + its rank among the equal ids of its own wave.  No workgroup waits for another.
 // Bound by latency: a chain of one load, three barriers and a scan.  Few buckets are counted in 64 columns per bucket, one
 // per lane, so that the ids of a wave never meet on one LDS address (ballots per bucket, the form before, took
-// 12.2 us for 8192 ids of 8 experts, this one 8.9); 65 to 256 ids get a workgroup of 256.
+// 12.2 us for 8192 ids of 8 experts, this one 8.4); 65 to 256 ids get a workgroup of 256.  What is left grows with the list: a
+// workgroup's LDS additions, about one a clock (21816 ids of 64 experts 18.2 us, 32768 22.2; 23.4 and 26.2 with half the loads
+// in flight and a pass per distinct bucket in the ranking).
 constexpr int PP_THREADS = 1024, PP_MAX_EXPERTS = 512, PP_BUCKETS = PP_MAX_EXPERTS + 2, PP_FEW = 66;
 
 template <int THREADS>
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __re
     for (int k = tid; k < nb; k += THREADS) { tot[k] = 0; pre[k] = 0; }
     if (few) for (int i = tid; i < nb * 64; i += THREADS) cells[i] = 0;
     __syncthreads();
-    constexpr int U = 4;                 // rounds whose loads are in flight together
+    constexpr int U = 8;                 // rounds whose loads are in flight together
     for (int r0 = 0; r0 < n; r0 += U * THREADS) {
         int v[U];
 #pragma unroll
@@ -118,18 +120,15 @@ __global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __re
         for (int e = tid; e <= E; e += THREADS) seg_indptr[e] = e == 0 ? 0 : (int64_t)tot[e + 1];
 
     // rank of a lane among the lanes of its wave with the same bucket, one leader per bucket publishes the count
-    int rank = 0;
-    uint64_t todo = __ballot(b >= 0);
-    while (todo) {                                       // one pass per distinct bucket of the wave
-        const int l = __ffsll((unsigned long long)todo) - 1;
-        const int v = __builtin_amdgcn_readlane(b, l);
-        const uint64_t m = __ballot(b == v);
-        if (b == v) {
-            rank = __popcll(m & ((1ull << lane) - 1ull));
-            if (lane == l) cells[wave * nb + b] = __popcll(m);
-        }
-        todo &= ~m;
+    // (one ballot per bit of the bucket number; a pass per distinct bucket of the wave is up to 64 of them with 64 experts)
+    uint64_t same = __ballot(b >= 0);
+    for (int bit = 0; nb >> bit; ++bit) {
+        const bool one = (b >> bit) & 1;
+        const uint64_t m = __ballot(one);
+        same &= one ? m : ~m;
     }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    if (b >= 0 && rank == 0) cells[wave * nb + b] = __popcll(same);
     if constexpr (WAVES > 1) __syncthreads();
     if (b >= 0) {
         int pos = tot[b] + pre[b] + rank;
