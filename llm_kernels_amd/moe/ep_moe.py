@@ -26,13 +26,20 @@ ROUTER_MAX_EXPERTS = 512
 ROUTER_MAX_TOPK = 64
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """A tensor that nothing but eager execution looks at: no subclass, transform (vmap, grad, forward mode), tracer or mode."""
+    return (type(t) is torch.Tensor and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t) and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None)
+
+
 def softmax_topk_router(router_logits: torch.Tensor, top_k: int = 2, renormalize: bool = True):
     """softmax over the experts in fp32 and its top_k: (ids int64, weights fp32) [.., top_k], largest first."""
-    if (router_logits.is_cuda and router_logits.dtype in (torch.float32, torch.float16, torch.bfloat16)
-            and 0 < top_k <= ROUTER_MAX_TOPK and top_k <= router_logits.shape[-1] <= ROUTER_MAX_EXPERTS
-            and not (router_logits.requires_grad and torch.is_grad_enabled())):
+    if (not torch.compiler.is_compiling() and _plain(router_logits) and router_logits.is_cuda
+            and router_logits.device.index == torch.cuda.current_device() and router_logits.dtype in (torch.float32, torch.float16, torch.bfloat16)
+            and 0 < top_k <= ROUTER_MAX_TOPK and top_k <= router_logits.shape[-1] <= ROUTER_MAX_EXPERTS):
         return _lib.host.softmax_topk(router_logits, top_k, renormalize)
-    # host tensors, training and larger routers
+    # host tensors, other devices than the current one, training, transforms, tracing and larger routers
     p = torch.softmax(router_logits.float(), dim=-1)
     w, ids = torch.topk(p, top_k, dim=-1)
     if renormalize:

@@ -42,6 +42,31 @@ def test_router_in_one_launch(dev, dtype, T, E, topk):
         assert torch.allclose(w.cpu().double(), ref, rtol=48 * 2 ** -24, atol=0)
 
 
+def test_router_under_transforms_and_tracing(dev):
+    """vmap, forward mode, functional gradients and tracing see the router's tensor operations, on the device as on the host."""
+    import torch.autograd.forward_ad as fwd
+    from torch.fx.experimental.proxy_tensor import make_fx
+    announce("router transforms")
+    torch.manual_seed(0)
+    x, d = torch.randn(3, 5, 8), torch.randn(3, 5, 8)
+
+    def weights(t):
+        return softmax_topk_router(t, 2)[1]
+
+    def check(f):
+        assert torch.allclose(f(x.to(dev), d.to(dev)).cpu(), f(x, d), rtol=1e-5, atol=1e-6)
+
+    check(lambda t, _: torch.func.vmap(weights)(t))
+    check(lambda t, _: torch.func.grad(lambda v: (weights(v) ** 2).sum())(t))
+    check(lambda t, u: torch.func.jvp(weights, (t,), (u,))[1])
+    check(lambda t, _: make_fx(weights)(t)(t + 1))
+
+    def dual(t, u):
+        with fwd.dual_level():
+            return fwd.unpack_dual(weights(fwd.make_dual(t, u))).tangent
+    check(dual)
+
+
 def test_router_breaks_ties_by_index(dev):
     announce("router ties")
     ids, w = softmax_topk_router(torch.zeros(5, 12, device=dev), 3)
