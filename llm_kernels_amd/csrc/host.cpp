@@ -6,6 +6,10 @@
 // 21 us of host time for 9 us of kernels), so the host was what such a layer ran at.  Here a call costs about 1 us
 // beside the launches themselves.  The library is still reached only through include/llmk.h: bind() resolves the entry
 // points of the library that the ctypes binding loaded.
+//
+// A function reads its arguments under the interpreter's lock and gives the lock up for everything that may wait:
+// allocations, conversions of an operand, and the launches (a full queue, code that is loaded on first use).  Other Python
+// threads run meanwhile, this function's other callers among them, so no two calls under way share scratch (see Scratch).
 #include <dlfcn.h>
 #include <string>
 #include <torch/csrc/Exceptions.h>
@@ -38,12 +42,13 @@ struct State {
 #undef X
 };
 
-struct Raised {};           // a Python exception is set
+// Ends a call with a Python exception; call() sets it, with the interpreter's lock held again (no type: it is set already).
+struct Raised {
+    PyObject* type = nullptr;
+    std::string msg;
+};
 
-[[noreturn]] void raise(PyObject* type, const std::string& msg) {
-    PyErr_SetString(type, msg.c_str());
-    throw Raised{};
-}
+[[noreturn]] void raise(PyObject* type, std::string msg) { throw Raised{type, std::move(msg)}; }
 inline void require(bool ok, const char* msg) {
     if (!ok) raise(PyExc_AssertionError, msg);
 }
@@ -113,26 +118,64 @@ inline int64_t rows_of(const at::Tensor& t, int64_t cols) {
     return t.numel() / cols;
 }
 
-// the scratch buffer of (device, stream), grown on demand: the same dictionary as the Python side's workspace()
-void* workspace(const Args& a, const at::Tensor& like, int64_t bytes) {
-    if (bytes <= 0) return nullptr;
-    const int dev = like.device().index();
-    PyObject* key = Py_BuildValue("(iK)", dev, (unsigned long long)(uintptr_t)stream_of(like));
-    if (!key) throw Raised{};
-    PyObject* held = PyDict_GetItemWithError(a.st->workspaces, key);
-    if (held && THPVariable_Check(held) && THPVariable_Unpack(held).numel() >= bytes) {
-        Py_DECREF(key);
-        return THPVariable_Unpack(held).data_ptr();
-    }
-    at::Tensor buf = empty({std::max<int64_t>(bytes, 1 << 20)}, at::kByte, like);
-    void* p = buf.data_ptr();
-    PyObject* obj = THPVariable_Wrap(std::move(buf));
-    const int rc = obj ? PyDict_SetItem(a.st->workspaces, key, obj) : -1;
-    Py_XDECREF(obj);
-    Py_DECREF(key);
-    if (rc) throw Raised{};
-    return p;
+// f() without the interpreter's lock: nothing in it touches a Python object
+template <class F> auto unlocked(F&& f) {
+    struct Release {
+        PyThreadState* ts = PyEval_SaveThread();
+        ~Release() { PyEval_RestoreThread(ts); }
+    } release;
+    return f();
 }
+
+// Scratch of one call: taken out of the dictionary {(device, stream): uint8 tensor} for as long as the call lasts, and put
+// back once its launches are queued.  Calls on one stream run one after the other there, so the next one may have the same
+// buffer; a call that another thread makes on that stream meanwhile finds none and allocates its own, because the launches
+// of the two may alternate.  Of two buffers that come back the larger one is kept.
+// (Made and destroyed under the interpreter's lock, get() anywhere.)
+class Scratch {
+    const Args& a;
+    const at::Tensor& like;
+    const int64_t need;
+    PyObject *key = nullptr, *held = nullptr;            // held: the dictionary's tensor, this call's while it lasts
+    at::Tensor fresh;                                    // or one of its own
+
+    static int64_t size(PyObject* o) { return o && THPVariable_Check(o) ? THPVariable_Unpack(o).numel() : 0; }
+
+public:
+    Scratch(const Args& args, const at::Tensor& t, int64_t bytes) : a(args), like(t), need(std::max<int64_t>(bytes, 0)) {
+        if (!need) return;
+        key = Py_BuildValue("(iK)", (int)t.device().index(), (unsigned long long)(uintptr_t)stream_of(t));
+        if (!key) throw Raised{};
+        PyObject* o = PyDict_GetItemWithError(a.st->workspaces, key);
+        if (!o) {
+            PyErr_Clear();
+            return;
+        }
+        if (size(o) >= need) Py_INCREF(held = o);
+        PyDict_DelItem(a.st->workspaces, key);           // one that is too small goes before its successor is allocated
+    }
+    Scratch(const Scratch&) = delete;
+    ~Scratch() {
+        if (!key) return;
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        if (fresh.defined()) held = THPVariable_Wrap(std::move(fresh));
+        if (held && size(PyDict_GetItemWithError(a.st->workspaces, key)) < size(held)) PyDict_SetItem(a.st->workspaces, key, held);
+        PyErr_Clear();                                   // a buffer that cannot be kept is freed, and the next call allocates
+        Py_XDECREF(held);
+        Py_DECREF(key);
+        PyErr_Restore(type, value, trace);
+    }
+    void* get() {
+        if (!need) return nullptr;
+        if (held) return THPVariable_Unpack(held).data_ptr();
+        if (!fresh.defined()) fresh = empty({std::max<int64_t>(need, 1 << 20)}, at::kByte, like);
+        return fresh.data_ptr();
+    }
+    // the size asked for, not the size of the buffer: what a kernel does with its scratch (K splits) then depends on the
+    // shape alone, never on what an earlier call left behind
+    int64_t bytes() const { return need; }
+};
 
 PyObject* wrap(at::Tensor t) {
     PyObject* o = THPVariable_Wrap(std::move(t));
@@ -162,17 +205,20 @@ PyObject* act_quant(const Args& a) {
     a.on_gpu(x);
     const int dt = float_code(x.scalar_type());
     const bool fp8 = form == 0 || form == 4;
-    at::Tensor y = empty(x.sizes(), fp8 ? at::kFloat8_e4m3fn : at::kChar, x);
-    at::Tensor s = empty(with_last(x, cols / block), form == 0 ? at::kFloat : at::kHalf, x);
     const int64_t groups = x.numel() / block;
-    if (form == 0)
-        a.check(a.st->llmk_act_quant_fp8(x.data_ptr(), dt, y.data_ptr(), (float*)s.data_ptr(), groups, (int)block, stream_of(x)), "llmk_act_quant_fp8");
-    else if (form == 4)
-        a.check(a.st->llmk_comm_quant_fp8(x.data_ptr(), dt, y.data_ptr(), s.data_ptr(), LLMK_F16, groups, (int)block, stream_of(x)), "llmk_comm_quant_fp8", PyExc_AssertionError);
-    else
-        a.check(a.st->llmk_act_quant_i8(x.data_ptr(), dt, (int8_t*)y.data_ptr(), s.data_ptr(), groups, (int)block,
-                                        form == 1 ? LLMK_ROUND_HALF_AWAY : LLMK_ROUND_HALF_UP, stream_of(x)),
-                "llmk_act_quant_i8", form == 3 ? PyExc_AssertionError : nullptr);
+    at::Tensor y, s;
+    unlocked([&] {
+        y = empty(x.sizes(), fp8 ? at::kFloat8_e4m3fn : at::kChar, x);
+        s = empty(with_last(x, cols / block), form == 0 ? at::kFloat : at::kHalf, x);
+        if (form == 0)
+            a.check(a.st->llmk_act_quant_fp8(x.data_ptr(), dt, y.data_ptr(), (float*)s.data_ptr(), groups, (int)block, stream_of(x)), "llmk_act_quant_fp8");
+        else if (form == 4)
+            a.check(a.st->llmk_comm_quant_fp8(x.data_ptr(), dt, y.data_ptr(), s.data_ptr(), LLMK_F16, groups, (int)block, stream_of(x)), "llmk_comm_quant_fp8", PyExc_AssertionError);
+        else
+            a.check(a.st->llmk_act_quant_i8(x.data_ptr(), dt, (int8_t*)y.data_ptr(), s.data_ptr(), groups, (int)block,
+                                            form == 1 ? LLMK_ROUND_HALF_AWAY : LLMK_ROUND_HALF_UP, stream_of(x)),
+                    "llmk_act_quant_i8", form == 3 ? PyExc_AssertionError : nullptr);
+    });
     return wrap_all(std::move(y), std::move(s));
 }
 
@@ -181,12 +227,15 @@ PyObject* rowwise_quant(const Args& a) {
     require(x.is_contiguous(), "Input tensor must be contiguous");
     a.on_gpu(x);
     const at::ScalarType t = x.scalar_type();
-    if (t != at::kFloat && t != at::kHalf && t != at::kBFloat16) x = x.to(at::kFloat);
-    const int64_t cols = last_size(x), rows = cols ? x.numel() / cols : 0;
-    at::Tensor y = empty(x.sizes(), at::kChar, x);
-    at::Tensor s = empty(x.sizes().slice(0, x.dim() - 1), at::kFloat, x);
-    a.check(a.st->llmk_quant_i8_rowwise(x.data_ptr(), float_code(x.scalar_type()), (int8_t*)y.data_ptr(), (float*)s.data_ptr(), rows, cols, stream_of(x)),
-            "llmk_quant_i8_rowwise");
+    at::Tensor y, s;
+    unlocked([&] {
+        if (t != at::kFloat && t != at::kHalf && t != at::kBFloat16) x = x.to(at::kFloat);
+        const int64_t cols = last_size(x), rows = cols ? x.numel() / cols : 0;
+        y = empty(x.sizes(), at::kChar, x);
+        s = empty(x.sizes().slice(0, x.dim() - 1), at::kFloat, x);
+        a.check(a.st->llmk_quant_i8_rowwise(x.data_ptr(), float_code(x.scalar_type()), (int8_t*)y.data_ptr(), (float*)s.data_ptr(), rows, cols, stream_of(x)),
+                "llmk_quant_i8_rowwise");
+    });
     return wrap_all(std::move(y), std::move(s));
 }
 
@@ -201,10 +250,14 @@ PyObject* weight_quant(const Args& g) {
     if (block == 0) raise(PyExc_ZeroDivisionError, "integer division or modulo by zero");
     const int dt = float_code(x.scalar_type());
     const int64_t N = x.size(0), K = x.size(1), nb = std::max<int64_t>(0, (N + block - 1) / block), kb = std::max<int64_t>(0, (K + block - 1) / block);
-    at::Tensor y = empty(x.sizes(), fp8 ? at::kFloat8_e4m3fn : at::kChar, x), s = empty({nb, kb}, fp8 ? at::kFloat : at::kHalf, x);
-    if (fp8) g.check(g.st->llmk_weight_quant_fp8_block(x.data_ptr(), dt, y.data_ptr(), (float*)s.data_ptr(), N, K, (int)block, stream_of(x)), "llmk_weight_quant_fp8_block");
-    else g.check(g.st->llmk_weight_quant_i8_block(x.data_ptr(), dt, (int8_t*)y.data_ptr(), s.data_ptr(), N, K, (int)block, 127.f, LLMK_ROUND_HALF_AWAY, 0, stream_of(x)),
-                 "llmk_weight_quant_i8_block");
+    at::Tensor y, s;
+    unlocked([&] {
+        y = empty(x.sizes(), fp8 ? at::kFloat8_e4m3fn : at::kChar, x);
+        s = empty({nb, kb}, fp8 ? at::kFloat : at::kHalf, x);
+        if (fp8) g.check(g.st->llmk_weight_quant_fp8_block(x.data_ptr(), dt, y.data_ptr(), (float*)s.data_ptr(), N, K, (int)block, stream_of(x)), "llmk_weight_quant_fp8_block");
+        else g.check(g.st->llmk_weight_quant_i8_block(x.data_ptr(), dt, (int8_t*)y.data_ptr(), s.data_ptr(), N, K, (int)block, 127.f, LLMK_ROUND_HALF_AWAY, 0, stream_of(x)),
+                     "llmk_weight_quant_i8_block");
+    });
     return wrap_all(std::move(y), std::move(s));
 }
 
@@ -217,15 +270,18 @@ PyObject* weight_dequant(const Args& g) {
     require(x.dim() == 2 && s.dim() == 2, "Input tensors must have 2 dimensions");
     g.on_gpu(x, s);
     const at::ScalarType out = default_dtype();
-    at::Tensor y = empty(x.sizes(), out, x);
-    if (fp8) {
-        const at::Tensor s32 = as_type(s, at::kFloat);
-        g.check(g.st->llmk_weight_dequant_fp8_block(x.data_ptr(), (const float*)s32.data_ptr(), y.data_ptr(), float_code(out), x.size(0), x.size(1), (int)block, stream_of(x)),
-                "llmk_weight_dequant_fp8_block");
-    } else {
-        g.check(g.st->llmk_weight_dequant_i8_block((const int8_t*)x.data_ptr(), s.data_ptr(), float_code(s.scalar_type()), y.data_ptr(), float_code(out), x.size(0), x.size(1), (int)block,
-                                                   stream_of(x)), "llmk_weight_dequant_i8_block");
-    }
+    at::Tensor y;
+    unlocked([&] {
+        y = empty(x.sizes(), out, x);
+        if (fp8) {
+            const at::Tensor s32 = as_type(s, at::kFloat);
+            g.check(g.st->llmk_weight_dequant_fp8_block(x.data_ptr(), (const float*)s32.data_ptr(), y.data_ptr(), float_code(out), x.size(0), x.size(1), (int)block, stream_of(x)),
+                    "llmk_weight_dequant_fp8_block");
+        } else {
+            g.check(g.st->llmk_weight_dequant_i8_block((const int8_t*)x.data_ptr(), s.data_ptr(), float_code(s.scalar_type()), y.data_ptr(), float_code(out), x.size(0), x.size(1), (int)block,
+                                                       stream_of(x)), "llmk_weight_dequant_i8_block");
+        }
+    });
     return wrap(std::move(y));
 }
 
@@ -233,22 +289,31 @@ PyObject* weight_dequant(const Args& g) {
 PyObject* w4a8_weight_quant(const Args& g) {
     const at::Tensor& x = g.tensor(0);
     const int64_t group = g.integer(1), N = x.size(0), K = x.size(1);
-    at::Tensor packed = empty({N / 8, K}, at::kInt, x), s = empty({(N + 127) / 128, K / 128}, at::kHalf, x);
-    at::Tensor s4 = empty({N, K / group}, at::kChar, x), z4 = empty({N, K / group}, at::kChar, x);
-    g.check(g.st->llmk_weight_quant_w4a8(x.data_ptr(), float_code(x.scalar_type()), (int32_t*)packed.data_ptr(), s.data_ptr(), (int8_t*)s4.data_ptr(), (int8_t*)z4.data_ptr(), N, K, (int)group,
-                                         stream_of(x)), "llmk_weight_quant_w4a8");
+    at::Tensor packed, s, s4, z4;
+    unlocked([&] {
+        packed = empty({N / 8, K}, at::kInt, x);
+        s = empty({(N + 127) / 128, K / 128}, at::kHalf, x);
+        s4 = empty({N, K / group}, at::kChar, x);
+        z4 = empty({N, K / group}, at::kChar, x);
+        g.check(g.st->llmk_weight_quant_w4a8(x.data_ptr(), float_code(x.scalar_type()), (int32_t*)packed.data_ptr(), s.data_ptr(), (int8_t*)s4.data_ptr(), (int8_t*)z4.data_ptr(), N, K, (int)group,
+                                             stream_of(x)), "llmk_weight_quant_w4a8");
+    });
     return wrap_all(std::move(packed), std::move(s), std::move(s4), std::move(z4));
 }
 
 // w4a8_weight_dequant(packed, s, s4, z4, block, group) -> fp16
 PyObject* w4a8_weight_dequant(const Args& g) {
-    const at::Tensor& y = g.tensor(0);
-    g.on_gpu(y, g.tensor(1), g.tensor(2), g.tensor(3));
-    const at::Tensor s = g.tensor(1).contiguous(), s4 = g.tensor(2).contiguous(), z4 = g.tensor(3).contiguous();
-    const int64_t K = y.size(1), N = y.size(0) * 8;
-    at::Tensor out = empty({N, K}, at::kHalf, y);
-    g.check(g.st->llmk_weight_dequant_w4a8((const int32_t*)y.data_ptr(), s.data_ptr(), (const int8_t*)s4.data_ptr(), (const int8_t*)z4.data_ptr(), out.data_ptr(), N, K, (int)g.integer(4),
-                                           (int)g.integer(5), stream_of(y)), "llmk_weight_dequant_w4a8");
+    const at::Tensor &y = g.tensor(0), &s_in = g.tensor(1), &s4_in = g.tensor(2), &z4_in = g.tensor(3);
+    g.on_gpu(y, s_in, s4_in, z4_in);
+    const int block = (int)g.integer(4), group = (int)g.integer(5);
+    at::Tensor out;
+    unlocked([&] {
+        const at::Tensor s = s_in.contiguous(), s4 = s4_in.contiguous(), z4 = z4_in.contiguous();
+        const int64_t K = y.size(1), N = y.size(0) * 8;
+        out = empty({N, K}, at::kHalf, y);
+        g.check(g.st->llmk_weight_dequant_w4a8((const int32_t*)y.data_ptr(), s.data_ptr(), (const int8_t*)s4.data_ptr(), (const int8_t*)z4.data_ptr(), out.data_ptr(), N, K, block, group,
+                                               stream_of(y)), "llmk_weight_dequant_w4a8");
+    });
     return wrap(std::move(out));
 }
 
@@ -256,15 +321,21 @@ PyObject* w4a8_weight_dequant(const Args& g) {
 PyObject* w4_quantize_nk(const Args& g) {
     const int64_t group = g.integer(1);
     if (group == 0) raise(PyExc_ZeroDivisionError, "integer division or modulo by zero");
-    require(g.tensor(0).dim() == 2 && g.tensor(0).size(1) % group == 0, "");
-    const at::ScalarType t = g.tensor(0).scalar_type();
+    const at::Tensor& in = g.tensor(0);
+    require(in.dim() == 2 && in.size(1) % group == 0, "");
+    const at::ScalarType t = in.scalar_type();
     require(t == at::kFloat || t == at::kHalf || t == at::kBFloat16, "weights must be fp32, fp16 or bf16");
-    g.on_gpu(g.tensor(0));
-    const at::Tensor w = g.tensor(0).contiguous();
-    const int64_t N = w.size(0), K = w.size(1);
-    at::Tensor packed = empty({N, K / 8}, at::kInt, w), s = empty({N, K / group}, at::kHalf, w), q = empty({N, K}, at::kByte, w);
-    g.check(g.st->llmk_quant_w4_nk(w.data_ptr(), float_code(t), (int32_t*)packed.data_ptr(), s.data_ptr(), (uint8_t*)q.data_ptr(), N, K, (int)group, stream_of(w)), "llmk_quant_w4_nk",
-            PyExc_AssertionError);
+    g.on_gpu(in);
+    at::Tensor packed, s, q;
+    unlocked([&] {
+        const at::Tensor w = in.contiguous();
+        const int64_t N = w.size(0), K = w.size(1);
+        packed = empty({N, K / 8}, at::kInt, w);
+        s = empty({N, K / group}, at::kHalf, w);
+        q = empty({N, K}, at::kByte, w);
+        g.check(g.st->llmk_quant_w4_nk(w.data_ptr(), float_code(t), (int32_t*)packed.data_ptr(), s.data_ptr(), (uint8_t*)q.data_ptr(), N, K, (int)group, stream_of(w)), "llmk_quant_w4_nk",
+                PyExc_AssertionError);
+    });
     return wrap_all(std::move(packed), std::move(s), std::move(q));
 }
 
@@ -281,11 +352,13 @@ PyObject* fp8_gemm(const Args& g) {
     const int64_t K = last_size(a), M = rows_of(a, K), N = b.size(0);
     require(a_s.scalar_type() == at::kFloat && b_s.scalar_type() == at::kFloat, "fp8 scales must be float32");
     const at::ScalarType out = default_dtype();
-    at::Tensor c = empty(with_last(a, N), out, a);
-    const int64_t need = g.st->llmk_gemm_workspace_bytes(M, N, K);
-    void* ws = workspace(g, a, need);
-    g.check(g.st->llmk_gemm_fp8_block(a.data_ptr(), (const float*)a_s.data_ptr(), b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), float_code(out), M, N, K,
-                                      ws, ws ? need : 0, stream_of(a)), "llmk_gemm_fp8_block", PyExc_AssertionError);
+    Scratch ws(g, a, g.st->llmk_gemm_workspace_bytes(M, N, K));
+    at::Tensor c;
+    unlocked([&] {
+        c = empty(with_last(a, N), out, a);
+        g.check(g.st->llmk_gemm_fp8_block(a.data_ptr(), (const float*)a_s.data_ptr(), b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), float_code(out), M, N, K,
+                                          ws.get(), ws.bytes(), stream_of(a)), "llmk_gemm_fp8_block", PyExc_AssertionError);
+    });
     return wrap(std::move(c));
 }
 
@@ -295,30 +368,34 @@ PyObject* int8_gemm(const Args& g) {
     const int64_t K = last_size(a), M = rows_of(a, K), N = b.size(0);
     require(a_s.scalar_type() == b_s.scalar_type(), "activation and weight scales must share a dtype");
     const at::ScalarType out = default_dtype();
-    at::Tensor c = empty(with_last(a, N), out, a);
-    const int64_t need = g.st->llmk_gemm_workspace_bytes(M, N, K);
-    void* ws = workspace(g, a, need);
-    g.check(g.st->llmk_gemm_i8_block((const int8_t*)a.data_ptr(), a_s.data_ptr(), (const int8_t*)b.data_ptr(), b_s.data_ptr(), float_code(a_s.scalar_type()), c.data_ptr(),
-                                     float_code(out), M, N, K, ws, ws ? need : 0, stream_of(a)), "llmk_gemm_i8_block", PyExc_AssertionError);
+    Scratch ws(g, a, g.st->llmk_gemm_workspace_bytes(M, N, K));
+    at::Tensor c;
+    unlocked([&] {
+        c = empty(with_last(a, N), out, a);
+        g.check(g.st->llmk_gemm_i8_block((const int8_t*)a.data_ptr(), a_s.data_ptr(), (const int8_t*)b.data_ptr(), b_s.data_ptr(), float_code(a_s.scalar_type()), c.data_ptr(),
+                                         float_code(out), M, N, K, ws.get(), ws.bytes(), stream_of(a)), "llmk_gemm_i8_block", PyExc_AssertionError);
+    });
     return wrap(std::move(c));
 }
 
 // int8_gemm_per_token(a, a_s, b, b_s, with int32 accumulators)
 PyObject* int8_gemm_per_token(const Args& g) {
-    const at::Tensor &a = g.tensor(0), &b = g.tensor(2);
+    const at::Tensor &a = g.tensor(0), &a_s_in = g.tensor(1), &b = g.tensor(2), &b_s_in = g.tensor(3);
     require(a.is_contiguous() && b.is_contiguous(), "Input tensors must be contiguous");
-    g.on_gpu(a, g.tensor(1), b, g.tensor(3));
+    g.on_gpu(a, a_s_in, b, b_s_in);
     const int64_t K = last_size(a), M = rows_of(a, K), N = b.size(0);
-    const at::Tensor a_s = as_type(g.tensor(1), at::kFloat).contiguous(), b_s = as_type(g.tensor(3), at::kFloat).contiguous();
-    require(a_s.numel() == M && b_s.numel() == N, "need one scale per token and per output channel");
+    require(a_s_in.numel() == M && b_s_in.numel() == N, "need one scale per token and per output channel");
     const at::ScalarType out = default_dtype();
-    at::Tensor c = empty(with_last(a, N), out, a), acc;
     const bool want_acc = g.integer(4) != 0;
-    if (want_acc) acc = empty(with_last(a, N), at::kInt, a);
-    const int64_t need = M <= 512 ? g.st->llmk_gemm_workspace_bytes(M, N, K) : 0;     // only the K split of mid-size M uses scratch here
-    void* ws = workspace(g, a, need);
-    g.check(g.st->llmk_gemm_i8_rowcol((const int8_t*)a.data_ptr(), (const float*)a_s.data_ptr(), (const int8_t*)b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), float_code(out),
-                                      want_acc ? (int32_t*)acc.data_ptr() : nullptr, M, N, K, ws, ws ? need : 0, stream_of(a)), "llmk_gemm_i8_rowcol", PyExc_AssertionError);
+    Scratch ws(g, a, M <= 512 ? g.st->llmk_gemm_workspace_bytes(M, N, K) : 0);        // only the K split of mid-size M uses scratch here
+    at::Tensor c, acc;
+    unlocked([&] {
+        const at::Tensor a_s = as_type(a_s_in, at::kFloat).contiguous(), b_s = as_type(b_s_in, at::kFloat).contiguous();
+        c = empty(with_last(a, N), out, a);
+        if (want_acc) acc = empty(with_last(a, N), at::kInt, a);
+        g.check(g.st->llmk_gemm_i8_rowcol((const int8_t*)a.data_ptr(), (const float*)a_s.data_ptr(), (const int8_t*)b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), float_code(out),
+                                          want_acc ? (int32_t*)acc.data_ptr() : nullptr, M, N, K, ws.get(), ws.bytes(), stream_of(a)), "llmk_gemm_i8_rowcol", PyExc_AssertionError);
+    });
     return want_acc ? wrap_all(std::move(c), std::move(acc)) : wrap(std::move(c));
 }
 
@@ -333,13 +410,15 @@ PyObject* w4a8_gemm(const Args& g) {
     const int group = (int)g.integer(6);
     require(a_s.scalar_type() == b_s.scalar_type(), "activation and weight scales must share a dtype");
     const at::ScalarType out = default_dtype();
-    at::Tensor c = empty(with_last(a, N), out, a);
     // what this shape's kernels use: nothing for the fused decode kernel with K <= 4096, fp32 partial sums for its
     // K ranges or the K slices of the fused tile kernels, the expanded int8 weights + the int8 GEMM's scratch otherwise
-    const int64_t need = g.st->llmk_gemm_w4a8_workspace_bytes(M, N, K, group);
-    void* ws = workspace(g, a, need);
-    g.check(g.st->llmk_gemm_w4a8((const int8_t*)a.data_ptr(), a_s.data_ptr(), (const int32_t*)b.data_ptr(), b_s.data_ptr(), float_code(a_s.scalar_type()), (const int8_t*)s4.data_ptr(),
-                                 (const int8_t*)z4.data_ptr(), c.data_ptr(), float_code(out), M, N, K, group, ws, ws ? need : 0, stream_of(a)), "llmk_gemm_w4a8", PyExc_AssertionError);
+    Scratch ws(g, a, g.st->llmk_gemm_w4a8_workspace_bytes(M, N, K, group));
+    at::Tensor c;
+    unlocked([&] {
+        c = empty(with_last(a, N), out, a);
+        g.check(g.st->llmk_gemm_w4a8((const int8_t*)a.data_ptr(), a_s.data_ptr(), (const int32_t*)b.data_ptr(), b_s.data_ptr(), float_code(a_s.scalar_type()), (const int8_t*)s4.data_ptr(),
+                                     (const int8_t*)z4.data_ptr(), c.data_ptr(), float_code(out), M, N, K, group, ws.get(), ws.bytes(), stream_of(a)), "llmk_gemm_w4a8", PyExc_AssertionError);
+    });
     return wrap(std::move(c));
 }
 
@@ -354,7 +433,6 @@ PyObject* w4a16_gemm(const Args& g) {
     require(w.size(1) * 8 == K, "packed weight must be [N, K/8]");
     require(x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16, "activations must be fp16 or bf16");
     const bool bf = x.scalar_type() == at::kBFloat16;
-    at::Tensor y = empty(with_last(x, N), x.scalar_type(), x);
     // bf16 at decode size runs on the weight-streaming ring kernel under exactly the conditions the library
     // checks (128-wide groups, K ranges of 4 to 32 steps, 8-byte aligned outputs, 32-bit lane offsets, and with more than
     // one K range M * N % 4 == 0 for the summing pass);
@@ -362,16 +440,20 @@ PyObject* w4a16_gemm(const Args& g) {
     const int64_t steps = K / 128, nz = std::max<int64_t>(1, (steps + 31) / 32), per = (steps + nz - 1) / nz;
     const bool ring_ok = group == 128 && per <= 32 && steps - (nz - 1) * per >= 4 &&
                          N * (K / 2) < (1ll << 32) && M * K * 2 < (1ll << 32);
-    const bool bf_decode = bf && M <= 64 && ring_ok && ((uintptr_t)y.data_ptr() & 7) == 0 && (nz == 1 || (M * N) % 4 == 0);
+    const bool bf_decode = bf && M <= 64 && ring_ok && (nz == 1 || (M * N) % 4 == 0);          // (the outputs are allocated here)
     int64_t need = 0;
     if (M > 64 || (bf && !bf_decode))
         // fp16 / bf16 copy of W for the compute-bound path, split-K partials behind it for mid-size M
         need = ((N * K * 2 + 255) / 256) * 256 + (M <= 512 ? 8 * M * N * 4 : 0);
     else if (K > 4096 || M > 16)
         need = std::max<int64_t>(8, (K + 4095) / 4096) * M * N * 4;                   // fp32 partial sums of K ranges / K slices
-    void* ws = workspace(g, x, need);
-    g.check(g.st->llmk_gemm_w4a16_nk(x.data_ptr(), (const int32_t*)w.data_ptr(), y.data_ptr(), s.data_ptr(), float_code(x.scalar_type()), M, N, K, group, ws, ws ? need : 0, stream_of(x)),
-            "llmk_gemm_w4a16_nk", PyExc_AssertionError);
+    Scratch ws(g, x, need);
+    at::Tensor y;
+    unlocked([&] {
+        y = empty(with_last(x, N), x.scalar_type(), x);
+        g.check(g.st->llmk_gemm_w4a16_nk(x.data_ptr(), (const int32_t*)w.data_ptr(), y.data_ptr(), s.data_ptr(), float_code(x.scalar_type()), M, N, K, group, ws.get(), ws.bytes(), stream_of(x)),
+                "llmk_gemm_w4a16_nk", PyExc_AssertionError);
+    });
     return wrap(std::move(y));
 }
 
@@ -388,7 +470,6 @@ PyObject* marlin_mul(const Args& g) {
     if (B.scalar_type() != at::kInt) fail("B matrix must be packed INT4 data (torch.int32)");
     if (!C.is_contiguous()) fail("C must be contiguous (the result is written in place)");
     if (C.size(0) != M) fail("C must have as many rows as A");
-    const at::Tensor a = A.contiguous(), b = B.contiguous(), sc = s.contiguous();
     int64_t group = -1;
     if (s.dim() == 2) {
         if (s.size(1) != N) fail("Scale tensor N dimension mismatch: expected " + std::to_string(N) + " but got " + std::to_string(s.size(1)));
@@ -396,22 +477,30 @@ PyObject* marlin_mul(const Args& g) {
         group = K / s.size(0);
         if (group == 0 || K % group) fail("K dimension not divisible by groupsize: K=" + std::to_string(K) + ", groupsize=" + std::to_string(group));
     }
-    if (b.numel() * 8 != K * N) fail("B does not hold K*N packed 4-bit values");
-    const int64_t need = g.st->llmk_gemm_w4a16_marlin_workspace_bytes(M, N, K);
-    void* ws = workspace(g, A, need);
-    g.check(g.st->llmk_gemm_w4a16_marlin(a.data_ptr(), (const int32_t*)b.data_ptr(), C.data_ptr(), sc.data_ptr(), M, N, K, (int)group, ws, ws ? need : 0, stream_of(A)),
-            "llmk_gemm_w4a16_marlin", PyExc_RuntimeError);
+    if (B.numel() * 8 != K * N) fail("B does not hold K*N packed 4-bit values");
+    Scratch ws(g, A, g.st->llmk_gemm_w4a16_marlin_workspace_bytes(M, N, K));
+    unlocked([&] {
+        const at::Tensor a = A.contiguous(), b = B.contiguous(), sc = s.contiguous();
+        g.check(g.st->llmk_gemm_w4a16_marlin(a.data_ptr(), (const int32_t*)b.data_ptr(), C.data_ptr(), sc.data_ptr(), M, N, K, (int)group, ws.get(), ws.bytes(), stream_of(A)),
+                "llmk_gemm_w4a16_marlin", PyExc_RuntimeError);
+    });
     Py_RETURN_NONE;
 }
 
 // ------------------------------------------------------------------ mixture of experts
 // softmax_topk(logits [.., E], topk, renormalize) -> (ids int64, weights fp32)
 PyObject* softmax_topk(const Args& g) {
-    const at::Tensor x = g.tensor(0).contiguous();
-    const int64_t topk = g.integer(1), E = last_size(x), T = rows_of(x, E);
-    at::Tensor ids = empty(with_last(x, topk), at::kLong, x), w = empty(with_last(x, topk), at::kFloat, x);
-    g.check(g.st->llmk_moe_softmax_topk(x.data_ptr(), float_code(x.scalar_type()), (int64_t*)ids.data_ptr(), (float*)w.data_ptr(), T, (int)E, (int)topk, g.integer(2) != 0, stream_of(x)),
-            "llmk_moe_softmax_topk");
+    const at::Tensor& in = g.tensor(0);
+    const int64_t topk = g.integer(1), E = last_size(in), T = rows_of(in, E);
+    const bool renorm = g.integer(2) != 0;
+    at::Tensor ids, w;
+    unlocked([&] {
+        const at::Tensor x = in.contiguous();
+        ids = empty(with_last(x, topk), at::kLong, x);
+        w = empty(with_last(x, topk), at::kFloat, x);
+        g.check(g.st->llmk_moe_softmax_topk(x.data_ptr(), float_code(x.scalar_type()), (int64_t*)ids.data_ptr(), (float*)w.data_ptr(), T, (int)E, (int)topk, renorm, stream_of(x)),
+                "llmk_moe_softmax_topk");
+    });
     return wrap_all(std::move(ids), std::move(w));
 }
 
@@ -420,9 +509,14 @@ PyObject* ep_preprocess(const Args& g) {
     const at::Tensor& ids = g.tensor(0);
     g.on_gpu(ids);
     const int64_t n = ids.numel(), E = g.integer(1);
-    at::Tensor sorted = empty({n}, ids.scalar_type(), ids), src2dst = empty({n}, at::kInt, ids), seg = empty({E + 1}, at::kLong, ids);
-    g.check(g.st->llmk_moe_ep_preprocess(ids.data_ptr(), id_bytes(ids), n, (int)E, sorted.data_ptr(), (int32_t*)src2dst.data_ptr(), (int64_t*)seg.data_ptr(), stream_of(ids)),
-            "llmk_moe_ep_preprocess");
+    at::Tensor sorted, src2dst, seg;
+    unlocked([&] {
+        sorted = empty({n}, ids.scalar_type(), ids);
+        src2dst = empty({n}, at::kInt, ids);
+        seg = empty({E + 1}, at::kLong, ids);
+        g.check(g.st->llmk_moe_ep_preprocess(ids.data_ptr(), id_bytes(ids), n, (int)E, sorted.data_ptr(), (int32_t*)src2dst.data_ptr(), (int64_t*)seg.data_ptr(), stream_of(ids)),
+                "llmk_moe_ep_preprocess");
+    });
     return wrap_all(std::move(sorted), std::move(src2dst), std::move(seg));
 }
 
@@ -436,9 +530,11 @@ QuantBuffers quant_buffers(int64_t rows, int64_t cols, int64_t fp8, const at::Te
     return {empty({rows, cols}, fp8 ? at::kFloat8_e4m3fn : at::kChar, like), empty({rows, cols / 128}, fp8 ? at::kFloat : at::kHalf, like),
             fp8 ? LLMK_KIND_FP8 : LLMK_KIND_I8};
 }
-at::Tensor f32_or_none(const Args& g, int i) { return g.none(i) ? at::Tensor() : as_type(g.tensor(i), at::kFloat).contiguous(); }
+// an optional tensor argument (undefined for None), and its fp32 / int64 form
+at::Tensor optional(const Args& g, int i) { return g.none(i) ? at::Tensor() : g.tensor(i); }
+at::Tensor f32_contiguous(const at::Tensor& t) { return t.defined() ? as_type(t, at::kFloat).contiguous() : t; }
 inline void* ptr_or_null(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
-at::Tensor long_contiguous(const at::Tensor& t) { return as_type(t, at::kLong).contiguous(); }
+at::Tensor long_contiguous(const at::Tensor& t) { return t.defined() ? as_type(t, at::kLong).contiguous() : t; }
 
 // pre_reorder_quant(input, src2dst, topk_ids, a1_scales, start, end, topk, hidden, fp8)
 PyObject* pre_reorder_quant(const Args& g) {
@@ -446,12 +542,16 @@ PyObject* pre_reorder_quant(const Args& g) {
     g.on_gpu(x, src2dst, ids);
     require(x.is_contiguous() && src2dst.is_contiguous() && ids.is_contiguous(), "");
     require(x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16, "");
-    const int64_t topk = g.integer(6), hidden = g.integer(7), T = rows_of(x, hidden);
-    QuantBuffers o = quant_buffers(T * topk, hidden, g.integer(8), x);
-    const at::Tensor sc = f32_or_none(g, 3);
-    g.check(g.st->llmk_moe_pre_reorder_quant(x.data_ptr(), float_code(x.scalar_type()), o.q.data_ptr(), o.s.data_ptr(), o.kind, LLMK_ROUND_HALF_AWAY, (const int32_t*)src2dst.data_ptr(),
-                                             ids.data_ptr(), id_bytes(ids), (const float*)ptr_or_null(sc), (int)g.integer(4), (int)g.integer(5), (int)topk, T, hidden, stream_of(x)),
-            "llmk_moe_pre_reorder_quant");
+    const int64_t start = g.integer(4), end = g.integer(5), topk = g.integer(6), hidden = g.integer(7), fp8 = g.integer(8), T = rows_of(x, hidden);
+    const at::Tensor scales = optional(g, 3);
+    QuantBuffers o;
+    unlocked([&] {
+        o = quant_buffers(T * topk, hidden, fp8, x);
+        const at::Tensor sc = f32_contiguous(scales);
+        g.check(g.st->llmk_moe_pre_reorder_quant(x.data_ptr(), float_code(x.scalar_type()), o.q.data_ptr(), o.s.data_ptr(), o.kind, LLMK_ROUND_HALF_AWAY, (const int32_t*)src2dst.data_ptr(),
+                                                 ids.data_ptr(), id_bytes(ids), (const float*)ptr_or_null(sc), (int)start, (int)end, (int)topk, T, hidden, stream_of(x)),
+                "llmk_moe_pre_reorder_quant");
+    });
     return wrap_all(std::move(o.q), std::move(o.s));
 }
 
@@ -461,12 +561,16 @@ PyObject* act_and_mul_quant(const Args& g) {
     g.on_gpu(x, ids);
     require(x.is_contiguous() && ids.is_contiguous(), "");
     require(x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16, "");
-    const int64_t two_i = g.integer(1), M = rows_of(x, two_i);
-    QuantBuffers o = quant_buffers(M, two_i / 2, g.integer(6), x);
-    const at::Tensor sc = f32_or_none(g, 3);
-    g.check(g.st->llmk_moe_act_and_mul_quant(x.data_ptr(), float_code(x.scalar_type()), o.q.data_ptr(), o.s.data_ptr(), o.kind, LLMK_ROUND_HALF_AWAY, ids.data_ptr(), id_bytes(ids),
-                                             (const float*)ptr_or_null(sc), (int)g.integer(4), (int)g.integer(5), M, two_i, (int)g.integer(7), stream_of(x)),
-            "llmk_moe_act_and_mul_quant");
+    const int64_t two_i = g.integer(1), start = g.integer(4), end = g.integer(5), fp8 = g.integer(6), act = g.integer(7), M = rows_of(x, two_i);
+    const at::Tensor scales = optional(g, 3);
+    QuantBuffers o;
+    unlocked([&] {
+        o = quant_buffers(M, two_i / 2, fp8, x);
+        const at::Tensor sc = f32_contiguous(scales);
+        g.check(g.st->llmk_moe_act_and_mul_quant(x.data_ptr(), float_code(x.scalar_type()), o.q.data_ptr(), o.s.data_ptr(), o.kind, LLMK_ROUND_HALF_AWAY, ids.data_ptr(), id_bytes(ids),
+                                                 (const float*)ptr_or_null(sc), (int)start, (int)end, M, two_i, (int)act, stream_of(x)),
+                "llmk_moe_act_and_mul_quant");
+    });
     return wrap_all(std::move(o.q), std::move(o.s));
 }
 
@@ -476,9 +580,11 @@ PyObject* post_reorder(const Args& g) {
     g.on_gpu(down, out, src2dst, ids, w);
     require(down.is_contiguous() && out.is_contiguous() && w.is_contiguous(), "");
     require(down.scalar_type() == out.scalar_type(), "");
-    const int64_t hidden = g.integer(8), T = rows_of(out, hidden);
-    g.check(g.st->llmk_moe_post_reorder(down.data_ptr(), out.data_ptr(), float_code(out.scalar_type()), (const int32_t*)src2dst.data_ptr(), ids.data_ptr(), id_bytes(ids), w.data_ptr(),
-                                        float_code(w.scalar_type()), (int)g.integer(5), (int)g.integer(6), (int)g.integer(7), T, hidden, stream_of(out)), "llmk_moe_post_reorder");
+    const int64_t start = g.integer(5), end = g.integer(6), topk = g.integer(7), hidden = g.integer(8), T = rows_of(out, hidden);
+    unlocked([&] {
+        g.check(g.st->llmk_moe_post_reorder(down.data_ptr(), out.data_ptr(), float_code(out.scalar_type()), (const int32_t*)src2dst.data_ptr(), ids.data_ptr(), id_bytes(ids), w.data_ptr(),
+                                            float_code(w.scalar_type()), (int)start, (int)end, (int)topk, T, hidden, stream_of(out)), "llmk_moe_post_reorder");
+    });
     Py_INCREF(g.v[1]);
     return g.v[1];
 }
@@ -501,17 +607,17 @@ PyObject* grouped_gemm(const Args& g) {
     require(a.scalar_type() == b.scalar_type(), "a and b must share a dtype after activation quantisation");
     const int kind = operand_kind(b.scalar_type());
     const bool scaled = kind == LLMK_KIND_I8 || kind == LLMK_KIND_FP8;
-    const at::Tensor seg = long_contiguous(g.tensor(4)), wi = g.none(5) ? at::Tensor() : long_contiguous(g.tensor(5));
-    at::Tensor sa, sb;
-    if (scaled) {
-        sa = g.tensor(6);
-        sb = as_type(g.tensor(7), sa.scalar_type()).contiguous();
-    }
-    const int64_t M = a.size(0), N = b.size(1), K = b.size(2), need = g.st->llmk_gemm_workspace_bytes(M, N, K);
-    void* ws = workspace(g, a, need);
-    g.check(g.st->llmk_grouped_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), kind, float_code(c.scalar_type()), (int)g.integer(3), M, N, K, (const int64_t*)seg.data_ptr(),
-                                    (const int64_t*)ptr_or_null(wi), ptr_or_null(sa), ptr_or_null(sb), scaled ? float_code(sa.scalar_type()) : 0, ws, ws ? need : 0, stream_of(a)),
-            "llmk_grouped_gemm", PyExc_AssertionError);
+    const int64_t E = g.integer(3), M = a.size(0), N = b.size(1), K = b.size(2);
+    const at::Tensor& seg_in = g.tensor(4);
+    const at::Tensor wi_in = optional(g, 5), sa = scaled ? g.tensor(6) : at::Tensor(), sb_in = scaled ? g.tensor(7) : at::Tensor();
+    Scratch ws(g, a, g.st->llmk_gemm_workspace_bytes(M, N, K));
+    unlocked([&] {
+        const at::Tensor seg = long_contiguous(seg_in), wi = long_contiguous(wi_in);
+        const at::Tensor sb = scaled ? as_type(sb_in, sa.scalar_type()).contiguous() : sb_in;
+        g.check(g.st->llmk_grouped_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), kind, float_code(c.scalar_type()), (int)E, M, N, K, (const int64_t*)seg.data_ptr(),
+                                        (const int64_t*)ptr_or_null(wi), ptr_or_null(sa), ptr_or_null(sb), scaled ? float_code(sa.scalar_type()) : 0, ws.get(), ws.bytes(), stream_of(a)),
+                "llmk_grouped_gemm", PyExc_AssertionError);
+    });
     Py_INCREF(g.v[2]);
     return g.v[2];
 }
@@ -526,20 +632,23 @@ PyObject* swiglu_fused(const Args& g) {
 
 // grouped_gemm_swiglu_quant(a, scale_a, b, scale_b, batch_size, seg_indptr, weight_indices, mid dtype code, act)
 PyObject* swiglu_quant(const Args& g) {
-    const at::Tensor &a = g.tensor(0), &b = g.tensor(2), &seg_in = g.tensor(5);
-    g.on_gpu(a, b, g.tensor(1), g.tensor(3), seg_in);
+    const at::Tensor &a = g.tensor(0), &sa_in = g.tensor(1), &b = g.tensor(2), &sb_in = g.tensor(3), &seg_in = g.tensor(5);
+    g.on_gpu(a, b, sa_in, sb_in, seg_in);
     require(a.is_contiguous() && b.is_contiguous() && a.scalar_type() == b.scalar_type() && b.dim() == 3 && last_size(a) == last_size(b), "");
     const int kind = operand_kind(b.scalar_type());
     require(kind == LLMK_KIND_I8 || kind == LLMK_KIND_FP8, "quant_dtype must be torch.int8 or torch.float8_e4m3fn");
-    const int64_t M = a.size(0), two_i = b.size(1), K = b.size(2);
-    QuantBuffers o = quant_buffers(M, two_i / 2, kind == LLMK_KIND_FP8, a);
-    const at::Tensor sa = g.tensor(1).contiguous(), sb = as_type(g.tensor(3), sa.scalar_type()).contiguous();
-    const at::Tensor seg = long_contiguous(seg_in), wi = g.none(6) ? at::Tensor() : long_contiguous(g.tensor(6));
-    const int64_t need = sa.scalar_type() == at::kFloat ? 0 : M * (K / 128) * 4;
-    void* ws = workspace(g, a, need);
-    g.check(g.st->llmk_grouped_gemm_swiglu_quant(a.data_ptr(), b.data_ptr(), o.q.data_ptr(), o.s.data_ptr(), kind, (int)g.integer(7), LLMK_ROUND_HALF_AWAY, (int)g.integer(4), M, two_i, K,
-                                                 (const int64_t*)seg.data_ptr(), (const int64_t*)ptr_or_null(wi), sa.data_ptr(), sb.data_ptr(), float_code(sa.scalar_type()),
-                                                 (int)g.integer(8), ws, ws ? need : 0, stream_of(a)), "llmk_grouped_gemm_swiglu_quant", PyExc_AssertionError);
+    const int64_t M = a.size(0), two_i = b.size(1), K = b.size(2), E = g.integer(4), mid = g.integer(7), act = g.integer(8);
+    const at::Tensor wi_in = optional(g, 6);
+    Scratch ws(g, a, sa_in.scalar_type() == at::kFloat ? 0 : M * (K / 128) * 4);
+    QuantBuffers o;
+    unlocked([&] {
+        o = quant_buffers(M, two_i / 2, kind == LLMK_KIND_FP8, a);
+        const at::Tensor sa = sa_in.contiguous(), sb = as_type(sb_in, sa.scalar_type()).contiguous();
+        const at::Tensor seg = long_contiguous(seg_in), wi = long_contiguous(wi_in);
+        g.check(g.st->llmk_grouped_gemm_swiglu_quant(a.data_ptr(), b.data_ptr(), o.q.data_ptr(), o.s.data_ptr(), kind, (int)mid, LLMK_ROUND_HALF_AWAY, (int)E, M, two_i, K,
+                                                     (const int64_t*)seg.data_ptr(), (const int64_t*)ptr_or_null(wi), sa.data_ptr(), sb.data_ptr(), float_code(sa.scalar_type()),
+                                                     (int)act, ws.get(), ws.bytes(), stream_of(a)), "llmk_grouped_gemm_swiglu_quant", PyExc_AssertionError);
+    });
     return wrap_all(std::move(o.q), std::move(o.s));
 }
 
@@ -572,7 +681,8 @@ PyObject* call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     try {
         return F(Args(self, args, n, N));
-    } catch (const Raised&) {
+    } catch (const Raised& r) {
+        if (r.type) PyErr_SetString(r.type, r.msg.c_str());
         return nullptr;
     }
     END_HANDLE_TH_ERRORS
