@@ -156,3 +156,59 @@ def test_threads_on_one_stream_get_the_serial_results(dev):
             t.join()
         torch.cuda.synchronize()
         assert not wrong
+
+
+def test_outputs_are_filled_under_deterministic_algorithms(dev):
+    """torch.use_deterministic_algorithms fills new tensors, so rows that an operator leaves unwritten are the same in every
+    run: the tokens of experts outside the local range here."""
+    announce("deterministic fill")
+    from llm_kernels_amd.moe import group_gemm_kernel as gk
+    torch.manual_seed(0)
+    T, E, H = 16, 4, 256
+    ids = torch.arange(T, device=dev).remainder(E).view(T, 1)
+    x = torch.randn(T, H, device=dev).bfloat16()
+    _, src2dst, seg = gk.run_moe_ep_preproess(ids, E)
+    first = seg.tolist()[2]                              # rows of experts 0 and 1: not local below
+    assert torch.utils.deterministic.fill_uninitialized_memory
+    torch.use_deterministic_algorithms(True)
+    try:
+        q, s = gk.pre_reorder_quant(x, src2dst, ids, None, 2, 3, 1, H, torch.int8)
+        qf, sf = gk.pre_reorder_quant(x, src2dst, ids, None, 2, 3, 1, H, torch.float8_e4m3fn)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert (q[:first] == 127).all() and s[:first].isnan().all()          # what torch.empty holds then
+    assert qf[:first].float().isnan().all() and sf[:first].isnan().all()
+    q1, s1 = gk.pre_reorder_quant(x, src2dst, ids, None, 2, 3, 1, H, torch.int8)
+    assert torch.equal(q[first:], q1[first:]) and torch.equal(s[first:], s1[first:])
+
+
+def test_dispatch_modes_see_the_allocations(dev):
+    announce("dispatch mode")
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Log(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.sizes = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if "empty" in func.__name__:
+                self.sizes.append((tuple(out.shape), out.dtype))
+            return out
+
+    torch.manual_seed(0)
+    x = torch.randn(3, 256, device=dev).bfloat16()
+    with Log() as log:
+        y, s = fp8_kernel.act_quant(x)
+    assert ((3, 256), torch.float8_e4m3fn) in log.sizes and ((3, 2), torch.float32) in log.sizes
+    y1, s1 = fp8_kernel.act_quant(x)
+    assert torch.equal(y.view(torch.uint8), y1.view(torch.uint8)) and torch.equal(s, s1)
+
+
+def test_the_profiler_sees_the_allocations(dev):
+    announce("profiler")
+    x = torch.randn(3, 256, device=dev).bfloat16()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        fp8_kernel.act_quant(x)
+    assert sum(e.name == "aten::empty" for e in prof.events()) == 2
