@@ -516,24 +516,32 @@ extern "C" int llmk_moe_ep_preprocess(const void* topk_ids, int ids_bytes, int64
 }
 
 template <int DT>
-static int launch_router(const void* logits, int64_t* ids, float* w, int64_t T, int E, int topk, bool renorm, hipStream_t st) {
-    // the narrowest group of lanes that holds a token's experts one each, then more experts per lane
+static int launch_router(const void* logits_all, int64_t* ids_all, float* w_all, int64_t T_all, int E, int topk, bool renorm, hipStream_t st) {
+    // the narrowest group of lanes that holds a token's experts one each, then more experts per lane; 2^24 tokens a launch
+    // (64 lanes each are a quarter of the 2^32 threads a grid may have)
+    constexpr int64_t ROWS = 1ll << 24;
+    for (int64_t t0 = 0; t0 < T_all; t0 += ROWS) {
+        const void* logits = (const uint8_t*)logits_all + t0 * E * (DT == LLMK_F32 ? 4 : 2);
+        int64_t* ids = ids_all + t0 * topk;
+        float* w = w_all + t0 * topk;
+        const int64_t T = std::min(ROWS, T_all - t0);
 #define CALL(L, V) softmax_topk_kernel<DT, L, V><<<(unsigned)cdiv64(T * L, 256), 256, 0, st>>>(logits, ids, w, T, E, topk, renorm)
-    if (E <= 8) CALL(8, 1);
-    else if (E <= 16) CALL(16, 1);
-    else if (E <= 32) CALL(32, 1);
-    else if (E <= 64) CALL(64, 1);
-    else if (E <= 128) CALL(64, 2);
-    else if (E <= 256) CALL(64, 4);
-    else CALL(64, 8);
+        if (E <= 8) CALL(8, 1);
+        else if (E <= 16) CALL(16, 1);
+        else if (E <= 32) CALL(32, 1);
+        else if (E <= 64) CALL(64, 1);
+        else if (E <= 128) CALL(64, 2);
+        else if (E <= 256) CALL(64, 4);
+        else CALL(64, 8);
 #undef CALL
-    LLMK_CHECK_LAUNCH("moe_softmax_topk");
+        LLMK_CHECK_LAUNCH("moe_softmax_topk");
+    }
     return LLMK_OK;
 }
 
 extern "C" int llmk_moe_softmax_topk(const void* logits, int dtype, int64_t* ids, float* weights, int64_t T, int E, int topk,
                                      int renormalize, void* stream) {
-    if (T < 0 || E < 1 || topk < 1 || topk > E || E > LLMK_ROUTER_MAX_EXPERTS || topk > LLMK_ROUTER_MAX_TOPK || T > (1ll << 24))
+    if (T < 0 || E < 1 || topk < 1 || topk > E || E > LLMK_ROUTER_MAX_EXPERTS || topk > LLMK_ROUTER_MAX_TOPK)
         LLMK_FAIL(LLMK_ERR_SHAPE, "moe_softmax_topk: T=%lld E=%d topk=%d", (long long)T, E, topk);
     if (T == 0) return LLMK_OK;
     if (!logits || !ids || !weights) LLMK_FAIL(LLMK_ERR_ARG, "moe_softmax_topk: null pointer");

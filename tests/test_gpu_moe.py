@@ -73,6 +73,21 @@ def test_router_breaks_ties_by_index(dev):
     assert ids.tolist() == [[0, 1, 2]] * 5 and torch.allclose(w, torch.full_like(w, 1 / 3))
 
 
+def test_router_takes_any_number_of_rows(dev):
+    """More rows than one launch takes: the rows on both sides of the launches' border get what a call of their own gives."""
+    announce("router rows", 2 ** 24 + 37)
+    T = 2 ** 24 + 37
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(3)
+    logits = torch.randn(T, 2, generator=gen, device=dev, dtype=torch.bfloat16)
+    ids, w = softmax_topk_router(logits, 1, False)
+    for lo, hi in ((0, 100), (2 ** 24 - 100, T)):
+        ids1, w1 = softmax_topk_router(logits[lo:hi], 1, False)
+        assert torch.equal(ids[lo:hi], ids1) and torch.equal(w[lo:hi], w1)
+    p = torch.softmax(logits.float(), -1)
+    assert torch.allclose(w, p.amax(-1, keepdim=True), rtol=48 * 2 ** -24, atol=0)
+
+
 @pytest.mark.parametrize("n,E", [(1, 3), (64, 512), (65, 64), (256, 63), (257, 65), (1024, 8), (1025, 64), (32768, 64)])
 def test_preprocess_workgroup_sizes(dev, n, E):
     """Edges of the workgroup sizes and of the two ways of counting (64 experts and below, above)."""
