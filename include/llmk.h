@@ -182,12 +182,15 @@ int llmk_gemm_w4a16_marlin(const void* a_f16, const int32_t* b, void* c_f16, con
 int llmk_quant_w4_nk(const void* w, int w_dtype, int32_t* packed, void* scales_f16, uint8_t* q, int64_t N,
                      int64_t K, int group, void* stream);
 /* Same product for W stored [N, K/8] int32 by pack_weights_over_cols (nibble i of a word = k*8+i)
- * with s fp16 [N, K/g]; a/c fp16 or bf16 (ac_dtype; bf16: M <= 64 with 128-wide groups streams the weights,
- * every other bf16 call multiplies a bf16 copy of W and needs the N*K*2-byte workspace).  workspace is optional for fp16:
- * M > 512 with N*K*2 bytes (16-byte aligned) runs as dequantise + tiled MFMA GEMM; 64 < M <= 512 (and
- * 32 < M <= 64 with large weights) runs on tile kernels that expand the packed words themselves and use
- * up to 8*M*N*4 bytes for split-K partial sums; M <= 64, K > 4096 with ceil(K/4096)*M*N*4 bytes runs as
- * K ranges with fp32 partial sums. */
+ * with s fp16 [N, K/g]; a/c fp16 or bf16 (ac_dtype).  workspace: llmk_gemm_w4a16_nk_workspace_bytes(...) bytes, 16-byte
+ * aligned, is what the path chosen for the shape uses:
+ *   - M <= 64 streams the weights: nothing for K <= 4096, fp32 partial sums of K ranges, ceil(K/4096)*M*N*4, beyond;
+ *   - 64 < M <= 512 (from 33 rows on large weights, to 1024 rows and more where it wins) runs on tile kernels that expand
+ *     the packed words themselves: fp32 partial sums of their K slices, at most 8*M*N*4;
+ *   - otherwise a 16-bit copy of W, N*K*2 bytes, that the tiled GEMM multiplies.
+ * With less, fp16 calls run on the streaming kernels unsplit; a bf16 call that neither streams (128-wide groups, K ranges of
+ * at least 512) nor expands (groups of whole 64) needs the N*K*2 bytes. */
+int64_t llmk_gemm_w4a16_nk_workspace_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int ac_dtype);
 int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* c, const void* s_f16,
                        int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize,
                        void* workspace, int64_t workspace_bytes, void* stream);

@@ -50,6 +50,7 @@ SIGNATURES = {
     "llmk_gemm_w4a8_workspace_bytes": [_l, _l, _l, _i],
     "llmk_gemm_w4a16_marlin_workspace_bytes": [_l, _l, _l],
     "llmk_gemm_w4a16_marlin": [_p, _p, _p, _p, _l, _l, _l, _i, _p, _l, _p],
+    "llmk_gemm_w4a16_nk_workspace_bytes": [_l, _l, _l, _i, _i],
     "llmk_gemm_w4a16_nk": [_p, _p, _p, _p, _i, _l, _l, _l, _i, _p, _l, _p],
     "llmk_convert_u4_to_f16": [_p, _p, _l, _p],
     "llmk_convert_u8_to_f16": [_p, _p, _l, _p],
@@ -75,7 +76,7 @@ SIGNATURES = {
     "llmk_grouped_gemm": [_p, _p, _p, _i, _i, _i, _l, _l, _l, _p, _p, _p, _p, _i, _p, _l, _p],
 }
 _RESTYPE = {"llmk_last_error": _c.c_char_p, "llmk_gemm_workspace_bytes": _l, "llmk_gemm_w4a8_workspace_bytes": _l,
-            "llmk_gemm_w4a16_marlin_workspace_bytes": _l}
+            "llmk_gemm_w4a16_marlin_workspace_bytes": _l, "llmk_gemm_w4a16_nk_workspace_bytes": _l}
 
 _lib = None
 

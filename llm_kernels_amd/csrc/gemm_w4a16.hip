@@ -881,7 +881,7 @@ int launch_nk_stream(const _Float16* A, const int32_t* B, const _Float16* S, _Fl
 // 14336 x 4096 122 and 105.  Beyond, every row tile expands the weights again and the fused form needs two rounds of
 // 256 x 256 tiles to win (fp16 4096 x 28672 x 4096: 741 vs 758 us, 2048 x 14336 x 4096: 198 vs 201; on one round 1300 x 6144
 // x 4096: 119 vs 86), the dearer bf16 expansion at most 2048 rows as well (1500 x 28672 x 4096: 319 vs 344, 4096 rows: 775 vs 762).
-bool w4_tiles_expand(int64_t M, int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes, bool wide = false, bool bf = false) {
+bool w4_tiles_expand(int64_t M, int64_t N, int64_t K, int64_t scratch, bool wide = false, bool bf = false) {
     if (M > 512) {
         if (!wide) return false;
         if (M > 1024) return ((M + 255) / 256) * ((N + 255) / 256) >= 512 && (!bf || M <= 2048);
@@ -895,44 +895,72 @@ bool w4_tiles_expand(int64_t M, int64_t N, int64_t K, const void* workspace, int
     const int64_t nk = N * K;
     if (!(K > 4096 ? nk >= ((int64_t)32 << 20) : nk >= ((int64_t)96 << 20))) return false;
     const int z = llmk::splitk_factor_half(M, N, K);
-    return z <= 1 || (workspace && workspace_bytes >= (int64_t)z * M * N * 4 && !((uintptr_t)workspace & 15));
+    return z <= 1 || scratch >= (int64_t)z * M * N * 4;
 }
+
+// what of a caller's workspace the kernels can use
+int64_t usable_scratch(const void* workspace, int64_t bytes) { return workspace && !((uintptr_t)workspace & 15) ? bytes : 0; }
 
 // Mid-size M (and large M on many tiles): the tile kernels expand the row-packed words themselves, so every weight byte is
 // read once; the separate expansion pass would write and re-read four times as much (bf16, 300 x 14336 x 4096: 26 us of
-// pass and 51 us of GEMM, 58 us in one kernel).  false: not a shape for them.
+// pass and 51 us of GEMM, 58 us in one kernel).  Which of them a shape takes, and its K slices:
+struct NkTiles {
+    enum { MID, MIDW, BIG } form;
+    int mt, z;
+};
 template <int KIND>
-bool launch_nk_tiles(const void* a, const int32_t* b_packed, void* c, const void* s, int dtype, int64_t M, int64_t N, int64_t K,
-                     int groupsize, void* workspace, int64_t workspace_bytes, hipStream_t st, int& rc) {
-    llmk::DirectArgs p{};
-    p.a = (const uint8_t*)a; p.b = (const uint8_t*)b_packed; p.b_s = s; p.c = c; p.c_dtype = dtype;
-    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = groupsize;
-    auto slices = [&](llmk::MidPlan& pl) {
-        if (pl.z > 1 && !(workspace && workspace_bytes >= (int64_t)pl.z * M * N * 4 && !((uintptr_t)workspace & 15))) pl.z = 1;
-    };
-    auto take = [&](const llmk::MidPlan& pl) { if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; } };
+NkTiles nk_tiles(const llmk::DirectArgs& p) {
+    const int64_t M = p.M, N = p.N, K = p.K;
     // few column tiles and short rows: the 64-column kernel with 512-byte K steps (128 x 4096 x 4096: 18.3 -> 14 us)
     if (2 * K <= 8192 && llmk::mid_wanted(M, N, 2 * K)) {       // (rows beyond 8 KB: measured only for the 8-bit kinds)
-        llmk::MidPlan pl = llmk::mid_plan(M, N, 2 * K);
-        slices(pl);
-        if (llmk::mid_eligible<KIND>(p, pl.mt, pl.z)) {
-            take(pl);
-            rc = pl.mt == 4 ? llmk::launch_mid<KIND, 4>(p, st, "gemm_w4a16_nk(mid)") : llmk::launch_mid<KIND, 2>(p, st, "gemm_w4a16_nk(mid)");
-            return true;
-        }
+        const llmk::MidPlan pl = llmk::mid_plan(M, N, 2 * K);
+        if (llmk::mid_eligible<KIND>(p, pl.mt, pl.z)) return {NkTiles::MID, pl.mt, pl.z};
     }
-    if (!llmk::dma_eligible(p, 2)) return false;
     // wider weights on one round of 128-column tiles: the 128-column form of that kernel
-    if (2 * K <= 8192 && llmk::midw_wanted(M, N, 2 * K) && (groupsize & (groupsize - 1)) == 0) {       // (longer rows: measured for fp8 only)
-        llmk::MidPlan pl = llmk::midw_plan(M, N, 2 * K);
-        slices(pl);
-        take(pl);
-        rc = pl.mt == 4 ? llmk::launch_mid<KIND, 4, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)")
-                        : llmk::launch_mid<KIND, 8, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)");
-        return true;
+    if (2 * K <= 8192 && llmk::midw_wanted(M, N, 2 * K) && (p.group & (p.group - 1)) == 0) {       // (longer rows: measured for fp8 only)
+        const llmk::MidPlan pl = llmk::midw_plan(M, N, 2 * K);
+        return {NkTiles::MIDW, pl.mt, pl.z};
     }
-    rc = llmk::launch_big_half<KIND, false>(p, st, "gemm_w4a16_nk(fused tiles)", workspace, workspace_bytes);
-    return true;
+    return {NkTiles::BIG, 0, llmk::splitk_factor_half(M, N, K)};
+}
+template <int KIND>
+int launch_nk_tiles(llmk::DirectArgs p, void* workspace, int64_t scratch, hipStream_t st) {
+    const NkTiles t = nk_tiles<KIND>(p);
+    if (t.form == NkTiles::BIG) return llmk::launch_big_half<KIND, false>(p, st, "gemm_w4a16_nk(fused tiles)", workspace, scratch);
+    if (t.z > 1 && scratch >= (int64_t)t.z * p.M * p.N * 4) { p.partial = (float*)workspace; p.ksplit = t.z; }
+    if (t.form == NkTiles::MID)
+        return t.mt == 4 ? llmk::launch_mid<KIND, 4>(p, st, "gemm_w4a16_nk(mid)") : llmk::launch_mid<KIND, 2>(p, st, "gemm_w4a16_nk(mid)");
+    return t.mt == 4 ? llmk::launch_mid<KIND, 4, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)")
+                     : llmk::launch_mid<KIND, 8, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)");
+}
+
+// The kernels of a call on the [N, K/8] layout, in the order in which they are preferred, and the scratch they use: what
+// llmk_gemm_w4a16_nk runs with `scratch` bytes there, and what llmk_gemm_w4a16_nk_workspace_bytes reports for any amount.
+struct NkPlan {
+    enum { RING, TILES, COPY, RANGES, STREAM, NONE } route;
+    int nz;
+    int64_t bytes;
+};
+NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scratch, bool c8) {
+    const int nz = (int)((K / 128 + 31) / 32);               // K ranges of the streaming kernels
+    const int64_t planes = nz > 1 ? (int64_t)nz * M * N * 4 : 0;
+    const bool sums = nz == 1 || ((M * N) % 4 == 0 && scratch >= planes);
+    llmk::DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
+    if (bf && M <= 64 && c8 && sums && nk_ring_ok(M, N, K, group, nz)) return {NkPlan::RING, nz, planes};
+    if (llmk::dma_eligible(p, 2)) {
+        if (w4_tiles_expand(M, N, K, scratch, true, bf) && group % 64 == 0) {
+            int z = bf ? nk_tiles<llmk::K_W4NKB>(p).z : nk_tiles<llmk::K_W4NK>(p).z;
+            if (M <= 64) z = max(z, llmk::splitk_factor_half(M, N, K));      // (w4_tiles_expand asks for these there)
+            return {NkPlan::TILES, 1, z > 1 ? (int64_t)z * M * N * 4 : 0};
+        }
+        // the 16-bit copy of W, and behind it whatever the 16-bit GEMM's K slices take
+        if ((M > 64 || bf) && scratch >= N * K * 2) return {NkPlan::COPY, 1, ((N * K * 2 + 255) & ~(int64_t)255) + (M <= 512 ? 8 * M * N * 4 : 0)};
+    }
+    if (bf) return {NkPlan::NONE, 1, 0};
+    // K > 4096: ranges of at most 4096 (each with resident activations) and fp32 partial sums
+    if (group % 128 == 0 && M <= 64 && nz > 1 && sums && c8 && ((K / 128 + nz - 1) / nz * 128) % group == 0) return {NkPlan::RANGES, nz, planes};
+    return {NkPlan::STREAM, 1, 0};
 }
 
 // launch shape of the Marlin-layout kernel for a given problem
@@ -988,7 +1016,7 @@ extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, 
     if (M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) LLMK_FAIL(LLMK_ERR_SHAPE, "gemm_w4a16_marlin: dimension too large");
 
     hipStream_t st = (hipStream_t)stream;
-    if (w4_tiles_expand(M, N, K, workspace, workspace_bytes) && K % 64 == 0 && groupsize % 64 == 0) {
+    if (w4_tiles_expand(M, N, K, usable_scratch(workspace, workspace_bytes)) && K % 64 == 0 && groupsize % 64 == 0) {
         // mid-size M: the 128-column tile kernels expand the Marlin units themselves (see gemm_w4a16_nk)
         llmk::DirectArgs p{};
         p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.b_s = s; p.c = c; p.c_dtype = LLMK_F16;
@@ -1049,6 +1077,13 @@ extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, 
     return LLMK_OK;
 }
 
+extern "C" int64_t llmk_gemm_w4a16_nk_workspace_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int ac_dtype) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
+    if (groupsize == -1) groupsize = (int)K;
+    if (groupsize < 8) return 0;
+    return nk_plan(M, N, K, groupsize, ac_dtype == LLMK_BF16, INT64_MAX, true).bytes;
+}
+
 extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* c, const void* s, int ac_dtype,
                                   int64_t M, int64_t N, int64_t K, int groupsize, void* workspace,
                                   int64_t workspace_bytes, void* stream) {
@@ -1067,47 +1102,41 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
     const _Float16* A = (const _Float16*)a;
     const _Float16* S = (const _Float16*)s;
     _Float16* C = (_Float16*)c;
-    // bf16: the weight-streaming ring kernel for decode sizes, everything else through the bf16 copy of W
-    const int nz_bf = (int)((K / 128 + 31) / 32);
-    const bool bf_ring = bf && M <= 64 && nk_ring_ok(M, N, K, groupsize, nz_bf) && !((uintptr_t)c & 7) &&
-                         (nz_bf == 1 || ((M * N) % 4 == 0 && workspace && workspace_bytes >= (int64_t)nz_bf * M * N * 4 &&
-                                         !((uintptr_t)workspace & 15)));
-    if (bf_ring) return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, nz_bf, (float*)workspace, true, st);
-    if (w4_tiles_expand(M, N, K, workspace, workspace_bytes, true, bf) && K % 64 == 0 && groupsize % 64 == 0) {
-        int rc = LLMK_OK;
-        const bool taken = bf ? launch_nk_tiles<llmk::K_W4NKB>(a, b_packed, c, s, ac_dtype, M, N, K, groupsize, workspace, workspace_bytes, st, rc)
-                              : launch_nk_tiles<llmk::K_W4NK>(a, b_packed, c, s, ac_dtype, M, N, K, groupsize, workspace, workspace_bytes, st, rc);
-        if (taken) return rc;
-    }
-    if ((M > 64 || bf) && K % 64 == 0 && workspace && workspace_bytes >= N * K * 2 && !((uintptr_t)workspace & 15)) {
-        // compute-bound: expand W once to fp16 / bf16 [N, K], then run the tiled MFMA GEMM on it
-        llmk::DirectArgs p{};
-        p.a = (const uint8_t*)a; p.b = (const uint8_t*)workspace; p.c = c; p.c_dtype = ac_dtype;
-        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
-        if (llmk::dma_eligible(p, 2)) {
+    const int64_t scratch = usable_scratch(workspace, workspace_bytes);
+    const NkPlan pl = nk_plan(M, N, K, groupsize, bf, scratch, !((uintptr_t)c & 7));
+    llmk::DirectArgs p{};
+    p.a = (const uint8_t*)a; p.c = c; p.c_dtype = ac_dtype;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
+    switch (pl.route) {
+        case NkPlan::RING:                               // bf16 decode; fp16 reaches that kernel through launch_nk_stream
+            return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, pl.nz, (float*)workspace, true, st);
+        case NkPlan::TILES:
+            p.b = (const uint8_t*)b_packed; p.b_s = s; p.group = groupsize;
+            return bf ? launch_nk_tiles<llmk::K_W4NKB>(p, workspace, scratch, st) : launch_nk_tiles<llmk::K_W4NK>(p, workspace, scratch, st);
+        case NkPlan::COPY: {
+            // compute-bound: expand W once to fp16 / bf16 [N, K], then run the tiled MFMA GEMM on it
+            p.b = (const uint8_t*)workspace;
             const unsigned blocks = (unsigned)cdiv64(N * (K / 8), 256);
             if (bf) nk_dequant_bf16_kernel<<<blocks, 256, 0, st>>>(b_packed, S, (unsigned short*)workspace, N, K, groupsize);
             else nk_dequant_kernel<<<blocks, 256, 0, st>>>(b_packed, S, (_Float16*)workspace, N, K, groupsize);
             LLMK_CHECK_LAUNCH("gemm_w4a16_nk(dequant)");
             const int64_t used = (N * K * 2 + 255) & ~(int64_t)255;
             void* rest = (uint8_t*)workspace + used;
-            const int64_t rest_bytes = workspace_bytes > used ? workspace_bytes - used : 0;
+            const int64_t rest_bytes = scratch > used ? scratch - used : 0;
             if (bf) return llmk::launch_big_half<llmk::K_BF16, false>(p, st, "gemm_w4a16_nk(tiled, bf16)", rest, rest_bytes);
             return llmk::launch_big_half<llmk::K_F16, false>(p, st, "gemm_w4a16_nk(tiled)", rest, rest_bytes);
         }
-    }
-    if (bf) LLMK_FAIL(LLMK_ERR_ARG, "gemm_w4a16_nk: this bf16 call needs a 16-byte aligned workspace of N*K*2 = %lld bytes (bf16 copy of W)",
+        case NkPlan::NONE:
+            LLMK_FAIL(LLMK_ERR_ARG, "gemm_w4a16_nk: this bf16 call needs a 16-byte aligned workspace of N*K*2 = %lld bytes (bf16 copy of W)",
                       (long long)(N * K * 2));
+        case NkPlan::RANGES:
+            return launch_nk_stream<1, 1>(A, b_packed, S, C, (int)M, (int)N, (int)K, groupsize, pl.nz, (float*)workspace, st);
+        case NkPlan::STREAM: break;
+    }
     if (groupsize % 128 == 0 && M <= 64) {
         // one 16-column block per tile: two blocks per tile (NT = 2) measured slower at every shape tried.
         // While the activations of a 16-row workgroup stay resident (K <= 4096), such workgroups side by side
         // beat taller ones by up to 2x.
-        // K > 4096: ranges of at most 4096 (each with resident activations) and fp32 partial sums, when the
-        // workspace holds them
-        const int nz = (int)((K / 128 + 31) / 32);
-        const bool ranges = nz > 1 && (M * N) % 4 == 0 && K % groupsize == 0 && ((K / 128 + nz - 1) / nz * 128) % groupsize == 0 &&
-                            workspace && workspace_bytes >= (int64_t)nz * M * N * 4 && !((uintptr_t)workspace & 15) && !((uintptr_t)c & 7);
-        if (ranges) return launch_nk_stream<1, 1>(A, b_packed, S, C, (int)M, (int)N, (int)K, groupsize, nz, (float*)workspace, st);
         if (M <= 16 || K <= 4096) return launch_nk_stream<1, 1>(A, b_packed, S, C, (int)M, (int)N, (int)K, groupsize, 1, nullptr, st);
         if (M <= 32) return launch_nk_stream<2, 1>(A, b_packed, S, C, (int)M, (int)N, (int)K, groupsize, 1, nullptr, st);
         return launch_nk_stream<4, 1>(A, b_packed, S, C, (int)M, (int)N, (int)K, groupsize, 1, nullptr, st);

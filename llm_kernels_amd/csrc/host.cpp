@@ -28,11 +28,11 @@ namespace {
     X(llmk_last_error) X(llmk_gemm_workspace_bytes) X(llmk_act_quant_fp8) X(llmk_act_quant_i8) X(llmk_comm_quant_fp8) \
     X(llmk_quant_i8_rowwise) X(llmk_gemm_fp8_block) X(llmk_gemm_i8_block) X(llmk_gemm_i8_rowcol) X(llmk_gemm_w4a8)    \
     X(llmk_gemm_w4a8_workspace_bytes) X(llmk_gemm_w4a16_marlin) X(llmk_gemm_w4a16_marlin_workspace_bytes)             \
-    X(llmk_gemm_w4a16_nk) X(llmk_moe_ep_preprocess) X(llmk_moe_pre_reorder_quant) X(llmk_moe_act_and_mul_quant)       \
-    X(llmk_moe_post_reorder) X(llmk_grouped_gemm) X(llmk_grouped_gemm_swiglu_quant)                                   \
-    X(llmk_grouped_gemm_swiglu_quant_fused) X(llmk_moe_softmax_topk) X(llmk_weight_quant_w4a8)                        \
-    X(llmk_weight_quant_i8_block) X(llmk_weight_quant_fp8_block) X(llmk_weight_dequant_fp8_block)                     \
-    X(llmk_weight_dequant_i8_block) X(llmk_weight_dequant_w4a8) X(llmk_quant_w4_nk)
+    X(llmk_gemm_w4a16_nk) X(llmk_gemm_w4a16_nk_workspace_bytes) X(llmk_moe_ep_preprocess)                             \
+    X(llmk_moe_pre_reorder_quant) X(llmk_moe_act_and_mul_quant) X(llmk_moe_post_reorder) X(llmk_grouped_gemm)         \
+    X(llmk_grouped_gemm_swiglu_quant) X(llmk_grouped_gemm_swiglu_quant_fused) X(llmk_moe_softmax_topk)                \
+    X(llmk_weight_quant_w4a8) X(llmk_weight_quant_i8_block) X(llmk_weight_quant_fp8_block)                            \
+    X(llmk_weight_dequant_fp8_block) X(llmk_weight_dequant_i8_block) X(llmk_weight_dequant_w4a8) X(llmk_quant_w4_nk)
 
 // one per imported module object: the package and the top-level module layout may both be imported
 struct State {
@@ -440,26 +440,12 @@ PyObject* w4a16_gemm(const Args& g) {
     const int64_t K = last_size(x), M = rows_of(x, K), N = w.size(0);
     require(w.size(1) * 8 == K, "packed weight must be [N, K/8]");
     require(x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16, "activations must be fp16 or bf16");
-    const bool bf = x.scalar_type() == at::kBFloat16;
-    // bf16 at decode size runs on the weight-streaming ring kernel under exactly the conditions the library
-    // checks (128-wide groups, K ranges of 4 to 32 steps, 8-byte aligned outputs, 32-bit lane offsets, and with more than
-    // one K range M * N % 4 == 0 for the summing pass);
-    // every other bf16 call goes through the bf16 copy of W and needs room for it
-    const int64_t steps = K / 128, nz = std::max<int64_t>(1, (steps + 31) / 32), per = (steps + nz - 1) / nz;
-    const bool ring_ok = group == 128 && per <= 32 && steps - (nz - 1) * per >= 4 &&
-                         N * (K / 2) < (1ll << 32) && M * K * 2 < (1ll << 32);
-    const bool bf_decode = bf && M <= 64 && ring_ok && (nz == 1 || (M * N) % 4 == 0);          // (the outputs are allocated here)
-    int64_t need = 0;
-    if (M > 64 || (bf && !bf_decode))
-        // fp16 / bf16 copy of W for the compute-bound path, split-K partials behind it for mid-size M
-        need = ((N * K * 2 + 255) / 256) * 256 + (M <= 512 ? 8 * M * N * 4 : 0);
-    else if (K > 4096 || M > 16)
-        need = std::max<int64_t>(8, (K + 4095) / 4096) * M * N * 4;                   // fp32 partial sums of K ranges / K slices
-    Scratch ws(g, x, need);
+    const int dt = float_code(x.scalar_type());
+    Scratch ws(g, x, g.st->llmk_gemm_w4a16_nk_workspace_bytes(M, N, K, group, dt));
     at::Tensor y;
     unlocked([&] {
         y = empty(with_last(x, N), x.scalar_type(), x);
-        g.check(g.st->llmk_gemm_w4a16_nk(x.data_ptr(), (const int32_t*)w.data_ptr(), y.data_ptr(), s.data_ptr(), float_code(x.scalar_type()), M, N, K, group, ws.get(), ws.bytes(), stream_of(x)),
+        g.check(g.st->llmk_gemm_w4a16_nk(x.data_ptr(), (const int32_t*)w.data_ptr(), y.data_ptr(), s.data_ptr(), dt, M, N, K, group, ws.get(), ws.bytes(), stream_of(x)),
                 "llmk_gemm_w4a16_nk", PyExc_AssertionError);
     });
     return wrap(std::move(y));

@@ -354,3 +354,41 @@ def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
     one[torch.arange(M), k] = 1.0
     y = w4a16.w4a16_gemm(one.bfloat16().to(dev), packed, s, gs)
     assert torch.equal(y.cpu(), deq.bfloat16().T[k])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M", [80, 300, 512])
+def test_w4a16_nk_expanding_tiles_hold_no_copy_of_the_weights(dev, dtype, M):
+    """The tiles that expand the packed words need room for split-K partial sums at most, not for a 16-bit copy of W."""
+    N, K = 14336, 4096
+    announce("w4a16_nk scratch", dtype, M, N, K)
+    torch.manual_seed(0)
+    packed, s, _ = w4a16.quantize_nk((torch.randn(N, K, device=dev) * 0.02).to(dtype), 128)
+    _lib.release_workspaces()
+    w4a16.w4a16_gemm(torch.randn(M, K, device=dev).to(dtype), packed, s, 128)
+    torch.cuda.synchronize()
+    assert sum(t.numel() for t in _lib._ws.values()) < N * K * 2
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,gs", [(16, 256, 4096, 128), (16, 256, 8192, 128), (40, 512, 4736, 128), (64, 9216, 4608, 128),
+                                      (33, 25600, 4096, 128), (48, 4096, 14336, 128), (100, 384, 2048, 64), (80, 512, 1024, 32),
+                                      (520, 1024, 1024, 128), (1300, 512, 512, 128)])
+def test_w4a16_nk_reported_scratch_is_what_the_call_uses(dev, dtype, M, N, K, gs):
+    """The reported number of bytes gives the bits that any larger workspace gives, and nothing behind it is written."""
+    announce("w4a16_nk reported scratch", dtype, M, N, K, gs)
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=dev).to(dtype)
+    packed, s, _ = w4a16.quantize_nk(torch.randn(N, K, device=dev) * 0.02, gs)
+    need = _lib.load().llmk_gemm_w4a16_nk_workspace_bytes(M, N, K, gs, _lib.dt(dtype))
+    room = max(need, N * K * 2 + 8 * M * N * 4) + 256
+    guard = torch.full((room + 256,), 0x5A, dtype=torch.uint8, device=dev)
+    outs = []
+    for n in (need, room):
+        y = torch.empty(M, N, dtype=dtype, device=dev)
+        _lib.call("llmk_gemm_w4a16_nk", _lib.ptr(x), _lib.ptr(packed), _lib.ptr(y), _lib.ptr(s), _lib.dt(dtype), M, N, K, gs,
+                  _lib.ptr(guard) if n else None, n, _lib.stream(x))
+        torch.cuda.synchronize()
+        assert (guard[n:] == 0x5A).all()
+        outs.append(y)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
