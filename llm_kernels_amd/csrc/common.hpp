@@ -17,6 +17,7 @@ typedef _Float16 v2h  __attribute__((ext_vector_type(2)));
 typedef _Float16 v4h  __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h  __attribute__((ext_vector_type(8)));
 typedef __bf16   v8bf __attribute__((ext_vector_type(8)));
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
 typedef unsigned short v8us __attribute__((ext_vector_type(8)));
 
 #define LLMK_WAVE 64

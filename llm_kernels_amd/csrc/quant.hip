@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void weight_quant_w4a8_kernel(const void* __re
                                                                 unsigned short* __restrict__ s, int8_t* __restrict__ s4,
                                                                 int8_t* __restrict__ z4, int64_t N, int64_t K) {
     constexpr float QMAX = 119.f;
-    __shared__ float red[4];
+    __shared__ unsigned red[4];
     const int t = threadIdx.x;
     const int64_t r0 = (int64_t)blockIdx.y * 128 + (t >> 4) * 8, c0 = (int64_t)blockIdx.x * 128 + (t & 15) * EPL;
     const bool live = r0 < N;                            // N is a multiple of 8: a thread's rows exist together
@@ -258,29 +258,47 @@ __global__ __launch_bounds__(256) void weight_quant_w4a8_kernel(const void* __re
 #pragma unroll
         for (int h = 0; h < CHUNKS; ++h)
             raw[j][h] = live ? ((const uint4*)((const uint8_t*)x + ((r0 + j) * K + c0) * (DT == LLMK_F32 ? 4 : 2)))[h] : make_uint4(0, 0, 0, 0);
-    float m = 0.f;
-    if constexpr (DT == LLMK_F16) {                      // two magnitudes per instruction
-        v2h mm = {(_Float16)0, (_Float16)0};
+    // The largest magnitude, by bit patterns, which order as integers (16 bits: two per instruction).  A floating-point
+    // maximum drops a quiet NaN, but of a signalling one it returns the quieted NaN, and the next maximum drops with it
+    // what the lane had seen before.  A NaN orders above infinity: a block that holds one looks again without.
+    constexpr unsigned INF = DT == LLMK_F32 ? 0x7f800000u : (DT == LLMK_F16 ? 0x7c00u : 0x7f80u);
+    auto largest = [&](auto drop_nan) __attribute__((always_inline)) {
+        constexpr bool DROP = decltype(drop_nan)::value;
+        unsigned top = 0;
+        v2us top2 = {0, 0};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const unsigned w[4] = {raw[j][0].x, raw[j][0].y, raw[j][0].z, raw[j][0].w};
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) asm("v_pk_max_f16 %0, %0, %1" : "+v"(mm) : "v"(w[e] & 0x7fff7fffu));
-        }
-        m = fmaxf((float)mm[0], (float)mm[1]);
-    } else {
+            for (int h = 0; h < CHUNKS; ++h) {
+                const unsigned w[4] = {raw[j][h].x, raw[j][h].y, raw[j][h].z, raw[j][h].w};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            float v[EPL];
-            load8<DT>(&raw[j][0], 0, v);
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) m = fmaxf(m, fabsf(v[e]));
-        }
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (DT == LLMK_F32) {
+                        const unsigned a = w[e] & 0x7fffffffu;
+                        top = max(top, DROP && a > INF ? 0u : a);
+                    } else {
+                        unsigned a = w[e] & 0x7fff7fffu;
+                        if constexpr (DROP) a = ((a & 0xffffu) > INF ? 0u : a & 0xffffu) | ((a >> 16) > INF ? 0u : a & 0xffff0000u);
+                        v2us a2;
+                        __builtin_memcpy(&a2, &a, 4);
+                        top2 = __builtin_elementwise_max(top2, a2);
+                    }
+                }
+            }
+        return DT == LLMK_F32 ? top : max((unsigned)top2[0], (unsigned)top2[1]);
+    };
+    auto over_block = [&](unsigned top) __attribute__((always_inline)) {
+        top = (unsigned)group_imax<64>((int)top);
+        if ((t & 63) == 0) red[t >> 6] = top;
+        __syncthreads();
+        return max(max(red[0], red[1]), max(red[2], red[3]));
+    };
+    unsigned top = over_block(largest(std::false_type{}));
+    if (top > INF) {
+        __syncthreads();
+        top = over_block(largest(std::true_type{}));
     }
-    m = group_max<64>(m);
-    if ((t & 63) == 0) red[t >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float m = DT == LLMK_F32 ? __uint_as_float(top) : (DT == LLMK_F16 ? f16_to_f32((unsigned short)top) : bf16_to_f32((unsigned short)top));
     const float sc = m / QMAX;
     const bool fast = div_by_ok(sc);
     const float rcp = fast ? 1.0f / sc : 0.f;

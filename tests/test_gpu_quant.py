@@ -178,3 +178,37 @@ def test_w4a8_weight_quant_in_one_pass(dev, dtype, N, K, group):
     want = torch.from_numpy(bp.pack_rows(y.cpu().numpy().astype("uint8"), 4, 32)[0])
     assert torch.equal(packed.cpu(), want)
     assert torch.equal(s, s_ref) and torch.equal(s4, s4_ref) and torch.equal(z4, z4_ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_w4a8_weight_quant_in_one_pass_of_nan_and_infinity(dev, dtype):
+    """NaN of both kinds and infinities among ordinary weights, in blocks of zeros and alone in a block: what the two level
+    kernels and the packing give one after the other."""
+    announce("w4a8 weight_quant one pass, NaN and infinity", dtype)
+    torch.manual_seed(5)
+    N, K = 264, 640
+    bits = {torch.float32: torch.int32, torch.float16: torch.int16, torch.bfloat16: torch.int16}[dtype]
+    quiet, signal = {torch.float32: (0x7fc00001, 0x7f800001), torch.float16: (0x7e01, 0x7c01), torch.bfloat16: (0x7fc1, 0x7f81)}[dtype]
+    w = (torch.randn(N, K) * 0.02).to(dtype)
+    w[128:256, 256:384] = 0
+    w[128, 5], w[2, 301] = 0.25, -0.25                   # the largest weight of a block, in front of a signalling NaN
+    v = w.view(bits)
+    for r, c, b in ((0, 0, quiet), (5, 127, quiet), (130, 5, signal), (255, 127, signal), (131, 260, quiet), (140, 300, signal),
+                    (4, 301, signal), (257, 513, signal)):
+        v[r, c] = b
+        v[r - 1 if r else 1, c] = b | (-2 ** 31 if bits == torch.int32 else -2 ** 15)      # and its negative
+    w[7, 128 + 3], w[200, 128 + 9], w[201, 128 + 11] = float("inf"), float("inf"), float("-inf")
+    w[260:, 384:512] = float("nan")                      # a block of nothing else (its last, partial rows)
+    w[256:260, 384:512] = float("nan")
+    wd = w.to(dev)
+    packed, s, s4, z4 = w4a8_kernel.weight_quant(wd)
+    y = torch.empty(N, K, dtype=torch.int8, device=dev)
+    s_ref, s4_ref, z4_ref = torch.empty_like(s), torch.empty_like(s4), torch.empty_like(z4)
+    _lib.call("llmk_weight_quant_i8_block", _lib.ptr(wd), _lib.dt(dtype), _lib.ptr(y), _lib.ptr(s_ref), N, K, 128, 119.0,
+              _lib.ROUND_HALF_UP, 1, None)
+    _lib.call("llmk_weight_quant_w4a8_level2", _lib.ptr(y), _lib.ptr(s4_ref), _lib.ptr(z4_ref), N, K, 128, None)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(bp.pack_rows(y.cpu().numpy().astype("uint8"), 4, 32)[0])
+    assert torch.equal(s.view(torch.int16), s_ref.view(torch.int16))
+    assert torch.equal(s4, s4_ref) and torch.equal(z4, z4_ref)
+    assert torch.equal(packed.cpu(), want)
