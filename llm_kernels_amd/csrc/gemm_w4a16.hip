@@ -573,7 +573,11 @@ __global__ __launch_bounds__(512) void w4a16_nk_stream_kernel(
 // fragment of constant 136 (the same for every tile).
 // (U = 4 for every K before; us per call: 16 x 28672 x 1024 13.6 -> 6.9, fp16 60 x 28672 x 1024 43.2 -> 15.6, 16 x 25600 x 1408
 // 13.9 -> 9.4, 16 x 4096 x 1024 5.2 -> 3.3, 60 x 15368 x 3072 25.0 -> 20.4, 3 x 4672 x 9088 in three ranges 14.9 -> 12.8.)
-template <int DEPTH, int U, bool BF = false>
+// FULL: every range is 8 U steps, so no share is moved back and nothing counts as zero.  The general form's selects cost such
+// a range up to 1.7 % (us, cold weights, before it | with it | FULL: bf16 16 x 6144 x 4096 7.73 | 7.86 | 7.72, 48 x 4096 x 4096
+// 10.57 | 10.70 | 10.55, 16 x 4096 x 4096 5.92 | 5.95 | 5.94; fp16 7.82 | 7.86 | 7.76).  Taken for U = 4, the range of 4096
+// elements: with U = 2 it measured slower (bf16 16 x 4096 x 2048 4.15 -> 4.37).
+template <int DEPTH, int U, bool FULL, bool BF>
 __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     const unsigned short* __restrict__ A, const int32_t* __restrict__ B, const _Float16* __restrict__ S,
     unsigned short* __restrict__ C, int M, int N, int Kfull, int Kc, float* __restrict__ partial) {
@@ -587,8 +591,8 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
     const int steps = K >> 7, ngroups = Kfull >> 7, kwords = Kfull >> 3;
     const int m0 = blockIdx.y * 16;
     const int ntiles = (N + 15) >> 4;
-    const int s0 = min(U * wave, steps - U);             // first step this wave loads
-    const int u0 = min(U * wave - s0, U);                // steps s0 .. s0 + u0 - 1 belong to other waves
+    const int s0 = FULL ? U * wave : min(U * wave, steps - U);           // first step this wave loads
+    const int u0 = FULL ? 0 : min(U * wave - s0, U);     // steps s0 .. s0 + u0 - 1 belong to other waves
 
     // ---- activations, requested first: row i of the wave's K slice (512 elements = 1 KiB) is one fully
     // coalesced load.  (Fetching the MFMA fragments straight from global memory costs 2 us per launch: every
@@ -652,7 +656,7 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
                 a[4 * u + j] = y;
             }
         }
-        if (u0 > 0) {
+        if (!FULL && u0 > 0) {
 #pragma unroll
             for (int i = 0; i < 4 * U; ++i)
                 if (i < 4 * u0) a[i] = (v4i){0, 0, 0, 0};
@@ -685,7 +689,7 @@ __global__ __launch_bounds__(512) void w4a16_nk_ring_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const unsigned sraw = (U < 4 ? (unsigned)(sc4 >> (16 * u)) : (unsigned)(u < 2 ? ts[0] : ts[1]) >> (16 * (u & 1))) & 0xffffu;
-            const float sc = u < u0 ? 0.f : f16_to_f32((unsigned short)sraw);
+            const float sc = !FULL && u < u0 ? 0.f : f16_to_f32((unsigned short)sraw);
             v4f t = bias[u];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -801,9 +805,16 @@ int launch_nk_ring(const void* A, const int32_t* B, const _Float16* S, void* C, 
     auto ring = [&](auto uc) {
         constexpr int U = decltype(uc)::value;
         auto run = [&](auto kern) { kern<<<rgrid, 512, rsmem, st>>>(a16, B, S, c16, M, N, K, Kc, part); };
-        if (per_wg >= 4) bf ? run(w4a16_nk_ring_kernel<4, U, true>) : run(w4a16_nk_ring_kernel<4, U, false>);
-        else if (per_wg == 3) bf ? run(w4a16_nk_ring_kernel<3, U, true>) : run(w4a16_nk_ring_kernel<3, U, false>);
-        else bf ? run(w4a16_nk_ring_kernel<2, U, true>) : run(w4a16_nk_ring_kernel<2, U, false>);
+        auto form = [&](auto full) {
+            constexpr bool FULL = decltype(full)::value;
+            if (per_wg >= 4) bf ? run(w4a16_nk_ring_kernel<4, U, FULL, true>) : run(w4a16_nk_ring_kernel<4, U, FULL, false>);
+            else if (per_wg == 3) bf ? run(w4a16_nk_ring_kernel<3, U, FULL, true>) : run(w4a16_nk_ring_kernel<3, U, FULL, false>);
+            else bf ? run(w4a16_nk_ring_kernel<2, U, FULL, true>) : run(w4a16_nk_ring_kernel<2, U, FULL, false>);
+        };
+        if constexpr (U == 4) {
+            if (steps == 8 * U && steps_all == nz * steps) return form(std::true_type{});
+        }
+        form(std::false_type{});
     };
     if (steps <= 8) ring(std::integral_constant<int, 1>{});
     else if (steps <= 16) ring(std::integral_constant<int, 2>{});

@@ -333,6 +333,13 @@ def test_w4a16_nk_decode_any_number_of_steps(dev, dtype, M, N, K):
         assert torch.equal(y[0].nan_to_num(0.0), ref[0].nan_to_num(0.0))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 4096), (17, 136, 4096), (64, 2600, 4096), (64, 5000, 4096), (16, 1000, 8192), (3, 72, 12288)])
+def test_w4a16_nk_decode_full_ranges(dev, dtype, M, N, K):
+    """Ranges of 32 steps, the form of the ring kernel without shares to move: every ring depth, one range and several."""
+    test_w4a16_nk_decode_any_number_of_steps(dev, dtype, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K,gs", [(65, 72, 128, 64), (130, 4096, 1024, 128), (512, 264, 4096, 128), (300, 14344, 512, 128),
                                       (200, 20000, 640, 128), (500, 8192, 384, 192), (600, 10000, 1024, 128), (1024, 28672, 256, 128)])
 def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
