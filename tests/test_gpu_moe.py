@@ -73,6 +73,40 @@ def test_router_breaks_ties_by_index(dev):
     assert ids.tolist() == [[0, 1, 2]] * 5 and torch.allclose(w, torch.full_like(w, 1 / 3))
 
 
+@pytest.mark.parametrize("E,topk", [(12, 12), (64, 9), (65, 64), (130, 9), (200, 64), (512, 64)])
+def test_router_breaks_ties_by_index_across_lanes(dev, E, topk):
+    """All equal, and two levels spread over the lanes and the experts of a lane: lower index first within a level."""
+    announce("router ties across lanes", E, topk)
+    torch.manual_seed(E)
+    logits = torch.randint(0, 2, (7, E)).float()
+    logits[0] = 0.25
+    ids, _ = softmax_topk_router(logits.to(dev), topk)
+    want = torch.sort(logits, dim=-1, descending=True, stable=True)[1][:, :topk]
+    assert torch.equal(ids.cpu(), want)
+
+
+@pytest.mark.parametrize("E,topk", [(5, 5), (8, 2), (33, 4), (64, 8), (200, 16)])
+def test_router_rows_of_nan_and_infinity(dev, E, topk):
+    """A NaN or +inf logit makes the row's softmax NaN, as torch's; its ids are distinct experts, other rows are untouched."""
+    announce("router NaN", E, topk)
+    torch.manual_seed(E)
+    clean = torch.randn(9, E)
+    logits = clean.clone()
+    logits[1, E - 1] = float("nan")
+    logits[4, 0] = float("inf")
+    logits[6] = float("-inf")
+    logits[7, : E - topk] = float("-inf")                # probabilities of zero behind the topk
+    ids, w = softmax_topk_router(logits.to(dev), topk)
+    ref, rid = torch.topk(torch.softmax(logits.double(), -1), topk, dim=-1)
+    for r in (1, 4, 6):
+        assert w[r].isnan().all() and ref[r].isnan().all()
+        assert sorted(set(ids[r].tolist())) == sorted(ids[r].tolist()) and 0 <= int(ids[r].min()) and int(ids[r].max()) < E
+    keep = [0, 2, 3, 5, 7, 8]
+    assert torch.equal(ids.cpu()[keep], rid[keep])
+    ids0, w0 = softmax_topk_router(clean.to(dev), topk)
+    assert torch.equal(ids[[0, 2, 3, 5, 8]], ids0[[0, 2, 3, 5, 8]]) and torch.equal(w[[0, 2, 3, 5, 8]], w0[[0, 2, 3, 5, 8]])
+
+
 def test_router_takes_any_number_of_rows(dev):
     """More rows than one launch takes: the rows on both sides of the launches' border get what a call of their own gives."""
     announce("router rows", 2 ** 24 + 37)
