@@ -116,6 +116,9 @@ class _Host:
         spec = importlib.util.spec_from_file_location("llmk_host", HOST_PATH)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
+        if mod.torch_version != torch.__version__:
+            raise LlmkError("llmk_host.so was built against torch %s, this is %s. Run `python -m llm_kernels_amd.build`"
+                            % (mod.torch_version, torch.__version__))
         mod.bind(LIB_PATH, LlmkError, _ws)
         for k, v in vars(mod).items():
             if not k.startswith("__"):

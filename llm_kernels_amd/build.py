@@ -49,7 +49,8 @@ def _host_module():
     inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
            sysconfig.get_paths()["include"]]
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           '-DLLMK_TORCH_VERSION="%s"' % torch.__version__]
     for d in inc:
         cmd += ["-isystem", d]
     cmd += [os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + os.path.join(t, "lib"), "-lc10", "-ltorch_cpu", "-ltorch", "-lc10_hip",

@@ -701,7 +701,9 @@ int clear(PyObject* self) {
     if (st) { Py_CLEAR(st->error); Py_CLEAR(st->workspaces); }
     return 0;
 }
-PyModuleDef_Slot slots[] = {{0, nullptr}};
+// the torch this module's C++ interface is that of: the loader refuses another
+int exec(PyObject* self) { return PyModule_AddStringConstant(self, "torch_version", LLMK_TORCH_VERSION); }
+PyModuleDef_Slot slots[] = {{Py_mod_exec, (void*)exec}, {0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "llmk_host", nullptr, sizeof(State), methods, slots, traverse, clear, nullptr};
 
 }  // namespace

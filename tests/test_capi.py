@@ -59,6 +59,30 @@ def test_product_refuses_cpu_tensors():
         bitpack.pack_weights_over_rows(torch.zeros(8, 8, dtype=torch.uint8), 4, 32, False)
 
 
+@pytest.mark.parametrize("what", ["host module missing", "library missing", "another torch"])
+def test_smoke_builds_what_cannot_be_loaded(monkeypatch, what):
+    import torch
+    import __graft_entry__
+
+    class Built(Exception):
+        pass
+
+    def build():
+        raise Built
+
+    monkeypatch.setattr(__graft_entry__, "build", build)
+    monkeypatch.setattr(_lib, "host", _lib._Host())               # nothing loaded yet
+    if what == "host module missing":
+        monkeypatch.setattr(_lib, "HOST_PATH", "/nonexistent/llmk_host.so")
+    elif what == "library missing":
+        monkeypatch.setattr(_lib, "_lib", None)
+        monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libllmk_gfx950.so")
+    else:
+        monkeypatch.setattr(torch, "__version__", "0.0")
+    with pytest.raises(Built):
+        __graft_entry__.smoke()
+
+
 def test_release_workspaces_drops_the_cached_scratch():
     saved = dict(_lib._ws)
     try:
