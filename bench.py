@@ -1,11 +1,12 @@
 #!/usr/bin/env python3
 """Throughput of the quantized-GEMM path on one MI355X, against its roofline, with a CPU baseline.
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME] [--headline-only] [--no-cpu] [--eager]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME] [--headline-only] [--no-cpu] [--eager] [--details FILE]
 
 A "step" is one GEMM call over one batch of synthetic input already resident in HBM.  Small-M
 (HBM-bound) workloads rotate through enough distinct weight copies to exceed the 256 MB on-die cache,
-so the figure is an HBM figure and not a cache figure.  Rank 0 prints ONE JSON line.
+so the figure is an HBM figure and not a cache figure.  Rank 0 prints ONE JSON line of at most MAX_LINE
+characters: the headline in full, the other cases one short record each; --details FILE writes everything measured.
 """
 import argparse
 import json
@@ -592,7 +593,9 @@ def calibration(dev):
     """What this box sustains on the two resources the roofline prices against, from the library's calibration
     kernels (llmk_calib_mfma: nothing but matrix instructions on random register operands, eight waves per CU;
     llmk_calib_read: a read without arithmetic, linear and with the decode kernels' addresses, of 1 GiB, four
-    times the memory-side cache).  Reported beside the published peaks, never instead of them."""
+    times the memory-side cache).  Reported beside the published peaks, never instead of them: roofline.peak stays HBM 8000
+    GB/s, fp8 / int8 5000 and fp16 / bf16 2500 TFLOP/s, which assume the 2400 MHz peak engine clock, where the clocks
+    reported here are what the chip holds under each load."""
     from llm_kernels_amd import _lib
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     st = _lib.stream(torch.empty(1, device=dev))
@@ -631,10 +634,11 @@ def calibration(dev):
     a, a_s = fp8_kernel.act_quant(torch.randn(M, K, device=dev).bfloat16())
     b, b_s = fp8_kernel.weight_quant(torch.randn(N, K, device=dev) * 0.02)
     c = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
-    wsp, wsn = _lib.gemm_workspace(dev, M, N, K)
+    wsn = _lib.load().llmk_gemm_workspace_bytes(M, N, K)
+    ws = torch.empty(max(wsn, 16), dtype=torch.uint8, device=dev)
     clocks.zero_()
     gemm = lambda: _lib.call("llmk_calib_gemm_fp8_clock", _lib.ptr(a), _lib.ptr(a_s), _lib.ptr(b), _lib.ptr(b_s), _lib.ptr(c),
-                             _lib.BF16, M, N, K, wsp, wsn, _lib.ptr(clocks), st)
+                             _lib.BF16, M, N, K, _lib.ptr(ws), wsn, _lib.ptr(clocks), st)
     for _ in range(50):
         gemm()
     dt_s = timed(gemm, reps=9)
@@ -651,10 +655,27 @@ def calibration(dev):
     for name, pattern, wgs in (("hbm_read_linear_gbs", 0, cus * 8), ("hbm_read_decode_tiles_gbs", 1, cus)):
         dt_s = timed(lambda: _lib.call("llmk_calib_read", _lib.ptr(_flush_buf), _flush_buf.numel(), pattern, _lib.ptr(sink), wgs, st))
         res[name] = round(_flush_buf.numel() / dt_s / 1e9, 1)
-    res["note"] = ("sustained rates of this box by the library's calibration kernels; roofline.peak stays the published "
-                   "figure (HBM 8000 GB/s; fp8 / int8 5000, fp16 / bf16 2500 TFLOP/s, which assume the 2400 MHz peak "
-                   "engine clock: the shader clocks above are what the chip holds under each load)")
     return res
+
+
+MAX_LINE = 7000           # characters of the printed line: logs that keep the last 8000 of the output have it whole
+
+
+def short_case(r):
+    """What the printed line carries of one of the other cases: time, rate and share of the roofline."""
+    out = {"workload": r["workload"], "us": r["us_per_launch"], "us_min": r["us_per_launch_min"], "us_max": r["us_per_launch_max"],
+           "achieved": r["roofline"]["achieved"], "unit": r["roofline"]["unit"], "frac": r["roofline"]["frac"]}
+    if r.get("cpu_baseline"):
+        out["cpu"] = r["cpu_baseline"]["value"]          # TFLOP/s (GB/s for a streaming operator)
+    return out
+
+
+def result_line(out):
+    """The one JSON line: `out` with its cases shortened."""
+    line = dict(out)
+    if "cases" in out:
+        line["cases"] = [short_case(r) for r in out["cases"]]
+    return json.dumps(line, separators=(",", ":"))
 
 
 def main():
@@ -667,6 +688,7 @@ def main():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-calibration", action="store_true", help="skip the sustained-MFMA / HBM-read calibration kernels")
     ap.add_argument("--eager", action="store_true", help="launch every step from Python instead of replaying a HIP graph")
+    ap.add_argument("--details", metavar="FILE", help="write every field of every case to FILE (JSON)")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py measures one GPU: this path has no multi-GPU part (run with --gpus 1)", file=sys.stderr)
@@ -745,7 +767,10 @@ def main():
     }
     if cases:
         out["cases"] = cases
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(result_line(out))
 
 
 if __name__ == "__main__":

@@ -42,3 +42,33 @@ def test_stream_workload_oracle_passes_run_on_host_inputs():
     assert set(host) == set(ops)
     for name, args in host.items():
         assert ops[name][2](*args) is not None, name
+
+
+def _record(name, unit):
+    """A record of the form bench.record() returns, every number as long as it gets."""
+    return {"workload": name, "M": 4096, "N": 128256, "K": 14336, "us_per_launch": 12345.67, "us_per_launch_min": 12345.67,
+            "us_per_launch_max": 12345.67, "timed_replays": 7, "preroll_ms": 1234.5, "preroll_replays": 12345,
+            "cache_flushed_before_each_replay": True, "us_per_launch_without_flush": 12345.67, "tflops": 12345.67, "gbs": 12345.6,
+            "alg_bytes": 10 ** 12, "flops": 1.234567890123456e+16, "weight_copies_rotated": 123, "wall_ms_per_step": 1234.5678,
+            "roofline": {"bound": "mfma", "achieved": 12345.6, "peak": 5000.0, "unit": unit, "frac": 0.1234, "traffic": 10 ** 12},
+            "cpu_baseline": {"value": 12.3456, "unit": unit, "cores": 16, "kind": "port", "cpu_model": "x" * 60, "sample": "x" * 250,
+                             "matmul_only_value": 12.3456}}
+
+
+def test_the_printed_line_fits_what_a_reader_keeps():
+    """The longest default run and the longest run of the streaming operators, and the keys a reader looks for."""
+    import json
+    head = {"metric": "m" * 80, "value": 12345.67, "unit": "TFLOP/s", "n_gpus": 1, "steps": 20000, "warmup": 20000,
+            "ms_per_step": 12.34567, "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "fp8_e4m3",
+            "data": "synthetic", "config": {"k%d" % i: "v" * 20 for i in range(20)}}
+    calib = {"a_name_of_the_usual_length_of_a_rate_%d" % i: 12345.6 for i in range(16)}
+    for names, unit in ((bench.HEADLINE_SET, "TFLOP/s"), (bench.STREAM_WORKLOADS, "GB/s")):
+        r = _record(names[0], unit)
+        out = dict(head, roofline=r["roofline"], cpu_baseline=r["cpu_baseline"], calibration=calib,
+                   cases=[_record(n, unit) for n in names])
+        line = bench.result_line(out)
+        assert len(line) < bench.MAX_LINE and "\n" not in line
+        got = json.loads(line)
+        assert all(got[k] == v for k, v in head.items()) and got["roofline"] == r["roofline"]
+        assert [c["workload"] for c in got["cases"]] == list(names)
+        assert all(c["us"] == 12345.67 and c["unit"] == unit and c["frac"] == 0.1234 for c in got["cases"])
