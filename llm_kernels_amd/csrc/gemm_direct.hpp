@@ -545,17 +545,17 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
     const bool vec = CAN_VEC && !resident && steps % 4 == 0;
     // short K: a batch of four steps per wave would mostly repeat the last step (K = 1408: 32 requests for 11 steps)
     constexpr int SU1 = MT == 1 ? 1 : 0, SU2 = MT == 1 ? 2 : 0, SU3 = MT == 1 ? 3 : 0;
-    const int variant = MT == 1 && steps <= 3 * NW ? 2 + (steps + NW - 1) / NW : (resident ? 1 : 0);
-    static std::atomic<int> slots_cache[6];   // resident workgroups on the whole device, per kernel variant
+    const int variant = MT == 1 && steps <= 3 * NW ? 1 + (steps + NW - 1) / NW : (resident ? 1 : 0);
+    static std::atomic<int> slots_cache[5];   // resident workgroups on the whole device, per kernel variant
     int slots = slots_cache[variant].load(std::memory_order_relaxed);
     if (slots == 0) {
         int dev = 0, cus = 0, per_cu = 0;
         hipError_t e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess)
-            e = variant == 2 || variant == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1>, NW * 64, 64 * 1024)
-                : variant == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2>, NW * 64, 64 * 1024)
-                : variant == 5 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3>, NW * 64, 64 * 1024)
+            e = variant == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1>, NW * 64, 64 * 1024)
+                : variant == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2>, NW * 64, 64 * 1024)
+                : variant == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3>, NW * 64, 64 * 1024)
                 : resident ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT>, NW * 64, 64 * 1024)
                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT>, NW * 64, 64 * 1024);
         if (e != hipSuccess) LLMK_FAIL(LLMK_ERR_LAUNCH, "%s: occupancy query failed: %s", name, hipGetErrorString(e));
@@ -574,9 +574,9 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
             return LLMK_OK;
         }
     }
-    if (variant == 2 || variant == 3) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1><<<grid, block, smem, stream>>>(p);
-    else if (variant == 4) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2><<<grid, block, smem, stream>>>(p);
-    else if (variant == 5) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3><<<grid, block, smem, stream>>>(p);
+    if (variant == 2) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1><<<grid, block, smem, stream>>>(p);
+    else if (variant == 3) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2><<<grid, block, smem, stream>>>(p);
+    else if (variant == 4) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3><<<grid, block, smem, stream>>>(p);
     else if (resident) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT><<<grid, block, smem, stream>>>(p);
     else gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT><<<grid, block, smem, stream>>>(p);
     LLMK_CHECK_LAUNCH(name);
@@ -599,8 +599,24 @@ int launch_direct_mt(const DirectArgs& p, hipStream_t stream, const char* name) 
     }
 }
 
+// K = 0: every sum is empty, the outputs of the rows (grouped: of the segments' rows) are zero.  A kernel of its own, because
+// the others clamp a step past the end to the last one, which there is none of.
+template <bool GROUPED>
+__global__ void empty_sums_kernel(DirectArgs p) {
+    const int64_t r0 = GROUPED ? p.seg_indptr[0] : 0, r1 = GROUPED ? p.seg_indptr[p.E] : p.M;
+    for (int64_t i = r0 * p.N + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < r1 * p.N; i += (int64_t)gridDim.x * blockDim.x) {
+        if (p.c) st_out(p.c, i, 0.f, p.c_dtype);
+        if (p.c_i32) p.c_i32[i] = 0;
+    }
+}
+
 template <int KIND, bool GROUPED>
 int launch_direct(const DirectArgs& p, int max_rows_per_segment_hint, hipStream_t stream, const char* name) {
+    if (p.K == 0) {
+        empty_sums_kernel<GROUPED><<<1024, 256, 0, stream>>>(p);
+        LLMK_CHECK_LAUNCH(name);
+        return LLMK_OK;
+    }
     // m-tiles per workgroup: 1 for decode-sized M, up to 4 otherwise.  When a wave's K share fits one batch at
     // one m-tile per workgroup (activations resident in registers), 16-row workgroups side by side beat taller
     // ones that have to re-read their activations for every column tile.

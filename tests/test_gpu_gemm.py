@@ -3,6 +3,8 @@
 Tolerance: |c - ref| <= 1e-2 * rms(ref) + 1e-2 * |ref| (rtol 1e-2 / atol 1e-2 relative to the output
 scale).  Integer accumulators are checked bit-exactly.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -491,3 +493,27 @@ def test_large_tiles_split_last_round(dev, kind, M, N, K, out):
     got = c.double().sum(0).cpu()
     ref_rms = g.gemm_blockwise(a[rows], a_s[rows], b, b_s).pow(2).mean().sqrt().item()
     assert bool(((got - want).abs() <= 1e-2 * ref_rms * (M ** 0.5) + 1e-2 * want.abs()).all()), "column sums"
+
+
+@pytest.mark.parametrize("M", [1, 40, 65, 600])
+def test_empty_sums_are_zero(dev, M):
+    """K = 0 through the C ABI: nothing is read, the outputs are zeros (grouped: of the segments' rows)."""
+    announce("K = 0", M)
+    N = 200
+    pad = torch.zeros(1 << 16, dtype=torch.uint8, device=dev)     # operands of no elements, somewhere in memory
+    mid = ctypes.c_void_p(pad.data_ptr() + (1 << 15))
+    st = _lib.stream(pad)
+    for dt in (torch.float32, torch.bfloat16):
+        for name, scales in (("llmk_gemm_fp8_block", ()), ("llmk_gemm_i8_block", (_lib.F16,))):
+            c = torch.full((M, N), 7.0, dtype=dt, device=dev)
+            _lib.call(name, mid, mid, mid, mid, *scales, _lib.ptr(c), _lib.dt(dt), M, N, 0, None, 0, st)
+            assert (c == 0).all()
+        c, acc = torch.full((M, N), 7.0, dtype=dt, device=dev), torch.full((M, N), 7, dtype=torch.int32, device=dev)
+        _lib.call("llmk_gemm_i8_rowcol", mid, mid, mid, mid, _lib.ptr(c), _lib.dt(dt), _lib.ptr(acc), M, N, 0, None, 0, st)
+        assert (c == 0).all() and (acc == 0).all()
+        for kind, sdt in ((_lib.KIND_I8, _lib.F16), (_lib.KIND_FP8, _lib.F32), (_lib.KIND_BF16, 0)):
+            c = torch.full((M + 2, N), 7.0, dtype=dt, device=dev)
+            seg = torch.tensor([1, 1 + M // 2, 1 + M // 2, 1 + M], dtype=torch.int64, device=dev)
+            _lib.call("llmk_grouped_gemm", mid, mid, _lib.ptr(c), kind, _lib.dt(dt), 3, M + 2, N, 0, _lib.ptr(seg), None, mid, mid, sdt,
+                      None, 0, st)
+            assert (c[1:-1] == 0).all() and (c[0] == 7).all() and (c[-1] == 7).all()
