@@ -161,29 +161,8 @@ def call(name, *args, exc=LlmkError):
     return rc
 
 
-def gemm_workspace(device, M, N, K):
-    """(pointer, nbytes) of the optional GEMM scratch for this shape, (None, 0) when none is needed."""
-    n = load().llmk_gemm_workspace_bytes(M, N, K)
-    if n <= 0:
-        return None, 0
-    buf = workspace(device, n)
-    # the size asked for, not the size of the cached buffer: what a kernel does with its scratch (K splits) then
-    # depends on the shape alone, never on what an earlier call left behind
-    return ptr(buf), int(n)
-
-
+# the operators' scratch, {(device, stream): uint8 tensor}: the host module takes a buffer out for the length of a call
 _ws = {}
-
-
-def workspace(device, nbytes):
-    """Per (device, stream) scratch buffer, grown on demand.  Calls issued on one stream are
-    ordered, so sharing the buffer between consecutive launches on that stream is safe."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    buf = _ws.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.empty(max(int(nbytes), 1 << 20), dtype=torch.uint8, device=device)
-        _ws[key] = buf
-    return buf
 
 
 def release_workspaces(device=None):

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __re
     }
     const int rank = __popcll(same & ((1ull << lane) - 1ull));
     if (b >= 0 && rank == 0) cells[wave * nb + b] = __popcll(same);
-    if constexpr (WAVES > 1) __syncthreads();
+    __syncthreads();
     if (b >= 0) {
         int pos = tot[b] + pre[b] + rank;
         for (int w = 0; w < wave; ++w) pos += cells[w * nb + b];

@@ -102,13 +102,5 @@ template <int N>
 __device__ __forceinline__ void ring_wait(v4i& a, v4i& b, v4i& c, v4i& d, v2i& e) {
     asm volatile("s_waitcnt vmcnt(%5)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e) : "n"(N) : "memory");
 }
-template <int N>
-__device__ __forceinline__ void ring_wait(v4i& a, v4i& b, v4i& c, v4i& d, v4i& e, v4i& f, v4i& g, v4i& h) {
-    asm volatile("s_waitcnt vmcnt(%8)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h) : "n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void ring_wait(int& a, int& b, int& c, int& d) {
-    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "n"(N) : "memory");
-}
 
 }  // namespace llmk
