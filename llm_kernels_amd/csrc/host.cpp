@@ -19,6 +19,7 @@
 #include <ATen/record_function.h>
 #include <c10/core/DefaultDtype.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 
 #include "../../include/llmk.h"
 
@@ -139,6 +140,8 @@ template <class F> auto unlocked(F&& f) {
 // back once its launches are queued.  Calls on one stream run one after the other there, so the next one may have the same
 // buffer; a call that another thread makes on that stream meanwhile finds none and allocates its own, because the launches
 // of the two may alternate.  Of two buffers that come back the larger one is kept.
+// Under capture a call takes a buffer from the graph's own pool instead: a graph goes on using it after the call, when one
+// from the dictionary may have been replaced by a larger one and its memory given to another tensor.
 // (Made and destroyed under the interpreter's lock, get() anywhere.)
 class Scratch {
     const Args& a;
@@ -147,11 +150,16 @@ class Scratch {
     PyObject *key = nullptr, *held = nullptr;            // held: the dictionary's tensor, this call's while it lasts
     at::Tensor fresh;                                    // or one of its own
 
+    bool capturing() const {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing((hipStream_t)stream_of(like), &status) != hipSuccess) (void)hipGetLastError();
+        return status != hipStreamCaptureStatusNone;
+    }
     static int64_t size(PyObject* o) { return o && THPVariable_Check(o) ? THPVariable_Unpack(o).numel() : 0; }
 
 public:
     Scratch(const Args& args, const at::Tensor& t, int64_t bytes) : a(args), like(t), need(std::max<int64_t>(bytes, 0)) {
-        if (!need) return;
+        if (!need || capturing()) return;
         key = Py_BuildValue("(iK)", (int)t.device().index(), (unsigned long long)(uintptr_t)stream_of(t));
         if (!key) throw Raised{};
         PyObject* o = PyDict_GetItemWithError(a.st->workspaces, key);

@@ -212,3 +212,34 @@ def test_the_profiler_sees_the_allocations(dev):
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
         fp8_kernel.act_quant(x)
     assert sum(e.name == "aten::empty" for e in prof.events()) == 2
+
+
+def test_a_captured_call_keeps_its_scratch(dev):
+    """A graph goes on using the scratch it was captured with: a later call on its stream that needs more must not hand that
+    memory to anyone else.  Replays, with eager calls between, give the eager result and write nothing of other tensors."""
+    announce("scratch of a captured call")
+    torch.manual_seed(0)
+
+    def operands(M, N, K):
+        w = fp8_kernel.weight_quant(torch.randn(N, K, device=dev) * 0.02)
+        return (*fp8_kernel.act_quant(torch.randn(M, K, device=dev).bfloat16()), *w)
+
+    small, large = operands(16, 1024, 8192), operands(16, 8192, 16384)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        want = fp8_kernel.fp8_gemm(*small)               # keeps scratch for this stream
+        stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = fp8_kernel.fp8_gemm(*small)
+    with torch.cuda.stream(stream):
+        fp8_kernel.fp8_gemm(*large)                      # replaces it by a larger one
+        others = [torch.full((1 << 18,), 0x5A, dtype=torch.uint8, device=dev) for _ in range(64)]
+        others += [torch.full((1 << 20,), 0x5A, dtype=torch.uint8, device=dev) for _ in range(16)]
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            fp8_kernel.fp8_gemm(*large)
+            stream.synchronize()
+            assert torch.equal(got, want)
+            assert all((t == 0x5A).all() for t in others)
