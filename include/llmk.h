@@ -113,7 +113,7 @@ int llmk_weight_dequant_w4a8(const int32_t* packed, const void* s_f16, const int
                              int group, void* stream);
 
 /* ------------------------------------------------------------------ dense quantized GEMMs
- * C[M,N] = sum_kb dot_kb(A, B) * a_s[m, kb] * b_s[n / 128, kb], K % 128 == 0, any M, N >= 1.
+ * C[M,N] = sum_kb dot_kb(A, B) * a_s[m, kb] * b_s[n / 128, kb], K % 128 == 0 (K = 0: zeros), any M, N >= 1.
  * A [M,K], B [N,K] both K-contiguous.  c_dtype selects the epilogue (torch default dtype).
  * workspace/workspace_bytes: optional scratch of llmk_gemm_workspace_bytes(M, N, K) bytes (fp32 activation
  * scales for large M, fp32 partial sums of the split-K / K-range variants); NULL/0 -> single-pass variants.
@@ -150,10 +150,13 @@ int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, cons
 /* b packed [N/8, K] int32, nibble (n % 8) of word [n/8, k]; b8 = int8((q - z4[n,kg]) * s4[n,kg]).
  * ref: quantization/w4a8_kernel.py:317-448 */
 /* workspace: llmk_gemm_w4a8_workspace_bytes(M, N, K, group_int4) bytes, 16-byte aligned, is what the path
- * chosen for the shape uses (0 for decode-size calls with K <= 4096: small M, group_int4 == 128, 16-byte aligned a
- * and b_packed run one fused kernel that reads the packed words once; fp32 partial sums of its K ranges,
- * ceil(K / 4096) * M * N * 4 bytes, for K > 4096; otherwise the expanded int8 weights, round16(N*K), and behind
- * them llmk_gemm_workspace_bytes(M,N,K) for the int8 tile kernels). */
+ * chosen for the shape uses.  With group_int4 == 128 and 16-byte aligned a and b_packed:
+ *   - decode size (M <= 64, more on small weights) runs one fused kernel that reads the packed words once: nothing for
+ *     K <= 4096, fp32 partial sums of its K ranges, ceil(K / 4096) * M * N * 4 bytes, beyond;
+ *   - 17 to 256 rows (see mid_rows and the plan in gemm_w4a8.hip) run on tile kernels that expand the words themselves:
+ *     fp32 partial sums of their K slices, optional (without: unsplit);
+ * everything else the expanded int8 weights, round16(N*K), needed, and behind them llmk_gemm_workspace_bytes(M,N,K) for
+ * the int8 tile kernels. */
 int64_t llmk_gemm_w4a8_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_int4);
 int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b_packed, const void* b_s,
                    int s_dtype, const int8_t* b_s4, const int8_t* b_z4, void* c, int c_dtype,
@@ -223,9 +226,9 @@ int llmk_moe_seg_indptr(const int64_t* sorted_ids, int64_t* seg_indptr, int64_t 
 int llmk_moe_src2dst(const int64_t* reorder_ids, int32_t* src2dst, int64_t num_toks, void* stream);
 /* ref: moe/group_gemm_kernel.py:48-78 (run_moe_ep_preproess) in one launch: stable sort of the num_toks
  * flattened expert ids (int32 / int64 by ids_bytes; sorted_ids has the same type), src2dst[i] = position of
- * id i in the sorted order, seg_indptr[e + 1] = number of ids <= e.  Every workgroup places 1024 ids and
- * reads the whole id list to do so: the entry point is for the id counts of one forward pass and fails
- * beyond the limits below;
+ * id i in the sorted order, seg_indptr[e + 1] = number of ids <= e.  Up to 256 ids are sorted by one
+ * workgroup; beyond, every workgroup places 1024 ids and reads the whole id list to do so: the entry point is for
+ * the id counts of one forward pass and fails beyond the limits below;
  * ids outside [0, num_experts) are ordered as one leading (negative) and one trailing group. */
 #define LLMK_MOE_PREPROCESS_MAX_EXPERTS 512
 #define LLMK_MOE_PREPROCESS_MAX_IDS 32768

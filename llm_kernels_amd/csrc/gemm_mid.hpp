@@ -332,7 +332,7 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
     constexpr int BN = mdp_bn(WIDE), NSUB = mdp_nsub(WIDE), RED_ROW = BN + 4;
     static_assert(BN * NSUB * 128 == MD_B && RED_ROW == (WIDE ? 132 : MD_RED_ROW), "weight stage of 32 KB");
     static_assert(KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL || KIND == K_F16 || KIND == K_BF16 || is_w4nk(KIND),
-                  "8- and 16-bit operands, or fp16 activations with row-packed 4-bit weights");
+                  "8- and 16-bit operands, or fp16 and bf16 activations with row-packed 4-bit weights");
     constexpr int BM = 16 * MT;
     // K_W4NK: the producers load packed words [N, K/8] and their group scales (fp16, groups of 64 * 2^j elements) and write
     // fp16 weight rows (q - 8) * scale into the weight stage; the rest is the fp16 kind

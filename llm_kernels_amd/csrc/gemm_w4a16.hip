@@ -1,4 +1,4 @@
-// W4A16 GEMM kernels: fp16 activations x 4-bit weights dequantised in registers.
+// W4A16 GEMM kernels: fp16 (row-packed layout: also bf16) activations x 4-bit weights dequantised in registers.
 //
 // nibble -> fp16 without integer->float converts: (q | 0x6400) is the fp16 number 1024 + q,
 // ((q << 4) | 0x6400) is 1024 + 16 q; one packed subtract / fma gives q - 8 exactly.

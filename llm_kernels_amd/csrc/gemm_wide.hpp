@@ -172,7 +172,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     const int r = lane & 15, g = lane >> 4;
     const int wm = wave >> 2, wn = wave & 3;
     constexpr bool SCALED = (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK);
-    // 4-bit weights (fp16 activations): the weight rows of a stage are not loaded into LDS but expanded there by
+    // 4-bit weights (fp16 or bf16 activations): the weight rows of a stage are not loaded into LDS but expanded there by
     // the threads themselves from packed words that travel HBM -> registers, see w4_request / w4_expand
     constexpr bool W4NK = is_w4nk(KIND), W4 = W4NK;
     static_assert(KIND != K_W4MARLIN && KIND != K_W4A8 && !(W4 && GROUPED), "4-bit weights: row-packed layout, dense launches only");
@@ -769,7 +769,7 @@ inline bool mid_wanted(int64_t M, int64_t N, int64_t kbytes) {
 
 // Shapes for the 128-column form of that kernel: shapes the 64-column form does not take, one round of 64- or 128-row
 // tiles, rows of at most 16 KB (256 x 14336 x 14336 118.4 -> 86.3 us, 128 x 14336 x 14336 85.4 -> 65.7, 128 x 4096 x 14336
-// in four K slices 28.4 -> 27.0).  Taken for fp8 and for fp16 activations with row-packed 4-bit weights, where it beats
+// in four K slices 28.4 -> 27.0).  Taken for fp8 and for fp16 and bf16 activations with row-packed 4-bit weights, where it beats
 // the 128-column tile kernels (fp8, us per launch, cold weights: 128 x 14336 x 4096 26.3 -> 23.2, 256 x 14336 x 4096
 // 37.6 -> 29.6, 256 x 6144 x 4096 23.6 -> 20.2, 128 x 28672 x 4096 44.3 -> 38.6, 384 x 8192 x 4096 35.1 -> 27.7,
 // 128 x 14336 x 8192 53.5 -> 38.9; 4-bit 128 x 14336 x 4096 37.1 -> 33.2, same elsewhere); the int8 kinds lose on it

@@ -142,8 +142,8 @@ __global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __re
 
 // The same for at most 64 ids: one wave, a lane per id, no LDS.  Every lane counts the ids of lower buckets and the equal
 // ids of lower lanes, one pass per distinct bucket.  What such a launch costs behind a kernel that streamed the experts'
-// weights is fetching its code from memory again, so the code is short (32 ids, 8 experts: 5.4 us in the general form,
-// 2.0 here).
+// weights is fetching its code from memory again, so the code is short (32 ids, 8 experts: launches back to back 5.4 us in
+// the general form, 2.0 here; in an expert layer of 16 tokens 5.9 and 4.7).
 __global__ __launch_bounds__(64) void ep_preprocess_wave_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
                                                                 void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
                                                                 int64_t* __restrict__ seg_indptr) {
@@ -176,7 +176,8 @@ __global__ __launch_bounds__(64) void ep_preprocess_wave_kernel(const void* __re
 // L lanes own one token, V experts each (expert v * L + lane), topk <= L; a wave owns 64 / L tokens.  Bound by latency: a token is a few
 // dozen bytes, and what the launch costs is one dependent chain (load, max, sum, topk rounds of an arg-max over the lanes),
 // so everything stays in registers and lanes.  As five torch kernels the same routing took 31 us of GPU time for 16 tokens
-// and 43 us for 4096; one launch here takes 2.1 and 3.4 us.
+// and 43 us for 4096; one launch here takes 1.9 and 2.8 us back to back, 5.3 and 5.0 in a layer of 8 experts, where its code
+// has to be fetched again behind the kernels that streamed the weights.
 // A probability is ranked by its bit pattern (monotone for the non-negative values, a NaN above all of them), joined with
 // the complement of the index, so equal values go to the lower index and one 64-bit maximum decides a round.
 template <int DT, int L, int V>
@@ -501,7 +502,7 @@ extern "C" int llmk_moe_ep_preprocess(const void* topk_ids, int ids_bytes, int64
                                       void* sorted_ids, int32_t* src2dst, int64_t* seg_indptr, void* stream) {
     if (num_experts < 0 || num_toks < 0) LLMK_FAIL(LLMK_ERR_SHAPE, "moe_ep_preprocess: negative size");
     if (num_experts > LLMK_MOE_PREPROCESS_MAX_EXPERTS || num_toks > LLMK_MOE_PREPROCESS_MAX_IDS)
-        LLMK_FAIL(LLMK_ERR_SHAPE, "moe_ep_preprocess: %lld ids of %d experts exceed the limits %d / %d of the one-workgroup sort",
+        LLMK_FAIL(LLMK_ERR_SHAPE, "moe_ep_preprocess: %lld ids of %d experts exceed the limits %d / %d of the one-launch sort",
                   (long long)num_toks, num_experts, LLMK_MOE_PREPROCESS_MAX_IDS, LLMK_MOE_PREPROCESS_MAX_EXPERTS);
     if (ids_bytes != 4 && ids_bytes != 8) LLMK_FAIL(LLMK_ERR_DTYPE, "moe_ep_preprocess: ids_bytes %d", ids_bytes);
     if (!seg_indptr || (num_toks && (!topk_ids || !sorted_ids || !src2dst))) LLMK_FAIL(LLMK_ERR_ARG, "moe_ep_preprocess: null pointer");

@@ -22,7 +22,7 @@ def _cdiv(a, b):
     return (a + b - 1) // b
 
 
-# limits of the one-workgroup sort behind llmk_moe_ep_preprocess (LLMK_MOE_PREPROCESS_MAX_* of the C header)
+# limits of the one-launch sort behind llmk_moe_ep_preprocess (LLMK_MOE_PREPROCESS_MAX_* of the C header)
 PREPROCESS_MAX_IDS = 32768
 PREPROCESS_MAX_EXPERTS = 512
 
