@@ -166,12 +166,13 @@ _ws = {}
 
 
 def release_workspaces(device=None):
-    """Drops the cached scratch buffers (of one device, or of all): the next call that needs scratch allocates
-    again.  The memory goes back to torch's allocator once the launches that use it have run (stream-ordered)."""
+    """Drops the cached scratch buffers (of one device, or of all) that no call under way has: the next call that needs scratch
+    allocates again.  The memory goes back to torch's allocator once the launches that use it have run (stream-ordered)."""
     index = None
     if device is not None:
         index = torch.device(device).index
         if index is None:                      # "cuda" without an ordinal: the current device
             index = torch.cuda.current_device()
-    for key in [k for k in _ws if index is None or k[0] == index]:
-        del _ws[key]
+    for key in list(_ws):                      # (calls of other threads take keys out and put them back meanwhile)
+        if index is None or key[0] == index:
+            _ws.pop(key, None)

@@ -2,6 +2,7 @@
 import ctypes
 import os
 import re
+import sys
 
 import pytest
 
@@ -81,6 +82,36 @@ def test_smoke_builds_what_cannot_be_loaded(monkeypatch, what):
         monkeypatch.setattr(torch, "__version__", "0.0")
     with pytest.raises(Built):
         __graft_entry__.smoke()
+
+
+def test_release_workspaces_while_calls_take_their_scratch():
+    """Calls of other threads take buffers out of the dictionary and put them back while it is walked."""
+    import threading
+    saved = dict(_lib._ws)
+    stop = threading.Event()
+
+    def calls():
+        while not stop.is_set():
+            for i in range(50):
+                _lib._ws.pop((0, i), None)
+            for i in range(50):
+                _lib._ws[(0, i)] = i
+
+    threads = [threading.Thread(target=calls) for _ in range(3)]
+    switch = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        for t in threads:
+            t.start()
+        for _ in range(500):
+            _lib.release_workspaces()
+    finally:
+        stop.set()
+        for t in threads:
+            t.join()
+        sys.setswitchinterval(switch)
+        _lib._ws.clear()
+        _lib._ws.update(saved)
 
 
 def test_release_workspaces_drops_the_cached_scratch():
