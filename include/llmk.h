@@ -151,10 +151,9 @@ int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, cons
  * ref: quantization/w4a8_kernel.py:317-448 */
 /* workspace: llmk_gemm_w4a8_workspace_bytes(M, N, K, group_int4) bytes, 16-byte aligned, is what the path
  * chosen for the shape uses.  With group_int4 == 128 and 16-byte aligned a and b_packed:
- *   - decode size (M <= 64, more on small weights) runs one fused kernel that reads the packed words once: nothing for
- *     K <= 4096, fp32 partial sums of its K ranges, ceil(K / 4096) * M * N * 4 bytes, beyond;
- *   - 17 to 256 rows (see mid_rows and the plan in gemm_w4a8.hip) run on tile kernels that expand the words themselves:
- *     fp32 partial sums of their K slices, optional (without: unsplit);
+ *   - up to 256 rows, and up to 512 where that is estimated to be faster (see the plan in gemm_w4a8.hip), one kernel unpacks
+ *     the words itself and reads them once per row tile: fp32 partial sums of its K slices, z * M * N * 4 bytes, optional up
+ *     to K = 32768 (without: unsplit); from 17 rows on llmk_gemm_workspace_bytes(M,N,K) is reported at least;
  * everything else the expanded int8 weights, round16(N*K), needed, and behind them llmk_gemm_workspace_bytes(M,N,K) for
  * the int8 tile kernels. */
 int64_t llmk_gemm_w4a8_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_int4);

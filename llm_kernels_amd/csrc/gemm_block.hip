@@ -136,7 +136,7 @@ extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8
         if (mid_wanted(M, N, K)) {
             MidPlan pl = mid_plan(M, N, K);
             if (pl.z > 1 && !(workspace && workspace_bytes >= (int64_t)pl.z * M * N * 4 && !((uintptr_t)workspace & 15))) pl.z = 1;
-            if (mid_eligible<K_I8_ROWCOL>(p, pl.mt, pl.z)) {
+            if (mid_eligible<K_I8_ROWCOL>(p)) {
                 if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; }
                 return pl.mt == 4 ? launch_mid<K_I8_ROWCOL, 4>(p, (hipStream_t)stream, "gemm_i8_rowcol(mid)")
                                   : launch_mid<K_I8_ROWCOL, 2>(p, (hipStream_t)stream, "gemm_i8_rowcol(mid)");

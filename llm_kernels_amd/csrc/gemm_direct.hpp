@@ -16,9 +16,7 @@ namespace llmk {
 enum : int { K_FP8_BLOCK = 0, K_I8_BLOCK = 1, K_I8_ROWCOL = 2, K_F16 = 3, K_BF16 = 4,
              K_W4NK = 5,      // fp16 activations x 4-bit weights packed [N, K/8] (tile kernels only)
              K_W4MARLIN = 6,  // the same with weights and scales in the Marlin layout
-             K_W4NKB = 8,     // K_W4NK with bf16 activations (bf16 weights (q - 8) * scale)
-             K_W4A8 = 7 };    // int8 activations x uint4 weights packed eight rows per word [N/8, K] with int8 zero
-                              // point and scale per (row, 128-K group) and 128 x 128 block scales (tile kernels only)
+             K_W4NKB = 8 };   // K_W4NK with bf16 activations (bf16 weights (q - 8) * scale)
 
 constexpr bool is_w4nk(int kind) { return kind == K_W4NK || kind == K_W4NKB; }
 // kinds whose activations (and expanded weights) are 16-bit
@@ -77,7 +75,7 @@ __device__ __forceinline__ v4f step_dot(const v8i& a, const v8i& b) {
     const v4f z = {0.f, 0.f, 0.f, 0.f};
     if constexpr (KIND == K_FP8_BLOCK) {
         return mfma_fp8_16x16x128(a, b, z);
-    } else if constexpr (KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL || KIND == K_W4A8) {
+    } else if constexpr (KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL) {
         v4i zi = {0, 0, 0, 0};
         v4i a0 = {a[0], a[1], a[2], a[3]}, a1 = {a[4], a[5], a[6], a[7]};
         v4i b0 = {b[0], b[1], b[2], b[3]}, b1 = {b[4], b[5], b[6], b[7]};
@@ -94,7 +92,7 @@ __device__ __forceinline__ v4f step_dot(const v8i& a, const v8i& b) {
 // product while later ones multiply converts it then too, a conversion right behind the MFMA waits for it.
 template <int KIND>
 __device__ __forceinline__ v4f step_raw(const v8i& a, const v8i& b) {
-    if constexpr (KIND == K_I8_BLOCK || KIND == K_W4A8) {
+    if constexpr (KIND == K_I8_BLOCK) {
         v4i t = mfma_i8_16x16x64((v4i){a[0], a[1], a[2], a[3]}, (v4i){b[0], b[1], b[2], b[3]}, (v4i){0, 0, 0, 0});
         t = mfma_i8_16x16x64((v4i){a[4], a[5], a[6], a[7]}, (v4i){b[4], b[5], b[6], b[7]}, t);
         return __builtin_bit_cast(v4f, t);
@@ -104,7 +102,7 @@ __device__ __forceinline__ v4f step_raw(const v8i& a, const v8i& b) {
 }
 template <int KIND>
 __device__ __forceinline__ v4f raw_f32(const v4f& t) {
-    if constexpr (KIND == K_I8_BLOCK || KIND == K_W4A8) {
+    if constexpr (KIND == K_I8_BLOCK) {
         const v4i i = __builtin_bit_cast(v4i, t);
         return (v4f){(float)i[0], (float)i[1], (float)i[2], (float)i[3]};
     } else {
@@ -128,8 +126,8 @@ struct DirectArgs {
     int kc_steps;          // weight-streaming kernel with K ranges: 128-byte steps per range (gridDim.z ranges)
     int group;             // K_W4NK / K_W4MARLIN: K elements per fp16 group scale
     long long* clocks;     // 256-column tile kernel, calibration only: workgroup 0 leaves the s_memtime and s_memrealtime ticks it lived
-    const int8_t* w4_s4;   // K_W4A8: second-level scales [N, K/128]
-    const int8_t* w4_z4;   // K_W4A8: zero points [N, K/128]
+    const int8_t* w4_s4;   // uint4 weights with two-level scales: second-level scales [N, K/128]
+    const int8_t* w4_z4;   // the same: zero points [N, K/128]
     int tail_split;        // 256-column tile kernel: the tiles of a short last round are split along K (partial = scratch)    // 256-column tile kernel with the gated-activation epilogue (grouped gate / up projection, N = 2 I): c receives the
     // 1 x 128 quantised activations [M, I] in the operand type, q_scale their scales [M, I / 128]
     void* q_scale;

@@ -13,10 +13,7 @@
 // column tile land on one XCD (same workgroup id modulo 8 when the column tiles are a multiple of 8) and walk K in
 // step, so that a weight line comes from HBM once.
 //
-// Two forms:
-//   gemm_mid_kernel     (K_W4A8): all eight waves load, unpack and multiply: wave (wn, kq) takes 32 columns of sub-block
-//                       kq.  The unpacking (q - z4) * s4 is vector-ALU work that wants every wave.
-//   gemm_mid_pc_kernel  (every other kind): four waves only request and stage operands, four only multiply; see there.
+// Four waves only request and stage operands, four only multiply: see gemm_mid_pc_kernel.
 //
 // All loads of a step are issued unconditionally (steps past the end repeat the last one) so that one
 // hand-counted s_waitcnt per step is exact; check_asm.py proves the register loads on every build.
@@ -30,13 +27,6 @@ constexpr int MD_BN = 64, MD_THREADS = 512;
 constexpr int MD_B = 4 * MD_BN * 128;                       // weight stage: [sub-block][column][128 B] = 32 KB
 constexpr int MD_S = 4 * 64 * 4;                            // activation-scale columns of a step: [sub-block][row] fp32
 constexpr int MD_RED_ROW = 68;                              // floats per row of the final reduction (64 + 4: bank spread)
-constexpr int md_a(int mt) { return 4 * 16 * mt * 128; }    // activation stage: [sub-block][row][128 B]
-constexpr int MD_NA = 2;                                    // activation stages
-constexpr int MD_NBS = 2;                                   // weight stages
-constexpr int md_stages(int mt) { return MD_NA * (md_a(mt) + MD_S) + MD_NBS * MD_B; }
-constexpr int md_red(int mt) { return 4 * 16 * mt * MD_RED_ROW * 4; }
-// stages (reused by the reduction), weight-scale table, K_W4A8 table of zero points and second-level scales
-constexpr int md_lds(int mt, int kt_tab) { return md_stages(mt) + D_MAX_KT * 4 + 128 * kt_tab; }
 
 // f(integral_constant<I>) for I = FIRST .. LAST - 1 (ring slots are compile-time indices)
 template <int I, int LAST, class F>
@@ -58,250 +48,9 @@ __device__ __forceinline__ void md_static_nested(int rem, F&& f) {
     }
 }
 
-// AS16: the activation scales are 16-bit (fp16 or bf16 by p.s_dtype) and are staged as they are (one zero-extended
-// element per dword slot of the scale column) instead of being widened to fp32 by a kernel of their own first.
-template <int KIND, int MT, bool AS16 = false>
-__global__ __launch_bounds__(MD_THREADS) void gemm_mid_kernel(DirectArgs p) {
-    static_assert(MT == 4 || MT == 2, "tile rows");
-    static_assert(KIND == K_W4A8, "the other kinds run on gemm_mid_pc_kernel");
-    constexpr int BM = 16 * MT;
-    constexpr int MD_A = md_a(MT);
-    constexpr int NB = 2;                                   // ring loads per thread and step
-    constexpr int MD_RING = 4;                              // ring slots: weights are requested MD_RING - 1 steps ahead
-    constexpr int NA = MT + 1;                              // direct-to-LDS loads per thread and step (activation pieces, scale column)
-    static_assert(md_red(MT) <= md_stages(MT), "the reduction reuses the stages");
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, g = lane >> 4, wn = wave & 1, kq = wave >> 1;
-    const int N = p.N;
-    const int K = p.K;                                      // row length in bytes (int8 activations)
-    const int KT_all = K >> 7;                              // 128-byte sub-blocks per row
-    int kt0 = 0, KT = KT_all;                               // sub-blocks [kt0, kt0 + KT) of this workgroup
-    if (p.ksplit > 1) {
-        // slices in whole steps of four sub-blocks (one weight-scale block each for the scaled kinds)
-        const int per = (((KT_all + p.ksplit - 1) / p.ksplit) + 3) & ~3;
-        kt0 = (int)blockIdx.z * per;
-        KT = max(0, min(per, KT_all - kt0));
-    }
-    const int nsteps = (KT + 3) >> 2;
-    const int n0 = blockIdx.x * MD_BN, m_start = blockIdx.y * BM, m_end = min(p.M, m_start + BM);
-
-    // LDS map
-    uint8_t* const a_st = lds;                              // [MD_NA][MD_A]
-    uint8_t* const b_st = lds + MD_NA * MD_A;               // [MD_NBS][MD_B]
-    uint8_t* const s_st = lds + MD_NA * MD_A + MD_NBS * MD_B;        // [MD_NA][MD_S]
-    float* const bsl = (float*)(lds + md_stages(MT));       // weight scale of the tile's column block per sub-block
-    uint8_t* const w4tab = lds + md_stages(MT) + D_MAX_KT * 4;   // [s4 | z4][sub-block][64 rows] bytes
-
-    // ---- per-thread source offsets.  A piece = 8 rows x 128 bytes = what one load instruction of a wave covers
-    // (lane: row lane >> 3, 16-byte chunk lane & 7, XOR-swizzled with (row >> 1) & 7 on the global side so that
-    // the fragment reads are conflict-free).  Wave w moves pieces MT w .. MT w + MT - 1 of the 4 x 2 MT activation
-    // pieces of a step: piece = (sub-block, row group).
-    const int row8 = lane >> 3;
-    uint32_t aoff[MT], alds[MT];
-    int asub[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int pq = MT * wave + i, sub = pq / (2 * MT), row = 8 * (pq % (2 * MT)) + row8;
-        const uint32_t chunk = (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
-        aoff[i] = (uint32_t)min(m_start + row, m_end - 1) * (uint32_t)K + chunk;
-        alds[i] = (uint32_t)(sub * (BM * 128) + 8 * (pq % (2 * MT)) * 128);     // + lane * 16 by the hardware
-        asub[i] = sub;
-    }
-    // weights: one wave per packed row (eight weight rows): lane l takes words 4 l .. 4 l + 3 of sub-blocks l >> 5
-    // (load 0) and 2 + (l >> 5) (load 1) of the step's 512 words
-    const uint32_t boff = (uint32_t)min((n0 >> 3) + wave, (N >> 3) - 1) * (uint32_t)(p.K * 4) + (uint32_t)(lane & 31) * 16u;
-    constexpr uint32_t SSZ = AS16 ? 2u : 4u;                // bytes per activation scale
-    const uint32_t soff = (uint32_t)min(m_start + min(lane, BM - 1), m_end - 1) * (uint32_t)KT_all * SSZ;
-
-    // sub-block `sub` of step s, clamped to the last one of the range: requests past the end repeat the last step
-    auto phys = [&](int s) { return min(s, nsteps - 1); };
-    auto kblock = [&](int s, int sub) { return kt0 + min(4 * phys(s) + sub, KT - 1); };
-
-    auto issue_a = [&](int s) {
-        const uint32_t st = lds_base + (uint32_t)(s % MD_NA) * MD_A;
-#pragma unroll
-        for (int i = 0; i < MT; ++i) dma16(st + alds[i], aoff[i], p.a + (int64_t)kblock(s, asub[i]) * 128);
-        const uint32_t ss = lds_base + MD_NA * MD_A + MD_NBS * MD_B + (uint32_t)(s % MD_NA) * MD_S + (uint32_t)(wave & 3) * 256u;
-        if constexpr (AS16) dma2(ss, soff, (const uint8_t*)p.a_s + (int64_t)kblock(s, wave & 3) * 2);
-        else dma4(ss, soff, (const uint8_t*)p.a_s + (int64_t)kblock(s, wave & 3) * 4);
-    };
-    // ring of weight registers: slot = step % 4
-    v4i ring[MD_RING][NB];
-    auto issue_b = [&](v4i (&rs)[NB], int s) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            // lane-dependent sub-block: the two halves of the wave read different 128-word runs of the row
-            const int kb0 = kblock(s, 2 * i), kb1 = kblock(s, 2 * i + 1);
-            const uint32_t off = boff + (uint32_t)((lane >> 5) ? kb1 - kb0 : 0) * 512u;
-            rs[i] = asm_load_b128(off, (const uint8_t*)p.b + (int64_t)kb0 * 512);
-        }
-    };
-    // the loads of slot `slot` have landed when at most `younger` loads issued after them are in flight
-    auto ring_ready = [&](v4i (&rs)[NB], auto younger_c) __attribute__((always_inline)) {
-        constexpr int Y = decltype(younger_c)::value;
-        asm volatile("s_waitcnt vmcnt(%2)" : "+v"(rs[0]), "+v"(rs[1]) : "n"(Y) : "memory");
-    };
-    // ring slot -> weight stage s & 1 (nobody has read that stage since the barrier of step s - 1), as int8 rows
-    // (q - z4) * s4.  Lane: words 4 kc .. 4 kc + 3 (kc = lane & 31) of sub-block 2 i + (lane >> 5); packed row = wave;
-    // row j of the packed row is tile column 8 wave + j.
-    auto produce = [&](const v4i (&rs)[NB], int s) __attribute__((always_inline)) {
-        uint8_t* st = b_st + (s % MD_NBS) * MD_B;
-        const int kc = lane & 31;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int sub = 2 * i + (lane >> 5);
-            const int kb = min(4 * phys(s) + sub, KT - 1);
-            const uint8_t* tabk = w4tab + kb * 64 + 8 * wave;
-            unsigned sp[4], cp[4], rows[8];
-            w4a8_row_consts(*(const uint2*)tabk, *(const uint2*)(tabk + 64 * KT), sp, cp);
-            w4a8_words_to_i8(rs[i], sp, cp, rows);
-            uint8_t* dst = st + sub * (MD_BN * 128) + (kc & 3) * 4;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int R = 8 * wave + j;
-                *(unsigned*)(dst + R * 128 + (((kc >> 2) ^ ((R >> 1) & 7)) * 16)) = rows[j];
-            }
-        }
-    };
-
-    // acc[i][j][q] = C[row 16 i + r][column 32 wn + 16 j + 4 g + q] summed over this wave's sub-blocks
-    v4f acc[MT][2];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) acc[i][0] = acc[i][1] = (v4f){0.f, 0.f, 0.f, 0.f};
-
-    // fragment read offsets inside a 16-row slab: chunks g and g + 4 of row r, swizzled
-    const int lo = r * 128 + ((g ^ ((r >> 1) & 7)) * 16);
-    const int hi = r * 128 + (((g + 4) ^ ((r >> 1) & 7)) * 16);
-    auto ldfrag = [&](const uint8_t* base) {
-        const v4i x = *(const v4i*)(base + lo), y = *(const v4i*)(base + hi);
-        return (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-    };
-    auto compute = [&](int s) {
-        const uint8_t* As = a_st + (s % MD_NA) * MD_A + kq * (BM * 128);
-        const uint8_t* Bs = b_st + (s % MD_NBS) * MD_B + kq * (MD_BN * 128) + (wn * 32) * 128;
-        const int kb = 4 * phys(s) + kq;
-        const bool live = kb < KT;                         // wave-uniform: sub-blocks past the range add nothing
-        // activation fragments one tile row ahead of their use
-        v8i bf[2], af[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) bf[j] = ldfrag(Bs + j * 2048);
-        af[0] = ldfrag(As);
-        const float* Ss = (const float*)(s_st + (s % MD_NA) * MD_S) + kq * 64 + r;
-        const float bs = live ? bsl[min(kb, KT - 1)] : 0.f;
-        float sa[MT];
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            if constexpr (AS16) {
-                const unsigned raw = ((const unsigned*)Ss)[16 * i];
-                sa[i] = (p.s_dtype == LLMK_F16 ? f16_to_f32((unsigned short)raw) : bf16_to_f32((unsigned short)raw)) * bs;
-            } else {
-                sa[i] = Ss[16 * i] * bs;
-            }
-        }
-        // the products of tile row i are scaled and accumulated while the matrix instructions of row i + 1 run
-        v4f t[2][2];
-#pragma unroll
-        for (int i = 0; i <= MT; ++i) {
-            if (i + 1 < MT) af[(i + 1) & 1] = ldfrag(As + (i + 1) * 2048);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if (i < MT) t[i & 1][j] = step_raw<KIND>(bf[j], af[i & 1]);
-                if (i > 0) acc[i - 1][j] += raw_f32<KIND>(t[(i - 1) & 1][j]) * sa[i - 1];
-            }
-            // nothing moves across a tile row: the lag of one row between product and accumulation stays, and
-            // the fragments of at most two rows are live
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-
-    const std::integral_constant<int, 0> c0;
-    const std::integral_constant<int, (MD_RING - 2) * NB> cpro;
-    const std::integral_constant<int, NB> cnb;
-
-    // ---- prologue: activations of step 0, weights of steps 0, 1, 2; tables by ordinary loads meanwhile
-    issue_a(0);
-    md_static_for<0, MD_RING - 1>([&](auto ic) __attribute__((always_inline)) { issue_b(ring[ic.value], ic.value); });
-    const int64_t bs_row = (int64_t)(n0 >> 7) * KT_all + kt0;
-    for (int i = tid; i < KT; i += MD_THREADS) bsl[i] = ld_scale(p.b_s, bs_row + i, p.s_dtype);
-    for (int i = tid; i < 64 * KT; i += MD_THREADS) {
-        const int row = i / KT, kk = i - row * KT;
-        const int64_t at = (int64_t)min(n0 + row, N - 1) * KT_all + kt0 + kk;
-        w4tab[kk * 64 + row] = (uint8_t)p.w4_s4[at];
-        w4tab[(KT + kk) * 64 + row] = (uint8_t)p.w4_z4[at];
-    }
-    __syncthreads();                                        // the table is read by produce()
-    ring_ready(ring[0], cpro);
-    produce(ring[0], 0);
-
-    // One step: wait for the activations of step s (requested a step ago; only the NB weight loads issued after
-    // them may stay in flight; with four ring slots that also vouches for slot s + 1, requested two steps ago),
-    // meet the others, request the activations of step s + 1 and the weights of step s + MD_RING - 1, multiply
-    // step s, and move the weights of step s + 1 from the ring into the other weight stage.
-    auto step = [&](auto slot_c, int s) __attribute__((always_inline)) {
-        constexpr int slot = decltype(slot_c)::value;
-        // (scheduling fences: without them the compiler carries the matrix instructions of a step across the next
-        // barrier, with all fragments of two steps live, and spills)
-        __builtin_amdgcn_sched_barrier(0);
-        ring_ready(ring[(slot + 1) % MD_RING], cnb);
-        __builtin_amdgcn_s_waitcnt(0xc07f);                 // lgkmcnt(0): this wave's LDS writes of produce() are done
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        issue_a(s + 1);
-        issue_b(ring[(slot + MD_RING - 1) % MD_RING], s + MD_RING - 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(s);
-        __builtin_amdgcn_sched_barrier(0);
-        produce(ring[(slot + 1) % MD_RING], s + 1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    int s = 0;
-    for (int rd = nsteps / MD_RING; rd > 0; --rd) {
-        md_static_for<0, MD_RING>([&](auto ic) __attribute__((always_inline)) { step(ic, s + ic.value); });
-        s += MD_RING;
-    }
-    md_static_nested<0, MD_RING - 1>(nsteps % MD_RING, [&](auto ic) __attribute__((always_inline)) { step(ic, s + ic.value); });
-    // everything requested has landed (also the repeated loads past the end) before the stages are reused
-    md_static_for<0, MD_RING>([&](auto ic) __attribute__((always_inline)) { ring_ready(ring[ic.value], c0); });
-    __syncthreads();
-
-    // ---- the four sub-block sums of every output meet in LDS: red[kq][row][column], rows of 68 floats
-    float* red = (float*)lds;
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            *(v4f*)(red + (kq * BM + 16 * i + r) * MD_RED_ROW + wn * 32 + 16 * j + 4 * g) = acc[i][j];
-    __syncthreads();
-    // thread: row tid >> 3, columns 8 (tid & 7) .. + 7
-    const int orow = tid >> 3, ocol = 8 * (tid & 7);
-    if (orow >= BM) return;
-    const int m = m_start + orow, n = n0 + ocol;
-    if (m >= m_end || n >= N) return;
-    v4f sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float* src = red + (q * BM + orow) * MD_RED_ROW + ocol;
-        sa += *(const v4f*)src;
-        sb += *(const v4f*)(src + 4);
-    }
-    const bool split = p.ksplit > 1;
-    void* cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
-    const int cdt = split ? LLMK_F32 : p.c_dtype;
-    const int esz = cdt == LLMK_F32 ? 4 : 2;
-    const bool vec_ok = ((((uintptr_t)cout) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
-    const int nv = N - n;
-    const int64_t off = (int64_t)m * N + n;
-    if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv, vec_ok);
-    else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv, vec_ok);
-    else store_run8<LLMK_F32>(cout, off, sa, sb, nv, vec_ok);
-}
-
 // ------------------------------------------------------------------------------------------------------------
-// Producer / consumer form of the same tile for 8- and 16-bit operands.  A cycle count of the kernel above (per wave and
-// phase) showed that it never waits for data: what a step costs is ISSUING its loads.  The CU's vector-memory path takes
+// Producer / consumer form.  A cycle count (per wave and phase) of a form in which all eight waves loaded and
+// multiplied showed that it never waits for data: what a step costs is ISSUING its loads.  The CU's vector-memory path takes
 // about 16 cycles per 1 KB instruction (64 bytes per clock, the 110 GB/s per CU), a step of a 64 x 64 tile is 64 such
 // instructions (about 1100 cycles), and a wave that is issuing loads cannot multiply: with all eight waves issuing behind
 // the barrier, then multiplying, then writing weight rows, the phases add up to 2900 cycles per step.  Here the roles are
@@ -669,16 +418,11 @@ inline MidPlan midw_plan(int64_t M, int64_t N, int64_t kbytes) {
     return pl;
 }
 
-// Eligibility: 32-bit source offsets, whole 128-byte sub-blocks, scale table size (as dma_eligible), and for the
-// K_W4A8 kind room for its table behind the stages.
+// Eligibility: 32-bit source offsets, whole 128-byte sub-blocks, scale table size (as dma_eligible).
 template <int KIND>
-inline bool mid_eligible(const DirectArgs& p, int mt, int ksplit) {
-    constexpr int ESZ = is_half(KIND) ? 2 : 1;
-    if (!dma_eligible(p, ESZ)) return false;
-    if (is_w4nk(KIND) && (p.group < 64 || (p.group & (p.group - 1)))) return false;      // groups of 64 * 2^j elements
-    const int KT_all = (p.K * ESZ) >> 7;
-    const int per = ksplit > 1 ? ((((KT_all + ksplit - 1) / ksplit) + 3) & ~3) : KT_all;
-    return md_lds(mt, KIND == K_W4A8 ? per : 0) <= D_LDS_MAX;
+inline bool mid_eligible(const DirectArgs& p) {
+    if (!dma_eligible(p, is_half(KIND) ? 2 : 1)) return false;
+    return !is_w4nk(KIND) || (p.group >= 64 && !(p.group & (p.group - 1)));               // groups of 64 * 2^j elements
 }
 
 // p.a_s: fp32, or with AS16 the 16-bit scales of dtype p.s_dtype as the caller passed them; p.s_dtype describes b_s
@@ -686,19 +430,13 @@ inline bool mid_eligible(const DirectArgs& p, int mt, int ksplit) {
 template <int KIND, int MT, bool AS16 = false, bool WIDE = false>
 int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
     static std::atomic<uint64_t> configured{0};
-    constexpr bool W4 = (KIND == K_W4A8);
-    static_assert(!(W4 && WIDE), "the 128-column form exists for the producer / consumer kernel only");
-    // the producer / consumer form, except for w4a8 (whose expansion is vector-ALU work that wants all eight waves)
-    auto kern = [] {
-        if constexpr (W4) return gemm_mid_kernel<KIND, MT, AS16>;
-        else return gemm_mid_pc_kernel<KIND, MT, AS16, WIDE>;
-    }();
+    auto kern = gemm_mid_pc_kernel<KIND, MT, AS16, WIDE>;
     constexpr int ESZ = is_half(KIND) ? 2 : 1;
     const int KT_all = (p.K * ESZ) >> 7;
     const bool split = p.ksplit > 1 && p.partial;
     const int per = split ? ((((KT_all + p.ksplit - 1) / p.ksplit) + 3) & ~3) : KT_all;
-    const int lds_bytes = W4 ? md_lds(MT, per) : mdp_lds(MT, WIDE);
-    if (lds_bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, lds_bytes);
+    constexpr int lds_bytes = mdp_lds(MT, WIDE);
+    static_assert(lds_bytes <= D_LDS_MAX, "stages and scale table fit in LDS");
     if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     // slices that would start past the end of K are not launched
     const int z = split ? (KT_all + per - 1) / per : 1;

@@ -925,7 +925,7 @@ NkTiles nk_tiles(const llmk::DirectArgs& p) {
     // few column tiles and short rows: the 64-column kernel with 512-byte K steps (128 x 4096 x 4096: 18.3 -> 14 us)
     if (2 * K <= 8192 && llmk::mid_wanted(M, N, 2 * K)) {       // (rows beyond 8 KB: measured only for the 8-bit kinds)
         const llmk::MidPlan pl = llmk::mid_plan(M, N, 2 * K);
-        if (llmk::mid_eligible<KIND>(p, pl.mt, pl.z)) return {NkTiles::MID, pl.mt, pl.z};
+        if (llmk::mid_eligible<KIND>(p)) return {NkTiles::MID, pl.mt, pl.z};
     }
     // wider weights on one round of 128-column tiles: the 128-column form of that kernel
     if (2 * K <= 8192 && llmk::midw_wanted(M, N, 2 * K) && (p.group & (p.group - 1)) == 0) {       // (longer rows: measured for fp8 only)

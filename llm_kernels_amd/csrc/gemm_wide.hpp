@@ -175,7 +175,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     // 4-bit weights (fp16 or bf16 activations): the weight rows of a stage are not loaded into LDS but expanded there by
     // the threads themselves from packed words that travel HBM -> registers, see w4_request / w4_expand
     constexpr bool W4NK = is_w4nk(KIND), W4 = W4NK;
-    static_assert(KIND != K_W4MARLIN && KIND != K_W4A8 && !(W4 && GROUPED), "4-bit weights: row-packed layout, dense launches only");
+    static_assert(KIND != K_W4MARLIN && !(W4 && GROUPED), "4-bit weights: row-packed layout, dense launches only");
     constexpr int ESZ = is_half(KIND) ? 2 : 1;
     const int N = p.N;
     const int K = p.K * ESZ;                 // row length in bytes
@@ -752,7 +752,7 @@ inline bool mid_m_prefers_tiles(int64_t M, int64_t N, int64_t K) {
 // Rows from which the mid-size kernels beat the weight-streaming ones: 33, and 17 on large weights (us per layer, quantiser
 // and GEMM, streaming or 64-row tiles | mid-size: fp8 64 x 14336 x 4096 28.4 | 23.0, 48 x 4096 x 4096 16.1 | 13.4, 20 x 14336
 // x 4096 23.0 | 20.2, but 20 x 4096 x 4096 11.2 | 12.7; per-token int8 64 x 15368 x 3072 48.7 | 21.9, 32 x 4096 x 4096 12.9 |
-// 15.0; w4a8 48 x 15368 x 3072 34.1 | 20.9, 32 x 4096 x 14336 27.9 | 23.0, 32 x 4096 x 4096 13.6 | 16.1).
+// 15.0).
 inline bool mid_rows(int64_t M, int64_t N, int64_t K) { return M > 32 || mid_m_prefers_tiles(M, N, K); }
 
 // Shapes for the mid-size kernel (gemm_mid.hpp): rows as above, at most one workgroup per CU and a K range of at
@@ -794,7 +794,7 @@ template <int KIND, bool GROUPED>
 TileChoice dma_tile_estimate(const DirectArgs& p) {
     // 4-bit weights: the row-packed layout, dense launches (the Marlin scatter of 2-byte pieces measured 4-9 % slower
     // inside the 256-column kernel than the dequantisation pass at every M > 512)
-    constexpr bool HAS_WIDE = KIND != K_W4MARLIN && KIND != K_W4A8 && !(GROUPED && is_w4nk(KIND));
+    constexpr bool HAS_WIDE = KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND));
     constexpr double WIDE = is_w4nk(KIND) ? 65.0 : 60.0, HALF = KIND == K_W4NK ? 42.0 : (KIND == K_W4NKB ? 46.0 : 36.0);
     const int64_t rows = GROUPED ? p.M / (p.E > 0 ? p.E : 1) : p.M;
     const int64_t groups = GROUPED ? p.E : 1;
@@ -814,12 +814,8 @@ TileChoice dma_tile_estimate(const DirectArgs& p) {
         }
         if (t_half < t4 && t_half <= t2 && t_half <= t1) return {9, t_half};
     }
-    int max_mi = 4;
-    if constexpr (KIND == K_W4A8) max_mi = w4a8_max_mi(p);       // the table of zero points and scales must fit behind the stages
-    if constexpr (KIND != K_W4A8) {
-        if (t4 <= t2 && t4 <= t1 && max_mi >= 4) return {4, t4};
-    }
-    if (t2 <= t1 && max_mi >= 2) return {2, t2};
+    if (t4 <= t2 && t4 <= t1) return {4, t4};
+    if (t2 <= t1) return {2, t2};
     return {1, t1};
 }
 template <int KIND, bool GROUPED>
@@ -831,13 +827,11 @@ int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* 
     if (!GROUPED && p.ksplit > 1) return launch_dma_mi<KIND, GROUPED, 1, AS16>(p, stream, name);
     const int choice = dma_tile_choice<KIND, GROUPED>(p);
     if constexpr (!AS16) {
-        if constexpr (KIND != K_W4MARLIN && KIND != K_W4A8 && !(GROUPED && is_w4nk(KIND))) {
+        if constexpr (KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND))) {
             if (choice == 9) return launch_wide<KIND, GROUPED, 4>(p, stream, name, ws, ws_bytes);
             if (choice == 8) return launch_wide<KIND, GROUPED, 8>(p, stream, name, ws, ws_bytes);
         }
-        if constexpr (KIND != K_W4A8) {
-            if (choice == 4) return launch_dma_mi<KIND, GROUPED, 4>(p, stream, name);
-        }
+        if (choice == 4) return launch_dma_mi<KIND, GROUPED, 4>(p, stream, name);
     }
     if (choice == 2) return launch_dma_mi<KIND, GROUPED, 2, AS16>(p, stream, name);
     return launch_dma_mi<KIND, GROUPED, 1, AS16>(p, stream, name);
@@ -855,7 +849,7 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
             MidPlan pl = mid_plan(p.M, p.N, p.K);
             const int64_t need = (int64_t)pl.z * p.M * p.N * 4;
             if (pl.z > 1 && !(workspace && workspace_bytes >= need && !(((uintptr_t)workspace) & 15))) pl.z = 1;
-            if (mid_eligible<KIND>(p, pl.mt, pl.z)) {
+            if (mid_eligible<KIND>(p)) {
                 if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; }
                 if (p.s_dtype != LLMK_F32) {
                     if constexpr (KIND != K_FP8_BLOCK)

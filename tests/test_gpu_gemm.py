@@ -235,6 +235,42 @@ def test_w4a8_mid_m_fused_tiles_exact_mixed_wrap(dev, M, N, K, sdt):
     assert torch.equal(c.cpu().long(), (a.double() @ b8.double().T).long())      # exact: every sum is far below 2^53
 
 
+@pytest.mark.parametrize("M,N,K,sdt", [
+    # every tile shape of the kernel whose waves stream their own K share, with ragged rows and columns and K steps that do
+    # not divide by the waves: 16 rows x 16, 32 and 64 columns, then 32, 48 and 64 rows
+    (7, 1048, 1152, torch.float16), (16, 4104, 2176, torch.float32), (5, 14344, 1280, torch.bfloat16),
+    (31, 6152, 896, torch.float16), (32, 14344, 1152, torch.float32), (47, 4104, 1280, torch.bfloat16),
+    (48, 14344, 1152, torch.float16), (64, 6152, 1280, torch.float32), (64, 14344, 1152, torch.bfloat16),
+    # four waves, more than one round of workgroups
+    (50, 24008, 1152, torch.float16), (95, 28680, 640, torch.float32), (256, 4104, 1152, torch.bfloat16),
+    # K slices; tables of more than one round of loads; more K steps than one workgroup takes
+    (1, 72, 16384, torch.float16), (40, 264, 33024, torch.float32), (20, 136, 65664, torch.float16), (300, 4104, 1024, torch.float16)])
+@pytest.mark.parametrize("scratch", [True, False])
+def test_w4a8_wave_kernel_exact(dev, M, N, K, sdt, scratch):
+    """Unit block scales, fp32 out, wild (s4, z4): exact integers (every sum is below 2^24), with the reported scratch and without."""
+    announce("w4a8 wave kernel", M, N, K, sdt, scratch)
+    if not scratch and K > 32768:
+        pytest.skip("beyond 256 K steps the slices need their sums")
+    torch.manual_seed(M * 7 + N)
+    wq = torch.randint(0, 16, (N, K), dtype=torch.uint8)
+    s4 = torch.randint(-128, 128, (N, K // 128), dtype=torch.int8)
+    z4 = torch.randint(-128, 128, (N, K // 128), dtype=torch.int8)
+    a = (torch.rand(M, K) < 64.0 / K).to(torch.int8) * torch.randint(-128, 128, (M, K), dtype=torch.int8)   # about 64 nonzeros a row
+    ad, packed = a.to(dev), torch.from_numpy(bp.pack_rows(wq.numpy(), 4, 32)[0]).to(dev)
+    ones_a, ones_b = torch.ones(M, K // 128, dtype=sdt, device=dev), torch.ones((N + 127) // 128, K // 128, dtype=sdt, device=dev)
+    s4d, z4d = s4.to(dev), z4.to(dev)
+    c = torch.full((M, N), 7.0, device=dev)
+    lib = _lib.load()
+    nbytes = lib.llmk_gemm_w4a8_workspace_bytes(M, N, K, 128) if scratch else 0
+    ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=dev)
+    _lib.call("llmk_gemm_w4a8", _lib.ptr(ad), _lib.ptr(ones_a), _lib.ptr(packed), _lib.ptr(ones_b), _lib.dt(sdt), _lib.ptr(s4d), _lib.ptr(z4d),
+              _lib.ptr(c), _lib.dt(torch.float32), M, N, K, 128, _lib.ptr(ws) if nbytes else None, nbytes, None)
+    b8 = q.w4a8_dequant_int8(wq, s4, z4)
+    ref = ad.double() @ b8.to(dev).double().T
+    assert ref.abs().max() < 2 ** 24
+    assert torch.equal(c.double(), ref)
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 4096, 4096), (256, 1024, 7168), (512, 4096, 4096), (384, 14336, 4096),
                                    (96, 2056, 14336)])
 def test_w4a8_mid_m_fused_tiles(dev, M, N, K):
