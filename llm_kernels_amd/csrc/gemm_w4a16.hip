@@ -3,6 +3,7 @@
 // nibble -> fp16 without integer->float converts: (q | 0x6400) is the fp16 number 1024 + q,
 // ((q << 4) | 0x6400) is 1024 + 16 q; one packed subtract / fma gives q - 8 exactly.
 #include <algorithm>
+#include "gemm_wave.hpp"
 #include "gemm_wide.hpp"
 #include "stream_ring.hpp"
 
@@ -945,12 +946,56 @@ int launch_nk_tiles(llmk::DirectArgs p, void* workspace, int64_t scratch, hipStr
                      : llmk::launch_mid<KIND, 8, false, true>(p, st, "gemm_w4a16_nk(mid, 128 columns)");
 }
 
+// What the kernels next to the wave kernels (gemm_wave.hpp) take for 17 to 512 rows, in us like the estimates there.  Up to 64
+// rows the ring kernel: its workgroups' tiles times the K steps of a wave, and the sums of its K ranges.  From there the tile
+// kernels by their form: the mid-size ones with 64 and 128 columns, the 128-column tile in K slices, or rounds of the tiles that
+// dma_tile_estimate chooses (at the rates of 4-bit weights).  A fit (3 to 10 % rms, 14 % for the K slices) to 350 shapes of M 17 to 520,
+// N 1024 to 28672, K 1024 to 14336, as are the wave kernels' estimates; choosing by both was 1 to 2 % behind the faster one of
+// each shape on average, and 1.16 (bf16 up to 64 rows) to 1.26 times faster than without the wave kernels.  Wave | other, us: bf16
+// 48 x 4096 x 4096 10.8 | 12.3, 80 x 4096 x 4096 12.6 | 19.2, 160 x 4096 x 14336 44.6 | 75.0, 96 x 14336 x 4096 31.1 | 37.8, fp16
+// 256 x 8192 x 8192 59.8 | 89.7, but 256 x 14336 x 4096 63.1 | 45.9 and bf16 24 x 4096 x 4096 9.6 | 9.2: every row tile unpacks the
+// weights again, and short rows of few columns leave its waves too little to do.
+template <int KIND>
+double nk_other_estimate(const llmk::DirectArgs& p) {
+    const int64_t M = p.M, N = p.N, K = p.K;
+    const double k = (double)K / 4096.0;
+    if (M <= 64) {
+        const int64_t nz = (K / 128 + 31) / 32, rows = ((M + 15) / 16) * nz, tiles = (N + 15) / 16;
+        const int64_t wg = std::max<int64_t>(1, LLMK_CUS / std::min<int64_t>(rows, LLMK_CUS)), per_wg = (tiles + wg - 1) / wg;
+        const double u = (double)((((K / 128 + nz - 1) / nz) + 7) / 8);
+        return 2.5 + 0.45 * u + (double)per_wg * (0.29 * u + 0.09) + (nz > 1 ? 2.9 : 0.0);
+    }
+    const NkTiles t = nk_tiles<KIND>(p);
+    if (t.form == NkTiles::MID) return 4.3 + (t.mt == 2 ? 12.0 : 17.0) * k / t.z + (t.z > 1 ? 2.5 : 0.0);
+    if (t.form == NkTiles::MIDW) return 4.4 + (t.mt == 4 ? 31.3 : 41.0) * k / t.z + (t.z > 1 ? 3.0 : 0.0);
+    if (t.z > 1) return 7.5 + 54.0 * k / t.z;
+    const llmk::TileChoice c = llmk::dma_tile_estimate<KIND, false>(p);
+    const double e = c.cost * k;
+    switch (c.choice) {
+        case 1: return 2.0 + 2.3 * e;
+        case 2: return 3.0 + 1.7 * e;
+        case 4: return 7.0 + 1.4 * e;
+        case 8: return 5.0 + 1.6 * e;
+        default: return 3.0 + 1.7 * e;
+    }
+}
+// The wave kernel for this call, or z = 0: taken 8 % below the others' estimate.
+template <int KIND>
+llmk::WavePlan nk_wave(const llmk::DirectArgs& p, int64_t scratch) {
+    llmk::WavePlan w{0, 0, 0, 0, 0.0};
+    const bool fits = KIND == llmk::K_W4NKB && p.M > 64 ? llmk::w4a16_wave_plan<KIND, KIND == llmk::K_W4NKB>(p.M, p.N, p.K, p.group, scratch, w)
+                                                        : llmk::w4a16_wave_plan<KIND>(p.M, p.N, p.K, p.group, scratch, w);
+    if (!fits || 1.08 * w.cost >= nk_other_estimate<KIND>(p)) w.z = 0;
+    return w;
+}
+
 // The kernels of a call on the [N, K/8] layout, in the order in which they are preferred, and the scratch they use: what
 // llmk_gemm_w4a16_nk runs with `scratch` bytes there, and what llmk_gemm_w4a16_nk_workspace_bytes reports for any amount.
 struct NkPlan {
-    enum { RING, TILES, COPY, RANGES, STREAM, NONE } route;
+    enum { RING, TILES, COPY, RANGES, STREAM, NONE, WAVE } route;
     int nz;
     int64_t bytes;
+    llmk::WavePlan wave;
 };
 NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scratch, bool c8) {
     const int nz = (int)((K / 128 + 31) / 32);               // K ranges of the streaming kernels
@@ -958,20 +1003,23 @@ NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scra
     const bool sums = nz == 1 || ((M * N) % 4 == 0 && scratch >= planes);
     llmk::DirectArgs p{};
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
-    if (bf && M <= 64 && c8 && sums && nk_ring_ok(M, N, K, group, nz)) return {NkPlan::RING, nz, planes};
+    llmk::WavePlan w{};
+    if (M > 16 && M <= 512) w = bf ? nk_wave<llmk::K_W4NKB>(p, scratch) : nk_wave<llmk::K_W4NK>(p, scratch);
+    if (w.z > 0) return {NkPlan::WAVE, 1, w.z > 1 ? w.z * M * N * 4 : 0, w};
+    if (bf && M <= 64 && c8 && sums && nk_ring_ok(M, N, K, group, nz)) return {NkPlan::RING, nz, planes, {}};
     if (llmk::dma_eligible(p, 2)) {
         if (w4_tiles_expand(M, N, K, scratch, true, bf) && group % 64 == 0) {
             int z = bf ? nk_tiles<llmk::K_W4NKB>(p).z : nk_tiles<llmk::K_W4NK>(p).z;
             if (M <= 64) z = max(z, llmk::splitk_factor_half(M, N, K));      // (w4_tiles_expand asks for these there)
-            return {NkPlan::TILES, 1, z > 1 ? (int64_t)z * M * N * 4 : 0};
+            return {NkPlan::TILES, 1, z > 1 ? (int64_t)z * M * N * 4 : 0, {}};
         }
         // the 16-bit copy of W, and behind it whatever the 16-bit GEMM's K slices take
-        if ((M > 64 || bf) && scratch >= N * K * 2) return {NkPlan::COPY, 1, ((N * K * 2 + 255) & ~(int64_t)255) + (M <= 512 ? 8 * M * N * 4 : 0)};
+        if ((M > 64 || bf) && scratch >= N * K * 2) return {NkPlan::COPY, 1, ((N * K * 2 + 255) & ~(int64_t)255) + (M <= 512 ? 8 * M * N * 4 : 0), {}};
     }
-    if (bf) return {NkPlan::NONE, 1, 0};
+    if (bf) return {NkPlan::NONE, 1, 0, {}};
     // K > 4096: ranges of at most 4096 (each with resident activations) and fp32 partial sums
-    if (group % 128 == 0 && M <= 64 && nz > 1 && sums && c8 && ((K / 128 + nz - 1) / nz * 128) % group == 0) return {NkPlan::RANGES, nz, planes};
-    return {NkPlan::STREAM, 1, 0};
+    if (group % 128 == 0 && M <= 64 && nz > 1 && sums && c8 && ((K / 128 + nz - 1) / nz * 128) % group == 0) return {NkPlan::RANGES, nz, planes, {}};
+    return {NkPlan::STREAM, 1, 0, {}};
 }
 
 // launch shape of the Marlin-layout kernel for a given problem
@@ -995,19 +1043,46 @@ MarlinPlan marlin_plan(int64_t M, int64_t N, int64_t K) {
     return pl;
 }
 
+// The wave kernel for a call on Marlin words, or z = 0: always up to 64 rows, up to 512 where it is estimated 8 % below the
+// 128-column tile kernels that expand the words in LDS (a fit of 3 to 7 % rms to 70 shapes: the scatter of the Marlin layout is most
+// of their time).  Choosing so was 1 % behind the faster one of each shape and 1.47 times faster than without the wave kernel over
+// 180 shapes of 16 to 528 rows.  Wave | other, us, cold weights: 16 x 4096 x 4096 9.9 | 10.6, 16 x 14336 x 4096 14.4 | 18.5, 32 x 28672
+// x 4096 25.6 | 47.2, 64 x 14336 x 4096 20.1 | 47.0, 96 x 4096 x 14336 26.9 | 52.2, 256 x 4096 x 4096 19.0 | 35.9, 192 x 14336 x 4096
+// 47.1 | 60.2, but 384 x 14336 x 4096 87.8 | 80.0.
+llmk::WavePlan marlin_wave(int64_t M, int64_t N, int64_t K, int group, int64_t scratch) {
+    llmk::WavePlan w{0, 0, 0, 0, 0.0};
+    if (M > 512 || !llmk::w4a16_wave_plan<llmk::K_W4MARLIN>(M, N, K, group, scratch, w)) { w.z = 0; return w; }
+    if (M > 64) {
+        llmk::DirectArgs p{};
+        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
+        const double k = (double)K / 4096.0;
+        const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128), z = std::min<int64_t>(llmk::splitk_factor_half(M, N, K), std::max<int64_t>(1, LLMK_CUS / tiles));
+        double other = 7.7 + 42.5 * k / z;
+        if (z == 1) {
+            const llmk::TileChoice c = llmk::dma_tile_estimate<llmk::K_W4MARLIN, false>(p);
+            other = c.choice == 1 ? 4.0 + 2.5 * c.cost * k : (c.choice == 2 ? 5.3 + 1.75 * c.cost * k : 5.0 + 1.58 * c.cost * k);
+        }
+        if (1.08 * w.cost >= other) w.z = 0;
+    }
+    return w;
+}
+
 }  // namespace
 
 extern "C" int64_t llmk_gemm_w4a16_marlin_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
+    // the group size is not known here: what the wave kernel's slices take with groups of 128, and what the others take
+    const llmk::WavePlan wave = marlin_wave(M, N, K, 128, INT64_MAX);
+    const int64_t slices = wave.z > 1 ? wave.z * M * N * 4 : 0;
     if (M > 64) {                                        // dequantised fp16 copy of W for the tiled GEMM (+ split-K partials)
         if (K % 64) return 0;
         const int z = llmk::splitk_factor_half(M, N, K);
-        return ((N * K * 2 + 255) & ~(int64_t)255) + (z > 1 ? (int64_t)z * M * N * 4 : 0);
+        return std::max(slices, ((N * K * 2 + 255) & ~(int64_t)255) + (z > 1 ? (int64_t)z * M * N * 4 : 0));
     }
     const MarlinPlan pl = marlin_plan(M, N, K);
     const int64_t zt = M > 16 && K % 64 == 0 ? llmk::splitk_factor_half(M, N, K) : 1;   // tile kernels with split-K
     const int64_t z = pl.z > zt ? pl.z : zt;
-    return z > 1 ? z * M * N * 4 : 0;
+    return std::max(slices, z > 1 ? z * M * N * 4 : 0);
 }
 
 extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, const void* s, int64_t M, int64_t N,
@@ -1027,6 +1102,13 @@ extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, 
     if (M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) LLMK_FAIL(LLMK_ERR_SHAPE, "gemm_w4a16_marlin: dimension too large");
 
     hipStream_t st = (hipStream_t)stream;
+    const llmk::WavePlan wave = marlin_wave(M, N, K, groupsize, usable_scratch(workspace, workspace_bytes));
+    if (wave.z > 0) {
+        llmk::DirectArgs p{};
+        p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.b_s = s; p.c = c; p.c_dtype = LLMK_F16;
+        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = groupsize; p.partial = (float*)workspace;
+        return llmk::launch_w4a16_wave_plan<llmk::K_W4MARLIN>(p, wave, st, "gemm_w4a16_marlin(wave)");
+    }
     if (w4_tiles_expand(M, N, K, usable_scratch(workspace, workspace_bytes)) && K % 64 == 0 && groupsize % 64 == 0) {
         // mid-size M: the 128-column tile kernels expand the Marlin units themselves (see gemm_w4a16_nk)
         llmk::DirectArgs p{};
@@ -1119,6 +1201,12 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
     p.a = (const uint8_t*)a; p.c = c; p.c_dtype = ac_dtype;
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
     switch (pl.route) {
+        case NkPlan::WAVE:
+            p.b = (const uint8_t*)b_packed; p.b_s = s; p.group = groupsize; p.partial = (float*)workspace;
+            // (bf16 beyond 64 rows: weights rounded to bf16, as every kernel of such calls has them)
+            if (!bf) return llmk::launch_w4a16_wave_plan<llmk::K_W4NK>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
+            return M > 64 ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)")
+                          : llmk::launch_w4a16_wave_plan<llmk::K_W4NKB>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
         case NkPlan::RING:                               // bf16 decode; fp16 reaches that kernel through launch_nk_stream
             return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, pl.nz, (float*)workspace, true, st);
         case NkPlan::TILES:

@@ -67,21 +67,20 @@ inline int64_t w4a8_widened_bytes(int64_t M, int64_t N, int64_t K) {
     return w4a8_a_s32_bytes(M, K) + ((((N + 127) / 128) * (K / 128) * 4 + 255) & ~(int64_t)255);
 }
 
-// Up to 256 rows the wave kernel beats both what it replaced and the two passes at every shape measured (see gemm_wave.hpp).
-// From there to 512 rows it is taken where its estimate is below that of the two passes: the expansion (1.5 bytes per weight
-// at 5 TB/s), the rounds of the int8 tiles (15 % above the fp8 estimates), 6 us for the two launches.  (us, wave | two passes:
-// 512 x 4096 x 4096 25.4 | 31.9, 384 x 4096 x 4096 22 | 30; every row tile unpacks the weights again, so large N K goes the
-// other way.)
+// Up to 128 rows the wave kernel beats both what it replaced and the two passes (1.45 times over 180 shapes of 1 to 520 rows).
+// From there to 512 rows it is taken 12 % below the estimate of the two passes: the expansion, the rounds of the int8 tiles, two
+// launches (a fit of 12 % rms to 25 shapes).  (us, wave | two passes: 512 x 4096 x 4096 25.4 | 31.9, 384 x 4096 x 4096 22 | 30, but 245 x 28672 x 4096 78.9 | 70.4; every row
+// tile unpacks the weights again, so large N K goes the other way.)
 W4A8Plan w4a8_plan(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch) {
     W4A8Plan pl{false, {}, 0};
     if (M <= 0 || N <= 0 || K <= 0) return pl;
     if (group_int4 == 128 && M <= 512 && N <= 0x7fffffff && K <= (1 << 25) && w4a8_wave_plan(M, N, K, scratch, pl.shape)) {
-        pl.wave = M <= 256;
+        pl.wave = M <= 128;
         if (!pl.wave) {
             DirectArgs q{};
             q.M = (int)M; q.N = (int)N; q.K = (int)K; q.E = 1;
-            const double two = 6.0 + (double)N * K * 1.5 / 5e6 + 1.15 * dma_tile_estimate<K_I8_BLOCK, false>(q).cost * K / 4096.0;
-            pl.wave = pl.shape.cost < two;
+            const double two = 10.0 + (double)N * K * 0.41e-6 + 0.72 * dma_tile_estimate<K_I8_BLOCK, false>(q).cost * K / 4096.0;
+            pl.wave = 1.12 * pl.shape.cost < two;
         }
     }
     const int64_t slices = pl.wave && pl.shape.z > 1 ? (int64_t)pl.shape.z * M * N * 4 : 0;

@@ -46,15 +46,70 @@ typedef unsigned short wv_us2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ wv_us2 wv_as_us2(unsigned u) { return __builtin_bit_cast(wv_us2, u); }
 __device__ __forceinline__ unsigned wv_bits(wv_us2 v) { return __builtin_bit_cast(unsigned, v); }
 
+// Tile of a workgroup.  Ids go to the eight XCDs round robin; each XCD takes an eighth of the list of tiles, column by column with
+// the row tiles of a column back to back, so that a column's weights are read through one L2.  (Columns dealt to the XCDs whole
+// give some of them more tiles than they have CUs: 216 x 2304 x 1280 16.3 us for 252 tiles, 9.1 this way.)
+struct WaveTile {
+    int col, row;
+};
+__device__ __forceinline__ WaveTile wave_tile(int M, int bm) {
+    const int lin = blockIdx.x, total = gridDim.x, rows = (M + bm - 1) / bm, x = lin & 7;
+    const int idx = x * (total >> 3) + min(x, total & 7) + (lin >> 3);
+    const int col = idx / rows;
+    return {col, idx - col * rows};
+}
+
 template <int N>
 __device__ __forceinline__ void wv_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// The end of a tile, behind the barrier that follows the waves' writes: red [wave][row][column], rows of 16 NT + 4 floats, is
+// summed over the waves in their order and stored (K slices: as fp32 sums).  A thread owns eight columns of a row.
+template <int NW, int MT, int NT>
+__device__ __forceinline__ void wv_store(const DirectArgs& p, const float* red, int n0, int m0, int m_end) {
+    constexpr int BM = 16 * MT, BN = 16 * NT, RED_ROW = BN + 4, RUNS = BN / 8, ROWS_PASS = (NW * 64) / RUNS;
+    const int tid = threadIdx.x, N = p.N;
+    const bool split = p.ksplit > 1;
+    void* cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
+    const int cdt = split ? LLMK_F32 : p.c_dtype;
+    const int esz = cdt == LLMK_F32 ? 4 : 2;
+    const bool vec_ok = ((((uintptr_t)cout) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
+    const int ocol = 8 * (tid % RUNS), nn = n0 + ocol, nv = N - nn;
+    if (nn >= N) return;
+#pragma unroll
+    for (int pass = 0; pass < (BM + ROWS_PASS - 1) / ROWS_PASS; ++pass) {
+        const int orow = pass * ROWS_PASS + tid / RUNS, m = m0 + orow;
+        if (orow >= BM || m >= m_end) continue;
+        v4f sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float* src = red + (w * BM + orow) * RED_ROW + ocol;
+            sa += *(const v4f*)src;
+            sb += *(const v4f*)(src + 4);
+        }
+        const int64_t off = (int64_t)m * N + nn;
+        if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv, vec_ok);
+        else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv, vec_ok);
+        else store_run8<LLMK_F32>(cout, off, sa, sb, nv, vec_ok);
+    }
+}
+
+// Summing pass of a launch whose K range was sliced.
+inline int wv_sum_slices(const DirectArgs& p, int z, hipStream_t stream, const char* name) {
+    const int64_t mn = (int64_t)p.M * p.N;
+    const unsigned blocks = (unsigned)cdiv64(cdiv64(mn, 4), 256);
+    if (p.c_dtype == LLMK_BF16) splitk_sum_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
+    else if (p.c_dtype == LLMK_F16) splitk_sum_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
+    else splitk_sum_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
+    LLMK_CHECK_LAUNCH(name);
+    return LLMK_OK;
+}
 
 // int8 activations [M, K] with a scale per row and 128 elements, uint4 weights packed eight rows per word [N / 8, K] with an int8
 // zero point and scale per row and 128 elements (groups) and a scale per 128 x 128 block: the int8 weight is
 // int8(int8(q - z4) * s4) with two's-complement wrap.
 // S32: fp32 scales, else 16-bit ones (fp16 or bf16 by p.s_dtype)
 template <int NW, int MT, int NT, int D, bool S32>
-__global__ __launch_bounds__((NW * 64)) void w4a8_wave_kernel(DirectArgs p) {
+__global__ __launch_bounds__(NW * 64) void w4a8_wave_kernel(DirectArgs p) {
     constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = wv_stage(MT, NT), LPS = wv_loads(MT, NT);
     constexpr int OFF_B = BM * 128, OFF_S = OFF_B + NT * 1024, TR = wv_tab_row(NT);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -69,8 +124,8 @@ __global__ __launch_bounds__((NW * 64)) void w4a8_wave_kernel(DirectArgs p) {
         kt0 = (int)blockIdx.z * per;
         KT = min(per, KT_all - kt0);
     }
-    const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM, m_end = min(p.M, m0 + BM);
-    if (n0 >= N) return;                                    // the grid is padded to a multiple of the XCDs
+    const WaveTile tile = wave_tile(p.M, BM);
+    const int n0 = tile.col * BN, m0 = tile.row * BM, m_end = min(p.M, m0 + BM);
     const int s_lo = wave * KT / NW, n = (wave + 1) * KT / NW - s_lo;
 
     uint8_t* const mine = lds + wave * (D * STAGE);
@@ -148,7 +203,7 @@ __global__ __launch_bounds__((NW * 64)) void w4a8_wave_kernel(DirectArgs p) {
 
     ring_wait<D * LPS>(t_s, t_z, t_bs);
     if (tid < BN * W) tab_put(t_col, t_w, t_shift, (unsigned)t_s, (unsigned)t_z);
-    for (int idx = tid + (NW * 64); idx < BN * W; idx += (NW * 64)) {
+    for (int idx = tid + NW * 64; idx < BN * W; idx += NW * 64) {
         int col, w, shift;
         const uint32_t at = tab_at(idx, col, w, shift);
         unsigned vs, vz;
@@ -282,30 +337,7 @@ __global__ __launch_bounds__((NW * 64)) void w4a8_wave_kernel(DirectArgs p) {
         }
     }
     __syncthreads();
-    constexpr int RUNS = BN / 8, ROWS_PASS = (NW * 64) / RUNS;
-    const bool split = p.ksplit > 1;
-    void* cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
-    const int cdt = split ? LLMK_F32 : p.c_dtype;
-    const int esz = cdt == LLMK_F32 ? 4 : 2;
-    const bool vec_ok = ((((uintptr_t)cout) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
-    const int ocol = 8 * (tid % RUNS), nn = n0 + ocol, nv = N - nn;
-    if (nn >= N) return;
-#pragma unroll
-    for (int pass = 0; pass < (BM + ROWS_PASS - 1) / ROWS_PASS; ++pass) {
-        const int orow = pass * ROWS_PASS + tid / RUNS, m = m0 + orow;
-        if (orow >= BM || m >= m_end) continue;
-        v4f sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const float* src = red + (w * BM + orow) * RED_ROW + ocol;
-            sa += *(const v4f*)src;
-            sb += *(const v4f*)(src + 4);
-        }
-        const int64_t off = (int64_t)m * N + nn;
-        if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv, vec_ok);
-        else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv, vec_ok);
-        else store_run8<LLMK_F32>(cout, off, sa, sb, nv, vec_ok);
-    }
+    wv_store<NW, MT, NT>(p, red, n0, m0, m_end);
 }
 
 template <int NW, int MT, int NT, int D, bool S32>
@@ -319,18 +351,346 @@ int launch_w4a8_wave(const DirectArgs& p, int z, hipStream_t stream, const char*
     DirectArgs q = p;
     q.ksplit = z;
     const int zg = (KT_all + per - 1) / per;
-    unsigned gx = (unsigned)((p.N + 16 * NT - 1) / (16 * NT)), gy = (unsigned)((p.M + 16 * MT - 1) / (16 * MT));
-    if (gy > 1) gx = (gx + 7) & ~7u;
-    kern<<<dim3(gx, gy, (unsigned)zg), (NW * 64), bytes, stream>>>(q);
+    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
+    kern<<<dim3(tiles, 1, (unsigned)zg), NW * 64, bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
-    if (z > 1) {
-        const int64_t mn = (int64_t)p.M * p.N;
-        const unsigned blocks = (unsigned)cdiv64(cdiv64(mn, 4), 256);
-        if (p.c_dtype == LLMK_BF16) splitk_sum_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, zg);
-        else if (p.c_dtype == LLMK_F16) splitk_sum_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, zg);
-        else splitk_sum_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, zg);
-        LLMK_CHECK_LAUNCH(name);
+    if (z > 1) return wv_sum_slices(p, zg, stream, name);
+    return LLMK_OK;
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// fp16 / bf16 activations [M, K], 4-bit weights with fp16 group scales: row-packed [N, K / 8] (K_W4NK, K_W4NKB) or Marlin words
+// (K_W4MARLIN).  K steps are 128 elements of weights and two halves of 64 elements (128 bytes) of activations: per wave one
+// stage of activation rows and two of packed words (a second stage of activations has no room beside 64 rows).
+// What bounds it: latency.  64 x 14336 x 4096, of 37600 cycles a wave lives: vector ALU 46 %, address path 52 %, LDS 30 %, MFMA 22 %;
+// a half's activations are requested one half ahead, which two waves per SIMD do not cover.  The words of a chunk come from LDS
+// with the order of the activations' dwords as the Marlin fragments want it; scattering them into rows was most of the tile kernel.
+// us per launch, before | now, cold weights: Marlin 16 x 14336 x 4096 18.5 | 14.4, 64 x 14336 x 4096 47.0 | 20.1, 96 x 4096 x 14336
+// 52.2 | 26.9, 256 x 4096 x 4096 35.9 | 19.0; [N, K / 8] bf16 48 x 22096 x 4352 42.4 | 32.4, 80 x 4096 x 4096 19.2 | 12.8, 160 x 4096 x
+// 14336 75.0 | 44.6, fp16 128 x 8192 x 8192 51.5 | 33.6.
+constexpr int wh_a(int mt) { return 16 * mt * 128; }
+constexpr bool wh_marlin(int kind) { return kind == K_W4MARLIN; }
+constexpr int wh_b(int kind, int nt) { return wh_marlin(kind) ? 4096 : nt * 1024; }     // Marlin: the whole 64-column chunk
+constexpr int wh_stage(int kind, int mt, int nt) { return wh_a(mt) + 2 * wh_b(kind, nt); }
+constexpr int wh_tab_cols(int kind, int nt) { return wh_marlin(kind) ? 64 : 16 * nt; }
+constexpr int wh_tab_row(int kind, int nt) { return 2 * wh_tab_cols(kind, nt) + 8; }
+constexpr int wh_lds(int kind, int nw, int mt, int nt, int groups) {
+    const int a = nw * wh_stage(kind, mt, nt) + wh_tab_row(kind, nt) * groups, b = wv_red(nw, mt, nt);
+    return a > b ? a : b;
+}
+
+// groups that `per` K steps touch, at most
+constexpr int wh_groups(int K, int group, int per) {
+    const int a = (per * 128 - 1) / group + 2, b = K / group;
+    return a < b ? a : b;
+}
+
+// PRE (bf16): the weights are (q - 8) * scale rounded to bf16, as the tile kernels of larger M have them, and sums run over
+// all of K; otherwise they are q - 8 exactly and the scale multiplies the fp32 sums of a half step.
+template <int KIND, int NW, int MT, int NT, bool PRE>
+__global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
+    static_assert(is_w4nk(KIND) || wh_marlin(KIND), "4-bit weights, 16-bit activations");
+    static_assert(!PRE || KIND == K_W4NKB, "scaled weights: bf16");
+    constexpr bool MARLIN = wh_marlin(KIND), BF = (KIND == K_W4NKB);
+    constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = wh_stage(KIND, MT, NT), OFF_B = wh_a(MT), WB = wh_b(KIND, NT), NB = WB / 1024;
+    constexpr int TR = wh_tab_row(KIND, NT), TC = wh_tab_cols(KIND, NT);
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int N = p.N, K = p.K, KT_all = K >> 7, G = K / p.group, nchunks = N >> 6;
+    int kt0 = 0, KT = KT_all;
+    if (p.ksplit > 1) {
+        const int per = (KT_all + p.ksplit - 1) / p.ksplit;
+        kt0 = (int)blockIdx.z * per;
+        KT = min(per, KT_all - kt0);
     }
+    // Marlin: the workgroups that share a chunk (64 columns) are neighbours in the list of tiles, so that one L2 serves them
+    const WaveTile tile = wave_tile(p.M, BM);
+    const int n0 = tile.col * BN, m0 = tile.row * BM, m_end = min(p.M, m0 + BM);
+    const int chunk = n0 >> 6, sub = MARLIN ? tile.col & (4 / NT - 1) : 0;
+    const int s_lo = wave * KT / NW, n = (wave + 1) * KT / NW - s_lo;
+
+    uint8_t* const mine = lds + wave * STAGE;
+    const uint32_t mine_addr = lds_base + (uint32_t)wave * STAGE;
+    uint8_t* const tab = lds + NW * STAGE;                   // [group][column] fp16
+
+    // ---- group scales of the tile, requested first (four per load)
+    const int g_lo = kt0 * 128 / p.group, GR = ((kt0 + KT) * 128 - 1) / p.group - g_lo + 1;
+    const int W = (GR + 3) >> 2, tab_n = MARLIN ? GR * 16 : BN * W;
+    const uint8_t* const tabp = (const uint8_t*)p.b_s + (MARLIN ? ((int64_t)g_lo * N + chunk * 64) * 2 : (int64_t)n0 * G * 2);
+    const uint32_t tab_last = (uint32_t)min((int64_t)(N - n0) * G * 2 - 8, (int64_t)0x7fffffff);
+    auto tab_at = [&](int idx, int& col, int& w, int& shift) {
+        if constexpr (MARLIN) {                              // col: unit of four scales, w: group
+            w = min(idx >> 4, GR - 1);
+            col = idx & 15;
+            shift = 0;
+            return (uint32_t)w * (uint32_t)(N * 2) + (uint32_t)col * 8u;
+        } else {
+            col = idx / W;
+            w = idx - col * W;
+            const uint32_t want = ((uint32_t)min(min(col, BN - 1), N - 1 - n0) * (uint32_t)G + (uint32_t)(g_lo + 4 * w)) * 2u;
+            const uint32_t at = min(want, tab_last);
+            shift = (int)(want - at) * 8;
+            return at;
+        }
+    };
+    auto tab_put = [&](int col, int w, int shift, uint64_t v) {
+        if constexpr (MARLIN) {
+            // scale 8 c + 2 j + b of a chunk belongs to column 16 j + 8 b + c
+            const int c = col >> 1, j = 2 * (col & 1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) *(unsigned short*)(tab + w * TR + 2 * (16 * (j + (e >> 1)) + 8 * (e & 1) + c)) = (unsigned short)(v >> (16 * e));
+        } else {
+            v = shift < 64 ? v >> shift : 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * w + e < GR) *(unsigned short*)(tab + (4 * w + e) * TR + 2 * col) = (unsigned short)(v >> (16 * e));
+        }
+    };
+    int t_col, t_w, t_shift;
+    v2i t_s;
+    {
+        const uint32_t at = tab_at(tid, t_col, t_w, t_shift);
+        t_s = ring_load_b64<0>(at, ring_base(tabp));
+    }
+
+    // ---- source offsets.  16-byte chunk c of activation row R lies at chunk c ^ swizzle(R): 16 rows x one chunk (row-packed) and
+    // 16 rows x four dwords of one chunk (Marlin) then fall into different banks.
+    auto swizzle = [](int row) { return MARLIN ? (((row >> 1) & 3) * 2) | ((row >> 3) & 1) : ((row >> 1) & 7); };
+    uint32_t aoff[2 * MT], boff[NB];
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+        const int row = 8 * i + (lane >> 3), sw = swizzle(row);
+        aoff[i] = (uint32_t)min(row, m_end - 1 - m0) * (uint32_t)(K * 2) + (uint32_t)((lane & 7) ^ sw) * 16u;
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        if constexpr (MARLIN) {
+            // strip 2 i + (lane >> 5) of the step: 512 contiguous bytes per chunk
+            boff[i] = (uint32_t)(2 * i + (lane >> 5)) * (uint32_t)(nchunks * 512) + (uint32_t)(lane & 31) * 16u;
+        } else {
+            // 64 bytes of each of 16 rows
+            const int row = 16 * i + (lane >> 2);
+            boff[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)(K >> 1) + (uint32_t)((lane & 3) ^ (((row >> 2) & 1) << 1)) * 16u;
+        }
+    }
+    const uint8_t* const ga = p.a + (int64_t)m0 * K * 2;
+    const uint8_t* const gb = p.b + (MARLIN ? (int64_t)chunk * 512 : (int64_t)n0 * (K >> 1));
+    const int64_t b_step = MARLIN ? (int64_t)nchunks * 4096 : 64;
+    auto issue_a = [&](int s, int h) __attribute__((always_inline)) {
+        const uint8_t* src = ga + ((int64_t)(kt0 + min(s, KT - 1)) * 2 + h) * 128;
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) dma16(mine_addr + i * 1024u, aoff[i], src);
+    };
+    auto issue_b = [&](int s, int slot) __attribute__((always_inline)) {
+        const uint8_t* src = gb + (int64_t)(kt0 + min(s, KT - 1)) * b_step;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) dma16(mine_addr + OFF_B + (uint32_t)slot * WB + i * 1024u, boff[i], src);
+    };
+    issue_b(s_lo, 0);
+    issue_a(s_lo, 0);
+    issue_b(s_lo + 1, 1);
+
+    ring_wait<2 * MT + 2 * NB>(t_s);
+    if (tid < tab_n) tab_put(t_col, t_w, t_shift, __builtin_bit_cast(uint64_t, t_s));
+    for (int idx = tid + NW * 64; idx < tab_n; idx += NW * 64) {
+        int col, w, shift;
+        const uint32_t at = tab_at(idx, col, w, shift);
+        uint64_t v;
+        __builtin_memcpy(&v, tabp + at, 8);
+        tab_put(col, w, shift, v);
+    }
+    __syncthreads();
+
+    // acc[mt][j][i] = C[row 16 mt + r][column 16 j + 4 g + i] over this wave's K steps
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+
+    // a[mt][f]: activation fragment of 32 of the half's 64 elements, in the order of the unpacked weights
+    v4i a[MT][2];
+    // w[j][f] (row-packed): the word of columns 16 j + r, elements 16 g + 8 f .. + 7 of the half
+    // w[st][j] (Marlin): word j of unit (c, g) of strip st of the half
+    unsigned w[MARLIN ? 4 : NT][MARLIN ? NT : 2];
+    const int swz = swizzle(r);
+    auto fetch = [&](int h, int slot) __attribute__((always_inline)) {
+        const uint8_t* bst = mine + OFF_B + slot * WB;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const uint8_t* row = mine + mt * 2048 + r * 128;
+                if constexpr (MARLIN) {
+                    // strips 2 f, 2 f + 1 of 16 elements: elements 2 g, 2 g + 1, 2 g + 8, 2 g + 9 of each
+#pragma unroll
+                    for (int st = 0; st < 2; ++st) {
+                        a[mt][f][2 * st] = *(const int*)(row + (((4 * f + 2 * st) ^ swz) * 16) + 4 * g);
+                        a[mt][f][2 * st + 1] = *(const int*)(row + (((4 * f + 2 * st + 1) ^ swz) * 16) + 4 * g);
+                    }
+                } else {
+                    a[mt][f] = *(const v4i*)(row + (((2 * g + f) ^ swz) * 16));
+                }
+            }
+        if constexpr (MARLIN) {
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                const uint8_t* u = bst + (4 * h + st) * 512 + (4 * (r & 7) + g) * 16 + sub * (4 * NT);
+                if constexpr (NT == 4) {
+                    const v4i x = *(const v4i*)u;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) w[st][j] = (unsigned)x[j];
+                } else if constexpr (NT == 2) {
+                    const v2i x = *(const v2i*)u;
+                    w[st][0] = (unsigned)x[0];
+                    w[st][1] = (unsigned)x[1];
+                } else {
+                    w[st][0] = *(const unsigned*)u;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const v2i x = *(const v2i*)(bst + (16 * j + r) * 64 + (((2 * h + (g >> 1)) ^ (((r >> 2) & 1) << 1)) * 16) + 8 * (g & 1));
+                w[j][0] = (unsigned)x[0];
+                w[j][1] = (unsigned)x[1];
+            }
+        }
+    };
+    auto lo8 = [](unsigned x) { return w4_as_u32(w4_as_h2((x & 0x000f000fu) | 0x64006400u) - (v2h){(_Float16)1032.f, (_Float16)1032.f}); };
+    auto hi8 = [](unsigned x) {
+        return w4_as_u32(w4_as_h2((x & 0x00f000f0u) | 0x64006400u) * (v2h){(_Float16)0.0625f, (_Float16)0.0625f} - (v2h){(_Float16)72.f, (_Float16)72.f});
+    };
+    auto mma = [](const v4i& x, const v4i& y, v4f c) {
+        if constexpr (BF) return mfma_bf16_16x16x32(__builtin_bit_cast(v8bf, x), __builtin_bit_cast(v8bf, y), c);
+        else return mfma_f16_16x16x32(__builtin_bit_cast(v8h, x), __builtin_bit_cast(v8h, y), c);
+    };
+    const int mshift = 8 * (r >> 3);
+    auto compute = [&](int s) __attribute__((always_inline)) {
+        const uint8_t* tr = tab + ((kt0 + s) * 128 / p.group - g_lo) * TR + 2 * (MARLIN ? sub * BN : 0) + (PRE ? 2 * r : 8 * g);
+        v4f init[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            init[mt] = (v4f){0.f, 0.f, 0.f, 0.f};
+            if constexpr (!MARLIN && !PRE) {
+                // a word unpacks in the order 0, 4, 1, 5, 2, 6, 3, 7: the same for the activations
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    const v4i x = a[mt][f];
+                    a[mt][f] = (v4i){(int)__builtin_amdgcn_perm((unsigned)x[2], (unsigned)x[0], 0x05040100u), (int)__builtin_amdgcn_perm((unsigned)x[2], (unsigned)x[0], 0x07060302u),
+                                     (int)__builtin_amdgcn_perm((unsigned)x[3], (unsigned)x[1], 0x05040100u), (int)__builtin_amdgcn_perm((unsigned)x[3], (unsigned)x[1], 0x07060302u)};
+                }
+            }
+            if constexpr (BF && !PRE) {
+                // bf16: a nibble becomes 128 + q, exactly; the missing - 136 of every product is where the sums start
+                const v4i c136 = {(int)0xc308c308u, (int)0xc308c308u, (int)0xc308c308u, (int)0xc308c308u};
+                init[mt] = mma(c136, a[mt][0], init[mt]);
+                init[mt] = mma(c136, a[mt][1], init[mt]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            if constexpr (PRE) {
+                const float sc = f16_to_f32(*(const unsigned short*)(tr + 32 * j));
+                const v4i b0 = w4_word_to_bf16x8(w[j][0], sc), b1 = w4_word_to_bf16x8(w[j][1], sc);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    acc[mt][j] = mma(b0, a[mt][0], acc[mt][j]);
+                    acc[mt][j] = mma(b1, a[mt][1], acc[mt][j]);
+                }
+                continue;
+            }
+            const uint64_t sw = *(const uint64_t*)(tr + 32 * j);
+            v4f sc;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc[i] = f16_to_f32((unsigned short)(sw >> (16 * i)));
+            v4i b[2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                if constexpr (MARLIN) {
+                    const unsigned u0 = w[2 * f][j] >> mshift, u1 = w[2 * f + 1][j] >> mshift;
+                    b[f] = (v4i){(int)lo8(u0), (int)hi8(u0), (int)lo8(u1), (int)hi8(u1)};
+                } else if constexpr (BF) {
+                    const unsigned x = w[j][f];
+                    b[f] = (v4i){(int)((x & 0x000f000fu) | 0x43004300u), (int)(((x >> 4) & 0x000f000fu) | 0x43004300u),
+                                 (int)(((x >> 8) & 0x000f000fu) | 0x43004300u), (int)(((x >> 12) & 0x000f000fu) | 0x43004300u)};
+                } else {
+                    const unsigned x = w[j][f], x8 = x >> 8;
+                    b[f] = (v4i){(int)lo8(x), (int)hi8(x), (int)lo8(x8), (int)hi8(x8)};
+                }
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                v4f t = mma(b[0], a[mt][0], init[mt]);
+                t = mma(b[1], a[mt][1], t);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[mt][j][i] = fmaf(t[i], sc[i], acc[mt][j][i]);
+            }
+        }
+    };
+    // the registers hold what they need of the stage: the next loads may overwrite it
+    auto fetched = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);                  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // Step s: half 0 needs the activations requested last and the words requested a step before them; the words of step
+    // s + 1, requested behind those activations, may stay in flight.  Half 1 needs activations requested behind them.
+    int slot = 0;
+    for (int i = 0; i < n; ++i) {
+        const int s = s_lo + i;
+        const bool more = i + 1 < n;
+        if (more) wv_wait_loads<NB>();
+        else wv_wait_loads<0>();
+        fetch(0, slot);
+        fetched();
+        issue_a(s, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s);
+        __builtin_amdgcn_sched_barrier(0);
+        wv_wait_loads<0>();
+        fetch(1, slot);
+        fetched();
+        if (more) {
+            issue_a(s + 1, 0);
+            if (i + 2 < n) issue_b(s + 2, slot);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s);
+        __builtin_amdgcn_sched_barrier(0);
+        slot ^= 1;
+    }
+    wv_wait_loads<0>();
+    __syncthreads();
+
+    float* red = (float*)lds;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) *(v4f*)(red + (wave * BM + 16 * mt + r) * (BN + 4) + 16 * j + 4 * g) = acc[mt][j];
+    __syncthreads();
+    wv_store<NW, MT, NT>(p, red, n0, m0, m_end);
+}
+
+template <int KIND, int NW, int MT, int NT, bool PRE>
+int launch_w4a16_wave(const DirectArgs& p, int z, hipStream_t stream, const char* name) {
+    static std::atomic<uint64_t> configured{0};
+    auto kern = w4a16_wave_kernel<KIND, NW, MT, NT, PRE>;
+    const int KT_all = p.K >> 7, per = (KT_all + z - 1) / z, groups = wh_groups(p.K, p.group, per);
+    const int bytes = wh_lds(KIND, NW, MT, NT, groups);
+    if (bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, bytes);
+    if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
+    DirectArgs q = p;
+    q.ksplit = z;
+    const int zg = (KT_all + per - 1) / per;
+    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
+    kern<<<dim3(tiles, 1, (unsigned)zg), NW * 64, bytes, stream>>>(q);
+    LLMK_CHECK_LAUNCH(name);
+    if (z > 1) return wv_sum_slices(p, zg, stream, name);
     return LLMK_OK;
 }
 
@@ -340,36 +700,83 @@ struct WavePlan {
     double cost;
 };
 
-// us of a tile of eight waves per K step of each of them, [mt - 1][log2 nt] (a fit to launches of 8 to 14 steps a wave)
-constexpr double WV_STEP_US[4][3] = {{0.68, 0.94, 1.38}, {1.04, 1.30, 1.68}, {1.43, 1.58, 1.90}, {1.75, 1.86, 2.30}};
+// Estimated microseconds of a launch without its K slices' sums.  Eight waves: base + rounds of 256 workgroups x (fixed + K steps
+// of a wave x step).  Four waves (64 columns): several workgroups share a CU and cover each other's prologue and reduction, so
+// their rounds count in fractions; slower on a single round (w4a8 64 x 14336 x 4096 18.2 against 17.0 us), faster from two on
+// (64 x 28672 x 4096 27.6 against 30.2, 128 rows 46.8 against 54).  The numbers are a fit (5 to 8 % rms) to 100 to 180 shapes of M
+// 1 to 520, N 1024 to 28672, K 1024 to 14336 a kind, every tile shape timed; [mt - 1][log2 nt], and [mt - 1] for four waves (0:
+// shape not built).
+struct WaveModel {
+    float base8[4][3], fixed8[4][3], step8[4][3], base4[4], step4[4];
+};
+constexpr WaveModel WV_W4A8 = {{{3.78f, 3.77f, 3.94f}, {3.69f, 3.84f, 3.81f}, {4.04f, 3.99f, 1.38f}, {3.85f, 1.75f, 1.46f}},
+                               {{0.10f, 0.00f, 0.00f}, {0.29f, 0.33f, 0.54f}, {0.00f, 0.39f, 3.16f}, {0.00f, 2.52f, 3.59f}},
+                               {{0.45f, 0.73f, 1.16f}, {0.52f, 0.78f, 1.39f}, {0.70f, 0.97f, 1.71f}, {0.88f, 1.22f, 1.97f}},
+                               {0.f, 0.f, 6.03f, 5.54f}, {0.f, 0.f, 1.06f, 1.28f}};
+constexpr WaveModel WV_NK = {{{4.12f, 4.10f, 1.50f}, {3.89f, 3.63f, 1.48f}, {3.60f, 1.76f, 1.38f}, {2.14f, 1.85f, 1.60f}},
+                             {{0.05f, 0.00f, 2.17f}, {0.05f, 0.36f, 2.65f}, {0.23f, 2.21f, 3.03f}, {1.75f, 1.91f, 2.86f}},
+                             {{0.48f, 0.76f, 1.52f}, {0.72f, 1.03f, 1.85f}, {0.98f, 1.38f, 2.22f}, {1.27f, 1.75f, 2.68f}},
+                             {5.42f, 4.67f, 4.98f, 0.f}, {0.80f, 1.17f, 1.49f, 0.f}};
+constexpr WaveModel WV_NKB = {{{4.29f, 4.16f, 1.27f}, {4.05f, 3.52f, 0.87f}, {3.98f, 1.53f, 0.87f}, {1.65f, 1.31f, 1.29f}},
+                              {{0.02f, 0.00f, 2.40f}, {0.00f, 0.27f, 3.23f}, {0.00f, 2.42f, 3.72f}, {2.45f, 3.05f, 3.77f}},
+                              {{0.46f, 0.73f, 1.37f}, {0.74f, 1.05f, 1.70f}, {1.00f, 1.32f, 2.03f}, {1.21f, 1.55f, 2.51f}},
+                              {4.12f, 3.88f, 4.64f, 0.f}, {0.90f, 1.21f, 1.52f, 0.f}};
+constexpr WaveModel WV_NKB_PRE = {{{4.27f, 4.14f, 1.97f}, {3.67f, 4.35f, 1.77f}, {3.53f, 1.94f, 1.41f}, {2.02f, 1.92f, 1.23f}},
+                                  {{0.23f, 0.00f, 1.85f}, {0.20f, 0.03f, 2.63f}, {0.21f, 2.07f, 3.39f}, {1.65f, 2.38f, 3.92f}},
+                                  {{0.47f, 0.99f, 2.20f}, {0.71f, 1.18f, 2.36f}, {0.95f, 1.50f, 2.52f}, {1.26f, 1.66f, 2.74f}},
+                                  {5.60f, 6.28f, 5.30f, 0.f}, {1.06f, 1.28f, 1.62f, 0.f}};
+constexpr WaveModel WV_MARLIN = {{{1.94f, 1.67f, 1.52f}, {1.76f, 1.81f, 1.64f}, {2.06f, 1.78f, 1.59f}, {2.22f, 1.84f, 1.41f}},
+                                 {{1.51f, 1.93f, 2.15f}, {1.76f, 2.14f, 2.51f}, {1.77f, 2.36f, 3.02f}, {1.89f, 2.46f, 3.45f}},
+                                 {{0.82f, 1.04f, 1.44f}, {1.05f, 1.28f, 1.79f}, {1.31f, 1.61f, 2.12f}, {1.54f, 1.88f, 2.53f}},
+                                 {4.60f, 5.15f, 5.21f, 0.f}, {0.84f, 1.15f, 1.50f, 0.f}};
+template <int KIND, bool PRE>
+constexpr const WaveModel& wave_model() {
+    if constexpr (KIND == K_W4MARLIN) return WV_MARLIN;
+    else if constexpr (KIND == K_W4NK) return WV_NK;
+    else if constexpr (PRE) return WV_NKB_PRE;
+    else return WV_NKB;
+}
 
-// The cheapest shape that fits.  Eight waves: rounds of 256 workgroups, each a fixed part (tables, first loads, reduction) and
-// its steps.  Four waves (48 and 64 rows, 64 columns): two workgroups share a CU and cover each other's fixed parts, so their
-// rounds are counted in fractions; slower on a single round (64 x 14336 x 4096 18.2 against 17.0 us), faster from two on
-// (64 x 28672 x 4096 27.6 against 30.2, 128 rows 46.8 against 54).  K slices cost a second launch and their fp32 sums.
-inline bool w4a8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
-    const int64_t KT = K >> 7;
+// The cheapest shape whose LDS (bytes(nw, mt, nt, K steps of a workgroup)) and scratch fit; K slices cost a second launch and
+// their fp32 sums.
+template <class Bytes>
+inline bool wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, const WaveModel& m, Bytes bytes, WavePlan& best) {
+    const int KT = (int)(K >> 7), zmin = (KT + WV_MAX_STEPS - 1) / WV_MAX_STEPS, zmax = zmin > 4 ? zmin : 4;
+    const double us_sum = (double)(M * N) * 8.0 / 6e6;
+    int64_t ct[3];
+    for (int j = 0; j < 3; ++j) ct[j] = (N + (16 << j) - 1) >> (4 + j);
     bool found = false;
-    for (int nw = 8; nw >= 4; nw -= 4)
-        for (int mt = 1; mt <= 4; ++mt)
-            for (int nt = 1; nt <= 4; nt *= 2) {
-                if ((mt > 1 && M <= 16 * (mt - 1)) || (nw == 4 && (mt < 3 || nt < 4))) continue;
-                const int64_t tiles = ((N + 16 * nt - 1) / (16 * nt)) * ((M + 16 * mt - 1) / (16 * mt));
-                const int64_t zmin = (KT + WV_MAX_STEPS - 1) / WV_MAX_STEPS;
-                for (int64_t z = zmin; z <= (zmin > 4 ? zmin : 4); z *= 2) {
-                    const int64_t per = (KT + z - 1) / z;
-                    if (z > 1 && ((z > zmin && (per < 8 || tiles * z > 320)) || scratch < z * M * N * 4)) continue;
-                    if (wv_lds(nw, mt, nt, wv_depth(mt, nt, per), (int)per) > D_LDS_MAX) continue;
-                    const int64_t steps = (per + nw - 1) / nw;
+    for (int z = zmin; z <= zmax; z *= 2) {
+        const int per = (KT + z - 1) / z, steps8 = (per + 7) >> 3, steps4 = (per + 3) >> 2;
+        if (z > 1 && ((z > zmin && per < 8) || scratch < z * M * N * 4)) continue;
+        for (int mt = 1; mt <= 4 && (mt == 1 || M > 16 * (mt - 1)); ++mt) {
+            const int64_t rt = (M + 16 * mt - 1) / (16 * mt);
+            for (int j = 0; j < 3; ++j) {
+                const int64_t wgs = ct[j] * rt * z;
+                if (z > zmin && wgs > LLMK_CUS + LLMK_CUS / 4) continue;
+                for (int nw = 8; nw >= 4; nw -= 4) {
+                    if (nw == 4 && (j < 2 || m.step4[mt - 1] == 0.f)) continue;
                     double cost;
-                    if (nw == 8) cost = (double)((tiles * z + LLMK_CUS - 1) / LLMK_CUS) * ((nt < 4 ? 2.5 : 4.5) + steps * WV_STEP_US[mt - 1][nt >> 1]);
-                    else cost = 6.0 + (tiles * z > LLMK_CUS ? (double)(tiles * z) / LLMK_CUS : 1.0) * steps * (mt == 4 ? 1.22 : 1.04);
-                    if (z > 1) cost += 3.5 + (double)(z * M * N) * 8.0 / 5e6;
-                    if (!found || cost < best.cost) best = WavePlan{nw, mt, nt, (int)z, cost};
+                    if (nw == 8) cost = m.base8[mt - 1][j] + (double)((wgs + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[mt - 1][j] + steps8 * m.step8[mt - 1][j]);
+                    else cost = m.base4[mt - 1] + (wgs > LLMK_CUS ? (double)wgs / LLMK_CUS : 1.0) * steps4 * m.step4[mt - 1];
+                    if (z > 1) cost += 3.0 + z * us_sum;
+                    if ((found && cost >= best.cost) || bytes(nw, mt, 1 << j, per) > D_LDS_MAX) continue;
+                    best = WavePlan{nw, mt, 1 << j, z, cost};
                     found = true;
                 }
             }
+        }
+    }
     return found;
+}
+inline bool w4a8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
+    return wave_plan(M, N, K, scratch, WV_W4A8, [](int nw, int mt, int nt, int per) { return wv_lds(nw, mt, nt, wv_depth(mt, nt, per), per); }, best);
+}
+// 16-bit activations: groups in whole K steps, and a scale table of at least one load
+template <int KIND, bool PRE = false>
+inline bool w4a16_wave_plan(int64_t M, int64_t N, int64_t K, int group, int64_t scratch, WavePlan& best) {
+    if (K % 128 || group % 128 || N * (K / group) < 4 || K > (1 << 24) || N * (K / 2) >= (1ll << 40)) return false;
+    return wave_plan(M, N, K, scratch, wave_model<KIND, PRE>(), [&](int nw, int mt, int nt, int per) { return wh_lds(KIND, nw, mt, nt, wh_groups((int)K, group, per)); }, best);
 }
 
 inline int launch_w4a8_wave_plan(const DirectArgs& p, const WavePlan& w, hipStream_t stream, const char* name) {
@@ -392,6 +799,23 @@ inline int launch_w4a8_wave_plan(const DirectArgs& p, const WavePlan& w, hipStre
         }
         return w.nt == 2 ? run(i8, mt, i2, i1) : run(i8, mt, i1, i1);
     };
+    return w.mt == 1 ? rows(i1) : (w.mt == 2 ? rows(i2) : (w.mt == 3 ? rows(i3) : rows(i4)));
+}
+
+template <int KIND, bool PRE = false>
+inline int launch_w4a16_wave_plan(const DirectArgs& p, const WavePlan& w, hipStream_t stream, const char* name) {
+    auto rows = [&](auto mt) {
+        constexpr int MT = decltype(mt)::value;
+        if constexpr (wave_model<KIND, PRE>().step4[MT - 1] != 0.f) {
+            if (w.nw == 4) return launch_w4a16_wave<KIND, 4, MT, 4, PRE>(p, w.z, stream, name);
+        }
+        return w.nt == 4 ? launch_w4a16_wave<KIND, 8, MT, 4, PRE>(p, w.z, stream, name)
+                         : (w.nt == 2 ? launch_w4a16_wave<KIND, 8, MT, 2, PRE>(p, w.z, stream, name) : launch_w4a16_wave<KIND, 8, MT, 1, PRE>(p, w.z, stream, name));
+    };
+    const std::integral_constant<int, 1> i1;
+    const std::integral_constant<int, 2> i2;
+    const std::integral_constant<int, 3> i3;
+    const std::integral_constant<int, 4> i4;
     return w.mt == 1 ? rows(i1) : (w.mt == 2 ? rows(i2) : (w.mt == 3 ? rows(i3) : rows(i4)));
 }
 

@@ -426,8 +426,7 @@ PyObject* w4a8_gemm(const Args& g) {
     const int group = (int)g.integer(6);
     require(a_s.scalar_type() == b_s.scalar_type(), "activation and weight scales must share a dtype");
     const at::ScalarType out = default_dtype();
-    // what this shape's kernels use: nothing for the fused decode kernel with K <= 4096, fp32 partial sums for its
-    // K ranges or the K slices of the fused tile kernels, the expanded int8 weights + the int8 GEMM's scratch otherwise
+    // what this shape's kernels use: fp32 sums of K slices, or the expanded int8 weights and the int8 GEMM's scratch
     Scratch ws(g, a, g.st->llmk_gemm_w4a8_workspace_bytes(M, N, K, group));
     at::Tensor c;
     unlocked([&] {

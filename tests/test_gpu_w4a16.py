@@ -340,6 +340,60 @@ def test_w4a16_nk_decode_full_ranges(dev, dtype, M, N, K):
     test_w4a16_nk_decode_any_number_of_steps(dev, dtype, M, N, K)
 
 
+# every tile shape of the kernels whose waves stream their own K share: 16 to 64 rows x 16 to 64 columns of a workgroup, four and
+# eight waves, ragged rows and columns, fewer K steps than waves, K slices; then groups of several K steps
+WAVE_NK = [(17, 8200, 4224, 128), (64, 8200, 128, 128), (33, 20008, 128, 128), (33, 8200, 8320, 128), (65, 8, 256, 128),
+           (97, 1032, 1152, 128), (65, 3000, 640, 128), (128, 520, 256, 128), (65, 2056, 1152, 128), (70, 4104, 896, 128),
+           (97, 1032, 384, 128), (250, 1032, 640, 128), (100, 4104, 1024, 128), (97, 3000, 896, 128), (49, 12296, 640, 128),
+           (17, 12296, 128, 128), (33, 4104, 4224, 128), (31, 14344, 1152, 128), (40, 6152, 2176, 128), (49, 14344, 896, 128),
+           (160, 1032, 640, 128), (100, 6152, 1024, 128), (97, 1000, 1152, 384), (80, 520, 2048, -1)]
+WAVE_MARLIN = [(32, 8256, 128, 128), (16, 4160, 8320, 128), (64, 12352, 128, 128), (32, 4160, 8320, 128), (48, 14400, 128, 128),
+               (48, 8256, 8320, 128), (16, 64, 128, 128), (16, 64, 8320, 128), (16, 4160, 128, 128), (48, 576, 8320, 128),
+               (16, 8256, 1152, 128), (32, 2112, 1152, 128), (32, 4160, 1152, 128), (32, 14400, 128, 128), (48, 3008, 1152, 128),
+               (256, 1088, 640, 128), (144, 576, 8320, 128), (48, 8256, 640, 128), (128, 1088, 8320, 128), (64, 8256, 640, 128),
+               (512, 1088, 640, 128), (80, 320, 1152, 384), (32, 192, 2048, 2048)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,gs", WAVE_NK)
+def test_w4a16_nk_wave_kernel(dev, dtype, M, N, K, gs):
+    """Small integers and power-of-two scales: every sum is exact in fp32, so the result is the rounded product; then an
+    infinite activation reaches its own row only (fp16)."""
+    announce("w4a16 nk wave kernel", dtype, M, N, K, gs)
+    torch.manual_seed(M + N + K)
+    g_ = K if gs == -1 else gs
+    x = torch.randint(-2, 3, (M, K), device=dev).to(dtype)
+    qn = torch.randint(0, 16, (N, K), dtype=torch.uint8)
+    s = torch.exp2(torch.randint(-4, 1, (N, K // g_)).float()).half().to(dev)
+    packed = torch.from_numpy(bp.pack_cols(qn.numpy(), 4, 32)[0]).to(dev)
+    w = ((qn.to(dev).double() - 8) * s.double().repeat_interleave(g_, 1)).T.contiguous()
+    assert torch.equal(w4a16.w4a16_gemm(x, packed, s, gs), (x.double() @ w).to(dtype))
+    if dtype == torch.float16:
+        x[1, K - 1] = float("inf")
+        y, ref = w4a16.w4a16_gemm(x, packed, s, gs), (x.double() @ w).to(dtype)
+        assert torch.equal(y[:1], ref[:1]) and torch.equal(y[2:], ref[2:]) and torch.equal(y[1].isfinite(), ref[1].isfinite())
+
+
+@pytest.mark.parametrize("M,N,K,gs", WAVE_MARLIN)
+@pytest.mark.parametrize("scratch", [True, False])
+def test_mul_wave_kernel(dev, M, N, K, gs, scratch):
+    """The same on Marlin words, with the scratch that is reported and without any."""
+    announce("marlin wave kernel", M, N, K, gs, scratch)
+    torch.manual_seed(M + N + K)
+    A = torch.randint(-2, 3, (M, K), device=dev).half()
+    qw = torch.randint(0, 16, (K, N), dtype=torch.int32, device=dev)
+    s = torch.exp2(torch.randint(-4, 1, (K // gs, N), device=dev).float()).half()
+    B, sp = QuantUtils.pack(qw, s, gs)
+    C = torch.full((M, N), 7.0, dtype=torch.half, device=dev)
+    nbytes = _lib.load().llmk_gemm_w4a16_marlin_workspace_bytes(M, N, K) if scratch else 0
+    ws = torch.full((nbytes + 256,), 0x5A, dtype=torch.uint8, device=dev)
+    _lib.call("llmk_gemm_w4a16_marlin", _lib.ptr(A), _lib.ptr(B), _lib.ptr(C), _lib.ptr(sp), M, N, K, gs, _lib.ptr(ws) if nbytes else None, nbytes,
+              _lib.stream(A))
+    ref = A.double() @ ((qw.double() - 8) * s.double().repeat_interleave(gs, 0))
+    assert torch.equal(C, ref.half())
+    assert (ws[nbytes:] == 0x5A).all()
+
+
 @pytest.mark.parametrize("M,N,K,gs", [(65, 72, 128, 64), (130, 4096, 1024, 128), (512, 264, 4096, 128), (300, 14344, 512, 128),
                                       (200, 20000, 640, 128), (500, 8192, 384, 192), (600, 10000, 1024, 128), (1024, 28672, 256, 128)])
 def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
