@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "gemm_wave.hpp"
 #include "gemm_wide.hpp"
 
 using namespace llmk;
@@ -18,32 +19,55 @@ int check_common(const char* name, const void* a, const void* b, int64_t M, int6
     return LLMK_OK;
 }
 
-// Decode-sized M with K beyond one resident batch per wave (32 steps): the weight-streaming kernel runs on
-// K ranges of at most 32 steps side by side (gridDim.z) and a second kernel adds their fp32 partial sums.
+// K ranges of decode-sized calls with long K: the planes of fp32 sums that their scratch is sized for.
 inline int stream_k_ranges(int64_t M, int64_t N, int64_t K) {
     if (M > 64 || K <= 4096 || mid_m_prefers_tiles(M, N, K)) return 1;
     return (int)((K / 128 + 31) / 32);
 }
 
+// What the tile kernels take for 17 to 512 rows, in us like the wave kernels' estimates (a fit of 5 to 15 % rms to 600 shapes): the
+// mid-size kernels with 64 and 128 columns, the 128-column tile in K slices, or rounds of the tiles that dma_tile_estimate chooses.
+// Up to 16 rows, and up to 64 on weights that no tile kernel fills the chip with or without scratch for their K slices, the wave
+// kernels have no rival.
 template <int KIND>
-int launch_stream(DirectArgs& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, const char* name) {
-    const int nz = stream_k_ranges(p.M, p.N, p.K);
-    const int64_t mn = (int64_t)p.M * p.N;
-    if (nz > 1 && workspace && workspace_bytes >= nz * mn * 4) {
-        const int steps = p.K / 128;
-        p.kc_steps = ((steps + nz - 1) / nz + 3) & ~3;         // even ranges, whole 4-step groups
-        p.partial = (float*)workspace;
-        p.ksplit = (steps + p.kc_steps - 1) / p.kc_steps;
-        int rc = launch_direct<KIND, false>(p, p.M, stream, name);
-        if (rc) return rc;
-        const unsigned blocks = (unsigned)((mn + 1023) / 1024);
-        if (p.c_dtype == LLMK_BF16) splitk_sum_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, p.ksplit);
-        else if (p.c_dtype == LLMK_F16) splitk_sum_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, p.ksplit);
-        else splitk_sum_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, p.ksplit);
-        LLMK_CHECK_LAUNCH(name);
-        return LLMK_OK;
+double tiles_estimate(const DirectArgs& p, bool scratch) {
+    const int64_t M = p.M, N = p.N, K = p.K;
+    const double k = (double)K / 4096.0;
+    if (M <= 16 || (M <= 64 && (!scratch || !(mid_m_prefers_tiles(M, N, K) || mid_wanted(M, N, K))))) return 1e30;
+    if (mid_wanted(M, N, K)) {
+        const MidPlan pl = mid_plan(M, N, K);
+        return (pl.mt == 2 ? 3.2 + 7.4 * k / pl.z : 4.0 + 7.2 * k / pl.z) + (pl.z > 1 ? 2.9 : 0.0);
     }
-    return launch_direct<KIND, false>(p, p.M, stream, name);
+    if (KIND == K_FP8_BLOCK && midw_wanted(M, N, K)) {
+        const MidPlan pl = midw_plan(M, N, K);
+        return (pl.mt == 4 ? 5.3 + 11.9 * k / pl.z : 6.7 + 19.2 * k / pl.z) + (pl.z > 1 ? 3.5 : 0.0);
+    }
+    const int z = splitk_factor(M, N, K);
+    if (z > 1) return 3.5 + 29.0 * k / z;
+    const TileChoice c = dma_tile_estimate<KIND, false>(p);
+    const double e = c.cost * k * (KIND == K_I8_BLOCK ? 1.12 : 1.0);
+    return c.choice == 1 ? 3.4 + 0.87 * e : (c.choice == 2 ? 5.0 + 0.7 * e : (c.choice == 8 ? 9.0 + 0.85 * e : 7.5 + 0.8 * e));
+}
+// The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels.  Over 550
+// random shapes of N 1024 to 28672 and K 1024 to 14336, against the kernels before: 1.34 to 1.48 times as fast at 1 to 16 rows, 1.26
+// to 1.50 at 17 to 64, 1.07 (fp8), 1.14 (int8) and 1.23 (per token) at 65 to 512; one in forty of them lost 5 to 10 %.  us, wave | tiles:
+// int8 29 x 4096 x 4096 5.1 | 8.5, fp8 64 x 4096 x 4096 6.2 | 9.4, fp8 200 x 1032 x 7168 7.6 | 15.1, per token 250 x 4096 x 14336 25.1 |
+// 28.1, but fp8 250 x 4096 x 14336 30.6 | 29.2, and from 513 rows on 0.8 times as fast.
+template <int KIND>
+WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspace_bytes) {
+    WavePlan w{0, 0, 0, 0, 0.0};
+    const int64_t scratch = workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0;
+    if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w) ||
+        1.08 * w.cost >= tiles_estimate<KIND>(p, workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K)))
+        w.nw = 0;
+    return w;
+}
+template <int KIND>
+int launch_block(const DirectArgs& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, const char* name) {
+    const WavePlan w = wave_choice<KIND>(p, workspace, workspace_bytes);
+    if (w.nw) return launch_w8_wave_plan<KIND>(p, w, workspace, stream, name);
+    if (p.K == 0) return launch_empty_sums<false>(p, stream, name);
+    return launch_big<KIND, false>(p, workspace, workspace_bytes, stream, name);
 }
 
 }  // namespace
@@ -79,9 +103,7 @@ extern "C" int llmk_gemm_fp8_block(const void* a, const float* a_s, const void* 
     DirectArgs p{};
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = LLMK_F32; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
-    if (M > 64 || ((mid_m_prefers_tiles(M, N, K) || mid_wanted(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K)))
-        return launch_big<K_FP8_BLOCK, false>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_fp8_block(tiled)");
-    return launch_stream<K_FP8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_fp8_block");
+    return launch_block<K_FP8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_fp8_block");
 }
 
 // llmk_gemm_fp8_block for the benchmark's calibration: the same launch, and workgroup 0 of the 256-column tile kernel
@@ -110,9 +132,7 @@ extern "C" int llmk_gemm_i8_block(const int8_t* a, const void* a_s, const int8_t
     DirectArgs p{};
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = s_dtype; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
-    if (M > 64 || ((mid_m_prefers_tiles(M, N, K) || mid_wanted(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K)))
-        return launch_big<K_I8_BLOCK, false>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_i8_block(tiled)");
-    return launch_stream<K_I8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_i8_block");
+    return launch_block<K_I8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_i8_block");
 }
 
 extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, const float* b_s, void* c,
@@ -126,9 +146,9 @@ extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8
     DirectArgs p{};
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.c_i32 = c_i32; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = LLMK_F32; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
+    const WavePlan wave = wave_choice<K_I8_ROWCOL>(p, workspace, workspace_bytes);
+    if (wave.nw) return launch_w8_wave_plan<K_I8_ROWCOL>(p, wave, workspace, (hipStream_t)stream, "gemm_i8_rowcol(wave)");
     // large M: the tile kernels accumulate int32 over the whole K range inside the MFMA and scale in the epilogue
-    // (from the rows that the mid-size kernel takes, and from 17 rows on large weights as for the block-scaled kinds: 64 x 4096
-    // x 14336 44.4 us on the weight-streaming kernel, 30.0 in K slices, 64 x 28672 x 4096 76.4 and 35.3)
     if ((M > 64 || ((mid_wanted(M, N, K) || mid_m_prefers_tiles(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K))) &&
         dma_eligible(p)) {
         // few tiles and a long K: K slices over the CUs, int32 partial sums in the workspace, one pass that adds
@@ -154,7 +174,7 @@ extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8
 
 // ------------------------------------------------------------------ llmk_gemm_fp8_block without a scratch argument
 // For callers that cannot allocate device memory (HIP graph capture, serving loops, harnesses that forbid
-// hipMalloc): the fp32 partial sums of the split-K / K-range kernels live in a file-scope device array instead
+// hipMalloc): the fp32 partial sums of the split-K kernels live in a file-scope device array instead
 // of a caller-provided buffer.  Every GPU the library runs on holds its own copy of the array until the
 // process ends; its address on a device is looked up once, with that device current, and only that address
 // (never the array's name, which is a host-side stand-in) is handed to kernels.

@@ -6,8 +6,9 @@
 // reduce through LDS.  This is the shape that wins when M is small and the GEMM is bound by
 // streaming B from HBM; for large M the LDS-tiled kernels take over.
 //
-// The same kernel serves the grouped (per-expert segment) GEMM: a tile then first locates its
-// segment from seg_indptr.
+// It serves the grouped (per-expert segment) GEMM, where a tile first locates its segment from
+// seg_indptr, and per-token int8 products that no other kernel's 32-bit offsets reach; the dense
+// products run on the wave kernels (gemm_wave.hpp).
 #pragma once
 #include "common.hpp"
 
@@ -123,7 +124,6 @@ struct DirectArgs {
     int M, N, K, E;
     float* partial;        // split-K: fp32 [ksplit][M][N] partial sums
     int ksplit;            // 0 / 1 = no split
-    int kc_steps;          // weight-streaming kernel with K ranges: 128-byte steps per range (gridDim.z ranges)
     int group;             // K_W4NK / K_W4MARLIN: K elements per fp16 group scale
     long long* clocks;     // 256-column tile kernel, calibration only: workgroup 0 leaves the s_memtime and s_memrealtime ticks it lived
     const int8_t* w4_s4;   // uint4 weights with two-level scales: second-level scales [N, K/128]
@@ -192,14 +192,11 @@ inline int grouped_row_tiles(int M, int E, int tile_rows) {
 // SDT: dtype code of the block scales, fixed at compile time so that a scale load is a plain typed load with
 // no branch (and hence no wait for memory) between it and the loads around it.
 // VEC: the weight scales of a batch are one vector load (needs four steps per batch and steps % 4 == 0).
-// KR: blockIdx.z selects a K range of p.kc_steps steps (short enough for RESIDENT); the workgroup writes its
-// fp32 sums to p.partial[blockIdx.z] and a second kernel adds the ranges.
-// SU: K steps per wave and batch where K is short (1 to 3), 0: the number that goes with MT.  (16 rows, us per layer, four
+// SU: K steps per wave and batch where K is short (1 to 3), 0: the number that goes with MT.  (16 rows of a dense product, us, four
 // steps against as many as needed: fp8 28672 x 1024 22.9 -> 12.2, 25728 x 1408 23.3 -> 16.1, 28672 x 2048 24.2 -> 18.1, 24000
 // x 2304 22.2 -> 19.4, 4096 x 1024 9.2 -> 6.3; per-token int8 28672 x 1024 23.7 -> 12.7.)
-template <int KIND, int MT, int NW, bool GROUPED, bool RESIDENT, int SDT, bool VEC = false, bool KR = false, int SU = 0>
+template <int KIND, int MT, int NW, bool GROUPED, bool RESIDENT, int SDT, bool VEC = false, int SU = 0>
 __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
-    static_assert(!KR || (RESIDENT && !GROUPED && !VEC), "K ranges: dense, resident activations");
     typedef typename ScaleIO<SDT>::Raw SRaw;
     constexpr bool HALF = (KIND == K_F16 || KIND == K_BF16);
     constexpr int ESZ = HALF ? 2 : 1;
@@ -211,9 +208,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: K-step indices stay scalar
     const int r = lane & 15, g = lane >> 4;
     const int K = p.K, N = p.N;
-    const int steps_all = K / KSTEP;                         // row length of the scale tables
-    const int kz0 = KR ? (int)blockIdx.z * p.kc_steps : 0;   // first step of this workgroup's K range
-    const int steps = KR ? min(p.kc_steps, steps_all - kz0) : steps_all;
+    const int steps = K / KSTEP;              // also the row length of the scale tables
 
     int m_start, m_end;
     const uint8_t* bbase = p.b;
@@ -235,9 +230,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int arow = min(m_start + 16 * mt + r, m_end - 1);
-        ap[mt] = p.a + ((int64_t)arow * K) * ESZ + 16 * g + (int64_t)kz0 * 128;
+        ap[mt] = p.a + ((int64_t)arow * K) * ESZ + 16 * g;
     }
-    if constexpr (KR) bbase += (int64_t)kz0 * 128;
 
     // A batch is U K-steps of this wave; all its loads are issued before any of them is consumed.  Steps
     // past the end are clamped to the last step and nullified.  When the whole K range of a wave fits in
@@ -262,7 +256,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
     auto load_b = [&](BBatch& t, int tile, int ks0) {
         const int nrow = min(tile * 16 + r, N - 1);
         const uint8_t* bp = bbase + ((int64_t)nrow * K) * ESZ + 16 * g;
-        const int64_t bs_row = bs_off + (int64_t)(tile * 16 / 128) * steps_all + kz0;
+        const int64_t bs_row = bs_off + (int64_t)(tile * 16 / 128) * steps;
         // all data loads first, then the scales as raw bits: nothing in here waits for memory
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -318,12 +312,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
         for (int q = 0; q < 4; ++q) {
             const int idx = (int)threadIdx.x + q * NW * 64;
             stage_as[q] = 0;
-            if constexpr (KR) {       // the rows of a K range are not contiguous in a_s
-                const int row = idx / steps, k = idx - row * steps;
-                if (idx < n_as) stage_as[q] = ((const SRaw*)p.a_s)[(int64_t)min(m_start + row, m_end - 1) * steps_all + kz0 + k];
-            } else {
-                if (idx < n_as) stage_as[q] = ((const SRaw*)p.a_s)[as_base + min(idx, n_as_valid - 1)];
-            }
+            if (idx < n_as) stage_as[q] = ((const SRaw*)p.a_s)[as_base + min(idx, n_as_valid - 1)];
         }
     }
     if (steps > 0 && tile < ntiles) {
@@ -441,8 +430,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectArgs p) {
                 float sum = 0.f;
 #pragma unroll
                 for (int w = 0; w < NW; ++w) sum += rbuf[w * MT * 256 + src];
-                if constexpr (KR) p.partial[((int64_t)blockIdx.z * p.M + m) * N + n] = sum;
-                else st_out(p.c, (int64_t)m * N + n, sum, p.c_dtype);
+                st_out(p.c, (int64_t)m * N + n, sum, p.c_dtype);
             }
         }
         if constexpr (RB == 1) __syncthreads();
@@ -505,33 +493,6 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
     const int ntiles = (p.N + 15) / 16;
     const int mtiles = GROUPED ? grouped_row_tiles(p.M, p.E, 16 * MT) : (p.M + 16 * MT - 1) / (16 * MT);
     if (ntiles == 0 || mtiles == 0) return LLMK_OK;
-    if constexpr (SCALED && !GROUPED && MT == 1) {
-        if (p.kc_steps > 0) {
-            // K ranges: every range fits one resident batch per wave; the caller adds the fp32 partial sums
-            if (p.kc_steps > NW * U || !p.partial) LLMK_FAIL(LLMK_ERR_ARG, "%s: bad K range setup", name);
-            const int nz = (steps + p.kc_steps - 1) / p.kc_steps;
-            const size_t smem_r = (size_t)2 * NW * 256 * sizeof(float) + (size_t)16 * p.kc_steps * sizeof(float);
-            static std::atomic<int> slots_r_cache{0};     // same value on every MI355X; recomputing it is harmless
-            int slots_r = slots_r_cache.load(std::memory_order_relaxed);
-            if (slots_r == 0) {
-                int dev = 0, cus = 0, per_cu = 0;
-                hipError_t e = hipGetDevice(&dev);
-                if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-                if (e == hipSuccess)
-                    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, 1, NW, false, true, SDT, false, true>, NW * 64, smem_r);
-                if (e != hipSuccess) LLMK_FAIL(LLMK_ERR_LAUNCH, "%s: occupancy query failed: %s", name, hipGetErrorString(e));
-                slots_r = max(1, cus * max(1, per_cu));
-                slots_r_cache.store(slots_r, std::memory_order_relaxed);
-            }
-            const int rows = mtiles * nz;
-            int gx = min(ntiles, max(1, slots_r / min(rows, slots_r)));
-            { const int per_wg = (ntiles + gx - 1) / gx; gx = (ntiles + per_wg - 1) / per_wg; }
-            gemm_direct_kernel<KIND, 1, NW, false, true, SDT, false, true>
-                <<<dim3((unsigned)gx, (unsigned)mtiles, (unsigned)nz), dim3(NW * 64), smem_r, stream>>>(p);
-            LLMK_CHECK_LAUNCH(name);
-            return LLMK_OK;
-        }
-    }
     const size_t smem = (size_t)(MT == 4 ? 1 : 2) * NW * MT * 256 * sizeof(float) + (SCALED ? (size_t)MT * 16 * steps * sizeof(float) : 0);
     if (smem > 64 * 1024) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: K=%d too large for the weight-streaming kernel's scale table", name, p.K);
     // Column tiles are processed persistently by as many workgroups as are resident at once (so that every
@@ -551,9 +512,9 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
         hipError_t e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess)
-            e = variant == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1>, NW * 64, 64 * 1024)
-                : variant == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2>, NW * 64, 64 * 1024)
-                : variant == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3>, NW * 64, 64 * 1024)
+            e = variant == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, SU1>, NW * 64, 64 * 1024)
+                : variant == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, SU2>, NW * 64, 64 * 1024)
+                : variant == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, SU3>, NW * 64, 64 * 1024)
                 : resident ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT>, NW * 64, 64 * 1024)
                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT>, NW * 64, 64 * 1024);
         if (e != hipSuccess) LLMK_FAIL(LLMK_ERR_LAUNCH, "%s: occupancy query failed: %s", name, hipGetErrorString(e));
@@ -572,9 +533,9 @@ int launch_direct_sdt(const DirectArgs& p, hipStream_t stream, const char* name)
             return LLMK_OK;
         }
     }
-    if (variant == 2) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU1><<<grid, block, smem, stream>>>(p);
-    else if (variant == 3) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU2><<<grid, block, smem, stream>>>(p);
-    else if (variant == 4) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, false, SU3><<<grid, block, smem, stream>>>(p);
+    if (variant == 2) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, SU1><<<grid, block, smem, stream>>>(p);
+    else if (variant == 3) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, SU2><<<grid, block, smem, stream>>>(p);
+    else if (variant == 4) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT, false, SU3><<<grid, block, smem, stream>>>(p);
     else if (resident) gemm_direct_kernel<KIND, MT, NW, GROUPED, true, SDT><<<grid, block, smem, stream>>>(p);
     else gemm_direct_kernel<KIND, MT, NW, GROUPED, false, SDT><<<grid, block, smem, stream>>>(p);
     LLMK_CHECK_LAUNCH(name);
@@ -608,18 +569,21 @@ __global__ void empty_sums_kernel(DirectArgs p) {
     }
 }
 
+template <bool GROUPED>
+int launch_empty_sums(const DirectArgs& p, hipStream_t stream, const char* name) {
+    empty_sums_kernel<GROUPED><<<1024, 256, 0, stream>>>(p);
+    LLMK_CHECK_LAUNCH(name);
+    return LLMK_OK;
+}
+
 template <int KIND, bool GROUPED>
 int launch_direct(const DirectArgs& p, int max_rows_per_segment_hint, hipStream_t stream, const char* name) {
-    if (p.K == 0) {
-        empty_sums_kernel<GROUPED><<<1024, 256, 0, stream>>>(p);
-        LLMK_CHECK_LAUNCH(name);
-        return LLMK_OK;
-    }
+    if (p.K == 0) return launch_empty_sums<GROUPED>(p, stream, name);
     // m-tiles per workgroup: 1 for decode-sized M, up to 4 otherwise.  When a wave's K share fits one batch at
     // one m-tile per workgroup (activations resident in registers), 16-row workgroups side by side beat taller
     // ones that have to re-read their activations for every column tile.
     constexpr int KSTEP = (KIND == K_F16 || KIND == K_BF16) ? 64 : 128;
-    if (max_rows_per_segment_hint <= 16 || p.K / KSTEP <= 32 || p.kc_steps > 0) return launch_direct_mt<KIND, 1, GROUPED>(p, stream, name);
+    if (max_rows_per_segment_hint <= 16 || p.K / KSTEP <= 32) return launch_direct_mt<KIND, 1, GROUPED>(p, stream, name);
     if (max_rows_per_segment_hint <= 32) return launch_direct_mt<KIND, 2, GROUPED>(p, stream, name);
     return launch_direct_mt<KIND, 4, GROUPED>(p, stream, name);
 }

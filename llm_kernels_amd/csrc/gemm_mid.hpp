@@ -1,5 +1,5 @@
 // Tile kernels for mid-size M (about 65 to 512 rows) on few column tiles: problems that neither fill the chip with
-// 128- or 256-column tiles nor fit the weight-streaming kernels, and whose weights mostly come cold from HBM.
+// 128- or 256-column tiles nor run on the wave kernels, and whose weights mostly come cold from HBM.
 //
 // What bounds the 64 x 128 tile of gemm_dma.hpp there is the per-step overhead: one barrier, twelve fragment reads
 // and a dependent wait per wave for four matrix instructions on 128 bytes of K.  Here a K step is 512 bytes = four

@@ -64,7 +64,8 @@ __device__ __forceinline__ void wv_wait_loads() { asm volatile("s_waitcnt vmcnt(
 
 // The end of a tile, behind the barrier that follows the waves' writes: red [wave][row][column], rows of 16 NT + 4 floats, is
 // summed over the waves in their order and stored (K slices: as fp32 sums).  A thread owns eight columns of a row.
-template <int NW, int MT, int NT>
+// ROWCOL: int32 sums, scaled per row and column here.
+template <int NW, int MT, int NT, bool ROWCOL = false>
 __device__ __forceinline__ void wv_store(const DirectArgs& p, const float* red, int n0, int m0, int m_end) {
     constexpr int BM = 16 * MT, BN = 16 * NT, RED_ROW = BN + 4, RUNS = BN / 8, ROWS_PASS = (NW * 64) / RUNS;
     const int tid = threadIdx.x, N = p.N;
@@ -80,13 +81,25 @@ __device__ __forceinline__ void wv_store(const DirectArgs& p, const float* red, 
         const int orow = pass * ROWS_PASS + tid / RUNS, m = m0 + orow;
         if (orow >= BM || m >= m_end) continue;
         v4f sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+        v4i ia = {0, 0, 0, 0}, ib = {0, 0, 0, 0};
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
             const float* src = red + (w * BM + orow) * RED_ROW + ocol;
-            sa += *(const v4f*)src;
-            sb += *(const v4f*)(src + 4);
+            if constexpr (ROWCOL) {
+                ia += *(const v4i*)src;
+                ib += *(const v4i*)(src + 4);
+            } else {
+                sa += *(const v4f*)src;
+                sb += *(const v4f*)(src + 4);
+            }
         }
         const int64_t off = (int64_t)m * N + nn;
+        if constexpr (ROWCOL) {
+            sa = __builtin_bit_cast(v4f, ia);
+            sb = __builtin_bit_cast(v4f, ib);
+            rowcol_epilogue8(p, sa, sb, m, off, nn, nv);
+            if (!p.c) continue;
+        }
         if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv, vec_ok);
         else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv, vec_ok);
         else store_run8<LLMK_F32>(cout, off, sa, sb, nv, vec_ok);
@@ -694,6 +707,189 @@ int launch_w4a16_wave(const DirectArgs& p, int z, hipStream_t stream, const char
     return LLMK_OK;
 }
 
+// ------------------------------------------------------------------------------------------------------------
+// 8-bit operands [M, K] and [N, K]: fp8 or int8 with a scale per row and 128 elements and per 128 x 128 weight block (K_FP8_BLOCK,
+// K_I8_BLOCK), or int8 with a scale per row and per column (K_I8_ROWCOL: int32 sums, scaled at the end).  S32 as above.
+// What it replaces at 1 to 16 rows kept activations in registers and walked column tiles with one barrier each; its fragment
+// loads (16 rows x 64 bytes an instruction) cost the address path four times what coalesced ones to LDS do.  Bound by weights
+// from L2 or HBM up to 16 rows (warm 28672 x 4096 6.0 TB/s, cold 3.6), by the address path and the latency of one stage from there.
+// us per launch, before | now, weights in the memory-side cache: fp8 4 x 4096 x 14336 15.3 | 11.1, 9 x 14336 x 4096 14.2 | 11.3, 12 x
+// 28672 x 4096 23.0 | 20.4, 16 x 4096 x 4096 6.7 | 4.5, int8 15 x 6144 x 4096 8.7 | 5.1, per token 9 x 3128 x 9472 11.2 | 5.4; weights
+// from HBM, fp8: 16 x 4096 x 4096 8.7 | 7.8, 16 x 14336 x 4096 18.7 | 18.2, 16 x 28672 x 4096 32.2 | 32.5, 16 x 4096 x 14336 20.4 | 19.3.
+constexpr int w8_stage(int mt, int nt) { return (16 * mt + 16 * nt) * 128 + 256; }
+constexpr int w8_lds(int nw, int mt, int nt, int d, int steps) {
+    const int a = nw * d * w8_stage(mt, nt) + 4 * steps, b = wv_red(nw, mt, nt);
+    return a > b ? a : b;
+}
+
+template <int KIND, int NW, int MT, int NT, int D, bool S32>
+__global__ __launch_bounds__(NW * 64) void w8_wave_kernel(DirectArgs p) {
+    constexpr bool SCALED = (KIND != K_I8_ROWCOL);
+    static_assert(KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL, "8-bit operands");
+    constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = w8_stage(MT, NT), LPS = 2 * MT + 2 * NT + (SCALED ? 1 : 0);
+    constexpr int OFF_B = BM * 128, OFF_S = OFF_B + BN * 128;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int N = p.N, K = p.K, KT_all = K >> 7;
+    int kt0 = 0, KT = KT_all;
+    if constexpr (SCALED) {
+        if (p.ksplit > 1) {
+            const int per = (KT_all + p.ksplit - 1) / p.ksplit;
+            kt0 = (int)blockIdx.z * per;
+            KT = min(per, KT_all - kt0);
+        }
+    }
+    const WaveTile tile = wave_tile(p.M, BM);
+    const int n0 = tile.col * BN, m0 = tile.row * BM, m_end = min(p.M, m0 + BM);
+    const int s_lo = wave * KT / NW, n = (wave + 1) * KT / NW - s_lo;
+    uint8_t* const mine = lds + wave * (D * STAGE);
+    const uint32_t mine_addr = lds_base + (uint32_t)wave * (D * STAGE);
+    float* const bsl = (float*)(lds + NW * D * STAGE);       // block scale of the tile's columns per K step
+
+    const bool s_f16 = p.s_dtype == LLMK_F16;
+    auto scale_f32 = [&](unsigned raw) { return S32 ? __uint_as_float(raw) : (s_f16 ? f16_to_f32((unsigned short)raw) : bf16_to_f32((unsigned short)raw)); };
+    constexpr uint32_t ssz = S32 ? 4u : 2u;
+    int t_bs = 0;
+    if constexpr (SCALED) {
+        const RingBase bsb = ring_base((const uint8_t*)p.b_s + ((int64_t)(n0 >> 7) * KT_all + kt0) * ssz);
+        const uint32_t bat = (uint32_t)min(tid, KT - 1) * ssz;
+        if constexpr (S32) t_bs = ring_load_b32<0>(bat, bsb);
+        else t_bs = ring_load_u16<0>(bat, bsb);
+    }
+
+    // ---- source offsets of the loads of a stage; 16-byte chunks swizzled within a row as in the tile kernels
+    uint32_t aoff[2 * MT], boff[2 * NT];
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        aoff[i] = (uint32_t)min(row, m_end - 1 - m0) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        boff[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    }
+    const uint32_t soff = (uint32_t)min(min(lane, BM - 1), m_end - 1 - m0) * (uint32_t)KT_all * ssz;
+    const uint8_t* const ga = p.a + (int64_t)m0 * K;
+    const uint8_t* const gb = p.b + (int64_t)n0 * K;
+    const uint8_t* const gs = (const uint8_t*)p.a_s + (int64_t)m0 * KT_all * ssz;
+    auto issue = [&](int slot, int s) __attribute__((always_inline)) {
+        const int kb = kt0 + min(s, KT - 1);
+        const uint32_t st = mine_addr + (uint32_t)slot * STAGE;
+#pragma unroll
+        for (int i = 0; i < 2 * NT; ++i) dma16(st + OFF_B + i * 1024u, boff[i], gb + (int64_t)kb * 128);
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) dma16(st + i * 1024u, aoff[i], ga + (int64_t)kb * 128);
+        if constexpr (SCALED) {
+            if constexpr (S32) dma4(st + OFF_S, soff, gs + (int64_t)kb * 4);
+            else dma2(st + OFF_S, soff, gs + (int64_t)kb * 2);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) issue(d, s_lo + d);
+    if constexpr (SCALED) {
+        ring_wait<D * LPS>(t_bs);
+        if (tid < KT) bsl[tid] = scale_f32((unsigned)t_bs);
+        for (int k = tid + NW * 64; k < KT; k += NW * 64) bsl[k] = ld_scale(p.b_s, (int64_t)(n0 >> 7) * KT_all + kt0 + k, p.s_dtype);
+        __syncthreads();
+    }
+
+    // acc[mt][j][i] = C[row 16 mt + r][column 16 j + 4 g + i] over this wave's K steps (K_I8_ROWCOL: int32 bits)
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+    const int swz = (r >> 1) & 7;
+    const int lo = r * 128 + ((g ^ swz) * 16), hi = r * 128 + (((g + 4) ^ swz) * 16);
+    auto ldfrag = [&](const uint8_t* base) {
+        const v4i x = *(const v4i*)(base + lo), y = *(const v4i*)(base + hi);
+        return (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    };
+    v8i af[MT], bf[NT];
+    unsigned a_sc[MT];
+    auto fetch = [&](int slot) __attribute__((always_inline)) {
+        const uint8_t* st = mine + slot * STAGE;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) bf[j] = ldfrag(st + OFF_B + j * 2048);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            af[mt] = ldfrag(st + mt * 2048);
+            if constexpr (SCALED) a_sc[mt] = *(const unsigned*)(st + OFF_S + (16 * mt + r) * 4);
+        }
+    };
+    auto compute = [&](int s) __attribute__((always_inline)) {
+        if constexpr (SCALED) {
+            const float bs = bsl[s];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const float sa = scale_f32(a_sc[mt]) * bs;
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const v4f t = raw_f32<KIND>(step_raw<KIND>(bf[j], af[mt]));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[mt][j][i] = fmaf(t[i], sa, acc[mt][j][i]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[mt][j] = mma_plain<KIND>(bf[j], af[mt], acc[mt][j]);
+        }
+    };
+
+    int i = 0, slot = 0;
+    for (; i + D < n; ++i) {
+        wv_wait_loads<(D - 1) * LPS>();
+        fetch(slot);
+        __builtin_amdgcn_s_waitcnt(0xc07f);                  // lgkmcnt(0): the slot is free
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        issue(slot, s_lo + i + D);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s_lo + i);
+        slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    md_static_for<0, D>([&](auto dc) __attribute__((always_inline)) {
+        constexpr int d = decltype(dc)::value;
+        if (i < n) {
+            wv_wait_loads<(D - 1 - d) * LPS>();
+            fetch(slot);
+            compute(s_lo + i);
+            slot = slot + 1 == D ? 0 : slot + 1;
+            ++i;
+        }
+    });
+    wv_wait_loads<0>();
+    __syncthreads();
+
+    float* red = (float*)lds;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) *(v4f*)(red + (wave * BM + 16 * mt + r) * (BN + 4) + 16 * j + 4 * g) = acc[mt][j];
+    __syncthreads();
+    wv_store<NW, MT, NT, KIND == K_I8_ROWCOL>(p, red, n0, m0, m_end);
+}
+
+template <int KIND, int NW, int MT, int NT, int D, bool S32>
+int launch_w8_wave(const DirectArgs& p, hipStream_t stream, const char* name) {
+    static std::atomic<uint64_t> configured{0};
+    auto kern = w8_wave_kernel<KIND, NW, MT, NT, D, S32>;
+    const int z = p.ksplit > 1 ? p.ksplit : 1;
+    const int bytes = w8_lds(NW, MT, NT, D, ((p.K >> 7) + z - 1) / z);
+    if (bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, bytes);
+    if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
+    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
+    kern<<<dim3(tiles, 1, (unsigned)z), NW * 64, bytes, stream>>>(p);
+    LLMK_CHECK_LAUNCH(name);
+    return z > 1 ? wv_sum_slices(p, z, stream, name) : LLMK_OK;
+}
+
 // Launch shape: waves per workgroup, row and column tiles of a wave, K slices over workgroups, estimated microseconds.
 struct WavePlan {
     int nw, mt, nt, z;
@@ -769,6 +965,84 @@ inline bool wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, const Wa
     }
     return found;
 }
+// 8-bit operands: an estimate of at least the weights at 6.1 TB/s, and K slices (a second launch and a write and a read of the
+// planes) only of block-scaled operands beyond 128 K steps, where few columns leave the chip idle: below they never won (fp8, us, whole
+// | sliced: 16 x 1024 x 32768 17.1 | 10.0, 20 x 136 x 65664 21.2 | 7.6).
+constexpr WaveModel WV_FP8 = {{{2.97f, 2.81f, 1.50f}, {2.68f, 2.71f, 1.46f}, {0.f, 1.67f, 1.34f}, {0.f, 1.56f, 1.38f}},
+                              {{0.00f, 0.00f, 1.10f}, {0.00f, 0.00f, 1.16f}, {0.f, 0.96f, 1.48f}, {0.f, 0.84f, 1.76f}},
+                              {{0.34f, 0.53f, 0.93f}, {0.55f, 0.85f, 1.21f}, {0.f, 1.04f, 1.46f}, {0.f, 1.31f, 1.73f}},
+                              {0.f, 3.66f, 5.20f, 4.97f}, {0.f, 0.57f, 0.72f, 0.88f}};
+constexpr WaveModel WV_I8 = {{{2.95f, 2.89f, 1.54f}, {3.03f, 2.96f, 1.47f}, {0.f, 1.84f, 1.44f}, {0.f, 1.81f, 1.28f}},
+                             {{0.03f, 0.03f, 1.30f}, {0.00f, 0.01f, 1.57f}, {0.f, 1.20f, 1.99f}, {0.f, 1.37f, 2.53f}},
+                             {{0.34f, 0.50f, 0.87f}, {0.51f, 0.73f, 1.13f}, {0.f, 0.97f, 1.39f}, {0.f, 1.19f, 1.63f}},
+                             {0.f, 3.73f, 5.00f, 4.60f}, {0.f, 0.56f, 0.73f, 0.88f}};
+constexpr WaveModel WV_I8_ROWCOL = {{{2.86f, 2.76f, 1.56f}, {2.90f, 2.76f, 1.28f}, {0.f, 1.65f, 1.10f}, {0.f, 1.55f, 0.95f}},
+                                    {{0.00f, 0.08f, 1.26f}, {0.06f, 0.12f, 1.83f}, {0.f, 1.39f, 2.46f}, {0.f, 1.54f, 3.11f}},
+                                    {{0.32f, 0.47f, 0.83f}, {0.45f, 0.65f, 1.02f}, {0.f, 0.80f, 1.20f}, {0.f, 0.96f, 1.38f}},
+                                    {0.f, 3.20f, 5.00f, 4.05f}, {0.f, 0.54f, 0.67f, 0.79f}};
+constexpr int w8_depth(int mt, int nt, int steps) { return mt == 1 && nt == 1 && steps >= 64 ? 2 : 1; }
+template <int KIND>
+inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
+    constexpr const WaveModel& m = KIND == K_FP8_BLOCK ? WV_FP8 : (KIND == K_I8_BLOCK ? WV_I8 : WV_I8_ROWCOL);
+    if (K < 128 || K > (1 << 22)) return false;
+    const int KT_all = (int)(K >> 7);
+    const int zmax = KIND == K_I8_ROWCOL || KT_all <= 128 ? 1 : 16;
+    bool found = false;
+    for (int z = 1; z <= zmax && (z == 1 || z * M * N * 4 <= scratch); ++z) {
+        const int KT = (KT_all + z - 1) / z, steps8 = (KT + 7) >> 3, steps4 = (KT + 3) >> 2;
+        if ((z - 1) * KT >= KT_all) continue;                // an empty slice
+        const double slices = z == 1 ? 0.0 : 4.5 + (double)(z * M * N) / 1.0e6;
+        for (int mt = 1; mt <= 4 && (mt == 1 || M > 16 * (mt - 1)); ++mt) {
+            const int64_t rt = (M + 16 * mt - 1) / (16 * mt);
+            for (int j = mt > 2; j < 3; ++j) {               // (16 columns with more than 32 rows: never the cheapest)
+                const int64_t rounds = (((N + (16 << j) - 1) >> (4 + j)) * rt * z + LLMK_CUS - 1) / LLMK_CUS;
+                for (int nw = 8; nw >= 4; nw -= 4) {
+                    if (nw == 4 && (j < 2 || m.step4[mt - 1] == 0.f)) continue;
+                    const double cost = slices + (nw == 8 ? m.base8[mt - 1][j] + (double)rounds * (m.fixed8[mt - 1][j] + steps8 * m.step8[mt - 1][j])
+                                                          : m.base4[mt - 1] + (double)rounds * steps4 * m.step4[mt - 1]);
+                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT), KT) > D_LDS_MAX) continue;
+                    best = WavePlan{nw, mt, 1 << j, z, cost};
+                    found = true;
+                }
+            }
+        }
+    }
+    const double weights = 2.0 + (double)(N * K) / 6.1e6;
+    if (found && best.cost < weights) best.cost = weights;
+    return found;
+}
+template <int KIND>
+inline int launch_w8_wave_plan(DirectArgs p, const WavePlan& w, void* scratch, hipStream_t stream, const char* name) {
+    if (w.z > 1) {
+        p.partial = (float*)scratch;
+        p.ksplit = w.z;
+    }
+    auto run = [&](auto nw, auto mt, auto nt, auto d) {
+        constexpr int NW = decltype(nw)::value, MT = decltype(mt)::value, NT = decltype(nt)::value, D = decltype(d)::value;
+        if constexpr (KIND == K_I8_BLOCK) {
+            if (p.s_dtype != LLMK_F32) return launch_w8_wave<KIND, NW, MT, NT, D, false>(p, stream, name);
+        }
+        return launch_w8_wave<KIND, NW, MT, NT, D, true>(p, stream, name);
+    };
+    const std::integral_constant<int, 1> i1;
+    const std::integral_constant<int, 2> i2;
+    const std::integral_constant<int, 3> i3;
+    const std::integral_constant<int, 4> i4;
+    const std::integral_constant<int, 8> i8;
+    auto rows = [&](auto mt) {
+        if constexpr (decltype(mt)::value > 1) {
+            if (w.nw == 4) return run(i4, mt, i4, i1);
+        } else {
+            if (w8_depth(1, w.nt, ((p.K >> 7) + w.z - 1) / w.z) == 2) return run(i8, mt, i1, i2);
+        }
+        if constexpr (decltype(mt)::value <= 2) {
+            if (w.nt == 1) return run(i8, mt, i1, i1);
+        }
+        return w.nt == 4 ? run(i8, mt, i4, i1) : run(i8, mt, i2, i1);
+    };
+    return w.mt == 1 ? rows(i1) : (w.mt == 2 ? rows(i2) : (w.mt == 3 ? rows(i3) : rows(i4)));
+}
+
 inline bool w4a8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
     return wave_plan(M, N, K, scratch, WV_W4A8, [](int nw, int mt, int nt, int per) { return wv_lds(nw, mt, nt, wv_depth(mt, nt, per), per); }, best);
 }

@@ -742,17 +742,14 @@ inline int splitk_factor(int64_t M, int64_t N, int64_t K) {
     return (int)(z > 8 ? 8 : (z < 1 ? 1 : z));
 }
 
-// 16 < M <= 64: the weight-streaming kernel re-reads the activations for every 16 columns, which costs more
-// than the 64-row tile kernel (with split-K when its tiles are few) once the weight matrix is large (measured
-// crossover between 17 M and 25 M elements).
+// 16 < M <= 64 on large weights: the 64-row tile kernel (with split-K when its tiles are few) is worth its scratch, if
+// the wave kernels do not beat it (from 17 M to 25 M elements on it beat streams of 16 columns that re-read the rows).
 inline bool mid_m_prefers_tiles(int64_t M, int64_t N, int64_t K) {
     return M > 16 && M <= 64 && N * K >= (int64_t)20 << 20;
 }
 
-// Rows from which the mid-size kernels beat the weight-streaming ones: 33, and 17 on large weights (us per layer, quantiser
-// and GEMM, streaming or 64-row tiles | mid-size: fp8 64 x 14336 x 4096 28.4 | 23.0, 48 x 4096 x 4096 16.1 | 13.4, 20 x 14336
-// x 4096 23.0 | 20.2, but 20 x 4096 x 4096 11.2 | 12.7; per-token int8 64 x 15368 x 3072 48.7 | 21.9, 32 x 4096 x 4096 12.9 |
-// 15.0).
+// Rows from which the mid-size kernels beat the 64-row tiles: 33, and 17 on large weights (us per layer, quantiser and GEMM, tiles
+// | mid-size: fp8 64 x 14336 x 4096 28.4 | 23.0, 20 x 14336 x 4096 23.0 | 20.2; per-token int8 64 x 15368 x 3072 48.7 | 21.9).
 inline bool mid_rows(int64_t M, int64_t N, int64_t K) { return M > 32 || mid_m_prefers_tiles(M, N, K); }
 
 // Shapes for the mid-size kernel (gemm_mid.hpp): rows as above, at most one workgroup per CU and a K range of at

@@ -271,6 +271,65 @@ def test_w4a8_wave_kernel_exact(dev, M, N, K, sdt, scratch):
     assert torch.equal(c.double(), ref)
 
 
+WAVE_8BIT = [
+    # every tile shape of the kernel whose waves stream their own K share (eight waves 16 to 64 rows x 16 to 64 columns, four waves
+    # 32 to 64 rows x 64), with ragged rows and columns and K steps that do not divide by the waves
+    (1, 72, 128), (7, 1051, 1152), (5, 14344, 1280), (16, 28680, 1152), (17, 41, 384), (31, 6152, 896), (33, 2051, 2432), (50, 40, 256),
+    (97, 41, 1792), (228, 528, 1536), (509, 144, 1536), (261, 936, 1280), (350, 360, 1408), (495, 328, 1152), (495, 744, 2944),
+    (492, 968, 1408), (331, 1392, 2688), (452, 624, 1280), (423, 1232, 1280), (446, 872, 1280), (355, 1104, 1920), (372, 2696, 2688),
+    (509, 1712, 1536), (467, 1720, 1920), (508, 792, 6656), (344, 2704, 1792), (504, 4320, 1536), (357, 3424, 3584), (351, 5424, 1280),
+    # two stages in flight; K slices (without scratch: a scale table of more than one round of loads, and one that leaves room for one
+    # stage only)
+    (9, 264, 8192), (40, 136, 66688), (2, 24, 3276800)]
+
+
+@pytest.mark.parametrize("M,N,K", WAVE_8BIT)
+@pytest.mark.parametrize("kind,sdt", [("fp8", torch.float32), ("i8", torch.float32), ("i8", torch.float16), ("i8", torch.bfloat16),
+                                      ("rowcol", torch.float32)])
+def test_8bit_wave_kernel_exact(dev, M, N, K, kind, sdt):
+    """Whole numbers up to 8, at most 64 of them a row, and power-of-two scales from 1/4 to 4: every sum is a multiple of 2^-4 of at
+    most 2^16, exact in fp32 in any order."""
+    announce("8-bit wave kernel", M, N, K, kind, sdt)
+    gen = torch.Generator(dev).manual_seed(M * 7 + N)
+    a = torch.randint(-8, 9, (M, K), generator=gen, device=dev, dtype=torch.int8)
+    a *= torch.rand(M, K, generator=gen, device=dev) < 64.0 / K
+    a *= a.ne(0).cumsum(1, dtype=torch.int32) <= 64
+    b = torch.randint(-8, 9, (N, K), generator=gen, device=dev, dtype=torch.int8)
+    pow2 = lambda *shape: torch.exp2(torch.randint(-2, 3, shape, generator=gen, device=dev).float())
+    c = torch.full((M, N), 7.0, device=dev)
+    nbytes = _lib.load().llmk_gemm_workspace_bytes(M, N, K)
+    ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=dev)
+    head, tail = (_lib.ptr(c), _lib.dt(torch.float32)), (M, N, K, _lib.ptr(ws), nbytes, None)
+    if kind == "rowcol":
+        a_s, b_s, c32 = pow2(M), pow2(N), torch.full((M, N), 7, dtype=torch.int32, device=dev)
+        _lib.call("llmk_gemm_i8_rowcol", _lib.ptr(a), _lib.ptr(a_s), _lib.ptr(b), _lib.ptr(b_s), *head, _lib.ptr(c32), *tail)
+        sums = torch.zeros(M, N, dtype=torch.float64, device=dev)
+        for k in range(0, K, 1 << 17):
+            sums += a[:, k:k + (1 << 17)].double() @ b[:, k:k + (1 << 17)].double().T
+        assert torch.equal(c32.double(), sums)
+        ref = sums * a_s[:, None].double() * b_s.double()
+    else:
+        a_s, b_s = pow2(M, K // 128), pow2((N + 127) // 128, K // 128)
+        ref = torch.zeros(M, N, dtype=torch.float64, device=dev)
+        for k in range(0, K, 1 << 17):
+            part = slice(k, k + (1 << 17))
+            ks = slice(k // 128, (k + (1 << 17)) // 128)
+            ref += (a[:, part].double() * a_s[:, ks].double().repeat_interleave(128, 1)) @ \
+                   (b[:, part].double() * b_s[:, ks].double().repeat_interleave(128, 1).repeat_interleave(128, 0)[:N]).T
+        if kind == "fp8":
+            a8, b8 = a.float().to(torch.float8_e4m3fn), b.float().to(torch.float8_e4m3fn)
+            call = lambda tail: _lib.call("llmk_gemm_fp8_block", _lib.ptr(a8), _lib.ptr(a_s), _lib.ptr(b8), _lib.ptr(b_s), *head, *tail)
+        else:
+            a_t, b_t = a_s.to(sdt), b_s.to(sdt)
+            call = lambda tail: _lib.call("llmk_gemm_i8_block", _lib.ptr(a), _lib.ptr(a_t), _lib.ptr(b), _lib.ptr(b_t), _lib.dt(sdt), *head, *tail)
+        if K > 16384:
+            call((M, N, K, None, 0, None))
+            assert torch.equal(c.double(), ref)
+            c.fill_(7.0)
+        call(tail)
+    assert torch.equal(c.double(), ref)
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 4096, 4096), (256, 1024, 7168), (512, 4096, 4096), (384, 14336, 4096),
                                    (96, 2056, 14336)])
 def test_w4a8_mid_m_fused_tiles(dev, M, N, K):
