@@ -40,7 +40,7 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
     }
     if (KIND == K_FP8_BLOCK && midw_wanted(M, N, K)) {
         const MidPlan pl = midw_plan(M, N, K);
-        return (pl.mt == 4 ? 5.3 + 11.9 * k / pl.z : 6.7 + 19.2 * k / pl.z) + (pl.z > 1 ? 3.5 : 0.0);
+        return (pl.mt == 4 ? 3.6 + 11.9 * k / pl.z : 5.2 + 19.2 * k / pl.z) + (pl.z > 1 ? 3.5 : 0.0);
     }
     const int z = splitk_factor(M, N, K);
     if (z > 1) return 3.5 + 29.0 * k / z;
@@ -50,7 +50,7 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
 }
 // The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels.  Over 550
 // random shapes of N 1024 to 28672 and K 1024 to 14336, against the kernels before: 1.34 to 1.48 times as fast at 1 to 16 rows, 1.26
-// to 1.50 at 17 to 64, 1.07 (fp8), 1.14 (int8) and 1.23 (per token) at 65 to 512; one in forty of them lost 5 to 10 %.  us, wave | tiles:
+// to 1.50 at 17 to 64, 1.09 (fp8), 1.14 (int8) and 1.23 (per token) at 65 to 512; one in forty of them lost 5 to 10 %.  us, wave | tiles:
 // int8 29 x 4096 x 4096 5.1 | 8.5, fp8 64 x 4096 x 4096 6.2 | 9.4, fp8 200 x 1032 x 7168 7.6 | 15.1, per token 250 x 4096 x 14336 25.1 |
 // 28.1, but fp8 250 x 4096 x 14336 30.6 | 29.2, and from 513 rows on 0.8 times as fast.
 template <int KIND>
