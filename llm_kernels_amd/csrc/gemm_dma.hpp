@@ -137,23 +137,29 @@ __device__ __forceinline__ unsigned asm_load_u16(uint32_t voff, const void* sbas
     return v;
 }
 
-// ---- epilogue helpers.  A lane owns two runs of 8 consecutive outputs (two MFMA results each) per row, so that
-// the four lane groups of a row write 64 contiguous bytes per store instruction (vector stores when the row
-// segment is 16-byte aligned).
+// ---- epilogue helpers.  A lane owns two runs of 8 consecutive outputs (two MFMA results each) per row, so that the four lane
+// groups of a row write 64 contiguous bytes per store instruction: one 16-byte store (two of fp32) at whatever alignment the
+// row has.  (The hardware takes vector accesses at the alignment of the elements.  Rows that do not start on 16 bytes, element
+// by element | so, the whole GEMM in us: fp8 1546 x 3748 x 1024 25.0 | 13.1, 3416 x 10038 x 3072 189 | 121, odd counts of 16-bit
+// outputs 1546 x 3745 x 1024 24.8 | 16.6, 2048 x 14335 x 4096 159 | 128, int8 4096 x 4095 x 4096 101 | 84.)
+template <typename T, int ALIGN>
+struct __attribute__((packed, aligned(ALIGN))) Loose {
+    T v;
+};
 template <int ODT>
-__device__ __forceinline__ void store_run8(void* c, int64_t off, const v4f& a, const v4f& b, int n_valid, bool vec_ok) {
-    if (vec_ok && n_valid >= 8) {
+__device__ __forceinline__ void store_run8(void* c, int64_t off, const v4f& a, const v4f& b, int n_valid) {
+    if (n_valid >= 8) {
         if constexpr (ODT == LLMK_F32) {
-            v4f* dst = (v4f*)((float*)c + off);
-            dst[0] = a;
-            dst[1] = b;
+            Loose<v4f, 4>* dst = (Loose<v4f, 4>*)((float*)c + off);
+            dst[0].v = a;
+            dst[1].v = b;
         } else {
             v4i w;
             w[0] = (int)(ODT == LLMK_F16 ? pack_f16x2(a[0], a[1]) : pack_bf16x2(a[0], a[1]));
             w[1] = (int)(ODT == LLMK_F16 ? pack_f16x2(a[2], a[3]) : pack_bf16x2(a[2], a[3]));
             w[2] = (int)(ODT == LLMK_F16 ? pack_f16x2(b[0], b[1]) : pack_bf16x2(b[0], b[1]));
             w[3] = (int)(ODT == LLMK_F16 ? pack_f16x2(b[2], b[3]) : pack_bf16x2(b[2], b[3]));
-            *(v4i*)((unsigned short*)c + off) = w;
+            ((Loose<v4i, 2>*)((unsigned short*)c + off))->v = w;
         }
     } else {
 #pragma unroll
@@ -163,11 +169,24 @@ __device__ __forceinline__ void store_run8(void* c, int64_t off, const v4f& a, c
         }
     }
 }
-__device__ __forceinline__ void store_run8_i32(int32_t* c, int64_t off, const v4f& a, const v4f& b, int n_valid, bool vec_ok) {
-    if (vec_ok && n_valid >= 8) {
-        v4f* dst = (v4f*)(c + off);
-        dst[0] = a;          // raw bits
-        dst[1] = b;
+// four consecutive outputs, likewise in one store
+template <int ODT>
+__device__ __forceinline__ void store_run4(void* c, int64_t off, const v4f& s) {
+    if constexpr (ODT == LLMK_F32) {
+        ((Loose<v4f, 4>*)((float*)c + off))->v = s;
+    } else {
+        typename FloatIO<ODT>::T h[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) FloatIO<ODT>::st(h, q, s[q]);
+        ((Loose<uint64_t, 2>*)((unsigned short*)c + off))->v =
+            (uint64_t)((unsigned)h[0] | (unsigned)h[1] << 16) | (uint64_t)((unsigned)h[2] | (unsigned)h[3] << 16) << 32;
+    }
+}
+__device__ __forceinline__ void store_run8_i32(int32_t* c, int64_t off, const v4f& a, const v4f& b, int n_valid) {
+    if (n_valid >= 8) {
+        Loose<v4f, 4>* dst = (Loose<v4f, 4>*)(c + off);
+        dst[0].v = a;        // raw bits
+        dst[1].v = b;
     } else {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -177,16 +196,25 @@ __device__ __forceinline__ void store_run8_i32(int32_t* c, int64_t off, const v4
     }
 }
 __device__ __forceinline__ void rowcol_epilogue8(const DirectArgs& p, v4f& a, v4f& b, int m, int64_t off, int nb, int n_valid) {
-    if (p.c_i32) {
-        const bool vec_i = ((((uintptr_t)p.c_i32) & 15) == 0) && (p.N % 4 == 0);
-        store_run8_i32(p.c_i32, off, a, b, n_valid, vec_i);
-    }
+    if (p.c_i32) store_run8_i32(p.c_i32, off, a, b, n_valid);
     if (!p.c) return;
     const float as = ((const float*)p.a_s)[m];
+    const float* const bs = (const float*)p.b_s + nb;
+    v4f sa, sb;
+    if (n_valid >= 8) {
+        sa = ((const Loose<v4f, 4>*)bs)->v;
+        sb = ((const Loose<v4f, 4>*)bs)[1].v;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            sa[q] = bs[min(q, n_valid - 1)];
+            sb[q] = bs[min(4 + q, n_valid - 1)];
+        }
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        a[q] = (float)__float_as_int(a[q]) * as * ((const float*)p.b_s)[nb + min(q, n_valid - 1)];
-        b[q] = (float)__float_as_int(b[q]) * as * ((const float*)p.b_s)[nb + min(4 + q, n_valid - 1)];
+        a[q] = (float)__float_as_int(a[q]) * as * sa[q];
+        b[q] = (float)__float_as_int(b[q]) * as * sb[q];
     }
 }
 
@@ -582,8 +610,6 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
     const bool split = !GROUPED && p.ksplit > 1;
     void* cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
     const int cdt = split ? LLMK_F32 : p.c_dtype;
-    const int esz = cdt == LLMK_F32 ? 4 : 2;
-    const bool vec_ok = ((((uintptr_t)cout) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int m = m_start + wm * WR + 16 * i + r;
@@ -602,9 +628,9 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
                     if (!p.c) continue;
                 }
             }
-            if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, acc[i][2 * h], acc[i][2 * h + 1], nv, vec_ok);
-            else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, acc[i][2 * h], acc[i][2 * h + 1], nv, vec_ok);
-            else store_run8<LLMK_F32>(cout, off, acc[i][2 * h], acc[i][2 * h + 1], nv, vec_ok);
+            if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, acc[i][2 * h], acc[i][2 * h + 1], nv);
+            else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, acc[i][2 * h], acc[i][2 * h + 1], nv);
+            else store_run8<LLMK_F32>(cout, off, acc[i][2 * h], acc[i][2 * h + 1], nv);
         }
     }
 }
@@ -614,7 +640,7 @@ template <int ODT>
 __global__ void splitk_sum_kernel(const float* __restrict__ partial, void* __restrict__ c, int64_t mn, int z) {
     const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (i >= mn) return;
-    if (i + 4 <= mn && mn % 4 == 0) {
+    if (i + 4 <= mn) {
         // four independent loads at a time (the partials come from other CUs' writes: every load is a long
         // round trip), added in slice order
         v4f s = {0.f, 0.f, 0.f, 0.f};
@@ -622,13 +648,12 @@ __global__ void splitk_sum_kernel(const float* __restrict__ partial, void* __res
         for (; k + 4 <= z; k += 4) {
             v4f t[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) t[j] = *(const v4f*)(partial + (int64_t)(k + j) * mn + i);
+            for (int j = 0; j < 4; ++j) t[j] = ((const Loose<v4f, 4>*)(partial + (int64_t)(k + j) * mn + i))->v;
 #pragma unroll
             for (int j = 0; j < 4; ++j) s += t[j];
         }
-        for (; k < z; ++k) s += *(const v4f*)(partial + (int64_t)k * mn + i);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) FloatIO<ODT>::st(c, i + q, s[q]);
+        for (; k < z; ++k) s += ((const Loose<v4f, 4>*)(partial + (int64_t)k * mn + i))->v;
+        store_run4<ODT>(c, i, s);
     } else {
         for (int64_t j = i; j < min(i + 4, mn); ++j) {
             float s = 0.f;
@@ -647,29 +672,27 @@ __global__ void splitk_sum_rowcol_kernel(const int32_t* __restrict__ partial, Di
     if (i >= mn) return;
     const float* as = (const float*)p.a_s;
     const float* bs = (const float*)p.b_s;
-    if (p.N % 4 == 0) {                       // the four elements share a row, every slice is 16-byte aligned
+    if (i + 4 <= mn) {
         v4i s = {0, 0, 0, 0};
         int k = 0;
         for (; k + 4 <= z; k += 4) {
             v4i t[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) t[j] = *(const v4i*)(partial + (int64_t)(k + j) * mn + i);
+            for (int j = 0; j < 4; ++j) t[j] = ((const Loose<v4i, 4>*)(partial + (int64_t)(k + j) * mn + i))->v;
 #pragma unroll
             for (int j = 0; j < 4; ++j) s += t[j];
         }
-        for (; k < z; ++k) s += *(const v4i*)(partial + (int64_t)k * mn + i);
-        if (p.c_i32) {
-            if ((((uintptr_t)p.c_i32) & 15) == 0) *(v4i*)(p.c_i32 + i) = s;
-            else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) p.c_i32[i + q] = s[q];
-            }
-        }
+        for (; k < z; ++k) s += ((const Loose<v4i, 4>*)(partial + (int64_t)k * mn + i))->v;
+        if (p.c_i32) ((Loose<v4i, 4>*)(p.c_i32 + i))->v = s;
         if (p.c) {
-            const int m = (int)(i / p.N), n = (int)(i % p.N);
-            const float am = as[m];
+            int m = (int)(i / p.N), n = (int)(i % p.N);
+            v4f o;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) FloatIO<ODT>::st(p.c, i + q, (float)s[q] * am * bs[n + q]);
+            for (int q = 0; q < 4; ++q) {
+                o[q] = (float)s[q] * as[m] * bs[n];
+                if (++n == p.N) { n = 0; ++m; }              // (m = M only behind the last element)
+            }
+            store_run4<ODT>(p.c, i, o);
         }
     } else {
         for (int64_t j = i; j < min(i + 4, mn); ++j) {

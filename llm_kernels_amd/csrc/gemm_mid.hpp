@@ -338,8 +338,6 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
     const bool split = p.ksplit > 1;
     void* cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
     const int cdt = split ? LLMK_F32 : p.c_dtype;
-    const int esz = cdt == LLMK_F32 ? 4 : 2;
-    const bool vec_ok = ((((uintptr_t)cout) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
     const int ocol = 8 * (tid % RUNS), n = n0 + ocol, nv = N - n;
     if (n >= N) return;
 #pragma unroll
@@ -375,9 +373,9 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
                 if (!p.c) continue;
             }
         }
-        if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv, vec_ok);
-        else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv, vec_ok);
-        else store_run8<LLMK_F32>(cout, off, sa, sb, nv, vec_ok);
+        if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv);
+        else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv);
+        else store_run8<LLMK_F32>(cout, off, sa, sb, nv);
     }
 }
 

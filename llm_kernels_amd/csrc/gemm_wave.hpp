@@ -72,8 +72,6 @@ __device__ __forceinline__ void wv_store(const DirectArgs& p, const float* red, 
     const bool split = p.ksplit > 1;
     void* cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
     const int cdt = split ? LLMK_F32 : p.c_dtype;
-    const int esz = cdt == LLMK_F32 ? 4 : 2;
-    const bool vec_ok = ((((uintptr_t)cout) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
     const int ocol = 8 * (tid % RUNS), nn = n0 + ocol, nv = N - nn;
     if (nn >= N) return;
 #pragma unroll
@@ -100,9 +98,9 @@ __device__ __forceinline__ void wv_store(const DirectArgs& p, const float* red, 
             rowcol_epilogue8(p, sa, sb, m, off, nn, nv);
             if (!p.c) continue;
         }
-        if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv, vec_ok);
-        else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv, vec_ok);
-        else store_run8<LLMK_F32>(cout, off, sa, sb, nv, vec_ok);
+        if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, sa, sb, nv);
+        else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, sa, sb, nv);
+        else store_run8<LLMK_F32>(cout, off, sa, sb, nv);
     }
 }
 

@@ -383,8 +383,6 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     auto stage_b = [&](int kt) { return lds + (kt & 1) * W_STAGE + W_A + (wn * 64) * 128; };
 
     // every lane writes two runs of 8 consecutive outputs of each of its rows; row i of the wave tile:
-    const int esz = p.c_dtype == LLMK_F32 ? 4 : 2;
-    const bool vec_ok = ((((uintptr_t)p.c) & 15) == 0) && (((int64_t)N * esz) % 16 == 0);
     auto store_row = [&](int i) {
         if constexpr (SWIGLU) return;        // nothing is stored before the epilogue below
         const int m = m_start + wm * 16 * R + 16 * i + r;
@@ -409,9 +407,9 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
                 rowcol_epilogue8(p, acc[i][2 * h], acc[i][2 * h + 1], m, off, nbh, nv);
                 if (!p.c) continue;
             }
-            if (p.c_dtype == LLMK_BF16) store_run8<LLMK_BF16>(p.c, off, acc[i][2 * h], acc[i][2 * h + 1], nv, vec_ok);
-            else if (p.c_dtype == LLMK_F16) store_run8<LLMK_F16>(p.c, off, acc[i][2 * h], acc[i][2 * h + 1], nv, vec_ok);
-            else store_run8<LLMK_F32>(p.c, off, acc[i][2 * h], acc[i][2 * h + 1], nv, vec_ok);
+            if (p.c_dtype == LLMK_BF16) store_run8<LLMK_BF16>(p.c, off, acc[i][2 * h], acc[i][2 * h + 1], nv);
+            else if (p.c_dtype == LLMK_F16) store_run8<LLMK_F16>(p.c, off, acc[i][2 * h], acc[i][2 * h + 1], nv);
+            else store_run8<LLMK_F32>(p.c, off, acc[i][2 * h], acc[i][2 * h + 1], nv);
         }
     };
 
@@ -670,6 +668,12 @@ __global__ __launch_bounds__(256) void wide_tail_sum_kernel(DirectArgs p, int es
         const int row = row0 + 4 * it;
         if (row >= rows) continue;
         const int64_t off = (int64_t)(wt.m_start + row) * p.N + n;
+        if (n + 4 <= p.N) {
+            if (p.c_dtype == LLMK_BF16) store_run4<LLMK_BF16>(p.c, off, s[it]);
+            else if (p.c_dtype == LLMK_F16) store_run4<LLMK_F16>(p.c, off, s[it]);
+            else store_run4<LLMK_F32>(p.c, off, s[it]);
+            continue;
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             if (n + q < p.N) st_out(p.c, off + q, s[it][q], p.c_dtype);

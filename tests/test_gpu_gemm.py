@@ -330,6 +330,45 @@ def test_8bit_wave_kernel_exact(dev, M, N, K, kind, sdt):
     assert torch.equal(c.double(), ref)
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 1051, 256), (200, 6146, 1024), (96, 4099, 4096), (600, 517, 1024), (700, 4093, 1024),
+                                   (1030, 10243, 512), (560, 2053, 8192), (400, 1027, 4096)])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", ["fp8", "i8", "rowcol"])
+def test_8bit_outputs_at_any_alignment(dev, M, N, K, out, kind):
+    """Outputs that start one element behind an aligned address, with rows of odd lengths, in every kernel and with K slices: what the
+    fp32 sums (exact: see above) round to, and not an element outside."""
+    announce("8-bit unaligned outputs", M, N, K, out, kind)
+    gen = torch.Generator(dev).manual_seed(M + N)
+    a = torch.randint(-8, 9, (M, K), generator=gen, device=dev, dtype=torch.int8)
+    a *= torch.rand(M, K, generator=gen, device=dev) < 48.0 / K
+    a *= a.ne(0).cumsum(1, dtype=torch.int32) <= 64
+    b = torch.randint(-8, 9, (N, K), generator=gen, device=dev, dtype=torch.int8)
+    ref = a.double() @ b.double().T
+    guard = 32
+    buf = torch.full((M * N + 2 * guard,), 77.0, dtype=out, device=dev)
+    c = buf[guard + 1:guard + 1 + M * N].view(M, N)
+    nbytes = _lib.load().llmk_gemm_workspace_bytes(M, N, K)
+    ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=dev)
+    tail = (M, N, K, _lib.ptr(ws), nbytes, None)
+    if kind == "rowcol":
+        ibuf = torch.full((M * N + 2 * guard,), 77, dtype=torch.int32, device=dev)
+        c32 = ibuf[guard + 1:guard + 1 + M * N].view(M, N)
+        one_a, one_b = torch.ones(M, device=dev), torch.ones(N, device=dev)
+        _lib.call("llmk_gemm_i8_rowcol", _lib.ptr(a), _lib.ptr(one_a), _lib.ptr(b), _lib.ptr(one_b), _lib.ptr(c), _lib.dt(out), _lib.ptr(c32), *tail)
+        assert torch.equal(c32.double(), ref)
+        assert (ibuf[:guard + 1] == 77).all() and (ibuf[guard + 1 + M * N:] == 77).all()
+    else:
+        one_a, one_b = torch.ones(M, K // 128, device=dev), torch.ones((N + 127) // 128, K // 128, device=dev)
+        if kind == "fp8":
+            a8, b8 = a.float().to(torch.float8_e4m3fn), b.float().to(torch.float8_e4m3fn)
+            _lib.call("llmk_gemm_fp8_block", _lib.ptr(a8), _lib.ptr(one_a), _lib.ptr(b8), _lib.ptr(one_b), _lib.ptr(c), _lib.dt(out), *tail)
+        else:
+            _lib.call("llmk_gemm_i8_block", _lib.ptr(a), _lib.ptr(one_a), _lib.ptr(b), _lib.ptr(one_b), _lib.dt(torch.float32), _lib.ptr(c),
+                      _lib.dt(out), *tail)
+    assert torch.equal(c, ref.to(out))
+    assert (buf[:guard + 1] == 77).all() and (buf[guard + 1 + M * N:] == 77).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 4096, 4096), (256, 1024, 7168), (512, 4096, 4096), (384, 14336, 4096),
                                    (96, 2056, 14336)])
 def test_w4a8_mid_m_fused_tiles(dev, M, N, K):
