@@ -80,14 +80,17 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
         // of an XCD share 8 weight tiles and 4 activation tiles.
         // By columns: XCD x (workgroup id mod 8) owns the column tiles x, x + 8, ... of every segment.
         // By segments: XCD x walks an eighth of the whole list, so an expert's weights and rows are read by one XCD (two
-        // where an eighth ends inside it).  
-        // Column counts that are multiples of eight go by columns: the XCDs then have the same mix of full and ragged tiles
-        // (4096 tokens, us per layer, by segments against by columns: 8 experts of 14336 1617, 1543; 16 experts 541, 529; 64
-        // experts of 1408, whose down projection has 8 column tiles, 367, 369).  Other counts go by segments, where the plain
-        // row-major walk reads every weight tile on several XCDs (64 experts of 1408, 11 column tiles of gate and up, 2727
-        // tokens: 420 row-major, 387 by segments; 4096 tokens 560, 516).
-        const int x = lin & 7;
-        const bool by_columns = gx % 8 == 0;
+        // where an eighth ends inside it).
+        // By columns, the XCDs have the same mix of full and ragged tiles, but every row is read by all of them.  That pays
+        // where a column has several row tiles to share its weights (8 experts, 28672 columns, fp8, us by segments | by columns:
+        // 278 rows an expert 407 | 391, 524 655 | 621, 1024 1008 | 994; 16 experts, 4096 columns: 244 rows 132 | 119, 478
+        // 152 | 145), and not with one column tile an XCD (64 experts of 2048 columns: 130 rows 42.6 | 51.5, 290 87 | 91, int8
+        // 433 125 | 131), with one row tile an expert (8 experts, 28672 columns: 182 rows 262 | 290, 211 280 | 317), nor with
+        // long segments of at least two experts an XCD on the 256-row tile (16 experts, 4096 columns: 552 rows 174 | 198, 682 196 |
+        // 205, 891 256 | 270; on the 128-row tile 347 rows lose 5 % of the layer).  Column counts that are no multiple of eight go by segments, where the plain row-major walk reads every weight
+        // tile on several XCDs (64 experts of 1408, 11 column tiles of gate and up, 2727 tokens: 420 row-major, 387 by segments).
+        const int x = lin & 7, rows = p.M / p.E;
+        const bool by_columns = gx % 8 == 0 && gx > 8 && 8 * rows > 7 * W_BM && (R == 4 || p.E < 16 || rows < 512);
         const int cx = by_columns ? gx >> 3 : gx;
         int want = lin >> 3;
         if (!by_columns) {

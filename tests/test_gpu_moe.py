@@ -354,6 +354,26 @@ def test_grouped_gemm_large_tiles_exact(dev, M, N, K):
     assert torch.all(out[used:] == 5.0)
 
 
+@pytest.mark.parametrize("E,rows,N", [(16, 100, 4096), (16, 300, 4096), (16, 600, 4096), (5, 600, 4096), (5, 700, 2048), (40, 210, 4352)])
+def test_grouped_gemm_tile_walks_exact(dev, E, rows, N):
+    """Both walks over the tiles of the large grouped kernel, on each side of the rule that chooses (one row tile an expert, several,
+    long segments of many experts, one column tile an XCD), with segments of unlike length: whole numbers, exact."""
+    announce("grouped tile walks", E, rows, N)
+    gen = torch.Generator().manual_seed(E + rows)
+    ends = torch.sort(torch.randint(0, E * rows + 1, (E - 1,), generator=gen)).values
+    if rows != 700:
+        ends = torch.arange(1, E) * rows + torch.randint(-20, 21, (E - 1,), generator=gen)
+    seg = torch.cat([torch.zeros(1, dtype=torch.int64), ends, torch.tensor([E * rows])])
+    a = torch.randint(-8, 9, (E * rows, 256), dtype=torch.int8, generator=gen)
+    b = torch.randint(-8, 9, (E, N, 256), dtype=torch.int8, generator=gen)
+    c = torch.full((E * rows, N), 5.0, dtype=torch.float32, device=dev)
+    _lib_call_grouped_i8(dev, a, torch.ones(E * rows, 2), b, torch.ones(E, (N + 127) // 128, 2), c, seg, torch.arange(E).flip(0))
+    ad, bd = a.to(dev).float(), b.to(dev).float()
+    for e in range(E):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        assert torch.equal(c[lo:hi], ad[lo:hi] @ bd[E - 1 - e].T), "segment %d" % e
+
+
 @pytest.mark.parametrize("M,N,K,E", [(9000, 2048, 8192, 6), (9000, 1280, 8192, 6), (4700, 4096, 14336, 3)])
 def test_grouped_gemm_split_last_round_exact(dev, M, N, K, E):
     """Long K and a number of 256 x 256 tiles that leaves a short last round: the tiles of that round are split
