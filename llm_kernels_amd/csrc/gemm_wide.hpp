@@ -52,23 +52,10 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
     t.e = 0;
     t.found = false;
     if constexpr (!GROUPED) {
-        // Within every round of 256 workgroups give each XCD a compact block of 8 x 4 tiles of one strip of four
-        // tile rows instead of every eighth tile of the grid, so that its L2 holds few operand rows and all XCDs of
-        // a round share the four activation row tiles.
-        const int gy = (p.M + W_BM - 1) / W_BM, total = gx * gy;
-        if (lin >= total) return t;
-        int bx = lin % gx, by = lin / gx;
-        constexpr int H = 4;      // strips of 8 or 16 tile rows measured 1-13 % slower
-        if (gy % H == 0) {
-            int lp = lin;
-            if (lin < (total & ~(LLMK_CUS - 1))) {
-                const int w = lin & (LLMK_CUS - 1);
-                lp = (lin & ~(LLMK_CUS - 1)) + (w & 7) * (LLMK_CUS / 8) + (w >> 3);
-            }
-            const int strip = lp / (H * gx), rr = lp % (H * gx);
-            bx = rr / H;
-            by = strip * H + rr % H;
-        }
+        const int gy = (p.M + W_BM - 1) / W_BM;
+        if (lin >= gx * gy) return t;
+        int bx, by;
+        xcd_tile(lin, gx, gy, bx, by);
         t.bx = bx;
         t.m_start = by * W_BM;
         t.m_end = min(p.M, t.m_start + W_BM);
@@ -87,8 +74,9 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
         // 152 | 145), and not with one column tile an XCD (64 experts of 2048 columns: 130 rows 42.6 | 51.5, 290 87 | 91, int8
         // 433 125 | 131), with one row tile an expert (8 experts, 28672 columns: 182 rows 262 | 290, 211 280 | 317), nor with
         // long segments of at least two experts an XCD on the 256-row tile (16 experts, 4096 columns: 552 rows 174 | 198, 682 196 |
-        // 205, 891 256 | 270; on the 128-row tile 347 rows lose 5 % of the layer).  Column counts that are no multiple of eight go by segments, where the plain row-major walk reads every weight
-        // tile on several XCDs (64 experts of 1408, 11 column tiles of gate and up, 2727 tokens: 420 row-major, 387 by segments).
+        // 205, 891 256 | 270; on the 128-row tile 347 rows lose 5 % of the layer).  Column counts that are no multiple of eight go
+        // by segments, where the plain row-major walk reads every weight tile on several XCDs (64 experts of 1408, 11 column tiles
+        // of gate and up, 2727 tokens: 420 row-major, 387 by segments).
         const int x = lin & 7, rows = p.M / p.E;
         const bool by_columns = gx % 8 == 0 && gx > 8 && 8 * rows > 7 * W_BM && (R == 4 || p.E < 16 || rows < 512);
         const int cx = by_columns ? gx >> 3 : gx;

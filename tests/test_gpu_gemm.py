@@ -369,6 +369,22 @@ def test_8bit_outputs_at_any_alignment(dev, M, N, K, out, kind):
     assert (buf[:guard + 1] == 77).all() and (buf[guard + 1 + M * N:] == 77).all()
 
 
+@pytest.mark.parametrize("M,N", [(1290, 16904), (1800, 8456), (2300, 8456), (2811, 8456), (4000, 2048), (900, 28672), (640, 16904)])
+def test_large_tile_order_exact(dev, M, N):
+    """Tile rows of 256 or 128 that are and are not a multiple of four, several rounds of workgroups and a part of one: every tile
+    is computed, and computed once."""
+    announce("large tile order", M, N)
+    gen = torch.Generator(dev).manual_seed(M + N)
+    a = torch.randint(-8, 9, (M, 128), generator=gen, device=dev, dtype=torch.int8)
+    b = torch.randint(-8, 9, (N, 128), generator=gen, device=dev, dtype=torch.int8)
+    one_a, one_b = torch.ones(M, device=dev), torch.ones(N, device=dev)
+    ref = (a.float() @ b.float().T)
+    c = torch.full((M, N), 7.5, device=dev)
+    _lib.call("llmk_gemm_i8_rowcol", _lib.ptr(a), _lib.ptr(one_a), _lib.ptr(b), _lib.ptr(one_b), _lib.ptr(c), _lib.dt(torch.float32), None, M, N,
+              128, None, 0, None)
+    assert torch.equal(c, ref)
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 4096, 4096), (256, 1024, 7168), (512, 4096, 4096), (384, 14336, 4096),
                                    (96, 2056, 14336)])
 def test_w4a8_mid_m_fused_tiles(dev, M, N, K):
