@@ -269,7 +269,16 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
         kt0 = (int)blockIdx.z * per;
         KT = max(0, min(per, KT_all - kt0));
     }
-    const int n0 = blockIdx.x * D_BN;
+    // The tile order of xcd_tile, but where one round of workgroups has a multiple of eight columns, which row-major order deals to
+    // the XCDs already (us, so | by xcd_tile: per token 512 x 4096 x 4096 14.8 | 15.6, fp8 1024 x 4096 x 4096 the same), and not for
+    // 16-bit operands and 4-bit weights, which load the L2 less per matrix instruction (fp16 688 x 3776 x 1920 27.9 | 29.9).  Row-major | by xcd_tile elsewhere: fp8 313 x
+    // 12336 x 2304 23.4 | 15.7, 576 x 2368 x 7680 30.4 | 25.7, per token 183 x 8424 x 2048 11.3 | 9.3; 132 cases of 90 to 3000 rows 2 %.
+    int tile_n = blockIdx.x, tile_m = blockIdx.y;
+    if constexpr (!GROUPED && ESZ == 1) {
+        const int gx = (int)gridDim.x, gy = (int)gridDim.y;
+        if (gx % 8 != 0 || gx * gy > (MI == 1 ? 2 : 1) * LLMK_CUS) xcd_tile((int)blockIdx.y * gx + (int)blockIdx.x, gx, gy, tile_n, tile_m);
+    }
+    const int n0 = tile_n * D_BN;
 
     int m_start, m_end;
     const uint8_t* bbase = p.b;
@@ -283,12 +292,12 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
         bbase += widx * (int64_t)N * K;
         bs_off = widx * (int64_t)((N + 127) / 128) * KT_all;
     } else {
-        m_start = blockIdx.y * BM;
+        m_start = tile_m * BM;
         m_end = min(p.M, m_start + BM);
     }
 
     float* bsl = (float*)(lds + D_NSTAGE * D_STAGE);
-    const int64_t bs_row = bs_off + (int64_t)blockIdx.x * KT_all + kt0;
+    const int64_t bs_row = bs_off + (int64_t)tile_n * KT_all + kt0;
 
     // ---- per-thread source offsets (bytes, 32 bit) of the 7 loads of a stage.
     // Load i of a wave fills LDS rows 8q .. 8q+7 with q = wave*4+i (A) or wave*2+i (B), q & 1 == i & 1.

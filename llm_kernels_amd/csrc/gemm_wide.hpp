@@ -45,7 +45,7 @@ __device__ __forceinline__ int wide_total_tiles(const DirectArgs& p, int gx) {
     return segment_entries(p.seg_indptr, p.E, W_BM, gx);
 }
 
-template <bool GROUPED, int R>
+template <bool GROUPED, int R, bool EIGHT>
 __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, int gx) {
     constexpr int W_BM = w_bm(R);
     WideTile t;
@@ -54,8 +54,20 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
     if constexpr (!GROUPED) {
         const int gy = (p.M + W_BM - 1) / W_BM;
         if (lin >= gx * gy) return t;
-        int bx, by;
-        xcd_tile(lin, gx, gy, bx, by);
+        int bx = lin % gx, by = lin / gx;
+        // The order of xcd_tile.  16-bit operands and 4-bit weights (not EIGHT), which load the L2 less per matrix instruction: in full
+        // rounds of whole strips only (bf16 x 4-bit 1033 x 4096 x 4096 54 us so, 57 everywhere).  8-bit operands: but for one round of a
+        // multiple of eight columns, which row-major order deals to the XCDs already.
+        if constexpr (EIGHT) {
+            if (gy % 4 == 0 || gx % 8 != 0 || gx * gy > LLMK_CUS) xcd_tile(lin, gx, gy, bx, by);
+        } else if (gy % 4 == 0) {
+            if (lin < (gx * gy & ~(LLMK_CUS - 1))) {
+                xcd_tile(lin, gx, gy, bx, by);
+            } else {
+                bx = lin % (4 * gx) / 4;
+                by = lin / (4 * gx) * 4 + lin % 4;
+            }
+        }
         t.bx = bx;
         t.m_start = by * W_BM;
         t.m_end = min(p.M, t.m_start + W_BM);
@@ -180,7 +192,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     const bool clocked = p.clocks && lin == 0 && tid == 0;
     long long clk0 = 0, wall0 = 0;
     if (clocked) { clk0 = clock64(); wall0 = wall_clock64(); }
-    WideTile wt = wide_tile_of<GROUPED, R>(p, lin, gx);
+    WideTile wt = wide_tile_of<GROUPED, R, !is_half(KIND)>(p, lin, gx);
     if (p.tail_split) {
         // (the tiles of all but the last round need nothing of this: for them the plan only confirms lin < full;
         // the segment pointers it reads are the ones the lookup above has just read)
@@ -193,7 +205,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
             kt0 = kpart * tp.ktz;
             KT = min(tp.ktz, KT_all - kt0);
             part = p.partial + (int64_t)(kpart * tp.ntail + idx) * (W_BM * W_BN);
-            wt = wide_tile_of<GROUPED, R>(p, lin, gx);
+            wt = wide_tile_of<GROUPED, R, !is_half(KIND)>(p, lin, gx);
         }
     }
     if (!wt.found) return;
@@ -634,14 +646,14 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
 // Adds the partial sums of the split last round (see wide_tail_plan) and writes the outputs of its tiles: grid
 // (tiles of that round, slices of 32 tile rows), the K ranges in ascending order (the result does not depend on
 // timing); a thread sums eight rows at a time so that eight loads are in flight per K range.
-template <bool GROUPED, int R>
+template <bool GROUPED, int R, bool EIGHT>
 __global__ __launch_bounds__(256) void wide_tail_sum_kernel(DirectArgs p, int esz) {
     constexpr int W_BM = w_bm(R);
     const int gx = (p.N + W_BN - 1) / W_BN;
     const WideTail tp = wide_tail_plan(wide_total_tiles<GROUPED, R>(p, gx), (p.K * esz) >> 7);
     const int idx = blockIdx.x;
     if (tp.z <= 1 || idx >= tp.ntail) return;
-    const WideTile wt = wide_tile_of<GROUPED, R>(p, tp.full + idx, gx);
+    const WideTile wt = wide_tile_of<GROUPED, R, EIGHT>(p, tp.full + idx, gx);
     if (!wt.found) return;
     const int rows = wt.m_end - wt.m_start, c4 = (threadIdx.x & 63) * 4, n = wt.bx * W_BN + c4;
     const int row0 = (int)blockIdx.y * 32 + (threadIdx.x >> 6);
@@ -703,7 +715,7 @@ int launch_wide(const DirectArgs& p0, hipStream_t stream, const char* name, void
     kern<<<grid, W_THREADS, W_LDS, stream>>>(p);
     LLMK_CHECK_LAUNCH(name);
     if (tail) {
-        wide_tail_sum_kernel<GROUPED, R><<<dim3(LLMK_CUS / 2, W_BM / 32), 256, 0, stream>>>(p, ESZ);
+        wide_tail_sum_kernel<GROUPED, R, !is_half(KIND)><<<dim3(LLMK_CUS / 2, W_BM / 32), 256, 0, stream>>>(p, ESZ);
         LLMK_CHECK_LAUNCH(name);
     }
     return LLMK_OK;
