@@ -686,6 +686,15 @@ __global__ __launch_bounds__(256) void wide_tail_sum_kernel(DirectArgs p, int es
 // scratch of the split last round: W_TAIL_ITEMS partial tiles of the larger tile shape
 constexpr int64_t w_tail_bytes() { return (int64_t)W_TAIL_ITEMS * w_bm(8) * W_BN * 4; }
 
+// The split is there for this kind, K is long enough, and the scratch holds it (planned for rounds of LLMK_CUS workgroups: taken only
+// on a device with that many CUs).
+template <int KIND>
+bool wide_tail_ok(const DirectArgs& p, const void* ws, int64_t ws_bytes) {
+    constexpr bool HAS = KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_F16 || KIND == K_BF16;
+    return HAS && ws && ws_bytes >= w_tail_bytes() && !((uintptr_t)ws & 15) && ((p.K * (is_half(KIND) ? 2 : 1)) >> 7) >= W_TAIL_MIN_KT &&
+           p.c && llmk_device_cus() == LLMK_CUS;
+}
+
 template <int KIND, bool GROUPED, int R = 8>
 int launch_wide(const DirectArgs& p0, hipStream_t stream, const char* name, void* ws = nullptr, int64_t ws_bytes = 0) {
     static std::atomic<uint64_t> configured{0};
@@ -701,12 +710,7 @@ int launch_wide(const DirectArgs& p0, hipStream_t stream, const char* name, void
     // here; grouped: the segment ends are known on the device only, so the kernel decides, from 256 tiles on)
     bool tail = false;
     p.tail_split = 0;
-    if constexpr (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_F16 || KIND == K_BF16) {
-        const int KT = (p.K * ESZ) >> 7;
-        // (the split is planned for rounds of LLMK_CUS workgroups: taken only on a device with that many CUs)
-        if (ws && ws_bytes >= w_tail_bytes() && !((uintptr_t)ws & 15) && KT >= W_TAIL_MIN_KT && p.c && llmk_device_cus() == LLMK_CUS)
-            tail = GROUPED ? (int64_t)grid.x * grid.y >= LLMK_CUS : wide_tail_plan((int)(grid.x * grid.y), KT).z > 1;
-    }
+    if (wide_tail_ok<KIND>(p, ws, ws_bytes)) tail = GROUPED ? (int64_t)grid.x * grid.y >= LLMK_CUS : wide_tail_plan((int)(grid.x * grid.y), (p.K * ESZ) >> 7).z > 1;
     if (tail) {
         p.tail_split = 1;
         p.partial = (float*)ws;
@@ -794,8 +798,12 @@ struct TileChoice {
     int choice;
     double cost;
 };
+// tail: there is scratch for a split last round of the 256-column tiles (dense launches), which then count what wide_tail_plan makes
+// of it: full rounds, the share of a tile's K steps that a work item multiplies, and the pass over the partial sums (us, tiles
+// of the 128-column kernels | split: fp8 976 x 2446 x 13568 67 | 49, 605 x 1076 x 13056 44 | 35, int8 791 x 2443 x 13440 78 | 56, 1031 x
+// 4096 x 14336 110 | 98).
 template <int KIND, bool GROUPED>
-TileChoice dma_tile_estimate(const DirectArgs& p) {
+TileChoice dma_tile_estimate(const DirectArgs& p, bool tail = false) {
     // 4-bit weights: the row-packed layout, dense launches (the Marlin scatter of 2-byte pieces measured 4-9 % slower
     // inside the 256-column kernel than the dequantisation pass at every M > 512)
     constexpr bool HAS_WIDE = KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND));
@@ -806,7 +814,14 @@ TileChoice dma_tile_estimate(const DirectArgs& p) {
     // the full ones (with the plain ceiling, segments of 128 +- a few rows looked like one 128-row tile each and
     // went to a tile shape that needed two; -8 % on the Mixtral forward at 256 and 512 tokens)
     auto rounds = [&](int bm, int bn) { return (((p.N + bn - 1) / bn) * groups * (GROUPED ? rows / bm + 1 : (rows + bm - 1) / bm) + LLMK_CUS - 1) / LLMK_CUS; };
-    const double t_wide = WIDE * rounds(256, 256), t_half = HALF * rounds(128, 256), t4 = 43.0 * rounds(256, 128), t2 = 26.0 * rounds(128, 128),
+    auto split = [&](int bm, double tile) -> double {
+        const int KT = (p.K * (is_half(KIND) ? 2 : 1)) >> 7;
+        const WideTail w = wide_tail_plan((int)(((p.N + 255) / 256) * ((p.M + bm - 1) / bm)), KT);
+        if (!tail || w.z <= 1) return tile * rounds(bm, 256);
+        const double sums = (6.0 + 0.1 * w.ntail * w.z * bm / 256) / (0.027 * KT);       // us, in units of the tile's costs
+        return tile * (w.full / LLMK_CUS + (double)w.ktz / KT) + sums;
+    };
+    const double t_wide = split(256, WIDE), t_half = split(128, HALF), t4 = 43.0 * rounds(256, 128), t2 = 26.0 * rounds(128, 128),
                  t1 = 16.0 * rounds(64, 128);
     if constexpr (HAS_WIDE) {
         if (t_wide <= t4 && t_wide <= t2 && t_wide <= t1) {
@@ -823,13 +838,13 @@ TileChoice dma_tile_estimate(const DirectArgs& p) {
     return {1, t1};
 }
 template <int KIND, bool GROUPED>
-int dma_tile_choice(const DirectArgs& p) { return dma_tile_estimate<KIND, GROUPED>(p).choice; }
+int dma_tile_choice(const DirectArgs& p, bool tail = false) { return dma_tile_estimate<KIND, GROUPED>(p, tail).choice; }
 
 // AS16 (16-bit activation scales staged as they are): the 64- and 128-row tiles of gemm_dma_kernel only, see launch_big
 template <int KIND, bool GROUPED, bool AS16 = false>
 int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* ws = nullptr, int64_t ws_bytes = 0) {
     if (!GROUPED && p.ksplit > 1) return launch_dma_mi<KIND, GROUPED, 1, AS16>(p, stream, name);
-    const int choice = dma_tile_choice<KIND, GROUPED>(p);
+    const int choice = dma_tile_choice<KIND, GROUPED>(p, !GROUPED && wide_tail_ok<KIND>(p, ws, ws_bytes));
     if constexpr (!AS16) {
         if constexpr (KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND))) {
             if (choice == 9) return launch_wide<KIND, GROUPED, 4>(p, stream, name, ws, ws_bytes);
@@ -887,7 +902,9 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
     if constexpr (HAS_AS16) {
         if (p.s_dtype != LLMK_F32) {
             const int z = GROUPED ? 1 : splitk_factor(p.M, p.N, p.K);
-            as16 = z > 1 || dma_tile_choice<KIND, GROUPED>(p) <= 2;
+            const int64_t widened = ((int64_t)p.M * (p.K >> 7) * 4 + 255) & ~(int64_t)255;
+            const bool tail = !GROUPED && workspace && wide_tail_ok<KIND>(p, (uint8_t*)workspace + widened, workspace_bytes - widened);
+            as16 = z > 1 || dma_tile_choice<KIND, GROUPED>(p, tail) <= 2;
         }
     }
     if (p.s_dtype != LLMK_F32 && !as16) {
