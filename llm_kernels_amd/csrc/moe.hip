@@ -40,16 +40,15 @@ __device__ __forceinline__ int64_t ld_id(const void* p, int64_t i, int bytes) {
 // chunk + its rank among the equal ids of its own wave.  No workgroup waits for another.
 // Bound by latency: a chain of one load, three barriers and a scan.  Few buckets are counted in 64 columns per bucket, one
 // per lane, so that the ids of a wave never meet on one LDS address (ballots per bucket, the form before, took
-// 12.2 us for 8192 ids of 8 experts, this one 8.4); 65 to 256 ids get a workgroup of 256.  What is left grows with the list: a
-// workgroup's LDS additions, about one a clock (21816 ids of 64 experts 18.2 us, 32768 22.2; 23.4 and 26.2 with half the loads
+// 12.2 us for 8192 ids of 8 experts, this one 8.4); lists that one workgroup holds have a kernel of their own.  What is left grows
+// with the list: a workgroup's LDS additions, about one a clock (21816 ids of 64 experts 18.2 us, 32768 22.2; 23.4 and 26.2 with half the loads
 // in flight and a pass per distinct bucket in the ranking).
 constexpr int PP_THREADS = 1024, PP_MAX_EXPERTS = 512, PP_BUCKETS = PP_MAX_EXPERTS + 2, PP_FEW = 66;
 
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
-                                                                void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
-                                                                int64_t* __restrict__ seg_indptr) {
-    constexpr int WAVES = THREADS / 64;
+__global__ __launch_bounds__(PP_THREADS) void ep_preprocess_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
+                                                                   void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
+                                                                   int64_t* __restrict__ seg_indptr) {
+    constexpr int THREADS = PP_THREADS, WAVES = THREADS / 64;
     __shared__ int tot[PP_BUCKETS];      // ids per bucket, then the bucket's first position
     __shared__ int pre[PP_BUCKETS];      // ids per bucket in front of this workgroup's chunk
     // either the columns of a few buckets (two counts per cell: ids in front of the chunk in the low half, the others in
@@ -137,6 +136,62 @@ __global__ __launch_bounds__(THREADS) void ep_preprocess_kernel(const void* __re
         const int64_t id = (b >= 1 && b <= E) ? (int64_t)(b - 1) : ld_id(ids, i, ids_bytes);
         if (ids_bytes == 8) ((int64_t*)sorted_out)[pos] = id; else ((int32_t*)sorted_out)[pos] = (int32_t)id;
         src2dst[i] = pos;
+    }
+}
+
+// The same for a list that one workgroup holds, an id per thread: the counts of its waves are all there is to count, so there
+// are no columns to clear, fill and add up, and the code is short (see below).  (us,
+// the kernel above | this one: 96 ids of 64 experts 8.9 | 2.8, 256 of 8 4.7 | 2.6, 588 of 16 5.0 | 3.2, 1000 of 64 7.6 | 3.9.)
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void ep_preprocess_one_kernel(const void* __restrict__ ids, int ids_bytes, int n, int E,
+                                                                    void* __restrict__ sorted_out, int32_t* __restrict__ src2dst,
+                                                                    int64_t* __restrict__ seg_indptr) {
+    constexpr int WAVES = THREADS / 64;
+    __shared__ int first[PP_BUCKETS];            // the bucket's first position
+    __shared__ int cells[WAVES * PP_BUCKETS];    // ids per wave and bucket
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = E + 2;
+    const bool live = tid < n;
+    const int64_t id = live ? ld_id(ids, tid, ids_bytes) : 0;
+    const int b = id < 0 ? 0 : (id >= E ? E + 1 : (int)id + 1);
+    for (int i = tid; i < WAVES * nb; i += THREADS) cells[i] = 0;
+    uint64_t same = __ballot(live);
+    for (int bit = 0; nb >> bit; ++bit) {
+        const bool one = (b >> bit) & 1;
+        const uint64_t m = __ballot(one);
+        same &= one ? m : ~m;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    __syncthreads();
+    if (live && rank == 0) cells[wave * nb + b] = __popcll(same);
+    __syncthreads();
+    if (wave == 0) {
+        // starts of the buckets, and of a bucket's waves in it: a run of buckets per lane, then a scan over the lanes
+        const int per = (nb + 63) / 64, b0 = lane * per, b1 = min(b0 + per, nb);
+        int sum = 0;
+        for (int k = b0; k < b1; ++k)
+            for (int w = 0; w < WAVES; ++w) sum += cells[w * nb + k];
+        int incl = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += t;
+        }
+        int run = incl - sum;
+        for (int k = b0; k < b1; ++k) {
+            first[k] = run;
+            for (int w = 0; w < WAVES; ++w) {
+                const int c = cells[w * nb + k];
+                cells[w * nb + k] = run;
+                run += c;
+            }
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e <= E; e += THREADS) seg_indptr[e] = e == 0 ? 0 : (int64_t)first[e + 1];
+    if (live) {
+        const int pos = cells[wave * nb + b] + rank;
+        if (ids_bytes == 8) ((int64_t*)sorted_out)[pos] = id; else ((int32_t*)sorted_out)[pos] = (int32_t)id;
+        src2dst[tid] = pos;
     }
 }
 
@@ -510,8 +565,9 @@ extern "C" int llmk_moe_ep_preprocess(const void* topk_ids, int ids_bytes, int64
     const unsigned grid = (unsigned)(num_toks > 0 ? cdiv64(num_toks, PP_THREADS) : 1);
     // one workgroup of the smallest size that holds the ids, chunks of PP_THREADS beyond
     if (num_toks <= 64) ep_preprocess_wave_kernel<<<1, 64, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
-    else if (num_toks <= 256) ep_preprocess_kernel<256><<<1, 256, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
-    else ep_preprocess_kernel<PP_THREADS><<<grid, PP_THREADS, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
+    else if (num_toks <= 256) ep_preprocess_one_kernel<256><<<1, 256, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
+    else if (num_toks <= PP_THREADS) ep_preprocess_one_kernel<PP_THREADS><<<1, PP_THREADS, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
+    else ep_preprocess_kernel<<<grid, PP_THREADS, 0, (hipStream_t)stream>>>(topk_ids, ids_bytes, (int)num_toks, num_experts, sorted_ids, src2dst, seg_indptr);
     LLMK_CHECK_LAUNCH("moe_ep_preprocess");
     return LLMK_OK;
 }
