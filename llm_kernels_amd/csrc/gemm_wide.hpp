@@ -55,9 +55,10 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
         const int gy = (p.M + W_BM - 1) / W_BM;
         if (lin >= gx * gy) return t;
         int bx = lin % gx, by = lin / gx;
-        // The order of xcd_tile.  16-bit operands and 4-bit weights (not EIGHT), which load the L2 less per matrix instruction: in full
-        // rounds of whole strips only (bf16 x 4-bit 1033 x 4096 x 4096 54 us so, 57 everywhere).  8-bit operands: but for one round of a
-        // multiple of eight columns, which row-major order deals to the XCDs already.
+        // The order of xcd_tile.  8-bit operands: but for one round of a multiple of eight columns, which row-major order deals to the
+        // XCDs already.  16-bit operands and 4-bit weights (not EIGHT), which load the L2 less per matrix instruction: only with more
+        // than a round (bf16 x 4-bit 1033 x 4096 x 4096 54 us so, 57 everywhere; 160 shapes of 1024 to 4096 rows 2 % faster than with
+        // row-major order where the tile rows are no multiple of four), and the last round of whole strips as it comes.
         if constexpr (EIGHT) {
             if (gy % 4 == 0 || gx % 8 != 0 || gx * gy > LLMK_CUS) xcd_tile(lin, gx, gy, bx, by);
         } else if (gy % 4 == 0) {
@@ -67,6 +68,8 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
                 bx = lin % (4 * gx) / 4;
                 by = lin / (4 * gx) * 4 + lin % 4;
             }
+        } else if (gx * gy > LLMK_CUS) {
+            xcd_tile(lin, gx, gy, bx, by);
         }
         t.bx = bx;
         t.m_start = by * W_BM;
@@ -801,7 +804,7 @@ struct TileChoice {
 // tail: there is scratch for a split last round of the 256-column tiles (dense launches), which then count what wide_tail_plan makes
 // of it: full rounds, the share of a tile's K steps that a work item multiplies, and the pass over the partial sums (us, tiles
 // of the 128-column kernels | split: fp8 976 x 2446 x 13568 67 | 49, 605 x 1076 x 13056 44 | 35, int8 791 x 2443 x 13440 78 | 56, 1031 x
-// 4096 x 14336 110 | 98).
+// 4096 x 14336 110 | 98).  8-bit operands: with 16-bit ones the split pays 1 % on average and loses up to 14 %.
 template <int KIND, bool GROUPED>
 TileChoice dma_tile_estimate(const DirectArgs& p, bool tail = false) {
     // 4-bit weights: the row-packed layout, dense launches (the Marlin scatter of 2-byte pieces measured 4-9 % slower
@@ -844,7 +847,7 @@ int dma_tile_choice(const DirectArgs& p, bool tail = false) { return dma_tile_es
 template <int KIND, bool GROUPED, bool AS16 = false>
 int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* ws = nullptr, int64_t ws_bytes = 0) {
     if (!GROUPED && p.ksplit > 1) return launch_dma_mi<KIND, GROUPED, 1, AS16>(p, stream, name);
-    const int choice = dma_tile_choice<KIND, GROUPED>(p, !GROUPED && wide_tail_ok<KIND>(p, ws, ws_bytes));
+    const int choice = dma_tile_choice<KIND, GROUPED>(p, !GROUPED && !is_half(KIND) && wide_tail_ok<KIND>(p, ws, ws_bytes));
     if constexpr (!AS16) {
         if constexpr (KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND))) {
             if (choice == 9) return launch_wide<KIND, GROUPED, 4>(p, stream, name, ws, ws_bytes);
