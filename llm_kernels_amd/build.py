@@ -74,7 +74,7 @@ def _assembly(src):
 # what tells that a source hand-issues loads into registers: the loaders themselves, the header of the ring
 # kernels, or a tile-kernel kind whose weight rows are expanded from hand-loaded packed words
 _ASM_LOAD_MARKS = ('asm volatile("global_load_dword', "ring_load_", "asm_load_", "stream_ring.hpp",
-                   "K_W4NK", "K_W4MARLIN", "K_W4A8")
+                   "K_W4NK", "K_W4MARLIN")
 
 
 def _has_asm_register_loads(src):

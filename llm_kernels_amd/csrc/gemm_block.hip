@@ -43,7 +43,7 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
         return (pl.mt == 4 ? 3.6 + 11.9 * k / pl.z : 5.2 + 19.2 * k / pl.z) + (pl.z > 1 ? 3.5 : 0.0);
     }
     const int z = splitk_factor(M, N, K);
-    if (z > 1) return 3.5 + 29.0 * k / z;
+    if (z > 1) return 3.0 + 26.0 * k / z;
     const TileChoice c = dma_tile_estimate<KIND, false>(p);
     const double e = c.cost * k * (KIND == K_I8_BLOCK ? 1.12 : 1.0);
     return c.choice == 1 ? 3.4 + 0.87 * e : (c.choice == 2 ? 5.0 + 0.7 * e : (c.choice == 8 ? 9.0 + 0.85 * e : 7.5 + 0.8 * e));

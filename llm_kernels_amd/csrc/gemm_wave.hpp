@@ -978,7 +978,7 @@ constexpr WaveModel WV_I8_ROWCOL = {{{2.86f, 2.76f, 1.56f}, {2.90f, 2.76f, 1.28f
                                     {{0.00f, 0.08f, 1.26f}, {0.06f, 0.12f, 1.83f}, {0.f, 1.39f, 2.46f}, {0.f, 1.54f, 3.11f}},
                                     {{0.32f, 0.47f, 0.83f}, {0.45f, 0.65f, 1.02f}, {0.f, 0.80f, 1.20f}, {0.f, 0.96f, 1.38f}},
                                     {0.f, 3.20f, 5.00f, 4.05f}, {0.f, 0.54f, 0.67f, 0.79f}};
-constexpr int w8_depth(int mt, int nt, int steps) { return mt == 1 && nt == 1 && steps >= 64 ? 2 : 1; }
+constexpr int w8_depth(int mt, int nt, int steps) { return mt == 1 && nt == 1 && steps >= 48 ? 2 : 1; }
 template <int KIND>
 inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
     constexpr const WaveModel& m = KIND == K_FP8_BLOCK ? WV_FP8 : (KIND == K_I8_BLOCK ? WV_I8 : WV_I8_ROWCOL);
@@ -1006,7 +1006,13 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
         }
     }
     const double weights = 2.0 + (double)(N * K) / 6.1e6;
-    if (found && best.cost < weights) best.cost = weights;
+    if (found && best.cost < weights) {
+        // Bound by the weights: up to 16 rows the narrowest tiles, four workgroups a CU, keep HBM busiest (fp8, us from HBM, 64
+        // columns | 16: 1 x 28672 x 4096 32.2 | 29.8, 8 x 18000 x 4096 27.3 | 21.4, 16 x 20000 x 6144 40.4 | 35.0, 1 x 128256 x 4096 101 | 94).
+        const double narrow = m.base8[0][0] + (double)(((N + 15) / 16 + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][0] + ((KT_all + 7) >> 3) * m.step8[0][0]);
+        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1, w8_depth(1, 1, KT_all), KT_all) <= D_LDS_MAX) best = WavePlan{8, 1, 1, 1, weights};
+        best.cost = weights;
+    }
     return found;
 }
 template <int KIND>
