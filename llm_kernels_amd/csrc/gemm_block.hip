@@ -57,9 +57,8 @@ template <int KIND>
 WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspace_bytes) {
     WavePlan w{0, 0, 0, 0, 0.0};
     const int64_t scratch = workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0;
-    if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w) ||
-        1.08 * w.cost >= tiles_estimate<KIND>(p, workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K)))
-        w.nw = 0;
+    if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w)) w.nw = 0;
+    else if (p.M > 16 && 1.08 * w.cost >= tiles_estimate<KIND>(p, workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K))) w.nw = 0;
     return w;
 }
 template <int KIND>

@@ -358,7 +358,8 @@ int launch_w4a8_wave(const DirectArgs& p, int z, hipStream_t stream, const char*
     const int KT_all = p.K >> 7, per = (KT_all + z - 1) / z;
     const int bytes = wv_lds(NW, MT, NT, D, per);
     if (bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, bytes);
-    if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
+    if (bytes > 64 * 1024)       // (less needs no leave, and asking for it costs a decode call 0.1 us)
+        if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     DirectArgs q = p;
     q.ksplit = z;
     const int zg = (KT_all + per - 1) / per;
@@ -694,7 +695,8 @@ int launch_w4a16_wave(const DirectArgs& p, int z, hipStream_t stream, const char
     const int KT_all = p.K >> 7, per = (KT_all + z - 1) / z, groups = wh_groups(p.K, p.group, per);
     const int bytes = wh_lds(KIND, NW, MT, NT, groups);
     if (bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, bytes);
-    if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
+    if (bytes > 64 * 1024)       // (less needs no leave, and asking for it costs a decode call 0.1 us)
+        if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     DirectArgs q = p;
     q.ksplit = z;
     const int zg = (KT_all + per - 1) / per;
@@ -881,7 +883,8 @@ int launch_w8_wave(const DirectArgs& p, hipStream_t stream, const char* name) {
     const int z = p.ksplit > 1 ? p.ksplit : 1;
     const int bytes = w8_lds(NW, MT, NT, D, ((p.K >> 7) + z - 1) / z);
     if (bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, bytes);
-    if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
+    if (bytes > 64 * 1024)       // (less needs no leave, and asking for it costs a decode call 0.1 us)
+        if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
     kern<<<dim3(tiles, 1, (unsigned)z), NW * 64, bytes, stream>>>(p);
     LLMK_CHECK_LAUNCH(name);
@@ -1007,10 +1010,13 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
     }
     const double weights = 2.0 + (double)(N * K) / 6.1e6;
     if (found && best.cost < weights) {
-        // Bound by the weights: up to 16 rows the narrowest tiles, four workgroups a CU, keep HBM busiest (fp8, us from HBM, 64
-        // columns | 16: 1 x 28672 x 4096 32.2 | 29.8, 8 x 18000 x 4096 27.3 | 21.4, 16 x 20000 x 6144 40.4 | 35.0, 1 x 128256 x 4096 101 | 94).
-        const double narrow = m.base8[0][0] + (double)(((N + 15) / 16 + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][0] + ((KT_all + 7) >> 3) * m.step8[0][0]);
-        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1, w8_depth(1, 1, KT_all), KT_all) <= D_LDS_MAX) best = WavePlan{8, 1, 1, 1, weights};
+        // Bound by the weights: up to 8 rows tiles of 16 columns, four workgroups a CU, keep HBM busiest, up to 16 rows, whose activations
+        // weigh more, tiles of 32 (fp8, us from HBM, 64 | 32 | 16 columns: 1 x 28672 x 4096 32.2 | 31.0 | 29.8, 8 x 18000 x 4096 27.3 | 23.2 |
+        // 21.4, 8 x 128256 x 4096 103 | 100 | 99, 16 x 57344 x 4096 57.4 | 52.3 | 56.2, 16 x 128256 x 4096 105 | 102 | 111).
+        const int j = M <= 8 ? 0 : 1;
+        const double narrow = m.base8[0][j] + (double)(((N + (16 << j) - 1) / (16 << j) + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
+        const int d = w8_depth(1, 1 << j, KT_all);
+        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX) best = WavePlan{8, 1, 1 << j, 1, weights};
         best.cost = weights;
     }
     return found;
