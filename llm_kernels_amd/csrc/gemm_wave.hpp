@@ -1012,8 +1012,9 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
     if (found && best.cost < weights) {
         // Bound by the weights: up to 8 rows tiles of 16 columns, four workgroups a CU, keep HBM busiest, up to 16 rows, whose activations
         // weigh more, tiles of 32 (fp8, us from HBM, 64 | 32 | 16 columns: 1 x 28672 x 4096 32.2 | 31.0 | 29.8, 8 x 18000 x 4096 27.3 | 23.2 |
-        // 21.4, 8 x 128256 x 4096 103 | 100 | 99, 16 x 57344 x 4096 57.4 | 52.3 | 56.2, 16 x 128256 x 4096 105 | 102 | 111).
-        const int j = M <= 8 ? 0 : 1;
+        // 21.4, 8 x 128256 x 4096 103 | 100 | 99, 16 x 57344 x 4096 57.4 | 52.3 | 56.2, 16 x 128256 x 4096 105 | 102 | 111),
+        // where those still make two a CU (16 x 4096 x 14336 22.1 | 18.1 with 32 | 16).
+        const int j = M <= 8 || N < 64 * LLMK_CUS ? 0 : 1;
         const double narrow = m.base8[0][j] + (double)(((N + (16 << j) - 1) / (16 << j) + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
         const int d = w8_depth(1, 1 << j, KT_all);
         if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX) best = WavePlan{8, 1, 1 << j, 1, weights};
