@@ -48,7 +48,8 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
     const double e = c.cost * k * (KIND == K_I8_BLOCK ? 1.12 : 1.0);
     return c.choice == 1 ? 3.4 + 0.87 * e : (c.choice == 2 ? 5.0 + 0.7 * e : (c.choice == 8 ? 9.0 + 0.85 * e : 7.5 + 0.8 * e));
 }
-// The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels.  Over 550
+// The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels (block-scaled
+// operands beyond 128 rows: 16 %, which covers weights from HBM: 256 x 4096 x 4096 fp8 16.1 | 15.2, int8 16.2 | 15.0).  Over 550
 // random shapes of N 1024 to 28672 and K 1024 to 14336, against the kernels before: 1.34 to 1.48 times as fast at 1 to 16 rows, 1.26
 // to 1.50 at 17 to 64, 1.09 (fp8), 1.14 (int8) and 1.23 (per token) at 65 to 512; one in forty of them lost 5 to 10 %.  us, wave | tiles:
 // int8 29 x 4096 x 4096 5.1 | 8.5, fp8 64 x 4096 x 4096 6.2 | 9.4, fp8 200 x 1032 x 7168 7.6 | 15.1, per token 250 x 4096 x 14336 25.1 |
@@ -58,7 +59,8 @@ WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspa
     WavePlan w{0, 0, 0, 0, 0.0};
     const int64_t scratch = workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0;
     if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w)) w.nw = 0;
-    else if (p.M > 16 && 1.08 * w.cost >= tiles_estimate<KIND>(p, workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K))) w.nw = 0;
+    const double margin = KIND != K_I8_ROWCOL && p.M > 128 ? 1.16 : 1.08;
+    if (w.nw && p.M > 16 && margin * w.cost >= tiles_estimate<KIND>(p, workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K))) w.nw = 0;
     return w;
 }
 template <int KIND>
