@@ -166,7 +166,8 @@ int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b_packed, co
  * C[M,N] (fp16) = A[M,K] (fp16) x ((nibble - 8) * s[k / groupsize, n]); B and s in the
  * simple-Marlin packed layout produced by QuantUtils.pack (B int32 [K/16, 2N], s fp16 [K/g, N]
  * permuted per 64 columns).  M, N, K % 16 == 0 (rc -1 otherwise, as the reference launcher),
- * additionally N % 64 == 0 and groupsize % 16 == 0.
+ * additionally N % 64 == 0 and groupsize % 16 == 0.  The weights are (nibble - 8) * s rounded to fp16 once for every M, as
+ * QuantUtils.fake_quantize gives them; sums are fp32.
  * ref: fast_dequant/simple_marlin/marlin_w4a16_gemm.cu:283-326 (simple_marlin_cuda),
  *      marlin_w4a16_gemm.cpp:23-111 (mul).                                                    */
 /* bytes of scratch llmk_gemm_w4a16_marlin uses for this shape (0 = none): fp32 split-K partial sums, and for
@@ -184,7 +185,9 @@ int llmk_gemm_w4a16_marlin(const void* a_f16, const int32_t* b, void* c_f16, con
 int llmk_quant_w4_nk(const void* w, int w_dtype, int32_t* packed, void* scales_f16, uint8_t* q, int64_t N,
                      int64_t K, int group, void* stream);
 /* Same product for W stored [N, K/8] int32 by pack_weights_over_cols (nibble i of a word = k*8+i)
- * with s fp16 [N, K/g]; a/c fp16 or bf16 (ac_dtype).  workspace: llmk_gemm_w4a16_nk_workspace_bytes(...) bytes, 16-byte
+ * with s fp16 [N, K/g]; a/c fp16 or bf16 (ac_dtype).  What the weights are depends on the shape alone: beyond 64 rows (fp16: also
+ * from 33 rows where the weight matrix is large) (nibble - 8) * s
+ * rounded to the type of a, otherwise nibble - 8 exactly with s on the fp32 sums of a group.  workspace: llmk_gemm_w4a16_nk_workspace_bytes(...) bytes, 16-byte
  * aligned, is what the path chosen for the shape uses:
  *   - M <= 64 streams the weights: nothing for K <= 4096, fp32 partial sums of K ranges, ceil(K/4096)*M*N*4, beyond;
  *   - 64 < M <= 512 (from 33 rows on large weights, to 1024 rows and more where it wins) runs on tile kernels that expand

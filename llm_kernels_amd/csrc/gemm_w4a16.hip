@@ -979,12 +979,19 @@ double nk_other_estimate(const llmk::DirectArgs& p) {
         default: return 3.0 + 1.7 * e;
     }
 }
+// What the weights of a call are, by its shape alone: (q - 8) * scale rounded to the activations' type, as in the tile kernels and in
+// the 16-bit copy of W, or q - 8 exactly with the scale on fp32 sums, as in the streaming kernels.  The wave kernel has both and
+// takes what those have that it stands in for: a row's result then does not hang on which kernel is faster.
+bool nk_rounded_weights(int64_t M, int64_t N, int64_t K, bool bf) {
+    if (M > 64) return true;
+    return !bf && w4_tiles_expand(M, N, K, INT64_MAX, true);
+}
 // The wave kernel for this call, or z = 0: taken 8 % below the others' estimate.
 template <int KIND>
 llmk::WavePlan nk_wave(const llmk::DirectArgs& p, int64_t scratch) {
     llmk::WavePlan w{0, 0, 0, 0, 0.0};
-    const bool fits = KIND == llmk::K_W4NKB && p.M > 64 ? llmk::w4a16_wave_plan<KIND, KIND == llmk::K_W4NKB>(p.M, p.N, p.K, p.group, scratch, w)
-                                                        : llmk::w4a16_wave_plan<KIND>(p.M, p.N, p.K, p.group, scratch, w);
+    const bool fits = nk_rounded_weights(p.M, p.N, p.K, KIND == llmk::K_W4NKB) ? llmk::w4a16_wave_plan<KIND, true>(p.M, p.N, p.K, p.group, scratch, w)
+                                                                                       : llmk::w4a16_wave_plan<KIND, false>(p.M, p.N, p.K, p.group, scratch, w);
     if (!fits || 1.08 * w.cost >= nk_other_estimate<KIND>(p)) w.z = 0;
     return w;
 }
@@ -1051,7 +1058,7 @@ MarlinPlan marlin_plan(int64_t M, int64_t N, int64_t K) {
 // 47.1 | 60.2, but 384 x 14336 x 4096 87.8 | 80.0.
 llmk::WavePlan marlin_wave(int64_t M, int64_t N, int64_t K, int group, int64_t scratch) {
     llmk::WavePlan w{0, 0, 0, 0, 0.0};
-    if (M > 512 || !llmk::w4a16_wave_plan<llmk::K_W4MARLIN>(M, N, K, group, scratch, w)) { w.z = 0; return w; }
+    if (M > 512 || !llmk::w4a16_wave_plan<llmk::K_W4MARLIN, true>(M, N, K, group, scratch, w)) { w.z = 0; return w; }
     if (M > 64) {
         llmk::DirectArgs p{};
         p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
@@ -1107,7 +1114,7 @@ extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, 
         llmk::DirectArgs p{};
         p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.b_s = s; p.c = c; p.c_dtype = LLMK_F16;
         p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = groupsize; p.partial = (float*)workspace;
-        return llmk::launch_w4a16_wave_plan<llmk::K_W4MARLIN>(p, wave, st, "gemm_w4a16_marlin(wave)");
+        return llmk::launch_w4a16_wave_plan<llmk::K_W4MARLIN, true>(p, wave, st, "gemm_w4a16_marlin(wave)");
     }
     if (w4_tiles_expand(M, N, K, usable_scratch(workspace, workspace_bytes)) && K % 64 == 0 && groupsize % 64 == 0) {
         // mid-size M: the 128-column tile kernels expand the Marlin units themselves (see gemm_w4a16_nk)
@@ -1203,10 +1210,11 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
     switch (pl.route) {
         case NkPlan::WAVE:
             p.b = (const uint8_t*)b_packed; p.b_s = s; p.group = groupsize; p.partial = (float*)workspace;
-            // (bf16 beyond 64 rows: weights rounded to bf16, as every kernel of such calls has them)
-            if (!bf) return llmk::launch_w4a16_wave_plan<llmk::K_W4NK>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
-            return M > 64 ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)")
-                          : llmk::launch_w4a16_wave_plan<llmk::K_W4NKB>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
+            if (nk_rounded_weights(M, N, K, bf))
+                return bf ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)")
+                          : llmk::launch_w4a16_wave_plan<llmk::K_W4NK, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
+            return bf ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, false>(p, pl.wave, st, "gemm_w4a16_nk(wave)")
+                      : llmk::launch_w4a16_wave_plan<llmk::K_W4NK, false>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
         case NkPlan::RING:                               // bf16 decode; fp16 reaches that kernel through launch_nk_stream
             return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, pl.nz, (float*)workspace, true, st);
         case NkPlan::TILES:

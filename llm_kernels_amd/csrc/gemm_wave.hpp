@@ -397,12 +397,15 @@ constexpr int wh_groups(int K, int group, int per) {
     return a < b ? a : b;
 }
 
-// PRE (bf16): the weights are (q - 8) * scale rounded to bf16, as the tile kernels of larger M have them, and sums run over
-// all of K; otherwise they are q - 8 exactly and the scale multiplies the fp32 sums of a half step.
+// PRE: the weights are (q - 8) * scale rounded to the activations' type, as the tile kernels of larger M have them (and the
+// reference's Marlin kernel: marlin_w4a16_gemm.cu:152-236), and sums run over all of K; otherwise they are q - 8 exactly and the scale
+// multiplies the fp32 sums of a half step.  Marlin words always, row-packed ones where the caller's rule says so.  (us, weights from
+// HBM, exact weights | rounded: Marlin 16 x 4096 x 4096 8.2 | 8.1, 64 x 14336 x 4096 18.4 | 18.0, 128 x 4096 x 4096 12.0 | 12.7, 16 x 4096 x
+// 14336 13.8 | 14.5, fp16 160 x 4096 x 14336 40.1 | 40.1: the scale is one more packed product a word, or a product an output and half step.)
 template <int KIND, int NW, int MT, int NT, bool PRE>
 __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
     static_assert(is_w4nk(KIND) || wh_marlin(KIND), "4-bit weights, 16-bit activations");
-    static_assert(!PRE || KIND == K_W4NKB, "scaled weights: bf16");
+    static_assert(PRE || !wh_marlin(KIND), "Marlin words: scaled weights");
     constexpr bool MARLIN = wh_marlin(KIND), BF = (KIND == K_W4NKB);
     constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = wh_stage(KIND, MT, NT), OFF_B = wh_a(MT), WB = wh_b(KIND, NT), NB = WB / 1024;
     constexpr int TR = wh_tab_row(KIND, NT), TC = wh_tab_cols(KIND, NT);
@@ -587,7 +590,7 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             init[mt] = (v4f){0.f, 0.f, 0.f, 0.f};
-            if constexpr (!MARLIN && !PRE) {
+            if constexpr (!MARLIN && !(BF && PRE)) {
                 // a word unpacks in the order 0, 4, 1, 5, 2, 6, 3, 7: the same for the activations
 #pragma unroll
                 for (int f = 0; f < 2; ++f) {
@@ -605,7 +608,7 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
         }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            if constexpr (PRE) {
+            if constexpr (BF && PRE) {
                 const float sc = f16_to_f32(*(const unsigned short*)(tr + 32 * j));
                 const v4i b0 = w4_word_to_bf16x8(w[j][0], sc), b1 = w4_word_to_bf16x8(w[j][1], sc);
 #pragma unroll
@@ -615,10 +618,6 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
                 }
                 continue;
             }
-            const uint64_t sw = *(const uint64_t*)(tr + 32 * j);
-            v4f sc;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc[i] = f16_to_f32((unsigned short)(sw >> (16 * i)));
             v4i b[2];
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
@@ -634,6 +633,24 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
                     b[f] = (v4i){(int)lo8(x), (int)hi8(x), (int)lo8(x8), (int)hi8(x8)};
                 }
             }
+            if constexpr (PRE) {
+                const _Float16 s1 = *(const _Float16*)(tr + 32 * j);
+                const v2h s2 = {s1, s1};
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) b[f][i] = (int)w4_as_u32(w4_as_h2((unsigned)b[f][i]) * s2);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    acc[mt][j] = mma(b[0], a[mt][0], acc[mt][j]);
+                    acc[mt][j] = mma(b[1], a[mt][1], acc[mt][j]);
+                }
+                continue;
+            }
+            const uint64_t sw = *(const uint64_t*)(tr + 32 * j);
+            v4f sc;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc[i] = f16_to_f32((unsigned short)(sw >> (16 * i)));
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 v4f t = mma(b[0], a[mt][0], init[mt]);
@@ -929,7 +946,7 @@ constexpr WaveModel WV_MARLIN = {{{1.94f, 1.67f, 1.52f}, {1.76f, 1.81f, 1.64f}, 
 template <int KIND, bool PRE>
 constexpr const WaveModel& wave_model() {
     if constexpr (KIND == K_W4MARLIN) return WV_MARLIN;
-    else if constexpr (KIND == K_W4NK) return WV_NK;
+    else if constexpr (KIND == K_W4NK) return WV_NK;             // (PRE or not)
     else if constexpr (PRE) return WV_NKB_PRE;
     else return WV_NKB;
 }
@@ -1058,7 +1075,7 @@ inline bool w4a8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, Wav
     return wave_plan(M, N, K, scratch, WV_W4A8, [](int nw, int mt, int nt, int per) { return wv_lds(nw, mt, nt, wv_depth(mt, nt, per), per); }, best);
 }
 // 16-bit activations: groups in whole K steps, and a scale table of at least one load
-template <int KIND, bool PRE = false>
+template <int KIND, bool PRE>
 inline bool w4a16_wave_plan(int64_t M, int64_t N, int64_t K, int group, int64_t scratch, WavePlan& best) {
     if (K % 128 || group % 128 || N * (K / group) < 4 || K > (1 << 24) || N * (K / 2) >= (1ll << 40)) return false;
     return wave_plan(M, N, K, scratch, wave_model<KIND, PRE>(), [&](int nw, int mt, int nt, int per) { return wh_lds(KIND, nw, mt, nt, wh_groups((int)K, group, per)); }, best);
@@ -1087,7 +1104,7 @@ inline int launch_w4a8_wave_plan(const DirectArgs& p, const WavePlan& w, hipStre
     return w.mt == 1 ? rows(i1) : (w.mt == 2 ? rows(i2) : (w.mt == 3 ? rows(i3) : rows(i4)));
 }
 
-template <int KIND, bool PRE = false>
+template <int KIND, bool PRE>
 inline int launch_w4a16_wave_plan(const DirectArgs& p, const WavePlan& w, hipStream_t stream, const char* name) {
     auto rows = [&](auto mt) {
         constexpr int MT = decltype(mt)::value;

@@ -394,6 +394,42 @@ def test_mul_wave_kernel(dev, M, N, K, gs, scratch):
     assert (ws[nbytes:] == 0x5A).all()
 
 
+def _row_differences(M, K, gs, dev, dtype):
+    """One +1 and one -1 a row, in the same group of K: the product is the difference of two weights of a column, exact in fp32."""
+    x = torch.zeros(M, K, dtype=dtype, device=dev)
+    m, g0 = torch.arange(M, device=dev), torch.randint(0, K // gs, (M,), device=dev) * gs
+    i = torch.randint(0, gs, (M,), device=dev)
+    x[m, g0 + i] = 1.0
+    x[m, g0 + (i + 1 + torch.randint(0, gs - 1, (M,), device=dev)) % gs] = -1.0
+    return x
+
+
+@pytest.mark.parametrize("M,N,K,gs", [(16, 4096, 4096, 128), (16, 64, 8320, 128), (48, 8256, 640, 128), (64, 12352, 128, 128), (80, 320, 1152, 384),
+                                      (256, 1088, 640, 128), (512, 4096, 1024, 128), (528, 1088, 640, 128)])
+def test_mul_multiplies_the_fake_quantised_weights(dev, M, N, K, gs):
+    """Whatever the number of rows: (q - 8) * s rounded to fp16 once, as fake_quantize gives it and the reference's kernel forms it."""
+    announce("marlin weights", M, N, K, gs)
+    torch.manual_seed(M + N + K)
+    W, qw, s = QuantUtils.fake_quantize((torch.randn(K, N, device=dev) * 0.02).half(), gs)
+    A = _row_differences(M, K, gs, dev, torch.float16)
+    C = torch.full((M, N), 7.0, dtype=torch.half, device=dev)
+    B, sp = QuantUtils.pack(qw, s, gs)
+    mul(A, B, C, sp, torch.zeros(N // 128 * 16 + 16, dtype=torch.int32, device=dev))
+    assert torch.equal(C, (A.double() @ W.double()).half())
+
+
+@pytest.mark.parametrize("M,N,K,gs", [(48, 4096, 8192, 128), (65, 2056, 1152, 128), (100, 4104, 1024, 128), (97, 1000, 1024, 256), (250, 1032, 640, 128),
+                                      (512, 4096, 1024, 128), (520, 1032, 640, 128)])
+def test_w4a16_nk_rounded_weights(dev, M, N, K, gs):
+    """fp16 beyond 64 rows (and from 33 on large weights): the weights rounded to fp16 in whichever kernel is taken."""
+    announce("w4a16 nk weights", M, N, K, gs)
+    torch.manual_seed(M + N + K)
+    packed, s, qn = w4a16.quantize_nk((torch.randn(N, K, device=dev) * 0.02).half(), gs)
+    W = ((qn.float() - 8).half() * s.repeat_interleave(gs, 1)).T.contiguous()
+    x = _row_differences(M, K, gs, dev, torch.float16)
+    assert torch.equal(w4a16.w4a16_gemm(x, packed, s, gs), (x.double() @ W.double()).half())
+
+
 @pytest.mark.parametrize("M,N,K,gs", [(65, 72, 128, 64), (130, 4096, 1024, 128), (512, 264, 4096, 128), (300, 14344, 512, 128),
                                       (200, 20000, 640, 128), (500, 8192, 384, 192), (600, 10000, 1024, 128), (1024, 28672, 256, 128)])
 def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
