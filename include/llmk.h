@@ -186,7 +186,7 @@ int llmk_quant_w4_nk(const void* w, int w_dtype, int32_t* packed, void* scales_f
                      int64_t K, int group, void* stream);
 /* Same product for W stored [N, K/8] int32 by pack_weights_over_cols (nibble i of a word = k*8+i)
  * with s fp16 [N, K/g]; a/c fp16 or bf16 (ac_dtype).  What the weights are depends on the shape alone: beyond 64 rows (fp16: also
- * from 33 rows where the weight matrix is large) (nibble - 8) * s
+ * from 33 rows where the weight matrix is large; bf16: also where groups are not 128 wide or K is below 512) (nibble - 8) * s
  * rounded to the type of a, otherwise nibble - 8 exactly with s on the fp32 sums of a group.  workspace: llmk_gemm_w4a16_nk_workspace_bytes(...) bytes, 16-byte
  * aligned, is what the path chosen for the shape uses:
  *   - M <= 64 streams the weights: nothing for K <= 4096, fp32 partial sums of K ranges, ceil(K/4096)*M*N*4, beyond;

@@ -981,16 +981,18 @@ double nk_other_estimate(const llmk::DirectArgs& p) {
 }
 // What the weights of a call are, by its shape alone: (q - 8) * scale rounded to the activations' type, as in the tile kernels and in
 // the 16-bit copy of W, or q - 8 exactly with the scale on fp32 sums, as in the streaming kernels.  The wave kernel has both and
-// takes what those have that it stands in for: a row's result then does not hang on which kernel is faster.
-bool nk_rounded_weights(int64_t M, int64_t N, int64_t K, bool bf) {
+// takes what those have that it stands in for: a row's result then does not hang on which kernel is faster, and a bf16 call
+// that the ring kernel never took keeps its infinities (an infinite activation times -136, where the exact sums start, is a NaN).
+bool nk_rounded_weights(int64_t M, int64_t N, int64_t K, int group, bool bf) {
     if (M > 64) return true;
-    return !bf && w4_tiles_expand(M, N, K, INT64_MAX, true);
+    const int nz = (int)((K / 128 + 31) / 32);
+    return bf ? !nk_ring_ok(M, N, K, group, nz) || (nz > 1 && (M * N) % 4) : w4_tiles_expand(M, N, K, INT64_MAX, true);
 }
 // The wave kernel for this call, or z = 0: taken 8 % below the others' estimate.
 template <int KIND>
 llmk::WavePlan nk_wave(const llmk::DirectArgs& p, int64_t scratch) {
     llmk::WavePlan w{0, 0, 0, 0, 0.0};
-    const bool fits = nk_rounded_weights(p.M, p.N, p.K, KIND == llmk::K_W4NKB) ? llmk::w4a16_wave_plan<KIND, true>(p.M, p.N, p.K, p.group, scratch, w)
+    const bool fits = nk_rounded_weights(p.M, p.N, p.K, p.group, KIND == llmk::K_W4NKB) ? llmk::w4a16_wave_plan<KIND, true>(p.M, p.N, p.K, p.group, scratch, w)
                                                                                        : llmk::w4a16_wave_plan<KIND, false>(p.M, p.N, p.K, p.group, scratch, w);
     if (!fits || 1.08 * w.cost >= nk_other_estimate<KIND>(p)) w.z = 0;
     return w;
@@ -1210,7 +1212,7 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
     switch (pl.route) {
         case NkPlan::WAVE:
             p.b = (const uint8_t*)b_packed; p.b_s = s; p.group = groupsize; p.partial = (float*)workspace;
-            if (nk_rounded_weights(M, N, K, bf))
+            if (nk_rounded_weights(M, N, K, groupsize, bf))
                 return bf ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)")
                           : llmk::launch_w4a16_wave_plan<llmk::K_W4NK, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
             return bf ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, false>(p, pl.wave, st, "gemm_w4a16_nk(wave)")

@@ -430,6 +430,22 @@ def test_w4a16_nk_rounded_weights(dev, M, N, K, gs):
     assert torch.equal(w4a16.w4a16_gemm(x, packed, s, gs), (x.double() @ W.double()).half())
 
 
+@pytest.mark.parametrize("M,N,K,gs", [(33, 20008, 128, 128), (40, 14344, 256, 128), (64, 8200, 384, 128), (31, 4104, 1152, 384), (97, 1032, 640, 128)])
+def test_w4a16_nk_bf16_infinite_activations(dev, M, N, K, gs):
+    """bf16 calls outside the ring kernel's shapes (128-wide groups, at least 512 of K): an infinite activation is an infinite output
+    of its sign, or NaN where the weight is zero, and reaches its own row only."""
+    announce("w4a16 nk bf16 infinities", M, N, K, gs)
+    torch.manual_seed(M + N + K)
+    x = torch.randint(-2, 3, (M, K), device=dev).to(torch.bfloat16)
+    qn = torch.randint(0, 16, (N, K), dtype=torch.uint8)
+    s = torch.exp2(torch.randint(-4, 1, (N, K // gs)).float()).half().to(dev)
+    packed = torch.from_numpy(bp.pack_cols(qn.numpy(), 4, 32)[0]).to(dev)
+    w = ((qn.to(dev).double() - 8) * s.double().repeat_interleave(gs, 1)).T.contiguous()
+    x[1, K - 1], x[2, 5] = float("inf"), float("-inf")
+    ref = (x.double() @ w).to(torch.bfloat16)
+    assert torch.allclose(w4a16.w4a16_gemm(x, packed, s, gs).float(), ref.float(), rtol=0, atol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("M,N,K,gs", [(65, 72, 128, 64), (130, 4096, 1024, 128), (512, 264, 4096, 128), (300, 14344, 512, 128),
                                       (200, 20000, 640, 128), (500, 8192, 384, 192), (600, 10000, 1024, 128), (1024, 28672, 256, 128)])
 def test_w4a16_nk_bf16_expanding_tiles(dev, M, N, K, gs):
