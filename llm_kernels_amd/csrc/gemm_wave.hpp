@@ -397,6 +397,27 @@ constexpr int wh_groups(int K, int group, int per) {
     return a < b ? a : b;
 }
 
+// Scales of a row-packed tile are loaded four at a time (8 bytes) at the offset of the first one, but no further than the end of the
+// table: a load there starts earlier and is shifted.  A last tile of fewer than four scales (one column and groups as long as K, say)
+// has its loads start in front of its own first column: `back` bytes, for a table of at least four scales in all (w4a16_wave_plan).
+struct WhTable {
+    int64_t back, last;          // bytes in front of the tile's first scale; offset (from there) of the last load
+};
+__host__ __device__ constexpr WhTable wh_table(int64_t scales) {       // from the tile's first column to the end of the table
+    const int64_t bytes = 2 * scales, back = bytes < 8 ? 8 - bytes : 0;
+    return {back, bytes + back - 8};
+}
+constexpr bool wh_table_covers(int64_t scales) {
+    const WhTable t = wh_table(scales);
+    for (int64_t i = 0; i < scales; ++i) {
+        const int64_t want = t.back + 2 * i, at = want < t.last ? want : t.last;
+        if (at < 0 || at + 8 > t.back + 2 * scales || want - at > 6) return false;
+    }
+    return true;
+}
+static_assert(wh_table_covers(1) && wh_table_covers(2) && wh_table_covers(3) && wh_table_covers(4) && wh_table_covers(5) && wh_table_covers(63),
+              "every load of scales ends inside the table and holds its scale");
+
 // PRE: the weights are (q - 8) * scale rounded to the activations' type, as the tile kernels of larger M have them (and the
 // reference's Marlin kernel: marlin_w4a16_gemm.cu:152-236), and sums run over all of K; otherwise they are q - 8 exactly and the scale
 // multiplies the fp32 sums of a half step.  Marlin words always, row-packed ones where the caller's rule says so.  (us, weights from
@@ -434,8 +455,9 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
     // ---- group scales of the tile, requested first (four per load)
     const int g_lo = kt0 * 128 / p.group, GR = ((kt0 + KT) * 128 - 1) / p.group - g_lo + 1;
     const int W = (GR + 3) >> 2, tab_n = MARLIN ? GR * 16 : BN * W;
-    const uint8_t* const tabp = (const uint8_t*)p.b_s + (MARLIN ? ((int64_t)g_lo * N + chunk * 64) * 2 : (int64_t)n0 * G * 2);
-    const uint32_t tab_last = (uint32_t)min((int64_t)(N - n0) * G * 2 - 8, (int64_t)0x7fffffff);
+    const WhTable range = wh_table((int64_t)(N - n0) * G);
+    const uint8_t* const tabp = (const uint8_t*)p.b_s + (MARLIN ? ((int64_t)g_lo * N + chunk * 64) * 2 : (int64_t)n0 * G * 2 - range.back);
+    const uint32_t tab_last = (uint32_t)min(range.last, (int64_t)0x7fffffff), tab_back = (uint32_t)range.back;
     auto tab_at = [&](int idx, int& col, int& w, int& shift) {
         if constexpr (MARLIN) {                              // col: unit of four scales, w: group
             w = min(idx >> 4, GR - 1);
@@ -445,7 +467,7 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
         } else {
             col = idx / W;
             w = idx - col * W;
-            const uint32_t want = ((uint32_t)min(min(col, BN - 1), N - 1 - n0) * (uint32_t)G + (uint32_t)(g_lo + 4 * w)) * 2u;
+            const uint32_t want = ((uint32_t)min(min(col, BN - 1), N - 1 - n0) * (uint32_t)G + (uint32_t)(g_lo + 4 * w)) * 2u + tab_back;
             const uint32_t at = min(want, tab_last);
             shift = (int)(want - at) * 8;
             return at;

@@ -374,6 +374,14 @@ def test_w4a16_nk_wave_kernel(dev, dtype, M, N, K, gs):
         assert torch.equal(y[:1], ref[:1]) and torch.equal(y[2:], ref[2:]) and torch.equal(y[1].isfinite(), ref[1].isfinite())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,gs", [(64, 8193, 128, 128), (33, 8193, 256, 256), (80, 1025, 256, 128), (97, 4097, 384, 128), (65, 33, 128, 128),
+                                      (97, 1025, 1152, -1), (160, 1026, 640, 640), (65, 3001, 640, 128), (100, 2051, 128, 128)])
+def test_w4a16_nk_wave_kernel_last_columns(dev, dtype, M, N, K, gs):
+    """A last tile of one to three columns and one to five groups: its few scales, at the very end of the table, reach their columns."""
+    test_w4a16_nk_wave_kernel(dev, dtype, M, N, K, gs)
+
+
 @pytest.mark.parametrize("M,N,K,gs", WAVE_MARLIN)
 @pytest.mark.parametrize("scratch", [True, False])
 def test_mul_wave_kernel(dev, M, N, K, gs, scratch):
