@@ -200,6 +200,16 @@ int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* c, const vo
                        int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize,
                        void* workspace, int64_t workspace_bytes, void* stream);
 
+/* ------------------------------------------------------------------ launch shapes of the dense products, for tests and profiles
+ * What a call with scratch_bytes of scratch gets where it runs on the kernels whose waves stream their own share of K (up to 512
+ * rows): returns 1 and shape = {waves of a workgroup, 16-row tiles, 16-column tiles, K slices, form}, else 0.  form: stages of a wave
+ * (8-bit activations), 1 / 0: rounded / exact weights (16-bit ones).  No device is needed.
+ * 8bit: kind LLMK_KIND_FP8 or LLMK_KIND_I8, per_token: llmk_gemm_i8_rowcol.  w4a16: marlin 1 or [N, K/8] 0 with activations of ac_dtype. */
+int llmk_gemm_8bit_wave_shape(int kind, int per_token, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes, int32_t* shape);
+int llmk_gemm_w4a8_wave_shape(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch_bytes, int32_t* shape);
+int llmk_gemm_w4a16_wave_shape(int marlin, int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes,
+                               int32_t* shape);
+
 /* ------------------------------------------------------------------ converters and the one-tile MFMA GEMM
  * ref: fast_dequant/fast_dtype_convert/fast_uint4_to_fp16.cu:21-109,112-127 (out[i] = nibble_i - 8, nibble i
  *      of word w at bits 4i; the natural order of the reference's "simple" kernel),

@@ -55,13 +55,17 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
 // int8 29 x 4096 x 4096 5.1 | 8.5, fp8 64 x 4096 x 4096 6.2 | 9.4, fp8 200 x 1032 x 7168 7.6 | 15.1, per token 250 x 4096 x 14336 25.1 |
 // 28.1, but fp8 250 x 4096 x 14336 30.6 | 29.2, and from 513 rows on 0.8 times as fast.
 template <int KIND>
-WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspace_bytes) {
+WavePlan wave_choice(const DirectArgs& p, int64_t scratch, bool tiles_scratch) {
     WavePlan w{0, 0, 0, 0, 0.0};
-    const int64_t scratch = workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0;
     if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w)) w.nw = 0;
     const double margin = KIND != K_I8_ROWCOL && p.M > 128 ? 1.16 : 1.08;
-    if (w.nw && p.M > 16 && margin * w.cost >= tiles_estimate<KIND>(p, workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K))) w.nw = 0;
+    if (w.nw && p.M > 16 && margin * w.cost >= tiles_estimate<KIND>(p, tiles_scratch)) w.nw = 0;
     return w;
+}
+template <int KIND>
+WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspace_bytes) {
+    return wave_choice<KIND>(p, workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0,
+                             workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K));
 }
 template <int KIND>
 int launch_block(const DirectArgs& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, const char* name) {
@@ -92,6 +96,16 @@ extern "C" int64_t llmk_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     // more than 512 rows and at least W_TAIL_MIN_KT K steps of 128 bytes (shorter tiles are never split): room for
     // the partial sums of a split last round of 256-column tiles behind the rest
     return workspace_core_bytes(M, N, K) + (K >= W_TAIL_MIN_KT * 128 && M > 512 ? w_tail_bytes() : 0);
+}
+
+extern "C" int llmk_gemm_8bit_wave_shape(int kind, int per_token, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes, int32_t* shape) {
+    if (!shape || M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+    DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
+    const bool full = scratch_bytes > 0 && scratch_bytes >= llmk_gemm_workspace_bytes(M, N, K);
+    const WavePlan w = kind == LLMK_KIND_FP8 ? wave_choice<K_FP8_BLOCK>(p, scratch_bytes, full)
+                                             : (per_token ? wave_choice<K_I8_ROWCOL>(p, scratch_bytes, full) : wave_choice<K_I8_BLOCK>(p, scratch_bytes, full));
+    return w.nw ? wave_shape(w, w8_depth(w.mt, w.nt, (int)(((K >> 7) + w.z - 1) / w.z)), shape) : 0;
 }
 
 extern "C" int llmk_gemm_fp8_block(const void* a, const float* a_s, const void* b, const float* b_s, void* c,

@@ -1094,6 +1094,20 @@ extern "C" int64_t llmk_gemm_w4a16_marlin_workspace_bytes(int64_t M, int64_t N, 
     return std::max(slices, z > 1 ? z * M * N * 4 : 0);
 }
 
+extern "C" int llmk_gemm_w4a16_wave_shape(int marlin, int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes,
+                                          int32_t* shape) {
+    if (!shape || M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
+    if (groupsize == -1) groupsize = (int)K;
+    if (groupsize < 8 || K % groupsize) return 0;
+    if (marlin) {
+        const llmk::WavePlan w = marlin_wave(M, N, K, groupsize, scratch_bytes);
+        return w.z > 0 ? llmk::wave_shape(w, 1, shape) : 0;
+    }
+    const bool bf = ac_dtype == LLMK_BF16;
+    const NkPlan pl = nk_plan(M, N, K, groupsize, bf, scratch_bytes, true);
+    return pl.route == NkPlan::WAVE ? llmk::wave_shape(pl.wave, nk_rounded_weights(M, N, K, groupsize, bf), shape) : 0;
+}
+
 extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, const void* s, int64_t M, int64_t N,
                                       int64_t K, int groupsize, void* workspace, int64_t workspace_bytes,
                                       void* stream) {

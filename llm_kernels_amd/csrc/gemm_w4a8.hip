@@ -95,6 +95,11 @@ extern "C" int64_t llmk_gemm_w4a8_workspace_bytes(int64_t M, int64_t N, int64_t 
     return w4a8_plan(M, N, K, group_int4, INT64_MAX).bytes;
 }
 
+extern "C" int llmk_gemm_w4a8_wave_shape(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch_bytes, int32_t* shape) {
+    const W4A8Plan pl = w4a8_plan(M, N, K, group_int4, scratch_bytes);
+    return pl.wave && shape ? wave_shape(pl.shape, wv_depth(pl.shape.mt, pl.shape.nt, ((K >> 7) + pl.shape.z - 1) / pl.shape.z), shape) : 0;
+}
+
 extern "C" int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b_packed, const void* b_s, int s_dtype,
                               const int8_t* b_s4, const int8_t* b_z4, void* c, int c_dtype, int64_t M, int64_t N,
                               int64_t K, int group_int4, void* workspace, int64_t workspace_bytes, void* stream) {

@@ -936,6 +936,12 @@ struct WavePlan {
     double cost;
 };
 
+inline int wave_shape(const WavePlan& w, int form, int32_t* shape) {
+    const int32_t v[5] = {w.nw, w.mt, w.nt, w.z, form};
+    for (int i = 0; i < 5; ++i) shape[i] = v[i];
+    return 1;
+}
+
 // Estimated microseconds of a launch without its K slices' sums.  Eight waves: base + rounds of 256 workgroups x (fixed + K steps
 // of a wave x step).  Four waves (64 columns): several workgroups share a CU and cover each other's prologue and reduction, so
 // their rounds count in fractions; slower on a single round (w4a8 64 x 14336 x 4096 18.2 against 17.0 us), faster from two on

@@ -235,7 +235,7 @@ def test_w4a8_mid_m_fused_tiles_exact_mixed_wrap(dev, M, N, K, sdt):
     assert torch.equal(c.cpu().long(), (a.double() @ b8.double().T).long())      # exact: every sum is far below 2^53
 
 
-@pytest.mark.parametrize("M,N,K,sdt", [
+WAVE_W4A8 = [
     # every tile shape of the kernel whose waves stream their own K share, with ragged rows and columns and K steps that do
     # not divide by the waves: 16 rows x 16, 32 and 64 columns, then 32, 48 and 64 rows
     (7, 1048, 1152, torch.float16), (16, 4104, 2176, torch.float32), (5, 14344, 1280, torch.bfloat16),
@@ -244,7 +244,13 @@ def test_w4a8_mid_m_fused_tiles_exact_mixed_wrap(dev, M, N, K, sdt):
     # four waves, more than one round of workgroups
     (50, 24008, 1152, torch.float16), (95, 28680, 640, torch.float32), (256, 4104, 1152, torch.bfloat16),
     # K slices; tables of more than one round of loads; more K steps than one workgroup takes
-    (1, 72, 16384, torch.float16), (40, 264, 33024, torch.float32), (20, 136, 65664, torch.float16), (300, 4104, 1024, torch.float16)])
+    (1, 72, 16384, torch.float16), (40, 264, 33024, torch.float32), (20, 136, 65664, torch.float16), (300, 4104, 1024, torch.float16),
+    # 16 rows x 32 columns, one stage; 32 to 64 rows x 16, 48 rows x 32
+    (1, 4184, 128, torch.bfloat16), (90, 1352, 256, torch.float32), (34, 4096, 2176, torch.float16), (49, 3096, 2176, torch.bfloat16),
+    (33, 31960, 1664, torch.float32)]
+
+
+@pytest.mark.parametrize("M,N,K,sdt", WAVE_W4A8)
 @pytest.mark.parametrize("scratch", [True, False])
 def test_w4a8_wave_kernel_exact(dev, M, N, K, sdt, scratch):
     """Unit block scales, fp32 out, wild (s4, z4): exact integers (every sum is below 2^24), with the reported scratch and without."""
@@ -280,7 +286,9 @@ WAVE_8BIT = [
     (509, 1712, 1536), (467, 1720, 1920), (508, 792, 6656), (344, 2704, 1792), (504, 4320, 1536), (357, 3424, 3584), (351, 5424, 1280),
     # two stages in flight; K slices (without scratch: a scale table of more than one round of loads, and one that leaves room for one
     # stage only)
-    (9, 264, 8192), (40, 136, 66688), (2, 24, 3276800)]
+    (9, 264, 8192), (40, 136, 66688), (2, 24, 3276800),
+    # 48 and 64 rows x 64 columns with eight and with four waves, 48 rows x 32
+    (33, 8225, 768), (49, 8203, 3072), (33, 57445, 128), (49, 90485, 128), (33, 5443, 640)]
 
 
 @pytest.mark.parametrize("M,N,K", WAVE_8BIT)

@@ -247,7 +247,10 @@ def test_w4a16_nk_large_tile_shapes(dev, M, N, K, gs):
     assert_close_scaled(y, ref, what="w4a16 nk large tiles")
 
 
-@pytest.mark.parametrize("M,N,K", [(128, 1024, 4096), (48, 4096, 14336), (300, 520, 1152), (16, 264, 8320)])
+WITHOUT_SCRATCH = [(128, 1024, 4096), (48, 4096, 14336), (300, 520, 1152), (16, 264, 8320), (49, 4160, 9472)]
+
+
+@pytest.mark.parametrize("M,N,K", WITHOUT_SCRATCH)
 def test_w4a16_without_scratch(dev, M, N, K):
     """The scratch of both w4a16 entry points is optional: without it the kernels run with one K slice (or the
     weight-streaming variant) and must agree with the oracle all the same."""
@@ -346,7 +349,11 @@ WAVE_NK = [(17, 8200, 4224, 128), (64, 8200, 128, 128), (33, 20008, 128, 128), (
            (97, 1032, 1152, 128), (65, 3000, 640, 128), (128, 520, 256, 128), (65, 2056, 1152, 128), (70, 4104, 896, 128),
            (97, 1032, 384, 128), (250, 1032, 640, 128), (100, 4104, 1024, 128), (97, 3000, 896, 128), (49, 12296, 640, 128),
            (17, 12296, 128, 128), (33, 4104, 4224, 128), (31, 14344, 1152, 128), (40, 6152, 2176, 128), (49, 14344, 896, 128),
-           (160, 1032, 640, 128), (100, 6152, 1024, 128), (97, 1000, 1152, 384), (80, 520, 2048, -1)]
+           (160, 1032, 640, 128), (100, 6152, 1024, 128), (97, 1000, 1152, 384), (80, 520, 2048, -1),
+           # the tiles that only exact weights or only rounded ones of the two types get with shapes like these
+           (34, 4096, 2176, 128), (33, 31960, 1664, 128), (17, 64, 4224, 128), (17, 2096, 4224, 128), (49, 7312, 512, 128),
+           (33, 2112, 4224, 128), (49, 3096, 2176, 128), (49, 4248, 9344, 128), (66, 64, 2176, 128), (17, 34824, 128, 128),
+           (162, 1352, 512, 128), (33, 2768, 4352, 128), (17, 8312, 4224, 128), (33, 4104, 4224, 128)]
 WAVE_MARLIN = [(32, 8256, 128, 128), (16, 4160, 8320, 128), (64, 12352, 128, 128), (32, 4160, 8320, 128), (48, 14400, 128, 128),
                (48, 8256, 8320, 128), (16, 64, 128, 128), (16, 64, 8320, 128), (16, 4160, 128, 128), (48, 576, 8320, 128),
                (16, 8256, 1152, 128), (32, 2112, 1152, 128), (32, 4160, 1152, 128), (32, 14400, 128, 128), (48, 3008, 1152, 128),

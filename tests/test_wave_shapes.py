@@ -1,0 +1,53 @@
+"""The shapes of the GPU tests of the kernels whose waves stream their own K share reach every tile that these kernels are built with."""
+import ctypes
+
+import torch
+
+from llm_kernels_amd import _lib
+from test_gpu_gemm import WAVE_8BIT, WAVE_W4A8
+from test_gpu_w4a16 import WAVE_MARLIN, WAVE_NK, WITHOUT_SCRATCH
+
+MUCH = 1 << 50
+
+
+def shape(name, *args):
+    """(waves, 16-row tiles, 16-column tiles, form) of a call, or None where it goes to another kernel."""
+    out = (ctypes.c_int32 * 5)()
+    if not getattr(_lib.load(), "llmk_gemm_%s_wave_shape" % name)(*args, ctypes.cast(out, ctypes.c_void_p)):
+        return None
+    return out[0], out[1], out[2], out[4]
+
+
+def eight(form, *but):
+    """Eight waves, 16 to 64 rows x 16, 32 or 64 columns."""
+    return {(8, mt, nt, form) for mt in (1, 2, 3, 4) for nt in (1, 2, 4) if (mt, nt) not in but}
+
+
+def four(form, *mt):
+    return {(4, m, 4, form) for m in mt}
+
+
+def test_8bit():
+    built = eight(1, (3, 1), (4, 1)) | four(1, 2, 3, 4) | {(8, 1, 1, 2)}
+    for kind, per_token in ((_lib.KIND_FP8, 0), (_lib.KIND_I8, 0), (_lib.KIND_I8, 1)):
+        got = set()
+        for M, N, K in WAVE_8BIT:
+            got.add(shape("8bit", kind, per_token, M, N, K, _lib.load().llmk_gemm_workspace_bytes(M, N, K)))
+        assert got - {None} == built, (kind, per_token, built - got)
+
+
+def test_w4a8():
+    built = eight(1) | four(1, 3, 4) | {(8, 1, 1, 2), (8, 1, 2, 2)}
+    got = {shape("w4a8", M, N, K, 128, scratch) for M, N, K, _ in WAVE_W4A8 for scratch in (MUCH, 0)}
+    assert got - {None} == built, built - got
+
+
+def test_w4a16():
+    got = {shape("w4a16", 1, _lib.F16, M, N, K, gs, scratch) for M, N, K, gs in WAVE_MARLIN for scratch in (MUCH, 0)}
+    built = eight(1, (4, 1), (4, 2)) | four(1, 1, 2, 3)
+    assert got - {None} == built, ("marlin", built - got)
+    for dt, built in ((_lib.F16, eight(0, (1, 4), (4, 1)) | four(0, 1, 2, 3) | eight(1) | four(1, 1, 2, 3)),
+                      (_lib.BF16, eight(0, (4, 1)) | four(0, 1, 2, 3) | eight(1, (1, 2), (1, 4)) | four(1, 2, 3))):
+        got = {shape("w4a16", 0, dt, M, N, K, gs, MUCH) for M, N, K, gs in WAVE_NK}
+        got |= {shape("w4a16", 0, dt, M, N, K, 128, 0) for M, N, K in WITHOUT_SCRATCH if dt == _lib.F16}
+        assert got - {None} == built, (dt, built - got, got - built)
