@@ -32,7 +32,7 @@ __global__ void w4a8_expand_kernel(const int32_t* __restrict__ packed, const int
     const int64_t kq = K / 4;
     if (idx >= (N / 8) * kq) return;
     const int64_t pr = idx / kq, k = (idx - pr * kq) * 4;
-    const v4i w = *(const v4i*)(packed + pr * K + k);
+    const v4i w = ((const Loose<v4i, 4>*)(packed + pr * K + k))->v;          // (a view of the words at any offset)
     const int64_t kg = K / group;
     const int64_t gi = k / group;
 #pragma unroll
@@ -74,19 +74,25 @@ inline int64_t w4a8_widened_bytes(int64_t M, int64_t N, int64_t K) {
 W4A8Plan w4a8_plan(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch) {
     W4A8Plan pl{false, {}, 0};
     if (M <= 0 || N <= 0 || K <= 0) return pl;
+    DirectArgs q{};
     if (group_int4 == 128 && M <= 512 && N <= 0x7fffffff && K <= (1 << 25) && w4a8_wave_plan(M, N, K, scratch, pl.shape)) {
+        q.M = (int)M; q.N = (int)N; q.K = (int)K; q.E = 1;
         pl.wave = M <= 128;
         if (!pl.wave) {
-            DirectArgs q{};
-            q.M = (int)M; q.N = (int)N; q.K = (int)K; q.E = 1;
             const double two = 10.0 + (double)N * K * 0.41e-6 + 0.72 * dma_tile_estimate<K_I8_BLOCK, false>(q).cost * K / 4096.0;
             pl.wave = 1.12 * pl.shape.cost < two;
         }
     }
     const int64_t slices = pl.wave && pl.shape.z > 1 ? (int64_t)pl.shape.z * M * N * 4 : 0;
+    const int64_t two_pass = w4a8_two_pass_scales_off(N, K) + w4a8_widened_bytes(M, N, K) + llmk_gemm_workspace_bytes(M, N, K);
+    // Words that do not start on 16 bytes go through the two passes.  Callers who pass what is reported may have such words with any
+    // shape but those of few rows or few tiles, whose scratch stays small: 64 rows, 128 with K up to 32768, 256 on one 64-column
+    // workgroup a CU with K up to 16384.
+    const bool small = M <= 64 || ((M <= 128 || (M <= 256 && mid_plan(M, N, K).tiles <= LLMK_CUS && K <= 16384)) && dma_eligible(q));
     // (from 17 rows on at least what the int8 GEMM of the shape can use, so that one buffer serves both)
-    if (pl.wave) pl.bytes = M <= 16 ? slices : std::max(slices, llmk_gemm_workspace_bytes(M, N, K));
-    else pl.bytes = w4a8_two_pass_scales_off(N, K) + w4a8_widened_bytes(M, N, K) + llmk_gemm_workspace_bytes(M, N, K);
+    if (!pl.wave) pl.bytes = two_pass;
+    else if (!small) pl.bytes = std::max(slices, two_pass);
+    else pl.bytes = M <= 16 ? slices : std::max(slices, llmk_gemm_workspace_bytes(M, N, K));
     return pl;
 }
 }  // namespace

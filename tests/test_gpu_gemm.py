@@ -277,6 +277,28 @@ def test_w4a8_wave_kernel_exact(dev, M, N, K, sdt, scratch):
     assert torch.equal(c.double(), ref)
 
 
+W4A8_ANY_WORDS = [(300, 4104, 1024), (200, 8200, 512), (512, 520, 2048), (100, 264, 33024)]
+
+
+@pytest.mark.parametrize("M,N,K", W4A8_ANY_WORDS)
+def test_w4a8_words_at_any_offset(dev, M, N, K):
+    """A view of packed words that starts on 4 bytes only: the two passes, in the scratch that the operator allocates."""
+    announce("w4a8 words at any offset", M, N, K)
+    torch.manual_seed(M + N)
+    wq = torch.randint(0, 16, (N, K), dtype=torch.uint8)
+    s4, z4 = (torch.randint(-128, 128, (N, K // 128), dtype=torch.int8) for _ in range(2))
+    a = (torch.rand(M, K) < 64.0 / K).to(torch.int8) * torch.randint(-128, 128, (M, K), dtype=torch.int8)
+    packed = torch.from_numpy(bp.pack_rows(wq.numpy(), 4, 32)[0])
+    words = torch.zeros(packed.numel() + 1, dtype=torch.int32, device=dev)[1:].view(packed.shape)
+    words.copy_(packed)
+    assert words.data_ptr() % 16 == 4
+    ones_a, ones_b = torch.ones(M, K // 128, dtype=torch.float16, device=dev), torch.ones((N + 127) // 128, K // 128, dtype=torch.float16, device=dev)
+    with default_dtype(torch.float32):
+        c = w4a8_kernel.w4a8_gemm(a.to(dev), ones_a, words, ones_b, s4.to(dev), z4.to(dev))
+    ref = a.to(dev).double() @ q.w4a8_dequant_int8(wq, s4, z4).to(dev).double().T
+    assert ref.abs().max() < 2 ** 24 and torch.equal(c.double(), ref)
+
+
 WAVE_8BIT = [
     # every tile shape of the kernel whose waves stream their own K share (eight waves 16 to 64 rows x 16 to 64 columns, four waves
     # 32 to 64 rows x 64), with ragged rows and columns and K steps that do not divide by the waves

@@ -4,7 +4,7 @@ import ctypes
 import torch
 
 from llm_kernels_amd import _lib
-from test_gpu_gemm import WAVE_8BIT, WAVE_W4A8
+from test_gpu_gemm import W4A8_ANY_WORDS, WAVE_8BIT, WAVE_W4A8
 from test_gpu_w4a16 import WAVE_MARLIN, WAVE_NK, WITHOUT_SCRATCH
 
 MUCH = 1 << 50
@@ -51,3 +51,9 @@ def test_w4a16():
         got = {shape("w4a16", 0, dt, M, N, K, gs, MUCH) for M, N, K, gs in WAVE_NK}
         got |= {shape("w4a16", 0, dt, M, N, K, 128, 0) for M, N, K in WITHOUT_SCRATCH if dt == _lib.F16}
         assert got - {None} == built, (dt, built - got, got - built)
+
+
+def test_w4a8_reports_the_two_passes():
+    """Where the operator has always had scratch for an expanded copy, words that are not 16-byte aligned rely on it."""
+    for M, N, K in W4A8_ANY_WORDS:
+        assert shape("w4a8", M, N, K, 128, MUCH) and _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128) >= N * K
