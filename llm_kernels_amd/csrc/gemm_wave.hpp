@@ -988,6 +988,9 @@ constexpr const WaveModel& wave_model() {
     else return WV_NKB;
 }
 
+// A launch has fewer than 2^32 threads.
+constexpr bool wv_grid_ok(int64_t tiles, int nw) { return tiles * nw * 64 <= 0xffffffffll; }
+
 // The cheapest shape whose LDS (bytes(nw, mt, nt, K steps of a workgroup)) and scratch fit; K slices cost a second launch and
 // their fp32 sums.
 template <class Bytes>
@@ -1011,7 +1014,7 @@ inline bool wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, const Wa
                     if (nw == 8) cost = m.base8[mt - 1][j] + (double)((wgs + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[mt - 1][j] + steps8 * m.step8[mt - 1][j]);
                     else cost = m.base4[mt - 1] + (wgs > LLMK_CUS ? (double)wgs / LLMK_CUS : 1.0) * steps4 * m.step4[mt - 1];
                     if (z > 1) cost += 3.0 + z * us_sum;
-                    if ((found && cost >= best.cost) || bytes(nw, mt, 1 << j, per) > D_LDS_MAX) continue;
+                    if ((found && cost >= best.cost) || bytes(nw, mt, 1 << j, per) > D_LDS_MAX || !wv_grid_ok(ct[j] * rt, nw)) continue;
                     best = WavePlan{nw, mt, 1 << j, z, cost};
                     found = true;
                 }
@@ -1050,12 +1053,12 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
         for (int mt = 1; mt <= 4 && (mt == 1 || M > 16 * (mt - 1)); ++mt) {
             const int64_t rt = (M + 16 * mt - 1) / (16 * mt);
             for (int j = mt > 2; j < 3; ++j) {               // (16 columns with more than 32 rows: never the cheapest)
-                const int64_t rounds = (((N + (16 << j) - 1) >> (4 + j)) * rt * z + LLMK_CUS - 1) / LLMK_CUS;
+                const int64_t tiles = ((N + (16 << j) - 1) >> (4 + j)) * rt, rounds = (tiles * z + LLMK_CUS - 1) / LLMK_CUS;
                 for (int nw = 8; nw >= 4; nw -= 4) {
                     if (nw == 4 && (j < 2 || m.step4[mt - 1] == 0.f)) continue;
                     const double cost = slices + (nw == 8 ? m.base8[mt - 1][j] + (double)rounds * (m.fixed8[mt - 1][j] + steps8 * m.step8[mt - 1][j])
                                                           : m.base4[mt - 1] + (double)rounds * steps4 * m.step4[mt - 1]);
-                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT), KT) > D_LDS_MAX) continue;
+                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT), KT) > D_LDS_MAX || !wv_grid_ok(tiles, nw)) continue;
                     best = WavePlan{nw, mt, 1 << j, z, cost};
                     found = true;
                 }
@@ -1071,7 +1074,7 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
         const int j = M <= 8 || N < 64 * LLMK_CUS ? 0 : 1;
         const double narrow = m.base8[0][j] + (double)(((N + (16 << j) - 1) / (16 << j) + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
         const int d = w8_depth(1, 1 << j, KT_all);
-        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX) best = WavePlan{8, 1, 1 << j, 1, weights};
+        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX && wv_grid_ok((N + (16 << j) - 1) >> (4 + j), 8)) best = WavePlan{8, 1, 1 << j, 1, weights};
         best.cost = weights;
     }
     return found;
@@ -1111,10 +1114,12 @@ inline int launch_w8_wave_plan(DirectArgs p, const WavePlan& w, void* scratch, h
 inline bool w4a8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
     return wave_plan(M, N, K, scratch, WV_W4A8, [](int nw, int mt, int nt, int per) { return wv_lds(nw, mt, nt, wv_depth(mt, nt, per), per); }, best);
 }
-// 16-bit activations: groups in whole K steps, and a scale table of at least one load
+// 16-bit activations: groups in whole K steps, a scale table of at least one load, and Marlin words whose eight strips of a K step, and
+// scales whose groups, lie within 32-bit offsets (strips are 8 N bytes apart, groups 2 N).
 template <int KIND, bool PRE>
 inline bool w4a16_wave_plan(int64_t M, int64_t N, int64_t K, int group, int64_t scratch, WavePlan& best) {
     if (K % 128 || group % 128 || N * (K / group) < 4 || K > (1 << 24) || N * (K / 2) >= (1ll << 40)) return false;
+    if (wh_marlin(KIND) && N * std::max<int64_t>(64, 2 * (K / group)) > 0xffffffffll) return false;
     return wave_plan(M, N, K, scratch, wave_model<KIND, PRE>(), [&](int nw, int mt, int nt, int per) {
         return wh_built<KIND, PRE>(nw, mt, nt) ? wh_lds(KIND, nw, mt, nt, wh_groups((int)K, group, per)) : D_LDS_MAX + 1;
     }, best);

@@ -57,3 +57,16 @@ def test_w4a8_reports_the_two_passes():
     """Where the operator has always had scratch for an expanded copy, words that are not 16-byte aligned rely on it."""
     for M, N, K in W4A8_ANY_WORDS:
         assert shape("w4a8", M, N, K, 128, MUCH) and _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128) >= N * K
+
+
+def test_offsets_and_grids_of_very_wide_weights():
+    """Marlin strips and groups beyond 32-bit offsets, and grids of 2^32 threads or more, are not taken."""
+    marlin = lambda N, K, gs: shape("w4a16", 1, _lib.F16, 16, N, K, gs, MUCH)
+    assert marlin((1 << 26) - 64, 128, 128) and not marlin(1 << 26, 128, 128)
+    assert marlin(1 << 24, 16384 - 128, 128) and not marlin(1 << 24, 16384, 128) and marlin(1 << 24, 16384, 256)
+    for N in (1 << 27, (1 << 27) + 1, 1 << 29, (1 << 31) - 1):
+        for M in (1, 16, 64, 512):
+            calls = [(N, shape("8bit", kind, per_token, M, N, 128, MUCH)) for kind, per_token in ((_lib.KIND_FP8, 0), (_lib.KIND_I8, 0), (_lib.KIND_I8, 1))]
+            calls += [(N // 8 * 8, shape("w4a8", M, N // 8 * 8, 128, 128, MUCH)), (N // 2, shape("w4a16", 0, _lib.F16, M, N // 2, 128, 128, MUCH))]
+            for n, got in calls:
+                assert got is None or -(-n // (16 * got[2])) * -(-M // (16 * got[1])) * got[0] * 64 < 1 << 32, (M, n, got)
