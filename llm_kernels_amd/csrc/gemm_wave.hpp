@@ -1038,7 +1038,13 @@ constexpr WaveModel WV_I8_ROWCOL = {{{2.86f, 2.76f, 1.56f}, {2.90f, 2.76f, 1.28f
                                     {{0.00f, 0.08f, 1.26f}, {0.06f, 0.12f, 1.83f}, {0.f, 1.39f, 2.46f}, {0.f, 1.54f, 3.11f}},
                                     {{0.32f, 0.47f, 0.83f}, {0.45f, 0.65f, 1.02f}, {0.f, 0.80f, 1.20f}, {0.f, 0.96f, 1.38f}},
                                     {0.f, 3.20f, 5.00f, 4.05f}, {0.f, 0.54f, 0.67f, 0.79f}};
-constexpr int w8_depth(int mt, int nt, int steps) { return mt == 1 && nt == 1 && steps >= 48 ? 2 : 1; }
+// Stages of a wave: two for 16 x 16 tiles where every wave has many K steps, and, on at most one workgroup a CU, where some wave has a
+// second one: nothing else covers the latency of its weights there, while from two workgroups a CU on the loads of one cover the other's
+// (us, weights from HBM, one | two stages: fp8 1 x 4096 x 4096 6.4 | 5.9, 1 x 2616 x 4096 6.0 | 5.3, int8 1 x 2408 x 3072 5.2 | 4.7, 1 x 4096 x
+// 5120 7.4 | 6.7, but 1 x 6144 x 4096 7.6 | 8.1, 1 x 14336 x 4096 13.1 | 14.1).
+constexpr int w8_depth(int mt, int nt, int steps, int64_t wgs) {
+    return mt == 1 && nt == 1 && (steps >= 48 || (steps > 8 && wgs <= LLMK_CUS)) ? 2 : 1;
+}
 template <int KIND>
 inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
     constexpr const WaveModel& m = KIND == K_FP8_BLOCK ? WV_FP8 : (KIND == K_I8_BLOCK ? WV_I8 : WV_I8_ROWCOL);
@@ -1058,7 +1064,7 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
                     if (nw == 4 && (j < 2 || m.step4[mt - 1] == 0.f)) continue;
                     const double cost = slices + (nw == 8 ? m.base8[mt - 1][j] + (double)rounds * (m.fixed8[mt - 1][j] + steps8 * m.step8[mt - 1][j])
                                                           : m.base4[mt - 1] + (double)rounds * steps4 * m.step4[mt - 1]);
-                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT), KT) > D_LDS_MAX || !wv_grid_ok(tiles, nw)) continue;
+                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT, tiles * z), KT) > D_LDS_MAX || !wv_grid_ok(tiles, nw)) continue;
                     best = WavePlan{nw, mt, 1 << j, z, cost};
                     found = true;
                 }
@@ -1072,12 +1078,17 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
         // 21.4, 8 x 128256 x 4096 103 | 100 | 99, 16 x 57344 x 4096 57.4 | 52.3 | 56.2, 16 x 128256 x 4096 105 | 102 | 111),
         // where those still make two a CU (16 x 4096 x 14336 22.1 | 18.1 with 32 | 16).
         const int j = M <= 8 || N < 64 * LLMK_CUS ? 0 : 1;
-        const double narrow = m.base8[0][j] + (double)(((N + (16 << j) - 1) / (16 << j) + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
-        const int d = w8_depth(1, 1 << j, KT_all);
-        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX && wv_grid_ok((N + (16 << j) - 1) >> (4 + j), 8)) best = WavePlan{8, 1, 1 << j, 1, weights};
+        const int64_t tiles = (N + (16 << j) - 1) >> (4 + j);
+        const double narrow = m.base8[0][j] + (double)((tiles + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
+        const int d = w8_depth(1, 1 << j, KT_all, tiles);
+        if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX && wv_grid_ok(tiles, 8)) best = WavePlan{8, 1, 1 << j, 1, weights};
         best.cost = weights;
     }
     return found;
+}
+inline int w8_depth(const WavePlan& w, int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((N + 16 * w.nt - 1) / (16 * w.nt)) * ((M + 16 * w.mt - 1) / (16 * w.mt));
+    return w8_depth(w.mt, w.nt, (int)(((K >> 7) + w.z - 1) / w.z), tiles * w.z);
 }
 template <int KIND>
 inline int launch_w8_wave_plan(DirectArgs p, const WavePlan& w, void* scratch, hipStream_t stream, const char* name) {
@@ -1101,7 +1112,7 @@ inline int launch_w8_wave_plan(DirectArgs p, const WavePlan& w, void* scratch, h
         if constexpr (decltype(mt)::value > 1) {
             if (w.nw == 4) return run(i4, mt, i4, i1);
         } else {
-            if (w8_depth(1, w.nt, ((p.K >> 7) + w.z - 1) / w.z) == 2) return run(i8, mt, i1, i2);
+            if (w8_depth(w, p.M, p.N, p.K) == 2) return run(i8, mt, i1, i2);
         }
         if constexpr (decltype(mt)::value <= 2) {
             if (w.nt == 1) return run(i8, mt, i1, i1);
