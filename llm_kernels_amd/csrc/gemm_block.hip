@@ -19,7 +19,9 @@ int check_common(const char* name, const void* a, const void* b, int64_t M, int6
     return LLMK_OK;
 }
 
-// K ranges of decode-sized calls with long K: the planes of fp32 sums that their scratch is sized for.
+// Planes of fp32 sums that the reported scratch of decode-sized calls is sized for, one per 4096 elements of K.  The wave kernels
+// slice K beyond 16384 only, into as many ranges as these planes hold at most; up to there nothing touches them, but the size is what
+// callers have been told, and what llmk_gemm_fp8_block_static accepts a shape by.
 inline int stream_k_ranges(int64_t M, int64_t N, int64_t K) {
     if (M > 64 || K <= 4096 || mid_m_prefers_tiles(M, N, K)) return 1;
     return (int)((K / 128 + 31) / 32);
@@ -105,7 +107,7 @@ extern "C" int llmk_gemm_8bit_wave_shape(int kind, int per_token, int64_t M, int
     const bool full = scratch_bytes > 0 && scratch_bytes >= llmk_gemm_workspace_bytes(M, N, K);
     const WavePlan w = kind == LLMK_KIND_FP8 ? wave_choice<K_FP8_BLOCK>(p, scratch_bytes, full)
                                              : (per_token ? wave_choice<K_I8_ROWCOL>(p, scratch_bytes, full) : wave_choice<K_I8_BLOCK>(p, scratch_bytes, full));
-    return w.nw ? wave_shape(w, w8_depth(w.mt, w.nt, (int)(((K >> 7) + w.z - 1) / w.z)), shape) : 0;
+    return w.nw ? wave_shape(w, w8_depth(w, M, N, K), shape) : 0;
 }
 
 extern "C" int llmk_gemm_fp8_block(const void* a, const float* a_s, const void* b, const float* b_s, void* c,
