@@ -50,17 +50,21 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
     const double e = c.cost * k * (KIND == K_I8_BLOCK ? 1.12 : 1.0);
     return c.choice == 1 ? 3.4 + 0.87 * e : (c.choice == 2 ? 5.0 + 0.7 * e : (c.choice == 8 ? 9.0 + 0.85 * e : 7.5 + 0.8 * e));
 }
-// The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels (block-scaled
-// operands beyond 128 rows: 16 %, which covers weights from HBM: 256 x 4096 x 4096 fp8 16.1 | 15.2, int8 16.2 | 15.0).  Over 550
-// random shapes of N 1024 to 28672 and K 1024 to 14336, against the kernels before: 1.34 to 1.48 times as fast at 1 to 16 rows, 1.26
-// to 1.50 at 17 to 64, 1.09 (fp8), 1.14 (int8) and 1.23 (per token) at 65 to 512; one in forty of them lost 5 to 10 %.  us, wave | tiles:
-// int8 29 x 4096 x 4096 5.1 | 8.5, fp8 64 x 4096 x 4096 6.2 | 9.4, fp8 200 x 1032 x 7168 7.6 | 15.1, per token 250 x 4096 x 14336 25.1 |
-// 28.1, but fp8 250 x 4096 x 14336 30.6 | 29.2, and from 513 rows on 0.8 times as fast.
+// The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels, or 16 %.  The
+// estimates are fitted to weights in the cache; from HBM the tile kernels, with more loads in flight a CU, lose less.  So 16 % for
+// block-scaled int8 from 65 rows on, fp8 from 129, and from 65 rows for weights beyond the L2s' 32 MB.  Measured on 237 random shapes of 65 to
+// 512 rows, N 1024 to 28672, K 1024 to 14336, weights from HBM, both kernels timed; speed against the tile kernels alone with margins of
+// 8 | 16 | 20 %: fp8 129 to 512 rows 1.015 | 1.019 | 1.005, int8 65 to 128 1.023 | 1.039 | 1.039, 129 to 512 1.022 | 1.028 | 1.028.  What
+// 8 % lost on large weights, us, wave | tiles: int8 90 x 14336 x 4096 24.3 | 21.1, 74 x 21400 x 12160 86.1 | 75.2, per token 81 x 21672 x 3584
+// 27.8 | 22.4, 427 x 5424 x 14208 77.1 | 62.8 (and gained: 280 x 4992 x 8960 9 %).  What the wave kernel gains: int8 29 x 4096 x 4096
+// 7.2 | 8.7, fp8 64 x 4096 x 4096 8.8 | 10.8, per token 337 x 3592 x 4608 17.9 | 21.0, 359 x 2112 x 10112 21.8 | 29.4; from 513 rows
+// on it is 0.8 times as fast.
 template <int KIND>
 WavePlan wave_choice(const DirectArgs& p, int64_t scratch, bool tiles_scratch) {
     WavePlan w{0, 0, 0, 0, 0.0};
     if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w)) w.nw = 0;
-    const double margin = KIND != K_I8_ROWCOL && p.M > 128 ? 1.16 : 1.08;
+    const bool cold = KIND == K_I8_BLOCK ? p.M > 64 : (KIND == K_FP8_BLOCK && p.M > 128);
+    const double margin = cold || (p.M > 64 && (int64_t)p.N * p.K > (32 << 20)) ? 1.16 : 1.08;
     if (w.nw && p.M > 16 && margin * w.cost >= tiles_estimate<KIND>(p, tiles_scratch)) w.nw = 0;
     return w;
 }
