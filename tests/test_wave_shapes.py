@@ -69,6 +69,7 @@ def test_8bit_beyond_64_rows():
     much = lambda kind, per_token, M, N, K: shape("8bit", kind, per_token, M, N, K, _lib.load().llmk_gemm_workspace_bytes(M, N, K))
     assert much(_lib.KIND_I8, 0, 90, 14336, 4096) is None
     assert much(_lib.KIND_I8, 1, 81, 21672, 3584) is None and much(_lib.KIND_I8, 1, 427, 5424, 14208) is None
+    assert much(_lib.KIND_I8, 1, 300, 4096, 14336) is None and much(_lib.KIND_I8, 0, 128, 4096, 14336) is None
     assert much(_lib.KIND_I8, 1, 337, 3592, 4608) and much(_lib.KIND_FP8, 0, 200, 1032, 7168) and much(_lib.KIND_I8, 0, 128, 2048, 4096)
 
 
