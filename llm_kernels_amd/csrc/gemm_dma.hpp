@@ -712,10 +712,17 @@ __global__ void splitk_sum_rowcol_kernel(const int32_t* __restrict__ partial, Di
         if (p.c) {
             int m = (int)(i / p.N), n = (int)(i % p.N);
             v4f o;
+            if (n + 4 <= p.N) {                                      // one row: its scale, and four column scales in one load
+                const float am = as[m];
+                const v4f b = ((const Loose<v4f, 4>*)(bs + n))->v;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                o[q] = (float)s[q] * as[m] * bs[n];
-                if (++n == p.N) { n = 0; ++m; }              // (m = M only behind the last element)
+                for (int q = 0; q < 4; ++q) o[q] = (float)s[q] * am * b[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    o[q] = (float)s[q] * as[m] * bs[n];
+                    if (++n == p.N) { n = 0; ++m; }          // (m = M only behind the last element)
+                }
             }
             store_run4<ODT>(p.c, i, o);
         }
