@@ -45,11 +45,15 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
         return (pl.mt == 4 ? 3.6 + 11.9 * k / pl.z : 5.2 + 19.2 * k / pl.z) + (pl.z > 1 ? 3.5 : 0.0);
     }
     const int z = splitk_factor(M, N, K);
-    // K slices of 64-row tiles: 21 us for K = 4096 while they are one round of workgroups, and where nothing is scaled per K step (us, weights in
-    // the cache: per token 128 x 4096 x 14336 in four slices 19.2, 300 x 4096 x 14336 in two 38.5, int8 128 x 4096 x 14336 21.5), else 26
-    // (int8 273 x 4096 x 14336 49.7).  Of 37 such shapes 26 throughout sent 11 to the wave kernel that lose 6 to 19 % there from HBM (int8
-    // 128 x 4096 x 14336 29.9 | 26.3, per token 300 x 4096 x 14336 48.1 | 42.5), this rule 3.
-    if (z > 1) return 3.0 + (KIND == K_I8_ROWCOL || ((M + 63) / 64) * ((N + 127) / 128) * z <= LLMK_CUS ? 21.0 : 26.0) * k / z;
+    // K slices of 64-row tiles, two launches: by whether they are one round of workgroups and whether every K step is scaled (a fit of 7 to 9 %
+    // rms to 37 shapes of int8 and per token).  A cost that is only proportional to the slices' length, 19 % rms, chose the slower kernel for
+    // 12 of them by 6 to 19 % with weights from HBM, this one for 2 by 7 % (us, wave | tiles: int8 128 x 4096 x 14336 29.9 | 26.3, per token
+    // 300 x 4096 x 14336 48.1 | 42.5, but 400 x 1030 x 9088 14.1 | 18.5).
+    if (z > 1) {
+        const bool one = ((M + 63) / 64) * ((N + 127) / 128) * z <= LLMK_CUS;
+        if (KIND == K_I8_ROWCOL) return one ? 7.0 + 13.5 * k / z : 10.0 + 16.5 * k / z;
+        return 8.0 + (one ? 15.0 : 24.0) * k / z;
+    }
     const TileChoice c = dma_tile_estimate<KIND, false>(p);
     const double e = c.cost * k * (KIND == K_I8_BLOCK ? 1.12 : 1.0);
     return c.choice == 1 ? 3.4 + 0.87 * e : (c.choice == 2 ? 5.0 + 0.7 * e : (c.choice == 8 ? 9.0 + 0.85 * e : 7.5 + 0.8 * e));

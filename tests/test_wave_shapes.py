@@ -70,6 +70,7 @@ def test_8bit_beyond_64_rows():
     assert much(_lib.KIND_I8, 0, 90, 14336, 4096) is None
     assert much(_lib.KIND_I8, 1, 81, 21672, 3584) is None and much(_lib.KIND_I8, 1, 427, 5424, 14208) is None
     assert much(_lib.KIND_I8, 1, 300, 4096, 14336) is None and much(_lib.KIND_I8, 0, 128, 4096, 14336) is None
+    assert much(_lib.KIND_I8, 1, 400, 1030, 9088) and much(_lib.KIND_I8, 0, 205, 1296, 8960)
     assert much(_lib.KIND_I8, 1, 337, 3592, 4608) and much(_lib.KIND_FP8, 0, 200, 1032, 7168) and much(_lib.KIND_I8, 0, 128, 2048, 4096)
 
 
