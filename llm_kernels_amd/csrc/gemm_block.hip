@@ -60,19 +60,19 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
 }
 // The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels, or 16 %.  The
 // estimates are fitted to weights in the cache; from HBM the tile kernels, with more loads in flight a CU, lose less.  So 16 % for
-// block-scaled int8 from 65 rows on, fp8 from 129, and from 65 rows for weights beyond the L2s' 32 MB.  Measured on 237 random shapes of 65 to
+// block-scaled operands beyond 128 rows, and from 65 rows for weights of 24 MB or more.  Measured on 237 random shapes of 65 to
 // 512 rows, N 1024 to 28672, K 1024 to 14336, weights from HBM, both kernels timed; speed against the tile kernels alone with margins of
 // 8 | 16 | 20 %: fp8 129 to 512 rows 1.015 | 1.019 | 1.005, int8 65 to 128 1.023 | 1.039 | 1.039, 129 to 512 1.022 | 1.028 | 1.028.  What
 // 8 % lost on large weights, us, wave | tiles: int8 90 x 14336 x 4096 24.3 | 21.1, 74 x 21400 x 12160 86.1 | 75.2, per token 81 x 21672 x 3584
-// 27.8 | 22.4, 427 x 5424 x 14208 77.1 | 62.8 (and gained: 280 x 4992 x 8960 9 %).  What the wave kernel gains: int8 29 x 4096 x 4096
-// 7.2 | 8.7, fp8 64 x 4096 x 4096 8.8 | 10.8, per token 337 x 3592 x 4608 17.9 | 21.0, 359 x 2112 x 10112 21.8 | 29.4; from 513 rows
-// on it is 0.8 times as fast.
+// 27.8 | 22.4, 427 x 5424 x 14208 77.1 | 62.8 (and gained: 280 x 4992 x 8960 9 %, on small ones int8 84 x 3952 x 1280 5.7 | 6.5).  What the
+// wave kernel gains: int8 29 x 4096 x 4096 7.2 | 8.7, fp8 64 x 4096 x 4096 8.8 | 10.8, per token 337 x 3592 x 4608 17.9 | 21.0, 359 x
+// 2112 x 10112 21.8 | 29.4; from 513 rows on it is 0.8 times as fast.
 template <int KIND>
 WavePlan wave_choice(const DirectArgs& p, int64_t scratch, bool tiles_scratch) {
     WavePlan w{0, 0, 0, 0, 0.0};
     if (p.M > 512 || !w8_wave_plan<KIND>(p.M, p.N, p.K, scratch, w)) w.nw = 0;
-    const bool cold = KIND == K_I8_BLOCK ? p.M > 64 : (KIND == K_FP8_BLOCK && p.M > 128);
-    const double margin = cold || (p.M > 64 && (int64_t)p.N * p.K > (32 << 20)) ? 1.16 : 1.08;
+    const bool cold = (KIND != K_I8_ROWCOL && p.M > 128) || (p.M > 64 && (int64_t)p.N * p.K >= (24 << 20));
+    const double margin = cold ? 1.16 : 1.08;
     if (w.nw && p.M > 16 && margin * w.cost >= tiles_estimate<KIND>(p, tiles_scratch)) w.nw = 0;
     return w;
 }
