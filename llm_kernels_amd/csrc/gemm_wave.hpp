@@ -1073,11 +1073,13 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
     }
     const double weights = 2.0 + (double)(N * K) / 6.1e6;
     if (found && best.cost < weights) {
-        // Bound by the weights: up to 8 rows tiles of 16 columns, four workgroups a CU, keep HBM busiest, up to 16 rows, whose activations
-        // weigh more, tiles of 32 (fp8, us from HBM, 64 | 32 | 16 columns: 1 x 28672 x 4096 32.2 | 31.0 | 29.8, 8 x 18000 x 4096 27.3 | 23.2 |
-        // 21.4, 8 x 128256 x 4096 103 | 100 | 99, 16 x 57344 x 4096 57.4 | 52.3 | 56.2, 16 x 128256 x 4096 105 | 102 | 111),
-        // where those still make two a CU (16 x 4096 x 14336 22.1 | 18.1 with 32 | 16).
-        const int j = M <= 8 || N < 64 * LLMK_CUS ? 0 : 1;
+        // Bound by the weights: tiles of 16 columns, four workgroups a CU, keep HBM busiest up to 8 rows, with K from 4096 on up to 12; beyond,
+        // where activations and the tiles' ends weigh more, tiles of 32 columns where those make 2.5 workgroups a CU (us, weights from HBM, 16 | 32 columns: fp8 9 x
+        // 28672 x 4096 23.6 | 24.8, 12 x 28672 x 4096 24.5 | 25.5, 10 x 24000 x 2304 13.4 | 12.5, 16 x 18000 x 4096 18.9 | 19.7, 14 x 20000 x 4096 19.1 | 20.0, 16 x 22000 x
+        // 4096 22.8 | 21.5, 16 x 24576 x 4096 23.3 | 21.9, 16 x 28672 x 4096 26.3 | 26.1, 16 x 32000 x 6144 44.0 | 39.0, 16 x 57344 x 4096
+        // 49.2 | 45.2, 16 x 128256 x 4096 104 | 95; weights in the cache 16 x 28672 x 4096 18.7 | 19.2; 64 columns: 1 x 28672 x 4096 32.2
+        // against 29.8 with 16).
+        const int j = M <= 8 || (M <= 12 && KT_all >= 32) || N < 80 * LLMK_CUS ? 0 : 1;
         const int64_t tiles = (N + (16 << j) - 1) >> (4 + j);
         const double narrow = m.base8[0][j] + (double)((tiles + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
         const int d = w8_depth(1, 1 << j, KT_all, tiles);

@@ -63,6 +63,16 @@ def test_8bit_second_stage():
             assert stages(M, N, K) == (8, 1), (kind, per_token, M, N, K)
 
 
+def test_8bit_columns_of_a_decode_tile():
+    """Weight-bound calls of 9 to 16 rows: 32 columns from 20480 columns on, with K of 4096 or more from 13 rows."""
+    for kind, per_token in ((_lib.KIND_FP8, 0), (_lib.KIND_I8, 0), (_lib.KIND_I8, 1)):
+        columns = lambda M, N, K: 16 * shape("8bit", kind, per_token, M, N, K, 0)[2]
+        for M, N, K in ((9, 28672, 4096), (12, 57344, 4096), (16, 18000, 4096), (9, 18000, 4096), (14, 20000, 4096)):
+            assert columns(M, N, K) == 16, (kind, per_token, M, N, K)
+        for M, N, K in ((16, 28672, 4096), (13, 24576, 4096), (16, 128256, 4096), (10, 24000, 2304)):
+            assert columns(M, N, K) == 32, (kind, per_token, M, N, K)
+
+
 def test_8bit_beyond_64_rows():
     """Large weights from HBM: the tile kernels, which were 1.15 to 1.24 times as fast there, also for 65 to 128 rows and for per-token
     scales; small ones stay with the waves."""
