@@ -56,11 +56,13 @@ __device__ __forceinline__ WideTile wide_tile_of(const DirectArgs& p, int lin, i
         if (lin >= gx * gy) return t;
         int bx = lin % gx, by = lin / gx;
         // The order of xcd_tile.  8-bit operands: but for one round of a multiple of eight columns, which row-major order deals to the
-        // XCDs already.  16-bit operands and 4-bit weights (not EIGHT), which load the L2 less per matrix instruction: only with more
+        // XCDs already, and for more rounds of such a number on up to seven tile rows, whose strips would be as uneven as two and five rows
+        // (us, weights from HBM, row-major | xcd_tile, 28672 x 4096: fp8 578 rows 95.5 | 108, 1200 156 | 168, 1790 216 | 219, but 2800 303 |
+        // 290, 3800 418 | 405; int8 578 111 | 122, 3800 467 | 466; per token 1200 144 | 156, 3800 364 | 352).  16-bit operands and 4-bit weights (not EIGHT), which load the L2 less per matrix instruction: only with more
         // than a round (bf16 x 4-bit 1033 x 4096 x 4096 54 us so, 57 everywhere; 160 shapes of 1024 to 4096 rows 2 % faster than with
         // row-major order where the tile rows are no multiple of four), and the last round of whole strips as it comes.
         if constexpr (EIGHT) {
-            if (gy % 4 == 0 || gx % 8 != 0 || gx * gy > LLMK_CUS) xcd_tile(lin, gx, gy, bx, by);
+            if (gy % 4 == 0 || gx % 8 != 0 || (gx * gy > LLMK_CUS && gy > 7)) xcd_tile(lin, gx, gy, bx, by);
         } else if (gy % 4 == 0) {
             if (lin < (gx * gy & ~(LLMK_CUS - 1))) {
                 xcd_tile(lin, gx, gy, bx, by);
