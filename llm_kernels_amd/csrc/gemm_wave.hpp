@@ -1041,10 +1041,13 @@ constexpr WaveModel WV_I8_ROWCOL = {{{2.86f, 2.76f, 1.56f}, {2.90f, 2.76f, 1.28f
 // Stages of a wave: two for 16 x 16 tiles where every wave has many K steps, and, on at most one workgroup a CU, where some wave has a
 // second one: nothing else covers the latency of its weights there, while from two workgroups a CU on the loads of one cover the other's
 // (us, weights from HBM, one | two stages: fp8 1 x 4096 x 4096 6.4 | 5.9, 1 x 2616 x 4096 6.0 | 5.3, int8 1 x 2408 x 3072 5.2 | 4.7, 1 x 4096 x
-// 5120 7.4 | 6.7, but 1 x 6144 x 4096 7.6 | 8.1, 1 x 14336 x 4096 13.1 | 14.1).
-constexpr int w8_depth(int mt, int nt, int steps, int64_t wgs) {
-    return mt == 1 && nt == 1 && (steps >= 48 || (steps > 8 && wgs <= LLMK_CUS)) ? 2 : 1;
+// 5120 7.4 | 6.7, but 1 x 6144 x 4096 7.6 | 8.1, 1 x 14336 x 4096 13.1 | 14.1).  From 9 rows on for weights below 16 MB only: more of
+// them at once do not come faster behind a cache full of dirty lines (fp8 16 x 4096 x 4096 8.5 | 8.7, 16 x 2048 x 4096 7.35 | 7.15, 16 x 4096 x 2048
+// 6.4 | 6.1).
+constexpr int w8_depth(int mt, int nt, int steps, int64_t wgs, bool few) {
+    return mt == 1 && nt == 1 && (steps >= 48 || (steps > 8 && wgs <= LLMK_CUS && few)) ? 2 : 1;
 }
+constexpr bool w8_few(int64_t M, int64_t N, int64_t K) { return M <= 8 || N * K < (16 << 20); }
 template <int KIND>
 inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WavePlan& best) {
     constexpr const WaveModel& m = KIND == K_FP8_BLOCK ? WV_FP8 : (KIND == K_I8_BLOCK ? WV_I8 : WV_I8_ROWCOL);
@@ -1064,7 +1067,7 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
                     if (nw == 4 && (j < 2 || m.step4[mt - 1] == 0.f)) continue;
                     const double cost = slices + (nw == 8 ? m.base8[mt - 1][j] + (double)rounds * (m.fixed8[mt - 1][j] + steps8 * m.step8[mt - 1][j])
                                                           : m.base4[mt - 1] + (double)rounds * steps4 * m.step4[mt - 1]);
-                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT, tiles * z), KT) > D_LDS_MAX || !wv_grid_ok(tiles, nw)) continue;
+                    if ((found && cost >= best.cost) || w8_lds(nw, mt, 1 << j, w8_depth(mt, 1 << j, KT, tiles * z, w8_few(M, N, K)), KT) > D_LDS_MAX || !wv_grid_ok(tiles, nw)) continue;
                     best = WavePlan{nw, mt, 1 << j, z, cost};
                     found = true;
                 }
@@ -1082,7 +1085,7 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
         const int j = M <= 8 || (M <= 12 && KT_all >= 32) || N < 80 * LLMK_CUS ? 0 : 1;
         const int64_t tiles = (N + (16 << j) - 1) >> (4 + j);
         const double narrow = m.base8[0][j] + (double)((tiles + LLMK_CUS - 1) / LLMK_CUS) * (m.fixed8[0][j] + ((KT_all + 7) >> 3) * m.step8[0][j]);
-        const int d = w8_depth(1, 1 << j, KT_all, tiles);
+        const int d = w8_depth(1, 1 << j, KT_all, tiles, w8_few(M, N, K));
         if (M <= 16 && best.z == 1 && narrow <= weights && w8_lds(8, 1, 1 << j, d, KT_all) <= D_LDS_MAX && wv_grid_ok(tiles, 8)) best = WavePlan{8, 1, 1 << j, 1, weights};
         best.cost = weights;
     }
@@ -1090,7 +1093,7 @@ inline bool w8_wave_plan(int64_t M, int64_t N, int64_t K, int64_t scratch, WaveP
 }
 inline int w8_depth(const WavePlan& w, int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((N + 16 * w.nt - 1) / (16 * w.nt)) * ((M + 16 * w.mt - 1) / (16 * w.mt));
-    return w8_depth(w.mt, w.nt, (int)(((K >> 7) + w.z - 1) / w.z), tiles * w.z);
+    return w8_depth(w.mt, w.nt, (int)(((K >> 7) + w.z - 1) / w.z), tiles * w.z, w8_few(M, N, K));
 }
 template <int KIND>
 inline int launch_w8_wave_plan(DirectArgs p, const WavePlan& w, void* scratch, hipStream_t stream, const char* name) {

@@ -54,12 +54,13 @@ def test_w4a16():
 
 
 def test_8bit_second_stage():
-    """Two stages where one workgroup a CU has nothing else to cover the latency of a wave's second K step, one from there on."""
+    """Two stages where one workgroup a CU has nothing else to cover the latency of a wave's second K step, one from there on and for 9
+    rows and more on weights of 16 MB."""
     for kind, per_token in ((_lib.KIND_FP8, 0), (_lib.KIND_I8, 0), (_lib.KIND_I8, 1)):
         stages = lambda M, N, K: shape("8bit", kind, per_token, M, N, K, 0)[::3]
-        for M, N, K in ((1, 4096, 4096), (2, 2408, 3072), (16, 4096, 1152), (1, 2616, 4096)):
+        for M, N, K in ((1, 4096, 4096), (8, 4096, 4096), (2, 2408, 3072), (16, 4096, 1152), (1, 2616, 4096), (16, 4088, 4096)):
             assert stages(M, N, K) == (8, 2), (kind, per_token, M, N, K)
-        for M, N, K in ((1, 4097, 4096), (1, 6144, 4096), (1, 4096, 1024)):
+        for M, N, K in ((1, 4097, 4096), (1, 6144, 4096), (1, 4096, 1024), (9, 4096, 4096), (16, 4096, 4096)):
             assert stages(M, N, K) == (8, 1), (kind, per_token, M, N, K)
 
 
