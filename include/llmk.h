@@ -116,7 +116,7 @@ int llmk_weight_dequant_w4a8(const int32_t* packed, const void* s_f16, const int
  * C[M,N] = sum_kb dot_kb(A, B) * a_s[m, kb] * b_s[n / 128, kb], K % 128 == 0 (K = 0: zeros), any M, N >= 1.
  * A [M,K], B [N,K] both K-contiguous.  c_dtype selects the epilogue (torch default dtype).
  * workspace/workspace_bytes: optional scratch of llmk_gemm_workspace_bytes(M, N, K) bytes (fp32 activation
- * scales for large M, fp32 partial sums of the split-K / K-range variants); NULL/0 -> single-pass variants.
+ * scales for large M, fp32 partial sums of K slices); NULL/0 -> single-pass variants.
  * ref: quantization/fp8_kernel.py:113-191 (a_s, b_s fp32)                                   */
 int llmk_gemm_fp8_block(const void* a_e4m3, const float* a_s, const void* b_e4m3, const float* b_s,
                         void* c, int c_dtype, int64_t M, int64_t N, int64_t K,
@@ -125,7 +125,7 @@ int llmk_gemm_fp8_block(const void* a_e4m3, const float* a_s, const void* b_e4m3
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same operands as
  * llmk_gemm_fp8_block, but the scratch is a device array built into the library (LLMK_STATIC_SCRATCH_BYTES per
  * GPU, held until the process ends); the call itself allocates and frees nothing.  The array serves the
- * activation scales / split-K / K-range partial sums, not the optional 64 MiB of a split last round of tiles:
+ * activation scales / partial sums of K slices, not the optional 64 MiB of a split last round of tiles:
  * results equal llmk_gemm_fp8_block with a workspace of llmk_gemm_workspace_bytes(M, N, K) bytes bit for bit
  * whenever that size holds no such 64 MiB (M <= 512 or K < 8192); beyond that the workspace entry may split its
  * last round of tiles along K and the two differ in the fp32 summation order only (same tolerance against the
@@ -140,8 +140,8 @@ int llmk_gemm_i8_block(const int8_t* a, const void* a_s, const int8_t* b, const 
                        void* workspace, int64_t workspace_bytes, void* stream);
 /* per-token x per-channel W8A8 with one full-K int32 accumulation (a scheme with
  * no counterpart function in the reference).  c may be NULL; c_i32 (raw accumulators) may be NULL.
- * M <= 64 streams the weights once; larger M runs on the MFMA tile kernels (int32 accumulation inside
- * the MFMA, c = float(acc) * a_s[m] * b_s[n] in the epilogue of either path).  With a workspace of
+ * Up to 16 rows, and up to 512 where it is estimated to be faster, waves stream their own share of K, otherwise the MFMA tile
+ * kernels run (int32 sums inside the MFMA, c = float(acc) * a_s[m] * b_s[n] in the epilogue of either path).  With a workspace of
  * llmk_gemm_workspace_bytes(M, N, K), shapes with few tiles and a long K are split along K; the slices' int32 sums
  * are added as integers before the scaling, so c and c_i32 do not depend on the split. */
 int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, const float* b_s,
@@ -151,9 +151,11 @@ int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, cons
  * ref: quantization/w4a8_kernel.py:317-448 */
 /* workspace: llmk_gemm_w4a8_workspace_bytes(M, N, K, group_int4) bytes, 16-byte aligned, is what the path
  * chosen for the shape uses.  With group_int4 == 128 and 16-byte aligned a and b_packed:
- *   - up to 256 rows, and up to 512 where that is estimated to be faster (see the plan in gemm_w4a8.hip), one kernel unpacks
- *     the words itself and reads them once per row tile: fp32 partial sums of its K slices, z * M * N * 4 bytes, optional up
- *     to K = 32768 (without: unsplit); from 17 rows on llmk_gemm_workspace_bytes(M,N,K) is reported at least;
+ *   - up to 128 rows, and from 129 to 512 where that is estimated to be faster (see the plan in gemm_w4a8.hip: 512 x 4096 x 4096, but
+ *     not 245 x 28672 x 4096), one kernel unpacks the words itself and reads them once per row tile: fp32 partial sums of its K
+ *     slices, z * M * N * 4 bytes, optional up to K = 32768 (without: unsplit).  From 17 rows on at least
+ *     llmk_gemm_workspace_bytes(M,N,K) is reported, and from 129 rows (257 where 64 x 64 tiles are at most one a CU), or with K beyond
+ *     32768 from 65, what the next line needs: words that are not 16-byte aligned go that way there;
  * everything else the expanded int8 weights, round16(N*K), needed, and behind them llmk_gemm_workspace_bytes(M,N,K) for
  * the int8 tile kernels. */
 int64_t llmk_gemm_w4a8_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_int4);
@@ -170,9 +172,10 @@ int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b_packed, co
  * QuantUtils.fake_quantize gives them; sums are fp32.
  * ref: fast_dequant/simple_marlin/marlin_w4a16_gemm.cu:283-326 (simple_marlin_cuda),
  *      marlin_w4a16_gemm.cpp:23-111 (mul).                                                    */
-/* bytes of scratch llmk_gemm_w4a16_marlin uses for this shape (0 = none): fp32 split-K partial sums, and for
- * M > 64 room for the fp16 copy of W that the two-pass path of large M multiplies.  Without it (workspace
- * NULL / too small) the kernels run with fewer K slices, large M on the weight-streaming kernel. */
+/* bytes of scratch llmk_gemm_w4a16_marlin uses for this shape (0 = none): fp32 partial sums of K slices (those of the kernel whose
+ * waves stream their own share of K, which takes every call up to 64 rows and most up to 512 whose groups are whole 128, and
+ * those of the kernels next to it), and for M > 64 room for the fp16 copy of W that the two-pass path of large M multiplies.
+ * Without it (workspace NULL / too small) the kernels run with fewer K slices, large M on the weight-streaming kernel. */
 int64_t llmk_gemm_w4a16_marlin_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int llmk_gemm_w4a16_marlin(const void* a_f16, const int32_t* b, void* c_f16, const void* s_f16,
                            int64_t M, int64_t N, int64_t K, int groupsize,
@@ -189,8 +192,11 @@ int llmk_quant_w4_nk(const void* w, int w_dtype, int32_t* packed, void* scales_f
  * from 33 rows where the weight matrix is large; bf16: also where groups are not 128 wide or K is below 512) (nibble - 8) * s
  * rounded to the type of a, otherwise nibble - 8 exactly with s on the fp32 sums of a group.  workspace: llmk_gemm_w4a16_nk_workspace_bytes(...) bytes, 16-byte
  * aligned, is what the path chosen for the shape uses:
- *   - M <= 64 streams the weights: nothing for K <= 4096, fp32 partial sums of K ranges, ceil(K/4096)*M*N*4, beyond;
- *   - 64 < M <= 512 (from 33 rows on large weights, to 1024 rows and more where it wins) runs on tile kernels that expand
+ *   - M <= 16, and up to 64 rows where the next is not estimated to be faster, streams the weights: nothing for K <= 4096, fp32 partial
+ *     sums of K ranges, ceil(K/4096)*M*N*4, beyond;
+ *   - 17 to 512 rows with groups in whole 128, where it is estimated to be faster: waves that stream their own share of K, fp32 partial
+ *     sums of at most four K slices (K <= 131072), z*M*N*4, optional up to K = 32768;
+ *   - 64 < M <= 512 otherwise (from 33 rows on large weights, to 1024 rows and more where it wins): tile kernels that expand
  *     the packed words themselves: fp32 partial sums of their K slices, at most 8*M*N*4;
  *   - otherwise a 16-bit copy of W, N*K*2 bytes, that the tiled GEMM multiplies.
  * With less, fp16 calls run on the streaming kernels unsplit; a bf16 call that neither streams (128-wide groups, K ranges of

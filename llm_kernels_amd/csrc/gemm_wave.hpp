@@ -751,10 +751,13 @@ int launch_w4a16_wave(const DirectArgs& p, int z, hipStream_t stream, const char
 // K_I8_BLOCK), or int8 with a scale per row and per column (K_I8_ROWCOL: int32 sums, scaled at the end).  S32 as above.
 // What it replaces at 1 to 16 rows kept activations in registers and walked column tiles with one barrier each; its fragment
 // loads (16 rows x 64 bytes an instruction) cost the address path four times what coalesced ones to LDS do.  Bound by weights
-// from L2 or HBM up to 16 rows (warm 28672 x 4096 6.0 TB/s, cold 3.6), by the address path and the latency of one stage from there.
-// us per launch, before | now, weights in the memory-side cache: fp8 4 x 4096 x 14336 15.3 | 11.1, 9 x 14336 x 4096 14.2 | 11.3, 12 x
-// 28672 x 4096 23.0 | 20.4, 16 x 4096 x 4096 6.7 | 4.5, int8 15 x 6144 x 4096 8.7 | 5.1, per token 9 x 3128 x 9472 11.2 | 5.4; weights
-// from HBM, fp8: 16 x 4096 x 4096 8.7 | 7.8, 16 x 14336 x 4096 18.7 | 18.2, 16 x 28672 x 4096 32.2 | 32.5, 16 x 4096 x 14336 20.4 | 19.3.
+// from L2 or HBM up to 16 rows (28672 x 4096: 6.1 TB/s from the memory-side cache, 4.6 from HBM), by the address path and the latency of
+// one stage from there.  us per launch, before | now, weights in the memory-side cache: fp8 4 x 4096 x 14336 15.3 | 11.1, 9 x 14336 x 4096 14.2 |
+// 11.3, 12 x 28672 x 4096 22.9 | 18.7, 16 x 4096 x 4096 6.9 | 4.6, int8 15 x 6144 x 4096 8.7 | 5.1, per token 9 x 3128 x 9472 11.2 |
+// 5.4; weights from HBM, fp8: 1 x 4096 x 4096 6.5 | 5.8, 16 x 4096 x 4096 7.0 | 6.7, 16 x 14336 x 4096 15.4 | 15.5, 9 x 28672 x 4096 25.4
+// | 23.4, 16 x 28672 x 4096 25.9 | 25.9, 12 x 128256 x 4096 98 | 95, 1 x 4096 x 14336 16.0 | 12.4, int8 12 x 4096 x 14336 16.4 | 14.1; int8
+// on short rows is slower than before: 1 x 4096 x 1536 4.0 | 4.3, 1 x 1144 x 1024 3.0 | 3.6 (a K step or two a wave, tables and a barrier in
+// front; with the block scales in registers instead 3.7).
 constexpr int w8_stage(int mt, int nt) { return (16 * mt + 16 * nt) * 128 + 256; }
 constexpr int w8_lds(int nw, int mt, int nt, int d, int steps) {
     const int a = nw * d * w8_stage(mt, nt) + 4 * steps, b = wv_red(nw, mt, nt);
