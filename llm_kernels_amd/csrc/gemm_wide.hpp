@@ -4,8 +4,8 @@
 // 256 x 128 tile, which is what bounds that kernel.
 //
 // Workgroup: 512 threads = 8 waves, 2 along M x 4 along N; wave tile 128 rows x 64 columns =
-// 8 x 4 MFMA tiles (128 accumulator registers per lane).  Two LDS stages of 66560 bytes
-// (A 32 KB, B 32 KB, activation-scale column 1 KB).  A step has two barriers: one in the middle, behind
+// 8 x 4 MFMA tiles (128 accumulator registers per lane).  Two LDS stages of 64 KB (A and B 32 KB each) and two windows
+// of activation scales, four K steps each (scale_window_load).  A step has two barriers: one in the middle, behind
 // which the weight rows of K step kt+2 are requested (every wave holds the weight fragments of step kt in
 // registers by then), and one before its last tile row, behind which the activation rows of step kt+2 are
 // requested and the fragments of step kt+1 fetched; the loads fly while step kt+1 is multiplied.
@@ -24,10 +24,25 @@ namespace llmk {
 // R = tile rows (of 16) per wave: 8 gives the 256 x 256 tile described above, 4 a 128 x 256 tile (wave tile
 // 64 x 64) with the same loop for problems with too few rows for a round of the large tile.
 constexpr int W_BN = 256, W_THREADS = 512;
-constexpr int W_B = W_BN * 128, W_S = 256 * 4;
+constexpr int W_B = W_BN * 128;
+constexpr int sw_bytes(int rows) { return rows * 4 * 4; }           // a window of activation scales: four K steps
 constexpr int w_bm(int r) { return 32 * r; }
-constexpr int w_stage(int r) { return w_bm(r) * 128 + W_B + W_S; }        // 66560 / 50176
-constexpr int w_lds(int r) { return 2 * w_stage(r) + 2 * D_MAX_KT * 4; }  // 135168 / 102400 bytes
+constexpr int w_stage(int r) { return w_bm(r) * 128 + W_B; }                                         // 65536 / 49152
+constexpr int w_lds(int r) { return 2 * w_stage(r) + 2 * sw_bytes(w_bm(r)) + 2 * D_MAX_KT * 4; }     // 141312 / 104448 bytes
+
+// Activation scales [M, K/128] of a tile go to LDS in windows of four K steps, [row][step] as dwords: one load instruction takes 16
+// rows x 4 steps, 16 lines, so a 256 x 256 tile needs 16 of them every four steps.  (A column of 64 rows per wave and step was 32, of 64
+// lines each.  Column per step | window, us, cached operands: fp8 4096 x 28672 x 4096 403 | 383, 4096 x 4096 x 4096 58.4 | 55.5, 2048 x 4096 x
+// 4096 34.4 | 33.4, int8 4096 x 4096 x 4096 72.5 | 69.7; the first 383 is 379 without any of these loads.  The 128-column kernels,
+// whose steps are shorter, lose what this saves to the instructions around it.)
+// element offset of the calling lane's row of block blk (16 rows): lane l requests row l >> 2, step kb + (l & 3)
+__device__ __forceinline__ uint32_t sw_row(int blk, int m_start, int m_end, int KT_all, int lane) {
+    return (uint32_t)min(m_start + 16 * blk + (lane >> 2), m_end - 1) * (uint32_t)KT_all;
+}
+// (steps past kt_end repeat the last one)
+__device__ __forceinline__ void sw_load(uint32_t lds_addr, uint32_t row, int kb, int kt_end, const void* a_s, int lane) {
+    dma4(lds_addr, (row + (uint32_t)min(kb + (lane & 3), kt_end - 1)) * 4u, a_s);
+}
 
 // ---- which tile a workgroup works on.  `lin` = linear workgroup id (blockIdx.y * gridDim.x + blockIdx.x), gx = column
 // tiles.  Workgroups go to the eight XCDs round robin by linear id, each XCD with its own L2, and 256 of them (one
@@ -167,10 +182,10 @@ constexpr int W_TAIL_ITEMS = LLMK_CUS;          // upper bound of ntail * z
 // the outputs equal those of GEMM + activation + quantiser bit for bit; the [M, 2 I] tensor never exists.
 template <int KIND, bool GROUPED, int R = 8, bool SWIGLU = false>
 __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
-    constexpr bool AS16 = false;             // 16-bit activation scales are widened before this kernel, see launch_big
+    // (16-bit activation scales are widened before this kernel, see launch_big)
     static_assert(R == 8 || R == 4, "tile rows per wave");
     static_assert(!SWIGLU || (GROUPED && (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK)), "gated epilogue: grouped block-scaled kinds");
-    constexpr int W_BM = w_bm(R), W_A = W_BM * 128, W_STAGE = w_stage(R);
+    constexpr int W_BM = w_bm(R), W_A = W_BM * 128, W_STAGE = w_stage(R), SW = 2 * W_STAGE;
     constexpr int AL = R / 2;                    // activation loads per thread and stage
     constexpr int W_EARLY_ROW = R == 8 ? 5 : 2;  // tile row in front of which the mid-step barrier sits
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -226,7 +241,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     const int I_half = N >> 1;               // SWIGLU: gate rows [0, I), up rows [I, 2 I) of the weight matrix
 
     // weight scales of the tile's two 128-column blocks, for every K step
-    float* bsl = (float*)(lds + 2 * W_STAGE);
+    float* bsl = (float*)(lds + SW + 2 * sw_bytes(W_BM));
     const int nblk = (N + 127) / 128;
 
     // ---- source offsets of the 9 loads of a stage.  Load i of a wave fills LDS rows 8q .. 8q+7,
@@ -253,11 +268,15 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
         const int wrow = SWIGLU ? (col < 128 ? n0 + col : I_half + n0 + col - 128) : min(n0 + col, N - 1);
         boff[i] = (uint32_t)wrow * (uint32_t)K + chunk;
     }
-    const uint32_t soff = (uint32_t)min(m_start + min((wave & 3) * 64 + lane, W_BM - 1), m_end - 1) * (uint32_t)KT_all * (AS16 ? 2u : 4u);
-    // (AS16: 16-bit activation scales staged as they are, see gemm_dma_kernel)
-    auto dma_scale = [&](uint32_t lds_addr, int kt_abs) {
-        if constexpr (AS16) dma2(lds_addr, soff, (const uint8_t*)p.a_s + (int64_t)kt_abs * 2);
-        else dma4(lds_addr, soff, (const uint8_t*)p.a_s + (int64_t)kt_abs * 4);
+    // scale window w (K steps 4 w .. 4 w + 3): 16 R / 4 blocks of 16 rows, R / 4 a wave
+    uint32_t srow[R / 4];
+#pragma unroll
+    for (int i = 0; i < R / 4; ++i) srow[i] = SCALED ? sw_row(wave + 8 * i, m_start, m_end, KT_all, lane) : 0;
+    auto request_scales = [&](int window) {
+        const int w = __builtin_amdgcn_readfirstlane(window);
+        const uint32_t st = lds_base + SW + (uint32_t)(w & 1) * sw_bytes(W_BM);
+#pragma unroll
+        for (int i = 0; i < R / 4; ++i) sw_load(st + (uint32_t)(wave + 8 * i) * 256u, srow[i], kt0 + 4 * w, kt0 + KT, p.a_s, lane);
     };
 
     // ---- 4-bit weights: a thread owns the same piece of the 128-column half h = 0, 1 of the tile as in the
@@ -332,16 +351,14 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) dma16(st + W_A + (uint32_t)(wave * 4 + i) * 1024u, boff[i], gb);
         }
-        if constexpr (SCALED) dma_scale(st + W_A + W_B + (uint32_t)(wave & 3) * 256u, kt0 + kt);
     };
 
     // The loads of a stage inside the loop, a quarter at a time (part 0..3): the weight rows behind the
-    // mid-step barrier, the activation rows and the scale column behind the barrier of the step.
+    // mid-step barrier, the activation rows behind the barrier of the step.
     auto issue_part = [&](int kt, int part) {
         const uint32_t st = lds_base + (uint32_t)(kt & 1) * W_STAGE;
         const uint8_t* ga = p.a + (int64_t)(kt0 + kt) * 128;
         if (part < AL) dma16(st + (uint32_t)(wave * AL + part) * 1024u, aoff[part < AL ? part : 0], ga);
-        if constexpr (SCALED) if (part == 3) dma_scale(st + W_A + W_B + (uint32_t)(wave & 3) * 256u, kt0 + kt);
     };
     auto issue_b_part = [&](int kt, int part) {
         const uint32_t st = lds_base + (uint32_t)(kt & 1) * W_STAGE;
@@ -356,6 +373,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
         for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
     if (KT > 0) issue(0);
+    if constexpr (SCALED) if (KT > 0) request_scales(0);
     if constexpr (W4) if (KT > 0) w4_expand(0);
     if constexpr (SCALED) {
         for (int i = tid; i < 2 * KT; i += W_THREADS) {
@@ -437,17 +455,10 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
         const uint8_t* As = stage_a(kt);
         float sa[R];
         if constexpr (SCALED && NR > 0) {
-            const float* Ss = (const float*)(lds + (kt & 1) * W_STAGE + W_A + W_B) + wm * 16 * R + r;
+            const float* Ss = (const float*)(lds + SW + ((kt >> 2) & 1) * sw_bytes(W_BM)) + (wm * 16 * R + r) * 4 + (kt & 3);
             const float bs = bsl[(wn >> 1) * D_MAX_KT + kt];
 #pragma unroll
-            for (int i = 0; i < NR; ++i) {
-                if constexpr (AS16) {
-                    const unsigned raw = ((const unsigned*)Ss)[i * 16];
-                    sa[i] = (p.s_dtype == LLMK_F16 ? f16_to_f32((unsigned short)raw) : bf16_to_f32((unsigned short)raw)) * bs;
-                } else {
-                    sa[i] = Ss[i * 16] * bs;
-                }
-            }
+            for (int i = 0; i < NR; ++i) sa[i] = Ss[i * 64] * bs;
         }
 #pragma unroll
         for (int i = 0; i < R; ++i) {
@@ -526,6 +537,21 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     const std::false_type no;
     auto run = [&](auto nr_c) {
         int kt = 0;
+        if constexpr (SCALED || KIND == K_F16 || KIND == K_BF16) {
+            // four steps without a branch between them (one in the loop makes the compiler spill): the window of steps kt + 4 .. kt + 7
+            // overwrites one that nobody reads since the barrier of step kt - 1, and the barrier of step kt waits for it
+            // (fp16, which has no scales, step by step | four at a time: 4096 x 4096 x 4096 82.4 | 81.3 us, 2048 x 4096 x 4096 49.6 | 48.7)
+            const int blocks = (KT - 2) >> 2;
+            for (int b = 0; b < blocks; ++b) {
+                if constexpr (SCALED) request_scales(b + 1);
+                step(4 * b, yes, yes, nr_c);
+                step(4 * b + 1, yes, yes, nr_c);
+                step(4 * b + 2, yes, yes, nr_c);
+                step(4 * b + 3, yes, yes, nr_c);
+            }
+            kt = 4 * max(blocks, 0);
+            if constexpr (SCALED) if (KT > 1) request_scales((kt >> 2) + 1);                    // (one step: nothing would wait for it)
+        }
         for (; kt + 2 < KT; ++kt) step(kt, yes, yes, nr_c);
         if (kt + 1 < KT) { step(kt, yes, no, nr_c); ++kt; }
         if (kt < KT) step(kt, no, no, nr_c);

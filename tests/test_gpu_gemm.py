@@ -136,6 +136,30 @@ def test_int8_per_token_int32_bit_exact(dev, M, N, K):
     assert ag.dtype == torch.int8 and asg.shape == (M,)
 
 
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 13])
+@pytest.mark.parametrize("M", [2000, 4000])            # the 128 x 256 and the 256 x 256 tile, the last tile row ragged
+@pytest.mark.parametrize("kind", ["fp8", "int8"])
+def test_scales_of_every_k_step_on_large_tiles(dev, kind, M, steps):
+    """Small integers under scales that are powers of two of their own in every row, column block and K step: every product and sum is
+    a whole number below 2^24, so the fp32 result is exact in any order, and a scale taken from another step or row shows."""
+    announce("scales on large tiles", kind, M, steps)
+    N, K = 4096, 128 * steps
+    gen = torch.Generator(device=dev).manual_seed(100 * steps + M)
+
+    def ints(lo, hi, *shape):
+        return torch.randint(lo, hi + 1, shape, device=dev, generator=gen)
+
+    a, b = ints(-3, 3, M, K), ints(-3, 3, N, K)
+    a_s, b_s = 2.0 ** ints(0, 4, M, steps).float(), 2.0 ** ints(0, 4, N // 128, steps).float()
+    ref = (a.double() * a_s.double().repeat_interleave(128, 1)) @ (b.double() * b_s.double().repeat_interleave(128, 1).repeat_interleave(128, 0)).t()
+    with default_dtype(torch.float32):
+        if kind == "fp8":
+            c = fp8_kernel.fp8_gemm(a.float().to(torch.float8_e4m3fn), a_s, b.float().to(torch.float8_e4m3fn), b_s)
+        else:
+            c = int8_kernel.int8_gemm(a.to(torch.int8), a_s, b.to(torch.int8), b_s)
+    assert torch.equal(c.double(), ref)
+
+
 # ------------------------------------------------------------------------------------------- w4a8
 @pytest.mark.parametrize("M,N,K", [(1, 128, 128), (16, 256, 512), (37, 136, 256), (16, 4096, 4096), (128, 1024, 7168),
                                    (5, 8, 128), (33, 264, 2048), (64, 4096, 4096), (17, 1032, 2176), (16, 14336, 4096),
