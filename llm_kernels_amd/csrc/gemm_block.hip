@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "gemm_duo.hpp"
 #include "gemm_wave.hpp"
 #include "gemm_wide.hpp"
 
@@ -81,9 +82,46 @@ WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspa
     return wave_choice<KIND>(p, workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0,
                              workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K));
 }
+// What the tile kernels take beyond 512 rows, in us: rounds of the tiles that dma_tile_estimate chooses (a fit of 3 to 5 % rms for the 128-column
+// ones, 7 to 10 % for the 256-column ones, to 80 to 140 shapes a kind).
+template <int KIND>
+double large_estimate(const DirectArgs& p, bool tail) {
+    const TileChoice c = dma_tile_estimate<KIND, false>(p, tail);
+    const double e = c.cost * (double)p.K / 4096.0;
+    struct { double a, b; } f[5] = {{2.6, 0.83}, {3.0, 0.80}, {6.0, 0.80}, {5.2, 0.82}, {4.6, 0.80}};
+    if (KIND == K_I8_BLOCK) { f[0] = {2.9, 0.97}; f[1] = {4.0, 0.86}; f[2] = {6.0, 0.95}; f[3] = {8.2, 1.03}; f[4] = {6.1, 0.94}; }
+    if (KIND == K_I8_ROWCOL) { f[0] = {3.3, 0.80}; f[1] = {5.9, 0.64}; f[2] = {6.0, 0.78}; f[3] = {10.2, 0.74}; f[4] = {6.2, 0.73}; }
+    const auto& s = f[c.choice == 1 ? 0 : (c.choice == 2 ? 1 : (c.choice == 4 ? 2 : c.choice - 5))];
+    return s.a + s.b * e;
+}
+// The kernel of two wave groups (gemm_duo.hpp) for this call, or mi = 0: 8 % below the estimate of what the call gets otherwise (w: the wave
+// kernel, if it does).  Over 300 random shapes of 64 to 4096 rows a kind this was 1.04 (fp8, int8, per token) times as fast as without,
+// 0.5 to 1 % behind the faster one of each shape, at worst 5 % (16 % once) slower.  Others | this one, us: fp8 1024 x 4096 x 4096 25.5 | 20.7, int8 28.8 |
+// 25.6, per token 23.9 | 20.3; the gain is largest where 96, 128 or 160 rows leave fewer rows of the last tiles empty than 64, 128 and
+// 256 do, and where few tiles can be split along K beyond 512 rows.
+template <int KIND>
+DuoPlan duo_choice(const DirectArgs& p, const WavePlan& w, int64_t scratch, bool tiles_scratch, bool tail) {
+    DuoPlan d = duo_plan<KIND>(p, scratch);
+    if (!d.mi) return d;
+    const double other = p.M <= 512 ? (w.nw ? 1.05 * w.cost : tiles_estimate<KIND>(p, tiles_scratch)) : large_estimate<KIND>(p, tail);
+    if (1.08 * d.cost >= other) d.mi = 0;
+    return d;
+}
+template <int KIND>
+DuoPlan duo_choice(const DirectArgs& p, const WavePlan& w, void* workspace, int64_t workspace_bytes) {
+    return duo_choice<KIND>(p, w, workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0,
+                            workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K), wide_tail_ok<KIND>(p, workspace, workspace_bytes));
+}
 template <int KIND>
 int launch_block(const DirectArgs& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, const char* name) {
     const WavePlan w = wave_choice<KIND>(p, workspace, workspace_bytes);
+    if (p.M > 64) {
+        const DuoPlan d = duo_choice<KIND>(p, w, workspace, workspace_bytes);
+        if (d.mi) {
+            if constexpr (KIND == K_I8_BLOCK) if (p.s_dtype != LLMK_F32) return launch_duo_plan<KIND, true>(p, d, workspace, stream, name);
+            return launch_duo_plan<KIND>(p, d, workspace, stream, name);
+        }
+    }
     if (w.nw) return launch_w8_wave_plan<KIND>(p, w, workspace, stream, name);
     if (p.K == 0) return launch_empty_sums<false>(p, stream, name);
     return launch_big<KIND, false>(p, workspace, workspace_bytes, stream, name);
@@ -92,7 +130,7 @@ int launch_block(const DirectArgs& p, void* workspace, int64_t workspace_bytes, 
 }  // namespace
 
 // scratch without the (fixed-size) part for a split last round of 256-column tiles
-static int64_t workspace_core_bytes(int64_t M, int64_t N, int64_t K) {
+static int64_t tiles_core_bytes(int64_t M, int64_t N, int64_t K) {
     // large-M kernels stream fp32 activation scales; 16-bit scales are widened into the workspace first;
     // mid-size M with few tiles adds the fp32 split-K partials behind them
     if (K <= 0) return 0;
@@ -104,6 +142,26 @@ static int64_t workspace_core_bytes(int64_t M, int64_t N, int64_t K) {
     int z = splitk_factor(M, N, K);
     if (M <= 512) z = std::max({z, mid_plan(M, N, K).z, midw_plan(M, N, K).z});      // the mid-size kernels' K slices
     return scales + (z > 1 ? (int64_t)z * M * N * 4 : 0);
+}
+
+// the same with the planes of the kernel of two wave groups, where a kind takes it in K slices
+template <int KIND>
+static int64_t duo_bytes(int64_t M, int64_t N, int64_t K) {
+    DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.s_dtype = LLMK_F32;
+    const WavePlan w = wave_choice<KIND>(p, INT64_MAX, true);
+    const DuoPlan d = duo_choice<KIND>(p, w, INT64_MAX, true, KIND != K_I8_ROWCOL && M > 512 && K >= W_TAIL_MIN_KT * 128);
+    return d.mi && d.z > 1 ? (int64_t)d.z * M * N * 4 : 0;
+}
+static int64_t workspace_core_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 64 || N <= 0 || K < 12 * 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return tiles_core_bytes(M, N, K);
+    // a call asks twice or three times and the plans of three kinds take a microsecond: a thread remembers its last shapes
+    struct Shape { int64_t M, N, K, bytes; };
+    static thread_local Shape seen[16] = {};
+    Shape& s = seen[(uint64_t)(M * 0x9E3779B97F4A7C15ull + N * 0xC2B2AE3D27D4EB4Full + K) >> 60];
+    if (s.M != M || s.N != N || s.K != K)
+        s = {M, N, K, std::max({tiles_core_bytes(M, N, K), duo_bytes<K_FP8_BLOCK>(M, N, K), duo_bytes<K_I8_BLOCK>(M, N, K), duo_bytes<K_I8_ROWCOL>(M, N, K)})};
+    return s.bytes;
 }
 
 extern "C" int64_t llmk_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -119,7 +177,26 @@ extern "C" int llmk_gemm_8bit_wave_shape(int kind, int per_token, int64_t M, int
     const bool full = scratch_bytes > 0 && scratch_bytes >= llmk_gemm_workspace_bytes(M, N, K);
     const WavePlan w = kind == LLMK_KIND_FP8 ? wave_choice<K_FP8_BLOCK>(p, scratch_bytes, full)
                                              : (per_token ? wave_choice<K_I8_ROWCOL>(p, scratch_bytes, full) : wave_choice<K_I8_BLOCK>(p, scratch_bytes, full));
-    return w.nw ? wave_shape(w, w8_depth(w, M, N, K), shape) : 0;
+    int32_t duo[2];
+    if (!w.nw || llmk_gemm_8bit_duo_shape(kind, per_token, M, N, K, scratch_bytes, duo)) return 0;
+    return wave_shape(w, w8_depth(w, M, N, K), shape);
+}
+
+extern "C" int llmk_gemm_8bit_duo_shape(int kind, int per_token, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes, int32_t* shape) {
+    if (!shape || M <= 64 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+    DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.s_dtype = LLMK_F32;
+    const bool full = scratch_bytes > 0 && scratch_bytes >= llmk_gemm_workspace_bytes(M, N, K);
+    auto plan = [&](auto kind_c) {
+        constexpr int KIND = decltype(kind_c)::value;
+        return duo_choice<KIND>(p, wave_choice<KIND>(p, scratch_bytes, full), scratch_bytes, full, KIND != K_I8_ROWCOL && full && M > 512 && K >= W_TAIL_MIN_KT * 128);
+    };
+    const DuoPlan d = kind == LLMK_KIND_FP8 ? plan(std::integral_constant<int, K_FP8_BLOCK>{})
+                                            : (per_token ? plan(std::integral_constant<int, K_I8_ROWCOL>{}) : plan(std::integral_constant<int, K_I8_BLOCK>{}));
+    if (!d.mi) return 0;
+    shape[0] = 32 * d.mi;
+    shape[1] = d.z;
+    return 1;
 }
 
 extern "C" int llmk_gemm_fp8_block(const void* a, const float* a_s, const void* b, const float* b_s, void* c,
@@ -176,6 +253,10 @@ extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8
     p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.c = c; p.c_i32 = c_i32; p.a_s = a_s; p.b_s = b_s;
     p.c_dtype = c_dtype; p.s_dtype = LLMK_F32; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
     const WavePlan wave = wave_choice<K_I8_ROWCOL>(p, workspace, workspace_bytes);
+    if (M > 64) {
+        const DuoPlan d = duo_choice<K_I8_ROWCOL>(p, wave, workspace, workspace_bytes);
+        if (d.mi) return launch_duo_plan<K_I8_ROWCOL>(p, d, workspace, (hipStream_t)stream, "gemm_i8_rowcol(duo)");
+    }
     if (wave.nw) return launch_w8_wave_plan<K_I8_ROWCOL>(p, wave, workspace, (hipStream_t)stream, "gemm_i8_rowcol(wave)");
     // large M: the tile kernels accumulate int32 over the whole K range inside the MFMA and scale in the epilogue
     if ((M > 64 || ((mid_wanted(M, N, K) || mid_m_prefers_tiles(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K))) &&

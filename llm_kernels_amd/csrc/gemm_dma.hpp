@@ -48,6 +48,13 @@ __device__ __forceinline__ void dma2(uint32_t lds_addr, uint32_t voff, const voi
 #define LLMK_WAIT_VMCNT_0 0x0F70
 
 
+// 16-bit scale (zero-extended element) -> fp32, without a branch: with one the compiler moves the scale FMAs out from between the matrix
+// instructions, behind the blocks of the branch.
+__device__ __forceinline__ float scale16_f32(unsigned raw, int dt) {
+    const unsigned f16 = dt == LLMK_F16 ? ~0u : 0u;
+    return __uint_as_float((__float_as_uint(f16_to_f32((unsigned short)raw)) & f16) | ((raw << 16) & ~f16));
+}
+
 // Unscaled kinds accumulate inside the MFMA over the whole K range: two 16x16x32 half-precision MFMAs, or two
 // 16x16x64 int8 MFMAs whose int32 accumulators travel as raw bits in the fp32 accumulator registers.
 template <int KIND>
@@ -98,15 +105,20 @@ __device__ __forceinline__ v4i w4_word_to_f16x8(unsigned w, v2h sc) {
     o[3] = (int)__builtin_amdgcn_perm(p37, p26, 0x07060302u);
     return o;
 }
-// The same for bf16, which has no packed arithmetic here: byte -> fp32 converts, one fma per weight ((q - 8) * scale is
-// exact in fp32: 15 significant bits) and one rounding to bf16, the value nk_dequant_bf16_kernel stores.
+// The same for bf16, which has no packed arithmetic here: the fp16 numbers 1024 + q and 1024 + 16 q are operands of one mixed fma per weight
+// ((q - 8) * scale is exact in fp32: 15 significant bits; so are 1032 * scale and 72 * scale), then one rounding to bf16, the value
+// nk_dequant_bf16_kernel stores.  17 instructions a word; by byte -> fp32 converts they were 28.
 __device__ __forceinline__ v4i w4_word_to_bf16x8(unsigned w, float sc) {
-    const unsigned even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
-    const float c = -8.0f * sc;
+    const float c8 = -1032.0f * sc, s16 = 0.0625f * sc, c72 = -72.0f * sc;
+    const unsigned w8 = w >> 8;
+    const v2h e0 = w4_as_h2((w & 0x000f000fu) | 0x64006400u), o0 = w4_as_h2((w & 0x00f000f0u) | 0x64006400u);      // elements 0, 4 and 1, 5
+    const v2h e1 = w4_as_h2((w8 & 0x000f000fu) | 0x64006400u), o1 = w4_as_h2((w8 & 0x00f000f0u) | 0x64006400u);    // 2, 6 and 3, 7
     v4i o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        o[i] = (int)pack_bf16x2(fmaf((float)((even >> (8 * i)) & 0xffu), sc, c), fmaf((float)((odd >> (8 * i)) & 0xffu), sc, c));
+    for (int h = 0; h < 2; ++h) {
+        o[2 * h] = (int)pack_bf16x2(fmaf((float)e0[h], sc, c8), fmaf((float)o0[h], s16, c72));
+        o[2 * h + 1] = (int)pack_bf16x2(fmaf((float)e1[h], sc, c8), fmaf((float)o1[h], s16, c72));
+    }
     return o;
 }
 // one packed word and its group scale (fp16 bits) -> eight weights in the activation type of the kind
@@ -514,7 +526,7 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
             for (int i = 0; i < MI; ++i) {
                 if constexpr (AS16) {
                     const unsigned raw = ((const unsigned*)Ss)[i * 16];
-                    sa[i] = (p.s_dtype == LLMK_F16 ? f16_to_f32((unsigned short)raw) : bf16_to_f32((unsigned short)raw)) * bs;
+                    sa[i] = scale16_f32(raw, p.s_dtype) * bs;
                 } else {
                     sa[i] = Ss[i * 16] * bs;
                 }
@@ -752,6 +764,25 @@ inline bool dma_eligible(const DirectArgs& p, int esz = 1) {
 
 constexpr int D_LDS_MAX = 160 * 1024;
 
+// the pass over z planes of partial sums
+template <int KIND>
+int launch_splitk_sum(const DirectArgs& p, int z, hipStream_t stream, const char* name) {
+    const int64_t mn = (int64_t)p.M * p.N;
+    const unsigned blocks = (unsigned)cdiv64(cdiv64(mn, 4), 256);
+    if constexpr (KIND == K_I8_ROWCOL) {
+        const int32_t* part = (const int32_t*)p.partial;
+        if (p.c_dtype == LLMK_BF16) splitk_sum_rowcol_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(part, p, mn, z);
+        else if (p.c_dtype == LLMK_F16) splitk_sum_rowcol_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(part, p, mn, z);
+        else splitk_sum_rowcol_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(part, p, mn, z);
+    } else {
+        if (p.c_dtype == LLMK_BF16) splitk_sum_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
+        else if (p.c_dtype == LLMK_F16) splitk_sum_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
+        else splitk_sum_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
+    }
+    LLMK_CHECK_LAUNCH(name);
+    return LLMK_OK;
+}
+
 // p.a_s: fp32, or with AS16 the 16-bit scales of dtype p.s_dtype as the caller passed them; p.s_dtype describes b_s.
 template <int KIND, bool GROUPED, int MI, bool AS16 = false>
 int launch_dma_mi(const DirectArgs& p, hipStream_t stream, const char* name) {
@@ -766,22 +797,7 @@ int launch_dma_mi(const DirectArgs& p, hipStream_t stream, const char* name) {
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
     kern<<<grid, D_THREADS, lds_bytes, stream>>>(p);
     LLMK_CHECK_LAUNCH(name);
-    if (split) {
-        const int64_t mn = (int64_t)p.M * p.N;
-        const unsigned blocks = (unsigned)cdiv64(cdiv64(mn, 4), 256);
-        if constexpr (KIND == K_I8_ROWCOL) {
-            const int32_t* part = (const int32_t*)p.partial;
-            if (p.c_dtype == LLMK_BF16) splitk_sum_rowcol_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(part, p, mn, p.ksplit);
-            else if (p.c_dtype == LLMK_F16) splitk_sum_rowcol_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(part, p, mn, p.ksplit);
-            else splitk_sum_rowcol_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(part, p, mn, p.ksplit);
-            LLMK_CHECK_LAUNCH(name);
-            return LLMK_OK;
-        }
-        if (p.c_dtype == LLMK_BF16) splitk_sum_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, p.ksplit);
-        else if (p.c_dtype == LLMK_F16) splitk_sum_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, p.ksplit);
-        else splitk_sum_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, p.ksplit);
-        LLMK_CHECK_LAUNCH(name);
-    }
+    if (split) return launch_splitk_sum<KIND>(p, p.ksplit, stream, name);
     return LLMK_OK;
 }
 

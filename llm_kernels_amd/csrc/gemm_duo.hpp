@@ -1,0 +1,469 @@
+// Tile kernel for problems of about one round of 32 MI x 128 tiles: two groups of four waves (one wave of each group per SIMD) take
+// turns.  K goes by in sub-blocks of 128 bytes; group p multiplies the sub-blocks u with u mod 2 == p, each wave a 16 MI x 64 share of
+// the tile.  In phase u group u mod 2 requests sub-block u + 3, fetches the fragments of sub-block u from LDS and (4-bit weights)
+// expands the weight rows of sub-block u + 1, while the other group does nothing but multiply sub-block u - 1 from registers; one
+// barrier ends the phase.  The two sums of an output meet in LDS at the end.
+//
+// What bounds it: the CU's path from L2 (32 KB a phase of a 128 x 128 tile, 0.31 us of the 0.25 us that its products take) and the start and end of
+// every phase.  Against the eight waves of gemm_dma_kernel, which share one 128-byte step: a wave tile is 64 x 64 instead of 32 x 64
+// (fragments of 16 KB instead of 24 for the same products), only waves that have nothing to multiply wait for the address path, and a
+// workgroup can be any multiple of 32 rows high, which is worth most where a few rows over a tile height would start another round.
+#pragma once
+#include <algorithm>
+
+#include "gemm_mid.hpp"
+
+namespace llmk {
+
+constexpr int DU_BN = 128, DU_THREADS = 512, DU_SLOTS = 4;
+// 4-bit weights: activations in four slots, expanded weight rows in two; otherwise both operands of a sub-block in one slot
+constexpr int du_a(int mi) { return 32 * mi * 128; }
+constexpr int du_b() { return DU_BN * 128; }
+constexpr int du_windows(int mi) { return 2 * 32 * mi * 4 * 4; }             // two windows of activation scales, four sub-blocks each
+constexpr int du_lds(int kind, int mi) {
+    return DU_SLOTS * du_a(mi) + (is_w4nk(kind) ? 2 : DU_SLOTS) * du_b() + (kind == K_FP8_BLOCK || kind == K_I8_BLOCK ? du_windows(mi) + D_MAX_KT * 4 : 0);
+}
+
+template <int KIND, int MI, bool AS16 = false>
+__global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
+    constexpr bool SCALED = (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK), ROWCOL = (KIND == K_I8_ROWCOL), W4NK = is_w4nk(KIND);
+    static_assert(SCALED || ROWCOL || W4NK, "8-bit operands, or 16-bit activations with row-packed 4-bit weights");
+    constexpr int ESZ = is_half(KIND) ? 2 : 1, BM = 32 * MI, WR = 16 * MI;
+    constexpr int A_SLOT = du_a(MI), B_SLOT = du_b(), B0 = DU_SLOTS * A_SLOT, NB = W4NK ? 2 : DU_SLOTS, SW = B0 + NB * B_SLOT;
+    constexpr int LP = MI + 4;                               // loads of a wave from one of its turns to the end of the next
+    constexpr int NSW = (2 * MI + 7) / 8;                    // scale loads per wave and window (16 rows x 4 sub-blocks each)
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4, w4 = wave & 3;
+    const int wm = (wave >> 1) & 1, wn = wave & 1;
+    const int N = p.N;
+    const int K = p.K * ESZ;                                 // row length in bytes
+    const int KT_all = K >> 7;
+    int kt0 = 0, KT = KT_all;                                // sub-blocks [kt0, kt0 + KT) of this workgroup
+    if (p.ksplit > 1) {
+        const int per = (KT_all + p.ksplit - 1) / p.ksplit;
+        kt0 = (int)blockIdx.z * per;
+        KT = max(0, min(per, KT_all - kt0));
+    }
+    int tile_n, tile_m;
+    xcd_tile((int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
+    const int n0 = tile_n * DU_BN, m_start = tile_m * BM, m_end = min(p.M, m_start + BM);
+    float* const bsl = (float*)(lds + SW + du_windows(MI));
+
+    // ---- source offsets (bytes, 32 bit).  A piece = 8 rows x 128 bytes = one load instruction; chunks XOR-swizzled with (row >> 1) & 7
+    // as everywhere.  Weight rows are permuted inside each 64 so that a lane ends up with two runs of 8 consecutive columns.
+    const int row8 = lane >> 3;
+    uint32_t aoff[MI], boff[4];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int R = 8 * (w4 * MI + i) + row8;
+        aoff[i] = (uint32_t)min(m_start + R, m_end - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((R >> 1) & 7)) * 16u;
+    }
+    auto column = [](int R) { const int rho = R & 63; return (R & 64) + 32 * (rho >> 5) + 8 * ((rho & 15) >> 2) + 4 * ((rho >> 4) & 1) + (rho & 3); };
+    if constexpr (!W4NK) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int R = 8 * (w4 * 4 + i) + row8;
+            boff[i] = (uint32_t)min(n0 + column(R), N - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((R >> 1) & 7)) * 16u;
+        }
+    }
+    // 4-bit weights: in phase f every thread expands 16 weights of sub-block f + 1, quarter t & 3 of weight row t >> 2, from a packed double
+    // word and a group scale requested four phases ago (set f & 3)
+    uint32_t w4_off = 0, w4_soff = 0, w4_dst = 0, w4_sw = 0;
+    int w4_shift = 0;
+    if constexpr (W4NK) {
+        const int R = tid >> 2, q = tid & 3;
+        const uint32_t n = (uint32_t)min(n0 + column(R), N - 1);
+        w4_off = n * (uint32_t)(p.K >> 1) + (uint32_t)q * 8u;
+        w4_soff = n * (uint32_t)(p.K / p.group) * 2u;
+        w4_dst = (uint32_t)(R * 128);
+        w4_sw = (uint32_t)(((2 * q) ^ ((R >> 1) & 7)) * 16);                  // chunk 2 q; chunk 2 q + 1 is at ^ 16
+        w4_shift = __builtin_ctz((unsigned)(p.group >> 6));
+    }
+    uint64_t w4_words[4] = {0, 0, 0, 0};
+    unsigned w4_scale[4] = {0, 0, 0, 0};
+    auto request_words = [&](int set, int u) __attribute__((always_inline)) {
+        if constexpr (W4NK) {
+            const int kb = kt0 + min(u, KT - 1);
+            w4_words[set] = asm_load_b64(w4_off, (const uint8_t*)p.b + (int64_t)kb * 32);
+            w4_scale[set] = asm_load_u16(w4_soff, (const uint8_t*)p.b_s + (int64_t)(kb >> w4_shift) * 2);
+        }
+    };
+    // every use of the words comes behind this (the wait is the caller's business)
+    auto words_landed = [&](int set) __attribute__((always_inline)) {
+        if constexpr (W4NK) asm volatile("" : "+v"(w4_words[set]), "+v"(w4_scale[set]) : : "memory");
+    };
+    auto expand_word = [&](int set, int u, int c) __attribute__((always_inline)) {
+        if constexpr (W4NK)
+            *(v4i*)(lds + B0 + (u & 1) * B_SLOT + w4_dst + (w4_sw ^ (uint32_t)(c * 16))) = w4_word_x8<KIND>((unsigned)(w4_words[set] >> (32 * c)), w4_scale[set]);
+    };
+    auto request = [&](int u) {                              // operands of sub-block u, by the four waves of one group
+        const uint32_t sa = lds_base + (uint32_t)(u & 3) * A_SLOT, sb = lds_base + B0 + (uint32_t)(u & 3) * B_SLOT;
+        const uint8_t* ga = p.a + (int64_t)(kt0 + u) * 128;
+        const uint8_t* gb = p.b + (int64_t)(kt0 + u) * 128;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) dma16(sa + (uint32_t)(w4 * MI + i) * 1024u, aoff[i], ga);
+        if constexpr (!W4NK) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dma16(sb + (uint32_t)(w4 * 4 + i) * 1024u, boff[i], gb);
+        }
+    };
+    // scale window w (sub-blocks 4 w .. 4 w + 3), [row][sub-block] dwords: lane l requests row l >> 2 of 16, sub-block 4 w + (l & 3)
+    uint32_t srow[NSW];
+#pragma unroll
+    for (int i = 0; i < NSW; ++i)
+        srow[i] = SCALED ? (uint32_t)min(m_start + 16 * min(wave + 8 * i, 2 * MI - 1) + (lane >> 2), m_end - 1) * (uint32_t)KT_all : 0;
+    auto request_scales = [&](int window) {
+        if constexpr (SCALED) {
+            const int w = __builtin_amdgcn_readfirstlane(window);
+            const uint32_t kb = (uint32_t)min(kt0 + 4 * w + (lane & 3), kt0 + KT - 1);
+#pragma unroll
+            for (int i = 0; i < NSW; ++i) {
+                const uint32_t dst = lds_base + SW + (uint32_t)(w & 1) * (du_windows(MI) / 2) + (uint32_t)min(wave + 8 * i, 2 * MI - 1) * 256u;
+                if constexpr (AS16) dma2(dst, (srow[i] + kb) * 2u, p.a_s);
+                else dma4(dst, (srow[i] + kb) * 4u, p.a_s);
+            }
+        }
+    };
+
+    // acc[i][j][q] = C[row 16 i + r][column 32 (j >> 1) + 8 g + 4 (j & 1) + q] of the wave's tile, over the group's sub-blocks.  The
+    // products of a tile row wait in t and are scaled while the next row is multiplied.
+    v4f acc[MI][4], t[4];
+    v8i bf[4], af[MI];
+    float sa[MI];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+        t[j] = (v4f){0.f, 0.f, 0.f, 0.f};
+    }
+    auto clear = [&]() {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bf[j] = (v8i){0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            af[i] = (v8i){0, 0, 0, 0, 0, 0, 0, 0};
+            sa[i] = 0.f;
+        }
+    };
+    clear();
+    const int lo = r * 128 + ((g ^ ((r >> 1) & 7)) * 16);
+    const int hi = r * 128 + (((g + 4) ^ ((r >> 1) & 7)) * 16);
+    auto ldfrag = [&](const uint8_t* base) {
+        const v4i x = *(const v4i*)(base + lo), y = *(const v4i*)(base + hi);
+        return (v8i){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    };
+    auto fetch = [&](int u) {
+        const uint8_t* const As = lds + (u & 3) * A_SLOT + wm * WR * 128;
+        const uint8_t* const Bs = lds + B0 + (u & (NB - 1)) * B_SLOT + wn * 64 * 128;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bf[j] = ldfrag(Bs + j * 2048);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) af[i] = ldfrag(As + i * 2048);
+        if constexpr (SCALED) {
+            const float bs = bsl[u];
+            const float* const Ss = (const float*)(lds + SW + ((u >> 2) & 1) * (du_windows(MI) / 2)) + (wm * WR + r) * 4 + (u & 3);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                if constexpr (AS16) {
+                    const unsigned raw = ((const unsigned*)Ss)[i * 64];
+                    sa[i] = scale16_f32(raw, p.s_dtype) * bs;
+                } else {
+                    sa[i] = Ss[i * 64] * bs;
+                }
+            }
+        }
+    };
+    // 4-bit weights: in the shadow of its matrix instructions the multiplying group expands its half of sub-block f + 1 of phase f (the slot's
+    // readers finished in the phase before), and requests the words of sub-block f + 5
+    auto multiply = [&](auto expand_c, int f) __attribute__((always_inline)) {
+        constexpr bool EXPAND = W4NK && decltype(expand_c)::value;
+        if constexpr (EXPAND) words_landed(f & 3);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            if constexpr (EXPAND) {
+                if (i < 2) expand_word(f & 3, f + 1, i);
+                if (i == 2) request_words(f & 3, f + 5);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (SCALED) {
+                    if (i > 0) acc[i - 1][j] += raw_f32<KIND>(t[j]) * sa[i - 1];
+                    t[j] = step_raw<KIND>(bf[j], af[i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    acc[i][j] = mma_plain<KIND>(bf[j], af[i], acc[i][j]);
+                }
+            }
+            if constexpr (EXPAND) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (SCALED) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[MI - 1][j] += raw_f32<KIND>(t[j]) * sa[MI - 1];
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    auto meet = [&](auto left_c) {                           // this wave's LDS accesses, and its loads but the left_c youngest, are done
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(left_c)::value < 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(left_c)::value < 0 ? 0 : decltype(left_c)::value) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    const std::integral_constant<int, -1> any;
+    const std::integral_constant<int, 0> none;
+    const std::integral_constant<int, LP> c_l;
+    const std::integral_constant<int, LP + (SCALED ? NSW : 0)> c_ls;
+
+    // Turn of the fetching group in phase u.  The operands requested in its last turn, two phases ago, have landed when only the loads since
+    // are in flight: sub-block u + 1 is complete, and so are the words that the group expands in the next two phases.  SCALES: this turn also
+    // requests the next scale window, behind its operands, so that the turn after it waits for it; the window it overwrites was last read
+    // in phase u - 1 or before.
+    auto turn = [&](int u, auto scales_c) __attribute__((always_inline)) {
+        constexpr bool SCALES = SCALED && decltype(scales_c)::value;
+        request(u + 3);
+        if constexpr (SCALES) request_scales((u >> 2) + 1);
+        fetch(u);
+        if constexpr (W4NK) {
+            __builtin_amdgcn_sched_barrier(0);
+            words_landed(u & 3);
+            expand_word(u & 3, u + 1, 0);
+            expand_word(u & 3, u + 1, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            request_words(u & 3, u + 5);
+        }
+        if constexpr (SCALES) meet(c_ls);
+        else meet(c_l);
+    };
+    // The same where little or nothing is left to request: every phase waits for all of it, and the words move up a set a phase.
+    auto last_words = [&](int f) __attribute__((always_inline)) {
+        if constexpr (W4NK) {
+            if (f + 1 < KT) {
+                expand_word(0, f + 1, 0);
+                expand_word(0, f + 1, 1);
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                w4_words[i] = w4_words[i + 1];
+                w4_scale[i] = w4_scale[i + 1];
+            }
+            request_words(3, f + 5);
+        }
+    };
+    auto last_meet = [&]() __attribute__((always_inline)) {
+        meet(none);
+        words_landed(3);
+    };
+    auto last_turn = [&](int u) __attribute__((always_inline)) {
+        if (u + 3 < KT) request(u + 3);
+        if constexpr (SCALED) if ((u & 3) < 2 && (u | 3) + 1 < KT) request_scales((u >> 2) + 1);
+        fetch(u);
+        last_words(u);
+        last_meet();
+    };
+    auto all_landed = [&]() __attribute__((always_inline)) {
+        if constexpr (W4NK) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < 4; ++i) words_landed(i);
+        }
+    };
+
+    // ---- the first three sub-blocks; 4-bit weights: the weight rows of the first, and the words of the four behind it
+    if (KT > 0) {
+        request_words(0, 0);
+        if (wave < 4) {
+            if (KT > 1) request(1);
+        } else {
+            request(0);
+            if (KT > 2) request(2);
+        }
+        request_scales(0);
+        if constexpr (SCALED) {
+            const int64_t bs_row = (int64_t)tile_n * KT_all + kt0;
+            for (int i = tid; i < KT; i += DU_THREADS) bsl[i] = ld_scale(p.b_s, bs_row + i, p.s_dtype);
+        }
+        all_landed();
+        expand_word(0, 0, 0);
+        expand_word(0, 0, 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) request_words(i, i + 1);
+        all_landed();
+    }
+    meet(none);
+
+    // ---- each group keeps half of the tile rows of its waves, passes the other half to its counterpart and stores the sums
+    constexpr int H = (MI + 1) / 2;
+    const bool split = p.ksplit > 1;
+    void* const cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
+    const int cdt = split ? LLMK_F32 : p.c_dtype;
+    auto finish = [&](auto grp_c) {
+        constexpr int G = decltype(grp_c)::value, KEEP = G ? H : 0, NKEEP = G ? MI - H : H, GIVE = G ? 0 : H, NGIVE = MI - NKEEP;
+        v4f* const give = (v4f*)lds + wave * (H * 4 * 64) + lane;
+        const v4f* const take = (const v4f*)lds + (wave ^ 4) * (H * 4 * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < NGIVE; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) give[(i * 4 + j) * 64] = acc[GIVE + i][j];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NKEEP; ++i) {
+            const int m = m_start + wm * WR + 16 * (KEEP + i) + r;
+            if (m >= m_end) continue;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int nb = n0 + wn * 64 + 32 * h + 8 * g, nv = N - nb;
+                if (nv <= 0) continue;
+                v4f s[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const v4f o = take[(i * 4 + 2 * h + e) * 64], mine = acc[KEEP + i][2 * h + e];
+                    if constexpr (ROWCOL) s[e] = __builtin_bit_cast(v4f, __builtin_bit_cast(v4i, o) + __builtin_bit_cast(v4i, mine));
+                    else s[e] = o + mine;
+                }
+                const int64_t off = (int64_t)m * N + nb;
+                if constexpr (ROWCOL) {
+                    if (!split) {                            // (a K slice leaves its int32 sums, see splitk_sum_rowcol_kernel)
+                        rowcol_epilogue8(p, s[0], s[1], m, off, nb, nv);
+                        if (!p.c) continue;
+                    }
+                }
+                if (cdt == LLMK_BF16) store_run8<LLMK_BF16>(cout, off, s[0], s[1], nv);
+                else if (cdt == LLMK_F16) store_run8<LLMK_F16>(cout, off, s[0], s[1], nv);
+                else store_run8<LLMK_F32>(cout, off, s[0], s[1], nv);
+            }
+        }
+    };
+
+    // Four phases a loop turn (the last operands they request are those of sub-block 4 q + 6), then phase by phase what is left.
+    const int rounds = KT >= 7 ? (KT - 3) >> 2 : 0;
+    if (wave < 4) {
+        for (int q = 0; q < rounds; ++q) {
+            turn(4 * q, yes);
+            multiply(yes, 4 * q + 1);
+            meet(any);
+            turn(4 * q + 2, no);
+            multiply(yes, 4 * q + 3);
+            meet(any);
+        }
+        all_landed();
+        for (int u = 4 * rounds; u < KT; u += 2) {
+            last_turn(u);
+            last_words(u + 1);
+            multiply(no, 0);
+            last_meet();
+        }
+        finish(std::integral_constant<int, 0>{});
+    } else {
+        for (int q = 0; q < rounds; ++q) {
+            multiply(yes, 4 * q);
+            meet(any);
+            turn(4 * q + 1, yes);
+            multiply(yes, 4 * q + 2);
+            meet(any);
+            turn(4 * q + 3, no);
+        }
+        all_landed();
+        for (int u = 4 * rounds; u < KT; u += 2) {
+            last_words(u);
+            multiply(no, 0);
+            last_meet();
+            if (u + 1 < KT) {
+                last_turn(u + 1);
+            } else {                                         // an odd number of sub-blocks: nothing left to multiply
+                clear();
+                meet(any);
+            }
+        }
+        multiply(no, 0);
+        finish(std::integral_constant<int, 1>{});
+    }
+}
+
+// p.a_s: fp32, or with AS16 the 16-bit scales of dtype p.s_dtype as the caller passed them; p.ksplit / p.partial select the K split.
+template <int KIND, int MI, bool AS16 = false>
+int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
+    static std::atomic<uint64_t> configured{0};
+    auto kern = gemm_duo_kernel<KIND, MI, AS16>;
+    constexpr int lds_bytes = du_lds(KIND, MI);
+    static_assert(lds_bytes <= D_LDS_MAX && 8 * ((MI + 1) / 2) * 4096 <= lds_bytes, "slots, and the exchange of half the sums in them, fit in LDS");
+    if (int rc = llmk_reserve_lds((const void*)kern, lds_bytes, configured, name)) return rc;
+    const bool split = p.ksplit > 1 && p.partial;
+    DirectArgs q = p;
+    q.ksplit = split ? p.ksplit : 1;
+    dim3 grid((unsigned)((p.N + DU_BN - 1) / DU_BN), (unsigned)((p.M + 32 * MI - 1) / (32 * MI)), (unsigned)q.ksplit);
+    if (grid.x == 0 || grid.y == 0) return LLMK_OK;
+    kern<<<grid, DU_THREADS, lds_bytes, stream>>>(q);
+    LLMK_CHECK_LAUNCH(name);
+    return split ? launch_splitk_sum<KIND>(q, q.ksplit, stream, name) : LLMK_OK;
+}
+
+// Tile heights that are built (32 mi rows).  Block-scaled kinds end at 128 rows: at 160 the fragments of a sub-block and the products that
+// wait for their scales spill.
+template <int KIND>
+constexpr bool duo_built(int mi) {
+    return mi >= 3 && mi <= (is_w4nk(KIND) ? 6 : (KIND == K_I8_ROWCOL ? 5 : 4));
+}
+// Estimated microseconds: base + rounds of 256 workgroups x (round + sub-blocks x step[mi - 3]) + out x MB of the output, and for K slices
+// split + plane x MB of the fp32 planes.  A fit of 4 to 7 % rms to 300 random shapes a kind of M 64 to 4096, N 1024 to 28672, K 1024 to
+// 14336, every height and up to eight slices timed, means of cached weights and of weights from HBM.
+struct DuoModel {
+    float base, round, step[4], split, plane, out;
+};
+template <int KIND>
+constexpr DuoModel duo_model() {
+    if (KIND == K_FP8_BLOCK) return {1.97f, 1.43f, {0.392f, 0.450f, 0.f, 0.f}, 3.6f, 0.47f, 0.45f};
+    if (KIND == K_I8_BLOCK) return {2.19f, 1.99f, {0.433f, 0.532f, 0.f, 0.f}, 2.9f, 0.49f, 0.43f};
+    if (KIND == K_I8_ROWCOL) return {2.79f, 1.59f, {0.355f, 0.406f, 0.470f, 0.f}, 2.9f, 0.47f, 0.57f};
+    return {2.29f, 1.78f, {0.421f, 0.487f, 0.561f, 0.639f}, 3.7f, 0.46f, 0.43f};
+}
+struct DuoPlan {
+    int mi, z;                                               // mi == 0: not for this kernel
+    double cost;
+};
+// The cheapest height and number of K slices with `scratch` bytes for their planes (at most DU_MAX_PLANES: what is reported as scratch
+// stays within the array that serves calls without any).
+constexpr int64_t DU_MAX_PLANES = LLMK_STATIC_SCRATCH_BYTES;
+template <int KIND>
+DuoPlan duo_plan(const DirectArgs& p, int64_t scratch) {
+    constexpr int ESZ = is_half(KIND) ? 2 : 1;
+    constexpr DuoModel m = duo_model<KIND>();
+    DuoPlan best{0, 1, 1e30};
+    if (p.M <= 64 || !dma_eligible(p, ESZ) || (is_w4nk(KIND) && (p.group < 64 || (p.group & (p.group - 1))))) return best;
+    const int KT = (p.K * ESZ) >> 7;
+    const int64_t gx = (p.N + DU_BN - 1) / DU_BN, planes = std::min(scratch, DU_MAX_PLANES);
+    const double out = (double)p.M * p.N * 1e-6;
+    for (int mi = 3; mi <= 6; ++mi) {
+        if (!duo_built<KIND>(mi)) continue;
+        const int64_t tiles = gx * ((p.M + 32 * mi - 1) / (32 * mi));
+        constexpr int Z[] = {1, 2, 3, 4, 6, 8};
+        for (int z : Z) {
+            if (z > 1 && (tiles * z > LLMK_CUS || KT / z < 6 || (int64_t)z * p.M * p.N * 4 > planes)) break;
+            const double rounds = (double)((tiles * z + LLMK_CUS - 1) / LLMK_CUS);
+            const double c = m.base + rounds * (m.round + (KT + z - 1) / z * m.step[mi - 3]) + 2.0 * m.out * out + (z > 1 ? m.split + 4.0 * m.plane * out * z : 0.0);
+            if (c < best.cost) best = {mi, z, c};
+        }
+    }
+    return best;
+}
+template <int KIND, bool AS16 = false>
+int launch_duo_plan(DirectArgs p, const DuoPlan& pl, void* workspace, hipStream_t stream, const char* name) {
+    if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; }
+    if constexpr (duo_built<KIND>(6)) if (pl.mi == 6) return launch_duo<KIND, 6, AS16>(p, stream, name);
+    if constexpr (duo_built<KIND>(5)) if (pl.mi == 5) return launch_duo<KIND, 5, AS16>(p, stream, name);
+    return pl.mi == 4 ? launch_duo<KIND, 4, AS16>(p, stream, name) : launch_duo<KIND, 3, AS16>(p, stream, name);
+}
+
+}  // namespace llmk

@@ -290,7 +290,7 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
                 for (int i = 0; i < MT; ++i) {
                     if constexpr (AS16) {
                         const unsigned raw = ((const unsigned*)Ss)[16 * i];
-                        sa[i] = (p.s_dtype == LLMK_F16 ? f16_to_f32((unsigned short)raw) : bf16_to_f32((unsigned short)raw)) * bs;
+                        sa[i] = scale16_f32(raw, p.s_dtype) * bs;
                     } else {
                         sa[i] = Ss[16 * i] * bs;
                     }
@@ -445,21 +445,7 @@ int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
     kern<<<grid, MD_THREADS, lds_bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
-    if (split) {
-        const int64_t mn = (int64_t)p.M * p.N;
-        const unsigned blocks = (unsigned)cdiv64(cdiv64(mn, 4), 256);
-        if constexpr (KIND == K_I8_ROWCOL) {
-            const int32_t* part = (const int32_t*)p.partial;
-            if (p.c_dtype == LLMK_BF16) splitk_sum_rowcol_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(part, p, mn, z);
-            else if (p.c_dtype == LLMK_F16) splitk_sum_rowcol_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(part, p, mn, z);
-            else splitk_sum_rowcol_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(part, p, mn, z);
-        } else {
-            if (p.c_dtype == LLMK_BF16) splitk_sum_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
-            else if (p.c_dtype == LLMK_F16) splitk_sum_kernel<LLMK_F16><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
-            else splitk_sum_kernel<LLMK_F32><<<blocks, 256, 0, stream>>>(p.partial, p.c, mn, z);
-        }
-        LLMK_CHECK_LAUNCH(name);
-    }
+    if (split) return launch_splitk_sum<KIND>(p, z, stream, name);
     return LLMK_OK;
 }
 

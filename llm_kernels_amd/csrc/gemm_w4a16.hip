@@ -3,6 +3,7 @@
 // nibble -> fp16 without integer->float converts: (q | 0x6400) is the fp16 number 1024 + q,
 // ((q << 4) | 0x6400) is 1024 + 16 q; one packed subtract / fma gives q - 8 exactly.
 #include <algorithm>
+#include "gemm_duo.hpp"
 #include "gemm_wave.hpp"
 #include "gemm_wide.hpp"
 #include "stream_ring.hpp"
@@ -998,15 +999,32 @@ llmk::WavePlan nk_wave(const llmk::DirectArgs& p, int64_t scratch) {
     return w;
 }
 
+// What a call beyond 512 rows gets without the kernel of two wave groups, in us: tiles that expand the words themselves (a fit of 2 to 6 % rms), or
+// the 16-bit copy of W and the 16-bit tiles (9 %).
+template <int KIND, int HALF_KIND>
+double nk_large_estimate(const llmk::DirectArgs& p, bool copy) {
+    const llmk::TileChoice c = copy ? llmk::dma_tile_estimate<HALF_KIND, false>(p) : llmk::dma_tile_estimate<KIND, false>(p);
+    const double e = c.cost * (double)p.K / 4096.0, nk = (double)p.N * p.K * 1e-6;
+    constexpr bool BF = KIND == llmk::K_W4NKB;
+    if (copy) return BF ? 6.3 + 1.37 * e + 0.44 * nk : 9.0 + 1.25 * e + 0.59 * nk;
+    switch (c.choice) {
+        case 1: return (BF ? 3.8 : 2.8) + (BF ? 2.08 : 2.19) * e;
+        case 2: return 3.6 + (BF ? 1.59 : 1.55) * e;
+        case 4: return 3.0 + (BF ? 1.38 : 1.45) * e;
+        default: return 2.0 + (BF ? 1.55 : 1.58) * e;
+    }
+}
+
 // The kernels of a call on the [N, K/8] layout, in the order in which they are preferred, and the scratch they use: what
 // llmk_gemm_w4a16_nk runs with `scratch` bytes there, and what llmk_gemm_w4a16_nk_workspace_bytes reports for any amount.
 struct NkPlan {
-    enum { RING, TILES, COPY, RANGES, STREAM, NONE, WAVE } route;
+    enum { RING, TILES, COPY, RANGES, STREAM, NONE, WAVE, DUO } route;
     int nz;
     int64_t bytes;
     llmk::WavePlan wave;
+    llmk::DuoPlan duo;
 };
-NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scratch, bool c8) {
+NkPlan nk_plan_others(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scratch, bool c8) {
     const int nz = (int)((K / 128 + 31) / 32);               // K ranges of the streaming kernels
     const int64_t planes = nz > 1 ? (int64_t)nz * M * N * 4 : 0;
     const bool sums = nz == 1 || ((M * N) % 4 == 0 && scratch >= planes);
@@ -1029,6 +1047,29 @@ NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scra
     // K > 4096: ranges of at most 4096 (each with resident activations) and fp32 partial sums
     if (group % 128 == 0 && M <= 64 && nz > 1 && sums && c8 && ((K / 128 + nz - 1) / nz * 128) % group == 0) return {NkPlan::RANGES, nz, planes, {}};
     return {NkPlan::STREAM, 1, 0, {}};
+}
+
+// The same with the kernel of two wave groups (gemm_duo.hpp) from 65 to 2048 rows, 8 % below the estimate of the route above.  Over 300 random shapes of
+// 64 to 4096 rows fp16 calls were 1.08 and bf16 calls 1.11 times as fast as without, 1 % behind the faster one of each shape.  Others | this
+// one, us: bf16 300 x 14336 x 4096 54 | 45.5, 1024 x 4096 x 4096 48 | 40.7.
+template <int KIND, int HALF_KIND>
+NkPlan nk_plan_of(int64_t M, int64_t N, int64_t K, int group, int64_t scratch, bool c8) {
+    constexpr bool BF = KIND == llmk::K_W4NKB;
+    const NkPlan pl = nk_plan_others(M, N, K, group, BF, scratch, c8);
+    if (M <= 64 || M > 2048) return pl;
+    llmk::DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
+    const llmk::DuoPlan d = llmk::duo_plan<KIND>(p, scratch);
+    if (!d.mi) return pl;
+    double other = 1e30;                                     // (streaming kernels this far out: no scratch for a copy)
+    if (pl.route == NkPlan::WAVE) other = 1.05 * pl.wave.cost;
+    else if (pl.route == NkPlan::TILES && M <= 512) other = nk_other_estimate<KIND>(p);
+    else if (pl.route == NkPlan::TILES || pl.route == NkPlan::COPY) other = nk_large_estimate<KIND, HALF_KIND>(p, pl.route == NkPlan::COPY);
+    if (1.08 * d.cost >= other) return pl;
+    return {NkPlan::DUO, 1, d.z > 1 ? (int64_t)d.z * M * N * 4 : 0, {}, d};
+}
+NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scratch, bool c8) {
+    return bf ? nk_plan_of<llmk::K_W4NKB, llmk::K_BF16>(M, N, K, group, scratch, c8) : nk_plan_of<llmk::K_W4NK, llmk::K_F16>(M, N, K, group, scratch, c8);
 }
 
 // launch shape of the Marlin-layout kernel for a given problem
@@ -1106,6 +1147,17 @@ extern "C" int llmk_gemm_w4a16_wave_shape(int marlin, int ac_dtype, int64_t M, i
     const bool bf = ac_dtype == LLMK_BF16;
     const NkPlan pl = nk_plan(M, N, K, groupsize, bf, scratch_bytes, true);
     return pl.route == NkPlan::WAVE ? llmk::wave_shape(pl.wave, nk_rounded_weights(M, N, K, groupsize, bf), shape) : 0;
+}
+
+extern "C" int llmk_gemm_w4a16_duo_shape(int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes, int32_t* shape) {
+    if (!shape || M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
+    if (groupsize == -1) groupsize = (int)K;
+    if (groupsize < 8 || groupsize % 8 || K % groupsize) return 0;
+    const NkPlan pl = nk_plan(M, N, K, groupsize, ac_dtype == LLMK_BF16, scratch_bytes, true);
+    if (pl.route != NkPlan::DUO) return 0;
+    shape[0] = 32 * pl.duo.mi;
+    shape[1] = pl.duo.z;
+    return 1;
 }
 
 extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, const void* s, int64_t M, int64_t N,
@@ -1231,6 +1283,10 @@ extern "C" int llmk_gemm_w4a16_nk(const void* a, const int32_t* b_packed, void* 
                           : llmk::launch_w4a16_wave_plan<llmk::K_W4NK, true>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
             return bf ? llmk::launch_w4a16_wave_plan<llmk::K_W4NKB, false>(p, pl.wave, st, "gemm_w4a16_nk(wave)")
                       : llmk::launch_w4a16_wave_plan<llmk::K_W4NK, false>(p, pl.wave, st, "gemm_w4a16_nk(wave)");
+        case NkPlan::DUO:
+            p.b = (const uint8_t*)b_packed; p.b_s = s; p.group = groupsize;
+            return bf ? llmk::launch_duo_plan<llmk::K_W4NKB>(p, pl.duo, workspace, st, "gemm_w4a16_nk(duo)")
+                      : llmk::launch_duo_plan<llmk::K_W4NK>(p, pl.duo, workspace, st, "gemm_w4a16_nk(duo)");
         case NkPlan::RING:                               // bf16 decode; fp16 reaches that kernel through launch_nk_stream
             return launch_nk_ring(a, b_packed, S, c, (int)M, (int)N, (int)K, pl.nz, (float*)workspace, true, st);
         case NkPlan::TILES:

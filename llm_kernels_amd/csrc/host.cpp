@@ -403,7 +403,8 @@ PyObject* int8_gemm_per_token(const Args& g) {
     require(a_s_in.numel() == M && b_s_in.numel() == N, "need one scale per token and per output channel");
     const at::ScalarType out = default_dtype();
     const bool want_acc = g.integer(4) != 0;
-    Scratch ws(g, a, M <= 512 ? g.st->llmk_gemm_workspace_bytes(M, N, K) : 0);        // only the K split of mid-size M uses scratch here
+    // (the scratch of K slices; not that of a split last round of tiles, which K from 8192 on has beyond 512 rows and this kind does not use)
+    Scratch ws(g, a, M <= 512 || K < 8192 ? g.st->llmk_gemm_workspace_bytes(M, N, K) : 0);
     at::Tensor c, acc;
     unlocked([&] {
         const at::Tensor a_s = as_type(a_s_in, at::kFloat).contiguous(), b_s = as_type(b_s_in, at::kFloat).contiguous();
