@@ -155,7 +155,9 @@ int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, cons
  *     not 245 x 28672 x 4096), one kernel unpacks the words itself and reads them once per row tile: fp32 partial sums of its K
  *     slices, z * M * N * 4 bytes, optional up to K = 32768 (without: unsplit).  From 17 rows on at least
  *     llmk_gemm_workspace_bytes(M,N,K) is reported, and from 129 rows (257 where 64 x 64 tiles are at most one a CU), or with K beyond
- *     32768 from 65, what the next line needs: words that are not 16-byte aligned go that way there;
+ *     32768 from 65, what the last line needs: words that are not 16-byte aligned go that way there;
+ *   - from 65 rows and K = 1024 on, where it is estimated to be faster, 96- or 128-row tiles that unpack the words once per workgroup: fp32
+ *     partial sums of its K slices, optional (reported is at least what it is without this kernel);
  * everything else the expanded int8 weights, round16(N*K), needed, and behind them llmk_gemm_workspace_bytes(M,N,K) for
  * the int8 tile kernels. */
 int64_t llmk_gemm_w4a8_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_int4);
@@ -217,6 +219,7 @@ int llmk_gemm_w4a16_wave_shape(int marlin, int ac_dtype, int64_t M, int64_t N, i
                                int32_t* shape);
 /* The same for the tile kernel whose two wave groups take turns (from 65 rows on): shape = {rows of a tile, K slices}.  w4a16: [N, K/8]. */
 int llmk_gemm_8bit_duo_shape(int kind, int per_token, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes, int32_t* shape);
+int llmk_gemm_w4a8_duo_shape(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch_bytes, int32_t* shape);
 int llmk_gemm_w4a16_duo_shape(int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes, int32_t* shape);
 
 /* ------------------------------------------------------------------ converters and the one-tile MFMA GEMM

@@ -17,6 +17,7 @@ namespace llmk {
 enum : int { K_FP8_BLOCK = 0, K_I8_BLOCK = 1, K_I8_ROWCOL = 2, K_F16 = 3, K_BF16 = 4,
              K_W4NK = 5,      // fp16 activations x 4-bit weights packed [N, K/8] (tile kernels only)
              K_W4MARLIN = 6,  // the same with weights and scales in the Marlin layout
+             K_W4A8 = 7,      // int8 activations x 4-bit weights packed [N/8, K] with two-level scales, as K_I8_BLOCK once expanded
              K_W4NKB = 8 };   // K_W4NK with bf16 activations (bf16 weights (q - 8) * scale)
 
 constexpr bool is_w4nk(int kind) { return kind == K_W4NK || kind == K_W4NKB; }

@@ -138,9 +138,10 @@ __device__ __forceinline__ uint64_t asm_load_b64(uint32_t voff, const void* sbas
     asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(v) : "v"(voff), "s"(sbase) : "memory");
     return v;
 }
+template <int OFF = 0>
 __device__ __forceinline__ v4i asm_load_b128(uint32_t voff, const void* sbase) {
     v4i v;
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(v) : "v"(voff), "s"(sbase) : "memory");
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(v) : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
     return v;
 }
 __device__ __forceinline__ unsigned asm_load_u16(uint32_t voff, const void* sbase) {

@@ -4,6 +4,8 @@
 // expands the weight rows of sub-block u + 1, while the other group does nothing but multiply sub-block u - 1 from registers; one
 // barrier ends the phase.  The two sums of an output meet in LDS at the end.
 //
+// K_W4A8: 1024 x 4096 x 4096 30.8 us in one launch, 36.7 as expansion pass and the int8 kernel (37.7 | 33.4 with the quantiser).
+//
 // What bounds it: the CU's path from L2 (32 KB a phase of a 128 x 128 tile, 0.31 us of the 0.25 us that its products take) and the start and end of
 // every phase.  Against the eight waves of gemm_dma_kernel, which share one 128-byte step: a wave tile is 64 x 64 instead of 32 x 64
 // (fragments of 16 KB instead of 24 for the same products), only waves that have nothing to multiply wait for the address path, and a
@@ -20,17 +22,21 @@ constexpr int DU_BN = 128, DU_THREADS = 512, DU_SLOTS = 4;
 constexpr int du_a(int mi) { return 32 * mi * 128; }
 constexpr int du_b() { return DU_BN * 128; }
 constexpr int du_windows(int mi) { return 2 * 32 * mi * 4 * 4; }             // two windows of activation scales, four sub-blocks each
-constexpr int du_lds(int kind, int mi) {
-    return DU_SLOTS * du_a(mi) + (is_w4nk(kind) ? 2 : DU_SLOTS) * du_b() + (kind == K_FP8_BLOCK || kind == K_I8_BLOCK ? du_windows(mi) + D_MAX_KT * 4 : 0);
+constexpr bool du_scaled(int kind) { return kind == K_FP8_BLOCK || kind == K_I8_BLOCK || kind == K_W4A8; }
+constexpr bool du_expands(int kind) { return is_w4nk(kind) || kind == K_W4A8; }
+constexpr int du_lds(int kind, int mi) {                                      // K_W4A8: + du_table bytes
+    return DU_SLOTS * du_a(mi) + (du_expands(kind) ? 2 : DU_SLOTS) * du_b() + (du_scaled(kind) ? du_windows(mi) + D_MAX_KT * 4 : 0);
 }
+constexpr int du_table(int sub_blocks) { return sub_blocks * DU_BN * 4; }     // second-level scales and zero points, see below
 
 template <int KIND, int MI, bool AS16 = false>
 __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
-    constexpr bool SCALED = (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK), ROWCOL = (KIND == K_I8_ROWCOL), W4NK = is_w4nk(KIND);
-    static_assert(SCALED || ROWCOL || W4NK, "8-bit operands, or 16-bit activations with row-packed 4-bit weights");
+    constexpr bool SCALED = du_scaled(KIND), ROWCOL = (KIND == K_I8_ROWCOL), W4NK = is_w4nk(KIND), W4A8 = (KIND == K_W4A8), EXPANDS = W4NK || W4A8;
+    static_assert(SCALED || ROWCOL || W4NK, "8-bit operands, or 4-bit weights");
+    constexpr int MATH = W4A8 ? K_I8_BLOCK : KIND;           // the products once the weights are expanded
     constexpr int ESZ = is_half(KIND) ? 2 : 1, BM = 32 * MI, WR = 16 * MI;
-    constexpr int A_SLOT = du_a(MI), B_SLOT = du_b(), B0 = DU_SLOTS * A_SLOT, NB = W4NK ? 2 : DU_SLOTS, SW = B0 + NB * B_SLOT;
-    constexpr int LP = MI + 4;                               // loads of a wave from one of its turns to the end of the next
+    constexpr int A_SLOT = du_a(MI), B_SLOT = du_b(), B0 = DU_SLOTS * A_SLOT, NB = EXPANDS ? 2 : DU_SLOTS, SW = B0 + NB * B_SLOT;
+    constexpr int LP = MI + (W4A8 ? 2 : 4);                  // loads of a wave from one of its turns to the end of the next
     constexpr int NSW = (2 * MI + 7) / 8;                    // scale loads per wave and window (16 rows x 4 sub-blocks each)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -62,7 +68,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         aoff[i] = (uint32_t)min(m_start + R, m_end - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((R >> 1) & 7)) * 16u;
     }
     auto column = [](int R) { const int rho = R & 63; return (R & 64) + 32 * (rho >> 5) + 8 * ((rho & 15) >> 2) + 4 * ((rho >> 4) & 1) + (rho & 3); };
-    if constexpr (!W4NK) {
+    if constexpr (!EXPANDS) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int R = 8 * (w4 * 4 + i) + row8;
@@ -99,13 +105,68 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         if constexpr (W4NK)
             *(v4i*)(lds + B0 + (u & 1) * B_SLOT + w4_dst + (w4_sw ^ (uint32_t)(c * 16))) = w4_word_x8<KIND>((unsigned)(w4_words[set] >> (32 * c)), w4_scale[set]);
     };
+    // int8 activations: its products keep the multiplying group's vector ALU busy, so the fetching one expands.  In its turn of phase u thread t
+    // of the group takes eight words of sub-block u + 1, packed row (t >> 4) & 15, elements 8 (t & 15) .. + 7, requested four phases ago (set
+    // (u >> 1) & 1).  A 16-bit lane holds q << 4 a, q being nibble a of a half word (a = 3: q); times s4 << (8 - 4 a) (a = 3: 8) plus
+    // (-z4 s4) << 8 its high byte is the int8 weight with its wrap.  tab: that factor and that term of every row of the tile, [sub-block][row].
+    unsigned* const tab = (unsigned*)(bsl + D_MAX_KT);
+    uint32_t w8_off = 0, w8_dst[2] = {0, 0};
+    if constexpr (W4A8) {
+        const int pr = (tid >> 4) & 15, k8 = tid & 15;
+        w8_off = (uint32_t)min((n0 >> 3) + pr, (N >> 3) - 1) * (uint32_t)(K * 4) + (uint32_t)k8 * 32u;
+        // LDS rows of the packed row's columns i: R0 + 16 (i >> 2) + (i & 3)
+        const int R0 = 64 * (pr >> 3) + 32 * ((pr >> 2) & 1) + 4 * (pr & 3);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) w8_dst[h] = (uint32_t)((R0 + 2 * h) * 128 + (((k8 >> 1) ^ (((R0 + 2 * h) >> 1) & 7)) * 16) + (k8 & 1) * 8);
+    }
+    v4i w8_words[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};
+    auto request_words8 = [&](int set, int u) __attribute__((always_inline)) {
+        if constexpr (W4A8) {
+            const uint8_t* const base = p.b + (int64_t)(kt0 + min(u, KT - 1)) * 512;
+            w8_words[set][0] = asm_load_b128(w8_off, base);
+            w8_words[set][1] = asm_load_b128<16>(w8_off, base);
+        }
+    };
+    auto words8_landed = [&](int set) __attribute__((always_inline)) {
+        if constexpr (W4A8) asm volatile("" : "+v"(w8_words[set][0]), "+v"(w8_words[set][1]) : : "memory");
+    };
+    auto expand8 = [&](int set, int u) __attribute__((always_inline)) {
+        if constexpr (W4A8) {
+            typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+            auto lanes = [](unsigned v) { return __builtin_bit_cast(us2, v); };
+            auto bits = [](us2 v) { return __builtin_bit_cast(unsigned, v); };
+            const v4i* const row = (const v4i*)(tab + u * DU_BN + 8 * ((tid >> 4) & 15));
+            const v4i sc[2] = {row[0], row[1]};
+            uint8_t* const dst = lds + B0 + (u & 1) * B_SLOT;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {           // nibbles 4 half .. + 3
+                const unsigned sel = half ? 0x07060302u : 0x05040100u;
+                unsigned h[4];                               // elements 2 e, 2 e + 1 of the eight
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    h[e] = __builtin_amdgcn_perm((unsigned)w8_words[set][e >> 1][2 * (e & 1) + 1], (unsigned)w8_words[set][e >> 1][2 * (e & 1)], sel);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const us2 v = lanes((unsigned)sc[half][a]), mul = __builtin_shufflevector(v, v, 0, 0), add = __builtin_shufflevector(v, v, 1, 1);
+                    unsigned y[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const us2 x = a == 3 ? lanes(h[e]) >> (unsigned short)12 : lanes(h[e] & (0x000f000fu << (4 * a)));
+                        y[e] = bits(x * mul + add);
+                    }
+                    const uint64_t o = (uint64_t)__builtin_amdgcn_perm(y[1], y[0], 0x07050301u) | (uint64_t)__builtin_amdgcn_perm(y[3], y[2], 0x07050301u) << 32;
+                    *(uint64_t*)(dst + w8_dst[a >> 1] + (a & 1) * 128 + half * 2048) = o;
+                }
+            }
+        }
+    };
     auto request = [&](int u) {                              // operands of sub-block u, by the four waves of one group
         const uint32_t sa = lds_base + (uint32_t)(u & 3) * A_SLOT, sb = lds_base + B0 + (uint32_t)(u & 3) * B_SLOT;
         const uint8_t* ga = p.a + (int64_t)(kt0 + u) * 128;
         const uint8_t* gb = p.b + (int64_t)(kt0 + u) * 128;
 #pragma unroll
         for (int i = 0; i < MI; ++i) dma16(sa + (uint32_t)(w4 * MI + i) * 1024u, aoff[i], ga);
-        if constexpr (!W4NK) {
+        if constexpr (!EXPANDS) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) dma16(sb + (uint32_t)(w4 * 4 + i) * 1024u, boff[i], gb);
         }
@@ -181,7 +242,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     auto multiply = [&](auto expand_c, int f) __attribute__((always_inline)) {
         constexpr bool EXPAND = W4NK && decltype(expand_c)::value;
         if constexpr (EXPAND) words_landed(f & 3);
-        __builtin_amdgcn_s_setprio(1);
+        if constexpr (W4NK) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
             if constexpr (EXPAND) {
@@ -191,8 +252,8 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if constexpr (SCALED) {
-                    if (i > 0) acc[i - 1][j] += raw_f32<KIND>(t[j]) * sa[i - 1];
-                    t[j] = step_raw<KIND>(bf[j], af[i]);
+                    if (i > 0) acc[i - 1][j] += raw_f32<MATH>(t[j]) * sa[i - 1];
+                    t[j] = step_raw<MATH>(bf[j], af[i]);
                     __builtin_amdgcn_sched_barrier(0);
                 } else {
                     acc[i][j] = mma_plain<KIND>(bf[j], af[i], acc[i][j]);
@@ -209,9 +270,9 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         }
         if constexpr (SCALED) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[MI - 1][j] += raw_f32<KIND>(t[j]) * sa[MI - 1];
+            for (int j = 0; j < 4; ++j) acc[MI - 1][j] += raw_f32<MATH>(t[j]) * sa[MI - 1];
         }
-        __builtin_amdgcn_s_setprio(0);
+        if constexpr (W4NK) __builtin_amdgcn_s_setprio(0);
     };
     auto meet = [&](auto left_c) {                           // this wave's LDS accesses, and its loads but the left_c youngest, are done
         __builtin_amdgcn_sched_barrier(0);
@@ -233,8 +294,17 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     // in phase u - 1 or before.
     auto turn = [&](int u, auto scales_c) __attribute__((always_inline)) {
         constexpr bool SCALES = SCALED && decltype(scales_c)::value;
+        // (the wave that ends the phase goes first; us with the multiplying wave first | none | the fetching one, 1024 x 4096 x 4096: int8 25.8 | 25.1 |
+        // 24.0, fp8 21.4 | 21.4 | 21.1, w4a8 35.5 | 31.7 | 30.8, per token the same, bf16 x 4-bit 42.0 | 43.3 | 44.7)
+        if constexpr (SCALED) __builtin_amdgcn_s_setprio(1);
         request(u + 3);
         if constexpr (SCALES) request_scales((u >> 2) + 1);
+        if constexpr (W4A8) {                                // (in front of the fragments, which leave no registers for it)
+            words8_landed((u >> 1) & 1);
+            expand8((u >> 1) & 1, u + 1);
+            request_words8((u >> 1) & 1, u + 5);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         fetch(u);
         if constexpr (W4NK) {
             __builtin_amdgcn_sched_barrier(0);
@@ -244,6 +314,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             __builtin_amdgcn_sched_barrier(0);
             request_words(u & 3, u + 5);
         }
+        if constexpr (SCALED) __builtin_amdgcn_s_setprio(0);
         if constexpr (SCALES) meet(c_ls);
         else meet(c_l);
     };
@@ -269,9 +340,17 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     auto last_turn = [&](int u) __attribute__((always_inline)) {
         if (u + 3 < KT) request(u + 3);
         if constexpr (SCALED) if ((u & 3) < 2 && (u | 3) + 1 < KT) request_scales((u >> 2) + 1);
+        if constexpr (W4A8) {
+            if (u + 1 < KT) expand8(0, u + 1);
+            w8_words[0][0] = w8_words[1][0];
+            w8_words[0][1] = w8_words[1][1];
+            request_words8(1, u + 5);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         fetch(u);
         last_words(u);
         last_meet();
+        words8_landed(1);
     };
     auto all_landed = [&]() __attribute__((always_inline)) {
         if constexpr (W4NK) {
@@ -279,11 +358,17 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) words_landed(i);
         }
+        if constexpr (W4A8) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            words8_landed(0);
+            words8_landed(1);
+        }
     };
 
     // ---- the first three sub-blocks; 4-bit weights: the weight rows of the first, and the words of the four behind it
     if (KT > 0) {
         request_words(0, 0);
+        request_words8(0, 0);
         if (wave < 4) {
             if (KT > 1) request(1);
         } else {
@@ -295,7 +380,32 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             const int64_t bs_row = (int64_t)tile_n * KT_all + kt0;
             for (int i = tid; i < KT; i += DU_THREADS) bsl[i] = ld_scale(p.b_s, bs_row + i, p.s_dtype);
         }
+        if constexpr (W4A8) {
+            // thread: four (or, at odd counts, one) sub-blocks of a row, rows of a wave side by side
+            const int8_t* const s4 = p.w4_s4 + (int64_t)n0 * KT_all + kt0;
+            const int8_t* const z4 = p.w4_z4 + (int64_t)n0 * KT_all + kt0;
+            const uint32_t row = (uint32_t)min(tid & (DU_BN - 1), N - 1 - n0) * (uint32_t)KT_all;
+            const int shift = (tid & 3) == 3 ? 8 : 8 - 4 * (tid & 3);
+            auto put = [&](int kb, unsigned s, unsigned z) {
+                tab[kb * DU_BN + (tid & (DU_BN - 1))] = (s & 0xffu) << shift | (0u - (z & 0xffu) * (s & 0xffu)) << 24;
+            };
+            if (((KT_all | KT | kt0) & 3) == 0) {
+                for (int kb = 4 * (tid >> 7); kb < KT; kb += 16) {
+                    const unsigned s = ((const Loose<unsigned, 1>*)(s4 + row + kb))->v, z = ((const Loose<unsigned, 1>*)(z4 + row + kb))->v;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) put(kb + b, s >> (8 * b), z >> (8 * b));
+                }
+            } else {
+                for (int kb = tid >> 7; kb < KT; kb += 4) put(kb, (uint8_t)s4[row + kb], (uint8_t)z4[row + kb]);
+            }
+        }
         all_landed();
+        if constexpr (W4A8) {
+            meet(none);                                      // the table
+            if (wave >= 4) expand8(0, 0);
+            request_words8(0, wave < 4 ? 1 : 2);
+            request_words8(1, wave < 4 ? 3 : 4);
+        }
         expand_word(0, 0, 0);
         expand_word(0, 0, 1);
 #pragma unroll
@@ -397,9 +507,12 @@ template <int KIND, int MI, bool AS16 = false>
 int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
     static std::atomic<uint64_t> configured{0};
     auto kern = gemm_duo_kernel<KIND, MI, AS16>;
-    constexpr int lds_bytes = du_lds(KIND, MI);
-    static_assert(lds_bytes <= D_LDS_MAX && 8 * ((MI + 1) / 2) * 4096 <= lds_bytes, "slots, and the exchange of half the sums in them, fit in LDS");
-    if (int rc = llmk_reserve_lds((const void*)kern, lds_bytes, configured, name)) return rc;
+    constexpr int fixed = du_lds(KIND, MI);
+    static_assert(fixed <= D_LDS_MAX && 8 * ((MI + 1) / 2) * 4096 <= fixed, "slots, and the exchange of half the sums in them, fit in LDS");
+    const int KT = (p.K * (is_half(KIND) ? 2 : 1)) >> 7, z = p.ksplit > 1 ? p.ksplit : 1;
+    const int lds_bytes = fixed + (KIND == K_W4A8 ? du_table((KT + z - 1) / z) : 0);
+    if (lds_bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, lds_bytes);
+    if (int rc = llmk_reserve_lds((const void*)kern, KIND == K_W4A8 ? D_LDS_MAX : fixed, configured, name)) return rc;
     const bool split = p.ksplit > 1 && p.partial;
     DirectArgs q = p;
     q.ksplit = split ? p.ksplit : 1;
@@ -407,7 +520,7 @@ int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
     kern<<<grid, DU_THREADS, lds_bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
-    return split ? launch_splitk_sum<KIND>(q, q.ksplit, stream, name) : LLMK_OK;
+    return split ? launch_splitk_sum<KIND == K_W4A8 ? K_I8_BLOCK : KIND>(q, q.ksplit, stream, name) : LLMK_OK;
 }
 
 // Tile heights that are built (32 mi rows).  Block-scaled kinds end at 128 rows: at 160 the fragments of a sub-block and the products that
@@ -424,8 +537,9 @@ struct DuoModel {
 };
 template <int KIND>
 constexpr DuoModel duo_model() {
-    if (KIND == K_FP8_BLOCK) return {1.97f, 1.43f, {0.392f, 0.450f, 0.f, 0.f}, 3.6f, 0.47f, 0.45f};
-    if (KIND == K_I8_BLOCK) return {2.19f, 1.99f, {0.433f, 0.532f, 0.f, 0.f}, 2.9f, 0.49f, 0.43f};
+    if (KIND == K_FP8_BLOCK) return {2.0f, 1.4f, {0.396f, 0.452f, 0.f, 0.f}, 3.4f, 0.50f, 0.48f};
+    if (KIND == K_I8_BLOCK) return {2.4f, 1.4f, {0.417f, 0.502f, 0.f, 0.f}, 2.9f, 0.58f, 0.57f};
+    if (KIND == K_W4A8) return {1.76f, 2.62f, {0.614f, 0.683f, 0.f, 0.f}, 3.0f, 0.55f, 0.37f};
     if (KIND == K_I8_ROWCOL) return {2.79f, 1.59f, {0.355f, 0.406f, 0.470f, 0.f}, 2.9f, 0.47f, 0.57f};
     return {2.29f, 1.78f, {0.421f, 0.487f, 0.561f, 0.639f}, 3.7f, 0.46f, 0.43f};
 }
@@ -451,6 +565,7 @@ DuoPlan duo_plan(const DirectArgs& p, int64_t scratch) {
         constexpr int Z[] = {1, 2, 3, 4, 6, 8};
         for (int z : Z) {
             if (z > 1 && (tiles * z > LLMK_CUS || KT / z < 6 || (int64_t)z * p.M * p.N * 4 > planes)) break;
+            if (KIND == K_W4A8 && du_lds(KIND, mi) + du_table((KT + z - 1) / z) > D_LDS_MAX) continue;
             const double rounds = (double)((tiles * z + LLMK_CUS - 1) / LLMK_CUS);
             const double c = m.base + rounds * (m.round + (KT + z - 1) / z * m.step[mi - 3]) + 2.0 * m.out * out + (z > 1 ? m.split + 4.0 * m.plane * out * z : 0.0);
             if (c < best.cost) best = {mi, z, c};

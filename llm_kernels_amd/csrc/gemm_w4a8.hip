@@ -1,5 +1,6 @@
 // W4A8 GEMM: int8 activations x row-packed uint4 weights with two-level scales.
 #include <algorithm>
+#include "gemm_duo.hpp"
 #include "gemm_wave.hpp"
 #include "gemm_wide.hpp"
 
@@ -56,9 +57,10 @@ __global__ void w4a8_expand_kernel(const int32_t* __restrict__ packed, const int
 // Which path a shape takes (pointer alignment aside) and the scratch that path uses.
 namespace {
 struct W4A8Plan {
-    bool wave;            // wave kernel, else expansion to int8 and the int8 GEMM
+    bool wave;            // wave kernel, else the kernel of two wave groups (duo.mi), else expansion to int8 and the int8 GEMM
     WavePlan shape;
     int64_t bytes;        // scratch the chosen path uses
+    DuoPlan duo;
 };
 // scratch layout of the two-pass path: int8 copy of W | fp32 activation scales | fp32 weight scales | the int8 GEMM's own
 inline int64_t w4a8_two_pass_scales_off(int64_t N, int64_t K) { return (N * K + 255) & ~(int64_t)255; }
@@ -71,8 +73,12 @@ inline int64_t w4a8_widened_bytes(int64_t M, int64_t N, int64_t K) {
 // From there to 512 rows it is taken 12 % below the estimate of the two passes: the expansion, the rounds of the int8 tiles, two
 // launches (a fit of 12 % rms to 25 shapes).  (us, wave | two passes: 512 x 4096 x 4096 25.4 | 31.9, 384 x 4096 x 4096 22 | 30, but 245 x 28672 x 4096 78.9 | 70.4; every row
 // tile unpacks the weights again, so large N K goes the other way.)
+// From 65 rows on the kernel of two wave groups, which expands the words itself, is taken 8 % below the estimate of either: the two passes are the
+// expansion, and the int8 tiles or that kernel on int8 weights, whichever is estimated faster (a fit of 7 % rms to 165 shapes).  Over 300
+// random shapes of 64 to 4096 rows this was 1.05 times as fast as without, at worst level.  Others | this one, us: 1024 x 4096 x 4096
+// 36.7 | 30.8, 425 x 6144 x 4096 32.5 | 25.3, 184 x 14272 x 1664 19.2 | 14.5, but 2373 x 6144 x 4096 79 | 107 and 91 x 5936 x 1024 7.1 | 9.5.
 W4A8Plan w4a8_plan(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch) {
-    W4A8Plan pl{false, {}, 0};
+    W4A8Plan pl{false, {}, 0, {0, 1, 0.0}};
     if (M <= 0 || N <= 0 || K <= 0) return pl;
     DirectArgs q{};
     if (group_int4 == 128 && M <= 512 && N <= 0x7fffffff && K <= (1 << 25) && w4a8_wave_plan(M, N, K, scratch, pl.shape)) {
@@ -93,6 +99,24 @@ W4A8Plan w4a8_plan(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scra
     if (!pl.wave) pl.bytes = two_pass;
     else if (!small) pl.bytes = std::max(slices, two_pass);
     else pl.bytes = M <= 16 ? slices : std::max(slices, llmk_gemm_workspace_bytes(M, N, K));
+    // (K from 1024 on: neither estimate was fitted to less)
+    if (M > 64 && K >= 1024 && group_int4 == 128 && M <= 0x7fffffff && N <= 0x7fffffff && K <= 0x7fffffff) {
+        q.M = (int)M; q.N = (int)N; q.K = (int)K; q.E = 1;
+        pl.duo = duo_plan<K_W4A8>(q, scratch);
+        if (pl.duo.mi) {
+            double other = 1.05 * pl.shape.cost;
+            if (!pl.wave) {
+                const TileChoice c = dma_tile_estimate<K_I8_BLOCK, false>(q);
+                const double tiles = (c.choice <= 2 ? 3.5 : 6.8) + (c.choice == 8 ? 1.03 : (c.choice == 2 ? 0.86 : 0.95)) * c.cost * (double)K / 4096.0;
+                other = 4.3 + (double)N * K * 0.23e-6 + 1.03 * std::min(tiles, duo_plan<K_I8_BLOCK>(q, INT64_MAX).cost);
+            }
+            if (1.08 * pl.duo.cost >= other) pl.duo.mi = 0;
+        }
+        if (pl.duo.mi) {
+            pl.wave = false;
+            if (pl.duo.z > 1) pl.bytes = std::max(pl.bytes, (int64_t)pl.duo.z * M * N * 4);
+        }
+    }
     return pl;
 }
 }  // namespace
@@ -106,6 +130,14 @@ extern "C" int llmk_gemm_w4a8_wave_shape(int64_t M, int64_t N, int64_t K, int gr
     return pl.wave && shape ? wave_shape(pl.shape, wv_depth(pl.shape.mt, pl.shape.nt, ((K >> 7) + pl.shape.z - 1) / pl.shape.z), shape) : 0;
 }
 
+extern "C" int llmk_gemm_w4a8_duo_shape(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch_bytes, int32_t* shape) {
+    const W4A8Plan pl = w4a8_plan(M, N, K, group_int4, scratch_bytes);
+    if (!pl.duo.mi || !shape) return 0;
+    shape[0] = 32 * pl.duo.mi;
+    shape[1] = pl.duo.z;
+    return 1;
+}
+
 extern "C" int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b_packed, const void* b_s, int s_dtype,
                               const int8_t* b_s4, const int8_t* b_z4, void* c, int c_dtype, int64_t M, int64_t N,
                               int64_t K, int group_int4, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -116,13 +148,16 @@ extern "C" int llmk_gemm_w4a8(const int8_t* a, const void* a_s, const int32_t* b
     if (!a || !a_s || !b_packed || !b_s || !b_s4 || !b_z4 || !c) LLMK_FAIL(LLMK_ERR_ARG, "gemm_w4a8: null pointer");
     const int64_t scratch = workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0;
     const W4A8Plan pl = w4a8_plan(M, N, K, group_int4, scratch);
-    if (pl.wave && !(((uintptr_t)a | (uintptr_t)b_packed) & 15)) {
+    if ((pl.wave || pl.duo.mi) && !(((uintptr_t)a | (uintptr_t)b_packed) & 15)) {
         if (s_dtype != LLMK_F32 && s_dtype != LLMK_F16 && s_dtype != LLMK_BF16) LLMK_FAIL(LLMK_ERR_DTYPE, "gemm_w4a8: s_dtype %d", s_dtype);
         if (c_dtype != LLMK_F32 && c_dtype != LLMK_F16 && c_dtype != LLMK_BF16) LLMK_FAIL(LLMK_ERR_DTYPE, "gemm_w4a8: c_dtype %d", c_dtype);
         DirectArgs p{};
         p.a = (const uint8_t*)a; p.b = (const uint8_t*)b_packed; p.c = c; p.a_s = a_s; p.b_s = b_s;
         p.w4_s4 = b_s4; p.w4_z4 = b_z4;
         p.c_dtype = c_dtype; p.s_dtype = s_dtype; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = 128;
+        if (pl.duo.mi)
+            return s_dtype == LLMK_F32 ? launch_duo_plan<K_W4A8>(p, pl.duo, workspace, (hipStream_t)stream, "gemm_w4a8(duo)")
+                                       : launch_duo_plan<K_W4A8, true>(p, pl.duo, workspace, (hipStream_t)stream, "gemm_w4a8(duo)");
         p.partial = (float*)workspace;
         return launch_w4a8_wave_plan(p, pl.shape, (hipStream_t)stream, "gemm_w4a8(wave)");
     }

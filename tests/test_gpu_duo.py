@@ -10,20 +10,18 @@ from llm_kernels_amd.fast_dequant import w4a16
 from llm_kernels_amd.quantization import fp8_kernel, int8_kernel
 from helpers import announce, assert_close_scaled, default_dtype
 
-# (M, N, K): tile rows, K slices
-FP8 = {(257, 6768, 128): (96, 1), (196, 8957, 256): (96, 1), (232, 8288, 384): (96, 1), (200, 8336, 640): (96, 1), (197, 8640, 768): (96, 1),
-       (210, 8311, 896): (96, 1), (289, 6864, 1024): (96, 1), (201, 8648, 1152): (96, 1), (198, 8312, 1280): (96, 1), (257, 6616, 1408): (96, 1),
-       (593, 224, 3072): (96, 4), (1450, 287, 4224): (96, 4), (301, 8280, 1536): (128, 1), (298, 8776, 1152): (128, 1), (290, 8435, 1280): (128, 1),
-       (290, 8224, 1408): (128, 1), (1351, 648, 6144): (128, 3)}
-INT8 = {(193, 8264, 896): (96, 1), (201, 8285, 1152): (96, 1), (257, 6824, 1408): (96, 1), (749, 1288, 6144): (96, 2), (582, 216, 3072): (96, 4),
-        (294, 8288, 4096): (128, 1), (307, 8287, 4224): (128, 1), (704, 1320, 6144): (128, 3)}
-PER_TOKEN = {(524, 3632, 1536): (96, 1), (519, 3607, 1152): (96, 1), (526, 248, 3072): (96, 4), (1011, 375, 4224): (96, 3), (289, 8424, 3072): (128, 1),
-             (291, 8344, 4224): (128, 1), (2042, 407, 6144): (128, 4), (450, 8256, 640): (160, 1), (451, 8888, 768): (160, 1), (452, 8391, 1152): (160, 1),
-             (590, 6536, 1408): (160, 1)}
-W4 = {(1081, 224, 128): (96, 1), (1465, 208, 256): (96, 1), (1054, 224, 384): (96, 1), (566, 216, 1152): (96, 3), (537, 240, 1280): (96, 3),
-      (659, 208, 2176): (96, 4), (850, 280, 4224): (96, 6), (1849, 1552, 384): (128, 1), (1080, 2704, 512): (128, 1), (865, 1104, 4224): (128, 4),
-      (1029, 3664, 128): (160, 1), (1538, 2456, 256): (160, 1), (1160, 3208, 384): (160, 1), (300, 14336, 4096): (160, 1), (148, 6672, 4224): (160, 4),
-      (1605, 2952, 128): (192, 1), (979, 4728, 256): (192, 1), (983, 4688, 384): (192, 1), (990, 4688, 512): (192, 1), (169, 6408, 6144): (192, 4)}
+FP8 = [(138, 11136, 128), (136, 11557, 256), (167, 11056, 384), (131, 10896, 640), (133, 11096, 768), (137, 11553, 896), (162, 11128, 1024), (131, 11616, 1152),
+       (142, 11264, 1280), (140, 11184, 1408), (751, 216, 3072), (572, 229, 4224), (1777, 224, 4224), (194, 11816, 1024), (209, 11291, 1152), (198, 11448, 1280),
+       (195, 11104, 1408), (2028, 392, 6144)]
+INT8 = [(133, 11136, 640), (138, 11373, 768), (141, 11744, 896), (135, 11040, 1152), (137, 11968, 1408), (2044, 456, 6144), (667, 216, 3072), (937, 381, 4224),
+        (197, 11248, 3072), (198, 11051, 4224)]
+PER_TOKEN = [(524, 3632, 1536), (519, 3607, 1152), (526, 248, 3072), (1011, 375, 4224), (289, 8424, 3072), (291, 8344, 4224), (2042, 407, 6144), (450, 8256, 640),
+             (451, 8888, 768), (452, 8391, 1152), (590, 6536, 1408)]
+W4A8 = [(538, 248, 1024), (543, 328, 1152), (581, 232, 1280), (530, 232, 1408), (545, 224, 1536), (676, 200, 1664), (541, 256, 4224), (576, 976, 4224), (194, 11280, 1024),
+        (198, 11008, 1152), (221, 10912, 1280), (195, 11544, 1408), (203, 7088, 6144), (1375, 272, 6144), (1636, 552, 4224), (79, 28672, 4096)]
+W4 = [(1081, 224, 128), (1465, 208, 256), (1054, 224, 384), (566, 216, 1152), (537, 240, 1280), (659, 208, 2176), (850, 280, 4224), (1849, 1552, 384), (1080, 2704, 512),
+      (865, 1104, 4224), (1029, 3664, 128), (1538, 2456, 256), (1160, 3208, 384), (300, 14336, 4096), (148, 6672, 4224), (1605, 2952, 128), (979, 4728, 256),
+      (983, 4688, 384), (990, 4688, 512), (169, 6408, 6144)]
 
 
 def shape(entry, *args):
@@ -35,20 +33,33 @@ def shape8(kind, per_token, M, N, K):
     return shape("llmk_gemm_8bit_duo_shape", kind, per_token, M, N, K, _lib.load().llmk_gemm_workspace_bytes(M, N, K))
 
 
+def shape_w4a8(M, N, K):
+    return shape("llmk_gemm_w4a8_duo_shape", M, N, K, 128, _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128))
+
+
+PLANS = ((FP8, 1, {96, 128}, lambda *c: shape8(_lib.KIND_FP8, 0, *c)), (INT8, 1, {96, 128}, lambda *c: shape8(_lib.KIND_I8, 0, *c)),
+         (PER_TOKEN, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_I8, 1, *c)), (W4A8, 1, {96, 128}, shape_w4a8),
+         (W4, 2, {96, 128, 160, 192}, lambda *c: shape("llmk_gemm_w4a16_duo_shape", _lib.F16, *c, 128, 1 << 50)))
+
+
 def test_the_cases_reach_every_tile():
-    for cases, kind, per_token, heights in ((FP8, _lib.KIND_FP8, 0, {96, 128}), (INT8, _lib.KIND_I8, 0, {96, 128}), (PER_TOKEN, _lib.KIND_I8, 1, {96, 128, 160})):
-        assert {rows for rows, _ in cases.values()} == heights
-        for call, want in cases.items():
-            assert shape8(kind, per_token, *call) == want, (kind, per_token, call)
-    assert {rows for rows, _ in W4.values()} == {96, 128, 160, 192}
-    for (M, N, K), want in W4.items():
-        assert shape("llmk_gemm_w4a16_duo_shape", _lib.F16, M, N, K, 128, 1 << 50) == want, (M, N, K)
+    """Every height, with one and with several slices, and every remainder of a slice's sub-blocks by the loop's four."""
+    for cases, size, heights, plan in PLANS:
+        got = {c: plan(*c) for c in cases}
+        assert None not in got.values(), got
+        assert {rows for rows, _ in got.values()} == heights and {z > 1 for _, z in got.values()} == {False, True}, got
+        assert {-(-c[2] * size // 128 // z) % 4 for c, (_, z) in got.items()} == {0, 1, 2, 3}, got
 
 
 def test_scratch_of_its_slices_is_reported_and_small():
-    """What is reported holds the planes of the slices, and never more than the array that serves calls without scratch of their own."""
-    for (M, N, K), (_, z) in {**FP8, **INT8, **PER_TOKEN}.items():
-        assert 4 * z * M * N * (z > 1) <= _lib.load().llmk_gemm_workspace_bytes(M, N, K) <= 32 << 20, (M, N, K)
+    """What is reported holds the planes of the slices, and for the 8-bit products never more than the array that serves calls without scratch."""
+    for cases, _, _, plan in PLANS[:3]:
+        for M, N, K in cases:
+            z = plan(M, N, K)[1]
+            assert 4 * z * M * N * (z > 1) <= _lib.load().llmk_gemm_workspace_bytes(M, N, K) <= 32 << 20, (M, N, K)
+    for M, N, K in W4A8:
+        z = shape_w4a8(M, N, K)[1]
+        assert 4 * z * M * N * (z > 1) <= _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128)
 
 
 def _ints(gen, dev, lo, hi, *size):
@@ -98,6 +109,41 @@ def test_per_token_exact(dev, M, N, K):
         c, acc = int8_kernel.int8_gemm_per_token(a, a_s, b, b_s, return_int32=True)
     assert torch.equal(acc.double(), ref)
     assert torch.equal(c, acc.float() * a_s[:, None] * b_s[None, :])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,scales", [(*c, (torch.float16, torch.bfloat16, torch.float32)[i % 3]) for i, c in enumerate(W4A8)])
+def test_two_level_weights_exact(dev, M, N, K, scales):
+    """Weights int8(int8(q - z4) * s4) of any scale and zero point, wrap included, under powers of two: exact in fp32.  Tables at any offset, and words
+    that are not 16-byte aligned, which go another way with the reported scratch."""
+    announce("duo w4a8", M, N, K, scales)
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    kb = K // 128
+    a, q = _ints(gen, dev, -3, 3, M, K), _ints(gen, dev, 0, 15, N, K)
+    near = _ints(gen, dev, 0, 7, N, kb) > 0                  # mostly small weights, so that the sums stay below 2^24
+    s4, z4 = torch.where(near, _ints(gen, dev, -1, 2, N, kb), _ints(gen, dev, -128, 127, N, kb)), torch.where(near, _ints(gen, dev, 0, 15, N, kb), _ints(gen, dev, -128, 127, N, kb))
+    wide = lambda t: t.repeat_interleave(128, 1)
+    b = ((q - wide(z4)).to(torch.int8).int() * wide(s4).int()).to(torch.int8)
+    a_s, b_s = (2.0 ** _ints(gen, dev, 0, 1, M, kb)).to(scales), (2.0 ** _ints(gen, dev, 0, 1, -(-N // 128), kb)).to(scales)
+    ref = (a.double() * wide(a_s.double())) @ (b.double() * wide(b_s.double()).repeat_interleave(128, 0)[:N]).t()
+    assert ref.abs().max() < 1 << 24
+    packed = torch.zeros(N // 8, K, dtype=torch.int64, device=dev)
+    for i in range(8):
+        packed |= q[i::8].long() << (4 * i)
+    packed = torch.where(packed >= 1 << 31, packed - (1 << 32), packed).int()
+    a8, bytes4 = a.to(torch.int8), torch.empty(2, N * kb + 1, dtype=torch.int8, device=dev)
+    bytes4[0, 1:], bytes4[1, 1:] = s4.to(torch.int8).flatten(), z4.to(torch.int8).flatten()
+    scratch = _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128)
+    ws = torch.empty(max(scratch, 16), dtype=torch.uint8, device=dev)
+    odd = torch.empty(N // 8 * K + 1, dtype=torch.int32, device=dev)[1:].copy_(packed.flatten())
+    for words in (packed, odd):
+        for room in (scratch, 0):
+            if room < N * K and (words is odd or not shape("llmk_gemm_w4a8_duo_shape", M, N, K, 128, room)):
+                continue                                     # (the expanded copy of the weights needs its scratch)
+            out = torch.full((M, N), float("nan"), device=dev)
+            _lib.call("llmk_gemm_w4a8", _lib.ptr(a8), _lib.ptr(a_s), _lib.ptr(words), _lib.ptr(b_s), _lib.dt(scales), _lib.ptr(bytes4[0, 1:]), _lib.ptr(bytes4[1, 1:]),
+                      _lib.ptr(out), _lib.F32, M, N, K, 128, _lib.ptr(ws) if room else None, room, _lib.stream(a8))
+            assert torch.equal(out.double(), ref), (room, words is odd)
 
 
 @pytest.mark.gpu
