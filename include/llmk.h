@@ -217,10 +217,10 @@ int llmk_gemm_8bit_wave_shape(int kind, int per_token, int64_t M, int64_t N, int
 int llmk_gemm_w4a8_wave_shape(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch_bytes, int32_t* shape);
 int llmk_gemm_w4a16_wave_shape(int marlin, int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes,
                                int32_t* shape);
-/* The same for the tile kernel whose two wave groups take turns (from 65 rows on): shape = {rows of a tile, K slices}.  w4a16: [N, K/8]. */
+/* The same for the tile kernel whose two wave groups take turns (from 65 rows on): shape = {rows of a tile, K slices}.  w4a16: marlin 1 or [N, K/8] 0. */
 int llmk_gemm_8bit_duo_shape(int kind, int per_token, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes, int32_t* shape);
 int llmk_gemm_w4a8_duo_shape(int64_t M, int64_t N, int64_t K, int group_int4, int64_t scratch_bytes, int32_t* shape);
-int llmk_gemm_w4a16_duo_shape(int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes, int32_t* shape);
+int llmk_gemm_w4a16_duo_shape(int marlin, int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes, int32_t* shape);
 
 /* ------------------------------------------------------------------ converters and the one-tile MFMA GEMM
  * ref: fast_dequant/fast_dtype_convert/fast_uint4_to_fp16.cu:21-109,112-127 (out[i] = nibble_i - 8, nibble i

@@ -57,7 +57,7 @@ SIGNATURES = {
     "llmk_gemm_w4a16_wave_shape": [_i, _i, _l, _l, _l, _i, _l, _p],
     "llmk_gemm_8bit_duo_shape": [_i, _i, _l, _l, _l, _l, _p],
     "llmk_gemm_w4a8_duo_shape": [_l, _l, _l, _i, _l, _p],
-    "llmk_gemm_w4a16_duo_shape": [_i, _l, _l, _l, _i, _l, _p],
+    "llmk_gemm_w4a16_duo_shape": [_i, _i, _l, _l, _l, _i, _l, _p],
     "llmk_convert_u4_to_f16": [_p, _p, _l, _p],
     "llmk_convert_u8_to_f16": [_p, _p, _l, _p],
     "llmk_convert_u8_to_bf16": [_p, _p, _l, _p],

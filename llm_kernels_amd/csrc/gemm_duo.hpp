@@ -23,7 +23,8 @@ constexpr int du_a(int mi) { return 32 * mi * 128; }
 constexpr int du_b() { return DU_BN * 128; }
 constexpr int du_windows(int mi) { return 2 * 32 * mi * 4 * 4; }             // two windows of activation scales, four sub-blocks each
 constexpr bool du_scaled(int kind) { return kind == K_FP8_BLOCK || kind == K_I8_BLOCK || kind == K_W4A8; }
-constexpr bool du_expands(int kind) { return is_w4nk(kind) || kind == K_W4A8; }
+constexpr bool du_w4a16(int kind) { return is_w4nk(kind) || kind == K_W4MARLIN; }
+constexpr bool du_expands(int kind) { return du_w4a16(kind) || kind == K_W4A8; }
 constexpr int du_lds(int kind, int mi) {                                      // K_W4A8: + du_table bytes
     return DU_SLOTS * du_a(mi) + (du_expands(kind) ? 2 : DU_SLOTS) * du_b() + (du_scaled(kind) ? du_windows(mi) + D_MAX_KT * 4 : 0);
 }
@@ -31,8 +32,9 @@ constexpr int du_table(int sub_blocks) { return sub_blocks * DU_BN * 4; }     //
 
 template <int KIND, int MI, bool AS16 = false>
 __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
-    constexpr bool SCALED = du_scaled(KIND), ROWCOL = (KIND == K_I8_ROWCOL), W4NK = is_w4nk(KIND), W4A8 = (KIND == K_W4A8), EXPANDS = W4NK || W4A8;
-    static_assert(SCALED || ROWCOL || W4NK, "8-bit operands, or 4-bit weights");
+    constexpr bool SCALED = du_scaled(KIND), ROWCOL = (KIND == K_I8_ROWCOL), W4A16 = du_w4a16(KIND), MARLIN = (KIND == K_W4MARLIN), W4A8 = (KIND == K_W4A8),
+                   EXPANDS = W4A16 || W4A8;
+    static_assert(SCALED || ROWCOL || W4A16, "8-bit operands, or 4-bit weights");
     constexpr int MATH = W4A8 ? K_I8_BLOCK : KIND;           // the products once the weights are expanded
     constexpr int ESZ = is_half(KIND) ? 2 : 1, BM = 32 * MI, WR = 16 * MI;
     constexpr int A_SLOT = du_a(MI), B_SLOT = du_b(), B0 = DU_SLOTS * A_SLOT, NB = EXPANDS ? 2 : DU_SLOTS, SW = B0 + NB * B_SLOT;
@@ -75,35 +77,63 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             boff[i] = (uint32_t)min(n0 + column(R), N - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((R >> 1) & 7)) * 16u;
         }
     }
-    // 4-bit weights: in phase f every thread expands 16 weights of sub-block f + 1, quarter t & 3 of weight row t >> 2, from a packed double
-    // word and a group scale requested four phases ago (set f & 3)
+    // 4-bit weights: in phase f every thread expands 16 weights of sub-block f + 1 from a packed double word and its scales, requested four
+    // phases ago (set f & 3).  Row-packed: quarter t & 3 of weight row t >> 2.  Marlin words: half h of the unit of strip sl, chunk ch, columns
+    // c of eight, k pair q: words 2 h + jj hold columns 16 (2 h + jj) + 8 b + c of the chunk, elements 2 q, 2 q + 1 of the strip in the low
+    // nibbles of byte b of both half words and 2 q + 8, 2 q + 9 in the high ones.  A wave holds all q, c & 3 and sl of one (h, c >> 2, ch):
+    // its lanes then write 64 different banks (with a wave on one strip four lanes met in a bank).
     uint32_t w4_off = 0, w4_soff = 0, w4_dst = 0, w4_sw = 0;
     int w4_shift = 0;
-    if constexpr (W4NK) {
+    int64_t w4_step = 32, w4_sstep = 2;                      // bytes per sub-block, and per group of scales
+    if constexpr (W4A16) w4_shift = __builtin_ctz((unsigned)(p.group >> 6));
+    if constexpr (is_w4nk(KIND)) {
         const int R = tid >> 2, q = tid & 3;
         const uint32_t n = (uint32_t)min(n0 + column(R), N - 1);
         w4_off = n * (uint32_t)(p.K >> 1) + (uint32_t)q * 8u;
         w4_soff = n * (uint32_t)(p.K / p.group) * 2u;
         w4_dst = (uint32_t)(R * 128);
         w4_sw = (uint32_t)(((2 * q) ^ ((R >> 1) & 7)) * 16);                  // chunk 2 q; chunk 2 q + 1 is at ^ 16
-        w4_shift = __builtin_ctz((unsigned)(p.group >> 6));
     }
+    if constexpr (MARLIN) {
+        const int q = lane & 3, c3 = (lane >> 2) & 3, sl = lane >> 4, h = wave & 1, c4 = (wave >> 1) & 1, ch = wave >> 2, c = 4 * c4 + c3;
+        const int chunks = N >> 6, chunk = min((n0 >> 6) + ch, chunks - 1);
+        w4_off = (uint32_t)((sl * chunks + chunk) * 32 + 4 * c + q) * 16u + (uint32_t)h * 8u;
+        w4_soff = (uint32_t)(64 * chunk + 8 * c + 4 * h) * 2u;
+        w4_step = (int64_t)chunks * 2048;
+        w4_sstep = (int64_t)N * 2;
+        w4_dst = (uint32_t)((64 * ch + 32 * h + 16 * c4 + c3) * 128 + 4 * q);  // LDS row of jj = b = 0; 4 (2 jj + b) rows on for the others
+        w4_sw = (uint32_t)(((2 * sl) ^ (c3 >> 1)) * 16);                       // its chunk; ^ 16 for the high nibbles, ^ 16 (4 jj + 2 b)
+    }
+    typedef typename std::conditional<MARLIN, uint64_t, unsigned>::type W4Scale;
     uint64_t w4_words[4] = {0, 0, 0, 0};
-    unsigned w4_scale[4] = {0, 0, 0, 0};
+    W4Scale w4_scale[4] = {0, 0, 0, 0};
     auto request_words = [&](int set, int u) __attribute__((always_inline)) {
-        if constexpr (W4NK) {
+        if constexpr (W4A16) {
             const int kb = kt0 + min(u, KT - 1);
-            w4_words[set] = asm_load_b64(w4_off, (const uint8_t*)p.b + (int64_t)kb * 32);
-            w4_scale[set] = asm_load_u16(w4_soff, (const uint8_t*)p.b_s + (int64_t)(kb >> w4_shift) * 2);
+            const uint8_t* const sc = (const uint8_t*)p.b_s + (int64_t)(kb >> w4_shift) * w4_sstep;
+            w4_words[set] = asm_load_b64(w4_off, (const uint8_t*)p.b + (int64_t)kb * w4_step);
+            if constexpr (MARLIN) w4_scale[set] = asm_load_b64(w4_soff, sc);
+            else w4_scale[set] = asm_load_u16(w4_soff, sc);
         }
     };
     // every use of the words comes behind this (the wait is the caller's business)
     auto words_landed = [&](int set) __attribute__((always_inline)) {
-        if constexpr (W4NK) asm volatile("" : "+v"(w4_words[set]), "+v"(w4_scale[set]) : : "memory");
+        if constexpr (W4A16) asm volatile("" : "+v"(w4_words[set]), "+v"(w4_scale[set]) : : "memory");
     };
     auto expand_word = [&](int set, int u, int c) __attribute__((always_inline)) {
-        if constexpr (W4NK)
-            *(v4i*)(lds + B0 + (u & 1) * B_SLOT + w4_dst + (w4_sw ^ (uint32_t)(c * 16))) = w4_word_x8<KIND>((unsigned)(w4_words[set] >> (32 * c)), w4_scale[set]);
+        uint8_t* const dst = lds + B0 + (u & 1) * B_SLOT + w4_dst;
+        if constexpr (is_w4nk(KIND)) *(v4i*)(dst + (w4_sw ^ (uint32_t)(c * 16))) = w4_word_x8<KIND>((unsigned)(w4_words[set] >> (32 * c)), w4_scale[set]);
+        if constexpr (MARLIN) {
+            const v2h k1032 = {(_Float16)1032.f, (_Float16)1032.f}, k16 = {(_Float16)0.0625f, (_Float16)0.0625f}, k72 = {(_Float16)72.f, (_Float16)72.f};
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const unsigned w = (unsigned)(w4_words[set] >> (32 * c)) >> (8 * b), s16 = (unsigned)(w4_scale[set] >> (16 * (2 * c + b))) & 0xffffu;
+                const v2h sc = w4_as_h2(s16 | (s16 << 16));
+                const uint32_t at = w4_sw ^ (uint32_t)(16 * (4 * c + 2 * b));
+                *(v2h*)(dst + 512 * (2 * c + b) + at) = (w4_as_h2((w & 0x000f000fu) | 0x64006400u) - k1032) * sc;
+                *(v2h*)(dst + 512 * (2 * c + b) + (at ^ 16u)) = (w4_as_h2((w & 0x00f000f0u) | 0x64006400u) * k16 - k72) * sc;
+            }
+        }
     };
     // int8 activations: its products keep the multiplying group's vector ALU busy, so the fetching one expands.  In its turn of phase u thread t
     // of the group takes eight words of sub-block u + 1, packed row (t >> 4) & 15, elements 8 (t & 15) .. + 7, requested four phases ago (set
@@ -240,9 +270,9 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     // 4-bit weights: in the shadow of its matrix instructions the multiplying group expands its half of sub-block f + 1 of phase f (the slot's
     // readers finished in the phase before), and requests the words of sub-block f + 5
     auto multiply = [&](auto expand_c, int f) __attribute__((always_inline)) {
-        constexpr bool EXPAND = W4NK && decltype(expand_c)::value;
+        constexpr bool EXPAND = W4A16 && decltype(expand_c)::value;
         if constexpr (EXPAND) words_landed(f & 3);
-        if constexpr (W4NK) __builtin_amdgcn_s_setprio(1);
+        if constexpr (W4A16) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
             if constexpr (EXPAND) {
@@ -272,7 +302,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[MI - 1][j] += raw_f32<MATH>(t[j]) * sa[MI - 1];
         }
-        if constexpr (W4NK) __builtin_amdgcn_s_setprio(0);
+        if constexpr (W4A16) __builtin_amdgcn_s_setprio(0);
     };
     auto meet = [&](auto left_c) {                           // this wave's LDS accesses, and its loads but the left_c youngest, are done
         __builtin_amdgcn_sched_barrier(0);
@@ -306,7 +336,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             __builtin_amdgcn_sched_barrier(0);
         }
         fetch(u);
-        if constexpr (W4NK) {
+        if constexpr (W4A16) {
             __builtin_amdgcn_sched_barrier(0);
             words_landed(u & 3);
             expand_word(u & 3, u + 1, 0);
@@ -320,7 +350,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     };
     // The same where little or nothing is left to request: every phase waits for all of it, and the words move up a set a phase.
     auto last_words = [&](int f) __attribute__((always_inline)) {
-        if constexpr (W4NK) {
+        if constexpr (W4A16) {
             if (f + 1 < KT) {
                 expand_word(0, f + 1, 0);
                 expand_word(0, f + 1, 1);
@@ -353,7 +383,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         words8_landed(1);
     };
     auto all_landed = [&]() __attribute__((always_inline)) {
-        if constexpr (W4NK) {
+        if constexpr (W4A16) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
             for (int i = 0; i < 4; ++i) words_landed(i);
@@ -527,7 +557,7 @@ int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
 // wait for their scales spill.
 template <int KIND>
 constexpr bool duo_built(int mi) {
-    return mi >= 3 && mi <= (is_w4nk(KIND) ? 6 : (KIND == K_I8_ROWCOL ? 5 : 4));
+    return mi >= 3 && mi <= (is_w4nk(KIND) ? 6 : (KIND == K_I8_ROWCOL || KIND == K_W4MARLIN ? 5 : 4));
 }
 // Estimated microseconds: base + rounds of 256 workgroups x (round + sub-blocks x step[mi - 3]) + out x MB of the output, and for K slices
 // split + plane x MB of the fp32 planes.  A fit of 4 to 7 % rms to 300 random shapes a kind of M 64 to 4096, N 1024 to 28672, K 1024 to
@@ -539,6 +569,7 @@ template <int KIND>
 constexpr DuoModel duo_model() {
     if (KIND == K_FP8_BLOCK) return {2.0f, 1.4f, {0.396f, 0.452f, 0.f, 0.f}, 3.4f, 0.50f, 0.48f};
     if (KIND == K_I8_BLOCK) return {2.4f, 1.4f, {0.417f, 0.502f, 0.f, 0.f}, 2.9f, 0.58f, 0.57f};
+    if (KIND == K_W4MARLIN) return {3.03f, 2.53f, {0.460f, 0.519f, 0.589f, 0.f}, 2.9f, 0.45f, 0.31f};
     if (KIND == K_W4A8) return {1.76f, 2.62f, {0.614f, 0.683f, 0.f, 0.f}, 3.0f, 0.55f, 0.37f};
     if (KIND == K_I8_ROWCOL) return {2.79f, 1.59f, {0.355f, 0.406f, 0.470f, 0.f}, 2.9f, 0.47f, 0.57f};
     return {2.29f, 1.78f, {0.421f, 0.487f, 0.561f, 0.639f}, 3.7f, 0.46f, 0.43f};
@@ -555,7 +586,7 @@ DuoPlan duo_plan(const DirectArgs& p, int64_t scratch) {
     constexpr int ESZ = is_half(KIND) ? 2 : 1;
     constexpr DuoModel m = duo_model<KIND>();
     DuoPlan best{0, 1, 1e30};
-    if (p.M <= 64 || !dma_eligible(p, ESZ) || (is_w4nk(KIND) && (p.group < 64 || (p.group & (p.group - 1))))) return best;
+    if (p.M <= 64 || !dma_eligible(p, ESZ) || (du_w4a16(KIND) && (p.group < 64 || (p.group & (p.group - 1))))) return best;
     const int KT = (p.K * ESZ) >> 7;
     const int64_t gx = (p.N + DU_BN - 1) / DU_BN, planes = std::min(scratch, DU_MAX_PLANES);
     const double out = (double)p.M * p.N * 1e-6;

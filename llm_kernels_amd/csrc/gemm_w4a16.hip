@@ -1093,6 +1093,16 @@ MarlinPlan marlin_plan(int64_t M, int64_t N, int64_t K) {
     return pl;
 }
 
+// What the 128-column tile kernels that expand Marlin words take for 65 to 512 rows, in us (see below).
+double marlin_tiles_estimate(int64_t M, int64_t N, int64_t K, int group) {
+    llmk::DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
+    const double k = (double)K / 4096.0;
+    const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128), z = std::min<int64_t>(llmk::splitk_factor_half(M, N, K), std::max<int64_t>(1, LLMK_CUS / tiles));
+    if (z > 1) return 7.7 + 42.5 * k / z;
+    const llmk::TileChoice c = llmk::dma_tile_estimate<llmk::K_W4MARLIN, false>(p);
+    return c.choice == 1 ? 4.0 + 2.5 * c.cost * k : (c.choice == 2 ? 5.3 + 1.75 * c.cost * k : 5.0 + 1.58 * c.cost * k);
+}
 // The wave kernel for a call on Marlin words, or z = 0: always up to 64 rows, up to 512 where it is estimated 8 % below the
 // 128-column tile kernels that expand the words in LDS (a fit of 3 to 7 % rms to 70 shapes: the scatter of the Marlin layout is most
 // of their time).  Choosing so was 1 % behind the faster one of each shape and 1.47 times faster than without the wave kernel over
@@ -1102,19 +1112,24 @@ MarlinPlan marlin_plan(int64_t M, int64_t N, int64_t K) {
 llmk::WavePlan marlin_wave(int64_t M, int64_t N, int64_t K, int group, int64_t scratch) {
     llmk::WavePlan w{0, 0, 0, 0, 0.0};
     if (M > 512 || !llmk::w4a16_wave_plan<llmk::K_W4MARLIN, true>(M, N, K, group, scratch, w)) { w.z = 0; return w; }
-    if (M > 64) {
-        llmk::DirectArgs p{};
-        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
-        const double k = (double)K / 4096.0;
-        const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128), z = std::min<int64_t>(llmk::splitk_factor_half(M, N, K), std::max<int64_t>(1, LLMK_CUS / tiles));
-        double other = 7.7 + 42.5 * k / z;
-        if (z == 1) {
-            const llmk::TileChoice c = llmk::dma_tile_estimate<llmk::K_W4MARLIN, false>(p);
-            other = c.choice == 1 ? 4.0 + 2.5 * c.cost * k : (c.choice == 2 ? 5.3 + 1.75 * c.cost * k : 5.0 + 1.58 * c.cost * k);
-        }
-        if (1.08 * w.cost >= other) w.z = 0;
-    }
+    if (M > 64 && 1.08 * w.cost >= marlin_tiles_estimate(M, N, K, group)) w.z = 0;
     return w;
+}
+// The kernel of two wave groups (gemm_duo.hpp) for a call on Marlin words, or mi = 0: from 65 rows on, 8 % below the estimate of the wave kernel, the
+// tiles above, or beyond 512 rows the 16-bit copy of W and the fp16 tiles (a fit of 10 % rms to 146 shapes).  Its threads scatter the words
+// without bank conflicts.  Over 300 random shapes of 64 to 4096 rows 1.06 times as fast as without, 0.5 % behind the faster one of each
+// shape, at worst 9 % slower.  Others | this one, us: 1024 x 4096 x 4096 52.7 | 43.7, 432 x 6144 x 4096 42.0 | 36.6, 1072 x 3200 x 6400 76 | 61,
+// 832 x 2560 x 2560 31.5 | 25.1, but 2384 x 6144 x 4096 106 | 134 and 416 x 1600 x 1664 9.0 | 16.7.
+llmk::DuoPlan marlin_duo(int64_t M, int64_t N, int64_t K, int group, const llmk::WavePlan& wave, int64_t scratch) {
+    if (M <= 64 || K % 64) return {0, 1, 0.0};
+    llmk::DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
+    llmk::DuoPlan d = llmk::duo_plan<llmk::K_W4MARLIN>(p, scratch);
+    if (!d.mi) return d;
+    double other = wave.z > 0 ? 1.05 * wave.cost : marlin_tiles_estimate(M, N, K, group);
+    if (M > 512) other = 6.1 + 0.40e-6 * (double)N * K + 1.38 * llmk::dma_tile_estimate<llmk::K_F16, false>(p).cost * (double)K / 4096.0;
+    if (1.08 * d.cost >= other) d.mi = 0;
+    return d;
 }
 
 }  // namespace
@@ -1123,7 +1138,8 @@ extern "C" int64_t llmk_gemm_w4a16_marlin_workspace_bytes(int64_t M, int64_t N, 
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
     // the group size is not known here: what the wave kernel's slices take with groups of 128, and what the others take
     const llmk::WavePlan wave = marlin_wave(M, N, K, 128, INT64_MAX);
-    const int64_t slices = wave.z > 1 ? wave.z * M * N * 4 : 0;
+    const llmk::DuoPlan duo = marlin_duo(M, N, K, 128, wave, INT64_MAX);
+    const int64_t slices = std::max(wave.z > 1 ? wave.z * M * N * 4 : 0, duo.mi && duo.z > 1 ? duo.z * M * N * 4 : 0);
     if (M > 64) {                                        // dequantised fp16 copy of W for the tiled GEMM (+ split-K partials)
         if (K % 64) return 0;
         const int z = llmk::splitk_factor_half(M, N, K);
@@ -1142,21 +1158,27 @@ extern "C" int llmk_gemm_w4a16_wave_shape(int marlin, int ac_dtype, int64_t M, i
     if (groupsize < 8 || K % groupsize) return 0;
     if (marlin) {
         const llmk::WavePlan w = marlin_wave(M, N, K, groupsize, scratch_bytes);
-        return w.z > 0 ? llmk::wave_shape(w, 1, shape) : 0;
+        return w.z > 0 && !marlin_duo(M, N, K, groupsize, w, scratch_bytes).mi ? llmk::wave_shape(w, 1, shape) : 0;
     }
     const bool bf = ac_dtype == LLMK_BF16;
     const NkPlan pl = nk_plan(M, N, K, groupsize, bf, scratch_bytes, true);
     return pl.route == NkPlan::WAVE ? llmk::wave_shape(pl.wave, nk_rounded_weights(M, N, K, groupsize, bf), shape) : 0;
 }
 
-extern "C" int llmk_gemm_w4a16_duo_shape(int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes, int32_t* shape) {
-    if (!shape || M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
+extern "C" int llmk_gemm_w4a16_duo_shape(int marlin, int ac_dtype, int64_t M, int64_t N, int64_t K, int groupsize, int64_t scratch_bytes, int32_t* shape) {
+    if (!shape || M <= 0 || N <= 0 || K <= 0 || K % 64 || M > 0x7fffffff / 2 || N > 0x7fffffff / 2 || K > 0x7fffffff / 2) return 0;
     if (groupsize == -1) groupsize = (int)K;
-    if (groupsize < 8 || groupsize % 8 || K % groupsize) return 0;
-    const NkPlan pl = nk_plan(M, N, K, groupsize, ac_dtype == LLMK_BF16, scratch_bytes, true);
-    if (pl.route != NkPlan::DUO) return 0;
-    shape[0] = 32 * pl.duo.mi;
-    shape[1] = pl.duo.z;
+    if (groupsize < 8 || groupsize % 8 || K % groupsize || (!marlin && K % 128)) return 0;
+    llmk::DuoPlan d{0, 1, 0.0};
+    if (marlin) {
+        d = marlin_duo(M, N, K, groupsize, marlin_wave(M, N, K, groupsize, scratch_bytes), scratch_bytes);
+    } else {
+        const NkPlan pl = nk_plan(M, N, K, groupsize, ac_dtype == LLMK_BF16, scratch_bytes, true);
+        if (pl.route == NkPlan::DUO) d = pl.duo;
+    }
+    if (!d.mi) return 0;
+    shape[0] = 32 * d.mi;
+    shape[1] = d.z;
     return 1;
 }
 
@@ -1178,6 +1200,13 @@ extern "C" int llmk_gemm_w4a16_marlin(const void* a, const int32_t* b, void* c, 
 
     hipStream_t st = (hipStream_t)stream;
     const llmk::WavePlan wave = marlin_wave(M, N, K, groupsize, usable_scratch(workspace, workspace_bytes));
+    const llmk::DuoPlan duo = marlin_duo(M, N, K, groupsize, wave, usable_scratch(workspace, workspace_bytes));
+    if (duo.mi) {
+        llmk::DirectArgs p{};
+        p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.b_s = s; p.c = c; p.c_dtype = LLMK_F16;
+        p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = groupsize;
+        return llmk::launch_duo_plan<llmk::K_W4MARLIN>(p, duo, workspace, st, "gemm_w4a16_marlin(duo)");
+    }
     if (wave.z > 0) {
         llmk::DirectArgs p{};
         p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.b_s = s; p.c = c; p.c_dtype = LLMK_F16;

@@ -7,6 +7,8 @@ import torch
 
 from llm_kernels_amd import _lib
 from llm_kernels_amd.fast_dequant import w4a16
+from llm_kernels_amd.fast_dequant.simple_marlin.marlin import mul
+from llm_kernels_amd.fast_dequant.simple_marlin.utils import QuantUtils
 from llm_kernels_amd.quantization import fp8_kernel, int8_kernel
 from helpers import announce, assert_close_scaled, default_dtype
 
@@ -19,6 +21,8 @@ PER_TOKEN = [(524, 3632, 1536), (519, 3607, 1152), (526, 248, 3072), (1011, 375,
              (451, 8888, 768), (452, 8391, 1152), (590, 6536, 1408)]
 W4A8 = [(538, 248, 1024), (543, 328, 1152), (581, 232, 1280), (530, 232, 1408), (545, 224, 1536), (676, 200, 1664), (541, 256, 4224), (576, 976, 4224), (194, 11280, 1024),
         (198, 11008, 1152), (221, 10912, 1280), (195, 11544, 1408), (203, 7088, 6144), (1375, 272, 6144), (1636, 552, 4224), (79, 28672, 4096)]
+MARLIN = [(208, 8576, 768), (208, 8320, 640), (560, 2304, 4096), (576, 192, 1536), (528, 192, 1664), (544, 192, 2176), (800, 320, 4224), (528, 5440, 1024),
+          (528, 5632, 896), (208, 6784, 4224), (1168, 576, 4224), (1424, 320, 4224), (448, 8832, 512), (400, 8576, 640), (160, 7424, 4224)]
 W4 = [(1081, 224, 128), (1465, 208, 256), (1054, 224, 384), (566, 216, 1152), (537, 240, 1280), (659, 208, 2176), (850, 280, 4224), (1849, 1552, 384), (1080, 2704, 512),
       (865, 1104, 4224), (1029, 3664, 128), (1538, 2456, 256), (1160, 3208, 384), (300, 14336, 4096), (148, 6672, 4224), (1605, 2952, 128), (979, 4728, 256),
       (983, 4688, 384), (990, 4688, 512), (169, 6408, 6144)]
@@ -39,7 +43,8 @@ def shape_w4a8(M, N, K):
 
 PLANS = ((FP8, 1, {96, 128}, lambda *c: shape8(_lib.KIND_FP8, 0, *c)), (INT8, 1, {96, 128}, lambda *c: shape8(_lib.KIND_I8, 0, *c)),
          (PER_TOKEN, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_I8, 1, *c)), (W4A8, 1, {96, 128}, shape_w4a8),
-         (W4, 2, {96, 128, 160, 192}, lambda *c: shape("llmk_gemm_w4a16_duo_shape", _lib.F16, *c, 128, 1 << 50)))
+         (MARLIN, 2, {96, 128, 160}, lambda *c: shape("llmk_gemm_w4a16_duo_shape", 1, _lib.F16, *c, 128, _lib.load().llmk_gemm_w4a16_marlin_workspace_bytes(*c))),
+         (W4, 2, {96, 128, 160, 192}, lambda *c: shape("llmk_gemm_w4a16_duo_shape", 0, _lib.F16, *c, 128, 1 << 50)))
 
 
 def test_the_cases_reach_every_tile():
@@ -163,3 +168,25 @@ def test_row_packed_weights(dev, M, N, K, dtype):
     x = torch.randn(M, K, device=dev, generator=gen, dtype=torch.float32).to(dtype)
     ref = x.double() @ weights.double().t()
     assert_close_scaled(w4a16.w4a16_gemm(x, packed, scales, 128), ref, rtol=2 ** -8 if dtype == torch.bfloat16 else 2 ** -11, atol=2e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,group", [(*c, (128, 64, 256)[i % 3] if c[2] % 256 == 0 else (128, 64)[i % 2]) for i, c in enumerate(MARLIN)])
+def test_marlin_words(dev, M, N, K, group):
+    """As for the row-packed layout."""
+    announce("duo marlin", M, N, K, group)
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    ref, q, s = QuantUtils.fake_quantize((torch.randn(K, N, device=dev, generator=gen, dtype=torch.float32) * 0.02).half(), group)
+    words, scales = QuantUtils.pack(q, s, group)
+    weights = ((q.float() - 8) * s.float().repeat_interleave(group, 0)).half()
+    assert torch.equal(weights, ref)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+    workspace = torch.zeros(max(16, N // 128 * 16), dtype=torch.int32, device=dev)
+    k = (7 * torch.arange(M, device=dev) + 3) % K
+    x = torch.zeros(M, K, dtype=torch.float16, device=dev)
+    x[torch.arange(M, device=dev), k] = 1
+    mul(x, words, out, scales, workspace)
+    assert torch.equal(out, weights[k])
+    x = torch.randn(M, K, device=dev, generator=gen, dtype=torch.float32).half()
+    mul(x, words, out, scales, workspace)
+    assert_close_scaled(out, x.double() @ weights.double(), rtol=2 ** -11, atol=2e-5)
