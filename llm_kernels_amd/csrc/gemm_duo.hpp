@@ -30,8 +30,9 @@ constexpr int du_lds(int kind, int mi) {                                      //
 }
 constexpr int du_table(int sub_blocks) { return sub_blocks * DU_BN * 4; }     // second-level scales and zero points, see below
 
-template <int KIND, int MI, bool AS16 = false>
+template <int KIND, int MI, bool AS16 = false, bool GROUPED = false>
 __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
+    static_assert(!GROUPED || KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK, "grouped products: block-scaled 8-bit operands");
     constexpr bool SCALED = du_scaled(KIND), ROWCOL = (KIND == K_I8_ROWCOL), W4A16 = du_w4a16(KIND), MARLIN = (KIND == K_W4MARLIN), W4A8 = (KIND == K_W4A8),
                    EXPANDS = W4A16 || W4A8;
     static_assert(SCALED || ROWCOL || W4A16, "8-bit operands, or 4-bit weights");
@@ -50,14 +51,28 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     const int K = p.K * ESZ;                                 // row length in bytes
     const int KT_all = K >> 7;
     int kt0 = 0, KT = KT_all;                                // sub-blocks [kt0, kt0 + KT) of this workgroup
-    if (p.ksplit > 1) {
+    if (!GROUPED && p.ksplit > 1) {
         const int per = (KT_all + p.ksplit - 1) / p.ksplit;
         kt0 = (int)blockIdx.z * per;
         KT = max(0, min(per, KT_all - kt0));
     }
-    int tile_n, tile_m;
-    xcd_tile((int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
-    const int n0 = tile_n * DU_BN, m_start = tile_m * BM, m_end = min(p.M, m_start + BM);
+    int tile_n = (int)blockIdx.x, tile_m = 0, m_start, m_end;
+    const uint8_t* bbase = p.b;
+    int64_t bs_off = 0;                                      // block scales in front of this expert's
+    if constexpr (GROUPED) {
+        const SegmentTile sg = segment_of(p.seg_indptr, p.E, BM, 1, (int)blockIdx.y);
+        if (!sg.found) return;
+        m_start = sg.s0 + sg.rest * BM;
+        m_end = min(sg.s1, m_start + BM);
+        const int64_t widx = p.weight_indices ? p.weight_indices[sg.e] : sg.e;
+        bbase += widx * (int64_t)N * K;
+        bs_off = widx * (int64_t)((N + 127) / 128) * KT_all;
+    } else {
+        xcd_tile((int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
+        m_start = tile_m * BM;
+        m_end = min(p.M, m_start + BM);
+    }
+    const int n0 = tile_n * DU_BN;
     float* const bsl = (float*)(lds + SW + du_windows(MI));
 
     // ---- source offsets (bytes, 32 bit).  A piece = 8 rows x 128 bytes = one load instruction; chunks XOR-swizzled with (row >> 1) & 7
@@ -193,7 +208,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     auto request = [&](int u) {                              // operands of sub-block u, by the four waves of one group
         const uint32_t sa = lds_base + (uint32_t)(u & 3) * A_SLOT, sb = lds_base + B0 + (uint32_t)(u & 3) * B_SLOT;
         const uint8_t* ga = p.a + (int64_t)(kt0 + u) * 128;
-        const uint8_t* gb = p.b + (int64_t)(kt0 + u) * 128;
+        const uint8_t* gb = bbase + (int64_t)(kt0 + u) * 128;
 #pragma unroll
         for (int i = 0; i < MI; ++i) dma16(sa + (uint32_t)(w4 * MI + i) * 1024u, aoff[i], ga);
         if constexpr (!EXPANDS) {
@@ -277,7 +292,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         for (int i = 0; i < MI; ++i) {
             if constexpr (EXPAND) {
                 if (i < 2) expand_word(f & 3, f + 1, i);
-                if (i == 2) request_words(f & 3, f + 5);
+                if (i == (MI > 2 ? 2 : MI - 1)) request_words(f & 3, f + 5);
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -407,7 +422,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         }
         request_scales(0);
         if constexpr (SCALED) {
-            const int64_t bs_row = (int64_t)tile_n * KT_all + kt0;
+            const int64_t bs_row = bs_off + (int64_t)tile_n * KT_all + kt0;
             for (int i = tid; i < KT; i += DU_THREADS) bsl[i] = ld_scale(p.b_s, bs_row + i, p.s_dtype);
         }
         if constexpr (W4A8) {
@@ -446,7 +461,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 
     // ---- each group keeps half of the tile rows of its waves, passes the other half to its counterpart and stores the sums
     constexpr int H = (MI + 1) / 2;
-    const bool split = p.ksplit > 1;
+    const bool split = !GROUPED && p.ksplit > 1;
     void* const cout = split ? (void*)(p.partial + (int64_t)blockIdx.z * p.M * N) : p.c;
     const int cdt = split ? LLMK_F32 : p.c_dtype;
     auto finish = [&](auto grp_c) {
@@ -533,20 +548,21 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 }
 
 // p.a_s: fp32, or with AS16 the 16-bit scales of dtype p.s_dtype as the caller passed them; p.ksplit / p.partial select the K split.
-template <int KIND, int MI, bool AS16 = false>
+template <int KIND, int MI, bool AS16 = false, bool GROUPED = false>
 int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
     static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_duo_kernel<KIND, MI, AS16>;
+    auto kern = gemm_duo_kernel<KIND, MI, AS16, GROUPED>;
     constexpr int fixed = du_lds(KIND, MI);
     static_assert(fixed <= D_LDS_MAX && 8 * ((MI + 1) / 2) * 4096 <= fixed, "slots, and the exchange of half the sums in them, fit in LDS");
     const int KT = (p.K * (is_half(KIND) ? 2 : 1)) >> 7, z = p.ksplit > 1 ? p.ksplit : 1;
     const int lds_bytes = fixed + (KIND == K_W4A8 ? du_table((KT + z - 1) / z) : 0);
     if (lds_bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, lds_bytes);
     if (int rc = llmk_reserve_lds((const void*)kern, KIND == K_W4A8 ? D_LDS_MAX : fixed, configured, name)) return rc;
-    const bool split = p.ksplit > 1 && p.partial;
+    const bool split = !GROUPED && p.ksplit > 1 && p.partial;
     DirectArgs q = p;
     q.ksplit = split ? p.ksplit : 1;
-    dim3 grid((unsigned)((p.N + DU_BN - 1) / DU_BN), (unsigned)((p.M + 32 * MI - 1) / (32 * MI)), (unsigned)q.ksplit);
+    const int tiles_m = GROUPED ? grouped_row_tiles(p.M, p.E, 32 * MI) : (p.M + 32 * MI - 1) / (32 * MI);
+    dim3 grid((unsigned)((p.N + DU_BN - 1) / DU_BN), (unsigned)tiles_m, (unsigned)q.ksplit);
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
     kern<<<grid, DU_THREADS, lds_bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
@@ -610,6 +626,27 @@ int launch_duo_plan(DirectArgs p, const DuoPlan& pl, void* workspace, hipStream_
     if constexpr (duo_built<KIND>(6)) if (pl.mi == 6) return launch_duo<KIND, 6, AS16>(p, stream, name);
     if constexpr (duo_built<KIND>(5)) if (pl.mi == 5) return launch_duo<KIND, 5, AS16>(p, stream, name);
     return pl.mi == 4 ? launch_duo<KIND, 4, AS16>(p, stream, name) : launch_duo<KIND, 3, AS16>(p, stream, name);
+}
+
+// Grouped products: tile height (mi; 0: not for this kernel) where an expert's rows are one tile and all tiles one round of the chip.
+// The rows of a segment are only known on the device: mean + 1.5 standard deviations of an even routing are taken for the longest.
+// There each workgroup reads its share of the weights once, and the deeper queue of loads is what counts (us, the 64- and 128-row
+// tiles of gemm_dma_kernel | these: fp8 8 experts of 4096 x 14336, 362 rows 88 | 84, 512 98 | 88, 860 135 | 101; int8 452 rows 158 | 88;
+// over 299 random shapes inside the rule 1.13 fp8, 1.20 int8, eight of them lose 3 to 17 %).  Outside it they are level or behind:
+// above 200 tiles of up to 64 rows from 7168 columns or fewer, two workgroups a CU of the 64-row tile keep as much in flight
+// (8 x 4096 x 7168, 256 rows 37 | 39), and with more than one round (16 experts of 4096 x 4096, 1448 rows) the 256-column tiles
+// take 44 us, these 54.  From 5120 columns: 16 x 4096 x 2048, 980 rows 27 | 28.
+inline int grouped_duo_mi(const DirectArgs& p) {
+    if (p.E <= 0 || p.K < 5120 || !dma_eligible(p)) return 0;
+    const double rows = (double)p.M / p.E, longest = rows + 1.5 * __builtin_sqrt(rows);
+    const int64_t tiles = (int64_t)p.E * ((p.N + DU_BN - 1) / DU_BN);
+    if (rows < 20.0 || longest > 128.0 || tiles > LLMK_CUS || (tiles > 200 && p.K < 8192 && rows < 64.0)) return 0;
+    return longest <= 64.0 ? 2 : (longest <= 96.0 ? 3 : 4);
+}
+template <int KIND, bool AS16>
+int launch_grouped_duo(const DirectArgs& p, int mi, hipStream_t stream, const char* name) {
+    if (mi == 2) return launch_duo<KIND, 2, AS16, true>(p, stream, name);
+    return mi == 3 ? launch_duo<KIND, 3, AS16, true>(p, stream, name) : launch_duo<KIND, 4, AS16, true>(p, stream, name);
 }
 
 }  // namespace llmk

@@ -1,5 +1,6 @@
 // Single-GPU expert-parallel MoE path: segment bookkeeping, token permute / un-permute,
 // gated activation, and the grouped GEMM over one GPU's experts.
+#include "gemm_duo.hpp"
 #include "gemm_wide.hpp"
 #include "quant_util.hpp"
 
@@ -728,6 +729,10 @@ extern "C" int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind
     // leaves each of them a fraction of the column workgroups (measured: tile kernels faster from six row tiles).
     const bool big = M > 64 * (int64_t)E || (M > 2 * (int64_t)E && N * K >= ((int64_t)20 << 20)) ||
                      grouped_row_tiles((int)M, E, 16) >= 6;
+    const int duo = big && scaled && (kind == LLMK_KIND_I8 || s_dtype == LLMK_F32) ? grouped_duo_mi(p) : 0;
+    if (duo && kind == LLMK_KIND_FP8) return launch_grouped_duo<K_FP8_BLOCK, false>(p, duo, st, "grouped_gemm(fp8, duo)");
+    if (duo && s_dtype == LLMK_F32) return launch_grouped_duo<K_I8_BLOCK, false>(p, duo, st, "grouped_gemm(i8, duo)");
+    if (duo) return launch_grouped_duo<K_I8_BLOCK, true>(p, duo, st, "grouped_gemm(i8, duo)");
     if (big && kind == LLMK_KIND_I8) return launch_big<K_I8_BLOCK, true>(p, workspace, workspace_bytes, st, "grouped_gemm(i8, tiled)");
     if (big && kind == LLMK_KIND_FP8) return launch_big<K_FP8_BLOCK, true>(p, workspace, workspace_bytes, st, "grouped_gemm(fp8, tiled)");
     if (big && kind == LLMK_KIND_F16 && dma_eligible(p, 2)) return launch_big_half<K_F16, true>(p, st, "grouped_gemm(f16, tiled)");

@@ -428,6 +428,43 @@ def test_grouped_gemm_many_segments_exact(dev, E, rows, N, K):
     assert torch.all(out[used:] == 5.0)
 
 
+@pytest.mark.parametrize("kind,scales", [("fp8", torch.float32), ("int8", torch.float32), ("int8", torch.float16), ("int8", torch.bfloat16)])
+@pytest.mark.parametrize("E,rows,N,K", [(3, 20, 272, 5120), (3, 52, 200, 5248), (3, 54, 128, 5376), (3, 82, 264, 5504), (4, 84, 328, 5632), (4, 112, 136, 5760),
+                                        (70, 40, 136, 5120), (3, 20, 8800, 5248)])
+def test_grouped_gemm_one_tile_an_expert(dev, kind, scales, E, rows, N, K):
+    """The tile heights of the two-group kernel on both sides of their borders, every remainder of K by its loop of four, and one shape
+    beyond it (201 tiles of short segments): segments longer than a tile, of one row and empty, rows behind the last one keep their fill
+    value, permuted weight indices, ragged columns.  Scales are powers of two and the operands small whole numbers: sums below 2^24
+    quarters, exact in every order."""
+    from llm_kernels_amd import _lib
+    announce("grouped one tile an expert", kind, scales, E, rows, N, K)
+    gen = torch.Generator().manual_seed(E + rows + N + K)
+    lens = torch.randint(rows - 8, rows + 9, (E,), generator=gen)
+    lens[0], lens[1] = 1, 2 * rows + 40
+    if E > 2:
+        lens[2] = 0
+    seg = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    used, M = int(seg[-1]), rows * E
+    M = max(M, used + 1)
+    a = torch.randint(-7, 8, (M, K), generator=gen).to(dev)
+    b = torch.randint(-7, 8, (E, N, K), generator=gen, dtype=torch.int8).to(dev)
+    a_s = (2.0 ** torch.randint(-1, 2, (M, K // 128), generator=gen)).to(dev, scales)
+    b_s = (2.0 ** torch.randint(-1, 2, (E, (N + 127) // 128, K // 128), generator=gen)).to(dev, scales)
+    qt = torch.float8_e4m3fn if kind == "fp8" else torch.int8
+    widx = torch.randperm(E, generator=gen)
+    c = torch.full((M, N), 5.0, dtype=torch.float32, device=dev)
+    d = [t.contiguous() for t in (a.to(qt), b.to(qt), seg.to(dev), widx.to(dev))]
+    work = torch.empty(_lib.load().llmk_gemm_workspace_bytes(M, N, K), dtype=torch.uint8, device=dev)
+    _lib.call("llmk_grouped_gemm", _lib.ptr(d[0]), _lib.ptr(d[1]), _lib.ptr(c), _lib.KIND_FP8 if kind == "fp8" else _lib.KIND_I8, _lib.F32, E, M, N, K,
+              _lib.ptr(d[2]), _lib.ptr(d[3]), _lib.ptr(a_s), _lib.ptr(b_s), _lib.dt(scales), _lib.ptr(work), work.numel(), _lib.stream(c))
+    for e in range(E):
+        lo, hi = int(seg[e]), int(seg[e + 1])
+        w = int(widx[e])
+        wide = b[w].float() * b_s[w].float().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
+        assert torch.equal(c[lo:hi], (a[lo:hi].float() * a_s[lo:hi].float().repeat_interleave(128, 1)) @ wide.T), "segment %d" % e
+    assert torch.all(c[used:] == 5.0)
+
+
 def _lib_call_grouped_i8(dev, a, a_s, b, b_s, c, seg, widx):
     """grouped_gemm_triton on activations that are already int8 with their 1 x 128 scales."""
     d = [t.to(dev).contiguous() for t in (a, a_s, b, b_s, seg.long(), widx.long())]
