@@ -25,10 +25,21 @@ constexpr int du_windows(int mi) { return 2 * 32 * mi * 4 * 4; }             // 
 constexpr bool du_scaled(int kind) { return kind == K_FP8_BLOCK || kind == K_I8_BLOCK || kind == K_W4A8; }
 constexpr bool du_w4a16(int kind) { return is_w4nk(kind) || kind == K_W4MARLIN; }
 constexpr bool du_expands(int kind) { return du_w4a16(kind) || kind == K_W4A8; }
+// 160 rows of block-scaled operands: the registers just suffice, see the end of the main loop.  (us, cached weights | from HBM, without this tile ->
+// with it: fp8 145 x 25320 x 6528 45.7 | 60.1 -> 35.4 | 49.2, 918 x 4224 x 6528 42.9 | 51.2 -> 31.9 | 39.2, 1194 x 4096 x 14336 80 | 90 -> 69 | 78, int8 157 x
+// 28672 x 4096 37.9 | 43.2 -> 28.7 | 37.0, 287 x 14336 x 4096 31.9 | 42.4 -> 26.1 | 29.8, 1262 x 4096 x 4096 35.7 | 34.7 -> 29.2 | 29.1)
+constexpr bool du_tight(int kind, int mi) { return du_scaled(kind) && !du_expands(kind) && mi > 4; }
 constexpr int du_lds(int kind, int mi) {                                      // K_W4A8: + du_table bytes
     return DU_SLOTS * du_a(mi) + (du_expands(kind) ? 2 : DU_SLOTS) * du_b() + (du_scaled(kind) ? du_windows(mi) + D_MAX_KT * 4 : 0);
 }
 constexpr int du_table(int sub_blocks) { return sub_blocks * DU_BN * 4; }     // second-level scales and zero points, see below
+
+// An offset in a register of its own: the compiler multiplies and adds in 64 bits and then keeps both halves for as long as the lower one is used.
+__device__ __forceinline__ uint32_t only32(uint32_t x) {
+    uint32_t y;
+    asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+    return y;
+}
 
 template <int KIND, int MI, bool AS16 = false, bool GROUPED = false>
 __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
@@ -39,6 +50,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     constexpr int MATH = W4A8 ? K_I8_BLOCK : KIND;           // the products once the weights are expanded
     constexpr int ESZ = is_half(KIND) ? 2 : 1, BM = 32 * MI, WR = 16 * MI;
     constexpr int A_SLOT = du_a(MI), B_SLOT = du_b(), B0 = DU_SLOTS * A_SLOT, NB = EXPANDS ? 2 : DU_SLOTS, SW = B0 + NB * B_SLOT;
+    constexpr bool TIGHT = du_tight(KIND, MI);
     constexpr int LP = MI + (W4A8 ? 2 : 4);                  // loads of a wave from one of its turns to the end of the next
     constexpr int NSW = (2 * MI + 7) / 8;                    // scale loads per wave and window (16 rows x 4 sub-blocks each)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -77,20 +89,23 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 
     // ---- source offsets (bytes, 32 bit).  A piece = 8 rows x 128 bytes = one load instruction; chunks XOR-swizzled with (row >> 1) & 7
     // as everywhere.  Weight rows are permuted inside each 64 so that a lane ends up with two runs of 8 consecutive columns.
-    const int row8 = lane >> 3;
+    auto column = [](int R) { const int rho = R & 63; return (R & 64) + 32 * (rho >> 5) + 8 * ((rho & 15) >> 2) + 4 * ((rho >> 4) & 1) + (rho & 3); };
+    auto a_offset = [&](int i, int l) {
+        const int R = 8 * (w4 * MI + i) + (l >> 3);
+        const uint32_t off = (uint32_t)min(m_start + R, m_end - 1) * (uint32_t)K + (uint32_t)((l & 7) ^ ((R >> 1) & 7)) * 16u;
+        return TIGHT ? only32(off) : off;
+    };
+    auto b_offset = [&](int i, int l) {
+        const int R = 8 * (w4 * 4 + i) + (l >> 3);
+        const uint32_t off = (uint32_t)min(n0 + column(R), N - 1) * (uint32_t)K + (uint32_t)((l & 7) ^ ((R >> 1) & 7)) * 16u;
+        return TIGHT ? only32(off) : off;
+    };
     uint32_t aoff[MI], boff[4];
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        const int R = 8 * (w4 * MI + i) + row8;
-        aoff[i] = (uint32_t)min(m_start + R, m_end - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((R >> 1) & 7)) * 16u;
-    }
-    auto column = [](int R) { const int rho = R & 63; return (R & 64) + 32 * (rho >> 5) + 8 * ((rho & 15) >> 2) + 4 * ((rho >> 4) & 1) + (rho & 3); };
+    for (int i = 0; i < MI; ++i) aoff[i] = a_offset(i, lane);
     if constexpr (!EXPANDS) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int R = 8 * (w4 * 4 + i) + row8;
-            boff[i] = (uint32_t)min(n0 + column(R), N - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((R >> 1) & 7)) * 16u;
-        }
+        for (int i = 0; i < 4; ++i) boff[i] = b_offset(i, lane);
     }
     // 4-bit weights: in phase f every thread expands 16 weights of sub-block f + 1 from a packed double word and its scales, requested four
     // phases ago (set f & 3).  Row-packed: quarter t & 3 of weight row t >> 2.  Marlin words: half h of the unit of strip sl, chunk ch, columns
@@ -383,6 +398,16 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         words_landed(3);
     };
     auto last_turn = [&](int u) __attribute__((always_inline)) {
+        if constexpr (TIGHT) {                               // (worked out again: no registers to keep them through these turns)
+            int l = lane;
+            asm volatile("" : "+v"(l));
+#pragma unroll
+            for (int i = 0; i < MI; ++i) aoff[i] = a_offset(i, l);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) boff[i] = b_offset(i, l);
+#pragma unroll
+            for (int i = 0; i < NSW; ++i) srow[i] = (uint32_t)min(m_start + 16 * min(wave + 8 * i, 2 * MI - 1) + (l >> 2), m_end - 1) * (uint32_t)KT_all;
+        }
         if (u + 3 < KT) request(u + 3);
         if constexpr (SCALED) if ((u & 3) < 2 && (u | 3) + 1 < KT) request_scales((u >> 2) + 1);
         if constexpr (W4A8) {
@@ -504,6 +529,10 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 
     // Four phases a loop turn (the last operands they request are those of sub-block 4 q + 6), then phase by phase what is left.
     const int rounds = KT >= 7 ? (KT - 3) >> 2 : 0;
+    auto nothing_left = [&]() __attribute__((always_inline)) {               // an odd number of sub-blocks: nothing left to multiply
+        clear();
+        meet(any);
+    };
     if (wave < 4) {
         for (int q = 0; q < rounds; ++q) {
             turn(4 * q, yes);
@@ -513,14 +542,16 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             multiply(yes, 4 * q + 3);
             meet(any);
         }
-        all_landed();
-        for (int u = 4 * rounds; u < KT; u += 2) {
-            last_turn(u);
-            last_words(u + 1);
-            multiply(no, 0);
-            last_meet();
+        if constexpr (!TIGHT) {
+            all_landed();
+            for (int u = 4 * rounds; u < KT; u += 2) {
+                last_turn(u);
+                last_words(u + 1);
+                multiply(no, 0);
+                last_meet();
+            }
+            finish(std::integral_constant<int, 0>{});
         }
-        finish(std::integral_constant<int, 0>{});
     } else {
         for (int q = 0; q < rounds; ++q) {
             multiply(yes, 4 * q);
@@ -530,20 +561,38 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             meet(any);
             turn(4 * q + 3, no);
         }
-        all_landed();
-        for (int u = 4 * rounds; u < KT; u += 2) {
-            last_words(u);
+        if constexpr (!TIGHT) {
+            all_landed();
+            for (int u = 4 * rounds; u < KT; u += 2) {
+                last_words(u);
+                multiply(no, 0);
+                last_meet();
+                if (u + 1 < KT) last_turn(u + 1);
+                else nothing_left();
+            }
             multiply(no, 0);
-            last_meet();
-            if (u + 1 < KT) {
-                last_turn(u + 1);
-            } else {                                         // an odd number of sub-blocks: nothing left to multiply
-                clear();
-                meet(any);
+            finish(std::integral_constant<int, 1>{});
+        }
+    }
+    if constexpr (TIGHT) {
+        // one loop for both groups: with a loop each, the compiler keeps the registers of the second through the first and spills (a loop each is
+        // 1.3 us faster where they suffice: the registers move between the main loops and this one)
+        for (int f = 4 * rounds; f < ((KT + 1) & ~1); ++f) {
+            if ((f & 1) != (wave >> 2)) {
+                multiply(no, 0);
+                last_meet();
+            } else if (f < KT) {
+                last_turn(f);
+            } else {
+                nothing_left();
             }
         }
-        multiply(no, 0);
-        finish(std::integral_constant<int, 1>{});
+        if (wave < 4) {
+            finish(std::integral_constant<int, 0>{});
+        } else {
+            multiply(no, 0);
+            finish(std::integral_constant<int, 1>{});
+        }
     }
 }
 
@@ -569,11 +618,11 @@ int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
     return split ? launch_splitk_sum<KIND == K_W4A8 ? K_I8_BLOCK : KIND>(q, q.ksplit, stream, name) : LLMK_OK;
 }
 
-// Tile heights that are built (32 mi rows).  Block-scaled kinds end at 128 rows: at 160 the fragments of a sub-block and the products that
-// wait for their scales spill.
+// Tile heights that are built (32 mi rows); at the next one the fragments of a sub-block, the sums and what waits to be expanded or scaled
+// spill.
 template <int KIND>
 constexpr bool duo_built(int mi) {
-    return mi >= 3 && mi <= (is_w4nk(KIND) ? 6 : (KIND == K_I8_ROWCOL || KIND == K_W4MARLIN ? 5 : 4));
+    return mi >= 3 && mi <= (is_w4nk(KIND) ? 6 : (KIND == K_W4A8 ? 4 : 5));
 }
 // Estimated microseconds: base + rounds of 256 workgroups x (round + sub-blocks x step[mi - 3]) + out x MB of the output, and for K slices
 // split + plane x MB of the fp32 planes.  A fit of 4 to 7 % rms to 300 random shapes a kind of M 64 to 4096, N 1024 to 28672, K 1024 to
@@ -583,8 +632,8 @@ struct DuoModel {
 };
 template <int KIND>
 constexpr DuoModel duo_model() {
-    if (KIND == K_FP8_BLOCK) return {2.0f, 1.4f, {0.396f, 0.452f, 0.f, 0.f}, 3.4f, 0.50f, 0.48f};
-    if (KIND == K_I8_BLOCK) return {2.4f, 1.4f, {0.417f, 0.502f, 0.f, 0.f}, 2.9f, 0.58f, 0.57f};
+    if (KIND == K_FP8_BLOCK) return {2.0f, 1.4f, {0.396f, 0.452f, 0.515f, 0.f}, 3.4f, 0.50f, 0.48f};
+    if (KIND == K_I8_BLOCK) return {2.4f, 1.4f, {0.417f, 0.502f, 0.585f, 0.f}, 2.9f, 0.58f, 0.57f};
     if (KIND == K_W4MARLIN) return {3.03f, 2.53f, {0.460f, 0.519f, 0.589f, 0.f}, 2.9f, 0.45f, 0.31f};
     if (KIND == K_W4A8) return {1.76f, 2.62f, {0.614f, 0.683f, 0.f, 0.f}, 3.0f, 0.55f, 0.37f};
     if (KIND == K_I8_ROWCOL) return {2.79f, 1.59f, {0.355f, 0.406f, 0.470f, 0.f}, 2.9f, 0.47f, 0.57f};
@@ -614,7 +663,11 @@ DuoPlan duo_plan(const DirectArgs& p, int64_t scratch) {
             if (z > 1 && (tiles * z > LLMK_CUS || KT / z < 6 || (int64_t)z * p.M * p.N * 4 > planes)) break;
             if (KIND == K_W4A8 && du_lds(KIND, mi) + du_table((KT + z - 1) / z) > D_LDS_MAX) continue;
             const double rounds = (double)((tiles * z + LLMK_CUS - 1) / LLMK_CUS);
-            const double c = m.base + rounds * (m.round + (KT + z - 1) / z * m.step[mi - 3]) + 2.0 * m.out * out + (z > 1 ? m.split + 4.0 * m.plane * out * z : 0.0);
+            // the tight tile: its shared last loop costs 1.8 us a tile, and beyond 512 rows and a round of them the 256-column tiles are the
+            // faster ones, which their estimates there do not show (fp8 2337 x 4096 x 4096 45.0 | 49.3 this one, int8 2375 x 28672 x 4096 320 | 333)
+            if (du_tight(KIND, mi) && p.M > 512 && tiles > LLMK_CUS) break;
+            const double round = m.round + (du_tight(KIND, mi) ? 1.8 : 0.0);
+            const double c = m.base + rounds * (round + (KT + z - 1) / z * m.step[mi - 3]) + 2.0 * m.out * out + (z > 1 ? m.split + 4.0 * m.plane * out * z : 0.0);
             if (c < best.cost) best = {mi, z, c};
         }
     }
