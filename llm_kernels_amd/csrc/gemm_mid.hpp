@@ -113,7 +113,13 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
         KT = max(0, min(per, KT_all - kt0));
     }
     const int nsteps = (KT + NSUB - 1) / NSUB;
-    const int n0 = blockIdx.x * BN, m_start = blockIdx.y * BM, m_end = min(p.M, m_start + BM);
+    // The tile order of xcd_tile where row-major order does not deal whole columns to the XCDs already (one row of tiles: it does; per token 34 x
+    // 12816 x 4864 14.2 row-major, 15.0 so), and the operands do not fit an XCD's L2
+    // of 4 MB anyway (there its divisions are all one sees: 4-bit weights 158 x 4784 x 1152 8.4 us row-major, 8.9 so).  us, row-major | so: fp8
+    // 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840 15.2 | 10.8, int8 145 x 5056 x 3840 14.4 | 10.6, 4-bit weights 346 x 4160 x 1920 17.7 | 16.6.
+    int tile_n = (int)blockIdx.x, tile_m = (int)blockIdx.y;
+    if (gridDim.x % 8 != 0 && gridDim.y > 1 && (int64_t)N * (W4NK ? K >> 2 : K) + (int64_t)p.M * K > (4 << 20)) xcd_tile(tile_m * (int)gridDim.x + tile_n, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
+    const int n0 = tile_n * BN, m_start = tile_m * BM, m_end = min(p.M, m_start + BM);
     float* const bsl = (float*)(lds + (mdp_lds(MT, WIDE) - D_MAX_KT * 4));
 
     // acc[i][j][e] = C[row 16 i + r][column 64 half + 16 j + 4 g + e] summed over sub-block ksub of all steps (consumers)

@@ -10,6 +10,7 @@ import torch
 
 from oracle import gemm_ref as g, quant_ref as q, bitpack_ref as bp
 from llm_kernels_amd import _lib
+from llm_kernels_amd.fast_dequant import w4a16
 from llm_kernels_amd.quantization import fp8_kernel, int8_kernel, w4a8_kernel
 from helpers import announce, assert_close_scaled, default_dtype
 
@@ -510,6 +511,34 @@ def test_mid_and_small_tile_kernels_exact_integers(dev, M, N, K):
         _, acc = int8_kernel.int8_gemm_per_token(a.to(dev), torch.ones(M).to(dev), b.to(dev), torch.ones(N).to(dev),
                                                  return_int32=True)
         assert torch.equal(acc.cpu().long(), ref), "int8 per token"
+
+
+@pytest.mark.parametrize("M,N,K", [(398, 3352, 5504), (384, 2496, 3840), (145, 5056, 3840), (237, 3384, 7808), (223, 1872, 11392), (70, 12353, 1280),
+                                   (506, 3133, 3328), (97, 5504, 10368), (33, 8321, 2048), (120, 11331, 4224), (200, 9473, 2176)])
+def test_mid_size_tiles_in_the_order_of_the_xcds(dev, M, N, K):
+    """Column tiles that are no multiple of eight and operands beyond 4 MB: the tiles are dealt to the XCDs in blocks, with one to eight tile rows,
+    a ragged last one and K slices.  Small integers: every partial sum is exact, also with fp16 and bf16 activations on 4-bit weights."""
+    announce("mid-size tile order", M, N, K)
+    gen = torch.Generator(device=dev).manual_seed(M + N + K)
+    a = torch.randint(-7, 8, (M, K), device=dev, generator=gen)
+    b = torch.randint(-7, 8, (N, K), device=dev, generator=gen)
+    ref = a.double() @ b.double().T
+    ones, wones = torch.ones(M, K // 128, device=dev), torch.ones((N + 127) // 128, K // 128, device=dev)
+    with default_dtype(torch.float32):
+        assert torch.equal(int8_kernel.int8_gemm(a.to(torch.int8), ones.half(), b.to(torch.int8), wones.half()).double(), ref), "int8"
+        assert torch.equal(fp8_kernel.fp8_gemm(a.float().to(torch.float8_e4m3fn), ones, b.float().to(torch.float8_e4m3fn), wones).double(), ref), "fp8"
+        _, acc = int8_kernel.int8_gemm_per_token(a.to(torch.int8), torch.ones(M, device=dev), b.to(torch.int8), torch.ones(N, device=dev), return_int32=True)
+        assert torch.equal(acc.double(), ref), "per token"
+    nib = (b + 8).view(N, K // 8, 8)                         # element i of a word in bits 4 i .. 4 i + 3
+    words = torch.zeros(N, K // 8, dtype=torch.int64, device=dev)
+    for i in range(8):
+        words |= nib[:, :, i] << (4 * i)
+    words = torch.where(words >= 1 << 31, words - (1 << 32), words).to(torch.int32)
+    scales = torch.full((N, K // 128), 2.0 ** -10, dtype=torch.float16, device=dev)
+    # half a last place of the rounded sum: 11 significant bits in fp16, 8 in bf16, so at most 2^-11 and 2^-8 of the value
+    for dt, half in ((torch.float16, 2.0 ** -11), (torch.bfloat16, 2.0 ** -8)):
+        y = w4a16.w4a16_gemm(a.to(dt), words, scales, 128).double() * 1024
+        assert bool(((y - ref).abs() <= half * ref.abs()).all()), dt
 
 
 @pytest.mark.parametrize("M,N,K", [(130, 9000, 640), (300, 5000, 1152), (500, 3208, 384), (100, 16000, 256), (128, 20000, 640),
