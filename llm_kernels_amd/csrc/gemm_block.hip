@@ -32,13 +32,17 @@ inline int stream_k_ranges(int64_t M, int64_t N, int64_t K) {
 // mid-size kernels with 64 and 128 columns, the 128-column tile in K slices, or rounds of the tiles that dma_tile_estimate chooses.
 // Up to 16 rows, and up to 64 on weights that no tile kernel fills the chip with or without scratch for their K slices, the wave
 // kernels have no rival.
+// hbm: the mean of weights in the cache and weights from HBM (nk: the weights' MB) where it is far from the former, which is what the estimate of
+// the two-group kernel gives: 64-row tiles beyond 8 KB rows 1.07, K slices in more than a round 1.11 to 1.16, 128-row tiles 1.04 to 1.08,
+// 128 x 256 tiles 0.88 times the other one (600 timings of 200 random shapes of 65 to 512 rows; 3 to 7 % rms so).
 template <int KIND>
-double tiles_estimate(const DirectArgs& p, bool scratch) {
+double tiles_estimate(const DirectArgs& p, bool scratch, bool hbm = false) {
     const int64_t M = p.M, N = p.N, K = p.K;
-    const double k = (double)K / 4096.0;
+    const double k = (double)K / 4096.0, nk = (double)N * K * 1e-6, plane = 4e-6 * (double)M * N;
     if (M <= 16 || (M <= 64 && (!scratch || !(mid_m_prefers_tiles(M, N, K) || mid_wanted(M, N, K))))) return 1e30;
     if (mid_wanted(M, N, K)) {
         const MidPlan pl = mid_plan(M, N, K);
+        if (hbm && K > 8192 && pl.z == 1) return 3.6 + 6.7 * k + 0.06 * nk;
         return (pl.mt == 2 ? 3.2 + 7.4 * k / pl.z : 4.0 + 7.2 * k / pl.z) + (pl.z > 1 ? 2.9 : 0.0);
     }
     if (KIND == K_FP8_BLOCK && midw_wanted(M, N, K)) {
@@ -52,11 +56,14 @@ double tiles_estimate(const DirectArgs& p, bool scratch) {
     // 300 x 4096 x 14336 48.1 | 42.5, but 400 x 1030 x 9088 14.1 | 18.5).
     if (z > 1) {
         const bool one = ((M + 63) / 64) * ((N + 127) / 128) * z <= LLMK_CUS;
+        if (hbm && !one) return (KIND == K_I8_ROWCOL ? 8.2 + 13.2 * k / z : 1.8 + 22.7 * k / z) + 0.59 * z * plane + 0.076 * nk;
         if (KIND == K_I8_ROWCOL) return one ? 7.0 + 13.5 * k / z : 10.0 + 16.5 * k / z;
         return 8.0 + (one ? 15.0 : 24.0) * k / z;
     }
     const TileChoice c = dma_tile_estimate<KIND, false>(p);
     const double e = c.cost * k * (KIND == K_I8_BLOCK ? 1.12 : 1.0);
+    if (hbm && c.choice == 2) return 5.0 + (KIND == K_I8_BLOCK ? 0.77 : 0.74) * e;
+    if (hbm && c.choice == 9 && KIND != K_I8_BLOCK) return 7.0 + 0.69 * e;
     return c.choice == 1 ? 3.4 + 0.87 * e : (c.choice == 2 ? 5.0 + 0.7 * e : (c.choice == 8 ? 9.0 + 0.85 * e : 7.5 + 0.8 * e));
 }
 // The wave kernel for this call (gemm_wave.hpp), or nw = 0: up to 512 rows, where it is estimated 8 % below the tile kernels, or 16 %.  The
@@ -98,12 +105,14 @@ double large_estimate(const DirectArgs& p, bool tail) {
 // kernel, if it does).  Over 300 random shapes of 64 to 4096 rows a kind this was 1.04 (fp8, int8, per token) times as fast as without,
 // 0.5 to 1 % behind the faster one of each shape, at worst 5 % (16 % once) slower.  Others | this one, us: fp8 1024 x 4096 x 4096 25.5 | 20.7, int8 28.8 |
 // 25.6, per token 23.9 | 20.3; the gain is largest where 96, 128 or 160 rows leave fewer rows of the last tiles empty than 64, 128 and
-// 256 do, and where few tiles can be split along K beyond 512 rows.
+// 256 do, and where few tiles can be split along K beyond 512 rows.  Up to 512 rows the others are estimated with weights from HBM in the mean (450
+// shapes 1.007 fp8, 1.002 int8, 1.005 per token times as fast as with their cached times, us, cached | HBM: fp8 129 x 4096 x 14336 22.8 | 33.6 -> 20.7 |
+// 23.9, int8 110 x 15992 x 12032 48.5 | 66.3 -> 40.6 | 49.0, per token 452 x 3176 x 10112 31.1 | 37.5 -> 24.7 | 30.3; at worst 3.5 % slower).
 template <int KIND>
 DuoPlan duo_choice(const DirectArgs& p, const WavePlan& w, int64_t scratch, bool tiles_scratch, bool tail) {
     DuoPlan d = duo_plan<KIND>(p, scratch);
     if (!d.mi) return d;
-    const double other = p.M <= 512 ? (w.nw ? 1.05 * w.cost : tiles_estimate<KIND>(p, tiles_scratch)) : large_estimate<KIND>(p, tail);
+    const double other = p.M <= 512 ? (w.nw ? 1.05 * w.cost : tiles_estimate<KIND>(p, tiles_scratch, true)) : large_estimate<KIND>(p, tail);
     if (1.08 * d.cost >= other) d.mi = 0;
     return d;
 }

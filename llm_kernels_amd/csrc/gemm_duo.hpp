@@ -632,8 +632,8 @@ struct DuoModel {
 };
 template <int KIND>
 constexpr DuoModel duo_model() {
-    if (KIND == K_FP8_BLOCK) return {2.0f, 1.4f, {0.396f, 0.452f, 0.515f, 0.f}, 3.4f, 0.50f, 0.48f};
-    if (KIND == K_I8_BLOCK) return {2.4f, 1.4f, {0.417f, 0.502f, 0.585f, 0.f}, 2.9f, 0.58f, 0.57f};
+    if (KIND == K_FP8_BLOCK) return {2.0f, 1.4f, {0.396f, 0.452f, 0.515f, 0.f}, 3.0f, 0.47f, 0.48f};
+    if (KIND == K_I8_BLOCK) return {2.4f, 1.4f, {0.417f, 0.502f, 0.585f, 0.f}, 3.1f, 0.45f, 0.57f};
     if (KIND == K_W4MARLIN) return {3.03f, 2.53f, {0.460f, 0.519f, 0.589f, 0.f}, 2.9f, 0.45f, 0.31f};
     if (KIND == K_W4A8) return {1.76f, 2.62f, {0.614f, 0.683f, 0.f, 0.f}, 3.0f, 0.55f, 0.37f};
     if (KIND == K_I8_ROWCOL) return {2.79f, 1.59f, {0.355f, 0.406f, 0.470f, 0.f}, 2.9f, 0.47f, 0.57f};

@@ -114,9 +114,9 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
     }
     const int nsteps = (KT + NSUB - 1) / NSUB;
     // The tile order of xcd_tile where row-major order does not deal whole columns to the XCDs already (one row of tiles: it does; per token 34 x
-    // 12816 x 4864 14.2 row-major, 15.0 so), and the operands do not fit an XCD's L2
-    // of 4 MB anyway (there its divisions are all one sees: 4-bit weights 158 x 4784 x 1152 8.4 us row-major, 8.9 so).  us, row-major | so: fp8
-    // 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840 15.2 | 10.8, int8 145 x 5056 x 3840 14.4 | 10.6, 4-bit weights 346 x 4160 x 1920 17.7 | 16.6.
+    // 12816 x 4864 14.2 us row-major, 15.0 so) and the operands do not fit an XCD's L2 of 4 MB anyway (there its divisions are all one sees:
+    // 4-bit weights 158 x 4784 x 1152 8.4 row-major, 8.9 so).  Row-major | so: fp8 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840 15.2 | 10.8, int8
+    // 145 x 5056 x 3840 14.4 | 10.6, 4-bit weights 346 x 4160 x 1920 17.7 | 16.6.
     int tile_n = (int)blockIdx.x, tile_m = (int)blockIdx.y;
     if (gridDim.x % 8 != 0 && gridDim.y > 1 && (int64_t)N * (W4NK ? K >> 2 : K) + (int64_t)p.M * K > (4 << 20)) xcd_tile(tile_m * (int)gridDim.x + tile_n, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
     const int n0 = tile_n * BN, m_start = tile_m * BM, m_end = min(p.M, m_start + BM);

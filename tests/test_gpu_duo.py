@@ -14,13 +14,13 @@ from helpers import announce, assert_close_scaled, default_dtype
 
 FP8 = [(138, 11136, 128), (136, 11557, 256), (167, 11056, 384), (131, 10896, 640), (133, 11096, 768), (137, 11553, 896), (162, 11128, 1024), (131, 11616, 1152),
        (142, 11264, 1280), (140, 11184, 1408), (751, 216, 3072), (572, 229, 4224), (1777, 224, 4224), (194, 11816, 1024), (209, 11291, 1152), (198, 11448, 1280),
-       (195, 11104, 1408), (2028, 392, 6144), (129, 21994, 640), (131, 21893, 768), (160, 23063, 896), (145, 23235, 1024), (130, 21768, 1152), (153, 22459, 1280),
-       (129, 22056, 1408), (130, 16472, 3072), (1111, 4001, 4224)]
+       (195, 11104, 1408), (2028, 392, 6144), (130, 21768, 1152), (153, 22459, 1280),
+       (129, 22056, 1408), (129, 22198, 1536), (131, 22127, 1664), (129, 16472, 1920), (130, 16472, 3072), (1111, 4001, 4224)]
 INT8 = [(133, 11136, 640), (138, 11373, 768), (141, 11744, 896), (135, 11040, 1152), (137, 11968, 1408), (2044, 456, 6144), (667, 216, 3072), (937, 381, 4224),
         (197, 11248, 3072), (198, 11051, 4224), (129, 22921, 768), (131, 22120, 1152), (147, 21854, 1280), (160, 23189, 1408), (145, 23239, 1536),
         (145, 8197, 7680), (1210, 4090, 4096)]
-PER_TOKEN = [(524, 3632, 1536), (519, 3607, 1152), (526, 248, 3072), (1011, 375, 4224), (289, 8424, 3072), (291, 8344, 4224), (2042, 407, 6144), (450, 8256, 640),
-             (451, 8888, 768), (452, 8391, 1152), (590, 6536, 1408)]
+PER_TOKEN = [(524, 3632, 1536), (519, 3607, 1152), (526, 248, 3072), (1011, 375, 4224), (289, 8424, 3072), (291, 8344, 4224), (2042, 407, 6144), (386, 9363, 768),
+             (452, 8391, 1152), (590, 6536, 1408)]
 W4A8 = [(538, 248, 1024), (543, 328, 1152), (581, 232, 1280), (530, 232, 1408), (545, 224, 1536), (676, 200, 1664), (541, 256, 4224), (576, 976, 4224), (194, 11280, 1024),
         (198, 11008, 1152), (221, 10912, 1280), (195, 11544, 1408), (203, 7088, 6144), (1375, 272, 6144), (1636, 552, 4224), (79, 28672, 4096)]
 MARLIN = [(208, 8576, 768), (208, 8320, 640), (560, 2304, 4096), (576, 192, 1536), (528, 192, 1664), (544, 192, 2176), (800, 320, 4224), (528, 5440, 1024),
