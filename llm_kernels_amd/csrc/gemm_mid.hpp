@@ -75,7 +75,8 @@ constexpr int mdp_lds(int mt, bool wide = false) {
     return (2 * mdp_stage(mt, wide) > mdp_red(mt, wide) ? 2 * mdp_stage(mt, wide) : mdp_red(mt, wide)) + D_MAX_KT * 4;
 }
 
-template <int KIND, int MT, bool AS16 = false, bool WIDE = false>
+// XCDS: the tiles are dealt to the XCDs in blocks (xcd_tile) instead of in row-major order, see launch_mid.
+template <int KIND, int MT, bool AS16, bool WIDE, bool XCDS>
 __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
     static_assert(WIDE ? (MT == 8 || MT == 4) : (MT == 4 || MT == 2), "tile rows");
     constexpr int BN = mdp_bn(WIDE), NSUB = mdp_nsub(WIDE), RED_ROW = BN + 4;
@@ -113,12 +114,8 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
         KT = max(0, min(per, KT_all - kt0));
     }
     const int nsteps = (KT + NSUB - 1) / NSUB;
-    // The tile order of xcd_tile where row-major order does not deal whole columns to the XCDs already (one row of tiles: it does; per token 34 x
-    // 12816 x 4864 14.2 us row-major, 15.0 so) and the operands do not fit an XCD's L2 of 4 MB anyway (there its divisions are all one sees:
-    // 4-bit weights 158 x 4784 x 1152 8.4 row-major, 8.9 so).  Row-major | so: fp8 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840 15.2 | 10.8, int8
-    // 145 x 5056 x 3840 14.4 | 10.6, 4-bit weights 346 x 4160 x 1920 17.7 | 16.6.
     int tile_n = (int)blockIdx.x, tile_m = (int)blockIdx.y;
-    if (gridDim.x % 8 != 0 && gridDim.y > 1 && (int64_t)N * (W4NK ? K >> 2 : K) + (int64_t)p.M * K > (4 << 20)) xcd_tile(tile_m * (int)gridDim.x + tile_n, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
+    if constexpr (XCDS) xcd_tile(tile_m * (int)gridDim.x + tile_n, (int)gridDim.x, (int)gridDim.y, tile_n, tile_m);
     const int n0 = tile_n * BN, m_start = tile_m * BM, m_end = min(p.M, m_start + BM);
     float* const bsl = (float*)(lds + (mdp_lds(MT, WIDE) - D_MAX_KT * 4));
 
@@ -433,15 +430,12 @@ inline bool mid_eligible(const DirectArgs& p) {
 // (and those).  p.ksplit / p.partial select the K split.
 template <int KIND, int MT, bool AS16 = false, bool WIDE = false>
 int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
-    static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_mid_pc_kernel<KIND, MT, AS16, WIDE>;
     constexpr int ESZ = is_half(KIND) ? 2 : 1;
     const int KT_all = (p.K * ESZ) >> 7;
     const bool split = p.ksplit > 1 && p.partial;
     const int per = split ? ((((KT_all + p.ksplit - 1) / p.ksplit) + 3) & ~3) : KT_all;
     constexpr int lds_bytes = mdp_lds(MT, WIDE);
     static_assert(lds_bytes <= D_LDS_MAX, "stages and scale table fit in LDS");
-    if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     // slices that would start past the end of K are not launched
     const int z = split ? (KT_all + per - 1) / per : 1;
     DirectArgs q = p;
@@ -449,8 +443,23 @@ int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
     constexpr int BN = mdp_bn(WIDE);
     dim3 grid((unsigned)((p.N + BN - 1) / BN), (unsigned)((p.M + 16 * MT - 1) / (16 * MT)), (unsigned)z);
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
-    kern<<<grid, MD_THREADS, lds_bytes, stream>>>(q);
-    LLMK_CHECK_LAUNCH(name);
+    auto launch = [&](auto xcds_c) {
+        static std::atomic<uint64_t> configured{0};
+        auto kern = gemm_mid_pc_kernel<KIND, MT, AS16, WIDE, decltype(xcds_c)::value>;
+        if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
+        kern<<<grid, MD_THREADS, lds_bytes, stream>>>(q);
+        LLMK_CHECK_LAUNCH(name);
+        return (int)LLMK_OK;
+    };
+    // Blocks of tiles where row-major order does not deal whole columns to the XCDs already (one row of tiles: it does; per token 34 x 12816 x 4864
+    // 14.2 us row-major, 15.0 so), the operands do not fit an XCD's L2 of 4 MB anyway (4-bit weights 158 x 4784 x 1152 8.4 row-major, 8.9
+    // so), and neither two tile rows of short operand rows (fp8 99 x 9232 x 1152 6.7 | 8.8 cached | from HBM, 7.1 | 9.2 so) nor a few columns in
+    // K slices (330 x 448 x 12288 13.1, 13.9 so) leave little to share.  Row-major | so: fp8 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840
+    // 15.2 | 10.8, int8 145 x 5056 x 3840 14.4 | 10.6, 4-bit weights 346 x 4160 x 1920 17.7 | 16.6.  A kernel each: with the order's divisions in
+    // one kernel, every short call fetched them first (fp8 148 x 3968 x 128 4.6 | 5.0 -> 4.7 | 5.3, 200 x 6144 x 2048 8.2 | 10.3 -> 8.3 | 10.8).
+    const int64_t row = (int64_t)p.K * ESZ, bytes = p.N * row / (is_w4nk(KIND) ? 4 : 1) + p.M * row;
+    const bool xcds = grid.x > 8 && grid.x % 8 != 0 && grid.y > (row < 2048 ? 2 : 1) && bytes > (4 << 20);
+    if (int rc = xcds ? launch(std::true_type{}) : launch(std::false_type{})) return rc;
     if (split) return launch_splitk_sum<KIND>(p, z, stream, name);
     return LLMK_OK;
 }
