@@ -327,6 +327,8 @@ int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind, int c_dty
                       int64_t M, int64_t N, int64_t K, const int64_t* seg_indptr,
                       const int64_t* weight_indices, const void* scale_a, const void* scale_b,
                       int s_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+/* Rows of a tile where block-scaled operands of this shape run on the kernel of two wave groups (fp8: with fp32 scales), else 0. */
+int llmk_grouped_gemm_duo_rows(int E, int64_t M, int64_t N, int64_t K);
 
 /* ------------------------------------------------------------------ calibration (benchmark harness only)
  * No counterpart in the reference and not on the product path: what the chip sustains on the two resources the

@@ -685,16 +685,21 @@ int launch_duo_plan(DirectArgs p, const DuoPlan& pl, void* workspace, hipStream_
 // The rows of a segment are only known on the device: mean + 1.5 standard deviations of an even routing are taken for the longest.
 // There each workgroup reads its share of the weights once, and the deeper queue of loads is what counts (us, the 64- and 128-row
 // tiles of gemm_dma_kernel | these: fp8 8 experts of 4096 x 14336, 362 rows 88 | 84, 512 98 | 88, 860 135 | 101; int8 452 rows 158 | 88;
-// over 299 random shapes inside the rule 1.13 fp8, 1.20 int8, eight of them lose 3 to 17 %).  Outside it they are level or behind:
+// over 299 random shapes inside the rule 1.13 fp8, 1.20 int8).  Outside it they are level or behind:
 // above 200 tiles of up to 64 rows from 7168 columns or fewer, two workgroups a CU of the 64-row tile keep as much in flight
 // (8 x 4096 x 7168, 256 rows 37 | 39), and with more than one round (16 experts of 4096 x 4096, 1448 rows) the 256-column tiles
 // take 44 us, these 54.  From 5120 columns: 16 x 4096 x 2048, 980 rows 27 | 28.
+// Up to half a round and from some 85 rows on, two 64-row tiles an expert stream the weights on twice the CUs: 77 shapes there were 0.92 times
+// as fast on these tiles, with weights from HBM 0.85 (8 experts of 592 x 6912, 684 rows 24.2 | 24.2 cached, 29.7 | 37.0 from HBM; int8 2 of
+// 1448 x 9856, 167 rows 39 | 49).  128-row tiles from 90 rows: a segment beyond 96 would start another round of 96-row ones (int8 8 of
+// 4096 x 14336, 645 rows 117 | 128).
 inline int grouped_duo_mi(const DirectArgs& p) {
     if (p.E <= 0 || p.K < 5120 || !dma_eligible(p)) return 0;
     const double rows = (double)p.M / p.E, longest = rows + 1.5 * __builtin_sqrt(rows);
     const int64_t tiles = (int64_t)p.E * ((p.N + DU_BN - 1) / DU_BN);
     if (rows < 20.0 || longest > 128.0 || tiles > LLMK_CUS || (tiles > 200 && p.K < 8192 && rows < 64.0)) return 0;
-    return longest <= 64.0 ? 2 : (longest <= 96.0 ? 3 : 4);
+    if (longest > 85.0 && tiles <= LLMK_CUS / 2) return 0;
+    return longest <= 64.0 ? 2 : (longest <= 90.0 ? 3 : 4);
 }
 template <int KIND, bool AS16>
 int launch_grouped_duo(const DirectArgs& p, int mi, hipStream_t stream, const char* name) {

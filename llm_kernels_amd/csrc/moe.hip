@@ -703,6 +703,22 @@ extern "C" int llmk_moe_post_reorder(const void* down_out, void* out, int dtype,
     return LLMK_OK;
 }
 
+// Tile kernels when the average segment is longer than 64 rows, and from two rows per expert up when the
+// expert weights are large (measured on 8 experts of 4096 x 14336, whole forward, tile vs weight-streaming
+// kernel: 256 vs 158 us at 1 token, 295 vs 289 us at 8, 344 vs 374 us at 16, 362 vs 481 us at 64).
+// Also with several short segments: the weight-streaming kernel spreads its workgroups over the row tiles and
+// leaves each of them a fraction of the column workgroups (measured: tile kernels faster from six row tiles).
+static bool grouped_tiles(const DirectArgs& p) {
+    return p.M > 64 * (int64_t)p.E || (p.M > 2 * (int64_t)p.E && (int64_t)p.N * p.K >= ((int64_t)20 << 20)) || grouped_row_tiles(p.M, p.E, 16) >= 6;
+}
+
+extern "C" int llmk_grouped_gemm_duo_rows(int E, int64_t M, int64_t N, int64_t K) {
+    if (E <= 0 || M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+    DirectArgs p{};
+    p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = E;
+    return grouped_tiles(p) ? 32 * grouped_duo_mi(p) : 0;
+}
+
 extern "C" int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind, int c_dtype, int E, int64_t M,
                                  int64_t N, int64_t K, const int64_t* seg_indptr, const int64_t* weight_indices,
                                  const void* scale_a, const void* scale_b, int s_dtype, void* workspace,
@@ -722,13 +738,7 @@ extern "C" int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind
     p.seg_indptr = seg_indptr; p.weight_indices = weight_indices;
     p.c_dtype = c_dtype; p.s_dtype = s_dtype; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = E;
     hipStream_t st = (hipStream_t)stream;
-    // Tile kernels when the average segment is longer than 64 rows, and from two rows per expert up when the
-    // expert weights are large (measured on 8 experts of 4096 x 14336, whole forward, tile vs weight-streaming
-    // kernel: 256 vs 158 us at 1 token, 295 vs 289 us at 8, 344 vs 374 us at 16, 362 vs 481 us at 64).
-    // Also with several short segments: the weight-streaming kernel spreads its workgroups over the row tiles and
-    // leaves each of them a fraction of the column workgroups (measured: tile kernels faster from six row tiles).
-    const bool big = M > 64 * (int64_t)E || (M > 2 * (int64_t)E && N * K >= ((int64_t)20 << 20)) ||
-                     grouped_row_tiles((int)M, E, 16) >= 6;
+    const bool big = grouped_tiles(p);
     const int duo = big && scaled && (kind == LLMK_KIND_I8 || s_dtype == LLMK_F32) ? grouped_duo_mi(p) : 0;
     if (duo && kind == LLMK_KIND_FP8) return launch_grouped_duo<K_FP8_BLOCK, false>(p, duo, st, "grouped_gemm(fp8, duo)");
     if (duo && s_dtype == LLMK_F32) return launch_grouped_duo<K_I8_BLOCK, false>(p, duo, st, "grouped_gemm(i8, duo)");
@@ -750,9 +760,7 @@ extern "C" int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind
 // kernel, 0 = none (the caller runs the grouped GEMM and the activation kernel instead)
 static int swiglu_tile_rows(int kind, const DirectArgs& p) {
     if (p.N % 256 || p.K % 128 || !dma_eligible(p)) return 0;
-    const bool big = p.M > 64 * (int64_t)p.E || (p.M > 2 * (int64_t)p.E && (int64_t)p.N * p.K >= ((int64_t)20 << 20)) ||
-                     grouped_row_tiles(p.M, p.E, 16) >= 6;
-    if (!big) return 0;
+    if (!grouped_tiles(p)) return 0;
     const int choice = kind == LLMK_KIND_FP8 ? dma_tile_choice<K_FP8_BLOCK, true>(p) : dma_tile_choice<K_I8_BLOCK, true>(p);
     return choice == 8 ? 8 : (choice == 9 ? 4 : 0);
 }

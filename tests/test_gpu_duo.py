@@ -11,6 +11,7 @@ from llm_kernels_amd.fast_dequant.simple_marlin.marlin import mul
 from llm_kernels_amd.fast_dequant.simple_marlin.utils import QuantUtils
 from llm_kernels_amd.quantization import fp8_kernel, int8_kernel
 from helpers import announce, assert_close_scaled, default_dtype
+from test_gpu_moe import GROUPED_DUO
 
 FP8 = [(138, 11136, 128), (136, 11557, 256), (167, 11056, 384), (131, 10896, 640), (133, 11096, 768), (137, 11553, 896), (162, 11128, 1024), (131, 11616, 1152),
        (142, 11264, 1280), (140, 11184, 1408), (751, 216, 3072), (572, 229, 4224), (1777, 224, 4224), (194, 11816, 1024), (209, 11291, 1152), (198, 11448, 1280),
@@ -67,6 +68,19 @@ def test_scratch_of_its_slices_is_reported_and_small():
     for M, N, K in W4A8:
         z = shape_w4a8(M, N, K)[1]
         assert 4 * z * M * N * (z > 1) <= _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128)
+
+
+def test_grouped_cases_reach_every_tile():
+    """The heights of the grouped form; not where an expert's rows are two 64-row tiles that leave CUs free: those stream the weights on twice as many
+    (8 experts of 592 x 6912, 684 rows 29.7 us from HBM, 37.0 on the tall tiles)."""
+    rows = lambda E, M, N, K: _lib.load().llmk_grouped_gemm_duo_rows(E, M, N, K)
+    for height, cases in GROUPED_DUO.items():
+        assert {rows(E, n * E + max(0, 42 - n), N, K) for E, n, N, K in cases} == {height}, cases
+        assert {K // 128 % 4 for _, _, _, K in cases} == {0, 1, 2, 3}, cases
+    for E, M, N, K in ((8, 684, 592, 6912), (2, 167, 1448, 9856), (9, 809, 664, 5760), (7, 619, 1992, 7936), (3, 254, 992, 8576)):
+        assert rows(E, M, N, K) == 0, (E, M, N, K)
+    for E, M, N, K, height in ((8, 362, 4096, 14336, 64), (8, 512, 4096, 14336, 96), (8, 645, 4096, 14336, 128), (8, 860, 4096, 14336, 128), (3, 166, 304, 5760, 96)):
+        assert rows(E, M, N, K) == height, (E, M, N, K)
 
 
 def _ints(gen, dev, lo, hi, *size):

@@ -428,12 +428,18 @@ def test_grouped_gemm_many_segments_exact(dev, E, rows, N, K):
     assert torch.all(out[used:] == 5.0)
 
 
+# (experts, rows an expert, N, K) by the tile height of the two-group kernel, each with every remainder of K by its loop of four
+GROUPED_DUO = {64: [(3, 20, 272, 5120), (3, 52, 200, 5248), (3, 30, 130, 5376), (5, 44, 264, 5504)],
+               96: [(3, 54, 128, 5376), (3, 72, 264, 5504), (44, 76, 264, 5632), (4, 60, 200, 5760)],
+               128: [(44, 78, 264, 5504), (44, 84, 300, 5632), (66, 112, 136, 5760), (33, 90, 520, 5376)]}
+
+
 @pytest.mark.parametrize("kind,scales", [("fp8", torch.float32), ("int8", torch.float32), ("int8", torch.float16), ("int8", torch.bfloat16)])
 @pytest.mark.parametrize("E,rows,N,K", [(3, 20, 272, 5120), (3, 52, 200, 5248), (3, 54, 128, 5376), (3, 82, 264, 5504), (4, 84, 328, 5632), (4, 112, 136, 5760),
-                                        (70, 40, 136, 5120), (3, 20, 8800, 5248)])
+                                        (70, 40, 136, 5120), (3, 20, 8800, 5248)] + GROUPED_DUO[64][2:] + GROUPED_DUO[96][1:] + GROUPED_DUO[128])
 def test_grouped_gemm_one_tile_an_expert(dev, kind, scales, E, rows, N, K):
-    """The tile heights of the two-group kernel on both sides of their borders, every remainder of K by its loop of four, and one shape
-    beyond it (201 tiles of short segments): segments longer than a tile, of one row and empty, rows behind the last one keep their fill
+    """The tile heights of the two-group kernel on both sides of their borders, every remainder of K by its loop of four, and shapes
+    beyond it (201 tiles of short segments, few tiles of long ones): segments longer than a tile, of one row and empty, rows behind the last one keep their fill
     value, permuted weight indices, ragged columns.  Scales are powers of two and the operands small whole numbers: sums below 2^24
     quarters, exact in every order."""
     from llm_kernels_amd import _lib
