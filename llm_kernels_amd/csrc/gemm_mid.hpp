@@ -453,12 +453,13 @@ int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
     };
     // Blocks of tiles where row-major order does not deal whole columns to the XCDs already (one row of tiles: it does; per token 34 x 12816 x 4864
     // 14.2 us row-major, 15.0 so), the operands do not fit an XCD's L2 of 4 MB anyway (4-bit weights 158 x 4784 x 1152 8.4 row-major, 8.9
-    // so), and neither two tile rows of short operand rows (fp8 99 x 9232 x 1152 6.7 | 8.8 cached | from HBM, 7.1 | 9.2 so) nor a few columns in
-    // K slices (330 x 448 x 12288 13.1, 13.9 so) leave little to share.  Row-major | so: fp8 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840
+    // so), and none of these leaves little to gain: two tile rows of short operand rows (fp8 99 x 9232 x 1152 6.7 | 8.8 cached | from HBM, 7.1 | 9.2
+    // so), a few columns in K slices (330 x 448 x 12288 13.1, 13.9 so), an odd multiple of four columns, where an XCD gets every fourth one
+    // anyway, on four tile rows or more (449 x 1792 x 3072 8.0, 8.4 so; 16 shapes 0.99 times as fast).  Row-major | so: fp8 398 x 3352 x 5504 27.5 | 18.5, 384 x 2496 x 3840
     // 15.2 | 10.8, int8 145 x 5056 x 3840 14.4 | 10.6, 4-bit weights 346 x 4160 x 1920 17.7 | 16.6.  A kernel each: with the order's divisions in
     // one kernel, every short call fetched them first (fp8 148 x 3968 x 128 4.6 | 5.0 -> 4.7 | 5.3, 200 x 6144 x 2048 8.2 | 10.3 -> 8.3 | 10.8).
     const int64_t row = (int64_t)p.K * ESZ, bytes = p.N * row / (is_w4nk(KIND) ? 4 : 1) + p.M * row;
-    const bool xcds = grid.x > 8 && grid.x % 8 != 0 && grid.y > (row < 2048 ? 2 : 1) && bytes > (4 << 20);
+    const bool xcds = grid.x > 8 && grid.x % 8 != 0 && grid.y > (row < 2048 ? 2 : 1) && (grid.x % 4 != 0 || grid.y < 4) && bytes > (4 << 20);
     if (int rc = xcds ? launch(std::true_type{}) : launch(std::false_type{})) return rc;
     if (split) return launch_splitk_sum<KIND>(p, z, stream, name);
     return LLMK_OK;
