@@ -673,6 +673,16 @@ DuoPlan duo_plan(const DirectArgs& p, int64_t scratch) {
     }
     return best;
 }
+inline bool duo_beyond_a_round(const DirectArgs& p, const DuoPlan& d) {
+    return (int64_t)((p.N + DU_BN - 1) / DU_BN) * ((p.M + 32 * d.mi - 1) / (32 * d.mi)) * d.z > LLMK_CUS;
+}
+// A choice by two estimates: this kernel's has to be this much below the other one.
+constexpr double DU_MARGIN = 1.08;
+// The same in more than a round of workgroups against 256-row tiles of 4-bit weights: both estimates are 4 to 8 % off there, in opposite
+// directions (a row of these tiles a CU more or less, and every one of them expands the weights again).  Of 195 shapes 64 fell between the two margins,
+// 0.99 times as fast on this kernel (us, others | this one: fp16 976 x 10616 x 7168 161 | 176, 201 x 23784 x 9728 152 | 165, Marlin words 432 x 13056
+// x 9472 140 | 158, 1920 x 4544 x 3968 84 | 90).
+constexpr double DU_MARGIN_TALL = 1.20;
 template <int KIND, bool AS16 = false>
 int launch_duo_plan(DirectArgs p, const DuoPlan& pl, void* workspace, hipStream_t stream, const char* name) {
     if (pl.z > 1) { p.partial = (float*)workspace; p.ksplit = pl.z; }

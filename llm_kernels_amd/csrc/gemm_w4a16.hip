@@ -1006,6 +1006,9 @@ double nk_large_estimate(const llmk::DirectArgs& p, bool copy) {
     const llmk::TileChoice c = copy ? llmk::dma_tile_estimate<HALF_KIND, false>(p) : llmk::dma_tile_estimate<KIND, false>(p);
     const double e = c.cost * (double)p.K / 4096.0, nk = (double)p.N * p.K * 1e-6;
     constexpr bool BF = KIND == llmk::K_W4NKB;
+    // (few short tiles, where the passes are mostly their launches: 2 % rms to 176 shapes of up to 1024 columns.  With the estimate of the larger ones 58 of
+    // them went to the kernel of two wave groups and were 3 to 14 % slower: fp16 1240 x 72 x 640 7.6 | 8.6, 2007 x 440 x 2048 16.2 | 18.7, bf16 1027 x 208 x 1024 9.7 | 10.9)
+    if (copy && c.choice == 1) return 4.45 + 1.24 * e + 1.3 * std::min(nk, 4.0) + 0.5 * std::max(nk - 4.0, 0.0) + 0.54e-6 * (double)p.M * p.N;
     if (copy) return BF ? 6.3 + 1.37 * e + 0.44 * nk : 9.0 + 1.25 * e + 0.59 * nk;
     switch (c.choice) {
         case 1: return (BF ? 3.8 : 2.8) + (BF ? 2.08 : 2.19) * e;
@@ -1061,11 +1064,17 @@ NkPlan nk_plan_of(int64_t M, int64_t N, int64_t K, int group, int64_t scratch, b
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
     const llmk::DuoPlan d = llmk::duo_plan<KIND>(p, scratch);
     if (!d.mi) return pl;
-    double other = 1e30;                                     // (streaming kernels this far out: no scratch for a copy)
+    double other = 1e30, margin = llmk::DU_MARGIN;           // (streaming kernels this far out: no scratch for a copy)
+    const bool copy = pl.route == NkPlan::COPY, tiles = pl.route == NkPlan::TILES;
     if (pl.route == NkPlan::WAVE) other = 1.05 * pl.wave.cost;
-    else if (pl.route == NkPlan::TILES && M <= 512) other = nk_other_estimate<KIND>(p);
-    else if (pl.route == NkPlan::TILES || pl.route == NkPlan::COPY) other = nk_large_estimate<KIND, HALF_KIND>(p, pl.route == NkPlan::COPY);
-    if (1.08 * d.cost >= other) return pl;
+    else if (tiles && M <= 512) other = nk_other_estimate<KIND>(p);
+    else if (tiles || copy) other = nk_large_estimate<KIND, HALF_KIND>(p, copy);
+    if ((tiles || copy) && llmk::duo_beyond_a_round(p, d)) {
+        // (fp16 tiles that expand the words themselves: all of them; bf16 256 x 256 ones not, 25 shapes are 1.07 times as fast here)
+        const int choice = copy ? llmk::dma_tile_estimate<HALF_KIND, false>(p).choice : llmk::dma_tile_estimate<KIND, false>(p).choice;
+        if (copy ? choice == 8 : (!BF || choice == 4)) margin = llmk::DU_MARGIN_TALL;
+    }
+    if (margin * d.cost >= other) return pl;
     return {NkPlan::DUO, 1, d.z > 1 ? (int64_t)d.z * M * N * 4 : 0, {}, d};
 }
 NkPlan nk_plan(int64_t M, int64_t N, int64_t K, int group, bool bf, int64_t scratch, bool c8) {
@@ -1126,9 +1135,11 @@ llmk::DuoPlan marlin_duo(int64_t M, int64_t N, int64_t K, int group, const llmk:
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.group = group;
     llmk::DuoPlan d = llmk::duo_plan<llmk::K_W4MARLIN>(p, scratch);
     if (!d.mi) return d;
-    double other = wave.z > 0 ? 1.05 * wave.cost : marlin_tiles_estimate(M, N, K, group);
-    if (M > 512) other = 6.1 + 0.40e-6 * (double)N * K + 1.38 * llmk::dma_tile_estimate<llmk::K_F16, false>(p).cost * (double)K / 4096.0;
-    if (1.08 * d.cost >= other) d.mi = 0;
+    double other = wave.z > 0 ? 1.05 * wave.cost : marlin_tiles_estimate(M, N, K, group), margin = llmk::DU_MARGIN;
+    const llmk::TileChoice c = M > 512 ? llmk::dma_tile_estimate<llmk::K_F16, false>(p) : llmk::dma_tile_estimate<llmk::K_W4MARLIN, false>(p);
+    if (M > 512) other = 6.1 + 0.40e-6 * (double)N * K + 1.38 * c.cost * (double)K / 4096.0;
+    if ((M > 512 || wave.z <= 0) && c.choice == (M > 512 ? 8 : 4) && llmk::duo_beyond_a_round(p, d)) margin = llmk::DU_MARGIN_TALL;
+    if (margin * d.cost >= other) d.mi = 0;
     return d;
 }
 

@@ -23,12 +23,22 @@ INT8 = [(133, 11136, 640), (138, 11373, 768), (141, 11744, 896), (135, 11040, 11
 PER_TOKEN = [(524, 3632, 1536), (519, 3607, 1152), (526, 248, 3072), (1011, 375, 4224), (289, 8424, 3072), (291, 8344, 4224), (2042, 407, 6144), (386, 9363, 768),
              (452, 8391, 1152), (590, 6536, 1408)]
 W4A8 = [(538, 248, 1024), (543, 328, 1152), (581, 232, 1280), (530, 232, 1408), (545, 224, 1536), (676, 200, 1664), (541, 256, 4224), (576, 976, 4224), (194, 11280, 1024),
-        (198, 11008, 1152), (221, 10912, 1280), (195, 11544, 1408), (203, 7088, 6144), (1375, 272, 6144), (1636, 552, 4224), (79, 28672, 4096)]
+        (198, 11008, 1152), (221, 10912, 1280), (195, 11544, 1408), (203, 7088, 6144), (1375, 272, 6144), (1636, 552, 4224), (79, 28672, 4096),
+        (68, 19016, 1024), (65, 13184, 1152), (71, 14352, 1280), (68, 16264, 1408), (593, 72, 3968), (824, 112, 2304), (792, 80, 2560)]
 MARLIN = [(208, 8576, 768), (208, 8320, 640), (560, 2304, 4096), (576, 192, 1536), (528, 192, 1664), (544, 192, 2176), (800, 320, 4224), (528, 5440, 1024),
           (528, 5632, 896), (208, 6784, 4224), (1168, 576, 4224), (1424, 320, 4224), (448, 8832, 512), (400, 8576, 640), (160, 7424, 4224)]
 W4 = [(1081, 224, 128), (1465, 208, 256), (1054, 224, 384), (566, 216, 1152), (537, 240, 1280), (659, 208, 2176), (850, 280, 4224), (1849, 1552, 384), (1080, 2704, 512),
       (865, 1104, 4224), (1029, 3664, 128), (1538, 2456, 256), (1160, 3208, 384), (300, 14336, 4096), (148, 6672, 4224), (1605, 2952, 128), (979, 4728, 256),
-      (983, 4688, 384), (990, 4688, 512), (169, 6408, 6144)]
+      (983, 4688, 384), (990, 4688, 512), (169, 6408, 6144), (1802, 1072, 128), (1803, 1064, 256), (66, 17144, 384), (65, 22424, 512), (1064, 2720, 128),
+      (1155, 2464, 256), (65, 17696, 512), (684, 72, 640), (1842, 1544, 640), (1744, 1672, 768), (130, 22552, 128), (135, 22336, 256), (132, 22680, 384), (132, 22112, 512),
+      (129, 16800, 640), (322, 11008, 256), (325, 10952, 384), (324, 11256, 512)]
+# those of them that other kernels take, being faster: few short tiles (us, others | this kernel: w4a8 1718 x 160 x 1152 9.6 | 10.7, fp16 1240 x 72 x 640
+# 7.6 | 8.6), and in one of the two activation types the tiles of 16-bit or 128-column kernels
+ELSEWHERE = {"w4a8": [*W4A8[:6], (1636, 552, 4224)],
+             "fp16": [*W4[:3], (1029, 3664, 128), (1538, 2456, 256), (65, 17696, 512), (684, 72, 640), (130, 22552, 128), (135, 22336, 256), (132, 22680, 384),
+                      (132, 22112, 512), (322, 11008, 256), (325, 10952, 384), (324, 11256, 512)],
+             "bf16": [*W4[:3], (1849, 1552, 384), (1029, 3664, 128), (1538, 2456, 256), (1605, 2952, 128), (979, 4728, 256), (983, 4688, 384), (990, 4688, 512),
+                      (1064, 2720, 128), (1155, 2464, 256)]}
 
 
 def shape(entry, *args):
@@ -44,28 +54,48 @@ def shape_w4a8(M, N, K):
     return shape("llmk_gemm_w4a8_duo_shape", M, N, K, 128, _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128))
 
 
-PLANS = ((FP8, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_FP8, 0, *c)), (INT8, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_I8, 0, *c)),
-         (PER_TOKEN, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_I8, 1, *c)), (W4A8, 1, {96, 128}, shape_w4a8),
-         (MARLIN, 2, {96, 128, 160}, lambda *c: shape("llmk_gemm_w4a16_duo_shape", 1, _lib.F16, *c, 128, _lib.load().llmk_gemm_w4a16_marlin_workspace_bytes(*c))),
-         (W4, 2, {96, 128, 160, 192}, lambda *c: shape("llmk_gemm_w4a16_duo_shape", 0, _lib.F16, *c, 128, 1 << 50)))
+def shape_w4a16(marlin, dtype, group, *case):
+    scratch = _lib.load().llmk_gemm_w4a16_marlin_workspace_bytes(*case) if marlin else _lib.load().llmk_gemm_w4a16_nk_workspace_bytes(*case, group, dtype)
+    return shape("llmk_gemm_w4a16_duo_shape", marlin, dtype, *case, group, scratch)
+
+
+PLANS = (("fp8", FP8, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_FP8, 0, *c)), ("int8", INT8, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_I8, 0, *c)),
+         ("per token", PER_TOKEN, 1, {96, 128, 160}, lambda *c: shape8(_lib.KIND_I8, 1, *c)), ("w4a8", W4A8, 1, {96, 128}, shape_w4a8),
+         ("marlin", MARLIN, 2, {96, 128, 160}, lambda *c: shape_w4a16(1, _lib.F16, 128, *c)),
+         ("fp16", W4, 2, {96, 128, 160, 192}, lambda *c: shape_w4a16(0, _lib.F16, 128, *c)), ("bf16", W4, 2, {96, 128, 160, 192}, lambda *c: shape_w4a16(0, _lib.BF16, 128, *c)))
 
 
 def test_the_cases_reach_every_tile():
     """Every height, with one and with several slices, and every remainder of a slice's sub-blocks by the loop's four."""
-    for cases, size, heights, plan in PLANS:
+    for kind, cases, size, heights, plan in PLANS:
         got = {c: plan(*c) for c in cases}
-        assert None not in got.values(), got
-        assert {rows for rows, _ in got.values()} == heights and {z > 1 for _, z in got.values()} == {False, True}, got
-        assert {-(-c[2] * size // 128 // z) % 4 for c, (_, z) in got.items()} == {0, 1, 2, 3}, got
+        assert {c for c in cases if not got[c]} == set(ELSEWHERE.get(kind, ())), (kind, got)
+        got = {c: p for c, p in got.items() if p}
+        assert {rows for rows, _ in got.values()} == heights and {z > 1 for _, z in got.values()} == {False, True}, (kind, got)
+        assert {-(-c[2] * size // 128 // z) % 4 for c, (_, z) in got.items()} == {0, 1, 2, 3}, (kind, got)
+
+
+def test_calls_that_are_faster_elsewhere():
+    """Shapes that were measured slower on this kernel, and neighbours that are faster on it: short K on one row tile of int8 weights from HBM, more than a round of
+    workgroups up to 512 rows, 256-row tiles of 4-bit weights beyond a round, few short tiles of two passes."""
+    plan = {kind: p for kind, _, _, _, p in PLANS}
+    for kind, case, took in (("int8", (97, 20048, 1664), False), ("int8", (111, 18304, 1664), False), ("per token", (131, 19264, 1664), False), ("per token", (150, 17248, 1792), False),
+                             ("fp8", (130, 16472, 3072), True), ("int8", (97, 20048, 3200), True), ("per token", (159, 17248, 3200), True),
+                             ("per token", (500, 17848, 11904), False), ("fp8", (289, 23480, 2304), False), ("fp8", (129, 16472, 1920), True),
+                             ("fp16", (976, 10616, 7168), False), ("fp16", (201, 23784, 9728), False), ("bf16", (1384, 7224, 9344), False), ("marlin", (432, 13056, 9472), False),
+                             ("marlin", (1920, 4544, 3968), False), ("fp16", (300, 14336, 4096), True), ("bf16", (300, 14336, 4096), True),
+                             ("w4a8", (1718, 160, 1152), False), ("w4a8", (3723, 112, 1664), False), ("w4a8", (1024, 4096, 4096), True),
+                             ("fp16", (1240, 72, 640), False), ("fp16", (2007, 440, 2048), False), ("bf16", (1027, 208, 1024), False), ("fp16", (1086, 536, 6016), True)):
+        assert (plan[kind](*case) is not None) == took, (kind, case)
 
 
 def test_scratch_of_its_slices_is_reported_and_small():
     """What is reported holds the planes of the slices, and for the 8-bit products never more than the array that serves calls without scratch."""
-    for cases, _, _, plan in PLANS[:3]:
+    for _, cases, _, _, plan in PLANS[:3]:
         for M, N, K in cases:
             z = plan(M, N, K)[1]
             assert 4 * z * M * N * (z > 1) <= _lib.load().llmk_gemm_workspace_bytes(M, N, K) <= 32 << 20, (M, N, K)
-    for M, N, K in W4A8:
+    for M, N, K in set(W4A8) - set(ELSEWHERE["w4a8"]):
         z = shape_w4a8(M, N, K)[1]
         assert 4 * z * M * N * (z > 1) <= _lib.load().llmk_gemm_w4a8_workspace_bytes(M, N, K, 128)
 
