@@ -39,9 +39,8 @@ extern "C" {
 
 int         llmk_version(void);
 const char* llmk_last_error(void);
-/* Bytes of scratch llmk_gemm_fp8_block / _i8_block / _w4a8 / llmk_grouped_gemm can use for this shape
- * (0 = none; M = all rows of a grouped launch).  The scratch is optional: without it, or with less of it, a
- * slower kernel variant runs.  For M > 512 and K >= 8192 it ends with 64 MiB for the partial sums of a split
+/* Bytes of scratch llmk_gemm_fp8_block / _i8_block / _i8_rowcol can use for this shape, the largest of the three (0 = none).
+ * The scratch is optional: without it, or with less of it, a slower kernel variant runs.  For M > 512 and K >= 8192 it ends with 64 MiB for the partial sums of a split
  * last round of tiles (shorter K is never split there). */
 int64_t     llmk_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
@@ -142,8 +141,9 @@ int llmk_gemm_i8_block(const int8_t* a, const void* a_s, const int8_t* b, const 
  * no counterpart function in the reference).  c may be NULL; c_i32 (raw accumulators) may be NULL.
  * Up to 16 rows, and up to 512 where it is estimated to be faster, waves stream their own share of K, otherwise the MFMA tile
  * kernels run (int32 sums inside the MFMA, c = float(acc) * a_s[m] * b_s[n] in the epilogue of either path).  With a workspace of
- * llmk_gemm_workspace_bytes(M, N, K), shapes with few tiles and a long K are split along K; the slices' int32 sums
+ * llmk_gemm_i8_rowcol_workspace_bytes(M, N, K), shapes with few tiles and a long K are split along K; the slices' int32 sums
  * are added as integers before the scaling, so c and c_i32 do not depend on the split. */
+int64_t llmk_gemm_i8_rowcol_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8_t* b, const float* b_s,
                         void* c, int c_dtype, int32_t* c_i32, int64_t M, int64_t N, int64_t K,
                         void* workspace, int64_t workspace_bytes, void* stream);
@@ -322,7 +322,9 @@ int llmk_moe_expert_scales(const float* sa, const float* sb, const int64_t* seg_
 /* C[seg[e]:seg[e+1], :] = A[seg[e]:seg[e+1], :] x B[weight_indices[e]]^T  for e < E.
  * a [M,K], b [E,N,K], c [M,N]; scale_a [M,K/128], scale_b [E,ceil(N/128),K/128] for the
  * block-scaled kinds (s_dtype = dtype code of both), NULL otherwise.  workspace: optional scratch of
- * llmk_gemm_workspace_bytes(M, N, K) bytes. */
+ * llmk_grouped_gemm_workspace_bytes(kind, s_dtype, M, N, K) bytes, M being all rows: fp32 activation scales for 16-bit ones, and
+ * for M > 512 and K >= 8192 64 MiB for the partial sums of a split last round of tiles. */
+int64_t llmk_grouped_gemm_workspace_bytes(int kind, int s_dtype, int64_t M, int64_t N, int64_t K);
 int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind, int c_dtype, int E,
                       int64_t M, int64_t N, int64_t K, const int64_t* seg_indptr,
                       const int64_t* weight_indices, const void* scale_a, const void* scale_b,

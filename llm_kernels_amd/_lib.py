@@ -47,6 +47,7 @@ SIGNATURES = {
     "llmk_gemm_i8_block": [_p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _p, _l, _p],
     "llmk_gemm_i8_rowcol": [_p, _p, _p, _p, _p, _i, _p, _l, _l, _l, _p, _l, _p],
     "llmk_gemm_w4a8": [_p, _p, _p, _p, _i, _p, _p, _p, _i, _l, _l, _l, _i, _p, _l, _p],
+    "llmk_gemm_i8_rowcol_workspace_bytes": [_l, _l, _l],
     "llmk_gemm_w4a8_workspace_bytes": [_l, _l, _l, _i],
     "llmk_gemm_w4a16_marlin_workspace_bytes": [_l, _l, _l],
     "llmk_gemm_w4a16_marlin": [_p, _p, _p, _p, _l, _l, _l, _i, _p, _l, _p],
@@ -79,10 +80,12 @@ SIGNATURES = {
     "llmk_calib_mfma": [_i, _i, _p, _p, _i, _p, _p],
     "llmk_calib_read": [_p, _l, _i, _p, _i, _p],
     "llmk_calib_gemm_fp8_clock": [_p, _p, _p, _p, _p, _i, _l, _l, _l, _p, _l, _p, _p],
+    "llmk_grouped_gemm_workspace_bytes": [_i, _i, _l, _l, _l],
     "llmk_grouped_gemm_duo_rows": [_i, _l, _l, _l],
     "llmk_grouped_gemm": [_p, _p, _p, _i, _i, _i, _l, _l, _l, _p, _p, _p, _p, _i, _p, _l, _p],
 }
-_RESTYPE = {"llmk_last_error": _c.c_char_p, "llmk_gemm_workspace_bytes": _l, "llmk_gemm_w4a8_workspace_bytes": _l,
+_RESTYPE = {"llmk_last_error": _c.c_char_p, "llmk_gemm_workspace_bytes": _l, "llmk_gemm_i8_rowcol_workspace_bytes": _l,
+            "llmk_grouped_gemm_workspace_bytes": _l, "llmk_gemm_w4a8_workspace_bytes": _l,
             "llmk_gemm_w4a16_marlin_workspace_bytes": _l, "llmk_gemm_w4a16_nk_workspace_bytes": _l}
 
 _lib = None

@@ -28,6 +28,25 @@ inline int stream_k_ranges(int64_t M, int64_t N, int64_t K) {
     return (int)((K / 128 + 31) / 32);
 }
 
+// scratch of the kernels beside the one of two wave groups, without the (fixed-size) part for a split last round of 256-column tiles
+int64_t tiles_core_bytes(int64_t M, int64_t N, int64_t K) {
+    // large-M kernels stream fp32 activation scales; 16-bit scales are widened into the workspace first;
+    // mid-size M with few tiles adds the fp32 split-K partials behind them
+    if (K <= 0) return 0;
+    if (M <= 64 && !mid_m_prefers_tiles(M, N, K) && !mid_wanted(M, N, K)) {
+        const int nz = stream_k_ranges(M, N, K);
+        return nz > 1 ? (int64_t)nz * M * N * 4 : 0;
+    }
+    const int64_t scales = (M * (K / 128) * 4 + 255) & ~(int64_t)255;
+    int z = splitk_factor(M, N, K);
+    if (M <= 512) z = std::max({z, mid_plan(M, N, K).z, midw_plan(M, N, K).z});      // the mid-size kernels' K slices
+    return scales + (z > 1 ? (int64_t)z * M * N * 4 : 0);
+}
+// Is there scratch for a decode-sized call's K slices on the tile kernels?  (from 65 rows on nothing is chosen by it)
+bool slices_fit(const DirectArgs& p, const void* workspace, int64_t workspace_bytes) {
+    return p.M > 64 || (workspace && workspace_bytes >= tiles_core_bytes(p.M, p.N, p.K));
+}
+
 // What the tile kernels take for 17 to 512 rows, in us like the wave kernels' estimates (a fit of 5 to 15 % rms to 600 shapes): the
 // mid-size kernels with 64 and 128 columns, the 128-column tile in K slices, or rounds of the tiles that dma_tile_estimate chooses.
 // Up to 16 rows, and up to 64 on weights that no tile kernel fills the chip with or without scratch for their K slices, the wave
@@ -87,7 +106,7 @@ WavePlan wave_choice(const DirectArgs& p, int64_t scratch, bool tiles_scratch) {
 template <int KIND>
 WavePlan wave_choice(const DirectArgs& p, const void* workspace, int64_t workspace_bytes) {
     return wave_choice<KIND>(p, workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0,
-                             workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K));
+                             slices_fit(p, workspace, workspace_bytes));
 }
 // What the tile kernels take beyond 512 rows, in us: rounds of the tiles that dma_tile_estimate chooses (a fit of 3 to 5 % rms for the 128-column
 // ones, 7 to 10 % for the 256-column ones, to 80 to 140 shapes a kind).
@@ -125,7 +144,7 @@ DuoPlan duo_choice(const DirectArgs& p, const WavePlan& w, int64_t scratch, bool
 template <int KIND>
 DuoPlan duo_choice(const DirectArgs& p, const WavePlan& w, void* workspace, int64_t workspace_bytes) {
     return duo_choice<KIND>(p, w, workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0,
-                            workspace && workspace_bytes >= llmk_gemm_workspace_bytes(p.M, p.N, p.K), wide_tail_ok<KIND>(p, workspace, workspace_bytes));
+                            slices_fit(p, workspace, workspace_bytes), wide_tail_ok<KIND>(p, workspace, workspace_bytes));
 }
 template <int KIND>
 int launch_block(const DirectArgs& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, const char* name) {
@@ -144,52 +163,44 @@ int launch_block(const DirectArgs& p, void* workspace, int64_t workspace_bytes, 
 
 }  // namespace
 
-// scratch without the (fixed-size) part for a split last round of 256-column tiles
-static int64_t tiles_core_bytes(int64_t M, int64_t N, int64_t K) {
-    // large-M kernels stream fp32 activation scales; 16-bit scales are widened into the workspace first;
-    // mid-size M with few tiles adds the fp32 split-K partials behind them
-    if (K <= 0) return 0;
-    if (M <= 64 && !mid_m_prefers_tiles(M, N, K) && !mid_wanted(M, N, K)) {
-        const int nz = stream_k_ranges(M, N, K);
-        return nz > 1 ? (int64_t)nz * M * N * 4 : 0;
-    }
-    const int64_t scales = (M * (K / 128) * 4 + 255) & ~(int64_t)255;
-    int z = splitk_factor(M, N, K);
-    if (M <= 512) z = std::max({z, mid_plan(M, N, K).z, midw_plan(M, N, K).z});      // the mid-size kernels' K slices
-    return scales + (z > 1 ? (int64_t)z * M * N * 4 : 0);
-}
-
-// the same with the planes of the kernel of two wave groups, where a kind takes it in K slices
+// planes of the kernel of two wave groups, where a kind takes it in K slices
 template <int KIND>
 static int64_t duo_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 64 || N <= 0 || K < 12 * 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     DirectArgs p{};
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.s_dtype = LLMK_F32;
     const WavePlan w = wave_choice<KIND>(p, INT64_MAX, true);
     const DuoPlan d = duo_choice<KIND>(p, w, INT64_MAX, true, KIND != K_I8_ROWCOL && M > 512 && K >= W_TAIL_MIN_KT * 128);
     return d.mi && d.z > 1 ? (int64_t)d.z * M * N * 4 : 0;
 }
+// (the plans of the three kinds take 0.2 us)
 static int64_t workspace_core_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 64 || N <= 0 || K < 12 * 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return tiles_core_bytes(M, N, K);
-    // a call asks twice or three times and the plans of three kinds take a microsecond: a thread remembers its last shapes
-    struct Shape { int64_t M, N, K, bytes; };
-    static thread_local Shape seen[16] = {};
-    Shape& s = seen[(uint64_t)(M * 0x9E3779B97F4A7C15ull + N * 0xC2B2AE3D27D4EB4Full + K) >> 60];
-    if (s.M != M || s.N != N || s.K != K)
-        s = {M, N, K, std::max({tiles_core_bytes(M, N, K), duo_bytes<K_FP8_BLOCK>(M, N, K), duo_bytes<K_I8_BLOCK>(M, N, K), duo_bytes<K_I8_ROWCOL>(M, N, K)})};
-    return s.bytes;
+    return std::max({tiles_core_bytes(M, N, K), duo_bytes<K_FP8_BLOCK>(M, N, K), duo_bytes<K_I8_BLOCK>(M, N, K), duo_bytes<K_I8_ROWCOL>(M, N, K)});
 }
+static int64_t tail_bytes(int64_t M, int64_t K) { return K >= W_TAIL_MIN_KT * 128 && M > 512 ? w_tail_bytes() : 0; }
 
 extern "C" int64_t llmk_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     // more than 512 rows and at least W_TAIL_MIN_KT K steps of 128 bytes (shorter tiles are never split): room for
     // the partial sums of a split last round of 256-column tiles behind the rest
-    return workspace_core_bytes(M, N, K) + (K >= W_TAIL_MIN_KT * 128 && M > 512 ? w_tail_bytes() : 0);
+    return workspace_core_bytes(M, N, K) + tail_bytes(M, K);
+}
+
+// Per-token products slice K up to 512 rows, and beyond on the kernel of two wave groups only; they widen no scales there and split no last round.
+extern "C" int64_t llmk_gemm_i8_rowcol_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    return std::max(M <= 512 ? tiles_core_bytes(M, N, K) : 0, duo_bytes<K_I8_ROWCOL>(M, N, K));
+}
+
+// Grouped products slice no K: fp32 activation scales where the caller's are 16-bit, and the split last round.
+extern "C" int64_t llmk_grouped_gemm_workspace_bytes(int kind, int s_dtype, int64_t M, int64_t N, int64_t K) {
+    if ((kind != LLMK_KIND_I8 && kind != LLMK_KIND_FP8) || M <= 0 || N <= 0 || K <= 0) return 0;
+    return (s_dtype == LLMK_F32 ? 0 : (M * (K / 128) * 4 + 255) & ~(int64_t)255) + tail_bytes(M, K);
 }
 
 extern "C" int llmk_gemm_8bit_wave_shape(int kind, int per_token, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes, int32_t* shape) {
     if (!shape || M <= 0 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     DirectArgs p{};
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1;
-    const bool full = scratch_bytes > 0 && scratch_bytes >= llmk_gemm_workspace_bytes(M, N, K);
+    const bool full = M > 64 || (scratch_bytes > 0 && scratch_bytes >= tiles_core_bytes(M, N, K));
     const WavePlan w = kind == LLMK_KIND_FP8 ? wave_choice<K_FP8_BLOCK>(p, scratch_bytes, full)
                                              : (per_token ? wave_choice<K_I8_ROWCOL>(p, scratch_bytes, full) : wave_choice<K_I8_BLOCK>(p, scratch_bytes, full));
     int32_t duo[2];
@@ -201,10 +212,10 @@ extern "C" int llmk_gemm_8bit_duo_shape(int kind, int per_token, int64_t M, int6
     if (!shape || M <= 64 || N <= 0 || K <= 0 || K % 128 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     DirectArgs p{};
     p.M = (int)M; p.N = (int)N; p.K = (int)K; p.E = 1; p.s_dtype = LLMK_F32;
-    const bool full = scratch_bytes > 0 && scratch_bytes >= llmk_gemm_workspace_bytes(M, N, K);
+    const bool tail = M > 512 && K >= W_TAIL_MIN_KT * 128 && scratch_bytes >= w_tail_bytes();
     auto plan = [&](auto kind_c) {
         constexpr int KIND = decltype(kind_c)::value;
-        return duo_choice<KIND>(p, wave_choice<KIND>(p, scratch_bytes, full), scratch_bytes, full, KIND != K_I8_ROWCOL && full && M > 512 && K >= W_TAIL_MIN_KT * 128);
+        return duo_choice<KIND>(p, wave_choice<KIND>(p, scratch_bytes, true), scratch_bytes, true, KIND != K_I8_ROWCOL && tail);
     };
     const DuoPlan d = kind == LLMK_KIND_FP8 ? plan(std::integral_constant<int, K_FP8_BLOCK>{})
                                             : (per_token ? plan(std::integral_constant<int, K_I8_ROWCOL>{}) : plan(std::integral_constant<int, K_I8_BLOCK>{}));
@@ -274,7 +285,7 @@ extern "C" int llmk_gemm_i8_rowcol(const int8_t* a, const float* a_s, const int8
     }
     if (wave.nw) return launch_w8_wave_plan<K_I8_ROWCOL>(p, wave, workspace, (hipStream_t)stream, "gemm_i8_rowcol(wave)");
     // large M: the tile kernels accumulate int32 over the whole K range inside the MFMA and scale in the epilogue
-    if ((M > 64 || ((mid_wanted(M, N, K) || mid_m_prefers_tiles(M, N, K)) && workspace && workspace_bytes >= llmk_gemm_workspace_bytes(M, N, K))) &&
+    if ((M > 64 || ((mid_wanted(M, N, K) || mid_m_prefers_tiles(M, N, K)) && slices_fit(p, workspace, workspace_bytes))) &&
         dma_eligible(p)) {
         // few tiles and a long K: K slices over the CUs, int32 partial sums in the workspace, one pass that adds
         // them as integers and scales (same bits as the unsplit kernel)

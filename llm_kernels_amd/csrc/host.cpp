@@ -28,6 +28,7 @@ namespace {
 #define LLMK_HOST_API(X)                                                                                              \
     X(llmk_last_error) X(llmk_gemm_workspace_bytes) X(llmk_act_quant_fp8) X(llmk_act_quant_i8) X(llmk_comm_quant_fp8) \
     X(llmk_quant_i8_rowwise) X(llmk_gemm_fp8_block) X(llmk_gemm_i8_block) X(llmk_gemm_i8_rowcol) X(llmk_gemm_w4a8)    \
+    X(llmk_gemm_i8_rowcol_workspace_bytes) X(llmk_grouped_gemm_workspace_bytes)                                       \
     X(llmk_gemm_w4a8_workspace_bytes) X(llmk_gemm_w4a16_marlin) X(llmk_gemm_w4a16_marlin_workspace_bytes)             \
     X(llmk_gemm_w4a16_nk) X(llmk_gemm_w4a16_nk_workspace_bytes) X(llmk_moe_ep_preprocess)                             \
     X(llmk_moe_pre_reorder_quant) X(llmk_moe_act_and_mul_quant) X(llmk_moe_post_reorder) X(llmk_grouped_gemm)         \
@@ -403,8 +404,7 @@ PyObject* int8_gemm_per_token(const Args& g) {
     require(a_s_in.numel() == M && b_s_in.numel() == N, "need one scale per token and per output channel");
     const at::ScalarType out = default_dtype();
     const bool want_acc = g.integer(4) != 0;
-    // (the scratch of K slices; not that of a split last round of tiles, which K from 8192 on has beyond 512 rows and this kind does not use)
-    Scratch ws(g, a, M <= 512 || K < 8192 ? g.st->llmk_gemm_workspace_bytes(M, N, K) : 0);
+    Scratch ws(g, a, g.st->llmk_gemm_i8_rowcol_workspace_bytes(M, N, K));
     at::Tensor c, acc;
     unlocked([&] {
         const at::Tensor a_s = as_type(a_s_in, at::kFloat).contiguous(), b_s = as_type(b_s_in, at::kFloat).contiguous();
@@ -612,7 +612,7 @@ PyObject* grouped_gemm(const Args& g) {
     const int64_t E = g.integer(3), M = a.size(0), N = b.size(1), K = b.size(2);
     const at::Tensor& seg_in = g.tensor(4);
     const at::Tensor wi_in = optional(g, 5), sa = scaled ? g.tensor(6) : at::Tensor(), sb_in = scaled ? g.tensor(7) : at::Tensor();
-    Scratch ws(g, a, g.st->llmk_gemm_workspace_bytes(M, N, K));
+    Scratch ws(g, a, g.st->llmk_grouped_gemm_workspace_bytes(kind, scaled ? float_code(sa.scalar_type()) : 0, M, N, K));
     unlocked([&] {
         const at::Tensor seg = long_contiguous(seg_in), wi = long_contiguous(wi_in);
         const at::Tensor sb = scaled ? as_type(sb_in, sa.scalar_type()).contiguous() : sb_in;

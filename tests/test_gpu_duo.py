@@ -1,6 +1,7 @@
 """The tile kernel whose two wave groups take turns (gemm_duo.hpp), on every tile height that is built: numbers of 128-byte sub-blocks around its
 loop of four and below it, one to six K slices, ragged rows and columns."""
 import ctypes
+import random
 
 import pytest
 import torch
@@ -9,6 +10,7 @@ from llm_kernels_amd import _lib
 from llm_kernels_amd.fast_dequant import w4a16
 from llm_kernels_amd.fast_dequant.simple_marlin.marlin import mul
 from llm_kernels_amd.fast_dequant.simple_marlin.utils import QuantUtils
+from llm_kernels_amd.moe.group_gemm_kernel import grouped_gemm_triton
 from llm_kernels_amd.quantization import fp8_kernel, int8_kernel
 from helpers import announce, assert_close_scaled, default_dtype
 from test_gpu_moe import GROUPED_DUO
@@ -22,6 +24,7 @@ INT8 = [(133, 11136, 640), (138, 11373, 768), (141, 11744, 896), (135, 11040, 11
         (145, 8197, 7680), (1210, 4090, 4096)]
 PER_TOKEN = [(524, 3632, 1536), (519, 3607, 1152), (526, 248, 3072), (1011, 375, 4224), (289, 8424, 3072), (291, 8344, 4224), (2042, 407, 6144), (386, 9363, 768),
              (452, 8391, 1152), (590, 6536, 1408)]
+PER_TOKEN_LONG = [(705, 1112, 10240), (887, 1856, 10752), (1260, 1904, 13696), (1099, 1528, 10496)]       # K slices beyond 512 rows and K = 8192
 W4A8 = [(538, 248, 1024), (543, 328, 1152), (581, 232, 1280), (530, 232, 1408), (545, 224, 1536), (676, 200, 1664), (541, 256, 4224), (576, 976, 4224), (194, 11280, 1024),
         (198, 11008, 1152), (221, 10912, 1280), (195, 11544, 1408), (203, 7088, 6144), (1375, 272, 6144), (1636, 552, 4224), (79, 28672, 4096),
         (68, 19016, 1024), (65, 13184, 1152), (71, 14352, 1280), (68, 16264, 1408), (593, 72, 3968), (824, 112, 2304), (792, 80, 2560)]
@@ -113,6 +116,50 @@ def test_grouped_cases_reach_every_tile():
         assert rows(E, M, N, K) == height, (E, M, N, K)
 
 
+def test_per_token_scratch():
+    """What is reported for a per-token product beyond 512 rows is what its K slices take, without the 64 MiB of a split last round, and the plan it gives
+    is the one that any amount gives."""
+    lib, rng = _lib.load(), random.Random(3)
+    slices = 0
+    for M, N, K in PER_TOKEN_LONG + [(rng.randint(513, 4096), rng.randint(64, 28672), 128 * rng.randint(1, 112)) for _ in range(3000)]:
+        got = lib.llmk_gemm_i8_rowcol_workspace_bytes(M, N, K)
+        plan = shape("llmk_gemm_8bit_duo_shape", _lib.KIND_I8, 1, M, N, K, got)
+        assert plan == shape("llmk_gemm_8bit_duo_shape", _lib.KIND_I8, 1, M, N, K, 1 << 40), (M, N, K)
+        assert got == (4 * plan[1] * M * N if plan and plan[1] > 1 else 0) <= lib.llmk_gemm_workspace_bytes(M, N, K), (M, N, K)
+        slices += got > 0 and K >= 8192
+    assert slices > 20
+    for M, N, K in ((16, 4096, 14336), (64, 4096, 4096), (300, 4096, 14336), (512, 1112, 10240)):
+        assert 0 < lib.llmk_gemm_i8_rowcol_workspace_bytes(M, N, K) <= lib.llmk_gemm_workspace_bytes(M, N, K), (M, N, K)
+
+
+def test_grouped_scratch():
+    """Scales that have to be widened and, from 513 rows and K = 8192, a split last round: nothing else."""
+    need = _lib.load().llmk_grouped_gemm_workspace_bytes
+    for kind in (_lib.KIND_I8, _lib.KIND_FP8):
+        assert need(kind, _lib.F32, 4000, 4096, 8064) == need(kind, _lib.F32, 512, 4096, 14336) == 0
+        assert need(kind, _lib.F16, 4000, 4096, 4096) == need(kind, _lib.BF16, 4000, 4096, 4096) == 4000 * 32 * 4
+        assert need(kind, _lib.F32, 513, 4096, 8192) == 64 << 20 and need(kind, _lib.F16, 640, 4096, 8192) == (64 << 20) + 640 * 64 * 4
+    assert need(_lib.KIND_F16, 0, 4000, 4096, 14336) == need(_lib.KIND_BF16, 0, 4000, 4096, 14336) == 0
+
+
+@pytest.mark.gpu
+def test_public_functions_reserve_what_they_use(dev):
+    """The scratch that is kept after a call: the planes of a per-token product's slices, nothing for a grouped one that needs none."""
+    announce("scratch of the public functions")
+    M, N, K = 887, 1856, 10752
+    _lib.release_workspaces()
+    int8_kernel.int8_gemm_per_token(torch.zeros(M, K, dtype=torch.int8, device=dev), torch.ones(M, device=dev), torch.zeros(N, K, dtype=torch.int8, device=dev),
+                                    torch.ones(N, device=dev))
+    rows, z = shape("llmk_gemm_8bit_duo_shape", _lib.KIND_I8, 1, M, N, K, 1 << 40)
+    assert z > 1 and [4 * z * M * N <= t.numel() < 64 << 20 for t in _lib._ws.values()] == [True]
+    _lib.release_workspaces()
+    E, M, N, K = 4, 900, 512, 1024
+    grouped_gemm_triton(torch.zeros(M, K, dtype=torch.int8, device=dev), torch.zeros(E, N, K, dtype=torch.int8, device=dev), torch.empty(M, N, dtype=torch.bfloat16, device=dev),
+                        E, True, torch.tensor([0, 200, 450, 700, M], device=dev), torch.arange(E, device=dev), False, torch.ones(M, K // 128, device=dev),
+                        torch.ones(E, N // 128, K // 128, device=dev), [128, 128])
+    assert not _lib._ws
+
+
 def _ints(gen, dev, lo, hi, *size):
     return torch.randint(lo, hi + 1, size, device=dev, generator=gen)
 
@@ -149,7 +196,7 @@ def test_block_scales_exact(dev, kind, M, N, K, scales):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", PER_TOKEN)
+@pytest.mark.parametrize("M,N,K", PER_TOKEN + PER_TOKEN_LONG)
 def test_per_token_exact(dev, M, N, K):
     announce("duo per token", M, N, K)
     gen = torch.Generator(device=dev).manual_seed(M + K)
