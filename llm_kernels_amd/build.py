@@ -72,14 +72,15 @@ def _assembly(src):
 
 
 # what tells that a source hand-issues loads into registers: the loaders themselves, the header of the ring
-# kernels, or a tile-kernel kind whose weight rows are expanded from hand-loaded packed words
+# kernels, a tile-kernel kind whose weight rows are expanded from hand-loaded packed words, or the mid-size kernels,
+# whose producers load all weight rows so
 _ASM_LOAD_MARKS = ('asm volatile("global_load_dword', "ring_load_", "asm_load_", "stream_ring.hpp",
-                   "K_W4NK", "K_W4MARLIN")
+                   "K_W4NK", "K_W4MARLIN", "K_W4A8", "launch_mid<")
 
 
 def _has_asm_register_loads(src):
     """True when this source itself names hand-issued register loads (directly, by including the ring header, or
-    by instantiating a tile-kernel kind that uses them): its assembly must then show at least one."""
+    by instantiating tile kernels that use them): its assembly must then show at least one."""
     text = open(src).read()
     return any(m in text for m in _ASM_LOAD_MARKS)
 
@@ -91,8 +92,8 @@ def build(jobs=None, verbose=True):
     jobs = jobs or min(8, len(srcs))
     # Kernels that load registers from inline asm are only correct while the compiler never touches the
     # destination before the hand-placed wait: prove it on the assembly of this very build, or fail.  EVERY
-    # source is checked (a source without such loads has nothing to flag); a source whose text, or a header it
-    # includes, contains hand-issued loads must show at least one in its assembly, otherwise the check has gone blind.
+    # source is checked (a source without such loads has nothing to flag); a source whose text names kernels that
+    # hand-issue loads must show at least one in its assembly, otherwise the check has gone blind.
     with cf.ThreadPoolExecutor(jobs) as ex:
         host_job = ex.submit(_host_module)
         asm_jobs = [(s, ex.submit(_assembly, s)) for s in srcs]

@@ -4,7 +4,7 @@ states after a VALU write, one after a write to M0).  Synthetic listings: the ac
 they can go wrong."""
 import os
 
-from llm_kernels_amd import check_asm
+from llm_kernels_amd import build, check_asm
 
 HEAD = "kern:\n"
 LOAD = "\t;;#ASMSTART\n\tglobal_load_dwordx2 v[10:11], v20, s[2:3]\n\t;;#ASMEND\n"
@@ -100,3 +100,10 @@ def test_rejects_lds_load_right_after_the_write_to_m0(tmp_path):
     body = "\t;;#ASMSTART\n\ts_mov_b32 m0, s5\n\tglobal_load_lds_dwordx4 v21, s[6:7]\n\t;;#ASMEND\n" + WAIT
     _, bad = _check(tmp_path, body)
     assert len(bad) == 1 and "M0" in bad[0]
+
+
+def test_sources_that_have_to_show_hand_issued_loads():
+    """The mid-size kernels' producers (8-bit products), packed 4-bit words with 16-bit and with 8-bit activations: were the check to see none of their loads,
+    the build has to fail."""
+    expected = {f for f in os.listdir(build.CSRC) if f.endswith(".hip") and build._has_asm_register_loads(os.path.join(build.CSRC, f))}
+    assert expected == {"gemm_block.hip", "gemm_w4a16.hip", "gemm_w4a8.hip"}
