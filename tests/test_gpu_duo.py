@@ -11,7 +11,7 @@ from llm_kernels_amd.fast_dequant import w4a16
 from llm_kernels_amd.fast_dequant.simple_marlin.marlin import mul
 from llm_kernels_amd.fast_dequant.simple_marlin.utils import QuantUtils
 from llm_kernels_amd.moe.group_gemm_kernel import grouped_gemm_triton
-from llm_kernels_amd.quantization import fp8_kernel, int8_kernel
+from llm_kernels_amd.quantization import fp8_kernel, int8_kernel, w4a8_kernel
 from helpers import announce, assert_close_scaled, default_dtype
 from test_gpu_moe import GROUPED_DUO
 
@@ -35,6 +35,9 @@ W4 = [(1081, 224, 128), (1465, 208, 256), (1054, 224, 384), (566, 216, 1152), (5
       (983, 4688, 384), (990, 4688, 512), (169, 6408, 6144), (1802, 1072, 128), (1803, 1064, 256), (66, 17144, 384), (65, 22424, 512), (1064, 2720, 128),
       (1155, 2464, 256), (65, 17696, 512), (684, 72, 640), (1842, 1544, 640), (1744, 1672, 768), (130, 22552, 128), (135, 22336, 256), (132, 22680, 384), (132, 22112, 512),
       (129, 16800, 640), (322, 11008, 256), (325, 10952, 384), (324, 11256, 512)]
+# (M, N, K, group) beside groups of 128: half of one to a whole row, K slices that start inside a group, and tiles of 96 to 192 rows
+W4_GROUPS = [(66, 8328, 1024, 64), (68, 80, 6144, 64), (620, 888, 1536, 256), (621, 64, 2048, 256), (535, 64, 1536, 256), (678, 1296, 2048, 1024), (965, 400, 4096, 1024),
+             (621, 64, 2048, 1024), (69, 20440, 1024, 1024), (621, 64, 2048, 2048), (169, 6408, 6144, 64), (169, 6408, 6144, 1024), (300, 14336, 4096, 4096)]
 # those of them that other kernels take, being faster: few short tiles (us, others | this kernel: w4a8 1718 x 160 x 1152 9.6 | 10.7, fp16 1240 x 72 x 640
 # 7.6 | 8.6), and in one of the two activation types the tiles of 16-bit or 128-column kernels
 ELSEWHERE = {"w4a8": [*W4A8[:6], (1636, 552, 4224)],
@@ -76,6 +79,13 @@ def test_the_cases_reach_every_tile():
         got = {c: p for c, p in got.items() if p}
         assert {rows for rows, _ in got.values()} == heights and {z > 1 for _, z in got.values()} == {False, True}, (kind, got)
         assert {-(-c[2] * size // 128 // z) % 4 for c, (_, z) in got.items()} == {0, 1, 2, 3}, (kind, got)
+
+
+def test_the_groups_reach_the_kernel():
+    plans = {(*c, dt): shape_w4a16(0, dt, c[3], *c[:3]) for c in W4_GROUPS for dt in (_lib.F16, _lib.BF16)}
+    assert None not in plans.values() and {p[0] for p in plans.values()} == {96, 160, 192}, plans
+    inside = {g for (M, N, K, g, _), (_, z) in plans.items() if z > 1 and -(-(K // 64) // z) * 64 % g}
+    assert inside == {256, 1024, 2048} and {g for (M, N, K, g, _), (_, z) in plans.items() if z == 1} == {64, 256, 1024, 4096}, plans
 
 
 def test_calls_that_are_faster_elsewhere():
@@ -261,6 +271,107 @@ def test_row_packed_weights(dev, M, N, K, dtype):
     x = torch.randn(M, K, device=dev, generator=gen, dtype=torch.float32).to(dtype)
     ref = x.double() @ weights.double().t()
     assert_close_scaled(w4a16.w4a16_gemm(x, packed, scales, 128), ref, rtol=2 ** -8 if dtype == torch.bfloat16 else 2 ** -11, atol=2e-5)
+
+
+def _packed_rows(codes):
+    """[N, K] codes -> [N, K/8] words, element i of a word in bits 4 i .. 4 i + 3."""
+    words = torch.zeros(codes.shape[0], codes.shape[1] // 8, dtype=torch.int64, device=codes.device)
+    for i in range(8):
+        words |= codes[:, i::8].long() << (4 * i)
+    return torch.where(words >= 1 << 31, words - (1 << 32), words).int()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,group", W4_GROUPS)
+def test_row_packed_groups(dev, M, N, K, group, dtype):
+    """Every group has a scale of its own: one element of a row gives a column of the rounded weights, to the bit, over all of K."""
+    announce("duo w4 groups", dtype, M, N, K, group)
+    gen = torch.Generator(device=dev).manual_seed(M + K + group)
+    codes, scales = _ints(gen, dev, 0, 15, N, K), (torch.rand(N, K // group, device=dev, generator=gen, dtype=torch.float32) * 0.02 + 0.001).half()
+    weights = ((codes.float() - 8) * scales.float().repeat_interleave(group, 1)).to(dtype)
+    packed = _packed_rows(codes)
+    k = (max(7, K // M | 1) * torch.arange(M, device=dev) + 3) % K
+    x = torch.zeros(M, K, dtype=dtype, device=dev)
+    x[torch.arange(M, device=dev), k] = 1
+    assert torch.equal(w4a16.w4a16_gemm(x, packed, scales, group), weights[:, k].t())
+    x = torch.randn(M, K, device=dev, generator=gen, dtype=torch.float32).to(dtype)
+    assert_close_scaled(w4a16.w4a16_gemm(x, packed, scales, group), x.double() @ weights.double().t(), rtol=2 ** -8 if dtype == torch.bfloat16 else 2 ** -11, atol=2e-5)
+
+
+NAN, INF = float("nan"), float("inf")
+
+
+def _only_their_rows(call, clean, dirty, rows, ref):
+    """Rows with values that are no numbers: what `ref` says is NaN or infinite is, and the other rows are what they are without them."""
+    before, after = call(clean), call(dirty)
+    others = torch.ones(before.shape[0], dtype=torch.bool, device=before.device)
+    others[list(rows)] = False
+    assert bool(before.isfinite().all()) and torch.equal(before[others], after[others])
+    got, want = after[list(rows)].cpu().double(), ref.cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and not bool(want.isfinite().all(1).any())
+    for inf in (INF, -INF):
+        assert torch.equal(got == inf, want == inf)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,M,N,K", [("fp8", 751, 216, 3072), ("fp8", 131, 11616, 1152), ("fp8", 198, 11448, 1280), ("fp8", 129, 16472, 1920), ("int8", 667, 216, 3072),
+                                        ("int8", 137, 11968, 1408), ("int8", 197, 11248, 3072), ("int8", 147, 21854, 1280), ("w4a8", 541, 256, 4224), ("w4a8", 203, 7088, 6144)])
+def test_scales_that_are_no_numbers(dev, kind, M, N, K):
+    """NaN and infinities among the activation scales (and, for fp8, the activations), in the first and the last K step: in their rows and nowhere else."""
+    announce("duo non-finite", kind, M, N, K)
+    assert {k: p for k, _, _, _, p in PLANS}[kind](M, N, K)
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    kb = K // 128
+    a, b = _ints(gen, dev, -3, 3, M, K), _ints(gen, dev, -3, 3, N, K)
+    scales = torch.float32 if kind == "fp8" else torch.float16
+    a_s, b_s = (2.0 ** _ints(gen, dev, 0, 3, M, kb)).to(scales), (2.0 ** _ints(gen, dev, 0, 3, -(-N // 128), kb)).to(scales)
+    a8 = a.float().to(torch.float8_e4m3fn) if kind == "fp8" else a.to(torch.int8)
+    bad_a, bad_s = a8.clone(), a_s.clone()
+    rows = [0, 17, 64, M - 1]
+    bad_s[0, 0], bad_s[17, kb - 1], bad_s[64, kb // 2], bad_s[M - 1, kb - 1] = INF, -INF, NAN, INF
+    if kind == "fp8":
+        rows.append(40)
+        bad_a[40, K - 1] = NAN
+    ref = sum((bad_a[rows, 128 * i:128 * i + 128].float().double() @ b[:, 128 * i:128 * i + 128].double().t()) *
+              (bad_s[rows, i:i + 1].double() * b_s[:, i].double().repeat_interleave(128)[:N]) for i in range(kb))
+    if kind == "w4a8":
+        one = torch.ones(N, kb, dtype=torch.int8, device=dev)
+        words = _packed_rows((b + 8).t().contiguous()).t().contiguous()
+        call = lambda v: w4a8_kernel.w4a8_gemm(*v, words, b_s, one, 8 * one, 128, 8, "row")
+    else:
+        b8 = b.float().to(torch.float8_e4m3fn) if kind == "fp8" else b.to(torch.int8)
+        call = lambda v: (fp8_kernel.fp8_gemm if kind == "fp8" else int8_kernel.int8_gemm)(*v, b8, b_s)
+    with default_dtype(torch.float32):
+        _only_their_rows(call, (a8, a_s), (bad_a, bad_s), rows, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,M,N,K", [("fp16", 659, 208, 2176), ("fp16", 865, 1104, 4224), ("fp16", 1605, 2952, 128), ("bf16", 659, 208, 2176), ("bf16", 300, 14336, 4096),
+                                        ("bf16", 169, 6408, 6144), ("marlin", 576, 192, 1536), ("marlin", 528, 5632, 896), ("marlin", 400, 8576, 640)])
+def test_activations_that_are_no_numbers(dev, kind, M, N, K):
+    """The same for 16-bit activations: infinities times the weights' signs, times a zero weight NaN."""
+    announce("duo non-finite", kind, M, N, K)
+    assert {k: p for k, _, _, _, p in PLANS}[kind](M, N, K)
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float16
+    x = torch.randn(M, K, device=dev, generator=gen, dtype=torch.float32).to(dtype)
+    bad, rows = x.clone(), [0, 17, 64, M - 1]
+    bad[0, 0], bad[17, K - 1], bad[64, K // 2], bad[M - 1, K - 1] = INF, -INF, NAN, INF
+    if kind == "marlin":
+        _, q, s = QuantUtils.fake_quantize((torch.randn(K, N, device=dev, generator=gen, dtype=torch.float32) * 0.02).half(), 128)
+        weights = ((q.double() - 8) * s.double().repeat_interleave(128, 0)).t()
+        words, s = QuantUtils.pack(q, s, 128)
+
+        def call(v):
+            out = torch.empty(M, N, dtype=dtype, device=dev)
+            mul(v, words, out, s, torch.zeros(max(16, N // 128 * 16), dtype=torch.int32, device=dev))
+            return out
+    else:
+        codes, scales = _ints(gen, dev, 0, 15, N, K), (torch.rand(N, K // 128, device=dev, generator=gen, dtype=torch.float32) * 0.01 + 0.001).half()
+        weights, words = (codes.double() - 8) * scales.double().repeat_interleave(128, 1), _packed_rows(codes)
+        call = lambda v: w4a16.w4a16_gemm(v, words, scales, 128)
+    _only_their_rows(call, x, bad, rows, bad[rows].cpu().double() @ weights.cpu().t())
 
 
 @pytest.mark.gpu

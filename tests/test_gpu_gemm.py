@@ -513,8 +513,16 @@ def test_mid_and_small_tile_kernels_exact_integers(dev, M, N, K):
         assert torch.equal(acc.cpu().long(), ref), "int8 per token"
 
 
-@pytest.mark.parametrize("M,N,K", [(398, 3352, 5504), (384, 2496, 3840), (145, 5056, 3840), (237, 3384, 7808), (223, 1872, 11392), (70, 12353, 1280),
-                                   (506, 3133, 3328), (97, 5504, 10368), (33, 8321, 2048), (120, 11331, 4224), (200, 9473, 2176)])
+# shapes that the mid-size kernels run in blocks of tiles an XCD, by the kinds that take them there: two to eight tile rows, both tile heights, 64 and 128
+# columns, K slices
+MID_BLOCKS = {("fp8", "int8", "per token"): [(97, 5560, 2176), (131, 3312, 1280), (197, 3104, 1280), (270, 3080, 1280), (130, 3904, 1152), (70, 12353, 1280), (506, 3133, 3328)],
+              ("fp8", "int8"): [(398, 3352, 5504), (384, 2496, 3840), (145, 5056, 3840), (237, 3384, 7808)],
+              ("fp8",): [(65, 8336, 2176), (130, 6616, 640), (261, 3384, 1152), (131, 1048, 12800), (236, 14024, 2176), (259, 10712, 384), (391, 6224, 640), (120, 11331, 4224)],
+              ("fp16", "bf16"): [(33, 5360, 1536), (33, 2608, 3072), (68, 7016, 1152), (149, 4400, 2176), (261, 2824, 2176), (65, 13504, 1152), (163, 6632, 1152), (202, 11040, 1152),
+                                 (389, 6696, 1152), (33, 8321, 2048)]}
+
+
+@pytest.mark.parametrize("M,N,K", [(223, 1872, 11392), (97, 5504, 10368), (200, 9473, 2176)] + [c for cases in MID_BLOCKS.values() for c in cases])
 def test_mid_size_tiles_in_the_order_of_the_xcds(dev, M, N, K):
     """Column tiles that are no multiple of eight and operands beyond 4 MB: the tiles are dealt to the XCDs in blocks, with one to eight tile rows,
     a ragged last one and K slices.  Small integers: every partial sum is exact, also with fp16 and bf16 activations on 4-bit weights."""
@@ -541,8 +549,10 @@ def test_mid_size_tiles_in_the_order_of_the_xcds(dev, M, N, K):
         assert bool(((y - ref).abs() <= half * ref.abs()).all()), dt
 
 
-@pytest.mark.parametrize("M,N,K", [(130, 9000, 640), (300, 5000, 1152), (500, 3208, 384), (100, 16000, 256), (128, 20000, 640),
-                                   (256, 14336, 4096), (512, 6144, 8192)])
+MID_128_COLUMNS = [(130, 9000, 640), (300, 5000, 1152), (500, 3208, 384), (100, 16000, 256), (128, 20000, 640), (236, 14024, 2176), (391, 6224, 640), (65, 8336, 2176)]
+
+
+@pytest.mark.parametrize("M,N,K", MID_128_COLUMNS + [(256, 14336, 4096), (512, 6144, 8192)])
 def test_fp8_one_round_of_128_column_tiles(dev, M, N, K):
     """fp8 block GEMM on weights too wide for the 64-column mid-size kernel that fit one round of 64- or 128-row by
     128-column tiles (the 128-column form of the producer / consumer kernel): ragged rows and columns, odd numbers of

@@ -4,7 +4,8 @@ import ctypes
 import torch
 
 from llm_kernels_amd import _lib
-from test_gpu_gemm import W4A8_ANY_WORDS, WAVE_8BIT, WAVE_W4A8
+from test_gpu_duo import shape8, shape_w4a16
+from test_gpu_gemm import MID_128_COLUMNS, MID_BLOCKS, W4A8_ANY_WORDS, WAVE_8BIT, WAVE_W4A8
 from test_gpu_w4a16 import WAVE_MARLIN, WAVE_NK, WITHOUT_SCRATCH
 
 MUCH = 1 << 50
@@ -102,3 +103,17 @@ def test_offsets_and_grids_of_very_wide_weights():
             calls += [(N // 8 * 8, shape("w4a8", M, N // 8 * 8, 128, 128, MUCH)), (N // 2, shape("w4a16", 0, _lib.F16, M, N // 2, 128, 128, MUCH))]
             for n, got in calls:
                 assert got is None or -(-n // (16 * got[2])) * -(-M // (16 * got[1])) * got[0] * 64 < 1 << 32, (M, n, got)
+
+
+def test_the_mid_size_cases_stay_with_the_tile_kernels():
+    """Neither the wave kernels nor the one of two wave groups takes the shapes that the tests of the mid-size kernels are for."""
+    def others(kind, M, N, K):
+        lib = _lib.load()
+        if kind in ("fp16", "bf16"):
+            dt = _lib.F16 if kind == "fp16" else _lib.BF16
+            return shape("w4a16", 0, dt, M, N, K, 128, lib.llmk_gemm_w4a16_nk_workspace_bytes(M, N, K, 128, dt)) or shape_w4a16(0, dt, 128, M, N, K)
+        k8 = (_lib.KIND_FP8, 0) if kind == "fp8" else (_lib.KIND_I8, int(kind == "per token"))
+        return shape("8bit", *k8, M, N, K, lib.llmk_gemm_workspace_bytes(M, N, K)) or shape8(*k8, M, N, K)
+    for kinds, cases in MID_BLOCKS.items():
+        assert {(kind, c): others(kind, *c) for kind in kinds for c in cases if others(kind, *c)} == {}
+    assert {c: others("fp8", *c) for c in MID_128_COLUMNS if others("fp8", *c)} == {}
