@@ -238,8 +238,8 @@ extern "C" int llmk_gemm_fp8_block(const void* a, const float* a_s, const void* 
     return launch_block<K_FP8_BLOCK>(p, workspace, workspace_bytes, (hipStream_t)stream, "gemm_fp8_block");
 }
 
-// llmk_gemm_fp8_block for the benchmark's calibration: the same launch, and workgroup 0 of the 256-column tile kernel
-// reports the ticks of the shader clock and of the 100 MHz clock it lived (clocks[0], clocks[1]); shapes that run on
+// The tile kernels of llmk_gemm_fp8_block for the benchmark's calibration, also where that call takes the kernel of two wave groups: workgroup 0 of
+// the 256-column tile kernel reports the ticks of the shader clock and of the 100 MHz clock it lived (clocks[0], clocks[1]); shapes that run on
 // other kernels leave clocks untouched.
 extern "C" int llmk_calib_gemm_fp8_clock(const void* a, const float* a_s, const void* b, const float* b_s, void* c,
                                          int c_dtype, int64_t M, int64_t N, int64_t K, void* workspace,

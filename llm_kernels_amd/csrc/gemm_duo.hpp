@@ -6,7 +6,7 @@
 //
 // K_W4A8: 1024 x 4096 x 4096 30.8 us in one launch, 36.7 as expansion pass and the int8 kernel (37.7 | 33.4 with the quantiser).
 //
-// What bounds it: the CU's path from L2 (32 KB a phase of a 128 x 128 tile, 0.31 us of the 0.25 us that its products take) and the start and end of
+// What bounds it: the CU's path from L2 (the 32 KB of a phase of a 128 x 128 tile take 0.31 us, its products 0.25) and the start and end of
 // every phase.  Against the eight waves of gemm_dma_kernel, which share one 128-byte step: a wave tile is 64 x 64 instead of 32 x 64
 // (fragments of 16 KB instead of 24 for the same products), only waves that have nothing to multiply wait for the address path, and a
 // workgroup can be any multiple of 32 rows high, which is worth most where a few rows over a tile height would start another round.

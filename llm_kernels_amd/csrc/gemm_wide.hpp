@@ -244,7 +244,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
     float* bsl = (float*)(lds + SW + 2 * sw_bytes(W_BM));
     const int nblk = (N + 127) / 128;
 
-    // ---- source offsets of the 9 loads of a stage.  Load i of a wave fills LDS rows 8q .. 8q+7,
+    // ---- source offsets of the R / 2 + 4 loads of a stage.  Load i of a wave fills LDS rows 8q .. 8q+7,
     // q = 4*wave + i.  A: LDS row R holds tile row R.  B: within each 64-row group, LDS row rho holds
     // tile column 32*(rho >> 5) + 8*((rho & 15) >> 2) + 4*((rho >> 4) & 1) + (rho & 3), so that MFMA j yields,
     // in lane group g, the four columns 32*(j >> 1) + 8g + 4*(j & 1) + (0..3): a lane ends up with two runs
