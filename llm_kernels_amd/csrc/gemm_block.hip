@@ -128,7 +128,7 @@ double large_estimate(const DirectArgs& p, bool tail) {
 // shapes 1.007 fp8, 1.002 int8, 1.005 per token times as fast as with their cached times, us, cached | HBM: fp8 129 x 4096 x 14336 22.8 | 33.6 -> 20.7 |
 // 23.9, int8 110 x 15992 x 12032 48.5 | 66.3 -> 40.6 | 49.0, per token 452 x 3176 x 10112 31.1 | 37.5 -> 24.7 | 30.3; at worst 3.5 % slower).
 // Two kinds of calls up to 512 rows are left to the others whatever the estimates say, which have no term for weights from HBM there: int8 and per-token
-// products of short K on one row tile (63 shapes 0.98 times as fast here, us, others | this one, from HBM: int8 97 x 20048 x 1664 14.1 | 15.9, per token
+// products of short K on one row tile (66 shapes 0.98 times as fast here, us, others | this one, from HBM: int8 97 x 20048 x 1664 14.1 | 15.9, per token
 // 131 x 19264 x 1664 15.1 | 17.6; fp8 gains there) and fp8 and per-token ones of more than a round of workgroups (18 shapes 0.98: per token 500 x
 // 17848 x 11904 131 | 176, fp8 289 x 23480 x 2304 33.1 | 41.1; int8 gains).
 template <int KIND>

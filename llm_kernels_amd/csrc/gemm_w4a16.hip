@@ -1006,7 +1006,7 @@ double nk_large_estimate(const llmk::DirectArgs& p, bool copy) {
     const llmk::TileChoice c = copy ? llmk::dma_tile_estimate<HALF_KIND, false>(p) : llmk::dma_tile_estimate<KIND, false>(p);
     const double e = c.cost * (double)p.K / 4096.0, nk = (double)p.N * p.K * 1e-6;
     constexpr bool BF = KIND == llmk::K_W4NKB;
-    // (few short tiles, where the passes are mostly their launches: 2 % rms to 176 shapes of up to 1024 columns.  With the estimate of the larger ones 58 of
+    // (few short tiles, where the passes are mostly their launches: 2 to 3 % rms to 176 shapes of up to 1024 columns.  With the estimate of the larger ones 58 of
     // them went to the kernel of two wave groups and were 3 to 14 % slower: fp16 1240 x 72 x 640 7.6 | 8.6, 2007 x 440 x 2048 16.2 | 18.7, bf16 1027 x 208 x 1024 9.7 | 10.9)
     if (copy && c.choice == 1) return 4.45 + 1.24 * e + 1.3 * std::min(nk, 4.0) + 0.5 * std::max(nk - 4.0, 0.0) + 0.54e-6 * (double)p.M * p.N;
     if (copy) return BF ? 6.3 + 1.37 * e + 0.44 * nk : 9.0 + 1.25 * e + 0.59 * nk;
