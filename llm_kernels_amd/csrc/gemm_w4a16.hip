@@ -1128,7 +1128,7 @@ llmk::WavePlan marlin_wave(int64_t M, int64_t N, int64_t K, int group, int64_t s
 // The kernel of two wave groups (gemm_duo.hpp) for a call on Marlin words, or mi = 0: from 65 rows on, 8 % below the estimate of the wave kernel, the
 // tiles above, or beyond 512 rows the 16-bit copy of W and the fp16 tiles (a fit of 10 % rms to 146 shapes).  Its threads scatter the words
 // without bank conflicts.  Over 300 random shapes of 64 to 4096 rows 1.06 times as fast as without, 0.5 % behind the faster one of each
-// shape, at worst 9 % slower.  Others | this one, us: 1024 x 4096 x 4096 52.7 | 43.7, 432 x 6144 x 4096 42.0 | 36.6, 1072 x 3200 x 6400 76 | 61,
+// shape; of 1070 more 3 were 5 to 8 % slower.  Others | this one, us: 1024 x 4096 x 4096 52.7 | 43.7, 432 x 6144 x 4096 42.0 | 36.6, 1072 x 3200 x 6400 76 | 61,
 // 832 x 2560 x 2560 31.5 | 25.1, but 2384 x 6144 x 4096 106 | 134 and 416 x 1600 x 1664 9.0 | 16.7.
 llmk::DuoPlan marlin_duo(int64_t M, int64_t N, int64_t K, int group, const llmk::WavePlan& wave, int64_t scratch) {
     if (M <= 64 || K % 64) return {0, 1, 0.0};

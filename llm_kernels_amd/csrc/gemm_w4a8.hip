@@ -75,7 +75,7 @@ inline int64_t w4a8_widened_bytes(int64_t M, int64_t N, int64_t K) {
 // tile unpacks the weights again, so large N K goes the other way.)
 // From 65 rows on the kernel of two wave groups, which expands the words itself, is taken 8 % below the estimate of either: the two passes are the
 // expansion, and the int8 tiles or that kernel on int8 weights, whichever is estimated faster (a fit of 7 % rms to 165 shapes).  Over 300
-// random shapes of 64 to 4096 rows this was 1.05 times as fast as without, at worst level.  Others | this one, us: 1024 x 4096 x 4096
+// random shapes of 64 to 4096 rows this was 1.05 times as fast as without; of 1070 more 5 were 5 to 10 % slower.  Others | this one, us: 1024 x 4096 x 4096
 // 36.7 | 30.8, 425 x 6144 x 4096 32.5 | 25.3, 184 x 14272 x 1664 19.2 | 14.5, but 2373 x 6144 x 4096 79 | 107 and 91 x 5936 x 1024 7.1 | 9.5.
 // The two passes of few tiles have an estimate of their own (7 % rms to 110 shapes of K below 3072): with the other one 48 of 161 shapes went to this kernel
 // and were 3 to 10 % slower (1718 x 160 x 1152 9.6 | 10.7, 3723 x 112 x 1664 11.6 | 13.0).
