@@ -122,7 +122,7 @@ double large_estimate(const DirectArgs& p, bool tail) {
 }
 // The kernel of two wave groups (gemm_duo.hpp) for this call, or mi = 0: 8 % below the estimate of what the call gets otherwise (w: the wave
 // kernel, if it does).  Over 300 random shapes of 64 to 4096 rows a kind this was 1.04 (fp8, int8, per token) times as fast as without,
-// 0.5 to 1 % behind the faster one of each shape; of 3000 more, cached weights and weights from HBM, 5 were 5 to 7 % slower.  Others | this one, us: fp8 1024 x 4096 x 4096 25.5 | 20.7, int8 28.8 |
+// 0.5 to 1 % behind the faster one of each shape; of 4110 more, cached weights and weights from HBM, 5 were 5 to 8 % slower.  Others | this one, us: fp8 1024 x 4096 x 4096 25.5 | 20.7, int8 28.8 |
 // 25.6, per token 23.9 | 20.3; the gain is largest where 96, 128 or 160 rows leave fewer rows of the last tiles empty than 64, 128 and
 // 256 do, and where few tiles can be split along K beyond 512 rows.  Up to 512 rows the others are estimated with weights from HBM in the mean (450
 // shapes 1.007 fp8, 1.002 int8, 1.005 per token times as fast as with their cached times, us, cached | HBM: fp8 129 x 4096 x 14336 22.8 | 33.6 -> 20.7 |
