@@ -357,23 +357,36 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         // (the wave that ends the phase goes first; us with the multiplying wave first | none | the fetching one, 1024 x 4096 x 4096: int8 25.8 | 25.1 |
         // 24.0, fp8 21.4 | 21.4 | 21.1, w4a8 35.5 | 31.7 | 30.8, per token the same, bf16 x 4-bit 42.0 | 43.3 | 44.7)
         if constexpr (SCALED) __builtin_amdgcn_s_setprio(1);
+        // 4-bit weights, 16-bit activations: the LDS reads go first, so that the wave's requests, which wait for the address path one by one, run beside
+        // them, and row-packed words are expanded in front of the requests too (Marlin words, whose expansion is eight scattered writes, behind
+        // them).  us, requests first | reads first, then requests | expansion in front of the requests: rows 300 x 14336 x 4096 bf16 44.1 | 42.7 | 41.9, fp16
+        // 44.9 | 43.4 | 42.6, bf16 512 x 6144 x 4096 36.7 | 37.9 | 35.8, fp16 1500 x 4096 x 4096 55.1 | 52.6 | 52.4, Marlin 320 x 14336 x 4096 47.0 | 43.4 |
+        // 46.7, 768 x 4096 x 7168 61.6 | 58.5 | 60.9.  8-bit operands: no difference (fp8 1024 x 4096 x 4096 25.9 | 25.8, int8 200 x 14336 x 4096 25.0 | 25.3).
+        auto expand_words = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            words_landed(u & 3);
+            expand_word(u & 3, u + 1, 0);
+            expand_word(u & 3, u + 1, 1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if constexpr (W4A16) {
+            fetch(u);
+            if constexpr (!MARLIN) expand_words();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         request(u + 3);
         if constexpr (SCALES) request_scales((u >> 2) + 1);
+        if constexpr (W4A16) {
+            if constexpr (MARLIN) expand_words();
+            request_words(u & 3, u + 5);
+        }
         if constexpr (W4A8) {                                // (in front of the fragments, which leave no registers for it)
             words8_landed((u >> 1) & 1);
             expand8((u >> 1) & 1, u + 1);
             request_words8((u >> 1) & 1, u + 5);
             __builtin_amdgcn_sched_barrier(0);
         }
-        fetch(u);
-        if constexpr (W4A16) {
-            __builtin_amdgcn_sched_barrier(0);
-            words_landed(u & 3);
-            expand_word(u & 3, u + 1, 0);
-            expand_word(u & 3, u + 1, 1);
-            __builtin_amdgcn_sched_barrier(0);
-            request_words(u & 3, u + 5);
-        }
+        if constexpr (!W4A16) fetch(u);
         if constexpr (SCALED) __builtin_amdgcn_s_setprio(0);
         if constexpr (SCALES) meet(c_ls);
         else meet(c_l);
