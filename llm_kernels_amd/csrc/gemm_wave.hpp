@@ -52,10 +52,10 @@ __device__ __forceinline__ unsigned wv_bits(wv_us2 v) { return __builtin_bit_cas
 struct WaveTile {
     int col, row;
 };
-__device__ __forceinline__ WaveTile wave_tile(int M, int bm) {
+__device__ __forceinline__ WaveTile wave_tile(int M, int bm, FastDiv by_rows) {
     const int lin = blockIdx.x, total = gridDim.x, rows = (M + bm - 1) / bm, x = lin & 7;
     const int idx = x * (total >> 3) + min(x, total & 7) + (lin >> 3);
-    const int col = idx / rows;
+    const int col = (int)by_rows((uint32_t)idx);
     return {col, idx - col * rows};
 }
 
@@ -80,16 +80,28 @@ __device__ __forceinline__ void wv_store(const DirectArgs& p, const float* red, 
         if (orow >= BM || m >= m_end) continue;
         v4f sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
         v4i ia = {0, 0, 0, 0}, ib = {0, 0, 0, 0};
+        // four waves' reads on their way before their first sum: few threads have an output here, and each would wait for one read after the other
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const float* src = red + (w * BM + orow) * RED_ROW + ocol;
-            if constexpr (ROWCOL) {
-                ia += *(const v4i*)src;
-                ib += *(const v4i*)(src + 4);
-            } else {
-                sa += *(const v4f*)src;
-                sb += *(const v4f*)(src + 4);
+        for (int w0 = 0; w0 < NW; w0 += 4) {
+            v4f part[4][2];
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) part[w][h] = *(const v4f*)(red + ((w0 + w) * BM + orow) * RED_ROW + ocol + 4 * h);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                if constexpr (ROWCOL) {
+                    ia += __builtin_bit_cast(v4i, part[w][0]);
+                    ib += __builtin_bit_cast(v4i, part[w][1]);
+                } else {
+                    sa += part[w][0];
+                    sb += part[w][1];
+                }
             }
+            // (the sums are made here: eight waves' reads at a time take more registers than the loop)
+            if constexpr (ROWCOL) asm volatile("" : "+v"(ia), "+v"(ib) : : "memory");
+            else asm volatile("" : "+v"(sa), "+v"(sb) : : "memory");
         }
         const int64_t off = (int64_t)m * N + nn;
         if constexpr (ROWCOL) {
@@ -135,7 +147,7 @@ __global__ __launch_bounds__(NW * 64) void w4a8_wave_kernel(DirectArgs p) {
         kt0 = (int)blockIdx.z * per;
         KT = min(per, KT_all - kt0);
     }
-    const WaveTile tile = wave_tile(p.M, BM);
+    const WaveTile tile = wave_tile(p.M, BM, p.by_rows);
     const int n0 = tile.col * BN, m0 = tile.row * BM, m_end = min(p.M, m0 + BM);
     const int s_lo = wave * KT / NW, n = (wave + 1) * KT / NW - s_lo;
 
@@ -152,10 +164,11 @@ __global__ __launch_bounds__(NW * 64) void w4a8_wave_kernel(DirectArgs p) {
     constexpr uint32_t ssz = S32 ? 4u : 2u;
     const int8_t* const tab4 = p.w4_s4 + (int64_t)n0 * KT_all;
     const int8_t* const tabz = p.w4_z4 + (int64_t)n0 * KT_all;
-    const int W = (KT + 3) >> 2;                             // dwords per column (the last one may reach past the range)
+    // dwords per column of a whole slice (the last ones may reach past the range)
+    const int W = p.words;
     const uint32_t tab_last = (uint32_t)min((int64_t)(N - n0) * KT_all - 4, (int64_t)0x7fffffff);
     auto tab_at = [&](int idx, int& col, int& w, int& shift) {
-        col = idx / W;
+        col = (int)p.by_words((uint32_t)idx);
         w = idx - col * W;
         const uint32_t want = (uint32_t)min(min(col, BN - 1), N - 1 - n0) * (uint32_t)KT_all + (uint32_t)(kt0 + 4 * w);
         const uint32_t at = min(want, tab_last);
@@ -362,8 +375,11 @@ int launch_w4a8_wave(const DirectArgs& p, int z, hipStream_t stream, const char*
         if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     DirectArgs q = p;
     q.ksplit = z;
-    const int zg = (KT_all + per - 1) / per;
-    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
+    const int zg = (KT_all + per - 1) / per, rows = (p.M + 16 * MT - 1) / (16 * MT);
+    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * rows);
+    q.by_rows = fast_div((uint32_t)rows);
+    q.words = (per + 3) >> 2;
+    q.by_words = fast_div((uint32_t)q.words);
     kern<<<dim3(tiles, 1, (unsigned)zg), NW * 64, bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
     if (z > 1) return wv_sum_slices(p, zg, stream, name);
@@ -383,7 +399,8 @@ int launch_w4a8_wave(const DirectArgs& p, int z, hipStream_t stream, const char*
 constexpr int wh_a(int mt) { return 16 * mt * 128; }
 constexpr bool wh_marlin(int kind) { return kind == K_W4MARLIN; }
 constexpr int wh_b(int kind, int nt) { return wh_marlin(kind) ? 4096 : nt * 1024; }     // Marlin: the whole 64-column chunk
-constexpr int wh_stage(int kind, int mt, int nt) { return wh_a(mt) + 2 * wh_b(kind, nt); }
+// 16 rows: a whole K step; more: the activations of a half, and the words of two steps
+constexpr int wh_stage(int kind, int mt, int nt) { return mt == 1 ? 2 * wh_a(1) + wh_b(kind, nt) : wh_a(mt) + 2 * wh_b(kind, nt); }
 constexpr int wh_tab_cols(int kind, int nt) { return wh_marlin(kind) ? 64 : 16 * nt; }
 constexpr int wh_tab_row(int kind, int nt) { return 2 * wh_tab_cols(kind, nt) + 8; }
 constexpr int wh_lds(int kind, int nw, int mt, int nt, int groups) {
@@ -428,14 +445,20 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
     static_assert(is_w4nk(KIND) || wh_marlin(KIND), "4-bit weights, 16-bit activations");
     static_assert(PRE || !wh_marlin(KIND), "Marlin words: scaled weights");
     constexpr bool MARLIN = wh_marlin(KIND), BF = (KIND == K_W4NKB);
-    constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = wh_stage(KIND, MT, NT), OFF_B = wh_a(MT), WB = wh_b(KIND, NT), NB = WB / 1024;
+    constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = wh_stage(KIND, MT, NT), WB = wh_b(KIND, NT), NB = WB / 1024;
+    // 16 rows: a step's words and activations are one request, and the wave waits once for them: us for Marlin words, halves | whole steps, weights in the
+    // cache (from HBM): 16 x 4096 x 4096 6.49 (7.22) | 6.30 (6.76), 16 x 14336 x 4096 10.4 (12.1) | 10.1 (11.7), 16 x 9984 x 1152 6.2 (6.7) | 5.8 (6.2).  Two
+    // stages of them are slower (6.85: twice the loads are issued in front of the scale table), and so are whole steps of 32 rows from HBM (32 x
+    // 14336 x 4096 14.1 | 14.7).
+    constexpr bool WHOLE = MT == 1;
+    constexpr int OFF_B = (WHOLE ? 2 : 1) * wh_a(MT);
     constexpr int TR = wh_tab_row(KIND, NT), TC = wh_tab_cols(KIND, NT);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int N = p.N, K = p.K, KT_all = K >> 7, G = K / p.group, nchunks = N >> 6;
+    const int N = p.N, K = p.K, KT_all = K >> 7, G = (int)p.by_group((uint32_t)KT_all), nchunks = N >> 6;
     int kt0 = 0, KT = KT_all;
     if (p.ksplit > 1) {
         const int per = (KT_all + p.ksplit - 1) / p.ksplit;
@@ -443,7 +466,7 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
         KT = min(per, KT_all - kt0);
     }
     // Marlin: the workgroups that share a chunk (64 columns) are neighbours in the list of tiles, so that one L2 serves them
-    const WaveTile tile = wave_tile(p.M, BM);
+    const WaveTile tile = wave_tile(p.M, BM, p.by_rows);
     const int n0 = tile.col * BN, m0 = tile.row * BM, m_end = min(p.M, m0 + BM);
     const int chunk = n0 >> 6, sub = MARLIN ? tile.col & (4 / NT - 1) : 0;
     const int s_lo = wave * KT / NW, n = (wave + 1) * KT / NW - s_lo;
@@ -453,8 +476,8 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
     uint8_t* const tab = lds + NW * STAGE;                   // [group][column] fp16
 
     // ---- group scales of the tile, requested first (four per load)
-    const int g_lo = kt0 * 128 / p.group, GR = ((kt0 + KT) * 128 - 1) / p.group - g_lo + 1;
-    const int W = (GR + 3) >> 2, tab_n = MARLIN ? GR * 16 : BN * W;
+    const int g_lo = (int)p.by_group((uint32_t)kt0), GR = (int)p.by_group((uint32_t)(kt0 + KT - 1)) - g_lo + 1;
+    const int W = p.words, tab_n = MARLIN ? GR * 16 : BN * W;
     const WhTable range = wh_table((int64_t)(N - n0) * G);
     const uint8_t* const tabp = (const uint8_t*)p.b_s + (MARLIN ? ((int64_t)g_lo * N + chunk * 64) * 2 : (int64_t)n0 * G * 2 - range.back);
     const uint32_t tab_last = (uint32_t)min(range.last, (int64_t)0x7fffffff), tab_back = (uint32_t)range.back;
@@ -465,7 +488,7 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
             shift = 0;
             return (uint32_t)w * (uint32_t)(N * 2) + (uint32_t)col * 8u;
         } else {
-            col = idx / W;
+            col = (int)p.by_words((uint32_t)idx);
             w = idx - col * W;
             const uint32_t want = ((uint32_t)min(min(col, BN - 1), N - 1 - n0) * (uint32_t)G + (uint32_t)(g_lo + 4 * w)) * 2u + tab_back;
             const uint32_t at = min(want, tab_last);
@@ -526,11 +549,23 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
 #pragma unroll
         for (int i = 0; i < NB; ++i) dma16(mine_addr + OFF_B + (uint32_t)slot * WB + i * 1024u, boff[i], src);
     };
-    issue_b(s_lo, 0);
-    issue_a(s_lo, 0);
-    issue_b(s_lo + 1, 1);
+    auto issue_step = [&](int s) __attribute__((always_inline)) {
+        issue_b(s, 0);
+        const uint8_t* src = ga + (int64_t)(kt0 + min(s, KT - 1)) * 256;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 2 * MT; ++i) dma16(mine_addr + (uint32_t)(h * wh_a(MT)) + i * 1024u, aoff[i], src + h * 128);
+    };
+    if constexpr (WHOLE) {
+        issue_step(s_lo);
+    } else {
+        issue_b(s_lo, 0);
+        issue_a(s_lo, 0);
+        issue_b(s_lo + 1, 1);
+    }
 
-    ring_wait<2 * MT + 2 * NB>(t_s);
+    ring_wait<WHOLE ? 4 * MT + NB : 2 * MT + 2 * NB>(t_s);
     if (tid < tab_n) tab_put(t_col, t_w, t_shift, __builtin_bit_cast(uint64_t, t_s));
     for (int idx = tid + NW * 64; idx < tab_n; idx += NW * 64) {
         int col, w, shift;
@@ -549,18 +584,22 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
         for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
     // a[mt][f]: activation fragment of 32 of the half's 64 elements, in the order of the unpacked weights
-    v4i a[MT][2];
-    // w[j][f] (row-packed): the word of columns 16 j + r, elements 16 g + 8 f .. + 7 of the half
-    // w[st][j] (Marlin): word j of unit (c, g) of strip st of the half
-    unsigned w[MARLIN ? 4 : NT][MARLIN ? NT : 2];
+    struct Half {
+        v4i a[MT][2];
+        // w[j][f] (row-packed): the word of columns 16 j + r, elements 16 g + 8 f .. + 7 of the half
+        // w[st][j] (Marlin): word j of unit (c, g) of strip st of the half
+        unsigned w[MARLIN ? 4 : NT][MARLIN ? NT : 2];
+    };
     const int swz = swizzle(r);
-    auto fetch = [&](int h, int slot) __attribute__((always_inline)) {
-        const uint8_t* bst = mine + OFF_B + slot * WB;
+    // half h of a step: activation rows at ast, words at bst
+    auto fetch = [&](Half& half, int h, const uint8_t* ast, const uint8_t* bst) __attribute__((always_inline)) {
+        auto &a = half.a;
+        auto &w = half.w;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
-                const uint8_t* row = mine + mt * 2048 + r * 128;
+                const uint8_t* row = ast + mt * 2048 + r * 128;
                 if constexpr (MARLIN) {
                     // strips 2 f, 2 f + 1 of 16 elements: elements 2 g, 2 g + 1, 2 g + 8, 2 g + 9 of each
 #pragma unroll
@@ -606,8 +645,10 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
         else return mfma_f16_16x16x32(__builtin_bit_cast(v8h, x), __builtin_bit_cast(v8h, y), c);
     };
     const int mshift = 8 * (r >> 3);
-    auto compute = [&](int s) __attribute__((always_inline)) {
-        const uint8_t* tr = tab + ((kt0 + s) * 128 / p.group - g_lo) * TR + 2 * (MARLIN ? sub * BN : 0) + (PRE ? 2 * r : 8 * g);
+    auto compute = [&](Half& half, int s) __attribute__((always_inline)) {
+        auto &a = half.a;
+        auto &w = half.w;
+        const uint8_t* tr = tab + ((int)p.by_group((uint32_t)(kt0 + s)) - g_lo) * TR + 2 * (MARLIN ? sub * BN : 0) + (PRE ? 2 * r : 8 * g);
         v4f init[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -689,31 +730,49 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    // Step s: half 0 needs the activations requested last and the words requested a step before them; the words of step
-    // s + 1, requested behind those activations, may stay in flight.  Half 1 needs activations requested behind them.
-    int slot = 0;
-    for (int i = 0; i < n; ++i) {
-        const int s = s_lo + i;
-        const bool more = i + 1 < n;
-        if (more) wv_wait_loads<NB>();
-        else wv_wait_loads<0>();
-        fetch(0, slot);
-        fetched();
-        issue_a(s, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(s);
-        __builtin_amdgcn_sched_barrier(0);
-        wv_wait_loads<0>();
-        fetch(1, slot);
-        fetched();
-        if (more) {
-            issue_a(s + 1, 0);
-            if (i + 2 < n) issue_b(s + 2, slot);
+    if constexpr (WHOLE) {
+        // everything of step s is in registers before step s + 1 is requested into its place
+        Half h0, h1;
+        for (int i = 0; i < n; ++i) {
+            const int s = s_lo + i;
+            wv_wait_loads<0>();
+            fetch(h0, 0, mine, mine + OFF_B);
+            fetch(h1, 1, mine + wh_a(MT), mine + OFF_B);
+            fetched();
+            if (i + 1 < n) issue_step(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(h0, s);
+            compute(h1, s);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        compute(s);
-        __builtin_amdgcn_sched_barrier(0);
-        slot ^= 1;
+    } else {
+        // Step s: half 0 needs the activations requested last and the words requested a step before them; the words of step
+        // s + 1, requested behind those activations, may stay in flight.  Half 1 needs activations requested behind them.
+        int slot = 0;
+        Half half;
+        for (int i = 0; i < n; ++i) {
+            const int s = s_lo + i;
+            const bool more = i + 1 < n;
+            if (more) wv_wait_loads<NB>();
+            else wv_wait_loads<0>();
+            fetch(half, 0, mine, mine + OFF_B + slot * WB);
+            fetched();
+            issue_a(s, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(half, s);
+            __builtin_amdgcn_sched_barrier(0);
+            wv_wait_loads<0>();
+            fetch(half, 1, mine, mine + OFF_B + slot * WB);
+            fetched();
+            if (more) {
+                issue_a(s + 1, 0);
+                if (i + 2 < n) issue_b(s + 2, slot);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            compute(half, s);
+            __builtin_amdgcn_sched_barrier(0);
+            slot ^= 1;
+        }
     }
     wv_wait_loads<0>();
     __syncthreads();
@@ -738,8 +797,12 @@ int launch_w4a16_wave(const DirectArgs& p, int z, hipStream_t stream, const char
         if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
     DirectArgs q = p;
     q.ksplit = z;
-    const int zg = (KT_all + per - 1) / per;
-    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
+    const int zg = (KT_all + per - 1) / per, rows = (p.M + 16 * MT - 1) / (16 * MT);
+    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * rows);
+    q.by_rows = fast_div((uint32_t)rows);
+    q.by_group = fast_div((uint32_t)p.group >> 7);
+    q.words = (groups + 3) >> 2;
+    q.by_words = fast_div((uint32_t)q.words);
     kern<<<dim3(tiles, 1, (unsigned)zg), NW * 64, bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
     if (z > 1) return wv_sum_slices(p, zg, stream, name);
@@ -784,7 +847,7 @@ __global__ __launch_bounds__(NW * 64) void w8_wave_kernel(DirectArgs p) {
             KT = min(per, KT_all - kt0);
         }
     }
-    const WaveTile tile = wave_tile(p.M, BM);
+    const WaveTile tile = wave_tile(p.M, BM, p.by_rows);
     const int n0 = tile.col * BN, m0 = tile.row * BM, m_end = min(p.M, m0 + BM);
     const int s_lo = wave * KT / NW, n = (wave + 1) * KT / NW - s_lo;
     uint8_t* const mine = lds + wave * (D * STAGE);
@@ -927,8 +990,11 @@ int launch_w8_wave(const DirectArgs& p, hipStream_t stream, const char* name) {
     if (bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, bytes);
     if (bytes > 64 * 1024)       // (less needs no leave, and asking for it costs a decode call 0.1 us)
         if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
-    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * ((p.M + 16 * MT - 1) / (16 * MT)));
-    kern<<<dim3(tiles, 1, (unsigned)z), NW * 64, bytes, stream>>>(p);
+    const int rows = (p.M + 16 * MT - 1) / (16 * MT);
+    const unsigned tiles = (unsigned)(((p.N + 16 * NT - 1) / (16 * NT)) * rows);
+    DirectArgs q = p;
+    q.by_rows = fast_div((uint32_t)rows);
+    kern<<<dim3(tiles, 1, (unsigned)z), NW * 64, bytes, stream>>>(q);
     LLMK_CHECK_LAUNCH(name);
     return z > 1 ? wv_sum_slices(p, z, stream, name) : LLMK_OK;
 }

@@ -409,6 +409,14 @@ def test_mul_wave_kernel(dev, M, N, K, gs, scratch):
     assert (ws[nbytes:] == 0x5A).all()
 
 
+@pytest.mark.parametrize("M,N,K,gs", [(16, 192, 1152, 384), (16, 64, 8576, 8576), (16, 1088, 3840, 640), (16, 128, 17024, 128), (16, 4160, 2304, 768),
+                                      (48, 192, 1152, 384), (64, 576, 8960, 1280)])
+def test_mul_wave_kernel_groups(dev, M, N, K, gs):
+    """Groups of any number of K steps, cut by waves and by K slices: every step finds its group."""
+    test_mul_wave_kernel(dev, M, N, K, gs, True)
+    test_mul_wave_kernel(dev, M, N, K, gs, False)
+
+
 def _row_differences(M, K, gs, dev, dtype):
     """One +1 and one -1 a row, in the same group of K: the product is the difference of two weights of a column, exact in fp32."""
     x = torch.zeros(M, K, dtype=dtype, device=dev)
