@@ -25,7 +25,7 @@ namespace llmk {
 constexpr int MD_BN = 64, MD_THREADS = 512;
 
 constexpr int MD_B = 4 * MD_BN * 128;                       // weight stage: [sub-block][column][128 B] = 32 KB
-constexpr int MD_S = 4 * 64 * 4;                            // activation-scale columns of a step: [sub-block][row] fp32
+constexpr int MD_S = 4 * 64 * 4;                            // activation scales of a step, dwords: [row][sub-block], WIDE [sub-block][row]
 constexpr int MD_RED_ROW = 68;                              // floats per row of the final reduction (64 + 4: bank spread)
 
 // f(integral_constant<I>) for I = FIRST .. LAST - 1 (ring slots are compile-time indices)
@@ -163,8 +163,14 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
         if constexpr (W4NK) w4_shift = __builtin_ctz((unsigned)(p.group >> 6));
         auto kblock_sub = [&](int s, int sub) { return kt0 + min(NSUB * min(max(s, 0), nsteps - 1) + sub, KT - 1); };
         constexpr uint32_t SSZ = AS16 ? 2u : 4u;
-        // scale column of a sub-block: 64 rows per producer (WIDE: the two producers of the sub-block take 64 rows each)
-        const uint32_t soff = (uint32_t)min(m_start + min(lane + 64 * half, BM - 1), m_end - 1) * (uint32_t)KT_all * SSZ;
+        // Activation scales of a step.  64-column tiles: [row][sub-block] dwords, a load takes the four scales of each of 16 rows, 16 lines (a column of
+        // 64 rows is 64 of them, a sixth of what the address path had to do in a step: us, column | rows, weights in the cache (from HBM), int8 250 x 4096 x
+        // 14336 33.3 (41.0) | 32.6 (37.9), 70 x 4096 x 4096 9.8 (10.3) | 9.6 (10.1), fp8 256 x 4096 x 7168 20.6 (24.1) | 20.2 (23.3)).  WIDE: the scale column of a
+        // sub-block, 64 rows per producer, the two producers of the sub-block take 64 rows each (32 rows x two scales were 1 % slower: fp8 256 x
+        // 6144 x 4096 17.8 | 18.2).
+        constexpr int NSC = WIDE ? 1 : BM / 16;              // loads for all rows of a 64-column tile
+        const uint32_t soff = WIDE ? (uint32_t)min(m_start + min(lane + 64 * half, BM - 1), m_end - 1) * (uint32_t)KT_all * SSZ
+                                   : ((uint32_t)min(m_start + (q % NSC) * 16 + (lane >> 2), m_end - 1) * (uint32_t)KT_all + (uint32_t)kt0) * SSZ;
         // sub-block ksub of step s, clamped to the last one of the range (requests past the end repeat it)
         auto kblock = [&](int s) { return kt0 + min(NSUB * min(max(s, 0), nsteps - 1) + ksub, KT - 1); };
         auto issue_a = [&](int s) {
@@ -173,9 +179,11 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
 #pragma unroll
             for (int i = 0; i < NPA; ++i) dma16(st + (uint32_t)(ksub * (BM * 128) + (arow0 + 8 * i) * 128), aoff[i], p.a + (int64_t)kb * 128);
             if constexpr (SCALED) {
-                const uint32_t ss = st + MD_A + MD_B + (uint32_t)(WIDE ? 2 * ksub + half : q) * 256u;
-                if constexpr (AS16) dma2(ss, soff, (const uint8_t*)p.a_s + (int64_t)kb * 2);
-                else dma4(ss, soff, (const uint8_t*)p.a_s + (int64_t)kb * 4);
+                const uint32_t ss = st + MD_A + MD_B + (uint32_t)(WIDE ? 2 * ksub + half : q % NSC) * 256u;
+                const uint32_t at = soff + (WIDE ? 0u : (uint32_t)min(4 * min(max(s, 0), nsteps - 1) + (lane & 3), KT - 1) * SSZ);
+                const uint8_t* const from = (const uint8_t*)p.a_s + (WIDE ? (int64_t)kb * SSZ : 0);
+                if constexpr (AS16) dma2(ss, at, from);
+                else dma4(ss, at, from);
             }
         };
         v4i ring[RB][NBR];
@@ -286,16 +294,17 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
             for (int j = 0; j < 4; ++j) bf[j] = ldfrag(Bs + j * 2048);
             af[0] = ldfrag(As);
             if constexpr (SCALED) {
-                const float* Ss = (const float*)(st + MD_A + MD_B) + ksub * (WIDE ? 128 : 64) + r;
+                constexpr int SROW = WIDE ? 1 : 4;           // dwords from a row's scale to the next one's
+                const float* Ss = (const float*)(st + MD_A + MD_B) + (WIDE ? ksub * 128 + r : r * 4 + ksub);
                 const float bs = live ? bsl[min(kb, KT - 1)] : 0.f;
                 float sa[MT];
 #pragma unroll
                 for (int i = 0; i < MT; ++i) {
                     if constexpr (AS16) {
-                        const unsigned raw = ((const unsigned*)Ss)[16 * i];
+                        const unsigned raw = ((const unsigned*)Ss)[16 * SROW * i];
                         sa[i] = scale16_f32(raw, p.s_dtype) * bs;
                     } else {
-                        sa[i] = Ss[16 * i] * bs;
+                        sa[i] = Ss[16 * SROW * i] * bs;
                     }
                 }
                 // the products of tile row i are scaled and accumulated while the matrix instructions of row i + 1 run

@@ -144,7 +144,20 @@ def test_scales_of_every_k_step_on_large_tiles(dev, kind, M, steps):
     """Small integers under scales that are powers of two of their own in every row, column block and K step: every product and sum is
     a whole number below 2^24, so the fp32 result is exact in any order, and a scale taken from another step or row shows."""
     announce("scales on large tiles", kind, M, steps)
-    N, K = 4096, 128 * steps
+    check_scales_of_every_k_step(dev, kind, M, 4096, steps, torch.float32)
+
+
+@pytest.mark.parametrize("steps", [1, 3, 4, 6, 9, 31, 62])
+@pytest.mark.parametrize("M,N", [(40, 1024), (70, 4096), (129, 2048), (250, 3968), (251, 1920)])
+@pytest.mark.parametrize("kind", ["fp8", "int8", "int8 fp16 scales"])
+def test_scales_of_every_k_step_on_mid_size_tiles(dev, kind, M, N, steps):
+    """The same where K steps of 512 bytes end inside a step, in 32- and 64-row tiles, ragged rows, 64 and 128 columns and K slices."""
+    announce("scales on mid-size tiles", kind, M, N, steps)
+    check_scales_of_every_k_step(dev, kind.split()[0], M, N, steps, torch.float16 if "fp16" in kind else torch.float32)
+
+
+def check_scales_of_every_k_step(dev, kind, M, N, steps, scales):
+    K = 128 * steps
     gen = torch.Generator(device=dev).manual_seed(100 * steps + M)
 
     def ints(lo, hi, *shape):
@@ -153,6 +166,7 @@ def test_scales_of_every_k_step_on_large_tiles(dev, kind, M, steps):
     a, b = ints(-3, 3, M, K), ints(-3, 3, N, K)
     a_s, b_s = 2.0 ** ints(0, 4, M, steps).float(), 2.0 ** ints(0, 4, N // 128, steps).float()
     ref = (a.double() * a_s.double().repeat_interleave(128, 1)) @ (b.double() * b_s.double().repeat_interleave(128, 1).repeat_interleave(128, 0)).t()
+    a_s, b_s = a_s.to(scales), b_s.to(scales)
     with default_dtype(torch.float32):
         if kind == "fp8":
             c = fp8_kernel.fp8_gemm(a.float().to(torch.float8_e4m3fn), a_s, b.float().to(torch.float8_e4m3fn), b_s)
