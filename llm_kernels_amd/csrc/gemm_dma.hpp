@@ -48,11 +48,13 @@ __device__ __forceinline__ void dma2(uint32_t lds_addr, uint32_t voff, const voi
 #define LLMK_WAIT_VMCNT_0 0x0F70
 
 
-// 16-bit scale (zero-extended element) -> fp32, without a branch: with one the compiler moves the scale FMAs out from between the matrix
-// instructions, behind the blocks of the branch.
-__device__ __forceinline__ float scale16_f32(unsigned raw, int dt) {
-    const unsigned f16 = dt == LLMK_F16 ? ~0u : 0u;
-    return __uint_as_float((__float_as_uint(f16_to_f32((unsigned short)raw)) & f16) | ((raw << 16) & ~f16));
+// 16-bit scale of dtype SDT (zero-extended element) -> fp32.  The dtype is known when the kernel is compiled: told apart without a branch (with one the
+// compiler moves the scale FMAs out from between the matrix instructions) a scale is five vector instructions, and loops that these bound had up to a tenth of
+// them for it.
+template <int SDT>
+__device__ __forceinline__ float scale16_f32(unsigned raw) {
+    if constexpr (SDT == LLMK_F16) return f16_to_f32((unsigned short)raw);
+    else return __uint_as_float(raw << 16);
 }
 
 // Unscaled kinds accumulate inside the MFMA over the whole K range: two 16x16x32 half-precision MFMAs, or two
@@ -248,10 +250,11 @@ __device__ __forceinline__ void xcd_tile(int lin, int gx, int gy, int& bx, int& 
 }
 
 // MI = 16-row tiles per wave along M (4, 2 or 1): the workgroup tile is 64*MI rows x 128 columns.
-// AS16: the activation scales are 16-bit (fp16 or bf16 by p.s_dtype) and are staged as they are, one zero-extended
+// SDT: dtype of the activation scales; 16-bit ones (AS16) are staged as they are, one zero-extended
 // element per dword slot of the scale column (global_load_lds_ushort), instead of being widened by a pass of their own.
-template <int KIND, bool GROUPED, int MI, bool AS16 = false>
+template <int KIND, bool GROUPED, int MI, int SDT = LLMK_F32>
 __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
+    constexpr bool AS16 = SDT != LLMK_F32;
     constexpr int BM = 64 * MI;              // tile rows
     constexpr int WR = 16 * MI;              // rows per wave
     constexpr int D_A = d_a(MI), D_STAGE = d_stage(MI);
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(D_THREADS) void gemm_dma_kernel(DirectArgs p) {
             for (int i = 0; i < MI; ++i) {
                 if constexpr (AS16) {
                     const unsigned raw = ((const unsigned*)Ss)[i * 16];
-                    sa[i] = scale16_f32(raw, p.s_dtype) * bs;
+                    sa[i] = scale16_f32<SDT>(raw) * bs;
                 } else {
                     sa[i] = Ss[i * 16] * bs;
                 }
@@ -784,20 +787,31 @@ int launch_splitk_sum(const DirectArgs& p, int z, hipStream_t stream, const char
     return LLMK_OK;
 }
 
+// f(integral_constant<dtype of the activation scales>)
+template <bool AS16, class F>
+int with_scale_type(int s_dtype, F&& f) {
+    if constexpr (!AS16) return f(std::integral_constant<int, LLMK_F32>{});
+    else return s_dtype == LLMK_F16 ? f(std::integral_constant<int, LLMK_F16>{}) : f(std::integral_constant<int, LLMK_BF16>{});
+}
+
 // p.a_s: fp32, or with AS16 the 16-bit scales of dtype p.s_dtype as the caller passed them; p.s_dtype describes b_s.
 template <int KIND, bool GROUPED, int MI, bool AS16 = false>
 int launch_dma_mi(const DirectArgs& p, hipStream_t stream, const char* name) {
-    static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_dma_kernel<KIND, GROUPED, MI, AS16>;
     constexpr int BM = 64 * MI;
     const int tiles_m = GROUPED ? grouped_row_tiles(p.M, p.E, BM) : (p.M + BM - 1) / BM;
     const bool split = !GROUPED && p.ksplit > 1 && p.partial;
     constexpr int lds_bytes = d_lds(MI);
-    if (int rc = llmk_reserve_lds((const void*)kern, lds_bytes, configured, name)) return rc;
     dim3 grid((unsigned)((p.N + D_BN - 1) / D_BN), (unsigned)tiles_m, split ? (unsigned)p.ksplit : 1u);
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
-    kern<<<grid, D_THREADS, lds_bytes, stream>>>(p);
-    LLMK_CHECK_LAUNCH(name);
+    auto launch = [&](auto sdt_c) {
+        static std::atomic<uint64_t> configured{0};
+        auto kern = gemm_dma_kernel<KIND, GROUPED, MI, decltype(sdt_c)::value>;
+        if (int rc = llmk_reserve_lds((const void*)kern, lds_bytes, configured, name)) return rc;
+        kern<<<grid, D_THREADS, lds_bytes, stream>>>(p);
+        LLMK_CHECK_LAUNCH(name);
+        return (int)LLMK_OK;
+    };
+    if (int rc = with_scale_type<AS16>(p.s_dtype, launch)) return rc;
     if (split) return launch_splitk_sum<KIND>(p, p.ksplit, stream, name);
     return LLMK_OK;
 }

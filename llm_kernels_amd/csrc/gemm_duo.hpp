@@ -41,9 +41,10 @@ __device__ __forceinline__ uint32_t only32(uint32_t x) {
     return y;
 }
 
-template <int KIND, int MI, bool AS16 = false, bool GROUPED = false>
+template <int KIND, int MI, int SDT = LLMK_F32, bool GROUPED = false>
 __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
     static_assert(!GROUPED || KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK, "grouped products: block-scaled 8-bit operands");
+    constexpr bool AS16 = SDT != LLMK_F32;
     constexpr bool SCALED = du_scaled(KIND), ROWCOL = (KIND == K_I8_ROWCOL), W4A16 = du_w4a16(KIND), MARLIN = (KIND == K_W4MARLIN), W4A8 = (KIND == K_W4A8),
                    EXPANDS = W4A16 || W4A8;
     static_assert(SCALED || ROWCOL || W4A16, "8-bit operands, or 4-bit weights");
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             for (int i = 0; i < MI; ++i) {
                 if constexpr (AS16) {
                     const unsigned raw = ((const unsigned*)Ss)[i * 64];
-                    sa[i] = scale16_f32(raw, p.s_dtype) * bs;
+                    sa[i] = scale16_f32<SDT>(raw) * bs;
                 } else {
                     sa[i] = Ss[i * 64] * bs;
                 }
@@ -612,22 +613,26 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
 // p.a_s: fp32, or with AS16 the 16-bit scales of dtype p.s_dtype as the caller passed them; p.ksplit / p.partial select the K split.
 template <int KIND, int MI, bool AS16 = false, bool GROUPED = false>
 int launch_duo(const DirectArgs& p, hipStream_t stream, const char* name) {
-    static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_duo_kernel<KIND, MI, AS16, GROUPED>;
     constexpr int fixed = du_lds(KIND, MI);
     static_assert(fixed <= D_LDS_MAX && 8 * ((MI + 1) / 2) * 4096 <= fixed, "slots, and the exchange of half the sums in them, fit in LDS");
     const int KT = (p.K * (is_half(KIND) ? 2 : 1)) >> 7, z = p.ksplit > 1 ? p.ksplit : 1;
     const int lds_bytes = fixed + (KIND == K_W4A8 ? du_table((KT + z - 1) / z) : 0);
     if (lds_bytes > D_LDS_MAX) LLMK_FAIL(LLMK_ERR_SHAPE, "%s: %d bytes of LDS needed", name, lds_bytes);
-    if (int rc = llmk_reserve_lds((const void*)kern, KIND == K_W4A8 ? D_LDS_MAX : fixed, configured, name)) return rc;
     const bool split = !GROUPED && p.ksplit > 1 && p.partial;
     DirectArgs q = p;
     q.ksplit = split ? p.ksplit : 1;
     const int tiles_m = GROUPED ? grouped_row_tiles(p.M, p.E, 32 * MI) : (p.M + 32 * MI - 1) / (32 * MI);
     dim3 grid((unsigned)((p.N + DU_BN - 1) / DU_BN), (unsigned)tiles_m, (unsigned)q.ksplit);
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
-    kern<<<grid, DU_THREADS, lds_bytes, stream>>>(q);
-    LLMK_CHECK_LAUNCH(name);
+    auto launch = [&](auto sdt_c) {
+        static std::atomic<uint64_t> configured{0};
+        auto kern = gemm_duo_kernel<KIND, MI, decltype(sdt_c)::value, GROUPED>;
+        if (int rc = llmk_reserve_lds((const void*)kern, KIND == K_W4A8 ? D_LDS_MAX : fixed, configured, name)) return rc;
+        kern<<<grid, DU_THREADS, lds_bytes, stream>>>(q);
+        LLMK_CHECK_LAUNCH(name);
+        return (int)LLMK_OK;
+    };
+    if (int rc = with_scale_type<AS16>(p.s_dtype, launch)) return rc;
     return split ? launch_splitk_sum<KIND == K_W4A8 ? K_I8_BLOCK : KIND>(q, q.ksplit, stream, name) : LLMK_OK;
 }
 

@@ -76,9 +76,10 @@ constexpr int mdp_lds(int mt, bool wide = false) {
 }
 
 // XCDS: the tiles are dealt to the XCDs in blocks (xcd_tile) instead of in row-major order, see launch_mid.
-template <int KIND, int MT, bool AS16, bool WIDE, bool XCDS>
+template <int KIND, int MT, int SDT, bool WIDE, bool XCDS>
 __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
     static_assert(WIDE ? (MT == 8 || MT == 4) : (MT == 4 || MT == 2), "tile rows");
+    constexpr bool AS16 = SDT != LLMK_F32;
     constexpr int BN = mdp_bn(WIDE), NSUB = mdp_nsub(WIDE), RED_ROW = BN + 4;
     static_assert(BN * NSUB * 128 == MD_B && RED_ROW == (WIDE ? 132 : MD_RED_ROW), "weight stage of 32 KB");
     static_assert(KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK || KIND == K_I8_ROWCOL || KIND == K_F16 || KIND == K_BF16 || is_w4nk(KIND),
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
                 for (int i = 0; i < MT; ++i) {
                     if constexpr (AS16) {
                         const unsigned raw = ((const unsigned*)Ss)[16 * SROW * i];
-                        sa[i] = scale16_f32(raw, p.s_dtype) * bs;
+                        sa[i] = scale16_f32<SDT>(raw) * bs;
                     } else {
                         sa[i] = Ss[16 * SROW * i] * bs;
                     }
@@ -452,14 +453,14 @@ int launch_mid(const DirectArgs& p, hipStream_t stream, const char* name) {
     constexpr int BN = mdp_bn(WIDE);
     dim3 grid((unsigned)((p.N + BN - 1) / BN), (unsigned)((p.M + 16 * MT - 1) / (16 * MT)), (unsigned)z);
     if (grid.x == 0 || grid.y == 0) return LLMK_OK;
-    auto launch = [&](auto xcds_c) {
+    auto launch = [&](auto xcds_c) { return with_scale_type<AS16>(p.s_dtype, [&](auto sdt_c) {
         static std::atomic<uint64_t> configured{0};
-        auto kern = gemm_mid_pc_kernel<KIND, MT, AS16, WIDE, decltype(xcds_c)::value>;
+        auto kern = gemm_mid_pc_kernel<KIND, MT, decltype(sdt_c)::value, WIDE, decltype(xcds_c)::value>;
         if (int rc = llmk_reserve_lds((const void*)kern, D_LDS_MAX, configured, name)) return rc;
         kern<<<grid, MD_THREADS, lds_bytes, stream>>>(q);
         LLMK_CHECK_LAUNCH(name);
         return (int)LLMK_OK;
-    };
+    }); };
     // Blocks of tiles where row-major order does not deal whole columns to the XCDs already (one row of tiles: it does; per token 34 x 12816 x 4864
     // 14.2 us row-major, 15.0 so), the operands do not fit an XCD's L2 of 4 MB anyway (4-bit weights 158 x 4784 x 1152 8.4 row-major, 8.9
     // so), and none of these leaves little to gain: two tile rows of short operand rows (fp8 99 x 9232 x 1152 6.7 | 8.8 cached | from HBM, 7.1 | 9.2
