@@ -40,8 +40,11 @@ __device__ __forceinline__ uint32_t sw_row(int blk, int m_start, int m_end, int 
     return (uint32_t)min(m_start + 16 * blk + (lane >> 2), m_end - 1) * (uint32_t)KT_all;
 }
 // (steps past kt_end repeat the last one)
+template <int SDT>
 __device__ __forceinline__ void sw_load(uint32_t lds_addr, uint32_t row, int kb, int kt_end, const void* a_s, int lane) {
-    dma4(lds_addr, (row + (uint32_t)min(kb + (lane & 3), kt_end - 1)) * 4u, a_s);
+    const uint32_t at = row + (uint32_t)min(kb + (lane & 3), kt_end - 1);
+    if constexpr (SDT == LLMK_F32) dma4(lds_addr, at * 4u, a_s);
+    else dma2(lds_addr, at * 2u, a_s);
 }
 
 // ---- which tile a workgroup works on.  `lin` = linear workgroup id (blockIdx.y * gridDim.x + blockIdx.x), gx = column
@@ -180,9 +183,11 @@ constexpr int W_TAIL_ITEMS = LLMK_CUS;          // upper bound of ntail * z
 // p.c receives [M, I] quantised values, p.q_scale their scales.  Every rounding point of the separate kernels is kept
 // (sums rounded to the tensor dtype p.c_dtype, activation and product in that dtype, the quantiser's own arithmetic), so
 // the outputs equal those of GEMM + activation + quantiser bit for bit; the [M, 2 I] tensor never exists.
-template <int KIND, bool GROUPED, int R = 8, bool SWIGLU = false>
+template <int KIND, bool GROUPED, int R = 8, bool SWIGLU = false, int SDT = LLMK_F32>
 __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
-    // (16-bit activation scales are widened before this kernel, see launch_big)
+    // SDT: dtype of the activation scales.  fp16 ones of int8 operands, as their quantisers make them, are taken as they are, others widened before this
+    // kernel, see launch_big.
+    static_assert(SDT == LLMK_F32 || (KIND == K_I8_BLOCK && SDT == LLMK_F16), "scales");
     static_assert(R == 8 || R == 4, "tile rows per wave");
     static_assert(!SWIGLU || (GROUPED && (KIND == K_FP8_BLOCK || KIND == K_I8_BLOCK)), "gated epilogue: grouped block-scaled kinds");
     constexpr int W_BM = w_bm(R), W_A = W_BM * 128, W_STAGE = w_stage(R), SW = 2 * W_STAGE;
@@ -276,7 +281,7 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
         const int w = __builtin_amdgcn_readfirstlane(window);
         const uint32_t st = lds_base + SW + (uint32_t)(w & 1) * sw_bytes(W_BM);
 #pragma unroll
-        for (int i = 0; i < R / 4; ++i) sw_load(st + (uint32_t)(wave + 8 * i) * 256u, srow[i], kt0 + 4 * w, kt0 + KT, p.a_s, lane);
+        for (int i = 0; i < R / 4; ++i) sw_load<SDT>(st + (uint32_t)(wave + 8 * i) * 256u, srow[i], kt0 + 4 * w, kt0 + KT, p.a_s, lane);
     };
 
     // ---- 4-bit weights: a thread owns the same piece of the 128-column half h = 0, 1 of the tile as in the
@@ -458,7 +463,10 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
             const float* Ss = (const float*)(lds + SW + ((kt >> 2) & 1) * sw_bytes(W_BM)) + (wm * 16 * R + r) * 4 + (kt & 3);
             const float bs = bsl[(wn >> 1) * D_MAX_KT + kt];
 #pragma unroll
-            for (int i = 0; i < NR; ++i) sa[i] = Ss[i * 64] * bs;
+            for (int i = 0; i < NR; ++i) {
+                if constexpr (SDT == LLMK_F32) sa[i] = Ss[i * 64] * bs;
+                else sa[i] = scale16_f32<SDT>(((const unsigned*)Ss)[i * 64]) * bs;
+            }
         }
 #pragma unroll
         for (int i = 0; i < R; ++i) {
@@ -726,10 +734,10 @@ bool wide_tail_ok(const DirectArgs& p, const void* ws, int64_t ws_bytes) {
            p.c && llmk_device_cus() == LLMK_CUS;
 }
 
-template <int KIND, bool GROUPED, int R = 8>
+template <int KIND, bool GROUPED, int R = 8, int SDT = LLMK_F32>
 int launch_wide(const DirectArgs& p0, hipStream_t stream, const char* name, void* ws = nullptr, int64_t ws_bytes = 0) {
     static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_wide_kernel<KIND, GROUPED, R>;
+    auto kern = gemm_wide_kernel<KIND, GROUPED, R, false, SDT>;
     constexpr int W_BM = w_bm(R), W_LDS = w_lds(R);
     constexpr int ESZ = is_half(KIND) ? 2 : 1;
     if (int rc = llmk_reserve_lds((const void*)kern, W_LDS, configured, name)) return rc;
@@ -758,10 +766,10 @@ int launch_wide(const DirectArgs& p0, hipStream_t stream, const char* name, void
 
 // The gated-activation form of the kernel (grouped gate / up projection, p.N = 2 I, I % 128 == 0): one column tile per
 // 128 gate columns; no split of the last round (its tiles would have to meet before the activation).
-template <int KIND, int R>
+template <int KIND, int R, int SDT = LLMK_F32>
 int launch_wide_swiglu(const DirectArgs& p, hipStream_t stream, const char* name) {
     static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_wide_kernel<KIND, true, R, true>;
+    auto kern = gemm_wide_kernel<KIND, true, R, true, SDT>;
     constexpr int W_BM = w_bm(R), W_LDS = w_lds(R);
     static_assert(8 * (R / 2) * 2 * 1024 + 2 * 2 * 2 * 16 * (R / 2) * 4 <= W_LDS, "exchange area and row maxima fit in the stages");
     if (int rc = llmk_reserve_lds((const void*)kern, W_LDS, configured, name)) return rc;
@@ -871,16 +879,17 @@ TileChoice dma_tile_estimate(const DirectArgs& p, bool tail = false) {
 template <int KIND, bool GROUPED>
 int dma_tile_choice(const DirectArgs& p, bool tail = false) { return dma_tile_estimate<KIND, GROUPED>(p, tail).choice; }
 
-// AS16 (16-bit activation scales staged as they are): the 64- and 128-row tiles of gemm_dma_kernel only, see launch_big
+// AS16 (16-bit activation scales staged as they are): the 64- and 128-row tiles of gemm_dma_kernel, fp16 ones also the 256-column tiles, see launch_big
 template <int KIND, bool GROUPED, bool AS16 = false>
 int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* ws = nullptr, int64_t ws_bytes = 0) {
     if (!GROUPED && p.ksplit > 1) return launch_dma_mi<KIND, GROUPED, 1, AS16>(p, stream, name);
     const int choice = dma_tile_choice<KIND, GROUPED>(p, !GROUPED && !is_half(KIND) && wide_tail_ok<KIND>(p, ws, ws_bytes));
+    if constexpr (KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND))) {
+        constexpr int SDT = AS16 ? LLMK_F16 : LLMK_F32;
+        if (choice == 9) return launch_wide<KIND, GROUPED, 4, SDT>(p, stream, name, ws, ws_bytes);
+        if (choice == 8) return launch_wide<KIND, GROUPED, 8, SDT>(p, stream, name, ws, ws_bytes);
+    }
     if constexpr (!AS16) {
-        if constexpr (KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND))) {
-            if (choice == 9) return launch_wide<KIND, GROUPED, 4>(p, stream, name, ws, ws_bytes);
-            if (choice == 8) return launch_wide<KIND, GROUPED, 8>(p, stream, name, ws, ws_bytes);
-        }
         if (choice == 4) return launch_dma_mi<KIND, GROUPED, 4>(p, stream, name);
     }
     if (choice == 2) return launch_dma_mi<KIND, GROUPED, 2, AS16>(p, stream, name);
@@ -935,7 +944,8 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
             const int z = GROUPED ? 1 : splitk_factor(p.M, p.N, p.K);
             const int64_t widened = ((int64_t)p.M * (p.K >> 7) * 4 + 255) & ~(int64_t)255;
             const bool tail = !GROUPED && workspace && wide_tail_ok<KIND>(p, (uint8_t*)workspace + widened, workspace_bytes - widened);
-            as16 = z > 1 || dma_tile_choice<KIND, GROUPED>(p, tail) <= 2;
+            const int choice = dma_tile_choice<KIND, GROUPED>(p, tail);
+            as16 = z > 1 || choice <= 2 || (choice >= 8 && p.s_dtype == LLMK_F16);
         }
     }
     if (p.s_dtype != LLMK_F32 && !as16) {
