@@ -635,12 +635,10 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
                             own[2 * q] = bf16_to_f32((unsigned short)b); own[2 * q + 1] = bf16_to_f32((unsigned short)(b >> 16));
                         }
                     }
+                    if constexpr (HALF == 0) gated_act8<IDT>(own, other, p.act, false, 1.0f, y[i][h]);
+                    else gated_act8<IDT>(other, own, p.act, false, 1.0f, y[i][h]);
 #pragma unroll
-                    for (int q = 0; q < EPL; ++q) {
-                        const float gv = HALF == 0 ? own[q] : other[q], up = HALF == 0 ? other[q] : own[q];
-                        y[i][h][q] = gated_act<IDT>(gv, up, p.act, false, 1.0f);
-                        m = fmaxf(m, fabsf(y[i][h][q]));
-                    }
+                    for (int q = 0; q < EPL; ++q) m = fmaxf(m, fabsf(y[i][h][q]));
                 }
                 m = fmaxf(m, __shfl_xor(m, 16, 64));
                 m = fmaxf(m, __shfl_xor(m, 32, 64));
@@ -653,11 +651,12 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
                 const float m = fmaxf(mx[i], rowmax[((wm * 2 + HALF) * 2 + (1 - w1)) * (16 * RH) + 16 * i + r]);
                 const int row = m_start + wm * 16 * R + 16 * (OWN + i) + r;
                 if (row >= m_end) continue;
+                const QuantScale<FP8Q> qs(m);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const int col = n0 + 64 * w1 + 32 * h + 8 * g;
-                    quant_store8<FP8Q>(y[i][h], m, p.c, (int64_t)row * I_half + col, p.q_scale, (int64_t)row * gcols + bx,
-                                       w1 == 0 && g == 0 && h == 0, p.round_mode);
+                    store_quant8<FP8Q>(quant8_by<FP8Q, true>(y[i][h], qs, p.round_mode), qs.sc, p.c, (int64_t)row * I_half + col, p.q_scale, (int64_t)row * gcols + bx,
+                                       w1 == 0 && g == 0 && h == 0);
                 }
             }
         };

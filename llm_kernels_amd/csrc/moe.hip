@@ -351,12 +351,10 @@ __global__ void act_and_mul_vec_kernel(const void* __restrict__ gateup, void* __
             load8<IDT>(gateup, row * two_i + c1, gv[1]);
             load8<IDT>(gateup, row * two_i + I + c1, up[1]);
         }
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) r[j] = gated_act<IDT>(gv[0][j], up[0][j], act, has_scale, scale);
+        gated_act8<IDT>(gv[0], up[0], act, has_scale, scale, r);
         store8<ODT>(out, row * I + c0, r);
         if (two) {
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) r[j] = gated_act<IDT>(gv[1][j], up[1][j], act, has_scale, scale);
+            gated_act8<IDT>(gv[1], up[1], act, has_scale, scale, r);
             store8<ODT>(out, row * I + c1, r);
         }
     }
@@ -395,11 +393,9 @@ __global__ void act_mul_quant_kernel(const void* __restrict__ gateup, void* __re
         const float scale = has_scale ? rnd<IDT>(1.0f / scales[e - start_e]) : 1.0f;
         float r[EPL];
         float m = 0.f;
+        gated_act8<IDT>(gv[k], up[k], act, has_scale, scale, r);
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) {
-            r[j] = gated_act<IDT>(gv[k][j], up[k][j], act, has_scale, scale);
-            m = fmaxf(m, fabsf(r[j]));
-        }
+        for (int j = 0; j < EPL; ++j) m = fmaxf(m, fabsf(r[j]));
         m = group_max<16>(m);
         if (!live[k] || !local) continue;
         quant_store8<FP8>(r, m, q_out, row[k] * I + col[k], s_out, grp[k], sub == 0, mode);
