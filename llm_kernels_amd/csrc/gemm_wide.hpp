@@ -885,8 +885,10 @@ int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* 
     const int choice = dma_tile_choice<KIND, GROUPED>(p, !GROUPED && !is_half(KIND) && wide_tail_ok<KIND>(p, ws, ws_bytes));
     if constexpr (KIND != K_W4MARLIN && !(GROUPED && is_w4nk(KIND))) {
         constexpr int SDT = AS16 ? LLMK_F16 : LLMK_F32;
-        if (choice == 9) return launch_wide<KIND, GROUPED, 4, SDT>(p, stream, name, ws, ws_bytes);
-        if (choice == 8) return launch_wide<KIND, GROUPED, 8, SDT>(p, stream, name, ws, ws_bytes);
+        if (!AS16 || p.s_dtype == SDT) {                     // (bf16 scales: the 64-row tiles)
+            if (choice == 9) return launch_wide<KIND, GROUPED, 4, SDT>(p, stream, name, ws, ws_bytes);
+            if (choice == 8) return launch_wide<KIND, GROUPED, 8, SDT>(p, stream, name, ws, ws_bytes);
+        }
     }
     if constexpr (!AS16) {
         if (choice == 4) return launch_dma_mi<KIND, GROUPED, 4>(p, stream, name);
@@ -934,14 +936,15 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
     // 16-bit activation scales: the int8 kind stages them as they are (AS16 instantiations); fp8 callers pass fp32
     // scales as a rule, 16-bit ones are widened into the workspace first
     constexpr bool HAS_AS16 = (KIND == K_I8_BLOCK);
-    // (only where the launch is short: the conversion inside the K loop costs the vector-ALU-bound int8 loop 4-5 %,
-    // the widening pass a launch of 5-7 us: 512 x 4096 x 4096 21.4 -> 17.8 us, 1024 x 4096 x 4096 28.0 -> 26.5 us, but
-    // 4096 x 14336 x 4096 277.6 -> 291 us when forced; the 64- and 128-row tiles are the short launches)
+    // On the 64- and 128-row tiles, and fp16 ones on the 256-column tiles.  The widening pass is a launch of 2.5 to 7 us, a conversion is one instruction
+    // a tile row and K step (512 x 4096 x 4096 21.4 -> 17.8 us, 1024 x 4096 x 4096 28.0 -> 26.5; 256-column tiles, fp16 scales 1500 x 4096 x 4096 45.3 -> 43.8,
+    // 2000 x 6144 x 4096 74.8 -> 73.0, 4096 x 14336 x 4096 level).  The 256 x 128 tile, and bf16 scales, which no quantiser here makes, on the
+    // 256-column ones keep the pass.
     bool as16 = false;
+    const int64_t widened = ((int64_t)p.M * (p.K >> 7) * 4 + 255) & ~(int64_t)255;
     if constexpr (HAS_AS16) {
         if (p.s_dtype != LLMK_F32) {
             const int z = GROUPED ? 1 : splitk_factor(p.M, p.N, p.K);
-            const int64_t widened = ((int64_t)p.M * (p.K >> 7) * 4 + 255) & ~(int64_t)255;
             const bool tail = !GROUPED && workspace && wide_tail_ok<KIND>(p, (uint8_t*)workspace + widened, workspace_bytes - widened);
             const int choice = dma_tile_choice<KIND, GROUPED>(p, tail);
             as16 = z > 1 || choice <= 2 || (choice >= 8 && p.s_dtype == LLMK_F16);
@@ -955,7 +958,7 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
         else scales_to_f32_kernel<LLMK_BF16><<<blocks, 256, 0, stream>>>(p.a_s, (float*)workspace, n);
         LLMK_CHECK_LAUNCH(name);
         p.a_s = workspace;
-        used = (n * 4 + 255) & ~(int64_t)255;
+        used = widened;
     }
     // Few 64-row tiles (mid-size M, moderate N): split K over workgroups so that every CU streams weights,
     // fp32 partials in the workspace, one summing pass.
@@ -970,7 +973,8 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
     if constexpr (HAS_AS16) {
         if (as16) {
             if (p.ksplit > 1 || !workspace) return launch_dma<KIND, GROUPED, true>(p, stream, name);
-            return launch_dma<KIND, GROUPED, true>(p, stream, name, workspace, workspace_bytes);                  // split last round
+            // split last round, in the scratch that as16 was decided for: with more of it the tile choice could be another one
+            return launch_dma<KIND, GROUPED, true>(p, stream, name, (uint8_t*)workspace + widened, workspace_bytes - widened);
         }
     }
     if (p.ksplit > 1 || !workspace || workspace_bytes <= used) return launch_dma<KIND, GROUPED>(p, stream, name);

@@ -156,7 +156,18 @@ def test_scales_of_every_k_step_on_mid_size_tiles(dev, kind, M, N, steps):
     check_scales_of_every_k_step(dev, kind.split()[0], M, N, steps, torch.float16 if "fp16" in kind else torch.float32)
 
 
-def check_scales_of_every_k_step(dev, kind, M, N, steps, scales):
+@pytest.mark.parametrize("scales", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("extra", [-16, 0, 256, 1 << 30])
+@pytest.mark.parametrize("M,N,steps", [(861, 2801, 200), (520, 264, 9)])
+def test_int8_scales_at_scratch_limits(dev, M, N, steps, extra, scales):
+    """16-bit activation scales where the split last round of 256-column tiles fits in the scratch, but not behind fp32 scales (861 x 2801 x 25600 is one of the
+    shapes that go to another tile with it): the scales are read as what they are, whatever scratch there is, and nothing behind it is written."""
+    announce("int8 scales, scratch", M, N, steps, extra, str(scales))
+    nbytes = min((64 << 20) + extra, _lib.load().llmk_gemm_workspace_bytes(M, N, 128 * steps))
+    check_scales_of_every_k_step(dev, "int8", M, N, steps, scales, nbytes)
+
+
+def check_scales_of_every_k_step(dev, kind, M, N, steps, scales, scratch=None):
     K = 128 * steps
     gen = torch.Generator(device=dev).manual_seed(100 * steps + M)
 
@@ -164,11 +175,18 @@ def check_scales_of_every_k_step(dev, kind, M, N, steps, scales):
         return torch.randint(lo, hi + 1, shape, device=dev, generator=gen)
 
     a, b = ints(-3, 3, M, K), ints(-3, 3, N, K)
-    a_s, b_s = 2.0 ** ints(0, 4, M, steps).float(), 2.0 ** ints(0, 4, N // 128, steps).float()
-    ref = (a.double() * a_s.double().repeat_interleave(128, 1)) @ (b.double() * b_s.double().repeat_interleave(128, 1).repeat_interleave(128, 0)).t()
+    a_s, b_s = 2.0 ** ints(0, 4, M, steps).float(), 2.0 ** ints(0, 4, -(-N // 128), steps).float()
+    ref = (a.double() * a_s.double().repeat_interleave(128, 1)) @ (b.double() * b_s.double().repeat_interleave(128, 1).repeat_interleave(128, 0)[:N]).t()
     a_s, b_s = a_s.to(scales), b_s.to(scales)
     with default_dtype(torch.float32):
-        if kind == "fp8":
+        if scratch is not None:
+            a, b = a.to(torch.int8), b.to(torch.int8)
+            c = torch.full((M, N), float("nan"), device=dev)
+            ws = torch.full((scratch + 256,), 0x5A, dtype=torch.uint8, device=dev)
+            _lib.call("llmk_gemm_i8_block", _lib.ptr(a), _lib.ptr(a_s), _lib.ptr(b), _lib.ptr(b_s), _lib.dt(scales), _lib.ptr(c), _lib.dt(torch.float32), M, N, K,
+                      _lib.ptr(ws), scratch, None)
+            assert (ws[scratch:] == 0x5A).all()
+        elif kind == "fp8":
             c = fp8_kernel.fp8_gemm(a.float().to(torch.float8_e4m3fn), a_s, b.float().to(torch.float8_e4m3fn), b_s)
         else:
             c = int8_kernel.int8_gemm(a.to(torch.int8), a_s, b.to(torch.int8), b_s)
