@@ -615,41 +615,60 @@ __global__ __launch_bounds__(W_THREADS) void gemm_wide_kernel(DirectArgs p) {
             // partner: same wm and wn & 1, other half
             const int partner = wm * 4 + (1 - HALF) * 2 + w1;
             const uint8_t* src = xch + (uint32_t)(partner * RH * 2) * 1024u + (uint32_t)lane * 16u;
+            const int row0 = m_start + wm * 16 * R + 16 * OWN;
             float y[RH][2][EPL], mx[RH];
+            // The partner's values are all requested before the first is used, the branch on the activation stands around all rows, empty tile rows of a ragged
+            // tile are passed over, and the rows' maxima cross the wave without LDS.  A read a half row, a branch behind it and two shuffles a row
+            // were a chain of eight LDS round trips and eight shuffles; with two waves a SIMD most of it was hidden (whole expert layers, us: 8 experts fp8
+            // 4096 tokens 1430 | 1425, 1184 tokens 593 | 587, int8 4096 tokens 1813 | 1805, 64 experts fp8 2000 tokens 265.8 | 264.3; the
+            // branch around eight elements instead of one before that 939 | 927 for this projection, 828 without activation and quantiser).
+            v4i got[RH][2];
 #pragma unroll
-            for (int i = 0; i < RH; ++i) {
-                float m = 0.f;
+            for (int i = 0; i < RH; ++i)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    float other[EPL], own[EPL];
-                    const v4i wo = *(const v4i*)(src + (i * 2 + h) * 1024);
-                    const v4i wm_ = pack8(acc[OWN + i][2 * h], acc[OWN + i][2 * h + 1]);
+                for (int h = 0; h < 2; ++h) got[i][h] = *(const v4i*)(src + (i * 2 + h) * 1024);
+            auto activate = [&](auto act_c) {
+                constexpr int ACT = decltype(act_c)::value;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const unsigned a = (unsigned)wo[q], b = (unsigned)wm_[q];
-                        if constexpr (IDT == LLMK_F16) {
-                            other[2 * q] = f16_to_f32((unsigned short)a); other[2 * q + 1] = f16_to_f32((unsigned short)(a >> 16));
-                            own[2 * q] = f16_to_f32((unsigned short)b); own[2 * q + 1] = f16_to_f32((unsigned short)(b >> 16));
-                        } else {
-                            other[2 * q] = bf16_to_f32((unsigned short)a); other[2 * q + 1] = bf16_to_f32((unsigned short)(a >> 16));
-                            own[2 * q] = bf16_to_f32((unsigned short)b); own[2 * q + 1] = bf16_to_f32((unsigned short)(b >> 16));
+                for (int i = 0; i < RH; ++i) {
+                    mx[i] = 0.f;
+                    if (row0 + 16 * i >= m_end) continue;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        float other[EPL], own[EPL];
+                        const v4i wo = got[i][h];
+                        const v4i wm_ = pack8(acc[OWN + i][2 * h], acc[OWN + i][2 * h + 1]);
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const unsigned a = (unsigned)wo[q], b = (unsigned)wm_[q];
+                            if constexpr (IDT == LLMK_F16) {
+                                other[2 * q] = f16_to_f32((unsigned short)a); other[2 * q + 1] = f16_to_f32((unsigned short)(a >> 16));
+                                own[2 * q] = f16_to_f32((unsigned short)b); own[2 * q + 1] = f16_to_f32((unsigned short)(b >> 16));
+                            } else {
+                                other[2 * q] = bf16_to_f32((unsigned short)a); other[2 * q + 1] = bf16_to_f32((unsigned short)(a >> 16));
+                                own[2 * q] = bf16_to_f32((unsigned short)b); own[2 * q + 1] = bf16_to_f32((unsigned short)(b >> 16));
+                            }
+                        }
+#pragma unroll
+                        for (int q = 0; q < EPL; ++q) {
+                            y[i][h][q] = gated_act<IDT, ACT>(HALF == 0 ? own[q] : other[q], HALF == 0 ? other[q] : own[q], false, 1.0f);
+                            mx[i] = fmaxf(mx[i], fabsf(y[i][h][q]));
                         }
                     }
-                    if constexpr (HALF == 0) gated_act8<IDT>(own, other, p.act, false, 1.0f, y[i][h]);
-                    else gated_act8<IDT>(other, own, p.act, false, 1.0f, y[i][h]);
-#pragma unroll
-                    for (int q = 0; q < EPL; ++q) m = fmaxf(m, fabsf(y[i][h][q]));
                 }
-                m = fmaxf(m, __shfl_xor(m, 16, 64));
-                m = fmaxf(m, __shfl_xor(m, 32, 64));
-                mx[i] = m;
-                if (g == 0) rowmax[((wm * 2 + HALF) * 2 + w1) * (16 * RH) + 16 * i + r] = m;
+            };
+            if (p.act == 0) activate(std::integral_constant<int, 0>{});
+            else activate(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int i = 0; i < RH; ++i) {
+                mx[i] = max_of_rows(mx[i]);
+                if (g == 0) rowmax[((wm * 2 + HALF) * 2 + w1) * (16 * RH) + 16 * i + r] = mx[i];
             }
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < RH; ++i) {
                 const float m = fmaxf(mx[i], rowmax[((wm * 2 + HALF) * 2 + (1 - w1)) * (16 * RH) + 16 * i + r]);
-                const int row = m_start + wm * 16 * R + 16 * (OWN + i) + r;
+                const int row = row0 + 16 * i + r;
                 if (row >= m_end) continue;
                 const QuantScale<FP8Q> qs(m);
 #pragma unroll

@@ -82,6 +82,13 @@ __device__ __forceinline__ int group_imin(int v) {
 // (LPG power of two <= 64).  Their bits order as integers, whose maximum needs no quieting of its operands.
 template <int LPG>
 __device__ __forceinline__ float group_max(float v) { return __int_as_float(group_imax<LPG>(__float_as_int(v))); }
+// the same over the four lanes l, l + 16, l + 32, l + 48: rows of 16 lanes change places between two registers, without a trip through LDS
+__device__ __forceinline__ float max_of_rows(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const int m = max((int)a[0], (int)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap((unsigned)m, (unsigned)m, false, false);
+    return __int_as_float(max((int)b[0], (int)b[1]));
+}
 
 
 // a / b from r = RN(1 / b): one product and the residual correction q - (q b - a) r, both in fma.  The
@@ -209,8 +216,7 @@ __device__ __forceinline__ float gated_act(float gv, float up, int act, bool has
     return act == 0 ? gated_act<IDT, 0>(gv, up, has_scale, scale) : gated_act<IDT, 1>(gv, up, has_scale, scale);
 }
 // eight of them.  The branch stands around all eight: one around each made every element a chain of its own, two transcendental instructions long, which
-// nothing ran beside (the gate / up projection of 8 experts, 4096 tokens, 256 x 256 tiles: 939 us | 927; with the
-// activation and the quantiser taken out 828).
+// nothing ran beside.
 template <int IDT>
 __device__ __forceinline__ void gated_act8(const float (&gv)[EPL], const float (&up)[EPL], int act, bool has_scale, float scale, float (&y)[EPL]) {
     if (act == 0) {

@@ -749,15 +749,35 @@ def test_gate_up_gemm_with_activation_epilogue_equals_three_kernels(dev, qdt, dt
     number of column tiles that is and is not a multiple of the XCD count, one empty segment, one shorter than a tile,
     ragged ends, permuted weight indices, rows behind the last segment untouched."""
     announce("gate/up + activation epilogue", qdt, dtype, act, rows, two_i, K)
-    E = 8
     torch.manual_seed(rows + two_i)
     used = rows - 5
-    cuts = sorted(torch.randint(0, used, (E - 3,)).tolist())
-    seg = torch.tensor([0, 37, 37] + cuts + [used], dtype=torch.int64, device=dev)     # segment 0: 37 rows, segment 1: empty
+    cuts = sorted(torch.randint(0, used, (5,)).tolist())
+    check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, [0, 37, 37] + cuts + [used])         # segment 0: 37 rows, segment 1: empty
+
+
+@pytest.mark.parametrize("qdt", [torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("dtype,act", [(torch.bfloat16, "silu"), (torch.float16, "gelu")])
+@pytest.mark.parametrize("rows,counts", [(8000, (1, 15, 16, 17, 63, 64, 65, 0)), (8000, (127, 128, 129, 191, 193, 255, 256, 257)), (4800, (1, 16, 17, 32, 33, 65, 127, 129)),
+                                         (4800, (31, 48, 49, 64, 80, 95, 96, 97))])
+def test_gate_up_activation_epilogue_of_part_tiles(dev, qdt, dtype, act, rows, counts):
+    """Segments that end at, one before and one behind a tile row, a wave's rows and a tile, in 256- and 128-row tiles; an infinite and a NaN scale in a row
+    each reach no other row."""
+    announce("gate/up + activation epilogue, part tiles", qdt, dtype, act, rows, counts)
+    torch.manual_seed(rows)
+    seg = [0]
+    for n in counts: seg.append(seg[-1] + n)
+    check_gate_up_epilogue(dev, qdt, dtype, act, rows, 4096, 256, seg, odd_rows=True)
+
+
+def check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, seg, odd_rows=False):
+    E, used = len(seg) - 1, seg[-1]
+    seg = torch.tensor(seg, dtype=torch.int64, device=dev)
     widx = torch.randperm(E).to(dev)
     act_quant = fp8_kernel.act_quant if qdt == torch.float8_e4m3fn else int8_kernel.act_quant
     wq = fp8_kernel.weight_quant if qdt == torch.float8_e4m3fn else int8_kernel.weight_quant
     a, a_s = act_quant((torch.randn(rows, K) * 2).to(dtype).to(dev))
+    if odd_rows:
+        a_s[7, 0], a_s[used - 3, 1] = float("inf"), float("nan")
     ws = [wq((torch.randn(two_i, K) * 0.3).to(dev)) for _ in range(E)]
     b = torch.stack([t[0].view(torch.uint8) for t in ws]).view(qdt)
     b_s = torch.stack([t[1] for t in ws])
@@ -770,9 +790,12 @@ def test_gate_up_gemm_with_activation_epilogue_equals_three_kernels(dev, qdt, dt
     ids = torch.zeros(rows, dtype=torch.int64, device=dev)
     q0, s0 = gk.act_and_mul_quant(c, two_i, ids, None, 0, E - 1, qdt, act)
     assert q1.shape == q0.shape and s1.shape == s0.shape and s1.dtype == s0.dtype
-    assert torch.equal(s1[:used].cpu(), s0[:used].cpu())
-    assert torch.equal(q1[:used].view(torch.uint8).cpu(), q0[:used].view(torch.uint8).cpu())
-    assert float(s0[:used].float().abs().max()) > 0
+    live = torch.ones(used, dtype=torch.bool)
+    if odd_rows: live[[7, used - 3]] = False
+    assert torch.equal(s1[:used].cpu()[live], s0[:used].cpu()[live])
+    assert torch.equal(q1[:used].view(torch.uint8).cpu()[live], q0[:used].view(torch.uint8).cpu()[live])
+    assert torch.equal(s1[:used].cpu().float().nan_to_num(-1.0), s0[:used].cpu().float().nan_to_num(-1.0))
+    assert float(s0[:used].cpu()[live].float().abs().max()) > 0
 
 
 def test_gate_up_activation_epilogue_refuses_small_shapes(dev):
