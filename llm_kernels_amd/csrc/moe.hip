@@ -363,7 +363,12 @@ __global__ void act_and_mul_vec_kernel(const void* __restrict__ gateup, void* __
 // Gated activation and 1 x 128 activation quantisation in one pass: 16 lanes own one group of 128 outputs,
 // 8 each.  The values quantised are exactly those the separate activation kernel would have stored in the
 // tensor dtype, so q and s equal those of the two-kernel sequence bit for bit.
-template <int IDT, bool FP8>
+// EIGHT: the branch on the activation stands around a thread's eight elements (gated_act8), faster where few waves share a SIMD: elements run beside each
+// other there.  With the chip full of waves those do so anyway, and a branch around each element is faster.  us, a branch around each | around
+// eight, bf16 to e4m3, SiLU (GELU): 32 x 14336 5.0 (5.05) | 4.6 (4.75), 1024 x 1408 5.5 (5.65) | 5.1 (5.4), 2048 x 2048 7.5 (7.8) | 7.4 (8.1), 8192 x
+// 2048 20.5 (21.9) | 21.7 (23.3), 8192 x 14336 121 (131) | 128 (144); to int8 4.4 (4.7) | 4.15 (4.3), 4.95 (5.2) | 4.7 (5.2), 6.9 (7.2) | 6.8 (7.5), 20.0
+// (21.7) | 20.7 (23.0), 118 (127) | 123 (139).  The line is two workgroups a CU, between 1024 x 1408 and 2048 x 2048.
+template <int IDT, bool FP8, bool EIGHT>
 __global__ void act_mul_quant_kernel(const void* __restrict__ gateup, void* __restrict__ q_out, void* __restrict__ s_out,
                                      const void* __restrict__ reorder_topk_ids, int ids_bytes,
                                      const float* __restrict__ scales, int start_e, int end_e, int64_t M, int64_t two_i,
@@ -393,9 +398,12 @@ __global__ void act_mul_quant_kernel(const void* __restrict__ gateup, void* __re
         const float scale = has_scale ? rnd<IDT>(1.0f / scales[e - start_e]) : 1.0f;
         float r[EPL];
         float m = 0.f;
-        gated_act8<IDT>(gv[k], up[k], act, has_scale, scale, r);
+        if constexpr (EIGHT) gated_act8<IDT>(gv[k], up[k], act, has_scale, scale, r);
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) m = fmaxf(m, fabsf(r[j]));
+        for (int j = 0; j < EPL; ++j) {
+            if constexpr (!EIGHT) r[j] = gated_act<IDT>(gv[k][j], up[k][j], act, has_scale, scale);
+            m = fmaxf(m, fabsf(r[j]));
+        }
         m = group_max<16>(m);
         if (!live[k] || !local) continue;
         quant_store8<FP8>(r, m, q_out, row[k] * I + col[k], s_out, grp[k], sub == 0, mode);
@@ -653,10 +661,13 @@ extern "C" int llmk_moe_act_and_mul_quant(const void* gateup, int in_dtype, void
     if (((uintptr_t)gateup | (uintptr_t)q_out) & 15) LLMK_FAIL(LLMK_ERR_ARG, "moe_act_and_mul_quant: buffers must be 16-byte aligned");
     const int64_t threads = M * (two_i / 256) * 16;
     const unsigned grid = (unsigned)cdiv64(threads, 256 * AMQ_UNROLL);
+    const bool eight = grid <= 2 * LLMK_CUS;
+#define CALL(FP8, EIGHT) act_mul_quant_kernel<IDT, FP8, EIGHT><<<grid, 256, 0, (hipStream_t)stream>>>(gateup, q_out, s_out, reorder_topk_ids, ids_bytes, scales, start_expert, end_expert, M, two_i, act, round_mode)
     LLMK_DISPATCH_FLOAT(in_dtype, IDT, {
-        if (kind == LLMK_KIND_FP8) act_mul_quant_kernel<IDT, true><<<grid, 256, 0, (hipStream_t)stream>>>(gateup, q_out, s_out, reorder_topk_ids, ids_bytes, scales, start_expert, end_expert, M, two_i, act, round_mode);
-        else act_mul_quant_kernel<IDT, false><<<grid, 256, 0, (hipStream_t)stream>>>(gateup, q_out, s_out, reorder_topk_ids, ids_bytes, scales, start_expert, end_expert, M, two_i, act, round_mode);
+        if (kind == LLMK_KIND_FP8) { if (eight) CALL(true, true); else CALL(true, false); }
+        else { if (eight) CALL(false, true); else CALL(false, false); }
     });
+#undef CALL
     LLMK_CHECK_LAUNCH("moe_act_and_mul_quant");
     return LLMK_OK;
 }

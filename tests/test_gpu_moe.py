@@ -721,6 +721,24 @@ def test_fused_quant_kernels_equal_the_two_kernel_sequence(dev, qdt, dtype, with
         assert torch.equal(s1.cpu()[local_rows], s0.cpu()[local_rows]), name
 
 
+@pytest.mark.parametrize("qdt", [torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("dtype,name", [(torch.bfloat16, "silu"), (torch.float16, "gelu")])
+@pytest.mark.parametrize("rows", [8191, 8192, 8193, 9001])
+def test_act_and_mul_quant_on_both_sides_of_the_kernel_choice(dev, qdt, dtype, name, rows):
+    """Two workgroups a CU are 8192 rows of two groups: the kernels of fewer and of more of them give what the two-kernel sequence gives."""
+    announce("fused activation, kernel choice", qdt, dtype, name, rows)
+    torch.manual_seed(rows)
+    I = 256
+    act_quant = fp8_kernel.act_quant if qdt == torch.float8_e4m3fn else int8_kernel.act_quant
+    ids = torch.zeros(rows, dtype=torch.int64, device=dev)
+    gateup = (torch.randn(rows, 2 * I) * 2).to(dtype).to(dev)
+    down = torch.empty(rows, I, dtype=dtype, device=dev)
+    (gk.silu_and_mul if name == "silu" else gk.gelu_and_mul)(gateup, down, 2 * I, ids, None, 0, 0)
+    q0, s0 = act_quant(down)
+    q1, s1 = gk.act_and_mul_quant(gateup, 2 * I, ids, None, 0, 0, qdt, name)
+    assert torch.equal(q1.view(torch.uint8).cpu(), q0.view(torch.uint8).cpu()) and torch.equal(s1.cpu(), s0.cpu())
+
+
 @pytest.mark.parametrize("kind", ["int8", "fp8"])
 def test_ep_moe_forward_fused_equals_unfused(dev, kind):
     announce("ep_moe fused vs unfused", kind)
