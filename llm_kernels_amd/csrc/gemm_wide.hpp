@@ -897,6 +897,17 @@ TileChoice dma_tile_estimate(const DirectArgs& p, bool tail = false) {
 template <int KIND, bool GROUPED>
 int dma_tile_choice(const DirectArgs& p, bool tail = false) { return dma_tile_estimate<KIND, GROUPED>(p, tail).choice; }
 
+// fp16 activation scales of int8 operands on the 256-column tiles: as they are up to 160 us by the estimate, widened by a pass in front of them beyond.  The
+// pass is a launch of 2 to 5 us, the conversions (one instruction a tile row and K step in a loop bound by vector instructions) cost 0.5 to 3 % of the time.
+// us, widened | as they are: 1487 x 4096 x 4096 37.9 | 36.1, 3909 x 4096 x 4096 74.9 | 73.2, 1671 x 4096 x 14336 122.5 | 121.6, 1332 x 11976 x 6016 153.6 |
+// 152.7, 3761 x 11864 x 7424 337 | 342, 2944 x 19320 x 9984 606 | 610; experts, 700 of 16 x 4096 x 2048 43.6 | 41.6, 1500 of 64 x 2816 x 2048 126.7 | 124.7, 3000 of
+// 64 x 2816 x 2048 226 | 228, 1500 of 8 x 28672 x 4096 481 | 496, 4096 of 8 x 4096 x 14336 576 | 595, with activation and quantiser 2200 of 8 x 28672 x 4096 702 |
+// 720 (tokens, two to eight experts each).  Of 119 shapes three lose 1.0 to 1.3 % this way (700 tokens of 8 x 28672 x 4096 273 as they are, 276 widened).  Without
+// room for the pass they are taken as they are.
+inline bool wide_f16_scales(const TileChoice& c, int K, int s_dtype, bool room) {
+    return s_dtype == LLMK_F16 && c.choice >= 8 && (!room || c.cost * K <= 160.0 * 4096.0);
+}
+
 // AS16 (16-bit activation scales staged as they are): the 64- and 128-row tiles of gemm_dma_kernel, fp16 ones also the 256-column tiles, see launch_big
 template <int KIND, bool GROUPED, bool AS16 = false>
 int launch_dma(const DirectArgs& p, hipStream_t stream, const char* name, void* ws = nullptr, int64_t ws_bytes = 0) {
@@ -955,18 +966,17 @@ int launch_big(DirectArgs p, void* workspace, int64_t workspace_bytes, hipStream
     // 16-bit activation scales: the int8 kind stages them as they are (AS16 instantiations); fp8 callers pass fp32
     // scales as a rule, 16-bit ones are widened into the workspace first
     constexpr bool HAS_AS16 = (KIND == K_I8_BLOCK);
-    // On the 64- and 128-row tiles, and fp16 ones on the 256-column tiles.  The widening pass is a launch of 2.5 to 7 us, a conversion is one instruction
-    // a tile row and K step (512 x 4096 x 4096 21.4 -> 17.8 us, 1024 x 4096 x 4096 28.0 -> 26.5; 256-column tiles, fp16 scales 1500 x 4096 x 4096 45.3 -> 43.8,
-    // 2000 x 6144 x 4096 74.8 -> 73.0, 4096 x 14336 x 4096 level).  The 256 x 128 tile, and bf16 scales, which no quantiser here makes, on the
-    // 256-column ones keep the pass.
+    // On the 64- and 128-row tiles, and fp16 ones on the 256-column tiles where wide_f16_scales says so (512 x 4096 x 4096 21.4 -> 17.8 us,
+    // 1024 x 4096 x 4096 28.0 -> 26.5).  The 256 x 128 tile, and bf16 scales, which no quantiser here makes, on the 256-column ones keep the pass.
     bool as16 = false;
     const int64_t widened = ((int64_t)p.M * (p.K >> 7) * 4 + 255) & ~(int64_t)255;
     if constexpr (HAS_AS16) {
         if (p.s_dtype != LLMK_F32) {
             const int z = GROUPED ? 1 : splitk_factor(p.M, p.N, p.K);
             const bool tail = !GROUPED && workspace && wide_tail_ok<KIND>(p, (uint8_t*)workspace + widened, workspace_bytes - widened);
-            const int choice = dma_tile_choice<KIND, GROUPED>(p, tail);
-            as16 = z > 1 || choice <= 2 || (choice >= 8 && p.s_dtype == LLMK_F16);
+            const TileChoice c = dma_tile_estimate<KIND, GROUPED>(p, tail);
+            const bool room = workspace && workspace_bytes >= (int64_t)p.M * (p.K >> 7) * 4;
+            as16 = z > 1 || c.choice <= 2 || wide_f16_scales(c, p.K, p.s_dtype, room);
         }
     }
     if (p.s_dtype != LLMK_F32 && !as16) {

@@ -765,11 +765,12 @@ extern "C" int llmk_grouped_gemm(const void* a, const void* b, void* c, int kind
 
 // which tile kernel the gated-activation form would run on for this shape: 8 / 4 = tile rows per wave of the 256-column
 // kernel, 0 = none (the caller runs the grouped GEMM and the activation kernel instead)
-static int swiglu_tile_rows(int kind, const DirectArgs& p) {
+static int swiglu_tile_rows(int kind, const DirectArgs& p, TileChoice* tile = nullptr) {
     if (p.N % 256 || p.K % 128 || !dma_eligible(p)) return 0;
     if (!grouped_tiles(p)) return 0;
-    const int choice = kind == LLMK_KIND_FP8 ? dma_tile_choice<K_FP8_BLOCK, true>(p) : dma_tile_choice<K_I8_BLOCK, true>(p);
-    return choice == 8 ? 8 : (choice == 9 ? 4 : 0);
+    const TileChoice c = kind == LLMK_KIND_FP8 ? dma_tile_estimate<K_FP8_BLOCK, true>(p) : dma_tile_estimate<K_I8_BLOCK, true>(p);
+    if (tile) *tile = c;
+    return c.choice == 8 ? 8 : (c.choice == 9 ? 4 : 0);
 }
 
 extern "C" int llmk_grouped_gemm_swiglu_quant_fused(int kind, int E, int64_t M, int64_t two_i, int64_t K) {
@@ -799,15 +800,16 @@ extern "C" int llmk_grouped_gemm_swiglu_quant(const void* a, const void* b, void
     p.seg_indptr = seg_indptr; p.weight_indices = weight_indices;
     p.c_dtype = mid_dtype; p.s_dtype = s_dtype; p.M = (int)M; p.N = (int)two_i; p.K = (int)K; p.E = E;
     p.act = act; p.round_mode = round_mode;
-    const int rows = swiglu_tile_rows(kind, p);
+    TileChoice tile{};
+    const int rows = swiglu_tile_rows(kind, p, &tile);
     if (!rows) LLMK_FAIL(LLMK_ERR_SHAPE, "grouped_gemm_swiglu_quant: shape E=%d M=%lld 2I=%lld K=%lld is not one the fused kernel takes (ask llmk_grouped_gemm_swiglu_quant_fused first)", E, (long long)M, (long long)two_i, (long long)K);
     hipStream_t st = (hipStream_t)stream;
     if (s_dtype != LLMK_F32) {
-        // 16-bit activation scales are widened first, as in front of the plain kernel, but for fp16 ones of int8 operands
+        // 16-bit activation scales are widened first, as in front of the plain kernel, fp16 ones of int8 operands where that is worth it
         const int64_t n = M * (K >> 7);
         if (!workspace || workspace_bytes < n * 4 || ((uintptr_t)workspace & 15)) LLMK_FAIL(LLMK_ERR_ARG, "grouped_gemm_swiglu_quant: 16-bit activation scales need %lld bytes of workspace", (long long)(n * 4));
         const unsigned blocks = (unsigned)cdiv64(n, 256);
-        if (s_dtype == LLMK_F16 && kind == LLMK_KIND_I8)
+        if (kind == LLMK_KIND_I8 && wide_f16_scales(tile, p.K, s_dtype, true))
             return rows == 8 ? launch_wide_swiglu<K_I8_BLOCK, 8, LLMK_F16>(p, st, "grouped_gemm_swiglu_quant(i8)") : launch_wide_swiglu<K_I8_BLOCK, 4, LLMK_F16>(p, st, "grouped_gemm_swiglu_quant(i8)");
         if (s_dtype == LLMK_F16) scales_to_f32_kernel<LLMK_F16><<<blocks, 256, 0, st>>>(scale_a, (float*)workspace, n);
         else if (s_dtype == LLMK_BF16) scales_to_f32_kernel<LLMK_BF16><<<blocks, 256, 0, st>>>(scale_a, (float*)workspace, n);

@@ -158,13 +158,22 @@ def test_scales_of_every_k_step_on_mid_size_tiles(dev, kind, M, N, steps):
 
 @pytest.mark.parametrize("scales", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("extra", [-16, 0, 256, 1 << 30])
-@pytest.mark.parametrize("M,N,steps", [(861, 2801, 200), (520, 264, 9)])
+@pytest.mark.parametrize("M,N,steps", [(861, 2801, 200), (520, 264, 9), (918, 8219, 64)])
 def test_int8_scales_at_scratch_limits(dev, M, N, steps, extra, scales):
     """16-bit activation scales where the split last round of 256-column tiles fits in the scratch, but not behind fp32 scales (861 x 2801 x 25600 is one of the
-    shapes that go to another tile with it): the scales are read as what they are, whatever scratch there is, and nothing behind it is written."""
+    shapes that go to another tile with it, 918 x 8219 x 8192 splits its last round with fp16 scales as they are): the scales are read as what they are, whatever
+    scratch there is, and nothing behind it is written."""
     announce("int8 scales, scratch", M, N, steps, extra, str(scales))
     nbytes = min((64 << 20) + extra, _lib.load().llmk_gemm_workspace_bytes(M, N, 128 * steps))
     check_scales_of_every_k_step(dev, "int8", M, N, steps, scales, nbytes)
+
+
+@pytest.mark.parametrize("scratch", [None, 0])
+@pytest.mark.parametrize("steps", [84, 85, 86, 87])
+def test_int8_fp16_scales_on_both_sides_of_the_widening_line(dev, steps, scratch):
+    """4000 x 4096: up to 85 K steps the 256-column tiles take fp16 scales as they are, from 86 on a pass widens them if there is scratch for it."""
+    announce("int8 fp16 scales, widened or not", steps, scratch)
+    check_scales_of_every_k_step(dev, "int8", 4000, 4096, steps, torch.float16, scratch)
 
 
 def check_scales_of_every_k_step(dev, kind, M, N, steps, scales, scratch=None):
