@@ -298,7 +298,8 @@ int llmk_moe_pre_reorder_quant(const void* x, int x_dtype, void* q_out, void* s_
  * scales scale_a [M, K/128], scale_b [E, 2I/128, K/128] of s_dtype; mid_dtype LLMK_F16 or LLMK_BF16 = the dtype the
  * separate GEMM would have written; act 0 silu, 1 tanh-gelu; q_out [M, I], s_out [M, I/128] as in
  * llmk_moe_act_and_mul_quant (no per-expert scales).  Rows outside every segment are left unwritten.  16-bit scales
- * need M * K/128 * 4 bytes of workspace.  Taken only for shapes that run on the 256-column tile kernel:
+ * need M * K/128 * 4 bytes of workspace, 16-byte aligned, but for fp16 ones of int8 operands, which long launches widen into it if it is
+ * there.  Taken only for shapes that run on the 256-column tile kernel:
  * llmk_grouped_gemm_swiglu_quant_fused returns 1 for those, 0 otherwise (then run the three calls), and the fused entry
  * fails with LLMK_ERR_SHAPE on a shape it does not take. */
 int llmk_grouped_gemm_swiglu_quant_fused(int kind, int E, int64_t M, int64_t two_i, int64_t K);

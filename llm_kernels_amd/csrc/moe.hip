@@ -805,12 +805,13 @@ extern "C" int llmk_grouped_gemm_swiglu_quant(const void* a, const void* b, void
     if (!rows) LLMK_FAIL(LLMK_ERR_SHAPE, "grouped_gemm_swiglu_quant: shape E=%d M=%lld 2I=%lld K=%lld is not one the fused kernel takes (ask llmk_grouped_gemm_swiglu_quant_fused first)", E, (long long)M, (long long)two_i, (long long)K);
     hipStream_t st = (hipStream_t)stream;
     if (s_dtype != LLMK_F32) {
-        // 16-bit activation scales are widened first, as in front of the plain kernel, fp16 ones of int8 operands where that is worth it
+        // 16-bit activation scales are widened first, as in front of the plain kernel, fp16 ones of int8 operands where that is worth it and there is room
         const int64_t n = M * (K >> 7);
-        if (!workspace || workspace_bytes < n * 4 || ((uintptr_t)workspace & 15)) LLMK_FAIL(LLMK_ERR_ARG, "grouped_gemm_swiglu_quant: 16-bit activation scales need %lld bytes of workspace", (long long)(n * 4));
+        const bool room = workspace && workspace_bytes >= n * 4 && !((uintptr_t)workspace & 15);
         const unsigned blocks = (unsigned)cdiv64(n, 256);
-        if (kind == LLMK_KIND_I8 && wide_f16_scales(tile, p.K, s_dtype, true))
+        if (kind == LLMK_KIND_I8 && wide_f16_scales(tile, p.K, s_dtype, room))
             return rows == 8 ? launch_wide_swiglu<K_I8_BLOCK, 8, LLMK_F16>(p, st, "grouped_gemm_swiglu_quant(i8)") : launch_wide_swiglu<K_I8_BLOCK, 4, LLMK_F16>(p, st, "grouped_gemm_swiglu_quant(i8)");
+        if (!room) LLMK_FAIL(LLMK_ERR_ARG, "grouped_gemm_swiglu_quant: 16-bit activation scales need %lld bytes of workspace", (long long)(n * 4));
         if (s_dtype == LLMK_F16) scales_to_f32_kernel<LLMK_F16><<<blocks, 256, 0, st>>>(scale_a, (float*)workspace, n);
         else if (s_dtype == LLMK_BF16) scales_to_f32_kernel<LLMK_BF16><<<blocks, 256, 0, st>>>(scale_a, (float*)workspace, n);
         else LLMK_FAIL(LLMK_ERR_DTYPE, "grouped_gemm_swiglu_quant: s_dtype %d", s_dtype);

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from oracle import moe_ref as m, quant_ref as q, gemm_ref as g
+from llm_kernels_amd import _lib
 from llm_kernels_amd.moe import group_gemm_kernel as gk
 from llm_kernels_amd.moe.ep_moe import ep_moe_forward, softmax_topk_router, EPMoE
 from llm_kernels_amd.moe.config import Config
@@ -814,6 +815,38 @@ def check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, seg, odd_rows=F
     assert torch.equal(q1[:used].view(torch.uint8).cpu()[live], q0[:used].view(torch.uint8).cpu()[live])
     assert torch.equal(s1[:used].cpu().float().nan_to_num(-1.0), s0[:used].cpu().float().nan_to_num(-1.0))
     assert float(s0[:used].cpu()[live].float().abs().max()) > 0
+
+
+@pytest.mark.parametrize("rows,E,K", [(4800, 8, 256), (6000, 4, 6144)])             # scales as they are, and widened where there is scratch
+def test_gate_up_activation_epilogue_without_scratch(dev, rows, E, K):
+    """fp16 scales of int8 operands need no scratch, and the results do not depend on it; other 16-bit scales are refused without."""
+    announce("gate/up + activation epilogue, scratch", rows, E, K)
+    torch.manual_seed(rows)
+    two_i, I, lib = 4096, 2048, _lib.load()
+    seg = torch.arange(E + 1, device=dev) * (rows // E)
+    widx = torch.arange(E, device=dev)
+    a = torch.randint(-100, 101, (rows, K), dtype=torch.int8, device=dev)
+    b = torch.randint(-100, 101, (E, two_i, K), dtype=torch.int8, device=dev)
+    a_s, b_s = torch.rand(rows, K // 128, device=dev) * 1e-3, torch.rand(E, two_i // 128, K // 128, device=dev) * 1e-3
+    assert lib.llmk_grouped_gemm_swiglu_quant_fused(_lib.KIND_I8, E, rows, two_i, K)
+
+    def run(kind, dtype, nbytes, offset=0):
+        q, s = torch.zeros(rows, I, dtype=torch.int8, device=dev), torch.zeros(rows, I // 128, dtype=torch.float32 if kind == _lib.KIND_FP8 else torch.float16, device=dev)
+        sa, sb, ws = a_s.to(dtype), b_s.to(dtype), torch.zeros(nbytes + offset + 256, dtype=torch.uint8, device=dev)
+        rc = lib.llmk_grouped_gemm_swiglu_quant(_lib.ptr(a), _lib.ptr(b), _lib.ptr(q), _lib.ptr(s), kind, _lib.BF16, 0, E, rows, two_i, K, _lib.ptr(seg), _lib.ptr(widx),
+                                                _lib.ptr(sa), _lib.ptr(sb), _lib.dt(dtype), 0, ws.data_ptr() + offset if nbytes else None, nbytes, None)
+        torch.cuda.synchronize()
+        assert (ws[nbytes + offset:] == 0).all()
+        return rc, q, s
+
+    need = rows * (K // 128) * 4
+    rc, q0, s0 = run(_lib.KIND_I8, torch.float16, need)
+    assert rc == 0 and float(s0.float().max()) > 0
+    for nbytes, offset in ((0, 0), (need - 4, 0), (need, 8)):
+        rc, q1, s1 = run(_lib.KIND_I8, torch.float16, nbytes, offset)
+        assert rc == 0 and torch.equal(q1, q0) and torch.equal(s1, s0)
+    for kind, dtype in ((_lib.KIND_I8, torch.bfloat16), (_lib.KIND_FP8, torch.float16)):
+        assert run(kind, dtype, 0)[0] != 0 and run(kind, dtype, need - 4)[0] != 0 and run(kind, dtype, need)[0] == 0
 
 
 def test_gate_up_activation_epilogue_refuses_small_shapes(dev):
