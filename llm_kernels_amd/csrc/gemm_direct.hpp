@@ -112,14 +112,14 @@ __device__ __forceinline__ v4f raw_f32(const v4f& t) {
     }
 }
 
-// Division by a number that the host knows, for numerators below 2^31: ceil(2^(32 + shift) / d) - 2^32 and a shift (Granlund and Montgomery, Division by
-// Invariant Integers using Multiplication, 1994).  A scalar division by a kernel argument is some 30 dependent instructions, and short launches had up to
-// four of them in front of their first load.  (With the reads of wv_store ahead of their sums, a captured layer, quantiser and product, us, weights from
-// HBM: fp8 16 x 4096 x 4096 7.9 | 7.6, int8 9 x 6144 x 4096 11.3 | 10.9, w4a8 3 x 4096 x 4096 8.4 | 7.9, 16 x 14336 x 4096 12.9 | 12.2, row-packed bf16 40 x
-// 4096 x 4096 8.4 | 8.0, Marlin 64 x 4096 x 4096 9.3 | 8.8; fp8 16 x 28672 x 4096 30.1 | 29.8.)
+// Division by a number d >= 1 that the host knows, for numerators below 2^31: with l = ceil(log2 d) the quotient is (floor(m n / 2^32) + n) >> l, m =
+// floor(2^32 (2^l - d) / d) + 1 (Granlund and Montgomery, Division by Invariant Integers using Multiplication, 1994).  A scalar division by a kernel
+// argument is some 30 dependent instructions, and short launches had up to four of them in front of their first load.  (With the reads of wv_store
+// ahead of their sums, a captured layer, quantiser and product, us, weights from HBM: fp8 16 x 4096 x 4096 7.9 | 7.6, int8 9 x 6144 x 4096 11.3 | 10.9,
+// w4a8 3 x 4096 x 4096 8.4 | 7.9, 16 x 14336 x 4096 12.9 | 12.2, row-packed bf16 40 x 4096 x 4096 8.4 | 8.0, Marlin 64 x 4096 x 4096 9.3 | 8.8.)
 struct FastDiv {
     uint32_t mul, shift;
-    __host__ __device__ uint32_t operator()(uint32_t n) const { return ((uint32_t)(((uint64_t)mul * n) >> 32) + n) >> shift; }
+    __host__ __device__ constexpr uint32_t operator()(uint32_t n) const { return ((uint32_t)(((uint64_t)mul * n) >> 32) + n) >> shift; }
 };
 constexpr FastDiv fast_div(uint32_t d) {
     uint32_t l = 0;
@@ -129,7 +129,7 @@ constexpr FastDiv fast_div(uint32_t d) {
 constexpr bool fast_div_ok(uint32_t d) {
     const uint32_t n[] = {0, 1, d - 1, d, d + 1, 2 * d - 1, 0x7fffffffu, 0x7fffffffu / d * d, 0x7fffffffu / d * d - 1};
     for (uint32_t x : n)
-        if (x < 0x80000000u && ((uint32_t)(((uint64_t)fast_div(d).mul * x) >> 32) + x) >> fast_div(d).shift != x / d) return false;
+        if (x < 0x80000000u && fast_div(d)(x) != x / d) return false;
     return true;
 }
 static_assert(fast_div_ok(1) && fast_div_ok(2) && fast_div_ok(3) && fast_div_ok(7) && fast_div_ok(8) && fast_div_ok(641) && fast_div_ok(65537) && fast_div_ok(0x3fffffffu),
@@ -152,14 +152,15 @@ struct DirectArgs {
     long long* clocks;     // 256-column tile kernel, calibration only: workgroup 0 leaves the s_memtime and s_memrealtime ticks it lived
     const int8_t* w4_s4;   // uint4 weights with two-level scales: second-level scales [N, K/128]
     const int8_t* w4_z4;   // the same: zero points [N, K/128]
-    int tail_split;        // 256-column tile kernel: the tiles of a short last round are split along K (partial = scratch)    // 256-column tile kernel with the gated-activation epilogue (grouped gate / up projection, N = 2 I): c receives the
+    int tail_split;        // 256-column tile kernel: the tiles of a short last round are split along K (partial = scratch)
+    // 256-column tile kernel with the gated-activation epilogue (grouped gate / up projection, N = 2 I): c receives the
     // 1 x 128 quantised activations [M, I] in the operand type, q_scale their scales [M, I / 128]
     void* q_scale;
-    // wave kernels: divisions by the launch's row tiles, by a scale group's K steps and by the table loads of a column
-    FastDiv by_rows, by_group, by_words;
-    int words;
     int act;               // 0 = SiLU, 1 = GELU (tanh form)
     int round_mode;        // int8 rounding of the quantiser
+    // wave kernels: divisions by the launch's row tiles, by a scale group's K steps and by the table loads of a column, and those loads
+    FastDiv by_rows, by_group, by_words;
+    int words;
 };
 
 // Grouped launches: a tile list in which segment e owns ceil(rows of e / bm) * mult consecutive entries.
