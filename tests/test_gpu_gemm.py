@@ -139,12 +139,12 @@ def test_int8_per_token_int32_bit_exact(dev, M, N, K):
 
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 13])
 @pytest.mark.parametrize("M", [2000, 4000])            # the 128 x 256 and the 256 x 256 tile, the last tile row ragged
-@pytest.mark.parametrize("kind", ["fp8", "int8"])
+@pytest.mark.parametrize("kind", ["fp8", "int8", "int8 fp16 scales", "int8 bf16 scales"])
 def test_scales_of_every_k_step_on_large_tiles(dev, kind, M, steps):
     """Small integers under scales that are powers of two of their own in every row, column block and K step: every product and sum is
     a whole number below 2^24, so the fp32 result is exact in any order, and a scale taken from another step or row shows."""
     announce("scales on large tiles", kind, M, steps)
-    check_scales_of_every_k_step(dev, kind, M, 4096, steps, torch.float32)
+    check_scales_of_every_k_step(dev, kind.split()[0], M, 4096, steps, torch.float16 if " fp16" in kind else torch.bfloat16 if "bf16" in kind else torch.float32)
 
 
 @pytest.mark.parametrize("steps", [1, 3, 4, 6, 9, 31, 62])

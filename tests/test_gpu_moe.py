@@ -761,7 +761,7 @@ def test_ep_moe_forward_fused_equals_unfused(dev, kind):
 
 @pytest.mark.parametrize("qdt", [torch.float8_e4m3fn, torch.int8])
 @pytest.mark.parametrize("dtype,act", [(torch.bfloat16, "silu"), (torch.float16, "gelu")])
-@pytest.mark.parametrize("rows,two_i,K", [(8000, 4096, 256), (4800, 4096, 256), (8000, 3840, 384)])
+@pytest.mark.parametrize("rows,two_i,K", [(8000, 4096, 256), (4800, 4096, 256), (8000, 3840, 384), (8000, 4096, 640), (4800, 4096, 1152)])
 def test_gate_up_gemm_with_activation_epilogue_equals_three_kernels(dev, qdt, dtype, act, rows, two_i, K):
     """grouped_gemm_swiglu_quant == act_and_mul_quant(grouped_gemm_triton(...)) bit for bit, values and scales, on shapes
     that the dispatch gives to the 256-row (8000 rows) and 128-row (4800 rows) tiles of the large grouped kernel: a
@@ -788,7 +788,38 @@ def test_gate_up_activation_epilogue_of_part_tiles(dev, qdt, dtype, act, rows, c
     check_gate_up_epilogue(dev, qdt, dtype, act, rows, 4096, 256, seg, odd_rows=True)
 
 
-def check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, seg, odd_rows=False):
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13])
+@pytest.mark.parametrize("N", [4096, 2048])             # the 256 x 256 and the 128 x 256 tile
+@pytest.mark.parametrize("kind", ["fp8", "int8", "int8 fp16 scales"])
+def test_grouped_scales_of_every_k_step(dev, kind, N, steps):
+    """Small integers under scales that are powers of two of their own in every row, column block and K step: every product and sum is a whole number
+    below 2^24, so the result is exact, and a scale taken from another step, row or segment shows."""
+    announce("grouped gemm, scales of every K step", kind, N, steps)
+    gen = torch.Generator(device=dev).manual_seed(steps + N)
+    ints = lambda lo, hi, *shape: torch.randint(lo, hi + 1, shape, device=dev, generator=gen)
+    K, E, seg = 128 * steps, 4, [0, 701, 1982, 2909, 4000]
+    a, b = ints(-3, 3, seg[-1], K), ints(-3, 3, E, N, K)
+    a_s, b_s = 2.0 ** ints(0, 4, seg[-1], steps).float(), 2.0 ** ints(0, 4, E, N // 128, steps).float()
+    widx = torch.tensor([2, 0, 3, 1], device=dev)
+    wide = lambda s, dim: s.double().repeat_interleave(128, dim)
+    ref = torch.cat([(a[lo:hi].double() * wide(a_s[lo:hi], 1)) @ (b[w].double() * wide(wide(b_s[w], 1), 0)).t() for lo, hi, w in zip(seg, seg[1:], widx.tolist())])
+    qdt = torch.float8_e4m3fn if kind == "fp8" else torch.int8
+    sdt = torch.float16 if "fp16" in kind else torch.float32
+    c = torch.empty(seg[-1], N, device=dev)
+    gk.grouped_gemm_triton(a.float().to(qdt), b.float().to(qdt), c, E, True, torch.tensor(seg, device=dev), widx, False, a_s.to(sdt), b_s.to(sdt), [128, 128])
+    assert torch.equal(c.double(), ref)
+
+
+@pytest.mark.parametrize("dtype,act", [(torch.bfloat16, "silu"), (torch.float16, "gelu")])
+@pytest.mark.parametrize("rows", [8000, 4800])
+def test_gate_up_activation_epilogue_of_nan_codes(dev, dtype, act, rows):
+    """Single e4m3 weights that are no numbers, in gate and up columns: a row's other values keep their finite maximum, and what is stored is NaN there only."""
+    announce("gate/up + activation epilogue, NaN codes", dtype, act, rows)
+    torch.manual_seed(rows + 1)
+    check_gate_up_epilogue(dev, torch.float8_e4m3fn, dtype, act, rows, 4096, 256, [rows // 8 * e for e in range(9)], nan_codes=True)
+
+
+def check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, seg, odd_rows=False, nan_codes=False):
     E, used = len(seg) - 1, seg[-1]
     seg = torch.tensor(seg, dtype=torch.int64, device=dev)
     widx = torch.randperm(E).to(dev)
@@ -800,6 +831,12 @@ def check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, seg, odd_rows=F
     ws = [wq((torch.randn(two_i, K) * 0.3).to(dev)) for _ in range(E)]
     b = torch.stack([t[0].view(torch.uint8) for t in ws]).view(qdt)
     b_s = torch.stack([t[1] for t in ws])
+    expected = torch.zeros(used, two_i // 2, dtype=torch.bool)
+    if nan_codes:
+        for w, column, k in ((0, 5, 3), (1, two_i // 2 + 300, 100), (2, 127, 0), (2, two_i // 2 + 128, K - 1), (3, two_i // 2 - 1, 64)):
+            b.view(torch.uint8)[w, column, k] = 0x7f if k & 1 else 0xff
+            e = widx.tolist().index(w)
+            expected[seg[e]:seg[e + 1], column % (two_i // 2)] = True
     assert gk.grouped_gemm_swiglu_quant_fused(a, b, E)
     q1, s1 = gk.grouped_gemm_swiglu_quant(a, a_s, b, b_s, E, seg, widx, dtype, act)
 
@@ -812,7 +849,13 @@ def check_gate_up_epilogue(dev, qdt, dtype, act, rows, two_i, K, seg, odd_rows=F
     live = torch.ones(used, dtype=torch.bool)
     if odd_rows: live[[7, used - 3]] = False
     assert torch.equal(s1[:used].cpu()[live], s0[:used].cpu()[live])
-    assert torch.equal(q1[:used].view(torch.uint8).cpu()[live], q0[:used].view(torch.uint8).cpu()[live])
+    u1, u0 = q1[:used].view(torch.uint8).cpu(), q0[:used].view(torch.uint8).cpu()
+    if qdt == torch.float8_e4m3fn:                          # (a NaN's sign is nobody's; to int8 NaN has no value)
+        nan = (u0 & 0x7f) == 0x7f
+        assert torch.equal((u1 & 0x7f) == 0x7f, nan) and torch.equal(u1[~nan], u0[~nan])
+        assert torch.equal(nan[live], expected[live])
+    else:
+        assert torch.equal(u1[live], u0[live])
     assert torch.equal(s1[:used].cpu().float().nan_to_num(-1.0), s0[:used].cpu().float().nan_to_num(-1.0))
     assert float(s0[:used].cpu()[live].float().abs().max()) > 0
 
