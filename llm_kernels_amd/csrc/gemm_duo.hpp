@@ -363,6 +363,8 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         // them).  us, requests first | reads first, then requests | expansion in front of the requests: rows 300 x 14336 x 4096 bf16 44.1 | 42.7 | 41.9, fp16
         // 44.9 | 43.4 | 42.6, bf16 512 x 6144 x 4096 36.7 | 37.9 | 35.8, fp16 1500 x 4096 x 4096 55.1 | 52.6 | 52.4, Marlin 320 x 14336 x 4096 47.0 | 43.4 |
         // 46.7, 768 x 4096 x 7168 61.6 | 58.5 | 60.9.  8-bit operands: no difference (fp8 1024 x 4096 x 4096 25.9 | 25.8, int8 200 x 14336 x 4096 25.0 | 25.3).
+        // 45 random shapes of 65 to 700 rows a kind, cached weights (from HBM): Marlin words 1.08 (1.055), fp16 rows 1.04 (1.03), bf16 1.03 (1.02) times as fast as
+        // with the requests first; wide row-packed weights from HBM lose up to 4.5 % (bf16 150 x 24856 x 13184 131 | 138 us).
         auto expand_words = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_sched_barrier(0);
             words_landed(u & 3);

@@ -169,7 +169,8 @@ __global__ __launch_bounds__(MD_THREADS) void gemm_mid_pc_kernel(DirectArgs p) {
         // 14336 33.3 (41.0) | 32.6 (37.9), 70 x 4096 x 4096 9.8 (10.3) | 9.6 (10.1), fp8 256 x 4096 x 7168 20.6 (24.1) | 20.2 (23.3)).  WIDE: the scale column of a
         // sub-block, 64 rows per producer, the two producers of the sub-block take 64 rows each (32 rows x two scales were 1 % slower: fp8 256 x
         // 6144 x 4096 17.8 | 18.2).
-        constexpr int NSC = WIDE ? 1 : BM / 16;              // loads for all rows of a 64-column tile
+        // loads for all rows of a 64-column tile (32-row tiles: two producers make each of the two, as every producer counts the same loads)
+        constexpr int NSC = WIDE ? 1 : BM / 16;
         const uint32_t soff = WIDE ? (uint32_t)min(m_start + min(lane + 64 * half, BM - 1), m_end - 1) * (uint32_t)KT_all * SSZ
                                    : ((uint32_t)min(m_start + (q % NSC) * 16 + (lane >> 2), m_end - 1) * (uint32_t)KT_all + (uint32_t)kt0) * SSZ;
         // sub-block ksub of step s, clamped to the last one of the range (requests past the end repeat it)

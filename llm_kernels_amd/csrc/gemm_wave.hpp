@@ -398,8 +398,9 @@ int launch_w4a8_wave(const DirectArgs& p, int z, hipStream_t stream, const char*
 
 // ------------------------------------------------------------------------------------------------------------
 // fp16 / bf16 activations [M, K], 4-bit weights with fp16 group scales: row-packed [N, K / 8] (K_W4NK, K_W4NKB) or Marlin words
-// (K_W4MARLIN).  K steps are 128 elements of weights and two halves of 64 elements (128 bytes) of activations: per wave one
-// stage of activation rows and two of packed words (a second stage of activations has no room beside 64 rows).
+// (K_W4MARLIN).  K steps are 128 elements of weights and two halves of 64 elements (128 bytes) of activations.  16-row tiles: a wave has one stage
+// for a whole step, words and both halves.  More rows: one stage of activation rows, half a step, requested a half ahead, and two of packed
+// words (a second stage of activations has no room beside 64 rows).
 // What bounds it: latency.  64 x 14336 x 4096, of 37600 cycles a wave lives: vector ALU 46 %, address path 52 %, LDS 30 %, MFMA 22 %;
 // a half's activations are requested one half ahead, which two waves per SIMD do not cover.  The words of a chunk come from LDS
 // with the order of the activations' dwords as the Marlin fragments want it; scattering them into rows was most of the tile kernel.
@@ -456,9 +457,13 @@ __global__ __launch_bounds__(NW * 64) void w4a16_wave_kernel(DirectArgs p) {
     static_assert(PRE || !wh_marlin(KIND), "Marlin words: scaled weights");
     constexpr bool MARLIN = wh_marlin(KIND), BF = (KIND == K_W4NKB);
     constexpr int BM = 16 * MT, BN = 16 * NT, STAGE = wh_stage(KIND, MT, NT), WB = wh_b(KIND, NT), NB = WB / 1024;
-    // 16 rows: a step's words and activations are one request, and the wave waits once for them: us for Marlin words, halves | whole steps, weights in the
-    // cache (from HBM): 16 x 4096 x 4096 6.49 (7.22) | 6.30 (6.76), 16 x 14336 x 4096 10.4 (12.1) | 10.1 (11.7), 16 x 9984 x 1152 6.2 (6.7) | 5.8 (6.2).  Two
-    // stages of them are slower (6.85: twice the loads are issued in front of the scale table), and so are whole steps of 32 rows from HBM (32 x
+    // 16 rows: a step's words and activations are one request, and the wave waits once for them: us, halves | whole steps, weights in the cache (from
+    // HBM): Marlin words 16 x 4096 x 4096 6.49 (7.22) | 6.30 (6.76), 16 x 14336 x 4096 10.4 (12.1) | 10.1 (11.7), 16 x 9984 x 1152 6.2 (6.7) | 5.8 (6.2); row-packed
+    // ones, fp16 20 x 1416 x 11904 9.6 (12.7) | 8.7 (11.0), 44 x 2240 x 5248 7.7 (9.2) | 7.5 (8.6), bf16 29 x 4096 x 14336 15.8 (18.4) | 13.7 (15.9), 34 x 4208 x 4864
+    // 9.7 (11.5) | 10.0 (11.3).  25 random shapes a type and width, 16, 32, 64 columns: bf16 1.11 (1.11), 1.12 (1.15), 0.98 (1.02) times as fast as in halves,
+    // fp16 1.07 (1.10), 1.03 (1.07), 1.03 (1.03).  The larger stage (5 KB a wave for 4 at 16 columns) costs no residency: of 57000 calls that get 16-row tiles
+    // of row-packed words all on eight waves are at most one workgroup a CU, those on four at most two.  Two stages of whole steps are
+    // slower (Marlin 16 x 4096 x 4096 6.85: twice the loads are issued in front of the scale table), and so are whole steps of 32 rows from HBM (Marlin 32 x
     // 14336 x 4096 14.1 | 14.7).
     constexpr bool WHOLE = MT == 1;
     constexpr int OFF_B = (WHOLE ? 2 : 1) * wh_a(MT);
@@ -1027,7 +1032,9 @@ inline int wave_shape(const WavePlan& w, int form, int32_t* shape) {
 // their rounds count in fractions; slower on a single round (w4a8 64 x 14336 x 4096 18.2 against 17.0 us), faster from two on
 // (64 x 28672 x 4096 27.6 against 30.2, 128 rows 46.8 against 54).  The numbers are a fit (5 to 8 % rms) to 100 to 180 shapes of M
 // 1 to 520, N 1024 to 28672, K 1024 to 14336 a kind, every tile shape timed; [mt - 1][log2 nt], and [mt - 1] for four waves (0:
-// shape not built).
+// shape not built).  They are of the kernels with a division in front of the loads and half steps on 16-row tiles.  On the present ones the tile that they
+// choose takes, against the fastest one that is built (45 random shapes of 1 to 300 rows a kind, all tiles timed, mean of cached weights and weights from HBM),
+// fp8 1.016 of its time, int8 and per token 1.010, w4a8 1.006, row-packed bf16 1.009, fp16 1.028, Marlin words 1.009.
 struct WaveModel {
     float base8[4][3], fixed8[4][3], step8[4][3], base4[4], step4[4];
 };
