@@ -363,8 +363,12 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
         // them).  us, requests first | reads first, then requests | expansion in front of the requests: rows 300 x 14336 x 4096 bf16 44.1 | 42.7 | 41.9, fp16
         // 44.9 | 43.4 | 42.6, bf16 512 x 6144 x 4096 36.7 | 37.9 | 35.8, fp16 1500 x 4096 x 4096 55.1 | 52.6 | 52.4, Marlin 320 x 14336 x 4096 47.0 | 43.4 |
         // 46.7, 768 x 4096 x 7168 61.6 | 58.5 | 60.9.  8-bit operands: no difference (fp8 1024 x 4096 x 4096 25.9 | 25.8, int8 200 x 14336 x 4096 25.0 | 25.3).
-        // 45 random shapes of 65 to 700 rows a kind, cached weights (from HBM): Marlin words 1.08 (1.055), fp16 rows 1.04 (1.03), bf16 1.03 (1.02) times as fast as
-        // with the requests first; wide row-packed weights from HBM lose up to 4.5 % (bf16 150 x 24856 x 13184 131 | 138 us).
+        // Random shapes of 65 to 520 rows, weights of 8 MB or more for the most part, cached (from HBM): Marlin words 1.08 (1.055) times as fast as with the requests first,
+        // row-packed ones on tiles of 96 | 128 | 160 | 192 rows fp16 1.03 (1.01) | 1.06 (1.03) | 1.06 (1.03) | 1.06 (1.03), bf16 1.01 (0.99) | 1.02 (1.01) | 1.04 (1.03) |
+        // 1.07 (1.03).  So bf16 on 96-row tiles keeps the requests first: little is expanded beside few rows, and wide weights wait for HBM (94 x 25864 x
+        // 6016 with the reads first 8 % slower).  What is left are single shapes of wide weights from HBM, with an odd number of K steps for the most part
+        // (rows of words then begin in the middle of a line): 2 to 8 % slower, 4 % faster cached (fp16 262 x 8896 x 8064).
+        constexpr bool READS_FIRST = W4A16 && !(KIND == K_W4NKB && MI == 3);
         auto expand_words = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_sched_barrier(0);
             words_landed(u & 3);
@@ -372,15 +376,16 @@ __global__ __launch_bounds__(DU_THREADS) void gemm_duo_kernel(DirectArgs p) {
             expand_word(u & 3, u + 1, 1);
             __builtin_amdgcn_sched_barrier(0);
         };
-        if constexpr (W4A16) {
+        if constexpr (READS_FIRST) {
             fetch(u);
             if constexpr (!MARLIN) expand_words();
             __builtin_amdgcn_sched_barrier(0);
         }
         request(u + 3);
         if constexpr (SCALES) request_scales((u >> 2) + 1);
+        if constexpr (W4A16 && !READS_FIRST) fetch(u);
         if constexpr (W4A16) {
-            if constexpr (MARLIN) expand_words();
+            if constexpr (MARLIN || !READS_FIRST) expand_words();
             request_words(u & 3, u + 5);
         }
         if constexpr (W4A8) {                                // (in front of the fragments, which leave no registers for it)
